@@ -5,23 +5,23 @@
 // Every output cell is summed in one order, whatever kernel computes it and whatever else is
 // in the batch: k is cut into slices of 64; a slice's products are added in ascending k by a
 // chain of fused multiply-adds that starts from zero; the slices' sums are added in ascending
-// order.  So a cell's bits do not depend on M, on the tile it falls in, or on which of the three
-// kernels ran:
+// order.  So a cell's bits do not depend on M, on the tile it falls in, or on which of the
+// kernels ran.  The matrix cores keep to it: v_mfma_f32_32x32x2_f32 adds its two products one after the other, each
+// fused and rounded as fmaf rounds it (denormals, infinities and NaN included: the tests compare bits), at twice the rate of the
+// vector units.
 //
-//  * tiled (any sizes): a 64 x 64 tile of C a workgroup, k in steps of 16 through LDS, a thread
-//    4 x 4 cells; after every fourth step (a slice) the chain's sum goes into the cell's total.
-//  * wide (prompts; rows of 16 bytes): a 128 x 64 tile a workgroup and 8 x 4 cells a thread, so
-//    that a k-step's 32 multiply-adds of a thread stand against three 16-byte reads from LDS
-//    where the tiled kernel has 16 against two; the next k-step's operands are on their way
-//    from memory while this one is multiplied, and LDS holds two k-steps, one barrier a step.
-//    (Tiles of 128 x 128 with 8 x 8 cells leave one wave a SIMD on square products of 2,048 and
-//    were slower at every size measured.)
-//  * skinny (M <= 64, rows of 16 bytes: a decode step, a short prompt portion): the tiled kernel
-//    would start N / 64 workgroups that walk all of k one step behind the other.  Here a workgroup
-//    owns 8 rows of W and every lane one (slice, row) pair: it asks for its 64 weights at once
-//    (64 KB on their way a workgroup), runs the chain for each row of A, and the slices' sums
-//    meet in LDS, where one thread a cell adds them in order.  N / 8 workgroups: one for every
-//    compute unit already at 2,048 rows of W.
+//  * tiled (any sizes, in practice rows that are no 16-byte words): a 64 x 64 tile of C a workgroup, k in steps of 16
+//    through LDS, a thread 4 x 4 cells; after every fourth step (a slice) the chain's sum goes into the cell's total.
+//  * wide (prompts; rows of 16 bytes): a 128 x 128 tile a workgroup on the matrix cores, two k-steps of 32 in LDS, the
+//    next one's operands on their way from memory; two workgroups a unit, so that one multiplies while the other waits
+//    at its barrier (2,048 x 16,384 x 2,048: 1,210 us, 114 TFLOP/s; on the vector units, 128 x 64 tiles, 65 to 85).
+//  * sliced (everything between): a 32 x 32 tile a workgroup, whose waves take slices of k in turn, so that a product of
+//    few tiles walks k in a quarter or an eighth of the steps (200 x 960 x 2,560: 458 us in the tiled kernel's 60
+//    workgroups, 24 here; 64 x 2,048 x 8,192: 565 in the skinny kernel, 65 here).
+//  * skinny (a few rows of 16 bytes: a decode step): a workgroup owns 4 or 16 rows of W and every lane one (slice, row)
+//    pair: all of a workgroup's weights (64 KB) are on their way at once, a lane runs the chain for each row of A, and the
+//    slices' sums meet in LDS, where one thread a cell adds them in order (1 x 960 x 2,560: 10.3 -> 5.5 us with whole lines
+//    through LDS and 4 rows of W a workgroup instead of 8; 1 x 49,152 x 960 64 -> 41 with 16).
 #include "common.h"
 
 using namespace gb;
@@ -96,53 +96,67 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   }
 }
 
-// ---- wide: 128 x 64 of C a workgroup, 8 x 4 cells a thread, two k-steps in LDS ------------------------------
-constexpr int WM = 128, WN = 64, WK = 16;
+// ---- matrix cores: v_mfma_f32_32x32x2_f32 --------------------------------------------------------------------
+// An operand of the instruction is one float a lane: row lane % 32, k = lane / 32.  A lane here loads 16-byte words: of
+// eight consecutive k of its row it has k = 4 (lane / 32) .. + 3, and pairs() turns the words into the four operands of
+// k = (0, 1), (2, 3), (4, 5), (6, 7) by swapping half waves.
+__device__ __forceinline__ void pairs(const f32x4& v, float (&p)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+  p[0] = __uint_as_float(a[0]);
+  p[1] = __uint_as_float(b[0]);
+  p[2] = __uint_as_float(a[1]);
+  p[3] = __uint_as_float(b[1]);
+}
+__device__ __forceinline__ f32x16 mfma(float a, float b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+// row of the 32 x 32 tile that register r of a lane holds; its column is lane % 32
+__device__ __forceinline__ int tile_row(int r, int lane) { return 8 * (r / 4) + 4 * (lane / 32) + r % 4; }
+
+// wide: 128 x 128 of C a workgroup, a wave 64 x 64; k-steps of 32 through two buffers in LDS
+constexpr int WM = 128, WN = 128, WK = 32;
+constexpr int WS = WK + 4;   // floats a row of a k-step: 144 bytes, so that the rows of a wave's reads lie on other banks
 static_assert(kSlice % WK == 0, "a slice is whole steps of the wide kernel");
 
-__global__ __launch_bounds__(256) void gemm_f32_wide_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w,
+__global__ __launch_bounds__(256, 2) void gemm_f32_wide_kernel(const float* __restrict__ a, int lda, const float* __restrict__ w,
                                                             int ldw, float* __restrict__ c, int ldc, int M, int N, int K,
                                                             int accumulate) {
-  constexpr int NB = WN / 64, CN = 4 * NB;   // blocks of 64 columns, columns a thread
-  __shared__ __attribute__((aligned(16))) float As[2][WK][WM + 4];
-  __shared__ __attribute__((aligned(16))) float Ws[2][WK][WN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
+  __shared__ __attribute__((aligned(16))) float As[2][WM * WS];
+  __shared__ __attribute__((aligned(16))) float Ws[2][WN * WS];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int wm = wave / 2 * 64, wn = wave % 2 * 64;
   const int m0 = blockIdx.y * WM, n0 = blockIdx.x * WN;
-  // a thread brings word lc of the k-step's four for rows lr and lr + 64 of the operands
-  const int lr = tid / 4, lc = tid % 4;
-  f32x4 pa[2], pw[NB];
+  // a thread brings word lc of the k-step's eight for rows lr, lr + 32, lr + 64 and lr + 96 of both operands
+  const int lr = tid / 8, lc = tid % 8;
+  f32x4 pa[4], pw[4];
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   auto fetch = [&](int k0) {
     const int gk = k0 + 4 * lc;   // K is whole words: a word is inside k or outside
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int gm = m0 + lr + 64 * h;
+    for (int h = 0; h < 4; ++h) {
+      const int gm = m0 + lr + 32 * h, gn = n0 + lr + 32 * h;
       pa[h] = (gm < M && gk < K) ? *reinterpret_cast<const f32x4*>(a + (size_t)gm * lda + gk) : zero;
-    }
-#pragma unroll
-    for (int h = 0; h < NB; ++h) {
-      const int gn = n0 + lr + 64 * h;
       pw[h] = (gn < N && gk < K) ? *reinterpret_cast<const f32x4*>(w + (size_t)gn * ldw + gk) : zero;
     }
   };
   auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) As[buf][4 * lc + i][lr + 64 * h] = pa[h][i];
-#pragma unroll
-      for (int h = 0; h < NB; ++h) Ws[buf][4 * lc + i][lr + 64 * h] = pw[h][i];
+    for (int h = 0; h < 4; ++h) {
+      *reinterpret_cast<f32x4*>(&As[buf][(lr + 32 * h) * WS + 4 * lc]) = pa[h];
+      *reinterpret_cast<f32x4*>(&Ws[buf][(lr + 32 * h) * WS + 4 * lc]) = pw[h];
     }
   };
-  // cells (ty*4 + i%4 + 64*(i/4), tx*4 + j%4 + 64*(j/4))
-  float acc[8][CN], total[8][CN];
+  f32x16 acc[2][2], total[2][2];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < CN; ++j) acc[i][j] = total[i][j] = 0.f;
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = total[i][j][r] = 0.f;
 
   const int steps = (K + WK - 1) / WK;
+  const int read = (lane % 32) * WS + 4 * (lane / 32);
   fetch(0);
   stash(0);
   __syncthreads();
@@ -150,115 +164,249 @@ __global__ __launch_bounds__(256) void gemm_f32_wide_kernel(const float* __restr
     const int buf = s & 1;
     if (s + 1 < steps) fetch((s + 1) * WK);
 #pragma unroll
-    for (int kk = 0; kk < WK; ++kk) {
-      float av[8], wv[CN];
+    for (int kk = 0; kk < WK; kk += 8) {
+      float av[2][4], wv[2][4];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&As[buf][kk][ty * 4 + 64 * h]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) av[4 * h + i] = x[i];
+      for (int i = 0; i < 2; ++i) {
+        pairs(*reinterpret_cast<const f32x4*>(&As[buf][(wm + 32 * i) * WS + read + kk]), av[i]);
+        pairs(*reinterpret_cast<const f32x4*>(&Ws[buf][(wn + 32 * i) * WS + read + kk]), wv[i]);
       }
 #pragma unroll
-      for (int h = 0; h < NB; ++h) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&Ws[buf][kk][tx * 4 + 64 * h]);
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wv[4 * h + i] = x[i];
-      }
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < CN; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma(av[i][q], wv[j][q], acc[i][j]);
     }
     if (((s + 1) * WK) % kSlice == 0 || s + 1 == steps) {   // a slice ends: its sum joins the total
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < CN; ++j) {
-          total[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
-        }
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            total[i][j][r] += acc[i][j][r];
+            acc[i][j][r] = 0.f;
+          }
     }
     // the other half of LDS was last read a step ago, before the barrier that every thread has passed since
     if (s + 1 < steps) stash(buf ^ 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int gm = m0 + ty * 4 + (i & 3) + 64 * (i >> 2);
-    if (gm >= M) continue;
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < CN; ++j) {
-      const int gn = n0 + tx * 4 + (j & 3) + 64 * (j >> 2);
+    for (int j = 0; j < 2; ++j) {
+      const int gn = n0 + wn + 32 * j + lane % 32;
       if (gn >= N) continue;
-      float* dst = c + (size_t)gm * ldc + gn;
-      *dst = accumulate ? *dst + total[i][j] : total[i][j];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int gm = m0 + wm + 32 * i + tile_row(r, lane);
+        if (gm >= M) continue;
+        float* dst = c + (size_t)gm * ldc + gn;
+        *dst = accumulate ? *dst + total[i][j][r] : total[i][j][r];
+      }
+    }
+}
+
+// sliced: 32 x 32 of C a workgroup, whose waves take the slices of k in turn; the slices' sums of a round meet in LDS,
+// where one thread adds a cell's in order.  A wave brings its slice of both operands straight into LDS, whole rows of
+// 256 bytes (word p of row r lies at position p ^ (r % 16), so that a read's 16 neighbouring rows spread over all
+// banks): loaded by the lanes that multiply them, an instruction of a wave touches 32 bytes of 32 rows, 100 cycles each.
+template <int NW>
+__global__ __launch_bounds__(NW * kWave) void gemm_f32_sliced_kernel(const float* __restrict__ a, int lda,
+                                                                     const float* __restrict__ w, int ldw,
+                                                                     float* __restrict__ c, int ldc, int M, int N, int K,
+                                                                     int accumulate) {
+  constexpr int T = 32, CELLS = T * T / (NW * kWave);   // cells a thread adds up
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // a wave's slice [2][32][64], then the sums [NW][32 * 32]
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  float* own = smem + wave * (2 * T * kSlice);
+  float* part = smem + NW * (2 * T * kSlice);
+  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+  const int slices = (K + kSlice - 1) / kSlice;
+  auto fetch = [&](int slice) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int row = (u % 8) * 4 + lane / 16;   // the first eight instructions bring A, the others W
+      // (a word beyond k is replaced by zeros where it is read, a row beyond m or n goes nowhere: any address inside will do)
+      const int k = slice * kSlice + 4 * ((lane % 16) ^ (row % 16));
+      const float* from = (u < 8 ? a + (size_t)min(m0 + row, M - 1) * lda : w + (size_t)min(n0 + row, N - 1) * ldw) + (k < K ? k : 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)(uintptr_t)from,
+                                       (__attribute__((address_space(3))) uint32_t*)(uint32_t)(uintptr_t)(own + u * 256), 16, 0, 0);
+    }
+  };
+  float total[CELLS];
+#pragma unroll
+  for (int e = 0; e < CELLS; ++e) total[e] = 0.f;
+  if (wave < slices) fetch(wave);
+  for (int s0 = 0; s0 < slices; s0 += NW) {
+    const int slice = s0 + wave;
+    if (slice < slices) {   // the same for a whole wave
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      f32x4 av[8], wv[8];
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      const int r = lane % 32;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int word = 2 * i + lane / 32;
+        const bool in = slice * kSlice + 4 * word < K;
+        const f32x4 x = *reinterpret_cast<const f32x4*>(own + r * kSlice + 4 * (word ^ (r % 16)));
+        const f32x4 y = *reinterpret_cast<const f32x4*>(own + (T + r) * kSlice + 4 * (word ^ (r % 16)));
+        av[i] = in ? x : zero;
+        wv[i] = in ? y : zero;
+      }
+      // every operand is in registers: the next slice may come in under the products
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (slice + NW < slices) fetch(slice + NW);
+      f32x16 acc;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[q] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float x[4], y[4];
+        pairs(av[i], x);
+        pairs(wv[i], y);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = mfma(x[q], y[q], acc);
+      }
+#pragma unroll
+      for (int q = 0; q < 16; ++q) part[wave * (T * T) + tile_row(q, lane) * T + lane % 32] = acc[q];
+    }
+    // (the sums must be there; the loads that are on their way need not)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int count = min(NW, slices - s0);
+#pragma unroll
+    for (int e = 0; e < CELLS; ++e) {
+      float v[NW];
+#pragma unroll
+      for (int q = 0; q < NW; ++q) v[q] = q < count ? part[q * (T * T) + tid + e * NW * kWave] : 0.f;
+#pragma unroll
+      for (int q = 0; q < NW; ++q)
+        if (q < count) total[e] += v[q];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+#pragma unroll
+  for (int e = 0; e < CELLS; ++e) {
+    const int cell = tid + e * NW * kWave;
+    const int cm = m0 + cell / T, cn = n0 + cell % T;
+    if (cm < M && cn < N) {
+      float* dst = c + (size_t)cm * ldc + cn;
+      *dst = accumulate ? *dst + total[e] : total[e];
     }
   }
 }
 
-// the wide kernel from so many of its tiles on; below that the small tiles spread the work further
-constexpr int kWideMinTiles = 64;
+template <int NW>
+int launch_sliced(const float* a, int lda, const float* w, int ldw, float* c, int ldc, int M, int N, int K, int accumulate,
+                  hipStream_t stream) {
+  const dim3 grid((N + 31) / 32, (M + 31) / 32);
+  GB_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d needs more than 65535 row tiles", M);
+  hipLaunchKernelGGL(gemm_f32_sliced_kernel<NW>, grid, dim3(NW * kWave), NW * (2 * 32 * kSlice + 32 * 32) * 4, stream, a, lda, w,
+                     ldw, c, ldc, M, N, K, accumulate);
+  return launched("gemm_f32 (sliced)");
+}
 
-// ---- skinny: 8 rows of W a workgroup, a lane a (slice, row) pair ------------------------------------------
-constexpr int SR = 8;             // rows of W a workgroup
-constexpr int SG = 256 / SR;      // slices in flight a workgroup: one a lane group of SR lanes
+// The wide kernel from so many of its tiles on: with fewer, units are idle while a tile walks all of k (us, wide / sliced:
+// 160 tiles, 400 x 5,120 x 960, 88 / 71; 200 tiles, 600 rows, 89 / 92; 256 tiles, 2,048 x 2,048 x 8,192, 711 / 912).
+constexpr int kWideMinTiles = 192;
+// Up to so many tiles a unit has one workgroup of the sliced kernel at most: eight waves then walk k in half the rounds
+// (200 x 960 x 2,560 29.7 -> 23.6 us).  With more, two workgroups of four waves share a unit, one's loads on their way
+// under the other's products (2,048 x 960 x 960 69.7 -> 64.0).
+constexpr int kFewTiles = 256;
+
+// ---- skinny: R rows of W a workgroup, a lane a (slice, row) pair ------------------------------------------
+// What a lane multiplies lies 256 bytes from what its neighbour does: loaded into registers by the lane itself, an
+// instruction of a wave would touch 64 lines of memory, each again by seven more.  So W goes through LDS: a wave's
+// instruction brings four slices of a row (a kilobyte in a run) straight into LDS, where a lane reads its own slice.
+// Word p of the slice of pair t lies at position p ^ (t % 16), so that the reads of 16 neighbouring lanes spread over all banks.
 constexpr int SV = kSlice / 4;    // 16-byte words a slice of one row
 
-template <int MT>   // rows of A a pass (the step's rows go MT at a time)
+template <int MT, int R>   // rows of A a pass (the step's rows go MT at a time); rows of W a workgroup
 __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
                                                               const float* __restrict__ w, int ldw,
                                                               float* __restrict__ c, int ldc, int M, int N, int K,
                                                               int accumulate) {
-  __shared__ float part[SG][SR][MT];
-  const int tid = threadIdx.x;
-  const int r = tid % SR, sl = tid / SR;
-  const int n = blockIdx.x * SR + r;
+  constexpr int SG = 256 / R;   // slices in flight a workgroup
+  extern __shared__ __attribute__((aligned(16))) float wl[];   // [R][SG][64], then part [SG][R][MT]
+  float* part = wl + 256 * kSlice;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int r = tid % R, sl = tid / R;
+  const int n0 = blockIdx.x * R;
   const int slices = (K + kSlice - 1) / kSlice;
   // the thread that adds the slices of cell (row cm of the pass, column cr)
-  const int cr = tid % SR, cm = tid / SR;
+  const int cr = tid % R, cm = tid / R;
 
   for (int m0 = 0; m0 < M; m0 += MT) {
     float total = 0.f;
     for (int s0 = 0; s0 < slices; s0 += SG) {
-      const int k0 = (s0 + sl) * kSlice;
-      const bool live = n < N && k0 < K;
-      f32x4 wv[SV];
 #pragma unroll
-      for (int i = 0; i < SV; ++i) {
-        const int k = k0 + 4 * i;
-        wv[i] = (live && k < K) ? *reinterpret_cast<const f32x4*>(w + (size_t)n * ldw + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < 16; ++u) {
+        // four slices of a row, which one wave brings: unit u of the wave's
+        const int unit = wave * 16 + u, row = unit / (SG / 4), first = unit % (SG / 4) * 4;
+        if (s0 + first >= slices) continue;                                // the same for the whole wave
+        const int mine = first + lane / 16;
+        const int word = (lane % 16) ^ ((mine * R + row) % 16);
+        // (a word beyond k or n is not used: any address inside W will do for it)
+        const int k = (s0 + mine) * kSlice + 4 * word;
+        const float* from = w + (size_t)min(n0 + row, N - 1) * ldw + (k < K ? k : 0);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)(uintptr_t)from,
+                                         (__attribute__((address_space(3))) uint32_t*)(uint32_t)(uintptr_t)(wl + unit * 256), 16, 0, 0);
       }
+      const int k0 = (s0 + sl) * kSlice;
+      const bool live = k0 < K;
+      // a single row of A is asked for before W has arrived
+      f32x4 x1[MT == 1 ? SV : 1];
+      if (MT == 1) {
+#pragma unroll
+        for (int i = 0; i < SV; ++i) {
+          const int k = k0 + 4 * i;
+          x1[MT == 1 ? i : 0] = *reinterpret_cast<const f32x4*>(a + (size_t)m0 * lda + (k < K ? k : 0));
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
       float acc[MT];
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[m] = 0.f;
       if (live) {
+        const float* own = wl + (r * SG + sl) * kSlice;
 #pragma unroll
         for (int i = 0; i < SV; ++i) {
           const int k = k0 + 4 * i;
           if (k < K) {
+            const f32x4 wv = *reinterpret_cast<const f32x4*>(own + 4 * (i ^ (tid % 16)));
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-              if (m0 + m < M) {
-                const f32x4 x = *reinterpret_cast<const f32x4*>(a + (size_t)(m0 + m) * lda + k);
-                acc[m] = fmaf(x[0], wv[i][0], acc[m]);
-                acc[m] = fmaf(x[1], wv[i][1], acc[m]);
-                acc[m] = fmaf(x[2], wv[i][2], acc[m]);
-                acc[m] = fmaf(x[3], wv[i][3], acc[m]);
+              if (MT == 1 || m0 + m < M) {
+                const f32x4 x = MT == 1 ? x1[MT == 1 ? i : 0] : *reinterpret_cast<const f32x4*>(a + (size_t)(m0 + m) * lda + k);
+                acc[m] = fmaf(x[0], wv[0], acc[m]);
+                acc[m] = fmaf(x[1], wv[1], acc[m]);
+                acc[m] = fmaf(x[2], wv[2], acc[m]);
+                acc[m] = fmaf(x[3], wv[3], acc[m]);
               }
             }
           }
         }
       }
 #pragma unroll
-      for (int m = 0; m < MT; ++m) part[sl][r][m] = acc[m];
+      for (int m = 0; m < MT; ++m) part[(sl * R + r) * MT + m] = acc[m];
       __syncthreads();
       if (cm < MT) {
         const int count = min(SG, slices - s0);
-        for (int s = 0; s < count; ++s) total += part[s][cr][cm];
+        for (int s = 0; s < count; s += 8) {
+          float v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[q] = part[(min(s + q, SG - 1) * R + cr) * MT + cm];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            if (s + q < count) total += v[q];
+        }
       }
-      __syncthreads();
+      if (s0 + SG < slices || m0 + MT < M) __syncthreads();
     }
-    const int gm = m0 + cm, gn = blockIdx.x * SR + cr;
+    const int gm = m0 + cm, gn = n0 + cr;
     if (cm < MT && gm < M && gn < N) {
       float* dst = c + (size_t)gm * ldc + gn;
       *dst = accumulate ? *dst + total : total;
@@ -266,46 +414,61 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
   }
 }
 
-template <int MT>
+template <int MT, int R>
 void launch_skinny(const float* a, int lda, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
-                   int accumulate, hipStream_t stream) {
-  static_assert(MT <= SG, "one thread a cell of a pass");
-  hipLaunchKernelGGL(gemm_f32_skinny_kernel<MT>, dim3((N + SR - 1) / SR), dim3(256), 0, stream, a, lda, w, ldw, c, ldc, M, N,
-                     K, accumulate);
+                        int accumulate, hipStream_t stream) {
+  static_assert(MT * R <= 256, "one thread a cell of a pass");
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, R>), dim3((N + R - 1) / R), dim3(256), 256 * (kSlice + MT) * 4, stream, a, lda,
+                     w, ldw, c, ldc, M, N, K, accumulate);
 }
-
 constexpr int kSkinnyMaxRows = 64;
+// Where the skinny kernel is the faster one (us, skinny / sliced, replayed from a graph over weights that no cache holds):
+// up to 4 rows of narrow products (960 x 960 at 1 and 4 rows 3.8 and 8.1 / 9.4, 2,048 x 8,192 17 and 29 / 63), up to 8
+// where k is long (2,048 x 8,192 at 8 rows 48 / 63, but 960 x 960 12.9 / 9.4); wide products read W at the memory's pace
+// with 16 rows a workgroup, and the sums of more than two rows of A then take longer than the matrix cores
+// (49,152 x 960 at 1, 2 and 4 rows 41, 50 and 67 / 53; with 4 rows of W a workgroup 67, 106 and 167).
+constexpr int kNarrow = 4096, kLongK = 2048;
+inline bool skinny_pays(int M, int N, int K) {
+  return N <= kNarrow ? M <= 4 || (M <= 8 && K >= kLongK) : M <= 2;
+}
 
 inline bool words_of_16_bytes(const void* p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0; }
 
 }  // namespace
 
-// which = 0: the kernel the sizes call for; 1: the tiled kernel; 2: the skinny kernel; 3: the wide kernel (the last
-// two refused where they do not apply).  All give the same bits; tests compare them.
+// which = 0: the kernel the sizes call for; 1: the tiled kernel; 2: the skinny kernel; 3: the wide kernel; 4 and 5: the
+// sliced kernel with four and eight waves (all but the tiled one refused where they do not apply).  All give the same
+// bits; tests compare them.
 extern "C" int gb_gemm_f32_by(const float* a, int lda, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
                               int accumulate, int which, hipStream_t stream) {
   GB_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   GB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: a leading dimension is shorter than its row (lda=%d ldw=%d ldc=%d)", lda, ldw, ldc);
-  GB_REQUIRE(which >= 0 && which <= 3, "gemm_f32: no kernel %d", which);
+  GB_REQUIRE(which >= 0 && which <= 5, "gemm_f32: no kernel %d", which);
   if (M == 0) return 0;
   const bool words = K % 4 == 0 && words_of_16_bytes(a, lda) && words_of_16_bytes(w, ldw);
   const bool skinny_fits = M <= kSkinnyMaxRows && words;
   GB_REQUIRE(which != 2 || skinny_fits, "gemm_f32: the skinny kernel takes at most %d rows of 16-byte words (M=%d K=%d)",
              kSkinnyMaxRows, M, K);
-  if (which == 2 || (which == 0 && skinny_fits)) {
-    if (M <= 1) launch_skinny<1>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 2) launch_skinny<2>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 4) launch_skinny<4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 8) launch_skinny<8>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else launch_skinny<16>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+  if (which == 2 || (which == 0 && skinny_fits && skinny_pays(M, N, K))) {
+    if (N > kNarrow && M <= 1) launch_skinny<1, 16>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+    else if (N > kNarrow && M <= 2) launch_skinny<2, 16>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+    else if (M <= 1) launch_skinny<1, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+    else if (M <= 2) launch_skinny<2, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+    else if (M <= 4) launch_skinny<4, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+    else launch_skinny<8, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
     return launched("gemm_f32 (skinny)");
   }
-  GB_REQUIRE(which != 3 || words, "gemm_f32: the wide kernel takes rows of 16-byte words (K=%d lda=%d ldw=%d)", K, lda, ldw);
+  GB_REQUIRE(which < 3 || words, "gemm_f32: the wide and the sliced kernel take rows of 16-byte words (K=%d lda=%d ldw=%d)", K, lda, ldw);
   const dim3 wide((N + WN - 1) / WN, (M + WM - 1) / WM);
   if (which == 3 || (which == 0 && words && (long long)wide.x * wide.y >= kWideMinTiles)) {
     GB_REQUIRE(wide.y <= 65535, "gemm_f32: M=%d needs more than 65535 row tiles", M);
     hipLaunchKernelGGL(gemm_f32_wide_kernel, wide, dim3(256), 0, stream, a, lda, w, ldw, c, ldc, M, N, K, accumulate);
     return launched("gemm_f32 (wide)");
+  }
+  if (which >= 4 || (which == 0 && words)) {
+    const bool few = (long long)((N + 31) / 32) * ((M + 31) / 32) <= kFewTiles;
+    return which == 4 || (which == 0 && !few) ? launch_sliced<4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream)
+                                              : launch_sliced<8>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
   }
   const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
   GB_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d needs more than 65535 row tiles", M);

@@ -85,7 +85,7 @@ def test_gemm_f32_is_summed_in_one_order_by_both_kernels_and_at_every_number_of_
 @pytest.mark.parametrize("N,K,M", [(331, 100, 200), (130, 260, 129), (2048, 2048, 300), (512, 8192, 65), (96, 4100, 331),
                                    (257, 16, 128), (128, 72, 1)])
 def test_gemm_f32_wide_kernel_gives_the_bits_of_the_tiled_kernel(N, K, M):
-    """The kernel for prompts (128 x 64 of C a workgroup, 8 x 4 cells a thread, two k-steps in LDS) keeps the one
+    """The kernel for prompts (128 x 128 of C a workgroup on the matrix cores, two k-steps in LDS) keeps the one
     summation order: the same bits as the tiled kernel, with and without accumulation, on tiles that hang over
     every edge; and it is refused where rows are no 16-byte words."""
     from glassbox_amd import ops
@@ -105,6 +105,32 @@ def test_gemm_f32_wide_kernel_gives_the_bits_of_the_tiled_kernel(N, K, M):
     if K > 4:
         assert lib.gb_gemm_f32_by(a.data_ptr() + 4, K, w.data_ptr(), K, c0.data_ptr(), N, M, N, K - 4, 0, 3, stream) == 1
         assert "wide" in lib.gb_last_error().decode()
+
+
+@pytest.mark.parametrize("N,K,M", [(33, 64, 31), (32, 68, 33), (65, 260, 64), (31, 1024, 1), (960, 2564, 9), (8, 512, 200)])
+def test_gemm_f32_matrix_core_kernels_round_as_the_tiled_kernel_does(N, K, M):
+    """The wide and the sliced kernel (four and eight waves; fewer slices than waves, one more, a last slice that k cuts) and
+    the product as it is dispatched give the bits of the tiled kernel's chains of fmaf: products that are denormal, huge
+    and cancelling ones, infinities and NaN in a row of each operand."""
+    from glassbox_amd import ops
+    lib = ops._lib("gemm_f32")
+    stream = torch.cuda.current_stream().cuda_stream
+    a, w, c0 = rnd(M, K, seed=21), rnd(N, K, seed=22), rnd(M, N, seed=23)
+    a[0] *= 1e-22
+    w[0] *= 1e-19
+    a[M // 2, K - 1], w[N // 2, 0], w[N - 1, K // 2] = float("inf"), 3e38, float("nan")
+    a, w, c0 = to_dev(a), to_dev(w), to_dev(c0)
+    for accumulate in (0, 1):
+        got = {}
+        for which in (1, 0, 3, 4, 5):
+            c = c0.clone()
+            rc = lib.gb_gemm_f32_by(a.data_ptr(), K, w.data_ptr(), K, c.data_ptr(), N, M, N, K, accumulate, which, stream)
+            assert rc == 0, lib.gb_last_error().decode()
+            got[which] = c.cpu()
+        assert torch.isnan(got[1]).any() and not torch.isnan(got[1]).all()
+        for which in (0, 3, 4, 5):
+            assert torch.equal(torch.isnan(got[which]), torch.isnan(got[1]))
+            assert torch.equal(torch.nan_to_num(got[which], 0.25), torch.nan_to_num(got[1], 0.25)), which
 
 
 def test_gemm_f32_takes_rows_that_are_no_words_of_16_bytes():
