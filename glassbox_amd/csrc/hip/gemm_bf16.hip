@@ -10,8 +10,8 @@
 //    can be its epilogue.  Its workgroups can also divide k (split k: a second pass adds their sums in order).
 //  * stream (65 to 128 rows, the mixed steps of serving): 128 x 32 or 128 x 64 tiles, both operands through deep
 //    rings in LDS, W asked for by a wave of its own.
-//  * ring   (a thousand rows and more, enough 256x256 tiles to fill the chip): 2x4 waves, a wave 4x2 such
-//    tiles; operands go from memory straight into a ring of LDS buffers in k-steps of 32.
+//  * ring   (a thousand rows and more, enough 256x256 tiles to fill the chip): 2x2 waves, a wave 8x8 tiles of
+//    v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
 //  * skinny (M <= 64, decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
 //    rows of W are few); its
 //    waves take interleaved 64-wide k blocks, stream W straight from memory into MFMA operands
@@ -45,7 +45,7 @@ __device__ __forceinline__ bf16x8 zero8() {
 
 // The gated unit of an EPI_SILU_MUL product, with the numbers that a clamped unit changes:
 // g' = min(g, limit), u' = clamp(u, -limit, limit), act = g' sigmoid(alpha g') (u' + plus).  As it stands here it is
-// silu(g) u to the bit.
+// silu(g) u.
 struct Glu {
   float limit = INFINITY;
   float alpha = 1.0f;
@@ -54,7 +54,11 @@ struct Glu {
 __device__ __forceinline__ float gated_unit(float g, float u, const Glu& p) {
   g = fminf(g, p.limit);
   u = fminf(fmaxf(u, -p.limit), p.limit);
-  return g / (1.0f + __expf(-(p.alpha * g))) * (u + p.plus);
+  // the reciprocal by the hardware's approximation, an ulp off at most, in a third of the instructions of a division (an epilogue
+  // of 256 x 128 units: 7.5 us of divisions a tile); of a sixteenth of the sum, so that the reciprocal of a finite one
+  // is a normal number
+  const float d = 1.0f + __expf(-(p.alpha * g));
+  return g * __builtin_amdgcn_rcpf(0.0625f * d) * 0.0625f * (u + p.plus);
 }
 
 // What a product of at most 64 rows may do for the RMS norm that follows it or precedes it.
@@ -404,25 +408,39 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 }
 
 // ------------------------------------------------------------------------- ring
-// Large products (many rows, many 256 x 256 tiles): a workgroup of 2 x 4 waves with a 256 x 256 tile, a wave
-// 4 x 2 tiles of 32 x 32.  The larger tile halves the operand bytes a flop needs, which is what bounds the
-// 128-wide kernel.  Operands go from memory straight into LDS (global_load_lds, 16 bytes a lane: a wave's
-// instruction fills 1 KB of LDS in lane order, so the lane decides which piece of memory lands where), in
-// k-steps of 32 through a ring of RING_STAGES buffers: nothing waits in registers, and a load has
-// RING_STAGES - 1 k-steps to arrive in.  A row of a k-step is 64 bytes = 4 pieces; piece c of row r lies at
-// position c ^ ((r >> 2) & 3), which spreads the 16-byte operand reads of a wave over all banks.
+// Large products (many rows, many 256 x 256 tiles): a workgroup of 2 x 2 waves with a 256 x 256 tile, a wave 8 x 8 tiles of
+// 16 x 16, whose sums fill the accumulation registers (one wave a SIMD).  Operands go from memory straight into LDS
+// (global_load_lds, 16 bytes a lane: a wave's instruction fills 1 KB of LDS in lane order, so the lane decides which
+// piece of memory lands where), in k-steps of 64, so that an instruction brings eight whole lines of 128 bytes.  LDS, all
+// of it, is a ring of five slots of 256 rows by 64 of k: A and W of the k-step that is multiplied, A and W of the next
+// and A of the one after.  A row of a k-step is 128 bytes = 8 pieces; piece c of row r lies at position
+// c ^ ((r >> 1) & 7), which spreads the 16-byte operand reads of 16 neighbouring rows over all banks.
 //
-// The compiler knows nothing of what those loads write: before every LDS read it would wait for all of them.
-// So the operand reads are inline assembly, and the waits are written here by hand:
-//   * lgkmcnt before the MFMAs that use an operand;
-//   * the barrier of k-step s stands between its two MFMA steps.  Before it a wave waits for its last operand
-//     reads of stage s (lgkmcnt) and for its own loads of stage s + 1 (vmcnt: loads retire in order).  After
-//     it, every wave's loads of stage s + 1 have landed, so its operands may be read (they arrive under the
-//     second MFMA step), and every wave is done with stage s, so the loads of k-step s + 1 may overwrite it.
-constexpr int RBK = 32, RING_STAGES = 4;
-constexpr int RGM = 2, RGN = 4, RTM = 4, RTN = 2;          // waves along m, n; 32 x 32 tiles of a wave along m, n
-constexpr int RBM = RGM * RTM * 32, RBN = RGN * RTN * 32;  // 256 x 256
-constexpr int RLA = RBM / 16 / (RGM * RGN), RLW = RBN / 16 / (RGM * RGN), RLPS = RLA + RLW;  // loads of a wave per stage
+// The matrix cores take W as their first operand and A as the second, so that a lane holds four neighbouring columns of a row of
+// C: an epilogue of whole words.
+//
+// The compiler knows nothing of what those loads write, and left to itself it keeps neither the accumulators in place nor
+// this order.  So the operand reads and the MFMAs are inline assembly, issued in the order written here (an operand read or a
+// request to memory between MFMAs costs no cycle of theirs), and the waits are written by hand:
+//   * lgkmcnt before the 64 MFMAs that use the operands (read among the 64 before them);
+//   * the barrier of a k-step stands between its two blocks of 64 MFMAs.  Before it a wave waits for its last operand
+//     reads of the k-step (lgkmcnt) and for its own loads of the next one (vmcnt: loads retire in order).  After it,
+//     every wave's loads of the next k-step have landed, so its operands may be read (they arrive under the second
+//     block), and every wave is done with this k-step's slots, so that W of k-step + 2 may overwrite its A, and A of
+//     k-step + 3 its W (in the next k-step's first block).
+//
+// What bounds it: power and the way from memory.  Multiplying 8,192^3, the chip runs at 1.7 GHz, and all-zero operands take 640 us
+// where random ones take 749; without requests to memory it would take 530.  The kernel before this one (eight waves of 128 x 64,
+// 32 x 32 x 16 MFMAs, k-steps of 32, so that a request brought half lines: twice the requests to the second-level cache) kept
+// the matrix cores busy for 71 % of the cycles.  us, before -> now, same box: 8,192^3 842 -> 749 (1,468 TFLOP/s);
+// 6,151 x 28,672 x 4,096 1,311 -> 1,120; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
+// (8,192^3: 850 where this took 805); tiles dealt to the dies in squares (no gain).
+constexpr int RBK = 64, RING_SLOTS = 5;
+constexpr int RGM = 2, RGN = 2, RT = 8;                  // waves along m, n; 16 x 16 tiles of a wave along m and along n
+constexpr int RBM = RGM * RT * 16, RBN = RGN * RT * 16;  // 256 x 256
+constexpr int RL = RBM / 8 / (RGM * RGN);                // loads of a wave that bring its share of a slot
+static_assert(RBM == RBN, "a slot of the ring holds either operand");
+constexpr int RING_MIN_K = 128, RING_K = 32;             // k is a multiple of 32 (a last k-step may be half of one)
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void glb_void;
 
@@ -445,6 +463,16 @@ __device__ __forceinline__ void lds_wait(bf16x8 (&fa)[NA], bf16x8 (&fb)[NB]) {
 template <int LEFT> __device__ __forceinline__ void vm_wait() {
   static_assert(LEFT >= 0 && LEFT < 64, "the counter has six bits");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | ((LEFT >> 4) << 14));
+}
+
+// four neighbouring columns of a row of C
+template <typename CT> __device__ __forceinline__ void store_c4(CT* c, const f32x4& v);
+template <> __device__ __forceinline__ void store_c4<float>(float* c, const f32x4& v) { *reinterpret_cast<f32x4*>(c) = v; }
+template <> __device__ __forceinline__ void store_c4<bf16>(bf16* c, const f32x4& v) {
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = (bf16)v[r];
+  *reinterpret_cast<bf16x4*>(c) = o;
 }
 
 // GROUPED: as the tiled kernel's (row tiles of 256 rows); a product that divides k writes grp.slice_rows rows a slice.
@@ -477,11 +505,8 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
     c += (size_t)z * (GROUPED ? grp.slice_rows : M) * ldc;
     K = min(k_slice, K - z * k_slice);
   }
-  __shared__ __attribute__((aligned(16))) bf16 As[RING_STAGES][RBM * RBK];
-  __shared__ __attribute__((aligned(16))) bf16 Ws[RING_STAGES][RBN * RBK];
-  constexpr bool SCALES = GROUPED && EPI == EPI_SILU_MUL;
-  __shared__ float in_scale[SCALES ? RBM : 1];   // the rows' factors (read behind the loop's barriers)
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  __shared__ __attribute__((aligned(16))) bf16 ring[RING_SLOTS][RBM * RBK];
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wm = wave / RGN, wn = wave % RGN;
   int m0 = by * RBM;
   const int half = N / 2;  // EPI_SILU_MUL: number of gate rows
@@ -494,197 +519,227 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
     M = tile[2];
     w += (size_t)group * grp.w_stride;
     up_off = grp.up_off;
-    if (SCALES && grp.in_scale && tid < RBM) in_scale[tid] = grp.in_scale[min(m0 + tid, M - 1)];
   }
-  // row of W behind row r of the workgroup's W tile (r = wn * 64 + j * 32 + column); with EPI_SILU_MUL a wave's
-  // first column tile holds gate rows and its second the up rows that belong to them
+  // row of W behind row r of the workgroup's W tile (r = wn * 128 + j * 16 + column); with EPI_SILU_MUL a wave's
+  // even column tiles hold gate rows and the odd ones the up rows that belong to them
   auto w_row = [&](int r) -> int {
     if (EPI == EPI_SILU_MUL) {
-      const int j = (r % (RTN * 32)) / 32;  // column tile of its wave: even ones hold gate rows, odd ones their up rows
-      const int n = bx * (RBN / 2) + (r / (RTN * 32)) * (RTN / 2 * 32) + (j / 2) * 32 + r % 32;
+      const int j = r % (RT * 16) / 16;
+      const int n = bx * (RBN / 2) + r / (RT * 16) * (RT / 2 * 16) + j / 2 * 16 + r % 16;
       return n < half ? (j % 2 ? up_off + n : n) : 0;
     }
     return min(bx * RBN + r, N - 1);
   };
-  // a wave's load instruction moves 16 rows x 4 pieces; rows beyond M or N are read from a row that exists
-  const bf16* asrc[RLA];
-  const bf16* wsrc[RLW];
+  // a wave's load instruction moves 8 rows x 8 pieces; rows beyond M or N are read from a row that exists
+  const bf16* asrc[RL];
+  const bf16* wsrc[RL];
 #pragma unroll
-  for (int t = 0; t < RLA; ++t) {
-    const int row = (wave * RLA + t) * 16 + lane / 4, piece = (lane % 4) ^ ((row >> 2) & 3);
+  for (int t = 0; t < RL; ++t) {
+    const int row = (wave * RL + t) * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
     int arow = min(m0 + row, M - 1);
     if constexpr (GROUPED) {
       if (grp.rows) arow = grp.rows[arow];
     }
     asrc[t] = a + (size_t)arow * lda + piece * 8;
-  }
-#pragma unroll
-  for (int t = 0; t < RLW; ++t) {
-    const int row = (wave * RLW + t) * 16 + lane / 4, piece = (lane % 4) ^ ((row >> 2) & 3);
     wsrc[t] = w + (size_t)w_row(row) * ldw + piece * 8;
   }
-  auto load_a = [&](int t, int stage, int k0) {
-    __builtin_amdgcn_global_load_lds((glb_void*)(asrc[t] + k0), (lds_void*)&As[stage][(wave * RLA + t) * 16 * RBK], 16, 0, 0);
+  auto load_a = [&](int t, int slot, int k0) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(asrc[t] + k0), (lds_void*)&ring[slot][(wave * RL + t) * 8 * RBK], 16, 0, 0);
   };
-  auto load_w = [&](int t, int stage, int k0) {
-    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[t] + k0), (lds_void*)&Ws[stage][(wave * RLW + t) * 16 * RBK], 16, 0, 0);
+  auto load_w = [&](int t, int slot, int k0) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[t] + k0), (lds_void*)&ring[slot][(wave * RL + t) * 8 * RBK], 16, 0, 0);
   };
-  f32x16 acc[RTM][RTN];
+  f32x4 acc[RT][RT];
 #pragma unroll
-  for (int i = 0; i < RTM; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < RTN; ++j)
+    for (int j = 0; j < RT; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-  // operand of MFMA step ks (0, 1): row lane % 32 of a 32-row tile, piece 2 ks + lane / 32
+  // operand of block kh (0, 1): row lane % 16 of a 16-row tile, piece 4 kh + lane / 16
   uint32_t off[2];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) off[ks] = 2 * ((lane % 32) * RBK + (((2 * ks + lane / 32) ^ ((lane >> 2) & 3)) * 8));
-  const uint32_t abase = (uint32_t)(uintptr_t)(lds_void*)&As[0][0] + 2 * wm * RTM * 32 * RBK;
-  const uint32_t wbase = (uint32_t)(uintptr_t)(lds_void*)&Ws[0][0] + 2 * wn * RTN * 32 * RBK;
-  constexpr uint32_t A_STAGE = 2 * RBM * RBK, W_STAGE = 2 * RBN * RBK, TILE = 2 * 32 * RBK;
+  for (int kh = 0; kh < 2; ++kh) off[kh] = 2 * ((lane % 16) * RBK + (((4 * kh + lane / 16) ^ ((lane >> 1) & 7)) * 8));
+  constexpr uint32_t SLOT = 2 * RBM * RBK, TILE = 2 * 16 * RBK;
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&ring[0][0];
+  const uint32_t abase = base + wm * RT * TILE, wbase = base + wn * RT * TILE;
 
-  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 32 that lie beyond the group's end
-  const int live = GROUPED ? min(max((M - m0 - wm * RTM * 32 + 31) / 32, 0), RTM) : RTM;
+  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end
+  const int live = GROUPED ? __builtin_amdgcn_readfirstlane(min(max((M - m0 - wm * RT * 16 + 15) / 16, 0), RT)) : RT;
 
-  const int steps = K / RBK;
-  bf16x8 fa[2][RTM], fw[2][RTN];
-  auto read_operands = [&](int stage, int ks) {
-#pragma unroll
-    for (int i = 0; i < RTM; ++i) fa[ks][i] = lds_read16(abase + stage * A_STAGE + i * TILE + off[ks]);
-#pragma unroll
-    for (int j = 0; j < RTN; ++j) fw[ks][j] = lds_read16(wbase + stage * W_STAGE + j * TILE + off[ks]);
+  // k-steps; where k is an odd number of halves the last one begins 32 earlier, and its first half, already summed, counts
+  // as zeros
+  const int steps = (K + RBK - 1) / RBK;
+  const bool odd = K % RBK != 0;
+  auto k_of = [&](int s) { return min(s * RBK, K - RBK); };
+  bf16x8 fa[2][RT], fw[2][RT];
+  auto read_a = [&](int set, int t, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
   };
-  // the MFMAs of MFMA step ks; with MORE, half of the loads of stage s + RING_STAGES - 1 are requested among them,
-  // one after a row of MFMAs (requests and arithmetic side by side, not in bursts)
-  auto multiply = [&](int ks, auto more, int nstage, int nk0) {
-#pragma unroll
-    for (int i = 0; i < RTM; ++i) {
-      if (!GROUPED || i < live) {
-#pragma unroll
-        for (int j = 0; j < RTN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks][i], fw[ks][j], acc[i][j], 0, 0, 0);
-      }
-      if (decltype(more)::value) {
-        constexpr int SLOTS = 2 * RTM;
-        const int slot = ks * RTM + i;
-#pragma unroll
-        for (int t = 0; t < RLA; ++t)
-          if ((t * SLOTS) / RLPS == slot) load_a(t, nstage, nk0);
-#pragma unroll
-        for (int t = 0; t < RLW; ++t)
-          if (((RLA + t) * SLOTS) / RLPS == slot) load_w(t, nstage, nk0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  auto read_w = [&](int set, int t, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
   };
-  // k-step s.  On entry the operands of its first MFMA step are on their way into registers.  The barrier stands
-  // between the two MFMA steps: by then this wave has read all it needs of stage s, and once every wave has,
-  // stage s + 1 (whose loads were waited for) may be read and the buffer of stage s overwritten (by the loads of
-  // k-step s + 1).  So the first operands of k-step s + 1 arrive under the second MFMA step of k-step s.
-  static_assert(RING_STAGES == 4 && RLPS % 2 == 0, "the wait counts below are written for four stages and an even number of loads a stage");
-  auto step = [&](int s, auto more) {
-    const int stage = s % RING_STAGES, nstage = (s + RING_STAGES - 1) % RING_STAGES, nk0 = (s + RING_STAGES - 1) * RBK;
-    read_operands(stage, 1);
-    lds_wait<RTM + RTN>(fa[0], fw[0]);
-    multiply(0, more, nstage, nk0);
-    lds_wait<0>(fa[1], fw[1]);
-    if (s + 1 < steps) {
-      // loads of this wave that may still be on their way: those of stage s + 2, and the half of stage s + 3 just asked for
-      if (decltype(more)::value)
-        vm_wait<RLPS + RLPS / 2>();
-      else if (s + 2 < steps)
-        vm_wait<RLPS>();
+  // The 64 MFMAs of operand set `set`; among them the reads of the other set from ra and rw, and (with `more`) a slot's
+  // loads from memory: of A among those of set 0, of W among those of set 1.
+  auto block = [&](auto which, uint32_t ra, uint32_t rw, bool more, int slot, int k0) {
+    constexpr int set = decltype(which)::value;
+#pragma unroll
+    for (int at = 0; at < RT * RT; ++at) {
+      const int i = at / RT, j = (i & 1) ? RT - 1 - at % RT : at % RT;
+      if constexpr (GROUPED)
+        asm volatile("s_cmp_le_i32 %3, %4\n\ts_cbranch_scc1 .Lbeyond%=\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n.Lbeyond%=:"
+                     : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]), "s"(live), "n"(i) : "scc");
       else
-        vm_wait<0>();
-      __builtin_amdgcn_s_barrier();
-      read_operands((s + 1) % RING_STAGES, 0);
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
+      if (at % 2 == 0 && at / 2 < RT) read_a(set ^ 1, at / 2, ra);
+      else if (at % 2 == 0 && at / 2 < 2 * RT) read_w(set ^ 1, at / 2 - RT, rw);
+      else if (at % 4 == 1 && at / 4 < RL && more) {
+        if constexpr (set == 1) load_w(at / 4, slot, k0);
+        else load_a(at / 4, slot, k0);
+      }
     }
-    multiply(1, more, nstage, nk0);
   };
-  using Yes = std::true_type;
-  using No = std::false_type;
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
 #pragma unroll
-  for (int s = 0; s < RING_STAGES - 1; ++s)
-    if (s < steps) {
+  for (int t = 0; t < RL; ++t) load_a(t, 0, k_of(0));
 #pragma unroll
-      for (int t = 0; t < RLA; ++t) load_a(t, s, s * RBK);
+  for (int t = 0; t < RL; ++t) load_w(t, 1, k_of(0));
+  if (steps > 1) {
 #pragma unroll
-      for (int t = 0; t < RLW; ++t) load_w(t, s, s * RBK);
-    }
-  if (steps >= 3)
-    vm_wait<2 * RLPS>();
-  else if (steps == 2)
-    vm_wait<RLPS>();
-  else
+    for (int t = 0; t < RL; ++t) load_a(t, 2, k_of(1));
+#pragma unroll
+    for (int t = 0; t < RL; ++t) load_w(t, 3, k_of(1));
+    vm_wait<2 * RL>();
+  } else {
     vm_wait<0>();
+  }
   __builtin_amdgcn_s_barrier();
-  read_operands(0, 0);
-  int s = 0;
-  for (; s + RING_STAGES - 1 < steps; ++s) step(s, Yes{});
-  for (; s < steps; ++s) step(s, No{});  // the last stages are on their way or have landed: nothing more is requested
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    read_a(0, t, abase + off[0]);
+    read_w(0, t, wbase + SLOT + off[0]);
+  }
+  int sa = 0, sw = 1;   // this k-step's slots
+  auto behind = [](int slot, int by) { return slot + by >= RING_SLOTS ? slot + by - RING_SLOTS : slot + by; };
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    const bool more = s + 2 < steps;
+    const int na = behind(sa, 2), nw = behind(sw, 2), k2 = k_of(s + 2);
+    lds_wait<0>(fa[0], fw[0]);
+    if (odd && s + 1 == steps) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) fa[0][t] = fw[0][t] = zero8();
+    }
+    block(First{}, abase + sa * SLOT + off[1], wbase + sw * SLOT + off[1], more, behind(sa, 4), k2);
+    lds_wait<0>(fa[1], fw[1]);
+    if (more) vm_wait<RL>();   // (A of k-step s + 2 may still be on its way)
+    else vm_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    block(Second{}, abase + na * SLOT + off[0], wbase + nw * SLOT + off[0], more, sa, k2);   // (behind the last: read, not used)
+    sa = na, sw = nw;
+  }
+  lds_wait<0>(fa[0], fw[0]);
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results, which the compiler does not know to wait for
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < RT; ++j) asm volatile("" : "+a"(acc[i][j]));
 
-  // accumulator layout of a 32x32 tile: lane holds column lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
-  if (EPI == EPI_SILU_MUL) {
-    const bool scaled = SCALES && grp.in_scale;
+  // A lane holds row lane % 16 of a tile and its columns 4 (lane / 16) .. + 3.
+  constexpr int OUT = EPI == EPI_SILU_MUL ? RT / 2 : RT;   // column tiles of the wave's results
+  const int cols = EPI == EPI_SILU_MUL ? half : N;
+  const int gm0 = m0 + wm * RT * 16, gn0 = bx * (RGN * OUT * 16) + wn * (OUT * 16);
+  auto result = [&](int i, int j, float factor) -> f32x4 {   // of row tile i, column tile j of the results
+    if constexpr (EPI == EPI_SILU_MUL) {
+      f32x4 v;
 #pragma unroll
-    for (int p = 0; p < RTN / 2; ++p) {
-      const int gn = bx * (RBN / 2) + wn * (RTN / 2 * 32) + p * 32 + lane % 32;
-      if (gn >= half) continue;
+      for (int r = 0; r < 4; ++r) v[r] = gated_unit(acc[i][2 * j][r] * factor, acc[i][2 * j + 1][r] * factor, glu);
+      return v;
+    } else {
+      return acc[i][j];
+    }
+  };
+  const bool scaled = GROUPED && EPI == EPI_SILU_MUL && grp.in_scale;
+  if (gn0 + OUT * 16 <= cols && (size_t)ldc * sizeof(CT) % 16 == 0 && (uintptr_t)c % 16 == 0) {   // the same for the whole wave
+    if constexpr (sizeof(CT) == 2) {
+      // As they lie, a store of the wave would write 32 bytes of 16 rows; so bfloat16 results go through LDS (32 KB of the
+      // wave's own: every wave has read its last operands) and out in runs of 128 or 256 bytes (8,192 x 16,384 x 128, a
+      // product that is mostly epilogue: 109 -> 83 us).
+      constexpr int ROW = OUT * 32, PIECES = ROW / 16;   // bytes and 16-byte pieces of a row
+      static_assert(RT * 16 * ROW * RGM * RGN <= (int)sizeof(ring), "the waves' rows fit the ring");
+      char* own = reinterpret_cast<char*>(&ring[0][0]) + wave * (RT * 16 * ROW);
 #pragma unroll
-      for (int i = 0; i < RTM; ++i) {
+      for (int i = 0; i < RT; ++i) {
+        const int row = i * 16 + lane % 16;
+        const float factor = scaled ? grp.in_scale[min(gm0 + row, M - 1)] : 1.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gm = m0 + wm * RTM * 32 + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
-          float g = acc[i][2 * p][r], u = acc[i][2 * p + 1][r];
-          if (SCALES && scaled) {
-            const float s = in_scale[wm * RTM * 32 + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4];
-            g *= s, u *= s;
-          }
-          if (gm < M) c[(size_t)gm * ldc + gn] = (CT)gated_unit(g, u, glu);
+        for (int j = 0; j < OUT; ++j)   // half a piece; piece p of a row lies at position p ^ (row % PIECES)
+          store_c4<CT>(reinterpret_cast<CT*>(own + row * ROW + ((2 * j + lane / 32) ^ (row % PIECES)) * 16 + lane / 16 % 2 * 8), result(i, j, factor));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      constexpr int AT_ONCE = 8, RUN = 64 / PIECES;   // rows a store of the wave covers
+#pragma unroll
+      for (int it = 0; it < RT * 16 / RUN; it += AT_ONCE) {
+        f32x4 v[AT_ONCE];
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+          const int row = (it + u) * RUN + lane / PIECES;
+          v[u] = *reinterpret_cast<const f32x4*>(own + row * ROW + ((lane % PIECES) ^ (row % PIECES)) * 16);
         }
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+          const int row = (it + u) * RUN + lane / PIECES;
+          if (gm0 + row < M) *reinterpret_cast<f32x4*>(c + (size_t)(gm0 + row) * ldc + gn0 + lane % PIECES * 8) = v[u];
+        }
+      }
+    } else {
+      // 64 bytes of 16 rows a store: through LDS and out in runs of 256 they were no faster
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int gm = gm0 + i * 16 + lane % 16;
+        if (gm < M) {
+          CT* to = c + (size_t)gm * ldc + gn0 + 4 * (lane / 16);
+          const float factor = scaled ? grp.in_scale[gm] : 1.f;
+          f32x4 old[OUT];   // a row's old values are all asked for before any is added to
+          if constexpr (EPI == EPI_ACCUMULATE)
+#pragma unroll
+            for (int j = 0; j < OUT; ++j) old[j] = *reinterpret_cast<const f32x4*>(to + j * 16);
+#pragma unroll
+          for (int j = 0; j < OUT; ++j) {
+            f32x4 v = result(i, j, factor);
+            if constexpr (EPI == EPI_ACCUMULATE) v = old[j] + v;
+            store_c4<CT>(to + j * 16, v);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     return;
   }
-  if constexpr (EPI == EPI_ACCUMULATE) {
-    // as in the tiled kernel: inside C, all old values of a tile are read before any is added to
-    if (m0 + (wm + 1) * RTM * 32 <= M && bx * RBN + (wn + 1) * RTN * 32 <= N) {
+  // the last columns of C, or rows of C that are no 16-byte words
 #pragma unroll
-      for (int i = 0; i < RTM; ++i) {
-        CT* base = c + (size_t)(m0 + wm * RTM * 32 + i * 32 + 4 * (lane / 32)) * ldc + bx * RBN + wn * RTN * 32 + lane % 32;
-        float old[RTN][16];
+  for (int i = 0; i < RT; ++i) {
+    const int gm = gm0 + i * 16 + lane % 16;
+    if (gm >= M) continue;
+    const float factor = scaled ? grp.in_scale[gm] : 1.f;
 #pragma unroll
-        for (int j = 0; j < RTN; ++j)
+    for (int j = 0; j < OUT; ++j) {
+      const f32x4 v = result(i, j, factor);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) old[j][r] = (float)base[(size_t)(8 * (r / 4) + r % 4) * ldc + j * 32];
-#pragma unroll
-        for (int j = 0; j < RTN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) base[(size_t)(8 * (r / 4) + r % 4) * ldc + j * 32] = (CT)(old[j][r] + acc[i][j][r]);
+      for (int r = 0; r < 4; ++r) {
+        const int gn = gn0 + j * 16 + 4 * (lane / 16) + r;
+        if (gn < cols) store_c<CT>(c + (size_t)gm * ldc + gn, v[r], EPI == EPI_ACCUMULATE);
       }
-      return;
     }
   }
-#pragma unroll
-  for (int i = 0; i < RTM; ++i)
-#pragma unroll
-    for (int j = 0; j < RTN; ++j) {
-      const int gn = bx * RBN + wn * RTN * 32 + j * 32 + lane % 32;
-      if (gn >= N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int gm = m0 + wm * RTM * 32 + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
-        if (gm < M) store_c<CT>(c + (size_t)gm * ldc + gn, acc[i][j][r], EPI == EPI_ACCUMULATE);
-      }
-    }
 }
 
 // The ring kernel pays where its tiles occupy at least three quarters of the compute units and the loads are whole
 // 16-byte pieces.
 inline bool ring_takes(const void* a, int lda, const void* w, int ldw, int K) {
-  return K % RBK == 0 && K >= RBK * RING_STAGES && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 &&
+  return K % RING_K == 0 && K >= RING_MIN_K && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 &&
          (uintptr_t)w % 16 == 0;
 }
 inline bool ring_pays(int epi, const void* a, int lda, const void* w, int ldw, int M, int N, int K) {
@@ -959,7 +1014,7 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
     if (want >= 2) {
       p.k_slice = ((K + want - 1) / want + TBK - 1) / TBK * TBK;
       p.slices = (K + p.k_slice - 1) / p.k_slice;
-      if (p.slices >= 2 && K - (p.slices - 1) * p.k_slice >= RBK * RING_STAGES) {
+      if (p.slices >= 2 && K - (p.slices - 1) * p.k_slice >= RING_MIN_K) {
         p.floats = (size_t)p.slices * M * N;
         p.ring = true;
         return p;
@@ -1953,8 +2008,8 @@ extern "C" int gb_gemm_bf16_grouped(const void* a, int lda, const int32_t* rows,
   const bf16* A = (const bf16*)a;
   const bf16* W = (const bf16*)w;
   if (tile_rows == 256) {
-    GB_REQUIRE(ring_takes(a, lda, w, ldw, K), "gemm_bf16_grouped: tiles of 256 rows need an inner size of whole 32s, %d and more, not %d", RBK * RING_STAGES, K);
-    const int k_slice = slices == 1 ? 0 : (K / RBK + slices - 1) / slices * RBK;
+    GB_REQUIRE(ring_takes(a, lda, w, ldw, K), "gemm_bf16_grouped: tiles of 256 rows need an inner size of whole 32s, %d and more, not %d", RING_MIN_K, K);
+    const int k_slice = slices == 1 ? 0 : (K / RING_K + slices - 1) / slices * RING_K;
     GB_REQUIRE(slices == 1 || (slices - 1) * (long long)k_slice < K, "gemm_bf16_grouped: %d slices of k=%d leave some without a step", slices, K);
     const int rbn = epilogue == EPI_SILU_MUL ? RBN / 2 : RBN;
     const dim3 rgrid((cols + rbn - 1) / rbn, tiles, slices), rblock(RGM * RGN * 64);

@@ -216,6 +216,47 @@ def test_gemm_bf16_large_products_through_the_lds_ring(M, N, K, mode):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
+@pytest.mark.parametrize("pad,shift", [(8, 0), (2, 0), (6, 2), (0, 4)])
+def test_gemm_bf16_ring_writes_rows_that_are_no_whole_words(mode, pad, shift):
+    """Rows of C that are longer than the product's, or begin between 16-byte words: the ring kernel's results are those
+    it writes into a dense C, to the bit, and nothing beside them is written."""
+    from glassbox_amd import ops
+    M, N, K = 1030, 14000, 160
+    a, w = to_dev(rnd(M, K, seed=11).bfloat16() * 0.25), to_dev(rnd(N, K, seed=12).bfloat16() * 0.25)
+    cols = N // 2 if mode == "silu" else N
+    dtype = torch.bfloat16 if mode in ("bf16", "silu") else torch.float32
+    dense = torch.full((M, cols), 0.5, device=DEV, dtype=dtype)
+    ops.gemm(a, w, dense, accumulate=(mode == "f32+"), silu_mul=(mode == "silu"))
+    room = torch.full((M * (cols + pad) + shift,), 0.5, device=DEV, dtype=dtype)
+    c = room[shift:].view(M, cols + pad)
+    ops.gemm(a, w, c[:, :cols], accumulate=(mode == "f32+"), silu_mul=(mode == "silu"))
+    assert torch.equal(c[:, :cols], dense)
+    assert bool((c[:, cols:] == 0.5).all()) and bool((room[:shift] == 0.5).all())
+
+
+@pytest.mark.parametrize("M", [5, 300, 1600])
+def test_gemm_bf16_gated_unit_at_the_ends_of_its_range(M):
+    """silu(gate) * up where the exponential or its reciprocal leaves the range, in the kernels that form it in their
+    epilogue (few rows, tiles, the ring): the formula's own values in 32-bit, infinities among them."""
+    from glassbox_amd import ops
+    I, K = 4096, 128
+    gates = torch.tensor([-3e38, -1e30, -200.0, -89.0, -88.0, -80.0, -1.0, -0.0, 0.0, 1e-30, 1.0, 80.0, 200.0, 1e30, float("inf"),
+                          float("-inf")]).bfloat16()
+    a, w = torch.zeros(M, K), torch.zeros(2 * I, K)
+    a[:, 0], w[:I, 0], w[I:, 0] = 1.0, gates.float().repeat(I // len(gates) + 1)[:I], 1.0
+    out = torch.full((M, I), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops.gemm(to_dev(a.bfloat16()), to_dev(w.bfloat16()), out, silu_mul=True)
+    g = w[:I, 0].double()
+    want = (g / (1 + torch.exp(-g)))[None, :].expand(M, I)
+    got = out.cpu().double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    fine = torch.isfinite(want)
+    # a bfloat16 result; where exp(-gate) leaves the 32-bit range (2^128, from -gate = 88.8 on) the formula in 32-bit is zero,
+    # which is at most 89 / 2^128 < 2^-121 off
+    assert ((got - want).abs()[fine] <= 2 ** -8 * want.abs()[fine] + 2.0 ** -121).all()
+
+
 @pytest.mark.parametrize("N,K,M,silu", [(96, 64, 1, False), (6144, 2048, 8, False), (352, 176, 5, True),
                                         (16384, 2048, 8, True), (480, 80, 33, False), (512, 4104, 64, True)])
 @pytest.mark.parametrize("gamma_dtype", [torch.float32, torch.bfloat16])
