@@ -1772,17 +1772,24 @@ def tuned_attention_supports(k_pages: torch.Tensor, n_heads: int, window: int, k
 
 
 @functools.lru_cache(maxsize=4096)   # a pure function of the sizes, asked for at every product
-def decode_chunk(n_decode: int, n_kv_heads: int, max_context: int) -> int:
-    """Keys per workgroup of the decode kernel: a multiple of 256.  With a workgroup for every compute
-    unit from requests and kv heads alone (or for half of them, if the context is short), each takes a whole
-    context (and sixteen waves: nothing is left to combine afterwards); otherwise small enough that the launch
-    has about a thousand workgroups."""
+def decode_chunk(n_decode: int, n_kv_heads: int, max_context: int, head_dim: int = 64) -> int:
+    """Keys per workgroup of the decode kernel: a multiple of 256.  A workgroup takes a whole context where there are enough
+    of them for that (sixteen waves each, four where head_dim is above 64 or the context is 512 keys at most), so that
+    nothing is left to combine afterwards; otherwise small enough that the launch has about a thousand workgroups.
+
+    Enough, measured (us, the whole context / chunks and the pass that combines them; requests x kv heads): up to 512 keys
+    always (3 x 1 of 300 keys 5.0 / 6.9; 1 x 8 of 128 dimensions 7.0 / 8.5); up to 1,024 keys 80 (16 x 5 9.6 / 9.8, 32 x 3
+    8.3 / 10.0, but 16 x 3 9.1 / 8.3); up to 2,048 keys 144 (30 x 5 12.4 / 15.8, but 24 x 5 16.1 / 14.9); beyond, 256
+    (53 x 5 of up to 2,300 keys 20.6 / 24.7, but 60 x 3 of 3,000 23.8 / 22.9).  Heads above 64: 192 (24 x 8 of 2,000 keys
+    36.9 / 37.6, but 16 x 8 of 1,000 18 / 15)."""
     groups = max(1, n_decode * n_kv_heads)
-    want_splits = 1 if groups >= 256 else min(256, max(1, 1024 // groups))   # the second pass combines up to 256
-    if groups >= 128 and max_context <= 1024:
-        # sixteen waves take a thousand keys in one round: the second pass would cost more than it saves (measured:
-        # 32 requests of SmolLM2-360M -6 % a step, 4 of SmolLM2-1.7B -2 %; with 64 workgroups or 2,048 keys it is slower)
-        want_splits = 1
+    if max_context <= 512:
+        enough = 1
+    elif head_dim > 64:
+        enough = 192 if max_context <= 2048 else 256
+    else:
+        enough = 80 if max_context <= 1024 else 144 if max_context <= 2048 else 256
+    want_splits = 1 if groups >= enough else min(256, max(1, 1024 // groups))   # the second pass combines up to 256
     chunk = -(-max_context // want_splits)
     return max(256, -(-chunk // 256) * 256)
 
@@ -1802,7 +1809,7 @@ def attention_decode(q: torch.Tensor, out: torch.Tensor, ctx, cache, n_heads: in
     mask_chunk = int(chunk)   # the runs of positions a token sees; ``chunk`` below is the keys a workgroup takes
     if mask_chunk:            # what is divided over workgroups is a run, from the tile of 64 keys that it begins in
         max_context = min(max_context, mask_chunk + 63)
-    chunk = decode_chunk(n_dec, nkv, max_context)
+    chunk = decode_chunk(n_dec, nkv, max_context, hd)
     splits = -(-max_context // chunk)
     ws_acc = ctx.buffer("attn_ws_acc", (n_dec * n_heads * splits * hd,), torch.float32)
     ws_ml = ctx.buffer("attn_ws_ml", (n_dec * n_heads * splits * 2,), torch.float32)

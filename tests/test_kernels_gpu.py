@@ -996,6 +996,29 @@ def test_tuned_decode_with_a_workgroup_per_request_and_kv_head(nh, nkv, hd, wind
     assert not bad, f"requests {bad[:8]} with contexts {[ctx_lens[i] for i in bad[:8]]}: {err[bad[:8]]}"
 
 
+@pytest.mark.parametrize("nh,nkv,hd,lens,bucket", [
+    # one workgroup a context: its tiles of 64 keys in runs of up to five a wave, and in turns beyond 16 x 5 tiles
+    (32, 32, 64, [1, 64, 65, 1024, 1025, 5119, 5120, 5121, 5184, 6143], 6144), (64, 32, 32, [5121, 320, 321, 5, 5056, 7000, 1, 6400], 7168),
+    # up to 512 keys: one workgroup of four waves, also for one request
+    (9, 3, 64, [1], 512), (8, 2, 128, [63, 64, 65, 257, 320, 321, 512], 512),
+    # the sizes around which a whole context and chunks of it change over
+    (10, 5, 64, [1000] * 16, 1024), (10, 5, 64, [999] * 15, 1024), (8, 8, 128, [2000] * 24, 2048), (8, 8, 128, [2000] * 23, 2048)])
+def test_tuned_decode_whatever_a_workgroup_and_a_wave_take(nh, nkv, hd, lens, bucket):
+    """Every way in which a context is dealt to workgroups and waves, against the plain kernel."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    k_pages, v_pages, tables, ks, vs = paged_setup(lens, nkv, hd, 16, seed=hd + nkv, dtype=torch.bfloat16)
+    ctx = BareContext([1] * len(lens), lens, tables, max_context=bucket)
+    q = to_dev((rnd(len(lens), nh * hd, seed=13) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out, twin = (torch.zeros(len(lens), nh * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    ops.attention_decode(q, out, ctx, cache, nh, 1 / math.sqrt(hd), 0)
+    ops.attention_plain(q, twin, ctx.positions, torch.arange(len(lens), dtype=torch.int32, device=DEV), ctx.tables[0], cache.k_pages,
+                        cache.v_pages, nh, 1 / math.sqrt(hd), 0)
+    # softmax weights in bfloat16 (2^-9 of each value's share) and a bfloat16 result on either side
+    assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
+
+
 def test_tuned_decode_finds_one_far_key_in_every_chunk_position():
     """One key is made to stand out: first and last slot of a page, chunk edges, the last position."""
     from types import SimpleNamespace
