@@ -10,7 +10,7 @@
 //    can be its epilogue.  Its workgroups can also divide k (split k: a second pass adds their sums in order).
 //  * stream (65 to 128 rows, the mixed steps of serving): 128 x 32 or 128 x 64 tiles, both operands through deep
 //    rings in LDS, W asked for by a wave of its own.
-//  * ring   (a thousand rows and more, enough 256x256 tiles to fill the chip): 2x2 waves, a wave 8x8 tiles of
+//  * ring   (some hundred rows and more, enough 256x256 tiles to fill the chip): 2x2 waves, a wave 8x8 tiles of
 //    v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
 //  * skinny (M <= 64, decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
 //    rows of W are few); its
@@ -736,8 +736,14 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
   }
 }
 
-// The ring kernel pays where its tiles occupy at least three quarters of the compute units and the loads are whole
-// 16-byte pieces.
+// The ring kernel pays where its tiles occupy at least three quarters of the compute units, from two row tiles on, and the
+// loads are whole 16-byte pieces.  (us, gate/up with SiLU-multiply, before / with it: 320 x 28,672 x 4,096 143 / 111,
+// 512 rows 161 / 116, 1,000 rows 287 / 209; 611 x 16,384 x 2,048 62 / 56, 1,000 rows 85 / 63.)
+constexpr int RING_MIN_ROWS = 257;
+// With slices of k: a thousand rows, or enough rows times k that a slice's sums, which go through memory, are the smaller
+// part (611 x 2,048 x 8,192 47.5 / 44.9, but 512 rows 34.8 / 43.2; 320 x 4,096 x 14,336 78 / 69, 1,000 rows 177 / 118; 611 x
+// 6,144 x 4,096 51 / 55).
+inline bool ring_slices_pay(int M, int K) { return M >= 1024 || (M >= RING_MIN_ROWS && (long long)M * K >= 4500000); }
 inline bool ring_takes(const void* a, int lda, const void* w, int ldw, int K) {
   return K % RING_K == 0 && K >= RING_MIN_K && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 &&
          (uintptr_t)w % 16 == 0;
@@ -746,7 +752,7 @@ inline bool ring_pays(int epi, const void* a, int lda, const void* w, int ldw, i
   if (!ring_takes(a, lda, w, ldw, K)) return false;
   const int cols = epi == EPI_SILU_MUL ? N / 2 : N, bn = epi == EPI_SILU_MUL ? RBN / 2 : RBN;
   const long long tiles = (long long)((M + RBM - 1) / RBM) * ((cols + bn - 1) / bn);
-  return M >= 1024 && tiles >= 192;
+  return M >= RING_MIN_ROWS && tiles >= 192;
 }
 
 template <int EPI, typename CT>
@@ -995,7 +1001,7 @@ int launch_stream(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc
 // and, as a skinny product, makes every workgroup read all of A.  Here the tiled kernel's workgroups
 // also divide k: workgroup (tile, z) sums slice z of k into copy z of a float32 C in a workspace, and a
 // second kernel adds the copies in the order of z and applies the epilogue.  Tiles of 64 or 128 rows; with
-// a thousand rows and more and a long k, the ring kernel's tiles of 256.
+// many rows and a long k (ring_slices_pay), the ring kernel's tiles of 256.
 struct SplitPlan {
   int bm, slices, k_slice;
   size_t floats;  // of workspace
@@ -1005,9 +1011,9 @@ struct SplitPlan {
 
 inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
   SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false};
-  // many rows, a long k and few 256 x 256 tiles (the down projection of a prompt portion): slices of k fill the
+  // many rows, a long k and few 256 x 256 tiles (the down projection of a prompt): slices of k fill the
   // chip with the ring kernel's tiles once; a slice keeps 1,024 of k or more
-  if (M >= 1024 && K >= 4096 && K % TBK == 0 && N % 8 == 0) {
+  if (ring_slices_pay(M, K) && K >= 4096 && K % TBK == 0 && N % 8 == 0) {
     const int tiles = ((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN);
     int want = tiles < 192 ? 256 / tiles : 1;
     if (want > K / 1024) want = K / 1024;
