@@ -1041,8 +1041,8 @@ extern "C" int gb_attention_decode_bf16_static(const void* q, int q_stride, void
 // How the prompt portions of a step are spread over the chip.  A pair of blocks of 32 tokens is the unit of work.
 // A compute unit is what a workgroup's waves share, and what bounds them together: so the pairs are spread over
 // workgroups first (four a workgroup only if that still gives every compute unit one), then a pair's keys over
-// waves (four a workgroup; eight where even single pairs leave compute units idle), and where the pairs are fewer
-// than half the compute units and the contexts long, over `parts` workgroups whose sums a second pass adds.
+// waves (four a workgroup; eight where even single pairs leave compute units idle), and where the pairs are at most
+// half the compute units and the contexts long, over `parts` workgroups whose sums a second pass adds.
 struct PrefillPlan {
   int per_group, split, parts;
 };
@@ -1053,19 +1053,24 @@ inline PrefillPlan prefill_plan(int max_q_len, int max_context, int nh, int n_se
   // has two such workgroups
   const long long four = hd <= 64 ? 2048 : 1024;
   PrefillPlan p{pairs >= four ? 4 : pairs >= 512 ? 2 : 1, 1, 1};
+  const int tiles = (max(max_context, max_q_len) + 63) / 64;
   if (hd <= 64) {
     p.split = 4 / p.per_group;
-    if (p.per_group == 1 && pairs <= 256) p.split = 8;  // (512 tokens of 32 heads at context 4,096: 43 -> 36 us)
+    // (512 tokens of 32 heads at context 4,096: 43 -> 36 us; not where eight waves would have a tile of 64 keys each at most:
+    // five prompts of 61 to 190 tokens, 15 heads, 14.1 -> 11.8)
+    if (p.per_group == 1 && pairs <= 256 && tiles > 4) p.split = 8;
   } else if (p.per_group < 4) {  // one block at a time: waves share keys only in a workgroup of one pair
     p.per_group = 1;
-    p.split = pairs <= 256 ? 8 : 4;  // (512 tokens of 32 heads of 128 at context 4,096: 80 -> 67 us)
+    p.split = pairs <= 256 && tiles > 4 ? 8 : 4;  // (512 tokens of 32 heads of 128 at context 4,096: 80 -> 67 us)
   }
   if (p.per_group == 1 && pairs <= 128) {
-    // a wave keeps at least four tiles of 64 keys; four waves a workgroup then, and up to eight workgroups a pair
-    const int tiles = (max(max_context, max_q_len) + 63) / 64;
-    int parts = (int)(256 / (pairs > 0 ? pairs : 1));
+    // two workgroups of four waves a compute unit, up to eight a pair; a wave keeps at least three tiles of 64 keys, or four
+    // steps of 32 (131 tokens at context 4,031, 32 heads of 64: one workgroup a unit, two a pair, 42.5 us, five a pair 34.6;
+    // 15 heads three, five and seven a pair 34.3, 29.7 and 32.1; 40 tokens at 2,040, 32 heads of 128, 31.2 -> 24.4)
+    const int least = hd <= 64 ? 3 : 2;
+    int parts = (int)(512 / (pairs > 0 ? pairs : 1));
     parts = parts > 8 ? 8 : parts;
-    while (parts > 1 && parts * 4 * 4 > tiles) --parts;
+    while (parts > 1 && parts * 4 * least > tiles) --parts;
     if (parts > 1) p.parts = parts, p.split = 4;
   }
   return p;
