@@ -38,6 +38,7 @@ GB_DEFINE_LAST_ERROR
 namespace {
 
 constexpr int kChunk = 256;
+constexpr int kEarlyPage = 16;   // chunk_alone: values asked for ahead with pages of this size
 constexpr int kMaxOwn = 16;   // (dimension, word) pairs a thread owns at most: head size * page size <= 16,384
 
 struct Running {
@@ -73,7 +74,7 @@ template <typename T>
 __device__ __forceinline__ float key_dot(const float* qs, const T* kb, int slot, int hd, int page_size, int piece) {
   float dot = 0.f;
   if (piece == 8) {
-#pragma unroll 4
+#pragma unroll 8
     for (int d0 = 0; d0 < hd; d0 += 8) {
       const T* kr = kb + ((size_t)(d0 / 8) * page_size + slot) * 8;
       float lo[4], hi[4];
@@ -136,6 +137,20 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   const int tid = threadIdx.x;
   const int ps = sh.page_size, hd = sh.hd;
   const int p = c0 + tid;
+  const int words = ps / 4, pairs = hd * words;
+  // The usual page and a pair a thread: the chunk's words of values are asked for before the scores, sixteen pages at
+  // once, where the loop below asks for four at a time after them (the sums are the same; SmolLM2-360M shapes, a prompt of
+  // 200 and 16 single tokens, 34.9 -> 33.9 ms).
+  const bool early = PER == 1 && ps == kEarlyPage && c0 % kEarlyPage == 0;
+  float ev[kChunk / kEarlyPage][4];
+  if (early && tid < pairs) {
+    const size_t at = (size_t)(tid / words) * ps + 4 * (tid % words);
+#pragma unroll
+    for (int i = 0; i < kChunk / kEarlyPage; ++i) {   // (behind the last page: that page again, not used)
+      const int page = table[min(c0 + i * kEarlyPage, hi) / kEarlyPage];
+      load_words<T>(v_pages + ((size_t)page * sh.nkv + kvh) * hd * ps + at, ev[i]);
+    }
+  }
   float s = -INFINITY;
   if (p <= hi) {
     const int page = table[p / ps];
@@ -146,9 +161,20 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   const float e = p <= hi ? expf(s - m_c) : 0.f;
   es[tid] = e;
   l_c = block_sum(e, scratch);   // also orders the writes of es before the reads below
-  const int words = ps / 4, pairs = hd * words;
 #pragma unroll
   for (int u = 0; u < PER; ++u) a_c[u] = 0.f;
+  if (early) {
+    if (tid < pairs) {
+      const int p0 = c0 + 4 * (tid % words);
+#pragma unroll
+      for (int i = 0; i < kChunk / kEarlyPage; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (p0 + i * kEarlyPage + j <= hi) a_c[0] = fmaf(es[p0 - c0 + i * kEarlyPage + j], ev[i][j], a_c[0]);
+    }
+    __syncthreads();   // es is written again by the next chunk
+    return;
+  }
   const int pg_last = hi / ps;
 #pragma unroll 4
   for (int pg = c0 / ps; pg <= pg_last; ++pg) {
