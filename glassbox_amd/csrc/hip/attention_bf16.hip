@@ -248,9 +248,11 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const float slope = MODE == kSloped && col < G ? ex.slopes[kvh * G + col] : 0.f;
   const int end = min(c0 + chunk, pos + 1);
   // Which of the chunk's tiles of 64 keys are the wave's.  Up to five a wave: a run of neighbouring ones (eight requests of
-  // 4,095 keys, 32 heads of 64, 42.1 us; every sixteenth tile 48.3: the waves then walk the pages side by side, and the heads'
+  // 4,095 keys, 32 heads of 64, 44.7 -> 42.1 us against page lookups by each lane and every sixteenth tile; every sixteenth tile
+  // with the scalar lookups was the slower, 45.6 -> 48.3: the waves then walk the pages side by side, it seems, and the heads'
   // workgroups meet on the same channels of the memory).  Longer contexts, and those whose first keys a window has passed: every
-  // WAVES-th tile, the waves' turns moved on from head to head and request to request (8,000 keys 82.6, in runs 86.8).
+  // WAVES-th tile, the waves' turns moved on from head to head and request to request.  There the scalar lookups lose: 8,000 keys
+  // 80.6 -> 82.6 (in runs 86.8).
   const int tiles = (end - c0 + 63) / 64, each = (tiles + WAVES - 1) / WAVES;
   const bool run = kept == 0 && lo < c0 + 64 && each <= 5;
   const int first = run ? wave * each : (wave + kvh + 5 * s) % WAVES, step = run ? 64 : 64 * WAVES;
