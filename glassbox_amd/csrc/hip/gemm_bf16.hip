@@ -45,7 +45,7 @@ __device__ __forceinline__ bf16x8 zero8() {
 
 // The gated unit of an EPI_SILU_MUL product, with the numbers that a clamped unit changes:
 // g' = min(g, limit), u' = clamp(u, -limit, limit), act = g' sigmoid(alpha g') (u' + plus).  As it stands here it is
-// silu(g) u.
+// silu(g) u to the bit.
 struct Glu {
   float limit = INFINITY;
   float alpha = 1.0f;
@@ -54,11 +54,7 @@ struct Glu {
 __device__ __forceinline__ float gated_unit(float g, float u, const Glu& p) {
   g = fminf(g, p.limit);
   u = fminf(fmaxf(u, -p.limit), p.limit);
-  // the reciprocal by the hardware's approximation, an ulp off at most, in a third of the instructions of a division (an epilogue
-  // of 256 x 128 units: 7.5 us of divisions a tile); of a sixteenth of the sum, so that the reciprocal of a finite one
-  // is a normal number
-  const float d = 1.0f + __expf(-(p.alpha * g));
-  return g * __builtin_amdgcn_rcpf(0.0625f * d) * 0.0625f * (u + p.plus);
+  return g / (1.0f + __expf(-(p.alpha * g))) * (u + p.plus);
 }
 
 // What a product of at most 64 rows may do for the RMS norm that follows it or precedes it.

@@ -259,6 +259,59 @@ def test_gemm_bf16_gated_unit_at_the_ends_of_its_range(M):
     assert ((got - want).abs()[fine] <= 2 ** -8 * want.abs()[fine] + 2.0 ** -121).all()
 
 
+@pytest.mark.parametrize("M", [5, 100, 300, 1600])
+@pytest.mark.parametrize("clamped", [False, True])
+def test_gemm_bf16_gated_unit_of_large_gates(M, clamped):
+    """Gates up to the largest a bfloat16 holds, beside an up of 0 among others: silu(gate) is the gate itself there, and
+    nothing on the way to it may leave the range (few rows, the stream kernel, tiles, the ring; the clamped unit with a
+    limit that no gate reaches)."""
+    from glassbox_amd import ops
+    I, K = 4096, 128
+    gates = torch.tensor([2.0 ** 123, 2.0 ** 124, 2.2e37, 2.0 ** 127, 3e38, -3e38, 1e30]).bfloat16().float()
+    ups = torch.tensor([1.0, 0.0, -1.0, 2.0 ** -60]).float()
+    a, w = torch.zeros(M, K), torch.zeros(2 * I, K)
+    a[:, 0], w[:I, 0], w[I:, 0] = 1.0, gates.repeat(I // len(gates) + 1)[:I], ups.repeat(I // len(ups))
+    out = torch.full((M, I), 7.0, device=DEV, dtype=torch.bfloat16)
+    if clamped:
+        ops.gemm_glu(to_dev(a.bfloat16()), to_dev(w.bfloat16()), out, 3.2e38, 1.0, 0.0)
+    else:
+        ops.gemm(to_dev(a.bfloat16()), to_dev(w.bfloat16()), out, silu_mul=True)
+    g, u = w[:I, 0], w[I:, 0]
+    want = (g / (1 + torch.exp(-g)) * u)[None, :].expand(M, I).double()
+    assert torch.isfinite(want).all()
+    assert ((out.cpu().double() - want).abs() <= 2 ** -8 * want.abs()).all()
+
+
+def test_gemm_bf16_gated_unit_rounds_alike_by_every_route():
+    """One row of float32 results with SiLU-multiply, alone and among so many rows that the stream kernel, the tiles, the
+    ring or slices of k take the product: the sums are exact (one nonzero k), so what the unit makes of them is the same to
+    the bit."""
+    from glassbox_amd import ops
+    I, K = 4096, 128
+    w = torch.zeros(2 * I, K)
+    w[:, 0] = rnd(2 * I, seed=31) * 3
+    w = to_dev(w.bfloat16())
+    rows = {}
+    for M in (1, 5, 40, 100, 200, 300, 1600):
+        a = torch.zeros(M, K, device=DEV, dtype=torch.bfloat16)
+        a[:, 0] = 1.0
+        out = torch.full((M, I), 7.0, device=DEV)
+        ops.gemm(a, w, out, silu_mul=True)
+        rows[M] = out.cpu()
+    wide, K = torch.zeros(2 * I, 4096, device=DEV, dtype=torch.bfloat16), 4096
+    wide[:, 0] = w[:, 0]
+    wide, few = wide[:2048].contiguous(), 1024          # the first gates, and the second thousand of them as their ups
+    for M in (5, 40, 200):
+        a = torch.zeros(M, K, device=DEV, dtype=torch.bfloat16)
+        a[:, 0] = 1.0
+        out = torch.full((M, few), 7.0, device=DEV)
+        ws = torch.empty(max(1, ops.gemm_split_floats(M, 2 * few, K)), device=DEV)
+        ops.gemm(a, wide, out, silu_mul=True, workspace=ws)
+        rows["divided", M] = out.cpu()
+    for key, out in rows.items():
+        assert torch.equal(out, (rows["divided", 5] if isinstance(key, tuple) else rows[1])[:1].expand_as(out)), key
+
+
 @pytest.mark.parametrize("N,K,M,silu", [(96, 64, 1, False), (6144, 2048, 8, False), (352, 176, 5, True),
                                         (16384, 2048, 8, True), (480, 80, 33, False), (512, 4104, 64, True)])
 @pytest.mark.parametrize("gamma_dtype", [torch.float32, torch.bfloat16])
