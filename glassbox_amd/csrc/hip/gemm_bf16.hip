@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "ring_steps.h"
 
 using namespace gb;
 
@@ -431,12 +432,11 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 // the matrix cores busy for 71 % of the cycles.  us, before -> now, same box: 8,192^3 842 -> 749 (1,468 TFLOP/s);
 // 6,151 x 28,672 x 4,096 1,311 -> 1,120; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
 // (8,192^3: 850 where this took 805); tiles dealt to the dies in squares (no gain).
-constexpr int RBK = 64, RING_SLOTS = 5;
+constexpr int RING_SLOTS = 5;   // (RBK, a k-step, and what slices of k may be: ring_steps.h)
 constexpr int RGM = 2, RGN = 2, RT = 8;                  // waves along m, n; 16 x 16 tiles of a wave along m and along n
 constexpr int RBM = RGM * RT * 16, RBN = RGN * RT * 16;  // 256 x 256
 constexpr int RL = RBM / 8 / (RGM * RGN);                // loads of a wave that bring its share of a slot
 static_assert(RBM == RBN, "a slot of the ring holds either operand");
-constexpr int RING_MIN_K = 128, RING_K = 32;             // k is a multiple of 32 (a last k-step may be half of one)
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void glb_void;
 
@@ -477,6 +477,7 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
                                                            CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice, Groups grp,
                                                            Glu glu) {
   int bx = blockIdx.x, by = blockIdx.y;
+  bool head = false;   // GROUPED: the slice begins the row (other products' slices are of 64 and more: it is all one to them)
   if (k_slice > 0) {  // split k: workgroup z of a tile sums its own slice of k into its own copy of C
     int z = blockIdx.z;
     if (GROUPED) {  // the tiles in the map's order, all slices of a tile before the next one's
@@ -484,6 +485,7 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
       bx = id % gx;
       z = id / gx % gz;
       by = id / gx / gz;
+      head = z == 0;
     }
     // The chip deals workgroups round its 8 dies by their number, and each die has a second-level cache of its
     // own.  With the grid as it stands a die would hold one column tile over all row tiles and all slices (8 + 32
@@ -564,11 +566,9 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
   // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end
   const int live = GROUPED ? __builtin_amdgcn_readfirstlane(min(max((M - m0 - wm * RT * 16 + 15) / 16, 0), RT)) : RT;
 
-  // k-steps; where k is an odd number of halves the last one begins 32 earlier, and its first half, already summed, counts
-  // as zeros
-  const int steps = (K + RBK - 1) / RBK;
-  const bool odd = K % RBK != 0;
-  auto k_of = [&](int s) { return min(s * RBK, K - RBK); };
+  // k-steps; the last may hold a half that counts as zeros
+  const int steps = ring_steps(K), dead = ring_dead_half(K, head);
+  auto k_of = [&](int s) { return ring_step_at(s, K, head); };
   bf16x8 fa[2][RT], fw[2][RT];
   auto read_a = [&](int set, int t, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
@@ -624,12 +624,18 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
     const bool more = s + 2 < steps;
     const int na = behind(sa, 2), nw = behind(sw, 2), k2 = k_of(s + 2);
     lds_wait<0>(fa[0], fw[0]);
-    if (odd && s + 1 == steps) {
+    if (dead == 0 && s + 1 == steps) {
 #pragma unroll
       for (int t = 0; t < RT; ++t) fa[0][t] = fw[0][t] = zero8();
     }
     block(First{}, abase + sa * SLOT + off[1], wbase + sw * SLOT + off[1], more, behind(sa, 4), k2);
     lds_wait<0>(fa[1], fw[1]);
+    if constexpr (GROUPED) {
+      if (dead == 1) {   // (the only k-step)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) fa[1][t] = fw[1][t] = zero8();
+      }
+    }
     if (more) vm_wait<RL>();   // (A of k-step s + 2 may still be on its way)
     else vm_wait<0>();
     __builtin_amdgcn_s_barrier();

@@ -460,6 +460,30 @@ def test_grouped_products_by_tiles_of_256_rows_with_k_divided():
     assert (got[256][1][258:258 + 900] - want).abs().max() < 1e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("k, slices", [(128, 4), (160, 5), (160, 2), (224, 4)])
+def test_grouped_products_with_slices_of_32(k, slices):
+    """Slices as short as half a k-step of the ring kernel, at the head of the row and behind it: each slice is the product
+    over its own k, whatever lies beside it (infinities there, which must not even be multiplied by zeros)."""
+    from glassbox_amd import ops
+    torch.manual_seed(k + slices)
+    E, n, out = 2, 300, 256
+    k_slice = -(-(k // 32) // slices) * 32
+    a, w = torch.randn(n, k).bfloat16(), torch.randn(out, E * k).bfloat16()
+    tile_map = torch.tensor([[0, 0, 270], [0, 256, 270], [1, 270, 300]], dtype=torch.int32, device=DEV)
+    want = [torch.cat([a[:270, z:z + k_slice].double() @ w[:, z:min(k, z + k_slice)].double().t(),
+                       a[270:, z:z + k_slice].double() @ w[:, k + z:min(2 * k, k + z + k_slice)].double().t()])
+            for z in range(0, k, k_slice)]
+    for z in range(slices):
+        # all other slices' k infinite, in the rows and in the matrices
+        alone = [t.clone() for t in (a, w.view(out, E, k))]
+        for t in alone:
+            t[..., :z * k_slice] = float("inf")
+            t[..., (z + 1) * k_slice:] = float("inf")
+        parts = torch.full((slices, n, out), 7.0, device=DEV)
+        ops.gemm_grouped(alone[0].to(DEV), None, alone[1].reshape(out, E * k).to(DEV), k, out, tile_map, 256, parts)
+        assert (parts[z].cpu().double() - want[z]).abs().max() < 1e-4 * (1 + want[z].abs().max())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ff, limit", [(12, 0.7), (30, 2.0), (7, 1.5)])
 def test_clamped_units_with_weights(ff, limit, dtype):
