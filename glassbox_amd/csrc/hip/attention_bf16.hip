@@ -248,14 +248,19 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const float slope = MODE == kSloped && col < G ? ex.slopes[kvh * G + col] : 0.f;
   const int end = min(c0 + chunk, pos + 1);
   // Which of the chunk's tiles of 64 keys are the wave's.  Up to five a wave: a run of neighbouring ones (eight requests of
-  // 4,095 keys, 32 heads of 64, 44.7 -> 42.1 us against page lookups by each lane and every sixteenth tile; every sixteenth tile
-  // with the scalar lookups was the slower, 45.6 -> 48.3: the waves then walk the pages side by side, it seems, and the heads'
-  // workgroups meet on the same channels of the memory).  Longer contexts, and those whose first keys a window has passed: every
-  // WAVES-th tile, the waves' turns moved on from head to head and request to request.  There the scalar lookups lose: 8,000 keys
-  // 80.6 -> 82.6 (in runs 86.8).
+  // 4,095 keys in neighbouring pages, 32 heads of 64, 44.7 -> 42.4 us against page lookups by each lane and every sixteenth
+  // tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile, from the wave's own number on,
+  // so that the order in which a request is summed depends on nothing but sizes (turns that began elsewhere in every row and
+  // head were as fast: 24 layers of eight requests of 5,600 and 7,200 keys 2,503 and 2,867 us a step, so 2,477 and 2,920).
+  // Runs of any length, in the same pages: 5,600 keys 58.0 -> 59.3, 6,500 66.1 -> 68.3, 8,000 81.7 -> 83.0, but 6,000
+  // 63.4 -> 62.3; heads of 128 (four waves) 24 requests of 1,700 31.5 -> 32.0, 32 of 3,000 (scattered) 63.2 either way.
+  // Against the lookups by each lane the scalar ones lose in turns where every unit has one workgroup and all are of one length
+  // (eight requests of 5,600, 6,500 and 8,000 keys 56.3, 65.4 and 77.9 us, here 58.0, 66.1 and 81.7), and win where lengths
+  // differ, which a launch does not know (eight of a quarter to all of 5,600, 6,500 and 8,000 keys 47.0, 53.0 and 63.8, here
+  // 43.4, 49.9 and 62.2; nine of 7,000 111.7 -> 108.2).
   const int tiles = (end - c0 + 63) / 64, each = (tiles + WAVES - 1) / WAVES;
   const bool run = kept == 0 && lo < c0 + 64 && each <= 5;
-  const int first = run ? wave * each : (wave + kvh + 5 * s) % WAVES, step = run ? 64 : 64 * WAVES;
+  const int first = run ? wave * each : wave, step = run ? 64 : 64 * WAVES;
   const int stop = run ? min(c0 + (first + each) * 64, end) : end;
   Pages next = pages_of(table, P, c0 + first * 64, lo, pos);
   for (int kb = c0 + first * 64; kb < stop; kb += step) {

@@ -1074,6 +1074,28 @@ def test_tuned_decode_whatever_a_workgroup_and_a_wave_take(nh, nkv, hd, lens, bu
     assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
 
 
+@pytest.mark.parametrize("nkv,G,hd,n,length,bucket,window,keep", [
+    # a whole context a workgroup: more tiles a wave than a run holds, sixteen and four waves; runs; a window; kept first keys
+    (32, 1, 64, 8, 5500, 6144, 0, 0), (8, 4, 128, 24, 1500, 2048, 0, 0), (32, 1, 64, 8, 4000, 4096, 0, 0),
+    (32, 1, 64, 8, 3001, 3072, 1024, 0), (32, 1, 64, 8, 3001, 3072, 1024, 64), (8, 4, 128, 24, 1999, 2048, 300, 70),
+    # chunks of a context
+    (4, 2, 64, 3, 9000, 9216, 0, 0)])
+def test_tuned_decode_gives_a_request_the_same_bits_in_every_row_and_head(nkv, G, hd, n, length, bucket, window, keep):
+    """One request in every row of a step, its keys, values and queries alike in every head: the order in which a context is
+    summed depends on sizes alone, so all heads of all rows are the same to the bit."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    k_pages, v_pages, tables, _, _ = paged_setup([length], 1, hd, 16, seed=hd + nkv, dtype=torch.bfloat16)
+    k_pages, v_pages = (t.expand(-1, nkv, -1, -1).contiguous() for t in (k_pages, v_pages))
+    ctx = BareContext([1] * n, [length] * n, tables.expand(n, -1), max_context=bucket)
+    q = to_dev((rnd(1, hd, seed=13) * 0.7).bfloat16().expand(n, nkv * G, hd).reshape(n, -1))
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out = torch.zeros(n, nkv * G * hd, device=DEV, dtype=torch.float32)
+    ops.attention_decode(q, out, ctx, cache, nkv * G, 1 / math.sqrt(hd), window, keep)
+    heads = out.view(n * nkv * G, hd)
+    assert bool(heads[0].any()) and torch.equal(heads, heads[:1].expand_as(heads))
+
+
 def test_tuned_decode_finds_one_far_key_in_every_chunk_position():
     """One key is made to stand out: first and last slot of a page, chunk edges, the last position."""
     from types import SimpleNamespace
