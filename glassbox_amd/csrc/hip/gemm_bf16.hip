@@ -563,7 +563,10 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
   const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&ring[0][0];
   const uint32_t abase = base + wm * RT * TILE, wbase = base + wn * RT * TILE;
 
-  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end
+  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end,
+  // in its second half, between whose MFMAs nothing else stands: a branch each eight of them, which their time hides.  (us of
+  // two experts of eight a token, 2,048 tokens, 4,096 units of 2,048, gate/up and down, traced: 159 and 113; a branch before
+  // every MFMA 226 and 152; the kernel with k-steps of 32 175 and 112.)
   const int live = GROUPED ? __builtin_amdgcn_readfirstlane(min(max((M - m0 - wm * RT * 16 + 15) / 16, 0), RT)) : RT;
 
   // k-steps; the last may hold a half that counts as zeros
@@ -576,6 +579,8 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
   auto read_w = [&](int set, int t, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
   };
+  constexpr int LIVE_FROM = RT / 2;
+  static_assert(RT == 8 && 2 * RT <= RT * LIVE_FROM / 2 && 4 * RL <= RT * LIVE_FROM, "the reads and the loads stand among the first half's MFMAs");
   // The 64 MFMAs of operand set `set`; among them the reads of the other set from ra and rw, and (with `more`) a slot's
   // loads from memory: of A among those of set 0, of W among those of set 1.
   auto block = [&](auto which, uint32_t ra, uint32_t rw, bool more, int slot, int k0) {
@@ -583,11 +588,23 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
 #pragma unroll
     for (int at = 0; at < RT * RT; ++at) {
       const int i = at / RT, j = (i & 1) ? RT - 1 - at % RT : at % RT;
-      if constexpr (GROUPED)
-        asm volatile("s_cmp_le_i32 %3, %4\n\ts_cbranch_scc1 .Lbeyond%=\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n.Lbeyond%=:"
-                     : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]), "s"(live), "n"(i) : "scc");
-      else
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
+      if constexpr (GROUPED) {
+        if (i >= LIVE_FROM) {
+          if (at % RT == 0)
+            asm volatile(
+                "s_cmp_le_i32 %17, %18\n\ts_cbranch_scc1 .Lbeyond%=\n\t"
+                "v_mfma_f32_16x16x32_bf16 %0, %8, %16, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %9, %16, %1\n\t"
+                "v_mfma_f32_16x16x32_bf16 %2, %10, %16, %2\n\tv_mfma_f32_16x16x32_bf16 %3, %11, %16, %3\n\t"
+                "v_mfma_f32_16x16x32_bf16 %4, %12, %16, %4\n\tv_mfma_f32_16x16x32_bf16 %5, %13, %16, %5\n\t"
+                "v_mfma_f32_16x16x32_bf16 %6, %14, %16, %6\n\tv_mfma_f32_16x16x32_bf16 %7, %15, %16, %7\n.Lbeyond%=:"
+                : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]),
+                  "+a"(acc[i][6]), "+a"(acc[i][7])
+                : "v"(fw[set][0]), "v"(fw[set][1]), "v"(fw[set][2]), "v"(fw[set][3]), "v"(fw[set][4]), "v"(fw[set][5]),
+                  "v"(fw[set][6]), "v"(fw[set][7]), "v"(fa[set][i]), "s"(live), "n"(i) : "scc");
+          continue;
+        }
+      }
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
       if (at % 2 == 0 && at / 2 < RT) read_a(set ^ 1, at / 2, ra);
       else if (at % 2 == 0 && at / 2 < 2 * RT) read_w(set ^ 1, at / 2 - RT, rw);
       else if (at % 4 == 1 && at / 4 < RL && more) {
