@@ -17,9 +17,10 @@
 // scheme on the 32x32x16 instruction (described at its kernel).
 //
 // Decoding splits a request's context into chunks of a multiple of 256 keys, one workgroup per
-// (chunk, kv head, request), four waves taking 64 keys each in turn; partial results are merged
-// in a fixed order (waves in LDS, chunks by a second kernel), so the result is the same on every
-// run.  crates/glassbox-core/src/model.rs:285-312 is the formula.
+// (chunk, kv head, request), whose waves (sixteen where one workgroup takes a whole context of more
+// than 512 keys and the head size allows, else four) take runs of up to five neighbouring tiles of 64
+// keys, or tiles in turn; partial results are merged in a fixed order (waves in LDS, chunks by a
+// second kernel), so the result is the same on every run and in every row of a step.  crates/glassbox-core/src/model.rs:285-312 is the formula.
 #include "attention_bf16.h"
 #include <type_traits>
 
@@ -207,7 +208,7 @@ __device__ __forceinline__ void store_out4(float* p, const f32x4& v) { *reinterp
 
 // ----------------------------------------------------------------------------- decode
 // grid (chunks, kv heads, requests); request s is row s of q and out, at position positions[s].
-// WAVES waves take 64 keys each in turn; dynamic LDS holds their partial results for the merge:
+// WAVES waves share a chunk's tiles of 64 keys (how, is said below); dynamic LDS holds their partial results for the merge:
 // WAVES * (32 + HD * G) floats, G the query heads per kv head.
 template <int HD, int WAVES, typename OT, int MODE = kPlainScores>
 __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restrict__ q, int q_stride, OT* __restrict__ out,
@@ -249,18 +250,21 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const int end = min(c0 + chunk, pos + 1);
   // Which of the chunk's tiles of 64 keys are the wave's.  Up to five a wave: a run of neighbouring ones (eight requests of
   // 4,095 keys in neighbouring pages, 32 heads of 64, 44.7 -> 42.4 us against page lookups by each lane and every sixteenth
-  // tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile, from the wave's own number on,
-  // so that the order in which a request is summed depends on nothing but sizes (turns that began elsewhere in every row and
-  // head were as fast: 24 layers of eight requests of 5,600 and 7,200 keys 2,503 and 2,867 us a step, so 2,477 and 2,920).
-  // Runs of any length, in the same pages: 5,600 keys 58.0 -> 59.3, 6,500 66.1 -> 68.3, 8,000 81.7 -> 83.0, but 6,000
-  // 63.4 -> 62.3; heads of 128 (four waves) 24 requests of 1,700 31.5 -> 32.0, 32 of 3,000 (scattered) 63.2 either way.
+  // tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile,
+  // and which wave begins where moves on from head to head and request to request (steps of 24 such layers, eight requests
+  // of 7,200 keys 2,865 us, where every wave begins at its own number 2,920; but of 5,600 2,502 and 2,477).  The results of the
+  // tiles from the first one on stand first in the merge, whichever wave had them, so that the order in which a request
+  // is summed depends on nothing but sizes.
+  // Runs of any length instead, in neighbouring pages: 5,600 keys 58.9 -> 59.3, 6,500 67.4 -> 68.3, 8,000 80.6 -> 83.0, 6,000
+  // 62.2 -> 62.3; heads of 128 (four waves) 24 requests of 1,700 31.8 -> 32.0, 32 of 3,000 (scattered) 63.3 -> 63.2.
   // Against the lookups by each lane the scalar ones lose in turns where every unit has one workgroup and all are of one length
-  // (eight requests of 5,600, 6,500 and 8,000 keys 56.3, 65.4 and 77.9 us, here 58.0, 66.1 and 81.7), and win where lengths
+  // (eight requests of 5,600, 6,500 and 8,000 keys 56.3, 65.4 and 77.9 us, here 58.9, 67.4 and 80.6), and win where lengths
   // differ, which a launch does not know (eight of a quarter to all of 5,600, 6,500 and 8,000 keys 47.0, 53.0 and 63.8, here
-  // 43.4, 49.9 and 62.2; nine of 7,000 111.7 -> 108.2).
+  // 45.3, 51.8 and 62.1; nine of 7,000 111.7, here 107.8).
   const int tiles = (end - c0 + 63) / 64, each = (tiles + WAVES - 1) / WAVES;
   const bool run = kept == 0 && lo < c0 + 64 && each <= 5;
-  const int first = run ? wave * each : wave, step = run ? 64 : 64 * WAVES;
+  const int place = run ? wave : (wave + kvh + 5 * s) % WAVES;   // where the wave's results stand in the merge
+  const int first = run ? wave * each : place, step = run ? 64 : 64 * WAVES;
   const int stop = run ? min(c0 + (first + each) * 64, end) : end;
   Pages next = pages_of(table, P, c0 + first * 64, lo, pos);
   for (int kb = c0 + first * 64; kb < stop; kb += step) {
@@ -274,17 +278,17 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   st.l += __shfl_xor(st.l, 16, kWave);
   st.l += __shfl_xor(st.l, 32, kWave);
   if (lane < 16) {
-    sm_m[wave * 16 + col] = st.m;
-    sm_l[wave * 16 + col] = st.l;
+    sm_m[place * 16 + col] = st.m;
+    sm_l[place * 16 + col] = st.l;
   }
   if (col < G) {
 #pragma unroll
     for (int b = 0; b < DB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sm_acc[((size_t)wave * HD + 16 * b + 4 * (lane >> 4) + r) * G + col] = st.acc[b][r];
+      for (int r = 0; r < 4; ++r) sm_acc[((size_t)place * HD + 16 * b + 4 * (lane >> 4) + r) * G + col] = st.acc[b][r];
   }
   __syncthreads();
-  // the waves' partial results, combined in wave order
+  // the waves' partial results, combined in the order of their first tiles
   for (int cell = tid; cell < HD * G; cell += WAVES * 64) {
     const int d = cell / G, cc = cell % G;
     float M = sm_m[cc];
