@@ -18,7 +18,7 @@
 //  * sliced (everything between): a 32 x 32 tile a workgroup, whose waves take slices of k in turn, so that a product of
 //    few tiles walks k in a quarter or an eighth of the steps (200 x 960 x 2,560: 458 us in the tiled kernel's 60
 //    workgroups, 24 here; 64 x 2,048 x 8,192: 565 in the skinny kernel, 65 here).
-//  * skinny (a few rows of 16 bytes: a decode step): a workgroup owns 4 or 16 rows of W and every lane one (slice, row)
+//  * skinny (a few rows of 16 bytes: a decode step): a workgroup owns 4, 8 or 16 rows of W and every lane one (slice, row)
 //    pair: all of a workgroup's weights (64 KB) are on their way at once, a lane runs the chain for each row of A, and the
 //    slices' sums meet in LDS, where one thread a cell adds them in order (1 x 960 x 2,560: 10.3 -> 5.5 us with whole lines
 //    through LDS and 4 rows of W a workgroup instead of 8; 1 x 49,152 x 960 64 -> 41 with 16).
@@ -311,6 +311,9 @@ int launch_sliced(const float* a, int lda, const float* w, int ldw, float* c, in
 // The wide kernel from so many of its tiles on: with fewer, units are idle while a tile walks all of k (us, wide / sliced:
 // 160 tiles, 400 x 5,120 x 960, 88 / 71; 200 tiles, 600 rows, 89 / 92; 256 tiles, 2,048 x 2,048 x 8,192, 711 / 912).
 constexpr int kWideMinTiles = 192;
+// And from so many rows on: a single row tile of 128 rows that is half empty takes as long as a full one (49,152 x 2,048 at 3,
+// 33 and 64 rows 306, 308 and 310 / sliced 107, 204 and 210; at 65 and 97 rows 309 and 310 / 309 and 409).
+constexpr int kWideMinRows = 65;
 // Up to so many tiles a unit has one workgroup of the sliced kernel at most: eight waves then walk k in half the rounds
 // (200 x 960 x 2,560 29.7 -> 23.6 us).  With more, two workgroups of four waves share a unit, one's loads on their way
 // under the other's products (2,048 x 960 x 960 69.7 -> 64.0).
@@ -423,13 +426,18 @@ void launch_skinny(const float* a, int lda, const float* w, int ldw, float* c, i
 }
 constexpr int kSkinnyMaxRows = 64;
 // Where the skinny kernel is the faster one (us, skinny / sliced, replayed from a graph over weights that no cache holds):
-// up to 4 rows of narrow products (960 x 960 at 1 and 4 rows 3.8 and 8.1 / 9.4, 2,048 x 8,192 17 and 29 / 63), up to 8
-// where k is long (2,048 x 8,192 at 8 rows 48 / 63, but 960 x 960 12.9 / 9.4); wide products read W at the memory's pace
-// with 16 rows a workgroup, and the sums of more than two rows of A then take longer than the matrix cores
-// (49,152 x 960 at 1, 2 and 4 rows 41, 50 and 67 / 53; with 4 rows of W a workgroup 67, 106 and 167).
-constexpr int kNarrow = 4096, kLongK = 2048;
+// up to 4 rows of narrow products (960 x 960 at 1 and 4 rows 4.2 and 8.5 / 9.8, 2,048 x 8,192 17 and 29 / 63), up to 6 where k
+// is long (576 x 1,536 10.4 and 11.5 at 5 and 6 rows / 13.5, but 960 x 960 10.3 / 9.9), up to 8 where it is longer and the
+// workgroups own 4 rows (2,048 x 8,192 48 / 64, 960 x 2,560 20.0 / 21.1, but 3,072 x 2,048 20.6 / 18.6); wide products
+// read W at the memory's pace with 16 rows a workgroup, and the sums of more than two rows of A then take longer than the
+// matrix cores (49,152 x 960 at 1, 2 and 4 rows 42, 50 and 68 / 54).
+// Rows of W a workgroup: the fewest that leave a unit no more than two workgroups, which is what its LDS holds (one row of A,
+// 4 / 8 / 16: 960 x 2,560 5.5 / 6.9 / 9.1, 2,304 x 576 6.3 / 4.9 / 4.7, 4,096 x 4,096 17.9 / 16.8 / 21.9, 5,120 x 960 10.5 / 9.2 /
+// 8.3; four rows of A, 3,072 x 576 14.8 / 8.9 / 9.0).
+constexpr int kTwoAUnit = 512, kNarrow = 8 * kTwoAUnit, kLongK = 1280, kLongerK = 2048;
 inline bool skinny_pays(int M, int N, int K) {
-  return N <= kNarrow ? M <= 4 || (M <= 8 && K >= kLongK) : M <= 2;
+  if (N > kNarrow) return M <= 2;
+  return M <= 4 || (M <= 6 && K >= kLongK) || (M <= 8 && K >= kLongerK && N <= 4 * kTwoAUnit);
 }
 
 inline bool words_of_16_bytes(const void* p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0; }
@@ -450,17 +458,26 @@ extern "C" int gb_gemm_f32_by(const float* a, int lda, const float* w, int ldw, 
   GB_REQUIRE(which != 2 || skinny_fits, "gemm_f32: the skinny kernel takes at most %d rows of 16-byte words (M=%d K=%d)",
              kSkinnyMaxRows, M, K);
   if (which == 2 || (which == 0 && skinny_fits && skinny_pays(M, N, K))) {
-    if (N > kNarrow && M <= 1) launch_skinny<1, 16>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (N > kNarrow && M <= 2) launch_skinny<2, 16>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 1) launch_skinny<1, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 2) launch_skinny<2, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else if (M <= 4) launch_skinny<4, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
-    else launch_skinny<8, 4>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream);
+#define GB_SKINNY(MT, R) launch_skinny<MT, R>(a, lda, w, ldw, c, ldc, M, N, K, accumulate, stream)
+    if (N > kNarrow && M <= 1) GB_SKINNY(1, 16);
+    else if (N > kNarrow && M <= 2) GB_SKINNY(2, 16);
+    else if (N > 4 * kTwoAUnit) {
+      if (M <= 1) GB_SKINNY(1, 8);
+      else if (M <= 2) GB_SKINNY(2, 8);
+      else if (M <= 4) GB_SKINNY(4, 8);
+      else GB_SKINNY(8, 8);
+    } else {
+      if (M <= 1) GB_SKINNY(1, 4);
+      else if (M <= 2) GB_SKINNY(2, 4);
+      else if (M <= 4) GB_SKINNY(4, 4);
+      else GB_SKINNY(8, 4);
+    }
+#undef GB_SKINNY
     return launched("gemm_f32 (skinny)");
   }
   GB_REQUIRE(which < 3 || words, "gemm_f32: the wide and the sliced kernel take rows of 16-byte words (K=%d lda=%d ldw=%d)", K, lda, ldw);
   const dim3 wide((N + WN - 1) / WN, (M + WM - 1) / WM);
-  if (which == 3 || (which == 0 && words && (long long)wide.x * wide.y >= kWideMinTiles)) {
+  if (which == 3 || (which == 0 && words && M >= kWideMinRows && (long long)wide.x * wide.y >= kWideMinTiles)) {
     GB_REQUIRE(wide.y <= 65535, "gemm_f32: M=%d needs more than 65535 row tiles", M);
     hipLaunchKernelGGL(gemm_f32_wide_kernel, wide, dim3(256), 0, stream, a, lda, w, ldw, c, ldc, M, N, K, accumulate);
     return launched("gemm_f32 (wide)");

@@ -107,7 +107,11 @@ def test_gemm_f32_wide_kernel_gives_the_bits_of_the_tiled_kernel(N, K, M):
         assert "wide" in lib.gb_last_error().decode()
 
 
-@pytest.mark.parametrize("N,K,M", [(33, 64, 31), (32, 68, 33), (65, 260, 64), (31, 1024, 1), (960, 2564, 9), (8, 512, 200)])
+@pytest.mark.parametrize("N,K,M", [(33, 64, 31), (32, 68, 33), (65, 260, 64), (31, 1024, 1), (960, 2564, 9), (8, 512, 200),
+                                   # as dispatched: 8 and 16 rows of W a workgroup, and few rows by so many of W that the wide
+                                   # kernel's tiles would do, on either side of where it begins
+                                   (3077, 580, 1), (3077, 580, 2), (3077, 580, 4), (3077, 1284, 6), (4105, 260, 2), (24600, 68, 64),
+                                   (24600, 68, 65)])
 def test_gemm_f32_matrix_core_kernels_round_as_the_tiled_kernel_does(N, K, M):
     """The wide and the sliced kernel (four and eight waves; fewer slices than waves, one more, a last slice that k cuts) and
     the product as it is dispatched give the bits of the tiled kernel's chains of fmaf: products that are denormal, huge
