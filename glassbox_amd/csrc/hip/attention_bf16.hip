@@ -248,13 +248,16 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const int col_lo = col < G ? lo : 1, col_hi = col < G ? pos : 0;
   const float slope = MODE == kSloped && col < G ? ex.slopes[kvh * G + col] : 0.f;
   const int end = min(c0 + chunk, pos + 1);
-  // Which of the chunk's tiles of 64 keys are the wave's.  Up to five a wave: a run of neighbouring ones (eight requests of
-  // 4,095 keys in neighbouring pages, 32 heads of 64, 44.7 -> 42.4 us against page lookups by each lane and every sixteenth
+  // Which of the chunk's tiles of 64 keys are the wave's.  Up to five for each of sixteen waves, or of four with heads above 64: a
+  // run of neighbouring ones (eight requests of 4,095 keys in neighbouring pages, 32 heads of 64, 44.7 -> 42.4 us against page
+  // lookups by each lane and every sixteenth
   // tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile,
   // and which wave begins where moves on from head to head and request to request (steps of 24 such layers, eight requests
   // of 7,200 keys 2,865 us, where every wave begins at its own number 2,920; but of 5,600 2,502 and 2,477).  The results of the
   // tiles from the first one on stand first in the merge, whichever wave had them, so that the order in which a request
   // is summed depends on nothing but sizes.
+  // Four waves of heads up to 64 take tiles in turn at any length: in runs, neighbouring pages, 32 requests of 512 keys, 32 heads,
+  // 25.1 -> 29.6 us (a step 2,050 -> 2,183), two of 8,000 26.8 -> 29.9 (1,644 -> 1,690), four of 4,000 a step 1,656 -> 1,700.
   // Runs of any length instead, in neighbouring pages: 5,600 keys 58.9 -> 59.3, 6,500 67.4 -> 68.3, 8,000 80.6 -> 83.0, 6,000
   // 62.2 -> 62.3; heads of 128 (four waves) 24 requests of 1,700 31.8 -> 32.0, 32 of 3,000 (scattered) 63.3 -> 63.2.
   // Against the lookups by each lane the scalar ones lose in turns where every unit has one workgroup and all are of one length
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   // differ, which a launch does not know (eight of a quarter to all of 5,600, 6,500 and 8,000 keys 47.0, 53.0 and 63.8, here
   // 45.3, 51.8 and 62.1; nine of 7,000 111.7, here 107.8).
   const int tiles = (end - c0 + 63) / 64, each = (tiles + WAVES - 1) / WAVES;
-  const bool run = kept == 0 && lo < c0 + 64 && each <= 5;
+  const bool run = (WAVES == 16 || HD > 64) && kept == 0 && lo < c0 + 64 && each <= 5;
   const int place = run ? wave : (wave + kvh + 5 * s) % WAVES;   // where the wave's results stand in the merge
   const int first = run ? wave * each : place, step = run ? 64 : 64 * WAVES;
   const int stop = run ? min(c0 + (first + each) * 64, end) : end;
