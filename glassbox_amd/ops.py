@@ -1780,13 +1780,14 @@ def decode_chunk(n_decode: int, n_kv_heads: int, max_context: int, head_dim: int
     Enough, measured (us, the whole context / chunks and the pass that combines them; requests x kv heads): up to 512 keys
     always (3 x 1 of 300 keys 5.0 / 6.9; 1 x 8 of 128 dimensions 7.0 / 8.5); up to 1,024 keys 80 (16 x 5 9.6 / 9.8, 32 x 3
     8.3 / 10.0, but 16 x 3 9.1 / 8.3); up to 2,048 keys 144 (30 x 5 12.4 / 15.8, but 24 x 5 16.1 / 14.9); beyond, 256
-    (53 x 5 of up to 2,300 keys 20.6 / 24.7, but 60 x 3 of 3,000 23.8 / 22.9).  Heads above 64: 192 (24 x 8 of 2,000 keys
-    36.9 / 37.6, but 16 x 8 of 1,000 18 / 15)."""
+    (53 x 5 of up to 2,300 keys 20.6 / 24.7, but 60 x 3 of 3,000 23.8 / 22.9).  Heads above 64: up
+    to 1,024 keys 144 (20 x 8 of 700 16.4 / 20.8, of 1,000 20.9 / 22.8, but 16 x 8 of 1,000 20.2 / 18.5); up to 2,048 192 (24 x
+    8 of 2,000 36.9 / 37.6); beyond, 256."""
     groups = max(1, n_decode * n_kv_heads)
     if max_context <= 512:
         enough = 1
     elif head_dim > 64:
-        enough = 192 if max_context <= 2048 else 256
+        enough = 144 if max_context <= 1024 else 192 if max_context <= 2048 else 256
     else:
         enough = 80 if max_context <= 1024 else 144 if max_context <= 2048 else 256
     want_splits = 1 if groups >= enough else min(256, max(1, 1024 // groups))   # the second pass combines up to 256
