@@ -1085,6 +1085,10 @@ inline PrefillPlan prefill_plan(int max_q_len, int max_context, int nh, int n_se
     int parts = (int)(512 / (pairs > 0 ? pairs : 1));
     parts = parts > 8 ? 8 : parts;
     while (parts > 1 && parts * 4 * least > tiles) --parts;
+    // not a few workgroups more than units, which some units would have two of (us, parts as they came / one a unit: 36 pairs at
+    // 8,200 keys 8 / 7, 44.0 / 38.6; 60 at 4,200 5 / 4, 35.1 / 32.1; 64 at 4,100 5 / 4, 33.9 / 32.6; from 330 on it is even or
+    // better: 45 at 8,100 8 / 5, 40.4 / 43.4, and 8,300 45.5 / 44.1, 75 at 4,300 5 / 3, 36.7 / 36.8)
+    if (parts > 1 && pairs * parts > 256 && pairs * parts <= 330) parts = (int)(256 / pairs);
     if (parts > 1) p.parts = parts, p.split = 4;
   }
   return p;
