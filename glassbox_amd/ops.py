@@ -1854,6 +1854,10 @@ def attention_prefill(q: torch.Tensor, out: torch.Tensor, ctx, cache, n_heads: i
         raise KernelError("attention_prefill: block tables must be int32 [requests, pages]")
     lib = _lib("attention_bf16")
     max_q, max_ctx = int(ctx.host["max_q_len"]), int(ctx.host["max_context"])
+    # The longest context only shapes the launch: no more of it than a portion's tokens see.  (Portions behind 4,000 and 8,000
+    # keys, 32 heads of 64, a window of 1,024 and 64 kept keys, had their few keys shared by up to eight workgroups.)
+    if window or chunk:
+        max_ctx = min(max_ctx, (int(window) + int(keep_first) or int(chunk)) + max_q)
     # the portions' rows follow the single-token requests' rows; few and short portions over long contexts share
     # their keys among workgroups, which need room for their sums
     first_row, n_rows = n_dec, q.shape[0] - n_dec

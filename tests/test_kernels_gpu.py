@@ -1186,6 +1186,27 @@ def test_tuned_prefill_short_portions_over_long_contexts(nh, nkv, hd, window):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,window,keep,chunk", [(8, 2, 64, 700, 70, 0), (8, 8, 128, 300, 0, 0), (4, 4, 64, 0, 0, 1024)])
+def test_tuned_prefill_behind_histories_that_windows_and_runs_leave_out(nh, nkv, hd, window, keep, chunk):
+    """Short portions behind long contexts of which their tokens see little: the launch is shaped by what they see, the same
+    results as the plain kernel's, and no workspace of a longer context's size is asked for."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    q_lens, ctx_lens = [100, 37], [5150, 3301]
+    k_pages, v_pages, tables, _, _ = paged_setup(ctx_lens, nkv, hd, 16, seed=hd + nh, dtype=torch.bfloat16)
+    ctx = BareContext(q_lens, ctx_lens, tables)
+    q = to_dev((rnd(sum(q_lens), nh * hd, seed=14) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out, twin = torch.zeros_like(q), torch.zeros_like(q)
+    ops.attention_prefill(q, out, ctx, cache, nh, 1 / math.sqrt(hd), window, keep, chunk)
+    parts = ops._prefill_parts(max(q_lens), (window + keep or chunk) + max(q_lens), nh, 2, hd)
+    assert parts < ops._prefill_parts(max(q_lens), max(ctx_lens), nh, 2, hd)
+    assert [k[1][0] for k in ctx._bufs] == ([parts * sum(q_lens) * nh * (hd + 2)] if parts > 1 else [])
+    ops.attention_plain(q, twin, ctx.positions, torch.tensor(ctx.tok_seq, dtype=torch.int32, device=DEV), ctx.tables[0],
+                        cache.k_pages, cache.v_pages, nh, 1 / math.sqrt(hd), window, keep_first=keep, chunk=chunk)
+    assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
+
+
 @pytest.mark.parametrize("nh,ctxlen,qlen", [(2, 200, 90), (64, 1200, 1090)])   # 32 and 64 tokens a wave
 def test_tuned_prefill_sees_exactly_the_causal_keys(nh, ctxlen, qlen):
     """A portion in the middle of a request (it starts at position 110): token t must find a marked
