@@ -435,6 +435,10 @@ def test_gemm_bf16_that_divides_k_does_the_next_norm(M, N, K, gamma_dtype):
                                    (200, 528, 8200), (40, 1008, 4104),
                                    # a thousand rows and more: slices of k through the 256 x 256 tiles
                                    (2048, 2048, 8192), (1100, 1008, 4160), (1024, 528, 5120),
+                                   # and some hundred rows, rows and columns that no tile divides: on either side of where a k of
+                                   # 8,192 is long enough, where few rows of a longer one are, and on the far side of 256 and 1,023
+                                   (549, 528, 8192), (550, 528, 8192), (611, 1040, 8192), (320, 528, 14336), (257, 528, 17536),
+                                   (1023, 528, 4416),
                                    # some hundred rows, a k of 2,048 and very few tiles
                                    (128, 2048, 2048), (300, 1008, 2112), (256, 1024, 2048)])
 @pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
