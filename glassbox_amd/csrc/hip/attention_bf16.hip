@@ -20,7 +20,8 @@
 // (chunk, kv head, request), whose waves (sixteen where one workgroup takes a whole context of more
 // than 512 keys and the head size allows, else four) take runs of up to five neighbouring tiles of 64
 // keys, or tiles in turn; partial results are merged in a fixed order (waves in LDS, chunks by a
-// second kernel), so the result is the same on every run and in every row of a step.  crates/glassbox-core/src/model.rs:285-312 is the formula.
+// second kernel), so the result is the same on every run and in every row of a step.
+// crates/glassbox-core/src/model.rs:285-312 is the formula.
 #include "attention_bf16.h"
 #include <type_traits>
 
@@ -250,8 +251,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const int end = min(c0 + chunk, pos + 1);
   // Which of the chunk's tiles of 64 keys are the wave's.  Up to five for each of sixteen waves, or of four with heads above 64: a
   // run of neighbouring ones (eight requests of 4,095 keys in neighbouring pages, 32 heads of 64, 44.7 -> 42.4 us against page
-  // lookups by each lane and every sixteenth
-  // tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile,
+  // lookups by each lane and every sixteenth tile; in scattered pages 43.3 -> 43.5).  Longer contexts, and those whose first keys a window has passed: every WAVES-th tile,
   // and which wave begins where moves on from head to head and request to request (steps of 24 such layers, eight requests
   // of 7,200 keys 2,865 us, where every wave begins at its own number 2,920; but of 5,600 2,502 and 2,477).  The results of the
   // tiles from the first one on stand first in the merge, whichever wave had them, so that the order in which a request

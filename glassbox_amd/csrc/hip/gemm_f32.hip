@@ -1,6 +1,7 @@
 // 32-bit matrix product for the true 32-bit path: C[M,N] (+)= A[M,K] . W[N,K]^T with
 // W in the nn.Linear layout [out, in] (crates/glassbox-core/src/kernels.rs:381,586).
-// Plain fused multiply-adds in 32-bit, no matrix-core mode of reduced precision.
+// Fused multiply-adds of 32 bits throughout, on the vector units or in the matrix cores' 32-bit instruction: no mode of
+// reduced precision.
 //
 // Every output cell is summed in one order, whatever kernel computes it and whatever else is
 // in the batch: k is cut into slices of 64; a slice's products are added in ascending k by a
@@ -30,7 +31,7 @@ GB_DEFINE_LAST_ERROR
 
 namespace {
 
-constexpr int kSlice = 64;   // the summation order's slice of k: both kernels keep to it
+constexpr int kSlice = 64;   // the summation order's slice of k: all four kernels keep to it
 
 constexpr int BM = 64, BN = 64, BK = 16, TM = 4, TN = 4;
 static_assert(kSlice % BK == 0, "a slice is whole steps of the tiled kernel");
@@ -424,7 +425,7 @@ void launch_skinny(const float* a, int lda, const float* w, int ldw, float* c, i
   hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, R>), dim3((N + R - 1) / R), dim3(256), 256 * (kSlice + MT) * 4, stream, a, lda,
                      w, ldw, c, ldc, M, N, K, accumulate);
 }
-constexpr int kSkinnyMaxRows = 64;
+constexpr int kSkinnyMaxRows = 64;   // in passes of eight; by itself (skinny_pays) it runs at up to eight
 // Where the skinny kernel is the faster one (us, skinny / sliced, replayed from a graph over weights that no cache holds):
 // up to 4 rows of narrow products (960 x 960 at 1 and 4 rows 4.2 and 8.5 / 9.8, 2,048 x 8,192 17 and 29 / 63), up to 6 where k
 // is long (576 x 1,536 10.4 and 11.5 at 5 and 6 rows / 13.5, but 960 x 960 10.3 / 9.9), up to 8 where it is longer and the

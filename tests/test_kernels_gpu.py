@@ -54,7 +54,7 @@ def test_gemm_f32(N, K, M, accumulate):
 @pytest.mark.parametrize("N,K", [(1, 32), (50, 160), (17, 64), (331, 100), (96, 4100), (2048, 2048), (512, 8192), (8, 16384)])
 def test_gemm_f32_is_summed_in_one_order_by_both_kernels_and_at_every_number_of_rows(N, K):
     """A cell's sum is cut into slices of 64 of k, each a chain of fused multiply-adds from zero, added in order
-    (``csrc/hip/gemm_f32.hip``): the skinny kernel (8 rows of W a workgroup, a lane a slice) and the tiled one give the
+    (``csrc/hip/gemm_f32.hip``): the skinny kernel (4, 8 or 16 rows of W a workgroup, a lane a slice) and the tiled one give the
     same bits, and a row of A gives the same bits alone, among 8 and among 70 rows, which is what lets batched
     and unbatched generation agree exactly in 32-bit."""
     from glassbox_amd import ops
