@@ -430,7 +430,7 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 // where random ones take 749; without requests to memory it would take 530.  The kernel before this one (eight waves of 128 x 64,
 // 32 x 32 x 16 MFMAs, k-steps of 32, so that a request brought half lines: twice the requests to the second-level cache) kept
 // the matrix cores busy for 71 % of the cycles.  us, before -> now, same box: 8,192^3 842 -> 749 (1,468 TFLOP/s);
-// 6,151 x 28,672 x 4,096 1,311 -> 1,120; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
+// 6,151 x 28,672 x 4,096 with SiLU-multiply (another box) 1,283 -> 1,143; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
 // (8,192^3: 850 where this took 805); tiles dealt to the dies in squares (no gain).
 constexpr int RING_SLOTS = 5;   // (RBK, a k-step, and what slices of k may be: ring_steps.h)
 constexpr int RGM = 2, RGN = 2, RT = 8;                  // waves along m, n; 16 x 16 tiles of a wave along m and along n
@@ -756,8 +756,8 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
 }
 
 // The ring kernel pays where its tiles occupy at least three quarters of the compute units, from two row tiles on, and the
-// loads are whole 16-byte pieces.  (us, gate/up with SiLU-multiply, before / with it: 320 x 28,672 x 4,096 143 / 111,
-// 512 rows 161 / 116, 1,000 rows 287 / 209; 611 x 16,384 x 2,048 62 / 56, 1,000 rows 85 / 63.)
+// loads are whole 16-byte pieces.  (us, gate/up with SiLU-multiply, before / with it: 320 x 28,672 x 4,096 139 / 104,
+// 512 rows 156 / 106, 1,000 rows 283 / 203; 611 x 16,384 x 2,048 58 / 53, 1,000 rows 79 / 57.)
 constexpr int RING_MIN_ROWS = 257;
 // With slices of k: a thousand rows, or enough rows times k that a slice's sums, which go through memory, are the smaller
 // part (611 x 2,048 x 8,192 47.5 / 44.9, but 512 rows 34.8 / 43.2; 320 x 4,096 x 14,336 78 / 69, 1,000 rows 177 / 118; 611 x
