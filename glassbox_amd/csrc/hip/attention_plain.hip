@@ -38,7 +38,7 @@ GB_DEFINE_LAST_ERROR
 namespace {
 
 constexpr int kChunk = 256;
-constexpr int kEarlyPage = 16;   // chunk_alone: values asked for ahead with pages of this size
+constexpr int kEarlyPage = 16;   // chunk_alone's AHEAD form: pages of this size
 constexpr int kMaxOwn = 16;   // (dimension, word) pairs a thread owns at most: head size * page size <= 16,384
 
 struct Running {
@@ -70,11 +70,11 @@ template <> __device__ __forceinline__ void load_words<bf16>(const bf16* p, floa
 }
 
 // dot(q, key) in ascending dimension; the key lies in pieces of `piece` elements (key_offset)
-template <typename T>
+template <typename T, int UNROLL>
 __device__ __forceinline__ float key_dot(const float* qs, const T* kb, int slot, int hd, int page_size, int piece) {
   float dot = 0.f;
   if (piece == 8) {
-#pragma unroll 8
+#pragma unroll UNROLL
     for (int d0 = 0; d0 < hd; d0 += 8) {
       const T* kr = kb + ((size_t)(d0 / 8) * page_size + slot) * 8;
       float lo[4], hi[4];
@@ -129,7 +129,10 @@ struct Chunks {
 
 // One chunk by itself: keys c0 .. hi of the token's request.  Leaves m_c, l_c and the thread's sums a_c.
 // `qs` holds the query, `es` (kChunk floats) and `scratch` (17) are the block's.
-template <typename T, int PER>
+// AHEAD, for launches of few workgroups over contexts long enough (ahead_pays), with a pair a thread at most, pages of kEarlyPage and chunks that begin with a
+// page: the chunk's words of values are asked for before the scores, sixteen pages at once, where the loop below asks for four
+// at a time after them.  The sums are the same.
+template <typename T, int PER, bool AHEAD>
 __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, float* es, float* scratch,
                                             const int32_t* __restrict__ table, const T* __restrict__ k_pages,
                                             const T* __restrict__ v_pages, int kvh, float slope, int pos, int c0, int hi, float& m_c,
@@ -138,15 +141,12 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   const int ps = sh.page_size, hd = sh.hd;
   const int p = c0 + tid;
   const int words = ps / 4, pairs = hd * words;
-  // The usual page and a pair a thread: the chunk's words of values are asked for before the scores, sixteen pages at
-  // once, where the loop below asks for four at a time after them (the sums are the same; SmolLM2-360M shapes, a prompt of
-  // 200 and 16 single tokens, 34.9 -> 33.9 ms).
-  const bool early = PER == 1 && ps == kEarlyPage && c0 % kEarlyPage == 0;
-  float ev[kChunk / kEarlyPage][4];
-  if (early && tid < pairs) {
+  static_assert(!AHEAD || PER == 1, "a thread's words of a chunk's pages are held in registers");
+  float ev[AHEAD ? kChunk / kEarlyPage : 1][4];
+  if (AHEAD && tid < pairs) {
     const size_t at = (size_t)(tid / words) * ps + 4 * (tid % words);
 #pragma unroll
-    for (int i = 0; i < kChunk / kEarlyPage; ++i) {   // (behind the last page: that page again, not used)
+    for (int i = 0; i < (AHEAD ? kChunk / kEarlyPage : 0); ++i) {   // (behind the last page: that page again, not used)
       const int page = table[min(c0 + i * kEarlyPage, hi) / kEarlyPage];
       load_words<T>(v_pages + ((size_t)page * sh.nkv + kvh) * hd * ps + at, ev[i]);
     }
@@ -155,7 +155,7 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   if (p <= hi) {
     const int page = table[p / ps];
     const T* kb = k_pages + ((size_t)page * sh.nkv + kvh) * ps * hd;
-    s = sh.score(key_dot<T>(qs, kb, p % ps, hd, ps, key_piece(hd)), slope, pos - p);
+    s = sh.score(key_dot<T, AHEAD ? 8 : 4>(qs, kb, p % ps, hd, ps, key_piece(hd)), slope, pos - p);
   }
   m_c = block_max(s, scratch);
   const float e = p <= hi ? expf(s - m_c) : 0.f;
@@ -163,11 +163,11 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   l_c = block_sum(e, scratch);   // also orders the writes of es before the reads below
 #pragma unroll
   for (int u = 0; u < PER; ++u) a_c[u] = 0.f;
-  if (early) {
+  if constexpr (AHEAD) {
     if (tid < pairs) {
       const int p0 = c0 + 4 * (tid % words);
 #pragma unroll
-      for (int i = 0; i < kChunk / kEarlyPage; ++i)
+      for (int i = 0; i < (AHEAD ? kChunk / kEarlyPage : 0); ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           if (p0 + i * kEarlyPage + j <= hi) a_c[0] = fmaf(es[p0 - c0 + i * kEarlyPage + j], ev[i][j], a_c[0]);
@@ -219,7 +219,7 @@ __device__ __forceinline__ void finish(const Shape& sh, float* comb, const float
 
 __device__ __forceinline__ int ws_stride(int per) { return per * kChunk + 2; }
 
-template <typename T, int PER, bool SPLIT>
+template <typename T, int PER, bool SPLIT, bool AHEAD>
 __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tables, const T* __restrict__ k_pages,
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
   if (SPLIT) {
     const int c = blockIdx.y, c0 = ch.first(c);
     float m_c, l_c, a_c[PER];
-    chunk_alone<T, PER>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
+    chunk_alone<T, PER, AHEAD>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
     float* cell = ws + ((size_t)blockIdx.x * max_chunks + c) * ws_stride(PER);
 #pragma unroll
     for (int u = 0; u < PER; ++u) cell[u * kChunk + tid] = a_c[u];
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
   for (int c = 0; c < n_chunks; ++c) {
     const int c0 = ch.first(c);
     float m_c, l_c, a_c[PER];
-    chunk_alone<T, PER>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
+    chunk_alone<T, PER, AHEAD>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
     merge_chunk<PER>(r, acc, m_c, l_c, a_c);
   }
   finish<T, PER>(sh, comb, acc, r, h, out + (size_t)t * out_stride + (size_t)h * sh.hd);
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(kChunk) void attention_plain_group_kernel(
     for (int c = 0; c < n_chunks; ++c) {
       const int c0 = ch.first(c);
       float m_c, l_c, a_c[PER];
-      chunk_alone<T, PER>(sh, qs + j * sh.hd, es, scratch + kGroup * 4, table, k_pages, v_pages, kvh, slope, pos, c0,
+      chunk_alone<T, PER, false>(sh, qs + j * sh.hd, es, scratch + kGroup * 4, table, k_pages, v_pages, kvh, slope, pos, c0,
                           ch.last(c, pos), m_c, l_c, a_c);
       merge_chunk<PER>(r, acc, m_c, l_c, a_c);
     }
@@ -516,14 +516,31 @@ inline int own_pairs(int hd, int page_size) {
   return 0;
 }
 
+// Where values are asked for ahead.  What it saves is a round trip to memory a chunk; what it costs are 64 registers a thread, and
+// sixteen loads whatever the chunk holds.  us, after / ahead, heads of 64, in 32-bit: 1,000 keys in four workgroups a head, 15 heads,
+// 13.5 / 12.7, eight requests of 300 keys 13.1 / 12.3, and of 256 10.6 / 9.9; but one of 20 keys 5.9 / 9.1, of 100 7.6 / 9.5; and of
+// many workgroups 64 requests of 700 keys 56 / 62, eight portions of 60 rows 44 / 64, 512 rows of a window of 256 101 / 140.
+// (200 keys 9.7 / 9.7, heads of 32 9.3 / 8.4.)  Not in bfloat16: 256 keys 10.5 / 10.2, 200 keys 9.7 / 10.0, and the context that a
+// captured step is launched for says little of those it has; nor where a workgroup walks several chunks, of which the last may be
+// short (16 rows of up to 300 keys 13.6 / 16.0).
+constexpr int kAheadGroups = 640, kAheadKeys = 200;
+template <typename T, int PER>
+constexpr bool kMayAhead = PER == 1 && sizeof(T) == 4;
+inline bool ahead_pays(const Shape& sh, bool spread, long long workgroups, int max_context) {
+  return sh.page_size == kEarlyPage && sh.window == 0 && sh.span == 0 && workgroups <= kAheadGroups && max_context >= kAheadKeys &&
+         (spread || max_context <= kChunk);
+}
+
 template <typename T, int PER>
 void launch(const void* q, int q_stride, void* out, int out_stride, const int32_t* positions, const int32_t* tok_seq,
             const int32_t* tables, const void* k_pages, const void* v_pages, int n, const Shape& sh, float* ws,
-            int max_chunks, bool grouped_form, hipStream_t stream) {
+            int max_chunks, int max_context, bool grouped_form, hipStream_t stream) {
   const size_t comb = sizeof(float) * sh.hd * (sh.page_size / 4);
   const size_t smem = sizeof(float) * (sh.hd + kChunk + 17) + comb;
+  const bool ahead = kMayAhead<T, PER> && ahead_pays(sh, ws != nullptr, (long long)n * sh.nh * (ws != nullptr ? max_chunks : 1), max_context);
   if (ws != nullptr) {
-    hipLaunchKernelGGL((attention_plain_kernel<T, PER, true>), dim3((unsigned)(n * sh.nh), (unsigned)max_chunks), dim3(kChunk),
+    const auto kernel = ahead ? attention_plain_kernel<T, PER, true, kMayAhead<T, PER>> : attention_plain_kernel<T, PER, true, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(n * sh.nh), (unsigned)max_chunks), dim3(kChunk),
                        smem, stream, (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables,
                        (const T*)k_pages, (const T*)v_pages, sh, ws, max_chunks);
     hipLaunchKernelGGL((attention_plain_merge_kernel<T, PER>), dim3((unsigned)(n * sh.nh)), dim3(kChunk), comb, stream,
@@ -537,7 +554,8 @@ void launch(const void* q, int q_stride, void* out, int out_stride, const int32_
                          (const T*)v_pages, sh, n);
     }
   } else {
-    hipLaunchKernelGGL((attention_plain_kernel<T, PER, false>), dim3((unsigned)(n * sh.nh)), dim3(kChunk), smem, stream,
+    const auto kernel = ahead ? attention_plain_kernel<T, PER, false, kMayAhead<T, PER>> : attention_plain_kernel<T, PER, false, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(n * sh.nh)), dim3(kChunk), smem, stream,
                        (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables, (const T*)k_pages,
                        (const T*)v_pages, sh, nullptr, 0);
   }
@@ -546,11 +564,11 @@ void launch(const void* q, int q_stride, void* out, int out_stride, const int32_
 template <typename T>
 int launch_by_pairs(int per, const void* q, int q_stride, void* out, int out_stride, const int32_t* positions,
                     const int32_t* tok_seq, const int32_t* tables, const void* k_pages, const void* v_pages, int n,
-                    const Shape& sh, float* ws, int max_chunks, bool grouped_form, hipStream_t stream) {
+                    const Shape& sh, float* ws, int max_chunks, int max_context, bool grouped_form, hipStream_t stream) {
 #define GB_PLAIN_CASE(P)                                                                                              \
   case P:                                                                                                             \
     launch<T, P>(q, q_stride, out, out_stride, positions, tok_seq, tables, k_pages, v_pages, n, sh, ws, max_chunks,       \
-                 grouped_form, stream);                                                                               \
+                 max_context, grouped_form, stream);                                                                               \
     break;
   switch (per) {
     GB_PLAIN_CASE(1) GB_PLAIN_CASE(2) GB_PLAIN_CASE(4) GB_PLAIN_CASE(8) GB_PLAIN_CASE(16)
@@ -610,10 +628,10 @@ extern "C" int gb_attention_plain(const void* q, int q_stride, void* out, int ou
   const Shape sh{nh, nkv, hd, page_size, window, table_stride, scale, keep_first, span, softcap, sinks, slopes};
   if (dtype == kF32)
     return launch_by_pairs<float>(per, q, q_stride, out, out_stride, positions, tok_seq, tables, k_pages, v_pages, n, sh, ws,
-                                  max_chunks, grouped != 0, stream);
+                                  max_chunks, max_context, grouped != 0, stream);
   if (dtype == kBF16)
     return launch_by_pairs<bf16>(per, q, q_stride, out, out_stride, positions, tok_seq, tables, k_pages, v_pages, n, sh, ws,
-                                 max_chunks, grouped != 0, stream);
+                                 max_chunks, max_context, grouped != 0, stream);
   return fail("attention_plain: unknown dtype %d", dtype);
 }
 

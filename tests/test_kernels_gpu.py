@@ -854,6 +854,38 @@ def test_attention_plain_spread_over_workgroups_gives_the_bits_of_one_workgroup(
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nkv,hd", [(2, 64), (8, 32), (4, 16)])
+def test_attention_plain_asks_for_values_ahead_where_workgroups_are_few(dtype, nkv, hd):
+    """32-bit launches of up to 640 workgroups over contexts of 200 keys and more ask for a chunk's values before its scores: chunks
+    that end around a page and around 256 keys, as a launch of few rows, of the last and the first number of rows on either side
+    of the line, with the longest context on either side of where it counts, and spread over workgroups: the same bits, and those of the float64 formula."""
+    from glassbox_amd import ops
+    nh = 8
+    ctx_lens = [1, 17, 191, 192, 193, 239, 240, 241, 255, 256, 257, 447, 448, 700]
+    k_pages, v_pages, tables, ks, vs = paged_setup(ctx_lens, nkv, hd, 16, seed=hd + nkv, dtype=dtype)
+    n = len(ctx_lens)
+    q, scale = rnd(n, nh * hd, seed=12).to(dtype), 1 / math.sqrt(hd)
+    rest = (to_dev(tables), to_dev(ops.pack_keys(k_pages)), to_dev(v_pages), nh, scale, 0)
+
+    def rows(count, spread=False, longest=700):
+        seq = [i % n for i in range(count)]
+        pos = torch.tensor([ctx_lens[i] - 1 for i in seq], dtype=torch.int32, device=DEV)
+        out = torch.full((count, nh * hd), 7.0, device=DEV, dtype=dtype)
+        floats = ops.attention_plain_split_floats(count, nh, hd, 16, 700) if spread else 0
+        more = dict(workspace=torch.full((floats,), float("nan"), device=DEV), max_context=700) if spread else dict(max_context=longest)
+        ops.attention_plain(to_dev(q[seq]), out, pos, torch.tensor(seq, dtype=torch.int32, device=DEV), *rest, **more)
+        return out.cpu()
+
+    few = rows(n)
+    for count, longest in ((10, 256), (10, 200), (10, 199), (n, 0)):    # (the first ten contexts are of up to 256 keys)
+        assert torch.equal(rows(count, longest=longest), few[:count])
+    want = plain_attention_rows(q, ks, vs, list(range(n)), [c - 1 for c in ctx_lens], nh, scale, 0)
+    assert (few.double() - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2 ** -7)
+    for count in (n, 26, 27):               # three chunks each: 336, 624 and 648
+        assert torch.equal(rows(count, spread=True), few[[i % n for i in range(count)]])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,page", [(4, 2, 16, 16), (8, 8, 64, 16), (3, 1, 32, 48), (2, 1, 128, 32), (2, 2, 256, 16),
                                             (5, 5, 80, 64)])
 def test_attention_plain_eight_rows_a_workgroup_gives_the_bits_of_one_row_a_workgroup(dtype, nh, nkv, hd, page):
