@@ -516,13 +516,13 @@ inline int own_pairs(int hd, int page_size) {
   return 0;
 }
 
-// Where values are asked for ahead.  What it saves is a round trip to memory a chunk; what it costs are 64 registers a thread, and
-// sixteen loads whatever the chunk holds.  us, after / ahead, heads of 64, in 32-bit: 1,000 keys in four workgroups a head, 15 heads,
-// 13.5 / 12.7, eight requests of 300 keys 13.1 / 12.3, and of 256 10.6 / 9.9; but one of 20 keys 5.9 / 9.1, of 100 7.6 / 9.5; and of
-// many workgroups 64 requests of 700 keys 56 / 62, eight portions of 60 rows 44 / 64, 512 rows of a window of 256 101 / 140.
-// (200 keys 9.7 / 9.7, heads of 32 9.3 / 8.4.)  Not in bfloat16: 256 keys 10.5 / 10.2, 200 keys 9.7 / 10.0, and the context that a
-// captured step is launched for says little of those it has; nor where a workgroup walks several chunks, of which the last may be
-// short (16 rows of up to 300 keys 13.6 / 16.0).
+// Where values are asked for ahead.  What it saves is a round trip to memory a chunk; what it costs are registers, and sixteen loads
+// whatever the chunk holds.  us, after / ahead, heads of 64, in 32-bit: one request of 1,000 keys, 15 heads, 13.5 / 13.0, eight of
+// 300 13.0 / 12.5, one of 256 10.6 / 9.9, of 200 9.7 / 9.7 (heads of 32 9.2 / 8.4), but of 100 7.6 / 9.5 and of 20 5.9 / 9.1; four chunks
+// each of 360, 432, 600 and 720 workgroups 20.6 / 19.2, 21.7 / 20.5, 23.1 / 22.9 and 24.3 / 24.9; 64 requests of 700 keys 56 / 62, eight
+// portions of 60 rows 44 / 64, 512 rows behind a window of 256 keys 101 / 140.  Not in bfloat16: 256 keys 10.5 / 10.2, 200 keys
+// 9.7 / 10.0, and the context that a captured step is launched for says little of those it has; nor where a workgroup
+// walks several chunks, of which the last may be short (16 rows of up to 300 keys 13.6 / 16.0).
 constexpr int kAheadGroups = 640, kAheadKeys = 200;
 template <typename T, int PER>
 constexpr bool kMayAhead = PER == 1 && sizeof(T) == 4;

@@ -430,7 +430,7 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 // where random ones take 749; without requests to memory it would take 530.  The kernel before this one (eight waves of 128 x 64,
 // 32 x 32 x 16 MFMAs, k-steps of 32, so that a request brought half lines: twice the requests to the second-level cache) kept
 // the matrix cores busy for 71 % of the cycles.  us, before -> now, same box: 8,192^3 842 -> 749 (1,468 TFLOP/s);
-// 6,151 x 28,672 x 4,096 with SiLU-multiply (another box) 1,283 -> 1,143; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
+// 6,151 x 28,672 x 4,096 with SiLU-multiply (another card) 1,283 -> 1,143; 6,151 x 4,096 x 14,336 676 -> 584.  Tried: the same with 32 x 32 x 16 MFMAs
 // (8,192^3: 850 where this took 805); tiles dealt to the dies in squares (no gain).
 constexpr int RING_SLOTS = 5;   // (RBK, a k-step, and what slices of k may be: ring_steps.h)
 constexpr int RGM = 2, RGN = 2, RT = 8;                  // waves along m, n; 16 x 16 tiles of a wave along m and along n
