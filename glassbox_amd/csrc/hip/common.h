@@ -88,6 +88,28 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
   return scratch[16];
 }
 
+// ---- arithmetic that several kernels do to the same bits --------------------------------------------------------
+// (multiplications and additions are spelled out as they are rounded: contracted by the compiler, each kernel could get
+// bits of its own)
+
+// The RMS norm's sum of squares of a row of d numbers in words of four: thread `tid` of norm_threads(d) has words tid, tid +
+// norm_threads(d), ... (zeros beyond the row), adds its own here, a wave's are added by wave_sum, the waves' in order from zero.
+__host__ __device__ constexpr int norm_threads(int d) { return d >= 1024 ? 256 : d >= 256 ? 128 : 64; }
+template <int V4> __device__ __forceinline__ float norm_squares(const f32x4 (&v)[V4]) {
+  float ss = fmaf(v[0][0], v[0][0], v[0][1] * v[0][1]);
+#pragma unroll
+  for (int i = 2; i < 4 * V4; ++i) ss = fmaf(v[i / 4][i % 4], v[i / 4][i % 4], ss);
+  return ss;
+}
+__device__ __forceinline__ float norm_scale(float total, int d, float eps) { return 1.0f / sqrtf(total / (float)d + eps); }
+
+// a pair of coordinates turned by an angle of cosine c and sine s
+__device__ __forceinline__ float turned_lo(float x0, float x1, float c, float s) { return fmaf(x0, c, -(x1 * s)); }
+__device__ __forceinline__ float turned_hi(float x0, float x1, float c, float s) { return fmaf(x1, c, x0 * s); }
+
+// silu(g) * u
+__device__ __forceinline__ float silu_times(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
 inline std::string& last_error() {
   static thread_local std::string msg;
   return msg;

@@ -91,7 +91,6 @@ __global__ void rmsnorm_words_kernel(const float* __restrict__ x, const G* __res
   const int r = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
   const float* xr = x + (size_t)(rows ? rows[r] : r) * d;
   f32x4 v[V4], g[V4];
-  float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < V4; ++j) {
     const int c = (tid + j * nt) * 4;
@@ -108,16 +107,12 @@ __global__ void rmsnorm_words_kernel(const float* __restrict__ x, const G* __res
       }
     }
   }
-#pragma unroll
-  for (int j = 0; j < V4; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
-  ss = wave_sum(ss);
+  const float ss = wave_sum(norm_squares(v));
   if (tid % kWave == 0) partial[tid / kWave] = ss;
   __syncthreads();
   float total = 0.f;
   for (int w = 0; w < (nt + kWave - 1) / kWave; ++w) total += partial[w];
-  const float s = 1.0f / sqrtf(total / (float)d + eps);
+  const float s = norm_scale(total, d, eps);
   O* orow = out + (size_t)r * d;
 #pragma unroll
   for (int j = 0; j < V4; ++j) {
@@ -141,7 +136,7 @@ extern "C" int gb_rmsnorm(const float* x, const void* gamma, int gamma_dtype, co
                           int out_dtype, int m, int d, float eps, hipStream_t stream) {
   GB_REQUIRE(m >= 0 && d > 0, "rmsnorm: bad sizes m=%d d=%d", m, d);
   if (m == 0) return 0;
-  const int threads = d >= 1024 ? 256 : (d >= 256 ? 128 : 64);
+  const int threads = norm_threads(d);
   const int per_thread = (d + threads - 1) / threads;
   // whole words where the rows allow it (every row then starts at a multiple of 16 bytes)
   const bool words = d % 4 == 0 && d <= 4 * 8 * threads && (uintptr_t)x % 16 == 0 && (uintptr_t)gamma % 16 == 0 &&
@@ -238,8 +233,8 @@ __global__ void rope_store_scalar_kernel(T* __restrict__ qkv, int row_stride, co
       if (p < pairs) {
         const int head = p / half, i = p % half;
         T* h = row + (size_t)head * hd;
-        const T y0 = from_f<T>(rotate ? x0[j] * cc[j] - x1[j] * sn[j] : x0[j]);
-        const T y1 = from_f<T>(rotate ? x1[j] * cc[j] + x0[j] * sn[j] : x1[j]);
+        const T y0 = from_f<T>(rotate ? turned_lo(x0[j], x1[j], cc[j], sn[j]) : x0[j]);
+        const T y1 = from_f<T>(rotate ? turned_hi(x0[j], x1[j], cc[j], sn[j]) : x1[j]);
         h[i] = y0;  // rotated keys stay in the row too: parts may read them back
         h[i + half] = y1;
         if (head >= nh && slot >= 0) {
@@ -292,10 +287,10 @@ __global__ void rope_store_kernel(T* __restrict__ qkv, int row_stride, const flo
     if (!is_v && rotate) {
       const float2 c = *reinterpret_cast<const float2*>(cosv + (size_t)t * half + j);
       const float2 sn = *reinterpret_cast<const float2*>(sinv + (size_t)t * half + j);
-      y0.a = from_f<T>(to_f(x0.a) * c.x - to_f(x1.a) * sn.x);
-      y0.b = from_f<T>(to_f(x0.b) * c.y - to_f(x1.b) * sn.y);
-      y1.a = from_f<T>(to_f(x1.a) * c.x + to_f(x0.a) * sn.x);
-      y1.b = from_f<T>(to_f(x1.b) * c.y + to_f(x0.b) * sn.y);
+      y0.a = from_f<T>(turned_lo(to_f(x0.a), to_f(x1.a), c.x, sn.x));
+      y0.b = from_f<T>(turned_lo(to_f(x0.b), to_f(x1.b), c.y, sn.y));
+      y1.a = from_f<T>(turned_hi(to_f(x0.a), to_f(x1.a), c.x, sn.x));
+      y1.b = from_f<T>(turned_hi(to_f(x0.b), to_f(x1.b), c.y, sn.y));
       *reinterpret_cast<P*>(head + j) = y0;  // rotated keys stay in the row too: parts may read them back
       *reinterpret_cast<P*>(head + half + j) = y1;
     }
@@ -560,7 +555,7 @@ __global__ void silu_mul_kernel(const T* __restrict__ gu, T* __restrict__ act, i
   const size_t t = idx / inter, c = idx % inter;
   const float g = to_f(gu[t * 2 * inter + c]);
   const float u = to_f(gu[t * 2 * inter + inter + c]);
-  act[idx] = from_f<T>(g / (1.0f + expf(-g)) * u);
+  act[idx] = from_f<T>(silu_times(g, u));
 }
 
 extern "C" int gb_silu_mul(const void* gu, void* act, int dtype, int n, int inter, hipStream_t stream) {

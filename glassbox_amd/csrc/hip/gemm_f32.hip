@@ -327,46 +327,157 @@ constexpr int kFewTiles = 256;
 // Word p of the slice of pair t lies at position p ^ (t % 16), so that the reads of 16 neighbouring lanes spread over all banks.
 constexpr int SV = kSlice / 4;    // 16-byte words a slice of one row
 
-template <int MT, int R>   // rows of A a pass (the step's rows go MT at a time); rows of W a workgroup
-__global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
+// What the skinny kernel may do besides the product, for a step of one or two rows (a decode step of the 32-bit path, whose
+// kernels are so short that what lies between them counts).  The bits are those of the kernels that each does by itself: the
+// expressions and the order of every sum are shared with them (common.h).
+//  * NORM: A is the residual, and the rows that are multiplied are its RMS norm's (gb_rmsnorm): in every workgroup a fifth wave,
+//    which asks for none of W and so need not wait for it, norms them into LDS while W is on its way.
+//  * EPI_UNIT: W stacks gate rows over as many up rows; C holds silu(gate) * up (gb_silu_mul).  A workgroup owns R / 2 gate rows
+//    and the up rows that go with them.
+//  * EPI_HEADS: W stacks nh query heads, nkv key heads and nkv value heads of hd rows; queries and keys are turned by
+//    their position's angles, and keys and values also go to their places in the pages (gb_rope_store).  A workgroup owns
+//    R / 2 pairs (i, i + hd / 2) of coordinates.
+// us, replayed from a graph over weights that no cache holds, each kernel by itself / in one, a row of 960: norm, product by 5,120
+// rows and unit 12.7 / 8.9 (the product alone 8.2); norm, product by 1,600 rows, rotation and cache write 8.9 / 6.2 (4.2); a row
+// of 576: 8.7 / 6.0 (4.7), 8.1 / 5.7 (3.6); of 2,048: 33.9 / 31.5 (29.1), 19.2 / 13.6 (13.5).
+enum : int { EPI_PLAIN = 0, EPI_UNIT = 2, EPI_HEADS = 3 };
+constexpr int kStepMaxRows = 2;
+struct StepExtras {
+  const float* gamma;   // of the norm, with NORM
+  float eps;
+  const float* cosv;    // [M][hd / 2], or null: nothing is turned
+  const float* sinv;
+  const int32_t* slots;   // [M], or null: nothing is stored
+  float* k_pages;
+  float* v_pages;
+  int nh, nkv, hd, page_size;
+};
+
+constexpr int kNormedFloats = 2560;   // of the rows that a workgroup norms (step_takes)
+
+// Wave `NV` times norm_threads' worth: one wave norms MT rows of K numbers into LDS; a lane stands for threads lane, lane + 64, ...
+// of the NV waves of the norm's own kernel.  Word p of slice t of a row lies at position p ^ (t % 16), for the reads of 16 lanes
+// on as many slices.
+template <int MT, int NV>
+__device__ __forceinline__ void norm_rows(const float* __restrict__ a, int lda, const float* __restrict__ gamma, float eps, int M, int K,
+                                          int lane, int slices, float* rows) {
+  constexpr int NW = kNormedFloats / 4 / kWave / MT;   // words a lane
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 x[MT][NW], g[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {   // (a word beyond k: the first one, not used)
+    const int k = 4 * (lane + kWave * i), from = k < K ? k : 0;
+    g[i] = *reinterpret_cast<const f32x4*>(gamma + from);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x[m][i] = *reinterpret_cast<const f32x4*>(a + (size_t)min(m, M - 1) * lda + from);
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    float total = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      constexpr int OWN = (NW + NV - 1) / NV < 1 ? 1 : (NW + NV - 1) / NV;
+      f32x4 own[OWN];
+#pragma unroll
+      for (int j = 0; j < OWN; ++j) {
+        const int i = v + j * NV;
+        own[j] = i < NW && 4 * (lane + kWave * i) < K ? x[m][i < NW ? i : 0] : zero;
+      }
+      total += wave_sum(norm_squares(own));
+    }
+    const float s = norm_scale(total, K, eps);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const int word = lane + kWave * i, t = word / SV, p = word % SV;
+      if (4 * word < K) {
+        f32x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = g[i][e] * (x[m][i][e] * s);
+        *reinterpret_cast<f32x4*>(rows + ((size_t)m * slices + t) * kSlice + 4 * (p ^ (t % 16))) = h;
+      }
+    }
+  }
+}
+
+template <int MT, int R, int EPI, bool NORM>   // rows of A a pass (the step's rows go MT at a time); rows of W a workgroup
+__global__ __launch_bounds__(NORM ? 256 + kWave : 256, NORM ? 4 : 1)   // (five waves: two workgroups a unit fit with four a SIMD)
+void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
                                                               const float* __restrict__ w, int ldw,
                                                               float* __restrict__ c, int ldc, int M, int N, int K,
-                                                              int accumulate) {
+                                                              int accumulate, StepExtras ex) {
   constexpr int SG = 256 / R;   // slices in flight a workgroup
-  extern __shared__ __attribute__((aligned(16))) float wl[];   // [R][SG][64], then part [SG][R][MT]
+  extern __shared__ __attribute__((aligned(16))) float wl[];   // [R][SG][64], then part [SG][R][MT], then with NORM the rows [MT][slices][64]
   float* part = wl + 256 * kSlice;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  float* rows = part + 256 * MT;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const bool works = !NORM || wave < 256 / kWave;   // (else: the wave that norms)
   const int r = tid % R, sl = tid / R;
   const int n0 = blockIdx.x * R;
   const int slices = (K + kSlice - 1) / kSlice;
   // the thread that adds the slices of cell (row cm of the pass, column cr)
   const int cr = tid % R, cm = tid / R;
+  // the row of W behind row t of the workgroup's (beyond the last: that one again)
+  const int half = EPI == EPI_HEADS ? ex.hd / 2 : N / 2;
+  auto w_row = [&](int t) -> int {
+    if constexpr (EPI == EPI_PLAIN) return min(n0 + t, N - 1);
+    const int pair = min(n0 / 2 + t % (R / 2), N / 2 - 1);
+    return (EPI == EPI_HEADS ? pair / half * ex.hd + pair % half : pair) + (t >= R / 2 ? half : 0);
+  };
+  // with EPI_HEADS the pair that a thread finishes
+  const int pair = n0 / 2 + cr;
+  const int head = EPI == EPI_HEADS ? pair / half : 0, at = EPI == EPI_HEADS ? pair % half : 0;
+  const bool finishes = EPI != EPI_PLAIN && cm < MT && cm < M && cr < R / 2 && pair < N / 2;
+  const bool is_value = EPI == EPI_HEADS && head >= ex.nh + ex.nkv;
+  float cs = 1.f, sn = 0.f;
+  int slot = -1;
+  if (NORM && !works) {   // (NORM: one pass)
+    switch (norm_threads(K) / kWave) {
+      case 1: norm_rows<MT, 1>(a, lda, ex.gamma, ex.eps, M, K, lane, slices, rows); break;
+      case 2: norm_rows<MT, 2>(a, lda, ex.gamma, ex.eps, M, K, lane, slices, rows); break;
+      default: norm_rows<MT, 4>(a, lda, ex.gamma, ex.eps, M, K, lane, slices, rows);
+    }
+  }
 
   for (int m0 = 0; m0 < M; m0 += MT) {
-    float total = 0.f;
+    float total = 0.f, old = 0.f;
+    const int gm = m0 + cm, gn = n0 + cr;
+    const bool owns = EPI == EPI_PLAIN && cm < MT && gm < M && gn < N;
     for (int s0 = 0; s0 < slices; s0 += SG) {
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         // four slices of a row, which one wave brings: unit u of the wave's
         const int unit = wave * 16 + u, row = unit / (SG / 4), first = unit % (SG / 4) * 4;
-        if (s0 + first >= slices) continue;                                // the same for the whole wave
+        if (!works || s0 + first >= slices) continue;                      // the same for the whole wave
         const int mine = first + lane / 16;
         const int word = (lane % 16) ^ ((mine * R + row) % 16);
         // (a word beyond k or n is not used: any address inside W will do for it)
         const int k = (s0 + mine) * kSlice + 4 * word;
-        const float* from = w + (size_t)min(n0 + row, N - 1) * ldw + (k < K ? k : 0);
+        const float* from = w + (size_t)w_row(row) * ldw + (k < K ? k : 0);
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)(uintptr_t)from,
                                          (__attribute__((address_space(3))) uint32_t*)(uint32_t)(uintptr_t)(wl + unit * 256), 16, 0, 0);
       }
+      // What the end will want from memory is asked for under W: a cell's old value; a pair's angle and its row's place in the pages.
+      // (Not before W: the compiler would wait for it there.)
+      if (EPI == EPI_PLAIN && accumulate && owns && s0 == 0) old = c[(size_t)gm * ldc + gn];
+      if constexpr (EPI == EPI_HEADS) {
+        if (finishes && s0 == 0) {
+          if (ex.cosv && !is_value) {
+            cs = ex.cosv[(size_t)cm * half + at];
+            sn = ex.sinv[(size_t)cm * half + at];
+          }
+          if (ex.slots && head >= ex.nh) slot = ex.slots[cm];
+        }
+      }
       const int k0 = (s0 + sl) * kSlice;
-      const bool live = k0 < K;
+      const bool live = works && k0 < K;
       // a single row of A is asked for before W has arrived
-      f32x4 x1[MT == 1 ? SV : 1];
-      if (MT == 1) {
+      constexpr bool EARLY = MT == 1 && !NORM;
+      f32x4 x1[EARLY ? SV : 1];
+      if constexpr (EARLY) {
 #pragma unroll
         for (int i = 0; i < SV; ++i) {
           const int k = k0 + 4 * i;
-          x1[MT == 1 ? i : 0] = *reinterpret_cast<const f32x4*>(a + (size_t)m0 * lda + (k < K ? k : 0));
+          x1[i] = *reinterpret_cast<const f32x4*>(a + (size_t)m0 * lda + (k < K ? k : 0));
         }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -384,7 +495,10 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
               if (MT == 1 || m0 + m < M) {
-                const f32x4 x = MT == 1 ? x1[MT == 1 ? i : 0] : *reinterpret_cast<const f32x4*>(a + (size_t)(m0 + m) * lda + k);
+                f32x4 x;
+                if constexpr (EARLY) x = x1[i];
+                else if constexpr (NORM) x = *reinterpret_cast<const f32x4*>(rows + ((size_t)m * slices + s0 + sl) * kSlice + 4 * (i ^ ((s0 + sl) % 16)));
+                else x = *reinterpret_cast<const f32x4*>(a + (size_t)(m0 + m) * lda + k);
                 acc[m] = fmaf(x[0], wv[0], acc[m]);
                 acc[m] = fmaf(x[1], wv[1], acc[m]);
                 acc[m] = fmaf(x[2], wv[2], acc[m]);
@@ -395,7 +509,8 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
         }
       }
 #pragma unroll
-      for (int m = 0; m < MT; ++m) part[(sl * R + r) * MT + m] = acc[m];
+      for (int m = 0; m < MT; ++m)
+        if (works) part[(sl * R + r) * MT + m] = acc[m];
       __syncthreads();
       if (cm < MT) {
         const int count = min(SG, slices - s0);
@@ -408,22 +523,50 @@ __global__ __launch_bounds__(256) void gemm_f32_skinny_kernel(const float* __res
             if (s + q < count) total += v[q];
         }
       }
-      if (s0 + SG < slices || m0 + MT < M) __syncthreads();
+      if (EPI != EPI_PLAIN || s0 + SG < slices || m0 + MT < M) __syncthreads();
     }
-    const int gm = m0 + cm, gn = n0 + cr;
-    if (cm < MT && gm < M && gn < N) {
-      float* dst = c + (size_t)gm * ldc + gn;
-      *dst = accumulate ? *dst + total : total;
+    if constexpr (EPI == EPI_PLAIN) {
+      if (owns) c[(size_t)gm * ldc + gn] = accumulate ? old + total : total;
+    } else {
+      // the two rows of a pair meet (every thread has read the slices' sums)
+      if (cm < MT) part[cm * R + cr] = total;
+      __syncthreads();
+      if (finishes) {   // (a launch has one pass)
+        const float lo = total, hi = part[cm * R + cr + R / 2];
+        if constexpr (EPI == EPI_UNIT) {
+          c[(size_t)cm * ldc + pair] = silu_times(lo, hi);
+        } else {
+          const bool turns = ex.cosv && !is_value;
+          const float y0 = turns ? turned_lo(lo, hi, cs, sn) : lo, y1 = turns ? turned_hi(lo, hi, cs, sn) : hi;
+          float* row = c + (size_t)cm * ldc + (size_t)head * ex.hd;
+          row[at] = y0;
+          row[half + at] = y1;
+          if (slot >= 0) {
+            const int page = slot / ex.page_size, off = slot % ex.page_size, piece = key_piece(ex.hd);
+            if (is_value) {
+              float* to = ex.v_pages + ((size_t)page * ex.nkv + (head - ex.nh - ex.nkv)) * ex.hd * ex.page_size + off;
+              to[(size_t)at * ex.page_size] = y0;
+              to[(size_t)(half + at) * ex.page_size] = y1;
+            } else {
+              float* to = ex.k_pages + ((size_t)page * ex.nkv + (head - ex.nh)) * ex.page_size * ex.hd;
+              to[key_offset(off, at, ex.page_size, piece)] = y0;
+              to[key_offset(off, half + at, ex.page_size, piece)] = y1;
+            }
+          }
+        }
+      }
     }
   }
 }
 
-template <int MT, int R>
+template <int MT, int R, int EPI = EPI_PLAIN, bool NORM = false>
 void launch_skinny(const float* a, int lda, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
-                        int accumulate, hipStream_t stream) {
+                        int accumulate, hipStream_t stream, const StepExtras& ex = StepExtras{}) {
   static_assert(MT * R <= 256, "one thread a cell of a pass");
-  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, R>), dim3((N + R - 1) / R), dim3(256), 256 * (kSlice + MT) * 4, stream, a, lda,
-                     w, ldw, c, ldc, M, N, K, accumulate);
+  const size_t rows = NORM ? (size_t)MT * ((K + kSlice - 1) / kSlice) * kSlice : 0;
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, R, EPI, NORM>), dim3((N + R - 1) / R), dim3(NORM ? 256 + kWave : 256),
+                     (256 * (kSlice + MT) + rows) * 4,
+                     stream, a, lda, w, ldw, c, ldc, M, N, K, accumulate, ex);
 }
 constexpr int kSkinnyMaxRows = 64;   // in passes of eight; by itself (skinny_pays) it runs at up to eight
 // Where the skinny kernel is the faster one (us, skinny / sliced, replayed from a graph over weights that no cache holds):
@@ -439,6 +582,13 @@ constexpr int kTwoAUnit = 512, kNarrow = 8 * kTwoAUnit, kLongK = 1280, kLongerK 
 inline bool skinny_pays(int M, int N, int K) {
   if (N > kNarrow) return M <= 2;
   return M <= 4 || (M <= 6 && K >= kLongK) || (M <= 8 && K >= kLongerK && N <= 4 * kTwoAUnit);
+}
+
+// A step's kernels in one: where the skinny kernel runs anyway, up to two rows; with the norm, as long as the rows that a
+// workgroup norms for itself leave LDS for two workgroups a unit (160 KB: 2 x (64 for W, 2 for the sums, 10)).
+inline bool step_takes(int M, int N, int K, bool norm) {
+  return M >= 1 && M <= kStepMaxRows && K % 4 == 0 && N % 2 == 0 && skinny_pays(M, N, K) &&
+         (!norm || M * ((K + kSlice - 1) / kSlice) * kSlice <= kNormedFloats);
 }
 
 inline bool words_of_16_bytes(const void* p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0; }
@@ -499,6 +649,37 @@ extern "C" int gb_gemm_f32(const float* a, int lda, const float* w, int ldw, flo
   return gb_gemm_f32_by(a, lda, w, ldw, c, ldc, M, N, K, accumulate, 0, stream);
 }
 
+// Whether gb_gemm_f32_step takes a product of M rows by N rows of W (with the norm before it).
+extern "C" int gb_gemm_f32_step_takes(int M, int N, int K, int norm) { return step_takes(M, N, K, norm != 0) ? 1 : 0; }
+
+// A product of one or two rows with what stands around it in a decode step, see StepExtras: gamma (or null): a is the
+// residual and is normed first; epilogue 0 stores, 2 forms the gated unit of stacked gate and up rows (C is [M, N / 2]), 3 turns
+// heads and writes the pages.  The bits are those of gb_rmsnorm, gb_gemm_f32, gb_silu_mul and gb_rope_store one after the other.
+extern "C" int gb_gemm_f32_step(const float* a, int lda, const float* w, int ldw, float* c, int ldc, int M, int N, int K,
+                                const float* gamma, float eps, int epilogue, const float* cosv, const float* sinv,
+                                const int32_t* slots, void* k_pages, void* v_pages, int nh, int nkv, int hd, int page_size,
+                                hipStream_t stream) {
+  GB_REQUIRE(N > 0 && K > 0 && step_takes(M, N, K, gamma != nullptr), "gemm_f32_step: not for M=%d N=%d K=%d", M, N, K);
+  GB_REQUIRE(epilogue == EPI_PLAIN || epilogue == EPI_UNIT || epilogue == EPI_HEADS, "gemm_f32_step: unknown epilogue %d", epilogue);
+  GB_REQUIRE(lda >= K && ldw >= K && ldc >= (epilogue == EPI_UNIT ? N / 2 : N), "gemm_f32_step: a leading dimension is shorter than its row (lda=%d ldw=%d ldc=%d)", lda, ldw, ldc);
+  GB_REQUIRE(words_of_16_bytes(a, lda) && words_of_16_bytes(w, ldw) && (uintptr_t)gamma % 16 == 0, "gemm_f32_step: rows of 16-byte words");
+  GB_REQUIRE(epilogue != EPI_HEADS || (hd >= 2 && hd % 2 == 0 && nh > 0 && nkv >= 0 && N == (nh + 2 * nkv) * hd && (cosv == nullptr) == (sinv == nullptr) &&
+                                       (!slots || (nkv > 0 && k_pages && v_pages && page_size > 0))),
+             "gemm_f32_step: N=%d is not (nh + 2 nkv) hd with nh=%d nkv=%d hd=%d, or pages or angles are missing", N, nh, nkv, hd);
+  const StepExtras ex{gamma, eps, cosv, sinv, slots, (float*)k_pages, (float*)v_pages, nh, nkv, hd, page_size};
+#define GB_STEP(MT, R, EPI)                                                                                                 \
+  if (epilogue == EPI && (M <= 1) == (MT == 1) && R == (N > kNarrow ? 16 : N > 4 * kTwoAUnit ? 8 : 4)) {                      \
+    if (gamma) launch_skinny<MT, R, EPI, true>(a, lda, w, ldw, c, ldc, M, N, K, 0, stream, ex);                             \
+    else launch_skinny<MT, R, EPI, false>(a, lda, w, ldw, c, ldc, M, N, K, 0, stream, ex);                                  \
+  }
+#define GB_STEPS(EPI) GB_STEP(1, 4, EPI) GB_STEP(1, 8, EPI) GB_STEP(1, 16, EPI) GB_STEP(2, 4, EPI) GB_STEP(2, 8, EPI) GB_STEP(2, 16, EPI)
+  GB_STEPS(EPI_PLAIN) GB_STEPS(EPI_UNIT) GB_STEPS(EPI_HEADS)
+#undef GB_STEPS
+#undef GB_STEP
+  return launched("gemm_f32 (step)");
+}
+
 // the launches of a layer can be recorded and made again for the layers like it (common.h)
+GB_TAPED(gb_gemm_f32_step)
 GB_TAPED(gb_gemm_f32)
 GB_TAPED(gb_gemm_f32_by)

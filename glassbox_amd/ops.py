@@ -201,6 +201,9 @@ _SIGS = {
     },
     "gemm_f32": {
         "gb_gemm_f32": [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _vp],
+        # a, lda, w, ldw, c, ldc, M, N, K, gamma, eps, epilogue, cos, sin, slots, k, v, nh, nkv, hd, page, stream
+        "gb_gemm_f32_step": [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _vp, _f, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
+        "gb_gemm_f32_step_takes": [_i, _i, _i, _i],
         "gb_gemm_f32_by": [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp],
     },
     "gemm_bf16": {
@@ -1645,6 +1648,53 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: 
 
 
 ROPE_PRODUCT_MAX_ROWS = 64
+
+
+STEP_F32_MAX_ROWS = 2   # gemm_f32.hip: rows of a step whose products take their neighbours' work (gb_gemm_f32_step)
+
+
+def step_f32_takes(M: int, N: int, K: int, norm: bool) -> bool:
+    """Whether ``gemm_step_f32`` takes a product of M rows by N rows of W of K columns, with the RMS norm before it or without."""
+    return M <= STEP_F32_MAX_ROWS and bool(_lib("gemm_f32").gb_gemm_f32_step_takes(M, N, K, 1 if norm else 0))
+
+
+def gemm_step_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms: Optional[tuple] = None, silu_mul: bool = False,
+                  heads: Optional[tuple] = None) -> None:
+    """A 32-bit product of one or two rows (``step_f32_takes``) with what stands around it, to the bits of the kernels that do
+    each by itself.  ``rms=(gamma, eps)``: a is the residual, its RMS-normed rows are multiplied.  ``silu_mul``: w stacks gate rows
+    over up rows, out holds silu(gate) * up.  ``heads=(n_heads, n_kv_heads, head_dim, cos, sin, slots, k_pages, v_pages)``: w stacks
+    query, key and value heads; queries and keys are turned as ``rope_store`` does (cos None: they are not) and keys and values
+    go to the pages at ``slots`` (None: nothing stored)."""
+    _dev(a, w, out)
+    M, K = a.shape
+    N = w.shape[0]
+    if any(t.dtype != torch.float32 for t in (a, w, out)) or w.shape[1] != K or out.shape != (M, N // 2 if silu_mul else N):
+        raise KernelError(f"gemm_step_f32: float32 of matching shapes: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
+    if not step_f32_takes(M, N, K, rms is not None) or (silu_mul and heads is not None):
+        raise KernelError(f"gemm_step_f32: not for {M} rows by {N} rows of {K} (step_f32_takes), or two epilogues at once")
+    gamma, eps = rms if rms is not None else (None, 0.0)
+    if gamma is not None and (gamma.dtype != torch.float32 or gamma.numel() != K or not gamma.is_contiguous()):
+        raise KernelError("gemm_step_f32: the norm takes a contiguous float32 gamma of K entries")
+    nh = nkv = hd = page_size = 0
+    cos = sin = slots = k_pages = v_pages = None
+    if heads is not None:
+        nh, nkv, hd, cos, sin, slots, k_pages, v_pages = heads
+        _dev(cos, sin, slots, k_pages, v_pages)
+        if N != (nh + 2 * nkv) * hd:
+            raise KernelError(f"gemm_step_f32: {N} rows of w are not ({nh} + 2 * {nkv}) heads of {hd}")
+        if slots is not None:
+            _i32(slots, "slots", M)
+            _, p_heads, page_size, p_hd = _check_pages(k_pages, v_pages, torch.float32, "gemm_step_f32")
+            if (p_heads, p_hd) != (nkv, hd):
+                raise KernelError("gemm_step_f32: pages do not have this layer's kv heads and head size")
+        if cos is not None and (sin is None or cos.shape[1] != hd // 2 or cos.shape[0] < M or cos.dtype != torch.float32
+                                or sin.dtype != torch.float32 or not cos.is_contiguous() or not sin.is_contiguous()
+                                or sin.shape != cos.shape):
+            raise KernelError("gemm_step_f32: cos/sin must be contiguous float32 [M, head_dim/2]")
+    lib = _lib("gemm_f32")
+    _launch(lib, lib.gb_gemm_f32_step, _p(a), _rows(a, "a"), _p(w), _rows(w, "w"), _p(out), _rows(out, "out"), M, N, K, _p(gamma),
+            float(eps), 2 if silu_mul else 3 if heads is not None else 0, _p(cos), _p(sin), _p(slots), _p(k_pages), _p(v_pages),
+            nh, nkv, hd, page_size, _stream())
 
 
 def gemm_rope(a: torch.Tensor, w: torch.Tensor, qkv: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,

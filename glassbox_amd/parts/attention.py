@@ -138,7 +138,22 @@ class PagedAttention(Mixer):
         if (ctx.dtype == torch.bfloat16 and ctx.fuse_norms and n <= ops.ROPE_PRODUCT_MAX_ROWS
                 and self.head_dim % 16 == 0):
             tables = self.position.fuse_spec(ctx, self.head_dim)
-        if tables is not None:
+        one_launch, takes = None, False   # 32-bit steps of one or two rows: norm, product, rotation and cache write in one
+        if ctx.dtype == torch.float32:
+            takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, norm is not None)
+            if norm is not None and not takes:   # nothing to fuse it into here: the norm gets its own pass after all
+                normed = ctx.buffer("h", (n, self.width), ctx.dtype)
+                ops.rmsnorm(h, norm[0], norm[1], normed)
+                h, norm = normed, None
+                takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, False)
+            if takes and self.head_dim % 2 == 0:
+                one_launch = self.position.fuse_spec(ctx, self.head_dim)
+        if one_launch is not None:
+            ops.gemm_step_f32(h, self.wqkv, qkv, rms=norm, heads=(self.n_heads, n_kv, self.head_dim, *one_launch, *store))
+        elif takes and norm is not None:
+            ops.gemm_step_f32(h, self.wqkv, qkv, rms=norm)
+            self.position.apply_and_store(ctx, qkv, self.n_heads, n_kv, self.head_dim, *store)
+        elif tables is not None:
             ops.gemm_rope(norm.rows if pre else h, self.wqkv, qkv, self.n_heads, n_kv, self.head_dim, tables[0],
                           tables[1], *store, rms=None if pre else norm, rms_parts=norm.as_gemm_arg() if pre else None)
         else:

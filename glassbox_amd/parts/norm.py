@@ -39,6 +39,8 @@ class RMSNorm(Norm):
     def load(self, tensors):
         w = tensors["weight"]
         self.weight = (w.float() + self.offset).contiguous() if self.offset else w.contiguous()
+        if self.weight.data_ptr() % 16:   # (a view into something larger: the kernels that norm on the way read whole words)
+            self.weight = self.weight.clone()
 
     def forward(self, ctx, x, rows=None, out_name="h"):
         m = x.shape[0] if rows is None else rows.numel()
@@ -53,9 +55,12 @@ class RMSNorm(Norm):
         return None
 
     def fuse_spec(self, ctx, n: int) -> Optional[Tuple[torch.Tensor, float]]:
-        """(gamma, eps) if the next matrix product may compute this norm itself: bfloat16 steps of
-        few rows, where a pass of its own costs more than the norm's arithmetic."""
+        """(gamma, eps) if the next matrix product may compute this norm itself: steps of few rows, where a pass of its own
+        costs more than the norm's arithmetic (of one or two in 32-bit, where the product may also refuse it:
+        ``ops.step_f32_takes``)."""
         if ctx.dtype == torch.bfloat16 and n <= ops.FUSED_NORM_MAX_ROWS and ctx.fuse_norms:
+            return (self.weight, self.eps)
+        if ctx.dtype == torch.float32 and n <= ops.STEP_F32_MAX_ROWS and ctx.fuse_norms and self.weight.dtype == torch.float32:
             return (self.weight, self.eps)
         return None
 

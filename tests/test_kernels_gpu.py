@@ -137,6 +137,61 @@ def test_gemm_f32_matrix_core_kernels_round_as_the_tiled_kernel_does(N, K, M):
             assert torch.equal(torch.nan_to_num(got[which], 0.25), torch.nan_to_num(got[1], 0.25)), which
 
 
+@pytest.mark.parametrize("M,K,inter,nh,nkv,hd", [
+    (1, 960, 2560, 15, 5, 64), (2, 576, 1536, 9, 3, 64),      # 16, 8 and 4 rows of W a workgroup
+    (1, 2560, 23, 3, 0, 2), (2, 1280, 1025, 2, 1, 6),         # the longest rows that a workgroup norms; pairs that a workgroup shares
+    (1, 4, 1, 1, 1, 20), (2, 252, 130, 5, 5, 100), (2, 260, 2049, 2, 1, 258), (1, 1028, 600, 33, 1, 64)])
+def test_gemm_step_f32_gives_the_bits_of_the_kernels_it_replaces(M, K, inter, nh, nkv, hd):
+    """Norm, product and gated unit, or norm, product, rotation and cache write, in one launch (csrc/hip/gemm_f32.hip,
+    StepExtras): the bits of the four kernels one after the other, with and without the norm, the angles and the pages."""
+    from glassbox_amd import ops
+    x, gamma = to_dev(rnd(M, K, seed=31) * 3), to_dev(rnd(K, seed=32))
+    wu, wh = to_dev(rnd(2 * inter, K, seed=33)), to_dev(rnd((nh + 2 * nkv) * hd, K, seed=34))
+    f32 = lambda *shape: torch.zeros(shape, dtype=torch.float32, device=DEV)
+    h = f32(M, K)
+    ops.rmsnorm(x, gamma, 1e-5, h)
+    pos = torch.tensor([5, 77][:M], dtype=torch.int32, device=DEV)
+    cos, sin = f32(M, hd // 2), f32(M, hd // 2)
+    ops.rope_table(pos, to_dev(rnd(hd // 2, seed=35).abs()), cos, sin)
+    slots = torch.tensor([18, 3][:M], dtype=torch.int32, device=DEV)
+    ran = 0
+    for rms in (None, (gamma, 1e-5)):
+        rows = h if rms else x
+        if ops.step_f32_takes(M, 2 * inter, K, rms is not None):
+            gu, want, got = f32(M, 2 * inter), f32(M, inter), f32(M, inter)
+            ops.gemm(rows, wu, gu)
+            ops.silu_mul(gu, want)
+            ops.gemm_step_f32(x, wu, got, rms=rms, silu_mul=True)
+            assert torch.equal(got, want)
+            ran += 1
+        if not ops.step_f32_takes(M, wh.shape[0], K, rms is not None):
+            continue
+        for angles in ((cos, sin), (None, None)):
+            for store in (True, False):
+                if store and nkv == 0:
+                    continue
+                outs = []
+                for fused in (False, True):
+                    qkv = f32(M, wh.shape[0])
+                    kp = torch.zeros(ops.key_pages_shape(2, max(nkv, 1), 16, hd), device=DEV)
+                    vp = f32(2, max(nkv, 1), hd, 16)
+                    place = (slots, kp, vp) if store else (None, None, None)
+                    if fused:
+                        ops.gemm_step_f32(x, wh, qkv, rms=rms, heads=(nh, nkv, hd, *angles, *place))
+                    else:
+                        ops.gemm(rows, wh, qkv)
+                        ops.rope_store(qkv, *angles, *place, nh, nkv, hd, rotate=angles[0] is not None)
+                    outs.append((qkv, kp, vp))
+                for got, want in zip(outs[1], outs[0]):
+                    assert torch.equal(got, want)
+                ran += 1
+    assert ran
+    # refused where it does not apply
+    assert not ops.step_f32_takes(M, 2, 2564 if M == 1 else 1284, True) and not ops.step_f32_takes(3, 64, 64, False)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_step_f32(to_dev(rnd(3, 64)), to_dev(rnd(8, 64)), f32(3, 8))
+
+
 def test_gemm_f32_takes_rows_that_are_no_words_of_16_bytes():
     """A k that is no multiple of 4, or operands that start in the middle of a word, go through the tiled kernel."""
     from glassbox_amd import ops
