@@ -28,7 +28,8 @@
 // request's tokens at consecutive positions (and no window moves their chunks apart) they read
 // the same keys and values, so a key or a word of values is loaded once and used for all eight,
 // each token's own sums being what they are in the other forms; other groups of eight (where one
-// request's rows end and the next one's begin) are walked one token after the other.
+// request's rows end and the next one's begin) are walked one token after the other.  The first two have a form for
+// 32-bit launches of few workgroups that asks for all a chunk needs at once (attention_plain_early_kernel).
 #include "common.h"
 
 using namespace gb;
@@ -38,7 +39,7 @@ GB_DEFINE_LAST_ERROR
 namespace {
 
 constexpr int kChunk = 256;
-constexpr int kEarlyPage = 16;   // chunk_alone's AHEAD form: pages of this size
+constexpr int kEarlyPage = 16;   // the early kernel's pages
 constexpr int kMaxOwn = 16;   // (dimension, word) pairs a thread owns at most: head size * page size <= 16,384
 
 struct Running {
@@ -70,11 +71,11 @@ template <> __device__ __forceinline__ void load_words<bf16>(const bf16* p, floa
 }
 
 // dot(q, key) in ascending dimension; the key lies in pieces of `piece` elements (key_offset)
-template <typename T, int UNROLL>
+template <typename T>
 __device__ __forceinline__ float key_dot(const float* qs, const T* kb, int slot, int hd, int page_size, int piece) {
   float dot = 0.f;
   if (piece == 8) {
-#pragma unroll UNROLL
+#pragma unroll 4
     for (int d0 = 0; d0 < hd; d0 += 8) {
       const T* kr = kb + ((size_t)(d0 / 8) * page_size + slot) * 8;
       float lo[4], hi[4];
@@ -129,10 +130,7 @@ struct Chunks {
 
 // One chunk by itself: keys c0 .. hi of the token's request.  Leaves m_c, l_c and the thread's sums a_c.
 // `qs` holds the query, `es` (kChunk floats) and `scratch` (17) are the block's.
-// AHEAD, for launches of few workgroups over contexts long enough (ahead_pays), with a pair a thread at most, pages of kEarlyPage and chunks that begin with a
-// page: the chunk's words of values are asked for before the scores, sixteen pages at once, where the loop below asks for four
-// at a time after them.  The sums are the same.
-template <typename T, int PER, bool AHEAD>
+template <typename T, int PER>
 __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, float* es, float* scratch,
                                             const int32_t* __restrict__ table, const T* __restrict__ k_pages,
                                             const T* __restrict__ v_pages, int kvh, float slope, int pos, int c0, int hi, float& m_c,
@@ -141,21 +139,11 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   const int ps = sh.page_size, hd = sh.hd;
   const int p = c0 + tid;
   const int words = ps / 4, pairs = hd * words;
-  static_assert(!AHEAD || PER == 1, "a thread's words of a chunk's pages are held in registers");
-  float ev[AHEAD ? kChunk / kEarlyPage : 1][4];
-  if (AHEAD && tid < pairs) {
-    const size_t at = (size_t)(tid / words) * ps + 4 * (tid % words);
-#pragma unroll
-    for (int i = 0; i < (AHEAD ? kChunk / kEarlyPage : 0); ++i) {   // (behind the last page: that page again, not used)
-      const int page = table[min(c0 + i * kEarlyPage, hi) / kEarlyPage];
-      load_words<T>(v_pages + ((size_t)page * sh.nkv + kvh) * hd * ps + at, ev[i]);
-    }
-  }
   float s = -INFINITY;
   if (p <= hi) {
     const int page = table[p / ps];
     const T* kb = k_pages + ((size_t)page * sh.nkv + kvh) * ps * hd;
-    s = sh.score(key_dot<T, AHEAD ? 8 : 4>(qs, kb, p % ps, hd, ps, key_piece(hd)), slope, pos - p);
+    s = sh.score(key_dot<T>(qs, kb, p % ps, hd, ps, key_piece(hd)), slope, pos - p);
   }
   m_c = block_max(s, scratch);
   const float e = p <= hi ? expf(s - m_c) : 0.f;
@@ -163,18 +151,6 @@ __device__ __forceinline__ void chunk_alone(const Shape& sh, const float* qs, fl
   l_c = block_sum(e, scratch);   // also orders the writes of es before the reads below
 #pragma unroll
   for (int u = 0; u < PER; ++u) a_c[u] = 0.f;
-  if constexpr (AHEAD) {
-    if (tid < pairs) {
-      const int p0 = c0 + 4 * (tid % words);
-#pragma unroll
-      for (int i = 0; i < (AHEAD ? kChunk / kEarlyPage : 0); ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (p0 + i * kEarlyPage + j <= hi) a_c[0] = fmaf(es[p0 - c0 + i * kEarlyPage + j], ev[i][j], a_c[0]);
-    }
-    __syncthreads();   // es is written again by the next chunk
-    return;
-  }
   const int pg_last = hi / ps;
 #pragma unroll 4
   for (int pg = c0 / ps; pg <= pg_last; ++pg) {
@@ -219,7 +195,7 @@ __device__ __forceinline__ void finish(const Shape& sh, float* comb, const float
 
 __device__ __forceinline__ int ws_stride(int per) { return per * kChunk + 2; }
 
-template <typename T, int PER, bool SPLIT, bool AHEAD>
+template <typename T, int PER, bool SPLIT>
 __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tables, const T* __restrict__ k_pages,
@@ -245,7 +221,7 @@ __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
   if (SPLIT) {
     const int c = blockIdx.y, c0 = ch.first(c);
     float m_c, l_c, a_c[PER];
-    chunk_alone<T, PER, AHEAD>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
+    chunk_alone<T, PER>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
     float* cell = ws + ((size_t)blockIdx.x * max_chunks + c) * ws_stride(PER);
 #pragma unroll
     for (int u = 0; u < PER; ++u) cell[u * kChunk + tid] = a_c[u];
@@ -262,10 +238,109 @@ __global__ __launch_bounds__(kChunk) void attention_plain_kernel(
   for (int c = 0; c < n_chunks; ++c) {
     const int c0 = ch.first(c);
     float m_c, l_c, a_c[PER];
-    chunk_alone<T, PER, AHEAD>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
+    chunk_alone<T, PER>(sh, qs, es, scratch, table, k_pages, v_pages, kvh, slope, pos, c0, ch.last(c, pos), m_c, l_c, a_c);
     merge_chunk<PER>(r, acc, m_c, l_c, a_c);
   }
   finish<T, PER>(sh, comb, acc, r, h, out + (size_t)t * out_stride + (size_t)h * sh.hd);
+}
+
+// ---- few workgroups: everything asked for at once ----------------------------------------------------------
+// A step of few tokens: its workgroups have a compute unit each, and what they take is the round trips to memory that wait for one
+// another.  So: a chunk's page numbers in one load (a lane a page), all words of a thread's key and all its words of
+// values at once, the query through the scalar unit, the waves' maxima and sums exchanged with one barrier each, the weights
+// of a word of slots as one LDS read.  The sums are those of chunk_alone.  Heads of 8 NP channels up to 64 (a (dimension, word)
+// pair a thread), pages of kEarlyPage, no window or runs: chunk c begins at key 256 c, with a page.
+// What bounded chunk_alone there (one request of 200 keys, cycles of 30,000): page numbers one at a time 8,000, a key's words two at
+// a time 6,000, a weight at a time out of LDS 6,000.  us a launch, heads of 64 (15 query, 5 key heads), replayed from a graph over
+// caches that no cache of the chip holds, before / with this: 100 keys 8.2 / 5.3, 200 keys 11.1 / 5.8, 600 keys in three chunks
+// 14.8 / 8.4, 1,000 keys 15.6 / 9.2.
+template <int NP, bool SPLIT>
+__global__ __launch_bounds__(kChunk) void attention_plain_early_kernel(
+    const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tables, const float* __restrict__ k_pages,
+    const float* __restrict__ v_pages, Shape sh, float* __restrict__ ws, int max_chunks) {
+  constexpr int HD = 8 * NP, PAGES = kChunk / kEarlyPage, WORDS = kEarlyPage / 4, PAIRS = HD * WORDS;
+  static_assert(PAIRS <= kChunk, "a pair a thread");
+  __shared__ __attribute__((aligned(16))) float es[kChunk];
+  __shared__ float most[kChunk / kWave], sums[kChunk / kWave], comb[PAIRS];
+  const int t = blockIdx.x / sh.nh, h = blockIdx.x % sh.nh;
+  const int kvh = h / (sh.nh / sh.nkv);
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int32_t* table = tables + (size_t)tok_seq[t] * sh.table_stride;
+  const float slope = sh.slope(h);
+  Running r{-INFINITY, 0.f};
+  float acc[1] = {0.f};
+  int c0 = SPLIT ? blockIdx.y * kChunk : 0;
+  // (asked for beside the position; what lies behind the token's pages is not used)
+  int pages = table[min(c0 / kEarlyPage + lane % PAGES, sh.table_stride - 1)];
+  const int pos = positions[t];
+  if (SPLIT && c0 > pos) return;
+  while (true) {   // (without SPLIT the rule below asks for one chunk; a context that is longer than it was said to be is walked)
+    const int hi = min(c0 + kChunk - 1, pos), last = hi / kEarlyPage - c0 / kEarlyPage;
+    f32x4 kw[2 * NP], vw[PAGES];
+    {
+      const int p = min(tid, hi - c0);   // (behind the last key: that key again, not used)
+      const float* kb = k_pages + ((size_t)__shfl(pages, p / kEarlyPage, kWave) * sh.nkv + kvh) * (kEarlyPage * HD) + p % kEarlyPage * 8;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        kw[2 * i] = *reinterpret_cast<const f32x4*>(kb + i * (kEarlyPage * 8));
+        kw[2 * i + 1] = *reinterpret_cast<const f32x4*>(kb + i * (kEarlyPage * 8) + 4);
+      }
+    }
+    const int own = min(tid, PAIRS - 1);
+#pragma unroll
+    for (int i = 0; i < PAGES; ++i) {
+      const int page = __builtin_amdgcn_readlane(pages, min(i, last));
+      vw[i] = *reinterpret_cast<const f32x4*>(v_pages + ((size_t)page * sh.nkv + kvh) * (HD * kEarlyPage) + own * 4);
+    }
+    const float* qh = q + (size_t)t * q_stride + (size_t)h * HD;   // (the same for every lane)
+    float dot = 0.f;
+#pragma unroll
+    for (int d = 0; d < HD; ++d) dot = fmaf(qh[d], kw[d / 4][d % 4], dot);
+    asm volatile("" : "+v"(dot));   // (or the loads of the keys would move behind those of the values, to where a lane needs its score)
+    const int p = c0 + tid;
+    const float s = p <= hi ? sh.score(dot, slope, pos - p) : -INFINITY;
+    const float m_w = wave_max(s);
+    if (lane == 0) most[wave] = m_w;
+    __syncthreads();
+    float m_c = most[0];
+#pragma unroll
+    for (int w = 1; w < kChunk / kWave; ++w) m_c = fmaxf(m_c, most[w]);
+    const float e = p <= hi ? expf(s - m_c) : 0.f;
+    es[tid] = e;
+    const float l_w = wave_sum(e);
+    if (lane == 0) sums[wave] = l_w;
+    __syncthreads();
+    float l_c = 0.f;
+#pragma unroll
+    for (int w = 0; w < kChunk / kWave; ++w) l_c += sums[w];
+    float a_c[1] = {0.f};
+    const int w0 = 4 * (own % WORDS);
+#pragma unroll
+    for (int i = 0; i < PAGES; ++i) {
+      const f32x4 e4 = *reinterpret_cast<const f32x4*>(&es[i * kEarlyPage + w0]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float next = fmaf(e4[j], vw[i][j], a_c[0]);
+        a_c[0] = c0 + i * kEarlyPage + w0 + j <= hi ? next : a_c[0];
+      }
+    }
+    if (SPLIT) {
+      float* cell = ws + ((size_t)blockIdx.x * max_chunks + blockIdx.y) * ws_stride(1);
+      cell[tid] = a_c[0];
+      if (tid == 0) {
+        cell[kChunk] = m_c;
+        cell[kChunk + 1] = l_c;
+      }
+      return;
+    }
+    merge_chunk<1>(r, acc, m_c, l_c, a_c);
+    c0 += kChunk;
+    if (c0 > pos) break;
+    pages = table[min(c0 / kEarlyPage + lane % PAGES, sh.table_stride - 1)];
+    __syncthreads();   // es, most and sums are written again
+  }
+  finish<float, 1>(sh, comb, acc, r, h, out + (size_t)t * out_stride + (size_t)h * HD);
 }
 
 // ---- several tokens a workgroup ------------------------------------------------------------------------------
@@ -476,7 +551,7 @@ __global__ __launch_bounds__(kChunk) void attention_plain_group_kernel(
     for (int c = 0; c < n_chunks; ++c) {
       const int c0 = ch.first(c);
       float m_c, l_c, a_c[PER];
-      chunk_alone<T, PER, false>(sh, qs + j * sh.hd, es, scratch + kGroup * 4, table, k_pages, v_pages, kvh, slope, pos, c0,
+      chunk_alone<T, PER>(sh, qs + j * sh.hd, es, scratch + kGroup * 4, table, k_pages, v_pages, kvh, slope, pos, c0,
                           ch.last(c, pos), m_c, l_c, a_c);
       merge_chunk<PER>(r, acc, m_c, l_c, a_c);
     }
@@ -516,19 +591,34 @@ inline int own_pairs(int hd, int page_size) {
   return 0;
 }
 
-// Where values are asked for ahead.  What it saves is a round trip to memory a chunk; what it costs are registers, and sixteen loads
-// whatever the chunk holds.  us, after / ahead, heads of 64, in 32-bit: one request of 1,000 keys, 15 heads, 13.5 / 13.0, eight of
-// 300 13.0 / 12.5, one of 256 10.6 / 9.9, of 200 9.7 / 9.7 (heads of 32 9.2 / 8.4), but of 100 7.6 / 9.5 and of 20 5.9 / 9.1; four chunks
-// each of 360, 432, 600 and 720 workgroups 20.6 / 19.2, 21.7 / 20.5, 23.1 / 22.9 and 24.3 / 24.9; 64 requests of 700 keys 56 / 62, eight
-// portions of 60 rows 44 / 64, 512 rows behind a window of 256 keys 101 / 140.  Not in bfloat16: 256 keys 10.5 / 10.2, 200 keys
-// 9.7 / 10.0, and the context that a captured step is launched for says little of those it has; nor where a workgroup
-// walks several chunks, of which the last may be short (16 rows of up to 300 keys 13.6 / 16.0).
-constexpr int kAheadGroups = 640, kAheadKeys = 200;
-template <typename T, int PER>
-constexpr bool kMayAhead = PER == 1 && sizeof(T) == 4;
-inline bool ahead_pays(const Shape& sh, bool spread, long long workgroups, int max_context) {
-  return sh.page_size == kEarlyPage && sh.window == 0 && sh.span == 0 && workgroups <= kAheadGroups && max_context >= kAheadKeys &&
-         (spread || max_context <= kChunk);
+// Where the early kernel pays: sixteen pages' words of values are loaded whatever a chunk holds, so where units have several
+// workgroups, contexts of 64 keys and more (us, chunk_alone / early: 15 workgroups of 20 keys 5.6 / 5.8, 240 of 20 and 33 keys
+// 6.3 / 6.1 and 7.3 / 6.3; 600 of 20, 48, 64 and 256 keys 7.6 / 8.6, 8.3 / 8.9, 9.2 / 9.2 and 19.3 / 15.9; 1,200 of 64 and 256
+// 14.8 / 13.8 and 38.5 / 26.3; 1,800, four chunks a request of 1,000 keys, 42.0 / 39.8).  Nor where a workgroup walks several
+// chunks, of which the last may be short.
+constexpr int kEarlyGroups = 2048, kEarlyAlone = 256, kEarlyKeys = 64, kEarlyAloneKeys = 32;
+inline bool early_pays(const Shape& sh, bool spread, long long workgroups, int max_context) {
+  return sh.page_size == kEarlyPage && sh.hd % 8 == 0 && sh.hd <= 64 && sh.window == 0 && sh.span == 0 && workgroups <= kEarlyGroups &&
+         max_context >= (workgroups <= kEarlyAlone ? kEarlyAloneKeys : kEarlyKeys) && (spread || max_context <= kChunk);
+}
+
+// The early kernel, if it is for these sizes (false: it is not).
+template <bool SPLIT>
+bool launch_early(const void* q, int q_stride, void* out, int out_stride, const int32_t* positions, const int32_t* tok_seq,
+                  const int32_t* tables, const void* k_pages, const void* v_pages, int n, const Shape& sh, float* ws, int max_chunks,
+                  int max_context, hipStream_t stream) {
+  if (!early_pays(sh, SPLIT, (long long)n * sh.nh * (SPLIT ? max_chunks : 1), max_context)) return false;
+  const dim3 grid((unsigned)(n * sh.nh), SPLIT ? (unsigned)max_chunks : 1u);
+  switch (sh.hd / 8) {
+#define GB_EARLY(NP)                                                                                                             \
+  case NP:                                                                                                                       \
+    hipLaunchKernelGGL((attention_plain_early_kernel<NP, SPLIT>), grid, dim3(kChunk), 0, stream, (const float*)q, q_stride, (float*)out, \
+                       out_stride, positions, tok_seq, tables, (const float*)k_pages, (const float*)v_pages, sh, ws, max_chunks); \
+    return true;
+    GB_EARLY(1) GB_EARLY(2) GB_EARLY(3) GB_EARLY(4) GB_EARLY(5) GB_EARLY(6) GB_EARLY(7) GB_EARLY(8)
+#undef GB_EARLY
+  }
+  return false;
 }
 
 template <typename T, int PER>
@@ -537,12 +627,13 @@ void launch(const void* q, int q_stride, void* out, int out_stride, const int32_
             int max_chunks, int max_context, bool grouped_form, hipStream_t stream) {
   const size_t comb = sizeof(float) * sh.hd * (sh.page_size / 4);
   const size_t smem = sizeof(float) * (sh.hd + kChunk + 17) + comb;
-  const bool ahead = kMayAhead<T, PER> && ahead_pays(sh, ws != nullptr, (long long)n * sh.nh * (ws != nullptr ? max_chunks : 1), max_context);
+  constexpr bool EARLY = PER == 1 && sizeof(T) == 4;
   if (ws != nullptr) {
-    const auto kernel = ahead ? attention_plain_kernel<T, PER, true, kMayAhead<T, PER>> : attention_plain_kernel<T, PER, true, false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(n * sh.nh), (unsigned)max_chunks), dim3(kChunk),
-                       smem, stream, (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables,
-                       (const T*)k_pages, (const T*)v_pages, sh, ws, max_chunks);
+    if (!EARLY || !launch_early<true>(q, q_stride, out, out_stride, positions, tok_seq, tables, k_pages, v_pages, n, sh, ws, max_chunks,
+                                      max_context, stream))
+      hipLaunchKernelGGL((attention_plain_kernel<T, PER, true>), dim3((unsigned)(n * sh.nh), (unsigned)max_chunks), dim3(kChunk),
+                         smem, stream, (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables,
+                         (const T*)k_pages, (const T*)v_pages, sh, ws, max_chunks);
     hipLaunchKernelGGL((attention_plain_merge_kernel<T, PER>), dim3((unsigned)(n * sh.nh)), dim3(kChunk), comb, stream,
                        (T*)out, out_stride, positions, sh, (const float*)ws, max_chunks);
   } else if (grouped_form && PER <= kGroupMaxOwn && sh.window == 0 && sh.span == 0) {   // (elsewhere the one-token form: the same bits)
@@ -553,9 +644,9 @@ void launch(const void* q, int q_stride, void* out, int out_stride, const int32_
                          (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables, (const T*)k_pages,
                          (const T*)v_pages, sh, n);
     }
-  } else {
-    const auto kernel = ahead ? attention_plain_kernel<T, PER, false, kMayAhead<T, PER>> : attention_plain_kernel<T, PER, false, false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(n * sh.nh)), dim3(kChunk), smem, stream,
+  } else if (!EARLY || !launch_early<false>(q, q_stride, out, out_stride, positions, tok_seq, tables, k_pages, v_pages, n, sh, nullptr, 0,
+                                            max_context, stream)) {
+    hipLaunchKernelGGL((attention_plain_kernel<T, PER, false>), dim3((unsigned)(n * sh.nh)), dim3(kChunk), smem, stream,
                        (const T*)q, q_stride, (T*)out, out_stride, positions, tok_seq, tables, (const T*)k_pages,
                        (const T*)v_pages, sh, nullptr, 0);
   }

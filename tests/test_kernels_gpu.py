@@ -940,6 +940,35 @@ def test_attention_plain_asks_for_values_ahead_where_workgroups_are_few(dtype, n
         assert torch.equal(rows(count, spread=True), few[[i % n for i in range(count)]])
 
 
+@pytest.mark.parametrize("hd", [8, 16, 24, 40, 48, 56, 64])
+def test_attention_plain_of_few_workgroups_gives_the_bits_of_the_walk(hd):
+    """The kernel that asks for a chunk's keys and values at once (attention_plain_early_kernel), one workgroup a row and a
+    workgroup a chunk: chunks that end around a page and around 256 keys, a cap and slopes and sinks; and a context that is longer
+    than the launch was told.  The same bits as the walk (no longest context given)."""
+    from glassbox_amd import ops
+    nh, nkv = 6, 2
+    ctx_lens = [1, 15, 16, 17, 64, 241, 255, 256, 257, 272, 511, 600]
+    k_pages, v_pages, tables, ks, vs = paged_setup(ctx_lens, nkv, hd, 16, seed=hd, dtype=torch.float32)
+    n, scale = len(ctx_lens), 1 / math.sqrt(hd)
+    q, pos, seq = to_dev(rnd(n, nh * hd, seed=3)), torch.tensor([c - 1 for c in ctx_lens], dtype=torch.int32, device=DEV), \
+        torch.arange(n, dtype=torch.int32, device=DEV)
+    args = (pos, seq, to_dev(tables), to_dev(ops.pack_keys(k_pages)), to_dev(v_pages), nh, scale, 0)
+    for more in ({}, dict(softcap=5.0), dict(slopes=to_dev(rnd(nh, seed=4).abs() * 0.1), sinks=to_dev(rnd(nh, seed=5)))):
+        def out(**kw):
+            o = torch.full((n, nh * hd), 7.0, device=DEV)
+            ops.attention_plain(q, o, *args, **more, **kw)
+            return o
+        walk = out()
+        floats = ops.attention_plain_split_floats(n, nh, hd, 16, 600)
+        assert floats > 0
+        assert torch.equal(out(max_context=256), walk)
+        assert torch.equal(out(max_context=600, workspace=torch.full((floats,), float("nan"), device=DEV)), walk)
+    want = plain_attention_rows(q.cpu(), ks, vs, list(range(n)), [c - 1 for c in ctx_lens], nh, scale, 0)
+    o = torch.empty(n, nh * hd, device=DEV)
+    ops.attention_plain(q, o, *args, max_context=256)
+    assert (o.cpu().double() - want).abs().max().item() < 2e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,page", [(4, 2, 16, 16), (8, 8, 64, 16), (3, 1, 32, 48), (2, 1, 128, 32), (2, 2, 256, 16),
                                             (5, 5, 80, 64)])
