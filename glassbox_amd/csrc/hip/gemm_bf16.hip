@@ -3,7 +3,7 @@
 // (crates/glassbox-core/src/kernels.rs:381,586).  Both operands are contiguous along k, which
 // is the layout MFMA operands want: every lane loads 8 consecutive k as one 16-byte word.
 //
-// Five kernels:
+// Six kernels:
 //  * tiled  (M > 64, prompt portions): a workgroup of 2x2 waves, each wave a block of 2x2 or 2x1
 //    v_mfma_f32_32x32x16_bf16 tiles (workgroup tile 128x128 or 128x64; 64 rows high where the taller tiles would be
 //    few), operands staged through LDS in k-steps of 64 with two buffers; the SiLU-multiply of stacked gate/up rows
@@ -19,6 +19,8 @@
 //    through LDS in a fixed order; it can norm float32 rows on the way, apply the SiLU-multiply, or
 //    (the QKV product) rotate the heads and write the key/value cache, or prepare the next norm where it adds
 //    into the residual.
+//  * held   (17 to 64 rows by many rows of W, decode steps of a busy server): a workgroup a compute unit holds the rows of
+//    A in registers and streams tiles of W through LDS.
 //  * folded (M <= 8 and few rows of W): the skinny kernel with two k ranges side by side in a tile,
 //    so that a workgroup owns 8 rows of W and there are twice as many workgroups.
 // In all, every output cell is summed in an order fixed by (K, kernel) alone, not by M or by
@@ -1015,6 +1017,309 @@ int launch_stream(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc
   return launched("gemm_bf16 (stream)");
 }
 
+// ------------------------------------------------------------------------- held
+// Products of 17 to 64 rows that read a large W (decode steps of a busy server: gate/up, QKV, the vocabulary).  W is what
+// they cost; but the skinny kernel reads all of A again in every workgroup, in front of the stream of W, and asks for W
+// in half lines.  Here a workgroup for every compute unit holds the rows of A in registers (a wave the k-blocks that are
+// its own: block b of 64 belongs to wave b % 8, MT x NB x 8 registers) and walks over several tiles of 16 rows of W.  A
+// wave brings its blocks of W from memory straight into a ring of its own in LDS (whole lines of 128 bytes, nontemporal,
+// five or six blocks of 2 KB: 80 or 96 KB on their way a compute unit) and takes them as MFMA operands from there: no barrier stands
+// between a load and its use, and the ring runs on over the ends of tiles.  The eight waves' sums of a tile meet in LDS
+// (two buffers, one barrier a tile); one wave adds them in the waves' order and finishes, the waves taking turns.
+//
+// MFMA row 4 q + e of a tile is such that a lane holds what the epilogue joins: with EPI_SILU_MUL e = 0, 1 are gate rows
+// and e = 2, 3 the up rows that belong to them, with EPI_ROPE the two halves of two pairs.
+//
+// The memory counter: loads and stores retire in the order of issue, so waiting for all but the youngest 2 (HS - 1)
+// means that a block has landed once HS - 1 blocks were asked for behind it, whatever else was issued in between.
+// The sums go through LDS by inline assembly: the compiler would wait for every load into LDS before an access of its own.
+constexpr int HWAVES = 8, HBLOCK = 16 * 64;   // waves, elements of a block
+__device__ __forceinline__ f32x4 lds_read_f4(uint32_t addr) {
+  f32x4 v;
+  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
+  return v;
+}
+
+template <int MT, int NB, int EPI, typename CT>
+__global__ __launch_bounds__(HWAVES * 64, 1) void gemm_held_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w,
+                                                                   int ldw, CT* __restrict__ c, int ldc, int M, int N, int K,
+                                                                   int k_slice, int tiles, float eps, const float* __restrict__ parts,
+                                                                   int n_parts, RopeExtras rope) {
+  constexpr int HS = MT == 4 ? 5 : 6;   // blocks of a wave's ring
+  constexpr int TURNS = MT == 3 ? 4 : MT, EVERY = HWAVES / TURNS;   // a wave finishes column block wave % TURNS of every EVERY-th tile
+  __shared__ __attribute__((aligned(16))) bf16 ring[HWAVES][HS][HBLOCK];
+  __shared__ __attribute__((aligned(16))) float part[2][HWAVES][MT][64][4];
+  __shared__ float squares[HWAVES][64];   // of each row, a wave's share of the partial sums
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int r = lane % 16, q = lane / 16;
+  const int full_k = K;
+  if (k_slice > 0) {   // workgroups (.., z) sum slice z of k into their own copy of C
+    const int z = blockIdx.y;
+    a += (size_t)z * k_slice;
+    w += (size_t)z * k_slice;
+    c += (size_t)z * M * ldc;
+    K = min(k_slice, K - z * k_slice);
+  }
+  const int stride = gridDim.x, mine = (tiles - (int)blockIdx.x + stride - 1) / stride;   // tiles of the workgroup
+  const int nb = (K / 64 - wave + HWAVES - 1) / HWAVES;   // k-blocks of the wave
+
+  // ---- the stream of W: a load of the wave brings 8 rows of a block, 128 bytes each; piece p of row i lies at p ^ (i & 7)
+  auto w_row = [&](int tile, int i) -> int {   // row of W behind MFMA row i of a tile
+    const int j = 2 * (i / 4) + (i & 1);
+    if (EPI == EPI_SILU_MUL) return min(tile * 8 + j, N / 2 - 1) + ((i & 2) ? N / 2 : 0);
+    if (EPI == EPI_ROPE) {
+      const int per_head = rope.hd / 16, head = tile / per_head, d0 = tile % per_head * 8;
+      return head * rope.hd + d0 + j + ((i & 2) ? rope.hd / 2 : 0);
+    }
+    return min(tile * 16 + i, N - 1);
+  };
+  // (Through the ring come first the wave's blocks of A, a column block's after the other's, then those of W.)
+  const bf16* src[2];
+  int at_cols = 0, at_tile = blockIdx.x, at_block = 0, slot_in = 0, asked = 0;
+  const int a_blocks = nb * MT, total = a_blocks + mine * nb;
+  auto aim = [&](bool of_a) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = u * 8 + lane / 8, k = wave * 64 + ((lane % 8) ^ (i & 7)) * 8;
+      if (of_a) src[u] = a + (size_t)min(at_cols * 16 + i, M - 1) * lda + k;
+      else src[u] = w + (size_t)w_row(at_tile, i) * ldw + k;
+    }
+  };
+  auto bring = [&](bool of_a) {
+    const int col = at_block * (HWAVES * 64);
+    if (of_a) {
+      __builtin_amdgcn_global_load_lds((glb_void*)(src[0] + col), (lds_void*)&ring[wave][slot_in][0], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void*)(src[1] + col), (lds_void*)&ring[wave][slot_in][512], 16, 0, 0);
+    } else {   // nontemporal: W is read once, in whole lines
+      __builtin_amdgcn_global_load_lds((glb_void*)(src[0] + col), (lds_void*)&ring[wave][slot_in][0], 16, 0, 2);
+      __builtin_amdgcn_global_load_lds((glb_void*)(src[1] + col), (lds_void*)&ring[wave][slot_in][512], 16, 0, 2);
+    }
+    slot_in = slot_in + 1 == HS ? 0 : slot_in + 1;
+    ++asked;
+    if (++at_block == nb) {
+      at_block = 0;
+      if (of_a) ++at_cols;
+      else at_tile += stride;
+    }
+  };
+  auto ask = [&]() {
+    const bool of_a = asked < a_blocks;
+    if (at_block == 0) aim(of_a);
+    bring(of_a);
+  };
+  auto ask_w = [&]() {   // once every block of A has been asked for
+    if (at_block == 0) aim(false);
+    bring(false);
+  };
+  // A norm before the product: its partial sums of squares, row `lane`'s, every eighth a wave; asked for ahead of the ring.
+  constexpr int PARTS_AT_ONCE = 32;
+  float got[PARTS_AT_ONCE];
+  if (parts != nullptr) {
+#pragma unroll
+    for (int u = 0; u < PARTS_AT_ONCE; ++u) {
+      const int p = wave + u * HWAVES;
+      got[u] = lane < M && p < n_parts ? parts[(size_t)p * 64 + lane] : 0.f;
+    }
+  }
+#pragma unroll 1
+  for (int s = 0; s < HS && s < total; ++s) ask();
+  if (parts != nullptr) {
+    float sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < PARTS_AT_ONCE; ++u) sum += got[u];
+    for (int p = wave + PARTS_AT_ONCE * HWAVES; p < n_parts; p += HWAVES) sum += lane < M ? parts[(size_t)p * 64 + lane] : 0.f;
+    // (read behind the first tile's barrier)
+    asm volatile("ds_write_b32 %0, %1" ::"v"((uint32_t)(uintptr_t)(lds_void*)&squares[wave][lane]), "v"(sum) : "memory");
+  }
+
+  // ---- what the wave's turns at finishing will need
+  const int t_mine = wave % TURNS, m_mine = t_mine * 16 + r;
+  const bool row_mine = t_mine < MT && m_mine < M;
+  float scale = 1.f;
+  float cs[2] = {1.f, 1.f}, sn[2] = {0.f, 0.f};
+  int slot = 0;
+  if constexpr (EPI == EPI_ROPE) {   // (at most EVERY tiles a workgroup: one turn a wave)
+    const int tile = blockIdx.x + wave / TURNS * stride, per_head = rope.hd / 16;
+    if (row_mine && wave / TURNS < mine) {
+      if (rope.slots) slot = rope.slots[m_mine];
+      if (rope.cosv && tile / per_head < rope.nh + rope.nkv) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const size_t at = (size_t)m_mine * (rope.hd / 2) + tile % per_head * 8 + 2 * q + e;
+          cs[e] = rope.cosv[at], sn[e] = rope.sinv[at];
+        }
+      }
+    }
+  }
+  // ---- the tiles
+  const uint32_t ring_base = (uint32_t)(uintptr_t)(lds_void*)&ring[wave][0][0];
+  const uint32_t part_base = (uint32_t)(uintptr_t)(lds_void*)&part[0][0][0][0][0];
+  uint32_t off[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) off[h] = 2 * (r * 64 + ((4 * h + q) ^ (r & 7)) * 8);
+  int slot_out = 0, left = total;   // blocks not yet taken
+  auto take = [&](bf16x8 (&f)[2]) {   // the next block of the ring as an operand: its place is free then
+    if (left >= HS) vm_wait<2 * (HS - 1)>();
+    else vm_wait<0>();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) f[h] = lds_read16(ring_base + slot_out * (2 * HBLOCK) + off[h]);
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[0]), "+v"(f[1])::"memory");
+    slot_out = slot_out + 1 == HS ? 0 : slot_out + 1;
+    --left;
+  };
+  bf16x8 fa[MT][NB][2];   // (rows behind M are a row that exists: what comes of them is not stored)
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (i < nb) {
+        take(fa[t][i]);
+        if (asked < total) ask();
+      }
+#pragma unroll 1
+  for (int ti = 0; ti < mine; ++ti) {
+    f32x4 acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (i < nb) {
+        bf16x8 fw[2];
+        take(fw);
+        if (asked < total) ask_w();
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[h], fa[t][i][h], acc[t], 0, 0, 0);
+      }
+    }
+    const uint32_t buf = part_base + (uint32_t)((ti & 1) * (HWAVES * MT * 1024) + lane * 16);
+    // (the MFMAs' results: the compiler does not know the assembly below to read them out of the registers at once)
+    static_assert(MT >= 2 && MT <= 4, "the wait names every column block's sums");
+    if constexpr (MT == 2) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]));
+    else if constexpr (MT == 3) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]));
+    else asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+#pragma unroll
+    for (int t = 0; t < MT; ++t) asm volatile("ds_write_b128 %0, %1" ::"v"(buf + (uint32_t)((wave * MT + t) * 1024)), "v"(acc[t]) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (t_mine >= MT || ti % EVERY != wave / TURNS) continue;
+    // D[n, m]: the lane holds column m = r and rows 4 q + e
+    f32x4 p[HWAVES];
+#pragma unroll
+    for (int wv = 0; wv < HWAVES; ++wv) p[wv] = lds_read_f4(buf + (uint32_t)((wv * MT + t_mine) * 1024));
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7])::"memory");
+    static_assert(HWAVES == 8, "the wait names the eight waves' sums");
+    f32x4 v = p[0];
+#pragma unroll
+    for (int wv = 1; wv < HWAVES; ++wv) v += p[wv];
+    if (parts != nullptr) {
+      if (ti < EVERY) {   // the wave's first turn
+        float sq[HWAVES];
+#pragma unroll
+        for (int wv = 0; wv < HWAVES; ++wv)
+          asm volatile("ds_read_b32 %0, %1" : "=v"(sq[wv]) : "v"((uint32_t)(uintptr_t)(lds_void*)&squares[wv][t_mine * 16 + r]) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(sq[0]), "+v"(sq[1]), "+v"(sq[2]), "+v"(sq[3]), "+v"(sq[4]), "+v"(sq[5]), "+v"(sq[6]), "+v"(sq[7])::"memory");
+        float sum = sq[0];
+#pragma unroll
+        for (int wv = 1; wv < HWAVES; ++wv) sum += sq[wv];
+        scale = 1.0f / sqrtf(sum / (float)full_k + eps);
+      }
+      v *= scale;
+    }
+    if (row_mine) {
+      const int tile = blockIdx.x + ti * stride;
+      if constexpr (EPI == EPI_SILU_MUL) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int j = tile * 8 + 2 * q + e;
+          if (j < N / 2) c[(size_t)m_mine * ldc + j] = (CT)gated_unit(v[e], v[2 + e], Glu{});
+        }
+      } else if constexpr (EPI == EPI_ROPE) {
+        const int per_head = rope.hd / 16, head = tile / per_head, dim0 = tile % per_head * 8 + 2 * q, half = rope.hd / 2;
+        const bool is_value = head >= rope.nh + rope.nkv;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          // (a product of its own each, as the skinny kernel's)
+          const float lo = is_value || !rope.cosv ? v[e] : v[e] * cs[e] - v[2 + e] * sn[e];
+          const float hi = is_value || !rope.cosv ? v[2 + e] : v[2 + e] * cs[e] + v[e] * sn[e];
+#pragma unroll
+          for (int up = 0; up < 2; ++up) {
+            const bf16 y = (bf16)(up ? hi : lo);
+            const int dim = dim0 + e + up * half;
+            c[(size_t)m_mine * ldc + head * rope.hd + dim] = (CT)y;
+            if (rope.slots != nullptr && head >= rope.nh) {
+              const int page = slot / rope.page_size, at = slot % rope.page_size;
+              if (!is_value)
+                rope.k_pages[((size_t)page * rope.nkv + (head - rope.nh)) * rope.page_size * rope.hd + key_offset(at, dim, rope.page_size, 8)] = y;
+              else
+                rope.v_pages[(((size_t)page * rope.nkv + (head - rope.nh - rope.nkv)) * rope.hd + dim) * rope.page_size + at] = y;
+            }
+          }
+        }
+      } else {
+        CT* to = c + (size_t)m_mine * ldc + tile * 16 + 4 * q;
+        if (tile * 16 + 16 <= N && ldc % 4 == 0 && (uintptr_t)c % (4 * sizeof(CT)) == 0) {
+          store_c4<CT>(to, v);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (tile * 16 + 4 * q + e < N) to[e] = (CT)v[e];
+        }
+      }
+    }
+  }
+}
+
+// Column blocks of 16 rows of A times k-blocks a wave: what fits the registers (MT x NB x 8 of them for A).
+inline int held_blocks(int K) { return (K / 64 + HWAVES - 1) / HWAVES; }
+inline bool held_takes(const void* a, int lda, const void* w, int ldw, int M, int K) {
+  return M > 16 && M <= 64 && K % 64 == 0 && held_blocks(K) <= (M <= 32 ? 8 : 4) && lda % 8 == 0 && ldw % 8 == 0 &&
+         (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
+}
+// Workgroups: as many as share the tiles evenly, at most one a compute unit (times the slices of k).
+inline int held_groups(int tiles, int slices) {
+  const int room = 256 / slices, each = (tiles + room - 1) / room;
+  return (tiles + each - 1) / each;
+}
+// Where it pays (us, the skinny kernel, the wide tiles or the stream kernel before / this one, each product alone):
+//   gate/up 28,672 x 4,096, 17 / 24 / 32 rows: 53 / 57 / 62 -> 42 / 45 / 45 (5.2 to 5.5 TB/s); vocabulary 128,256 x 4,096,
+//   24 rows: 242 -> 176 (6 TB/s); gate/up 16,384 x 2,048, 20 / 33 / 64 rows: 19 / 21.6 / 20.8 -> 15.7 / 17 / 18; gate/up 5,120 x 960
+//   behind partial sums of a norm, 20 / 53 rows: 8.6 / 12.5 -> 8.2 / 8.8; QKV 6,144 x 4,096, 24 rows 17.2 -> 15.3; 6,144 x 2,048,
+//   20 / 64 rows 11.2 / 16.7 -> 10.3 / 13.3.
+// Few tiles: a workgroup's rows of A are then more than its rows of W, and where a k of 960 is one block each for the sixteen waves of the
+// skinny kernel, those bring both as fast (QKV 1,600 x 960, 100 tiles, 53 rows: 6.6 -> 7.1; 3,072 x 960 with the unit, 192 tiles, 33 rows
+// 5.7 -> 5.9; 4,096 x 960 5.7 -> 5.7; a storing product of 160 tiles, which goes there in halves, 33 rows: 6.2 -> 5.5, of 128 tiles 4.6 ->
+// 5.4).  A longer k is several round trips there: from 2,048 on this one is ahead at 128 tiles (33 rows 8.7 -> 6.9, in slices of k before;
+// 17 rows 6.4 -> 5.8).  Of a k below 768 those are four waves, and this one's eight are ahead (960 x 576, 60 tiles, 53 rows: 7.1 -> 6.2).
+inline int held_tiles(int epi, int N) { return epi == EPI_SILU_MUL ? (N / 2 + 7) / 8 : (N + 15) / 16; }
+inline bool held_pays(int epi, int M, int N, int K) {
+  const int tiles = held_tiles(epi, N);
+  if (epi == EPI_ROPE) {   // a wave prepares one turn at finishing
+    const int groups = held_groups(tiles, 1);
+    if ((tiles + groups - 1) / groups > HWAVES / (M <= 32 ? 2 : 4)) return false;
+  }
+  return tiles >= (K < 768 ? 60 : K >= 2048 ? 128 : epi == EPI_STORE ? 160 : 257);
+}
+template <int EPI, typename CT>
+int launch_held(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice, int slices, float eps,
+                const float* parts, int n_parts, hipStream_t stream, const RopeExtras& rope = RopeExtras{}) {
+  const int tiles = held_tiles(EPI, N), mt = (M + 15) / 16;
+  const int nb = held_blocks(slices > 1 ? k_slice : K);
+  const dim3 grid(held_groups(tiles, slices), slices), block(HWAVES * 64);
+#define GB_H(MT, NB, FROM)                                                                                                      \
+  if (mt == (MT) && nb > (FROM) && nb <= (NB)) {                                                                                \
+    hipLaunchKernelGGL((gemm_held_kernel<(MT), (NB), EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, N, K,          \
+                       slices > 1 ? k_slice : 0, tiles, eps, parts, n_parts, rope);                                             \
+    return launched("gemm_bf16 (held)");                                                                                        \
+  }
+  GB_H(2, 2, 0) GB_H(2, 4, 2) GB_H(2, 8, 4) GB_H(3, 2, 0) GB_H(3, 4, 2) GB_H(4, 2, 0) GB_H(4, 4, 2)
+#undef GB_H
+  return fail("gemm_bf16 (held): %d rows by a k of %d do not fit the registers", M, K);
+}
+
 // ------------------------------------------------------------------------ split k
 // A product with few tiles (17 to a few hundred rows, or few rows of W) leaves most compute units idle
 // and, as a skinny product, makes every workgroup read all of A.  Here the tiled kernel's workgroups
@@ -1909,6 +2214,7 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
   const NormExtras extra{emit_gamma, emit_gamma_dtype == kF32, (bf16*)emit_h, emit_ldh, emit_ss, parts, n_parts};
   if (M == 0) return 0;
   const bf16* W = (const bf16*)w;
+  const bool held = !gamma && !emit_h && epilogue != EPI_ACCUMULATE && held_pays(epilogue, M, N, K) && held_takes(a, lda, w, ldw, M, K);
   if (split_ws != nullptr && M > 16 && !gamma && (!emit_h || emits == 2) && !parts) {  // more than the skinny kernels' best range
     const SplitPlan plan = split_plan(M, N, K, epilogue == EPI_SILU_MUL);
     if (plan.slices > 1 && (epilogue != EPI_SILU_MUL || N % 16 == 0) && (uintptr_t)split_ws % 16 == 0) {
@@ -1918,12 +2224,23 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
 #define GB_SP(EPI, CT) return launch_split<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, split_ws, plan, stream)
       if (epilogue == EPI_ACCUMULATE)
         return launch_split<EPI_ACCUMULATE, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, split_ws, plan, stream, &extra, eps);
-      if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_SP(EPI_SILU_MUL, bf16);
-      if (epilogue == EPI_SILU_MUL) GB_SP(EPI_SILU_MUL, float);
-      if (c_dtype == kF32) GB_SP(EPI_STORE, float);
-      GB_SP(EPI_STORE, bf16);
+      if (!held) {
+        if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_SP(EPI_SILU_MUL, bf16);
+        if (epilogue == EPI_SILU_MUL) GB_SP(EPI_SILU_MUL, float);
+        if (c_dtype == kF32) GB_SP(EPI_STORE, float);
+        GB_SP(EPI_STORE, bf16);
+      }
 #undef GB_SP
     }
+  }
+  if (held) {
+    const bf16* A = (const bf16*)a;
+#define GB_HD(EPI, CT) return launch_held<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream)
+    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_HD(EPI_SILU_MUL, bf16);
+    if (epilogue == EPI_SILU_MUL) GB_HD(EPI_SILU_MUL, float);
+    if (c_dtype == kF32) GB_HD(EPI_STORE, float);
+    GB_HD(EPI_STORE, bf16);
+#undef GB_HD
   }
   // The narrow tiles without slices: up to 128 rows wherever they give half the compute units a workgroup (with a
   // long enough k the plan above has divided it instead); up to 256 rows where the wide tiles would be few and k is
@@ -1942,7 +2259,7 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
     GB_ST(EPI_STORE, bf16);
 #undef GB_ST
   }
-  // 17 to 64 rows by very many rows of W (the vocabulary product of a large decode batch): measured twice as fast
+  // 17 to 64 rows by very many rows of W that the held kernel does not take (a long k): measured twice as fast
   // through the tiles below as through the skinny kernel with four column blocks (49,152 x 2,048: 102 -> about 50 us),
   // and with two column blocks as fast or faster (49,152 x 960 at 17 to 32 rows: 30 -> 25 us)
   const bool wide_head = M > 16 && N >= 32768 && !gamma && !parts;
@@ -2078,6 +2395,8 @@ extern "C" int gb_gemm_bf16_rope(const void* a, int lda, const void* w, int ldw,
   GB_REQUIRE(!parts || n_parts > 0, "gemm_bf16_rope: partial sums of a norm without a count");
   const NormExtras extra{nullptr, 0, nullptr, 0, nullptr, parts, n_parts};
   const RopeExtras rope{cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, 0};
+  if (!gamma && held_pays(EPI_ROPE, M, N, K) && held_takes(a, lda, w, ldw, M, K))
+    return launch_held<EPI_ROPE, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream, rope);
   if (gamma)
     return launch_skinny<EPI_ROPE, true, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, gamma, gamma_dtype == kF32,
                                                eps, extra, stream, rope);

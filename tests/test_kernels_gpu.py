@@ -570,6 +570,49 @@ def test_gemm_bf16_streams_products_of_some_hundred_rows(M, N, K, mode):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 2056, 64), (32, 2050, 576), (33, 2048, 960), (48, 8250, 1984), (49, 4112, 2048), (64, 5120, 960),
+                                   # a wave's most blocks of k; tiles that do not divide among the workgroups; a short k and few tiles
+                                   (24, 8240, 4096), (31, 33000, 448), (20, 976, 128), (64, 960, 704), (17, 6152, 2112)])
+@pytest.mark.parametrize("mode", ["bf16", "f32", "silu", "parts", "padded"])
+def test_gemm_bf16_holds_the_rows_and_streams_w(M, N, K, mode):
+    """17 to 64 rows by many rows of W, held in the registers of a workgroup for every compute unit: against the product in
+    float64, alone, with the gated unit, behind the partial sums of a norm, and into rows that are no whole words."""
+    from glassbox_amd import ops
+    a, w = rnd(M, K, seed=M).bfloat16(), (rnd(N, K, seed=N) / math.sqrt(K)).bfloat16()
+    prod = a.double() @ w.double().T
+    scale, parts = None, None
+    if mode == "parts":
+        n, eps = 75, 1e-5
+        parts = rnd(n, 64, seed=5).abs().float() + 0.1
+        prod = prod / torch.sqrt(parts[:, :M].double().sum(0) / K + eps).unsqueeze(1)
+        parts = (to_dev(parts), n, eps)
+    silu = mode in ("silu", "parts") and N % 16 == 0
+    want = prod if not silu else prod[:, :N // 2] / (1 + torch.exp(-prod[:, :N // 2])) * prod[:, N // 2:]
+    cols = want.shape[1]
+    room = torch.full((M, cols + 3), 7.0, device=DEV, dtype=torch.float32 if mode in ("f32", "padded") else torch.bfloat16)
+    out = room[:, 1:cols + 1] if mode == "padded" else room.view(-1)[:M * cols].view(M, cols)
+    ops.gemm(to_dev(a), to_dev(w), out, silu_mul=silu, rms_parts=parts)
+    got = out.cpu().double()
+    # a float32 sum of K products of 16-bit numbers: at most K roundings of 2^-24 of the sum of their magnitudes
+    size = a.double().abs() @ w.double().abs().T
+    tol = 2 ** -24 * K * size.max().item() * 1.5
+    if mode not in ("f32", "padded"):
+        # and of the result to 16 bits (the scale, the unit and its exponential: a few units of 2^-22)
+        tol = 2 ** -8 * want.abs().max().item() + 4 * tol * max(1.0, prod.abs().max().item())
+    assert (got - want).abs().max().item() <= tol
+    if mode == "padded":
+        assert (room[:, 0] == 7.0).all() and (room[:, cols + 1:] == 7.0).all()
+    again = torch.empty_like(out)
+    ops.gemm(to_dev(a), to_dev(w), again, silu_mul=silu, rms_parts=parts)
+    assert torch.equal(out, again)
+    # a row's bits do not depend on the rows beside it
+    if M > 33:
+        few = torch.empty(M - 1, cols, device=DEV, dtype=out.dtype)
+        ops.gemm(to_dev(a[1:]), to_dev(w), few, silu_mul=silu,
+                 rms_parts=None if parts is None else (to_dev(torch.cat([parts[0].cpu()[:, 1:], parts[0].cpu()[:, :1]], 1)), *parts[1:]))
+        assert torch.equal(few, out[1:])
+
+
 def test_gemm_bf16_split_k_is_the_same_on_every_run():
     from glassbox_amd import ops
     a, w = to_dev(rnd(8, 8192, seed=1).bfloat16()), to_dev(rnd(2048, 8192, seed=2).bfloat16())
@@ -774,6 +817,13 @@ def test_gemm_bf16_rotates_and_writes_the_cache(M, nh, nkv, hd, K, normed):
         assert (two.float() - qkv.float()).abs().max().item() <= 2 * tol
         assert (k2.float() - k_pages.float()).abs().max().item() <= 2 * tol
         assert (v2.float() - v_pages.float()).abs().max().item() <= 2 * tol
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K", [(17, 32, 32, 64, 2048), (24, 32, 8, 128, 4096), (64, 32, 32, 64, 2048), (33, 9, 3, 64, 576),
+                                           (48, 31, 9, 48, 128), (32, 40, 0, 64, 1024), (19, 129, 1, 16, 64), (64, 60, 2, 64, 1984)])
+def test_gemm_bf16_rotates_and_writes_the_cache_with_the_rows_held(M, nh, nkv, hd, K):
+    """The same where a workgroup holds the rows and walks over several tiles of W (a wave then prepares one of them)."""
+    test_gemm_bf16_rotates_and_writes_the_cache(M, nh, nkv, hd, K, False)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
