@@ -1331,10 +1331,33 @@ struct SplitPlan {
   size_t floats;  // of workspace
   bool ring;      // the ring kernel's 256 x 256 tiles, if the operands allow (else the tiled kernel's, same slices)
   bool stream;    // the stream kernel's 128 x 32 tiles, if the operands allow (else the tiled kernel's, same slices)
+  bool held;      // the held kernel's tiles of 16 rows of W, if the operands allow (else the tiled kernel's, same slices)
 };
 
+// Slices of k for the held kernel where its tiles alone are few (the O and down projections of 17 to 64 rows): four tiles a workgroup and
+// more, so that it reads more of W than of A; 512 of k and more; and what a wave can hold of a slice.  Fewer slices than the wide tiles
+// took, so that the pass behind them reads less.  (us, with that pass and the norm, before / now: 4,096 x 14,336, 24 / 53 rows 33.0 / 35.0 ->
+// 26.7 / 29.8; 4,096 x 4,096, 17.0 / 17.7 -> 13.7 / 15.5; 2,048 x 8,192, 16.1 / 17.0 -> 13.5 / 15.2; 2,048 x 2,048, 53 rows 10.5 -> 9.9; 576 x
+// 1,536, 53 rows 9.1 -> 7.6.)  Products of up to 32 rows by a k below 4,096 stay whole: the skinny kernel adds into the residual and
+// prepares the norm in one launch.
+inline int held_slice(int K, int slices) { return (K / 64 + slices - 1) / slices * 64; }
+inline int held_slices(int M, int N, int K) {
+  const int tiles = (N + 15) / 16, most = 64 * HWAVES * (M <= 32 ? 8 : 4), least = (K + most - 1) / most;
+  if (tiles > 256 || least > 16 || (M <= 32 && K < 4096)) return 1;
+  int want = (4 * 256 + tiles - 1) / tiles;
+  want = want > 16 ? 16 : want;
+  if (want > K / 512) want = K / 512;
+  return want < least ? least : want;
+}
 inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
-  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false};
+  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false, false};
+  if (M > 16 && M <= 64 && K % 64 == 0 && N % 8 == 0 && !silu && held_slices(M, N, K) > 1) {
+    p.k_slice = held_slice(K, held_slices(M, N, K));
+    p.slices = (K + p.k_slice - 1) / p.k_slice;
+    p.floats = (size_t)p.slices * M * N;
+    p.held = true;
+    return p;
+  }
   // many rows, a long k and few 256 x 256 tiles (the down projection of a prompt): slices of k fill the
   // chip with the ring kernel's tiles once; a slice keeps 1,024 of k or more
   if (ring_slices_pay(M, K) && K >= 4096 && K % TBK == 0 && N % 8 == 0) {
@@ -1363,7 +1386,7 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
       if (want < 2) return p;
       p.k_slice = ((K + want - 1) / want + SBK - 1) / SBK * SBK;
       p.slices = (K + p.k_slice - 1) / p.k_slice;
-      if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false};
+      if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, false};
       p.floats = (size_t)p.slices * M * N;
       p.stream = true;
       return p;
@@ -1386,7 +1409,7 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
   if (want < 2) return p;
   p.k_slice = ((K + want - 1) / want + TBK - 1) / TBK * TBK;
   p.slices = (K + p.k_slice - 1) / p.k_slice;
-  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false};
+  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, false};
   p.floats = (size_t)p.slices * M * N;
   // tiles of 64 rows where even with the slices a third of the compute units would have no workgroup
   if (tiles * p.slices < 168) p.bm = 64;
@@ -1481,6 +1504,63 @@ __global__ __launch_bounds__(256) void splitk_reduce_norm_kernel(const float* __
   }
 }
 
+// The same for the few rows of a decode step, which are as few workgroups: what bounds it are the round trips a thread makes one after
+// the other, so as many threads as the row has words of four columns (at most 1,024), and a word's old value, gamma and up to AT_ONCE
+// slices asked for together.  Same bits but for the order in which a row's squares are added.  (With
+// 256 threads and four slices at a time, of 24 rows of 4,096: sixteen slices 33.3 -> 30.2 us with their product, eight 16.8 -> 15.4.)
+constexpr int SPLIT_NORM_FEW = 64;
+inline int split_norm_threads(int N) { return N >= 4096 ? 1024 : (N / 4 + 63) / 64 * 64; }
+template <int AT_ONCE, typename G>
+__global__ __launch_bounds__(1024) void splitk_reduce_norm_few_kernel(const float* __restrict__ ws, int slices, float* __restrict__ c,
+                                                                      int ldc, int M, int N, const G* __restrict__ gamma, float eps,
+                                                                      bf16* __restrict__ h, int ldh) {
+  constexpr int WORDS = SPLIT_NORM_MAX / 4096;
+  __shared__ float partial[16];
+  const int m = blockIdx.x, tid = threadIdx.x, threads = blockDim.x;
+  const size_t copy = (size_t)M * N;
+  f32x4 r[WORDS];
+  float g[WORDS][4], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i) {
+    const int j = (tid + threads * i) * 4;
+    if (j >= N) break;
+    const float* row = ws + (size_t)m * N + j;
+    const f32x4 old = *reinterpret_cast<const f32x4*>(c + (size_t)m * ldc + j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) g[i][e] = (float)gamma[j + e];
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int z = 0; z < slices; z += AT_ONCE) {
+      f32x4 v[AT_ONCE];   // (behind the last slice: the last again, not added)
+#pragma unroll
+      for (int t = 0; t < AT_ONCE; ++t) v[t] = *reinterpret_cast<const f32x4*>(row + min(z + t, slices - 1) * copy);
+#pragma unroll
+      for (int t = 0; t < AT_ONCE; ++t)
+        if (z + t < slices) sum += v[t];
+    }
+    sum = old + sum;
+    *reinterpret_cast<f32x4*>(c + (size_t)m * ldc + j) = sum;
+    r[i] = sum;
+    ss += sum[0] * sum[0] + sum[1] * sum[1] + sum[2] * sum[2] + sum[3] * sum[3];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  if (tid % 64 == 0) partial[tid / 64] = ss;
+  __syncthreads();
+  float total = partial[0];
+  for (int w = 1; w < threads / 64; ++w) total += partial[w];
+  const float scale = 1.0f / sqrtf(total / (float)N + eps);
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i) {
+    const int j = (tid + threads * i) * 4;
+    if (j >= N) break;
+    bf16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (bf16)(g[i][e] * (r[i][e] * scale));
+    *reinterpret_cast<bf16x4*>(h + (size_t)m * ldh + j) = o;
+  }
+}
+
 // Folded tiles pay when the product has at most 8 rows and whole tiles of 16 rows of W would leave
 // compute units without a workgroup (measured: with 384 such tiles they no longer do).
 inline bool fold_pays(int M, int N) { return M <= 8 && (N + 15) / 16 < 256; }
@@ -1510,6 +1590,10 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
   const bool kfull = K % TBK == 0;
   const bool ring = plan.ring && ring_takes(a, lda, w, ldw, K);
   const bool streams = plan.stream && stream_takes(a, lda, w, ldw, K);
+  const bool held = plan.held && held_takes(a, lda, w, ldw, M, plan.k_slice);
+  if (held) {
+    if (int rc = launch_held<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, 0.f, nullptr, 0, stream)) return rc;
+  }
   if (streams) {
     if (int rc = launch_stream<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, stream)) return rc;
   }
@@ -1517,7 +1601,7 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
     hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, float>), dim3((N + RBN - 1) / RBN, (M + RBM - 1) / RBM, plan.slices), dim3(RGM * RGN * 64),
                        0, stream, a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, Groups{}, Glu{});
 #define GB_S(WM, FULL)                                                                                                   \
-  if (!ring && !streams && (plan.bm == 64 * WM) && kfull == FULL)                                                                   \
+  if (!ring && !streams && !held && (plan.bm == 64 * WM) && kfull == FULL)                                                                   \
     hipLaunchKernelGGL((gemm_tiled_kernel<WM, 2, 1, EPI_STORE, FULL, float>), grid, block, 0, stream, a, lda, w, ldw, ws, \
                        N, M, N, K, plan.k_slice, Groups{}, Glu{});
   GB_S(1, true) GB_S(1, false) GB_S(2, true) GB_S(2, false)
@@ -1526,12 +1610,17 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
   if (!second_pass) return 0;   // the caller adds the slices
   if constexpr (EPI == EPI_ACCUMULATE && std::is_same<CT, float>::value) {
     if (norm && norm->emit_h) {
-      if (norm->emit_gamma_f32)
-        hipLaunchKernelGGL((splitk_reduce_norm_kernel<float>), dim3(M), dim3(256), 0, stream, ws, plan.slices, c, ldc, M, N,
-                           (const float*)norm->emit_gamma, eps, norm->emit_h, norm->emit_ldh);
-      else
-        hipLaunchKernelGGL((splitk_reduce_norm_kernel<bf16>), dim3(M), dim3(256), 0, stream, ws, plan.slices, c, ldc, M, N,
-                           (const bf16*)norm->emit_gamma, eps, norm->emit_h, norm->emit_ldh);
+#define GB_RN(KERNEL, THREADS, G)                                                                                          \
+  hipLaunchKernelGGL(KERNEL, dim3(M), dim3(THREADS), 0, stream, ws, plan.slices, c, ldc, M, N, (const G*)norm->emit_gamma, eps, \
+                     norm->emit_h, norm->emit_ldh)
+#define GB_RNS(G)                                                                                                      \
+  if (M > SPLIT_NORM_FEW) GB_RN((splitk_reduce_norm_kernel<G>), 256, G);                                               \
+  else if (plan.slices > 8) GB_RN((splitk_reduce_norm_few_kernel<16, G>), split_norm_threads(N), G);                   \
+  else if (plan.slices > 4) GB_RN((splitk_reduce_norm_few_kernel<8, G>), split_norm_threads(N), G);                    \
+  else GB_RN((splitk_reduce_norm_few_kernel<4, G>), split_norm_threads(N), G);
+      if (norm->emit_gamma_f32) { GB_RNS(float) } else { GB_RNS(bf16) }
+#undef GB_RNS
+#undef GB_RN
       return launched("gemm_bf16 (split k, second pass with the norm)");
     }
   }
@@ -2161,7 +2250,9 @@ extern "C" int gb_gemm_bf16_emit_mode(int M, int N, int K) { return emit_mode(M,
 
 // Floats of workspace with which gb_gemm_bf16 would split k for this product (0: it would not).
 extern "C" long long gb_gemm_bf16_split_floats(int M, int N, int K) {
-  return M > 16 ? (long long)split_plan(M, N, K).floats : 0;
+  if (M <= 16) return 0;
+  const size_t plain = split_plan(M, N, K).floats, unit = split_plan(M, N, K, true).floats;   // (either may be asked for)
+  return (long long)(plain > unit ? plain : unit);
 }
 
 // Slices into which gb_gemm_bf16_partial divides k for a product of these sizes (1: it would not divide it).

@@ -481,6 +481,13 @@ def test_gemm_bf16_that_divides_k_does_the_next_norm(M, N, K, gamma_dtype):
         ops.gemm(to_dev(a), to_dev(w), res, accumulate=True, emit=(to_dev(g), h, eps))       # no workspace
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 14336), (24, 4096, 4160), (33, 576, 1536), (20, 96, 8192), (64, 72, 1088), (49, 8192, 1024),
+                                   (64, 4088, 16384), (32, 8, 4096)])
+def test_gemm_bf16_of_few_rows_that_divides_k_does_the_next_norm(M, N, K):
+    """17 to 64 rows: slices of one to sixteen, some of them short; rows of two words a thread, of a few words in all."""
+    test_gemm_bf16_that_divides_k_does_the_next_norm(M, N, K, torch.float32)
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 96, 4096), (33, 2048, 2048), (64, 2048, 8192), (100, 2048, 4160),
                                    # 128 narrow tiles are not enough to go without slices (Llama-3-8B's O and down projections)
                                    (96, 4096, 8192), (128, 4096, 4096),
