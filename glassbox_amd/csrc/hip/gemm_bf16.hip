@@ -8,8 +8,8 @@
 //    v_mfma_f32_32x32x16_bf16 tiles (workgroup tile 128x128 or 128x64; 64 rows high where the taller tiles would be
 //    few), operands staged through LDS in k-steps of 64 with two buffers; the SiLU-multiply of stacked gate/up rows
 //    can be its epilogue.  Its workgroups can also divide k (split k: a second pass adds their sums in order).
-//  * stream (65 to 128 rows, the mixed steps of serving): 128 x 32 or 128 x 64 tiles, both operands through deep
-//    rings in LDS, W asked for by a wave of its own.
+//  * block  (some hundred rows): tiles of 64 to 256 rows by 64 to 128 columns, whichever move the fewest bytes, both operands
+//    straight into LDS several k-steps ahead.
 //  * ring   (some hundred rows and more, enough 256x256 tiles to fill the chip): 2x2 waves, a wave 8x8 tiles of
 //    v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
 //  * skinny (M <= 64, decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
@@ -786,54 +786,28 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
   return launched("gemm_bf16 (ring)");
 }
 
-// ----------------------------------------------------------------------- stream
-// Products of 17 to a few hundred rows (the mixed steps of serving: a portion of a prompt beside decoded tokens,
-// a new turn behind a long history).  They are bound by reading W once, like decoding, but A no longer fits a
-// wave's registers; and with the wide tiles above few workgroups exist, each with little on its way from memory
-// (a chip-wide 5 TB/s at 2 us of latency wants some 40 KB in flight on every compute unit).
+// ------------------------------------------------------------------------ block
+// Products of some hundred rows (short prompts, a new turn behind a history, mixed steps; the narrow products of a longer prompt): too
+// few 256 x 256 tiles for the ring kernel.  A workgroup of 2 x 2 waves takes a tile of 32 RM rows by 32 CN rows of W, a wave RM x CN
+// tiles of 16 x 16 (W as the first operand: a lane holds four neighbouring columns of a row of C).  Both operands of a k-step of 64 go
+// from memory straight into a slot of LDS (a load of the wave brings eight whole lines; piece p of row r lies at p ^ ((r >> 1) & 7)), and
+// S slots are all on their way but the one that is multiplied: what bounds the tiled kernel here is a round trip to memory a k-step, with
+// one or two of them in registers ahead.  The height of a tile is chosen by the rows there are, in steps of 32: 131 rows are one tile of
+// 160 and not two of 128.
 //
-// Here a workgroup owns all 128 rows of a row tile and only 32 or 64 rows of W (TN = 1, 2), so that even the QKV
-// product of a 2,048-wide model has a workgroup for most compute units without dividing k.  Four waves compute,
-// each 32 rows of A by all of the workgroup's columns.  Both operands go from memory straight into LDS
-// (global_load_lds, 16 bytes a lane) in k-steps of 64 through two rings: six stages of A (16 KB each; A comes
-// from the second-level cache, every workgroup reads the same rows), asked for by the computing waves, and 14 or 7
-// stages of W (4 or 8 KB each: some 50 KB on their way from memory per compute unit), asked for by a fifth wave
-// that does nothing else.  A wave's loads retire in the order of issue: if one wave asked for both, waiting for
-// a stage of A would also wait for every stage of W asked for before it, and W would be three k-steps ahead,
-// not thirteen.  A row of a k-step is 128 bytes = 8 pieces; piece p of row r lies at position p ^ (r & 7), which
-// spreads the 16-byte operand reads of a wave over all banks.  Waits are written by hand as in the ring kernel.
-constexpr int SBK = 64, SBM = 128, SA_STAGES = 6;
-// Measured on SmolLM2-1.7B shapes (each product alone, replayed from a graph): up to 64 rows the skinny kernel is as
-// fast or faster (it keeps A in registers); from about 200 rows on the wide tiles that divide k are (a workgroup here
-// reads two LDS operands for every MFMA); between, this kernel gains 10 to 25 %.
-constexpr int STREAM_MAX_ROWS = 128;
-// Narrow tiles enough to fill the chip without dividing k.  (128 were taken for enough once: the 4,096 rows of W of a
-// Llama-3-8B projection then made 128 workgroups that walk all of k, and its O and down projections of 65 to 128 rows
-// took 29 and 81 us where the wide tiles with slices take 14 and 30.)
-constexpr int STREAM_FILLS = 192;
-// The fewest rows minus one that go to the stream kernel: 48 where it takes the product whole (gate/up of 64 rows:
-// SmolLM2-1.7B shapes 23.3 -> 22.0 us, Llama-3-8B shapes 82 -> 73; at 40 rows the wide tiles with slices are as fast or
-// faster), 32 where it divides k (the O projection of the 1.7B shapes at 40 to 64 rows 11.4 -> 9.6 us, the down projection
-// of the 360M shapes 11.1 -> 9.1).
-inline int stream_min_rows(int M, int N, int K, bool silu) {
-  const int tiles = ((N + 31) / 32) * ((M + 127) / 128);
-  const bool divides = tiles < STREAM_FILLS && K >= 1024 && K < 4096;  // as split_plan decides for the stream kernel's range
-  // (other products it would take whole stay with the skinny kernel up to 64 rows, and so does a SiLU-multiply product
-  // whose narrow tiles do not fill the chip: SmolLM2-360M's gate/up of 49 to 64 rows 8.7 us there, 10.3 here)
-  return divides ? 32 : (silu && tiles >= 2 * STREAM_FILLS) ? 48 : 64;
-}
-constexpr int SLA = SBM / 8 / 4;  // a computing wave's load instructions per stage of A (an instruction moves 8 rows x 8 pieces)
-template <int TN> struct StreamShape {
-  static constexpr int BN = 32 * TN, W_STAGES = TN == 1 ? 14 : 7, LW = BN / 8;  // LW: the loading wave's instructions per stage
-};
-
-template <int TN, int EPI, typename CT>
-__global__ __launch_bounds__(320, 1) void gemm_stream_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w,
-                                                             int ldw, CT* __restrict__ c, int ldc, int M, int N, int K,
-                                                             int k_slice) {
-  using S = StreamShape<TN>;
-  constexpr int BN = S::BN, SW = S::W_STAGES, LW = S::LW, DA = SA_STAGES - 1, DW = SW - 1;
-  static_assert((DW - 1) * LW < 64 && (DA - 1) * SLA < 64, "a wave counts at most 63 loads on their way");
+// As in the ring kernel the operand reads and MFMAs are inline assembly in the order written, the barrier of a k-step stands between its
+// two halves, and the waits are written by hand.  Before the barrier a wave has waited for its last operand reads of the k-step, so behind
+// it the k-step's slot is free for the loads of k-step + S; and for its own loads of the next k-step, whose first operands are read
+// under the second half's MFMAs.
+// us, the tiled kernel (or one of 128-row tiles with W asked for by a wave of its own, up to 128 rows) / this one, the product alone: gate/up
+// 16,384 x 2,048, 70 / 131 / 300 / 512 rows 22.4 / 28.6 / 39.4 / 46.2 -> 18.2 / 21.8 / 29.4 / 39.4 (744 -> 872 TFLOP/s at the last); 5,120 x 960, 131 /
+// 420 / 1,000 rows 10.5 / 13.4 / 25.5 -> 7.3 / 10.9 / 16.3; 28,672 x 4,096, 131 rows 78 -> 55 (4.2 TB/s of W); QKV 6,144 x 2,048, 131 rows 19.5 (in
+// slices) -> 13.2, 512 rows 23.9 -> 21.6; first passes in slices: 2,048 x 8,192, 131 rows 19.1 -> 13.9, 960 x 2,560, 611 rows 10.7 -> 9.9.
+template <int RM, int CN, int S, int EPI, typename CT>
+__global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w, int ldw,
+                                                            CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice, Glu glu) {
+  constexpr int BM = 32 * RM, BN = 32 * CN, ROWS = BM + BN, L = ROWS / 32;   // L: loads of a wave that bring its share of a slot
+  static_assert((S - 1) * L < 64, "a wave counts at most 63 loads on their way");
   if (k_slice > 0) {  // split k: workgroup z of a tile sums its own slice of k into its own copy of C
     const int z = blockIdx.z;
     a += (size_t)z * k_slice;
@@ -841,180 +815,204 @@ __global__ __launch_bounds__(320, 1) void gemm_stream_kernel(const bf16* __restr
     c += (size_t)z * M * ldc;
     K = min(k_slice, K - z * k_slice);
   }
-  __shared__ __attribute__((aligned(16))) bf16 As[SA_STAGES][SBM * SBK];
-  __shared__ __attribute__((aligned(16))) bf16 Ws[SW][BN * SBK];
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int bx = blockIdx.x, m0 = blockIdx.y * SBM;
-  const int half = N / 2;  // EPI_SILU_MUL: number of gate rows
-  const int steps = K / SBK;
-  // Every workgroup of a row tile reads the same rows of A.  If all walked k from 0 they would ask the same few
-  // channels of the second-level cache for the same lines at the same time; so each starts somewhere else and
-  // walks round (the order of a cell's sum depends on its column tile, never on the rows of the step).
-  const int rot = (int)((blockIdx.x * 13u + blockIdx.z * 5u) % (unsigned)steps);
-  auto k_of = [&](int step) {
-    const int t = step + rot;
-    return (t >= steps ? t - steps : t) * SBK;
+  __shared__ __attribute__((aligned(16))) bf16 slots[S][ROWS * RBK];   // the tile's rows of A, then those of W
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / 2, wn = wave % 2, bx = blockIdx.x, m0 = blockIdx.y * BM;
+  const int half = N / 2;  // EPI_SILU_MUL: number of gate rows; a wave's even column tiles hold gate rows, the odd ones their up rows
+  auto w_row = [&](int r) -> int {   // row of W behind row r of the tile's; rows beyond M or N are read from a row that exists
+    if (EPI == EPI_SILU_MUL) {
+      const int j = r % (CN * 16) / 16, n = min(bx * (BN / 2) + r / (CN * 16) * (CN / 2 * 16) + j / 2 * 16 + r % 16, half - 1);
+      return j % 2 ? half + n : n;
+    }
+    return min(bx * BN + r, N - 1);
   };
-
-  if (wave == 4) {
-    // ------------------------------------------------------------ the wave that asks for W
-    // row of W behind row r of the workgroup's W tile; with EPI_SILU_MUL (TN = 2) the first 32 rows are gate rows
-    // and the second 32 the up rows that belong to them; rows beyond N are read from a row that exists
-    auto w_row = [&](int r) -> int {
-      if (EPI == EPI_SILU_MUL) {
-        const int n = bx * 32 + r % 32;
-        return n < half ? (r / 32 ? half + n : n) : 0;
-      }
-      return min(bx * BN + r, N - 1);
-    };
-    const bf16* wsrc[LW];
+  const bf16* src[L];
 #pragma unroll
-    for (int t = 0; t < LW; ++t) {
-      const int row = t * 8 + lane / 8, piece = (lane % 8) ^ (row & 7);
-      wsrc[t] = w + (size_t)w_row(row) * ldw + piece * 8;
-    }
-    auto load_w = [&](int step) {
-#pragma unroll
-      for (int t = 0; t < LW; ++t)
-        __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[t] + k_of(step)), (lds_void*)&Ws[step % SW][t * 8 * SBK], 16, 0, 2);  // nontemporal: W is read once, in whole 128-byte lines
-    };
-    for (int t = 0; t < DW && t < steps; ++t) load_w(t);
-    // stage 0 has landed once at most the loads asked for after it are on their way
-    if (steps >= DW)
-      vm_wait<(DW - 1) * LW>();
-    else
-      vm_wait<0>();
-    __builtin_amdgcn_s_barrier();
-    for (int s = 0; s < steps; ++s) {
-      // everybody has passed the barrier of k-step s - 1: the buffer of stage s - 1 is free
-      const bool more = s + DW < steps;
-      if (more) load_w(s + DW);
-      if (s + 1 < steps) {
-        if (more)
-          vm_wait<(DW - 1) * LW>();  // stage s + 1 has landed: only what was asked for after it is on its way
-        else
-          vm_wait<0>();
-        __builtin_amdgcn_s_barrier();
-      }
-    }
-    return;
+  for (int t = 0; t < L; ++t) {
+    const int row = (wave * L + t) * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
+    src[t] = (row < BM ? a + (size_t)min(m0 + row, M - 1) * lda : w + (size_t)w_row(row - BM) * ldw) + piece * 8;
   }
-
-  // ---------------------------------------------------------------- the waves that compute
-  // a load instruction moves 8 rows x 8 pieces; rows beyond M are read from a row that exists
-  const bf16* asrc[SLA];
-#pragma unroll
-  for (int t = 0; t < SLA; ++t) {
-    const int row = (wave * SLA + t) * 8 + lane / 8, piece = (lane % 8) ^ (row & 7);
-    asrc[t] = a + (size_t)min(m0 + row, M - 1) * lda + piece * 8;
-  }
-  auto load_a = [&](int step) {
-#pragma unroll
-    for (int t = 0; t < SLA; ++t)
-      __builtin_amdgcn_global_load_lds((glb_void*)(asrc[t] + k_of(step)),
-                                       (lds_void*)&As[step % SA_STAGES][(wave * SLA + t) * 8 * SBK], 16, 0, 0);
+  auto load = [&](int t, int slot, int k0) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(src[t] + k0), (lds_void*)&slots[slot][(wave * L + t) * 8 * RBK], 16, 0, 0);
   };
-  f32x16 acc[TN];
+  // until k-step s has landed: of the k-steps up to `last` asked for, those behind s may be on their way
+  auto landed = [&](int s, int last) {
+    const int behind = last - s;
+    if (behind >= S - 1) vm_wait<(S - 1) * L>();
+    else if (S > 2 && behind == S - 2) vm_wait<(S > 2 ? S - 2 : 0) * L>();
+    else if (S > 3 && behind == S - 3) vm_wait<(S > 3 ? S - 3 : 0) * L>();
+    else if (S > 4 && behind == S - 4) vm_wait<(S > 4 ? S - 4 : 0) * L>();
+    else vm_wait<0>();
+  };
+  f32x4 acc[RM][CN];
 #pragma unroll
-  for (int j = 0; j < TN; ++j)
+  for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-
-  // operand of MFMA step kk (0..3): row lane % 32 of a 32-row tile, piece 2 kk + lane / 32
-  uint32_t off[4];
+    for (int j = 0; j < CN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t off[2];   // operand of half kh: row lane % 16 of a 16-row tile, piece 4 kh + lane / 16
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) off[kk] = 2 * ((lane % 32) * SBK + (((2 * kk + lane / 32) ^ (lane & 7)) * 8));
-  const uint32_t abase = (uint32_t)(uintptr_t)(lds_void*)&As[0][0] + 2 * wave * 32 * SBK;
-  const uint32_t wbase = (uint32_t)(uintptr_t)(lds_void*)&Ws[0][0];
-  constexpr uint32_t A_STAGE = 2 * SBM * SBK, W_STAGE = 2 * BN * SBK, TILE = 2 * 32 * SBK;
-
-  bf16x8 fa[2][4], fw[2][4 * TN];  // two sets: the operands of k-step s + 1 arrive under the MFMAs of k-step s
-  auto read_operands = [&](int s, int set) {
+  for (int kh = 0; kh < 2; ++kh) off[kh] = 2 * ((lane % 16) * RBK + (((4 * kh + lane / 16) ^ ((lane >> 1) & 7)) * 8));
+  constexpr uint32_t SLOT = 2 * ROWS * RBK, TILE = 2 * 16 * RBK;
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&slots[0][0];
+  const uint32_t abase = base + wm * RM * TILE, wbase = base + (BM / 16 + wn * CN) * TILE;
+  bf16x8 fa[2][RM], fw[2][CN];
+  auto read = [&](int set, int t, uint32_t at) {   // operand t of RM + CN of a half
+    if (t < RM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][t < RM ? t : 0]) : "v"(abase + at), "n"(t < RM ? t * TILE : 0) : "memory");
+    else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][t < RM ? 0 : t - RM]) : "v"(wbase + at), "n"(t < RM ? 0 : (t - RM) * TILE) : "memory");
+  };
+  const int steps = K / RBK;
+  // the MFMAs of operand set `set`; among them the reads of the other set from `at`, and (with `more`) a slot's loads
+  auto block = [&](auto which, uint32_t at, bool more, int slot, int k0) {
+    constexpr int set = decltype(which)::value, COUNT = RM * CN, EACH = (RM + CN + L + COUNT - 1) / COUNT;
+    int next = 0;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      fa[set][kk] = lds_read16(abase + (s % SA_STAGES) * A_STAGE + off[kk]);
+    for (int n = 0; n < COUNT; ++n) {
+      const int i = n / CN, j = (i & 1) ? CN - 1 - n % CN : n % CN;
+      if constexpr (COUNT > 24) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
+      else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
 #pragma unroll
-      for (int j = 0; j < TN; ++j) fw[set][kk * TN + j] = lds_read16(wbase + (s % SW) * W_STAGE + j * TILE + off[kk]);
+      for (int u = 0; u < EACH; ++u) {
+        if (next < RM + CN) read(set ^ 1, next, at);
+        else if (set == 1 && next < RM + CN + L && more) load(next - RM - CN, slot, k0);
+        ++next;
+      }
     }
   };
-  using Set0 = std::integral_constant<int, 0>;
-  using Set1 = std::integral_constant<int, 1>;
-
-  for (int t = 0; t < DA && t < steps; ++t) load_a(t);
-  if (steps >= DA)
-    vm_wait<(DA - 1) * SLA>();
-  else
-    vm_wait<0>();
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
+  const int first = min(S, steps);
+#pragma unroll 1
+  for (int s = 0; s < first; ++s)
+#pragma unroll
+    for (int t = 0; t < L; ++t) load(t, s, s * RBK);
+  landed(0, first - 1);
   __builtin_amdgcn_s_barrier();
-  read_operands(0, 0);
-  // k-step s, its operands in register set `mine`
-  auto step = [&](int s, auto mine) {
-    constexpr int set = decltype(mine)::value;
-    // everybody has passed the barrier of k-step s - 1: the buffer of stage s - 1 is free
-    const bool more = s + DA < steps;
-    if (more) load_a(s + DA);
-    lds_wait<0>(fa[set], fw[set]);  // all of this wave's reads of stage s have arrived
-    if (s + 1 < steps) {
-      if (more)
-        vm_wait<(DA - 1) * SLA>();  // this wave's part of stage s + 1 has landed
-      else
-        vm_wait<0>();
-      __builtin_amdgcn_s_barrier();
-      read_operands(s + 1, set ^ 1);
-    }
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][kk], fw[set][kk * TN + j], acc[j], 0, 0, 0);
-  };
-  for (int s = 0; s < steps; s += 2) {
-    step(s, Set0{});
-    if (s + 1 < steps) step(s + 1, Set1{});
+  for (int t = 0; t < RM + CN; ++t) read(0, t, off[0]);
+  int slot = 0;
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    const int next = slot + 1 == S ? 0 : slot + 1;
+    lds_wait<0>(fa[0], fw[0]);
+    block(First{}, slot * SLOT + off[1], false, 0, 0);
+    lds_wait<0>(fa[1], fw[1]);
+    if (s + 1 < steps) landed(s + 1, min(steps, s + S) - 1);
+    __builtin_amdgcn_s_barrier();
+    block(Second{}, next * SLOT + off[0], s + S < steps, slot, (s + S) * RBK);   // (behind the last: read, not used)
+    slot = next;
   }
+  lds_wait<0>(fa[0], fw[0]);
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results, which the compiler does not know to wait for
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < CN; ++j) {
+      if constexpr (RM * CN > 24) asm volatile("" : "+a"(acc[i][j]));
+      else asm volatile("" : "+v"(acc[i][j]));
+    }
 
-  // accumulator layout of a 32x32 tile: lane holds column lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
-  const int row0 = m0 + wave * 32 + 4 * (lane / 32);
-  if (EPI == EPI_SILU_MUL) {
-    const int gn = bx * 32 + lane % 32;
-    if (gn >= half) return;
+  // a lane holds row lane % 16 of a tile and its columns 4 (lane / 16) .. + 3
+  constexpr int OUT = EPI == EPI_SILU_MUL ? CN / 2 : CN;   // column tiles of the wave's results
+  const int cols = EPI == EPI_SILU_MUL ? half : N;
+  const int gn0 = bx * (2 * OUT * 16) + wn * (OUT * 16) + 4 * (lane / 16);
+  const bool words = ldc % 4 == 0 && (uintptr_t)c % (4 * sizeof(CT)) == 0;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int gm = row0 + 8 * (r / 4) + r % 4;
-      const float g = acc[0][r], u = acc[TN - 1][r];
-      if (gm < M) c[(size_t)gm * ldc + gn] = (CT)(g / (1.0f + __expf(-g)) * u);
+  for (int i = 0; i < RM; ++i) {
+    const int gm = m0 + (wm * RM + i) * 16 + lane % 16;
+    if (gm >= M) continue;
+    CT* to = c + (size_t)gm * ldc + gn0;
+    f32x4 v[OUT];
+#pragma unroll
+    for (int j = 0; j < OUT; ++j) {
+      if constexpr (EPI == EPI_SILU_MUL) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[j][r] = gated_unit(acc[i][2 * j][r], acc[i][2 * j + 1][r], glu);
+      } else {
+        v[j] = acc[i][j];
+      }
     }
-    return;
-  }
+    if (words && gn0 + (OUT - 1) * 16 + 4 <= cols) {
+      if constexpr (EPI == EPI_ACCUMULATE) {
+        f32x4 old[OUT];   // a row's old values are all asked for before any is added to
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int gn = bx * BN + j * 32 + lane % 32;
-    if (gn >= N) continue;
+        for (int j = 0; j < OUT; ++j) old[j] = *reinterpret_cast<const f32x4*>(to + j * 16);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int gm = row0 + 8 * (r / 4) + r % 4;
-      if (gm < M) store_c<CT>(c + (size_t)gm * ldc + gn, acc[j][r], EPI == EPI_ACCUMULATE);
+        for (int j = 0; j < OUT; ++j) v[j] = old[j] + v[j];
+      }
+#pragma unroll
+      for (int j = 0; j < OUT; ++j) store_c4<CT>(to + j * 16, v[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < OUT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (gn0 + j * 16 + r < cols) store_c<CT>(to + j * 16 + r, v[j][r], EPI == EPI_ACCUMULATE);
     }
   }
 }
 
-inline bool stream_takes(const void* a, int lda, const void* w, int ldw, int K) {
-  return K % SBK == 0 && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
+// Which tile, and into how many slices k is divided: what the launch takes is the rows (of 128 bytes) that its workgroups bring into LDS,
+// at some 13 TB/s over the whole chip, and a compute unit at most 65 GB/s, or 50 of tiles of 224 rows and more, whose operand reads
+// weigh more; and 3.5 us.  (Over tiles of 64 x 64 to 256 x 128, one to eight slices and the products of four models at 70 to 1,000
+// rows that is within a fifth of what was measured.)  Slices are written and read again.  So the tiles are those that fill the chip
+// once with the fewest bytes.
+struct BlockPlan {
+  int rm, cn, slices, k_slice;
+  float us;
+};
+inline BlockPlan block_plan(int M, int N, int K, bool silu, int least_slices, int most_slices) {
+  static const struct { int rm, cn; } tiles[] = {{2, 2}, {3, 2}, {4, 2}, {5, 2}, {6, 2}, {4, 3}, {5, 3},
+                                                 {2, 4}, {3, 4}, {4, 4}, {5, 4}, {6, 4}, {8, 4}};
+  static const int slices[] = {1, 2, 3, 4, 5, 6, 8};
+  BlockPlan best{0, 0, 1, 0, 1e30f};
+  const int steps = K / RBK;
+  for (const auto& t : tiles) {
+    if (silu && t.cn == 3) continue;
+    const long long all = (long long)((M + 32 * t.rm - 1) / (32 * t.rm)) * ((N + 32 * t.cn - 1) / (32 * t.cn));
+    for (int z : slices) {
+      if (z < least_slices) continue;
+      if (z > most_slices || (z > 1 && steps < 8 * z)) break;
+      const int each = (steps + z - 1) / z;
+      if ((steps + each - 1) / each != z) continue;
+      const float bytes = (float)each * (t.rm + t.cn) * (32 * 128);
+      const float chip = (float)(all * z) * bytes / 13e6f, unit = (float)((all * z + 255) / 256) * bytes / (t.rm + t.cn >= 7 ? 50e3f : 65e3f);
+      const float us = 3.5f + (chip > unit ? chip : unit) + (z > 1 ? 3.5f + z * (float)M * N * 8.f / 4.5e6f : 0.f);
+      if (us < best.us) best = BlockPlan{t.rm, t.cn, z, each * RBK, us};
+    }
+  }
+  return best;
 }
+inline bool block_takes(const void* a, int lda, const void* w, int ldw, int K) {
+  return K % RBK == 0 && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
+}
+// Sizes that are the block kernel's, if the operands allow: short products whose k is not formed into a gated unit stay with the tiled
+// kernel, whose fewer k-steps ahead start sooner (1,600 x 960, 131 rows: 6.3 us, 7.0 here).  Up to 64 rows: what the held kernel cannot hold.
+inline bool block_sizes(int M, int N, int K, bool silu) { return M > 32 && K % RBK == 0 && N % 8 == 0 && (silu ? N % 16 == 0 : K >= 1024); }
+// What the ring kernel takes, alike: a k-step of its 256 x 256 tiles 1.75 us.
+inline float ring_us(int M, int N, int K, int slices) {
+  const long long tiles = (long long)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN) * slices;
+  return 3.5f + (float)((tiles + 255) / 256) * ((K / slices + RBK - 1) / RBK) * 1.75f + (slices > 1 ? 3.5f + slices * (float)M * N * 8.f / 4.5e6f : 0.f);
+}
+
+// Slots of a tile: what fits LDS, once (one workgroup a compute unit) or, of the small tiles, twice.
+constexpr int block_slots(int rm, int cn) { return rm + cn <= 5 ? 80 / (4 * (rm + cn)) : 160 / (4 * (rm + cn)) > 5 ? 5 : 160 / (4 * (rm + cn)); }
 
 template <int EPI, typename CT>
-int launch_stream(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice, int slices,
-                  hipStream_t stream) {
-  const int cols = EPI == EPI_SILU_MUL ? N / 2 : N;
-  // the SiLU-multiply needs a gate tile and its up tile in one wave; otherwise narrow tiles while they are few
-  const int tn = EPI == EPI_SILU_MUL ? 2 : ((cols + 31) / 32) * ((M + SBM - 1) / SBM) * slices > 512 ? 2 : 1;
-  const int bn = EPI == EPI_SILU_MUL ? 32 : 32 * tn;
-  const dim3 grid((cols + bn - 1) / bn, (M + SBM - 1) / SBM, slices), block(320);
+int launch_block(int rm, int cn, const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice,
+                 int slices, hipStream_t stream, Glu glu = Glu{}) {
+  const int cols = EPI == EPI_SILU_MUL ? N / 2 : N, bn = EPI == EPI_SILU_MUL ? 16 * cn : 32 * cn;
+  const dim3 grid((cols + bn - 1) / bn, (M + 32 * rm - 1) / (32 * rm), slices), block(256);
   GB_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
-  if (tn == 2)
-    hipLaunchKernelGGL((gemm_stream_kernel<2, EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, N, K, k_slice);
-  else if constexpr (EPI != EPI_SILU_MUL)
-    hipLaunchKernelGGL((gemm_stream_kernel<1, EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, N, K, k_slice);
-  return launched("gemm_bf16 (stream)");
+#define GB_B(RM, CN)                                                                                                              \
+  if (rm == (RM) && cn == (CN)) {                                                                                                 \
+    hipLaunchKernelGGL((gemm_block_kernel<(RM), (CN), block_slots((RM), (CN)), EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, \
+                       ldc, M, N, K, slices > 1 ? k_slice : 0, glu);                                                              \
+    return launched("gemm_bf16 (block)");                                                                                         \
+  }
+  GB_B(2, 2) GB_B(3, 2) GB_B(4, 2) GB_B(5, 2) GB_B(6, 2) GB_B(2, 4) GB_B(3, 4) GB_B(4, 4) GB_B(5, 4) GB_B(6, 4) GB_B(8, 4)
+  if constexpr (EPI != EPI_SILU_MUL) { GB_B(4, 3) GB_B(5, 3) }
+#undef GB_B
+  return fail("gemm_bf16 (block): no tile of %d x %d", 32 * rm, 32 * cn);
 }
 
 // ------------------------------------------------------------------------- held
@@ -1284,7 +1282,7 @@ inline int held_groups(int tiles, int slices) {
   const int room = 256 / slices, each = (tiles + room - 1) / room;
   return (tiles + each - 1) / each;
 }
-// Where it pays (us, the skinny kernel, the wide tiles or the stream kernel before / this one, each product alone):
+// Where it pays (us, the skinny kernel, the wide tiles or narrow ones before / this one, each product alone):
 //   gate/up 28,672 x 4,096, 17 / 24 / 32 rows: 53 / 57 / 62 -> 42 / 45 / 45 (5.2 to 5.5 TB/s); vocabulary 128,256 x 4,096,
 //   24 rows: 242 -> 176 (6 TB/s); gate/up 16,384 x 2,048, 20 / 33 / 64 rows: 19 / 21.6 / 20.8 -> 15.7 / 17 / 18; gate/up 5,120 x 960
 //   behind partial sums of a norm, 20 / 53 rows: 8.6 / 12.5 -> 8.2 / 8.8; QKV 6,144 x 4,096, 24 rows 17.2 -> 15.3; 6,144 x 2,048,
@@ -1330,8 +1328,8 @@ struct SplitPlan {
   int bm, slices, k_slice;
   size_t floats;  // of workspace
   bool ring;      // the ring kernel's 256 x 256 tiles, if the operands allow (else the tiled kernel's, same slices)
-  bool stream;    // the stream kernel's 128 x 32 tiles, if the operands allow (else the tiled kernel's, same slices)
   bool held;      // the held kernel's tiles of 16 rows of W, if the operands allow (else the tiled kernel's, same slices)
+  int rm, cn;     // the block kernel's tiles of 32 rm x 32 cn, if the operands allow (else the tiled kernel's, same slices); 0: not
 };
 
 // Slices of k for the held kernel where its tiles alone are few (the O and down projections of 17 to 64 rows): four tiles a workgroup and
@@ -1350,7 +1348,7 @@ inline int held_slices(int M, int N, int K) {
   return want < least ? least : want;
 }
 inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
-  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false, false};
+  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false, 0, 0};
   if (M > 16 && M <= 64 && K % 64 == 0 && N % 8 == 0 && !silu && held_slices(M, N, K) > 1) {
     p.k_slice = held_slice(K, held_slices(M, N, K));
     p.slices = (K + p.k_slice - 1) / p.k_slice;
@@ -1358,6 +1356,13 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
     p.held = true;
     return p;
   }
+  // the block kernel's tiles, and as many slices as suit them, for a product that is divided; others keep what is in p
+  auto in_blocks = [&](const SplitPlan& p) {
+    if (!block_sizes(M, N, K, silu)) return p;
+    const BlockPlan b = block_plan(M, N, K, false, 2, 8);
+    if (!b.rm || (p.ring && (M >= 1024 || ring_us(M, N, K, p.slices) <= b.us))) return p;
+    return SplitPlan{p.bm, b.slices, b.k_slice, (size_t)b.slices * M * N, false, false, b.rm, b.cn};
+  };
   // many rows, a long k and few 256 x 256 tiles (the down projection of a prompt): slices of k fill the
   // chip with the ring kernel's tiles once; a slice keeps 1,024 of k or more
   if (ring_slices_pay(M, K) && K >= 4096 && K % TBK == 0 && N % 8 == 0) {
@@ -1370,38 +1375,20 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
       if (p.slices >= 2 && K - (p.slices - 1) * p.k_slice >= RING_MIN_K) {
         p.floats = (size_t)p.slices * M * N;
         p.ring = true;
-        return p;
+        return in_blocks(p);
       }
       p.slices = 1, p.k_slice = 0;
     }
   }
-  if (M > stream_min_rows(M, N, K, silu) && M <= STREAM_MAX_ROWS && K % SBK == 0 && N % 8 == 0) {
-    // the stream kernel's range: its tiles are narrow, so only products with few rows of W divide k at all
-    // (the O and down projections); a slice keeps 512 of k or more
-    const int tiles = ((N + 31) / 32) * ((M + SBM - 1) / SBM);
-    if (tiles >= STREAM_FILLS) return p;  // enough narrow tiles: no slices at all
-    if (K < 4096) {              // a long k (the down projection) is left to the wide tiles' slices below: measured faster
-      int want = (256 + tiles - 1) / tiles;
-      if (want > K / 512) want = K / 512;
-      if (want < 2) return p;
-      p.k_slice = ((K + want - 1) / want + SBK - 1) / SBK * SBK;
-      p.slices = (K + p.k_slice - 1) / p.k_slice;
-      if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, false};
-      p.floats = (size_t)p.slices * M * N;
-      p.stream = true;
-      return p;
-    }
-  }
+  if (M > 64 && M <= 128 && K % RBK == 0 && N % 8 == 0 && (N + 31) / 32 >= 192) return p;   // narrow tiles fill the chip
   const int tiles = ((N + 127) / 128) * ((M + p.bm - 1) / p.bm);
   if (tiles >= 192 || N % 8 != 0) return p;
-  // measured on SmolLM2-1.7B shapes: a long k (the down projection) always gains; a short one where the
-  // skinny kernel is at its weakest (33 to 64 rows: every workgroup reads all of A) and where the tiles are
-  // very few (the O projection of a portion of some hundred rows: 16 to 64 tiles)
-  if (K < 4096 && !(M > 32 && M <= 64) && !(M > 64 && K >= 2048 && tiles <= 128)) return p;
-  // a slice keeps at least 8 k-steps (shorter ones cost more in partial sums than they gain), and of a long k, beyond
-  // 64 rows, 16 k-steps: a workgroup of 128 rows has more to do in a k-step, and the pass that adds the slices reads
-  // half as much (same box: the down projection of 256 rows on SmolLM2-1.7B shapes 26.7 -> 24.2 us, of 384 rows
-  // 36.0 -> 30.6; Llama-3-8B's QKV of 192 to 256 rows 36-38 -> 31, its O projection 25-26 -> 23-24)
+  // measured on SmolLM2-1.7B shapes: a long k (the down projection) always gains; a short one where the skinny kernel is at its weakest (33
+  // to 64 rows: every workgroup reads all of A), up to 128 rows, and where the tiles are very few (the O projection of a portion of some
+  // hundred rows: 16 to 64 tiles)
+  if (K < 4096 && !(M > 32 && M <= 128 && K >= 1024) && !(M > 64 && K >= 2048 && tiles <= 128)) return p;
+  // the tiled kernel's slices keep at least 8 k-steps (shorter ones cost more in partial sums than they gain), and of a long k, beyond
+  // 64 rows, 16
   int want = (512 + tiles - 1) / tiles;
   want = want > 16 ? 16 : want;
   if (M > 64 && K >= 4096 && want > K / (16 * TBK)) want = K / (16 * TBK);
@@ -1409,11 +1396,11 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
   if (want < 2) return p;
   p.k_slice = ((K + want - 1) / want + TBK - 1) / TBK * TBK;
   p.slices = (K + p.k_slice - 1) / p.k_slice;
-  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, false};
+  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, 0, 0};
   p.floats = (size_t)p.slices * M * N;
   // tiles of 64 rows where even with the slices a third of the compute units would have no workgroup
   if (tiles * p.slices < 168) p.bm = 64;
-  return p;
+  return in_blocks(p);
 }
 
 // ws: [slices][M][N] float32.  Four columns a thread; EPI_SILU_MUL pairs column j with column N/2 + j.
@@ -1589,19 +1576,19 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
   const dim3 grid((N + 127) / 128, (M + plan.bm - 1) / plan.bm, plan.slices), block(256);
   const bool kfull = K % TBK == 0;
   const bool ring = plan.ring && ring_takes(a, lda, w, ldw, K);
-  const bool streams = plan.stream && stream_takes(a, lda, w, ldw, K);
+  const bool blocks = plan.rm && block_takes(a, lda, w, ldw, K);
+  if (blocks) {
+    if (int rc = launch_block<EPI_STORE, float>(plan.rm, plan.cn, a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, stream)) return rc;
+  }
   const bool held = plan.held && held_takes(a, lda, w, ldw, M, plan.k_slice);
   if (held) {
     if (int rc = launch_held<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, 0.f, nullptr, 0, stream)) return rc;
-  }
-  if (streams) {
-    if (int rc = launch_stream<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, stream)) return rc;
   }
   if (ring)
     hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, float>), dim3((N + RBN - 1) / RBN, (M + RBM - 1) / RBM, plan.slices), dim3(RGM * RGN * 64),
                        0, stream, a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, Groups{}, Glu{});
 #define GB_S(WM, FULL)                                                                                                   \
-  if (!ring && !streams && !held && (plan.bm == 64 * WM) && kfull == FULL)                                                                   \
+  if (!ring && !blocks && !held && (plan.bm == 64 * WM) && kfull == FULL)                                                                   \
     hipLaunchKernelGGL((gemm_tiled_kernel<WM, 2, 1, EPI_STORE, FULL, float>), grid, block, 0, stream, a, lda, w, ldw, ws, \
                        N, M, N, K, plan.k_slice, Groups{}, Glu{});
   GB_S(1, true) GB_S(1, false) GB_S(2, true) GB_S(2, false)
@@ -2306,6 +2293,13 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
   if (M == 0) return 0;
   const bf16* W = (const bf16*)w;
   const bool held = !gamma && !emit_h && epilogue != EPI_ACCUMULATE && held_pays(epilogue, M, N, K) && held_takes(a, lda, w, ldw, M, K);
+  const bool blocks = !held && !gamma && !parts && block_sizes(M, N, K, epilogue == EPI_SILU_MUL) && block_takes(a, lda, w, ldw, K);
+  const bool rings = ring_pays(epilogue, a, lda, w, ldw, M, N, K);
+  const BlockPlan undivided = blocks ? block_plan(M, N, K, epilogue == EPI_SILU_MUL, 1, 1) : BlockPlan{};
+  // a product that only stores needs no second pass: not divided where that takes less (QKV, 131 x 6,144 x 2,048: 16 us in slices, 13 whole)
+  auto whole = [&](const SplitPlan& plan) {
+    return blocks && epilogue != EPI_ACCUMULATE && plan.rm && undivided.us < block_plan(M, N, K, false, 2, 8).us;
+  };
   if (split_ws != nullptr && M > 16 && !gamma && (!emit_h || emits == 2) && !parts) {  // more than the skinny kernels' best range
     const SplitPlan plan = split_plan(M, N, K, epilogue == EPI_SILU_MUL);
     if (plan.slices > 1 && (epilogue != EPI_SILU_MUL || N % 16 == 0) && (uintptr_t)split_ws % 16 == 0) {
@@ -2315,7 +2309,7 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
 #define GB_SP(EPI, CT) return launch_split<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, split_ws, plan, stream)
       if (epilogue == EPI_ACCUMULATE)
         return launch_split<EPI_ACCUMULATE, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, split_ws, plan, stream, &extra, eps);
-      if (!held) {
+      if (!held && !whole(plan)) {
         if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_SP(EPI_SILU_MUL, bf16);
         if (epilogue == EPI_SILU_MUL) GB_SP(EPI_SILU_MUL, float);
         if (c_dtype == kF32) GB_SP(EPI_STORE, float);
@@ -2333,22 +2327,15 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
     GB_HD(EPI_STORE, bf16);
 #undef GB_HD
   }
-  // The narrow tiles without slices: up to 128 rows wherever they give half the compute units a workgroup (with a
-  // long enough k the plan above has divided it instead); up to 256 rows where the wide tiles would be few and k is
-  // too short to divide (the products of a narrow model: SmolLM2-360M's gate/up of 256 rows, 16.3 -> 11.2 us).
-  const int narrow_tiles = ((ncols + 31) / 32) * ((M + SBM - 1) / SBM), wide_tiles = ((N + 127) / 128) * ((M + 127) / 128);
-  const bool narrow_pays = M <= STREAM_MAX_ROWS ? narrow_tiles >= 64
-                                               : (M <= 2 * STREAM_MAX_ROWS && epilogue == EPI_SILU_MUL && narrow_tiles >= 64 && wide_tiles < 128 && K < 2048);
-  if (M > stream_min_rows(M, N, K, epilogue == EPI_SILU_MUL) && narrow_pays && !gamma && !parts && !emit_h && stream_takes(a, lda, w, ldw, K) &&
-      (epilogue != EPI_SILU_MUL || N % 16 == 0) && N < 32768) {
+  if (blocks && (M > 64 || epilogue != EPI_ACCUMULATE) && !emit_h && (!rings || undivided.us < ring_us(M, N, K, 1))) {
     const bf16* A = (const bf16*)a;
-#define GB_ST(EPI, CT) return launch_stream<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
-    if (epilogue == EPI_ACCUMULATE) GB_ST(EPI_ACCUMULATE, float);
-    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_ST(EPI_SILU_MUL, bf16);
-    if (epilogue == EPI_SILU_MUL) GB_ST(EPI_SILU_MUL, float);
-    if (c_dtype == kF32) GB_ST(EPI_STORE, float);
-    GB_ST(EPI_STORE, bf16);
-#undef GB_ST
+#define GB_BK(EPI, CT) return launch_block<EPI, CT>(undivided.rm, undivided.cn, A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
+    if (epilogue == EPI_ACCUMULATE) GB_BK(EPI_ACCUMULATE, float);
+    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_BK(EPI_SILU_MUL, bf16);
+    if (epilogue == EPI_SILU_MUL) GB_BK(EPI_SILU_MUL, float);
+    if (c_dtype == kF32) GB_BK(EPI_STORE, float);
+    GB_BK(EPI_STORE, bf16);
+#undef GB_BK
   }
   // 17 to 64 rows by very many rows of W that the held kernel does not take (a long k): measured twice as fast
   // through the tiles below as through the skinny kernel with four column blocks (49,152 x 2,048: 102 -> about 50 us),

@@ -577,6 +577,38 @@ def test_gemm_bf16_streams_products_of_some_hundred_rows(M, N, K, mode):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("M,N,K", [(66, 1040, 1024), (131, 6144, 2048), (131, 16384, 512), (200, 5120, 960), (224, 1600, 2048), (300, 6160, 1088),
+                                   (420, 16384, 576), (512, 6144, 2048), (611, 5120, 960), (1000, 5120, 960), (257, 2064, 4160), (64, 28672, 4096)])
+@pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu", "workspace"])
+def test_gemm_bf16_blocks_of_some_hundred_rows(M, N, K, mode):
+    """Tiles of 64 to 256 rows by 64 to 128 rows of W, several k-steps on their way: fewer k-steps than that, rows and columns that no
+    tile divides, with a workspace on offer; against float64, the same bits on every run, nothing beyond the last row and column."""
+    from glassbox_amd import ops
+    a, w = rnd(M, K, seed=1).bfloat16(), (rnd(N, K, seed=2) / math.sqrt(K)).bfloat16()
+    c0 = rnd(M, N, seed=3).float()
+    prod = (to_dev(a).double() @ to_dev(w).double().T)
+    want = prod
+    if mode == "silu":
+        want = prod[:, :N // 2] / (1 + torch.exp(-prod[:, :N // 2])) * prod[:, N // 2:]
+    elif mode == "f32+":
+        want = prod + to_dev(c0).double()
+    cols = want.shape[1]
+    ws = torch.empty(max(1, ops.gemm_split_floats(M, N, K)), device=DEV) if mode == "workspace" else None
+    outs = []
+    for _ in range(2):
+        frame = torch.full((M + 2, cols + 8), 7.0, device=DEV, dtype=torch.float32 if mode in ("f32", "f32+") else torch.bfloat16)
+        c = frame[:M, :cols]
+        if mode == "f32+":
+            c.copy_(to_dev(c0))
+        ops.gemm(to_dev(a), to_dev(w), c, accumulate=(mode == "f32+"), silu_mul=(mode == "silu"), workspace=ws)
+        assert (frame[M:] == 7.0).all() and (frame[:, cols:] == 7.0).all()
+        outs.append(c.clone())
+    # a float32 sum of K products of 16-bit numbers, and the rounding of the result to 16 bits
+    tol = 1e-4 * math.sqrt(K) + (2 ** -8) * want.abs().max().item() * (mode in ("bf16", "silu", "workspace"))
+    assert (outs[0].double() - want).abs().max().item() <= tol
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 2056, 64), (32, 2050, 576), (33, 2048, 960), (48, 8250, 1984), (49, 4112, 2048), (64, 5120, 960),
                                    # a wave's most blocks of k; tiles that do not divide among the workgroups; a short k and few tiles
                                    (24, 8240, 4096), (31, 33000, 448), (20, 976, 128), (64, 960, 704), (17, 6152, 2112)])
