@@ -18,7 +18,7 @@
 //
 // Decoding splits a request's context into chunks of a multiple of 256 keys, one workgroup per
 // (chunk, kv head, request), whose waves (sixteen where one workgroup takes a whole context of more
-// than 512 keys and the head size allows, else four) take runs of up to five neighbouring tiles of 64
+// than 512 keys and the head size allows, eight of other whole contexts where workgroups are few, else four) take runs of up to five neighbouring tiles of 64
 // keys, or tiles in turn; partial results are merged in a fixed order (waves in LDS, chunks by a
 // second kernel), so the result is the same on every run and in every row of a step.
 // crates/glassbox-core/src/model.rs:285-312 is the formula.
@@ -926,7 +926,13 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
   // more workgroups on a compute unit: 32 requests of 512 tokens, SmolLM2-1.7B shapes, 32 -> 23 us a layer)
   // (nor for heads above 64: sixteen waves of those have 128 registers each, which the larger heads do not fit
   // without spilling: Llama-3-8B shapes at 32 and 64 requests, 1,500 to 4,096 keys, 15 to 25 % faster with four)
-  const int waves = (splits == 1 && max_context > 512 && hd <= 64 && 16 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) ? 16 : 4;
+  // Eight waves for what is left to four of those, where no unit has a second workgroup whose loads could fill the gaps (us, four / eight
+  // waves: 3 x 1 heads of 64, 300 keys 5.35 / 4.87, 8 x 32 of 512 9.8 / 8.7; heads of 128, 20 x 8 of 600 and 1,000 15.0 / 13.0 and 21.5 /
+  // 19.6, of a quarter to all of 1,000 20.2 / 18.2, 24 x 8 of 1,700 34.5 / 32.1, 32 x 8 of 4,000 88.1 / 86.6); up to 256 keys four
+  // waves have a tile each.
+  const bool plain = ex.softcap <= 0.f && ex.slopes == nullptr && ex.span == 0, alone = n_decode * nkv <= 256;
+  int waves = (splits == 1 && max_context > 512 && hd <= 64 && 16 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) ? 16 : 4;
+  if (waves == 4 && plain && splits == 1 && alone && max_context > 256 && 8 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) waves = 8;
   const size_t lds = (size_t)waves * (32 + (size_t)hd * G) * sizeof(float);
   const dim3 grid(splits, nkv, n_decode), block(waves * 64);
   // capped and sloped scores are kernels of their own (bfloat16 results only), so that the others' score loops are what they were
@@ -955,6 +961,8 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
       else GB_DECODE(HD, 4, kRuns);                                 \
     } else if (waves == 16) {                                       \
       GB_DECODE(HD, 16, kPlainScores);                              \
+    } else if (waves == 8) {                                        \
+      GB_DECODE(HD, 8, kPlainScores);                               \
     } else {                                                        \
       GB_DECODE(HD, 4, kPlainScores);                               \
     }                                                               \

@@ -1824,7 +1824,7 @@ def tuned_attention_supports(k_pages: torch.Tensor, n_heads: int, window: int, k
 @functools.lru_cache(maxsize=4096)   # a pure function of the sizes, asked for at every product
 def decode_chunk(n_decode: int, n_kv_heads: int, max_context: int, head_dim: int = 64) -> int:
     """Keys per workgroup of the decode kernel: a multiple of 256.  A workgroup takes a whole context where there are enough
-    of them for that (sixteen waves each, four where head_dim is above 64 or the context is 512 keys at most), so that
+    of them for that (sixteen waves each, four or eight where head_dim is above 64 or the context is 512 keys at most), so that
     nothing is left to combine afterwards; otherwise small enough that the launch has about a thousand workgroups.
 
     Enough, measured (us, the whole context / chunks and the pass that combines them; requests x kv heads): up to 512 keys

@@ -1317,6 +1317,28 @@ def test_tuned_decode_gives_a_request_the_same_bits_in_every_row_and_head(nkv, G
     assert bool(heads[0].any()) and torch.equal(heads, heads[:1].expand_as(heads))
 
 
+@pytest.mark.parametrize("nh,nkv,hd,lens,bucket,window", [
+    # eight waves: a tile each or none, more tiles than waves in runs and beyond; the most workgroups, and one more
+    (9, 3, 64, [257, 1, 300], 300, 0), (32, 32, 64, [512, 449, 64, 65, 500, 320, 17, 511], 512, 0), (15, 5, 16, [511], 512, 100),
+    (32, 8, 128, [700] * 19 + [1, 129], 768, 0), (16, 8, 96, [2048, 1999] * 12, 2048, 0), (8, 4, 128, [1900] * 64, 2048, 300),
+    (8, 4, 128, [300] * 65, 512, 0)])
+def test_tuned_decode_of_whole_contexts_where_workgroups_are_few(nh, nkv, hd, lens, bucket, window):
+    """Against the plain kernel, which sums a context a chunk of 256 keys after the other."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    n = len(lens)
+    assert ops.decode_chunk(n, nkv, bucket, hd) >= bucket
+    k_pages, v_pages, tables, _, _ = paged_setup(lens, nkv, hd, 16, seed=hd + n, dtype=torch.bfloat16)
+    q = to_dev((rnd(n, nh * hd, seed=6) * 0.7).bfloat16())
+    ctx = BareContext([1] * n, lens, tables, max_context=bucket)
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out, twin = (torch.zeros(n, nh * hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    ops.attention_decode(q, out, ctx, cache, nh, 1 / math.sqrt(hd), window)
+    ops.attention_plain(q, twin, ctx.positions, torch.arange(n, dtype=torch.int32, device=DEV), ctx.tables[0], cache.k_pages,
+                        cache.v_pages, nh, 1 / math.sqrt(hd), window)
+    assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
+
+
 def test_tuned_decode_finds_one_far_key_in_every_chunk_position():
     """One key is made to stand out: first and last slot of a page, chunk edges, the last position."""
     from types import SimpleNamespace
