@@ -392,6 +392,7 @@ class TapeOperands:
             ptrs.append(t.data_ptr())
             sizes.append(span * t.element_size())
         self.sizes = tuple(sizes)
+        self.begins = tuple(p % 16 for p in ptrs)   # (which kernel takes an operand may depend on where in a word it begins)
         self.ptrs = (C.c_uint64 * max(1, n + places))(*ptrs)
         self.bytes = (C.c_uint64 * max(1, n + places))(*sizes)
         self.fixed, self.count = n, n + places
@@ -408,8 +409,10 @@ class TapeOperands:
         self.bytes[self.fixed + i] = t.numel() * t.element_size()
 
     def maps_onto(self, target: "TapeOperands") -> bool:
-        """Whether every pointer into these tensors has one place in ``target``'s: ranges that overlap here must be
-        moved by the same distance (the runner takes the first range that holds a pointer)."""
+        """Whether every pointer into these tensors has one place in ``target``'s, as far into a 16-byte word: ranges that
+        overlap here must be moved by the same distance (the runner takes the first range that holds a pointer)."""
+        if self.begins != target.begins:
+            return False
         for a, b in self.overlaps:
             if target.ptrs[a] - self.ptrs[a] != target.ptrs[b] - self.ptrs[b]:
                 return False
@@ -1653,9 +1656,12 @@ ROPE_PRODUCT_MAX_ROWS = 64
 STEP_F32_MAX_ROWS = 2   # gemm_f32.hip: rows of a step whose products take their neighbours' work (gb_gemm_f32_step)
 
 
-def step_f32_takes(M: int, N: int, K: int, norm: bool) -> bool:
-    """Whether ``gemm_step_f32`` takes a product of M rows by N rows of W of K columns, with the RMS norm before it or without."""
-    return M <= STEP_F32_MAX_ROWS and bool(_lib("gemm_f32").gb_gemm_f32_step_takes(M, N, K, 1 if norm else 0))
+def step_f32_takes(M: int, N: int, K: int, norm: bool, *operands: Optional[torch.Tensor]) -> bool:
+    """Whether ``gemm_step_f32`` takes a product of M rows by N rows of W of K columns, with the RMS norm before it or without;
+    with ``operands`` (the rows, W, the norm's gamma or None) also whether their rows begin at 16-byte words, which it needs and
+    ``gemm`` does not."""
+    return (M <= STEP_F32_MAX_ROWS and all(t is None or (t.data_ptr() % 16 == 0 and (t.dim() < 2 or t.stride(0) % 4 == 0)) for t in operands)
+            and bool(_lib("gemm_f32").gb_gemm_f32_step_takes(M, N, K, 1 if norm else 0)))
 
 
 def gemm_step_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms: Optional[tuple] = None, silu_mul: bool = False,
@@ -1670,9 +1676,9 @@ def gemm_step_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rms: Opti
     N = w.shape[0]
     if any(t.dtype != torch.float32 for t in (a, w, out)) or w.shape[1] != K or out.shape != (M, N // 2 if silu_mul else N):
         raise KernelError(f"gemm_step_f32: float32 of matching shapes: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
-    if not step_f32_takes(M, N, K, rms is not None) or (silu_mul and heads is not None):
-        raise KernelError(f"gemm_step_f32: not for {M} rows by {N} rows of {K} (step_f32_takes), or two epilogues at once")
     gamma, eps = rms if rms is not None else (None, 0.0)
+    if not step_f32_takes(M, N, K, rms is not None, a, w, gamma) or (silu_mul and heads is not None):
+        raise KernelError(f"gemm_step_f32: not for {M} rows by {N} rows of {K} (step_f32_takes), or two epilogues at once")
     if gamma is not None and (gamma.dtype != torch.float32 or gamma.numel() != K or not gamma.is_contiguous()):
         raise KernelError("gemm_step_f32: the norm takes a contiguous float32 gamma of K entries")
     nh = nkv = hd = page_size = 0

@@ -140,12 +140,12 @@ class PagedAttention(Mixer):
             tables = self.position.fuse_spec(ctx, self.head_dim)
         one_launch, takes = None, False   # 32-bit steps of one or two rows: norm, product, rotation and cache write in one
         if ctx.dtype == torch.float32:
-            takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, norm is not None)
+            takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, norm is not None, h, self.wqkv, norm[0] if norm is not None else None)
             if norm is not None and not takes:   # nothing to fuse it into here: the norm gets its own pass after all
                 normed = ctx.buffer("h", (n, self.width), ctx.dtype)
                 ops.rmsnorm(h, norm[0], norm[1], normed)
                 h, norm = normed, None
-                takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, False)
+                takes = ctx.tuned and ops.step_f32_takes(n, rows, self.width, False, h, self.wqkv)
             if takes and self.head_dim % 2 == 0:
                 one_launch = self.position.fuse_spec(ctx, self.head_dim)
         if one_launch is not None:

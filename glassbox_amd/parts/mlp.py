@@ -63,7 +63,8 @@ class SwiGLU(FeedForward):
             # the activation is applied where the product's tile is finished: gate_up never reaches memory
             ops.gemm(h, self.w_gate_up, act, silu_mul=True, rms=norm,
                      workspace=None if norm is not None else split_workspace(ctx, n, 2 * self.intermediate, self.width))
-        elif ctx.dtype == torch.float32 and ctx.tuned and ops.step_f32_takes(n, 2 * self.intermediate, self.width, norm is not None):
+        elif ctx.dtype == torch.float32 and ctx.tuned and ops.step_f32_takes(n, 2 * self.intermediate, self.width, norm is not None, h,
+                                                                              self.w_gate_up, norm[0] if norm is not None else None):
             ops.gemm_step_f32(h, self.w_gate_up, act, rms=norm, silu_mul=True)
         else:
             if norm is not None:   # nothing to fuse it into here: the norm gets its own pass after all

@@ -10,8 +10,8 @@ other kernels, and the recorded layer has decided that in the ordinary way.
 What makes two layers of a kind is decided here, from the parts themselves, and checked again before each replay:
 
 * the block says ``all_taped()``: every part in it does all of its device work through ``glassbox_amd.ops``,
-  and decides what to launch by nothing but the step (``ctx``), its own constants and the arguments of its
-  ``forward`` (``Part.taped``);
+  and decides what to launch by nothing but the step (``ctx``), its own constants, the arguments of its
+  ``forward`` and where in a 16-byte word its tensors begin (``Part.taped``);
 * the blocks have one ``signature``: the same classes, arranged alike, with the same constants (every
   attribute that is a number, a string, a truth value or a tuple or list of such, but for those whose names begin
   with an underscore; an attribute of any other kind, tensors and parts aside, makes blocks differ unless they hold
@@ -22,7 +22,7 @@ What makes two layers of a kind is decided here, from the parts themselves, and 
   norm to be prepared, the kind and shapes of the cache layer, the residual buffer (or, in a model that keeps every
   layer's residual in a buffer of its own, ``moving``, its shape: the residual is then one of the tensors exchanged);
 * their tensors (the attributes of the parts that are tensors, the cache layer's pages and state, the gamma of a
-  norm to prepare), listed in the same order, have the same sizes.
+  norm to prepare), listed in the same order, have the same sizes and begin at the same place in a 16-byte word.
 
 A pointer in a recorded launch that points into the n-th tensor of the recorded layer is replaced by the same
 place in the n-th tensor of the layer at hand; every other argument (buffers of the step's workspace, the step's
@@ -214,8 +214,8 @@ class LayerTapes:
             target = site.tensors(moved)
             fits = lambda r: target.sizes == r.operands.sizes and r.operands.maps_onto(target)
             if not fits(rec):
-                # a part of this layer has not made a tensor that the recorded layer's part made on its walk, or a tensor
-                # that the recorded layer held in two places is two tensors here: a kind by itself
+                # a part of this layer has not made a tensor that the recorded layer's part made on its walk, a tensor
+                # that the recorded layer held in two places is two tensors here, or one begins elsewhere in a word: a kind by itself
                 key = (key, target.sizes)
                 rec = self.records.get(key)
             if rec is not None and rec.epoch == epoch and fits(rec):

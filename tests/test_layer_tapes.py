@@ -163,6 +163,21 @@ def test_a_tensor_held_in_two_places_must_go_to_one_tensor():
     assert ops.TapeOperands([big, big[8:24]]).overlaps == [(0, 1)]
 
 
+def test_a_tensor_that_begins_elsewhere_in_a_word_makes_a_layer_another_kind():
+    """Which kernel a part launches may depend on whether its operands begin at 16-byte words."""
+    def at(elements):
+        room = torch.zeros(72)
+        first = (-room.data_ptr() // 4) % 4 + elements
+        return room[first:first + 64]
+    recorded = ops.TapeOperands([at(0), at(1)])
+    assert recorded.maps_onto(ops.TapeOperands([at(0), at(1)])) and recorded.maps_onto(ops.TapeOperands([at(4), at(5)]))
+    assert not recorded.maps_onto(ops.TapeOperands([at(0), at(0)])) and not recorded.maps_onto(ops.TapeOperands([at(1), at(1)]))
+    tape = ops.start_tape()
+    ops.stop_tape()
+    with pytest.raises(ops.KernelError, match="do not match"):
+        ops.run_tape(tape, recorded, ops.TapeOperands([at(0), at(0)]))
+
+
 def test_a_layers_tensors_come_in_one_order_and_include_cache_and_the_next_norm():
     a, b = block(), block()
     load_random(a)

@@ -107,6 +107,49 @@ def test_attention_part_with_rotary(model_dirs, window):
         at += n
 
 
+@pytest.mark.parametrize("what", ["weight", "rows", "gamma"])
+@pytest.mark.parametrize("normed", [False, True])
+def test_parts_of_single_32_bit_rows_take_operands_that_begin_inside_a_word(model_dirs, what, normed):
+    """A matrix, rows or a norm's weight that begin 4 bytes behind a 16-byte word (views into something larger), in a step of
+    one row, whose products otherwise do their neighbours' work too: the bits of the aligned ones."""
+    from glassbox_amd import ops
+    from glassbox_amd.parts.attention import PagedAttention
+    from glassbox_amd.parts.base import LayerCache
+    from glassbox_amd.parts.mlp import SwiGLU
+    from glassbox_amd.parts.rotary import NoPosition
+    eng = bare_engine(model_dirs.get("A"))
+    ctx, _ = context_for(eng, [1])
+    d, nh, nkv, hd, inter = 64, 6, 2, 16, 96
+    assert ctx.tuned and ops.step_f32_takes(1, nh * hd, d, normed) and ops.step_f32_takes(1, 2 * inter, d, normed)
+    w = {"q_proj.weight": rnd(nh * hd, d, seed=1, scale=0.3), "o_proj.weight": rnd(d, nh * hd, seed=4, scale=0.2)}
+    m = {"gate_proj.weight": rnd(inter, d, seed=5), "up_proj.weight": rnd(inter, d, seed=6), "down_proj.weight": rnd(d, inter, seed=7)}
+    h, gamma = rnd(1, d, seed=8), rnd(d, seed=9) + 1
+
+    def place(t, inside):
+        room = torch.empty(t.numel() + 1, device=DEV)
+        out = room[1:].view(t.shape) if inside else torch.empty(t.shape, device=DEV)
+        assert out.data_ptr() % 16 == (4 if inside else 0)
+        return out.copy_(t)
+
+    cache = LayerCache(torch.zeros(ops.key_pages_shape(32, nkv, 16, hd), device=DEV), torch.zeros(32, nkv, hd, 16, device=DEV), 0)
+    outs = []
+    for off in (False, True):
+        rows, g = place(h, off and what == "rows"), place(gamma, off and what == "gamma")
+        norm = dict(norm=(g, 1e-5)) if normed else {}
+        attn = PagedAttention(d, nh, nkv, hd, NoPosition(), shares_kv=True)
+        attn.load({k: place(v, off and what == "weight" and k[0] == "q") for k, v in w.items()})
+        ffn = SwiGLU(d, inter)
+        ffn.load({k: place(v, False) for k, v in m.items()})
+        if off and what == "weight":
+            ffn.w_gate_up = place(ffn.w_gate_up, True)
+        x, y = torch.zeros(1, d, device=DEV), torch.zeros(1, d, device=DEV)
+        attn.forward(ctx, rows, x, cache, **norm)
+        ffn.forward(ctx, rows, y, **norm)
+        outs.append((x, y))
+    assert outs[0][1].any()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
 # ------------------------------------------------------------------- the toy architecture
 def register_toy():
     """Everything the toy needs, defined here: configuration, a stateful mixer, the builder."""
