@@ -359,30 +359,40 @@ __global__ __launch_bounds__(256, WN == 2 ? 2 : 1) void gemm_tiled_kernel(const 
     }
 }
 
-// Tile of the workgroup, 128 x (64 WN), and the depth of the register prefetch.  128 x 128 re-reads
+// Tile of the workgroup, bm x (64 wn), how many there are, and the depth of the register prefetch.  128 x 128 re-reads
 // the operands least; 128 x 64 when that would leave compute units idle.  The wide tile's registers
 // allow two workgroups a compute unit only with one k-step of prefetch, the narrow tile's with two.
-inline void tiled_plan(int M, int N, int* wn, int* depth) {
-  const int blocks = ((M + 127) / 128) * ((N + 127) / 128);
-  *wn = blocks < 384 ? 1 : 2;
-  *depth = *wn == 1 ? 2 : 1;
+// Tiles of 64 rows where those of 128 would leave a third of the compute units without a workgroup (the
+// products of a narrow model at some hundred rows): a workgroup's time is its k-steps' arithmetic, and half the
+// rows halve it.  A SiLU-multiply product, whose workgroups take 128 rows of W each, gains up to 300 workgroups
+// (two of the smaller ones share a compute unit: gate/up of 256 rows on SmolLM2-1.7B shapes 34 -> 30 us, of 640 to
+// 896 rows on SmolLM2-360M shapes 17 -> 14 and 24 -> 20 us; the other products lose from 168 on).
+struct TiledGrid {
+  int wn, depth, bm, cols, rows;   // cols x rows workgroups
+  long long groups() const { return (long long)cols * rows; }
+};
+inline TiledGrid tiled_grid(int epi, int M, int N) {
+  const long long blocks = (long long)((M + 127) / 128) * ((N + 127) / 128);
+  TiledGrid g;
+  g.wn = blocks < 384 ? 1 : 2;
+  g.depth = g.wn == 1 ? 2 : 1;
+  if (epi == EPI_SILU_MUL) g.wn = 2;  // a wave's two column tiles are gate and up
+  const int cols = epi == EPI_SILU_MUL ? N / 2 : N, bn = epi == EPI_SILU_MUL ? 64 : 64 * g.wn;
+  g.cols = (cols + bn - 1) / bn;
+  const bool low = M > 64 && (long long)g.cols * ((M + 127) / 128) < (epi == EPI_SILU_MUL ? 300 : 168);
+  g.bm = low ? 64 : 128;
+  if (low) g.depth = g.wn == 1 ? 2 : 1;
+  g.rows = (M + g.bm - 1) / g.bm;
+  return g;
 }
 
 template <int EPI, typename CT>
 int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, hipStream_t stream,
                  Glu glu = Glu{}) {
-  int wn, depth;
-  tiled_plan(M, N, &wn, &depth);
-  if (EPI == EPI_SILU_MUL) wn = 2;  // a wave's two column tiles are gate and up
-  const int cols = EPI == EPI_SILU_MUL ? N / 2 : N, bn = EPI == EPI_SILU_MUL ? 64 : 64 * wn;
-  // Tiles of 64 rows where those of 128 would leave a third of the compute units without a workgroup (the
-  // products of a narrow model at some hundred rows): a workgroup's time is its k-steps' arithmetic, and half the
-  // rows halve it.  A SiLU-multiply product, whose workgroups take 128 rows of W each, gains up to 300 workgroups
-  // (two of the smaller ones share a compute unit: gate/up of 256 rows on SmolLM2-1.7B shapes 34 -> 30 us, of 640 to
-  // 896 rows on SmolLM2-360M shapes 17 -> 14 and 24 -> 20 us; the other products lose from 168 on).
-  const bool low = M > 64 && ((cols + bn - 1) / bn) * ((M + 127) / 128) < (EPI == EPI_SILU_MUL ? 300 : 168);
-  const int bm = low ? 64 : 128;
-  const dim3 grid((cols + bn - 1) / bn, (M + bm - 1) / bm), block(256);
+  const TiledGrid g = tiled_grid(EPI, M, N);
+  const int wn = g.wn, depth = g.depth;
+  const bool low = g.bm == 64;
+  const dim3 grid(g.cols, g.rows), block(256);
   GB_REQUIRE(grid.y <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
   const bool kfull = K % TBK == 0;  // then no load needs a check against K
 #define GB_T(WM, B, D)                                                                                                      \
@@ -395,7 +405,6 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
                          M, N, K, 0, Groups{}, glu);                                                                                       \
   }
   if (low) {
-    depth = wn == 1 ? 2 : 1;
     GB_T(1, 2, 1)
     if (EPI != EPI_SILU_MUL) { GB_T(1, (EPI == EPI_SILU_MUL ? 2 : 1), 2) }
   } else {
@@ -1330,6 +1339,7 @@ struct SplitPlan {
   bool ring;      // the ring kernel's 256 x 256 tiles, if the operands allow (else the tiled kernel's, same slices)
   bool held;      // the held kernel's tiles of 16 rows of W, if the operands allow (else the tiled kernel's, same slices)
   int rm, cn;     // the block kernel's tiles of 32 rm x 32 cn, if the operands allow (else the tiled kernel's, same slices); 0: not
+  float us;       // with those, block_plan's estimate
 };
 
 // Slices of k for the held kernel where its tiles alone are few (the O and down projections of 17 to 64 rows): four tiles a workgroup and
@@ -1348,7 +1358,7 @@ inline int held_slices(int M, int N, int K) {
   return want < least ? least : want;
 }
 inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
-  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false, 0, 0};
+  SplitPlan p{M <= 64 ? 64 : 128, 1, 0, 0, false, false, 0, 0, 0.f};
   if (M > 16 && M <= 64 && K % 64 == 0 && N % 8 == 0 && !silu && held_slices(M, N, K) > 1) {
     p.k_slice = held_slice(K, held_slices(M, N, K));
     p.slices = (K + p.k_slice - 1) / p.k_slice;
@@ -1361,7 +1371,7 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
     if (!block_sizes(M, N, K, silu)) return p;
     const BlockPlan b = block_plan(M, N, K, false, 2, 8);
     if (!b.rm || (p.ring && (M >= 1024 || ring_us(M, N, K, p.slices) <= b.us))) return p;
-    return SplitPlan{p.bm, b.slices, b.k_slice, (size_t)b.slices * M * N, false, false, b.rm, b.cn};
+    return SplitPlan{p.bm, b.slices, b.k_slice, (size_t)b.slices * M * N, false, false, b.rm, b.cn, b.us};
   };
   // many rows, a long k and few 256 x 256 tiles (the down projection of a prompt): slices of k fill the
   // chip with the ring kernel's tiles once; a slice keeps 1,024 of k or more
@@ -1396,7 +1406,7 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
   if (want < 2) return p;
   p.k_slice = ((K + want - 1) / want + TBK - 1) / TBK * TBK;
   p.slices = (K + p.k_slice - 1) / p.k_slice;
-  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, 0, 0};
+  if (p.slices < 2) return SplitPlan{p.bm, 1, 0, 0, false, false, 0, 0, 0.f};
   p.floats = (size_t)p.slices * M * N;
   // tiles of 64 rows where even with the slices a third of the compute units would have no workgroup
   if (tiles * p.slices < 168) p.bm = 64;
@@ -2218,6 +2228,38 @@ int launch_skinny(const void* a, int lda, const bf16* w, int ldw, CT* c, int ldc
   return launch_skinny_mt<4, EPI, RMS, CT>(tiles, a, lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rope, stream);
 }
 
+// Which kernel takes a product, and how.  `emits`: emit_mode if the next norm is to be prepared, else 0; `workspace`: one is there.
+enum : int { kTiled = 0, kRing = 1, kFew = 2 /* skinny or folded */, kHeld = 3, kBlock = 4, kSlices = 5 };
+struct Route {
+  int kernel;
+  BlockPlan block;   // the block kernel's tile for the whole product, where it may take it
+  SplitPlan split;   // the slices that were on offer (kSlices: taken)
+};
+inline Route route(int epi, const void* a, int lda, const void* w, int ldw, int M, int N, int K, bool gamma, bool parts, int emits, bool workspace) {
+  Route r{kTiled, BlockPlan{}, SplitPlan{}};
+  const bool silu = epi == EPI_SILU_MUL;
+  const bool held = !gamma && !emits && epi != EPI_ACCUMULATE && held_pays(epi, M, N, K) && held_takes(a, lda, w, ldw, M, K);
+  const bool blocks = !held && !gamma && !parts && block_sizes(M, N, K, silu) && block_takes(a, lda, w, ldw, K);
+  const bool rings = ring_pays(epi, a, lda, w, ldw, M, N, K);
+  if (blocks) r.block = block_plan(M, N, K, silu, 1, 1);
+  if (workspace && M > 16 && !gamma && emits != 1 && !parts) {  // more than the skinny kernels' best range
+    r.split = split_plan(M, N, K, silu);
+    if (r.split.slices <= 1 || (silu && N % 16 != 0)) r.split = SplitPlan{};
+    // a product that only stores needs no second pass: not divided where that takes less (QKV, 131 x 6,144 x 2,048: 16 us in slices, 13 whole)
+    const bool whole = blocks && epi != EPI_ACCUMULATE && r.split.rm && r.block.us < r.split.us;
+    if (r.split.slices > 1 && !held && !whole) return r.kernel = kSlices, r;
+  }
+  if (held) return r.kernel = kHeld, r;
+  if (blocks && (M > 64 || epi != EPI_ACCUMULATE) && !emits && (!rings || r.block.us < ring_us(M, N, K, 1))) return r.kernel = kBlock, r;
+  // 17 to 64 rows by very many rows of W that the held kernel does not take (a long k): measured twice as fast
+  // through the tiles as through the skinny kernel with four column blocks (49,152 x 2,048: 102 -> about 50 us),
+  // and with two column blocks as fast or faster (49,152 x 960 at 17 to 32 rows: 30 -> 25 us)
+  const bool wide_head = M > 16 && N >= 32768 && !gamma && !parts;
+  if (M <= 64 && !wide_head) return r.kernel = kFew, r;
+  if (rings) r.kernel = kRing;
+  return r;
+}
+
 }  // namespace
 
 // epilogue: 0 store, 1 accumulate (float32 C), 2 SiLU-multiply of stacked gate/up rows (C is [M, N/2]).
@@ -2265,6 +2307,13 @@ extern "C" int gb_gemm_bf16_partial(const void* a, int lda, const void* w, int l
                                         nullptr, 0.f, false);
 }
 
+// The kernel that gb_gemm_bf16 (epilogues 0 to 2, no gamma, no norm to prepare; with a workspace or without) or gb_gemm_bf16_rope
+// (epilogue 3, no gamma) launches for these sizes: 0 tiled, 1 ring, 2 skinny or folded, 3 held, 4 block, 5 slices of k.
+extern "C" int gb_gemm_bf16_route(int M, int N, int K, int epilogue, int parts, int workspace) {
+  if (epilogue == EPI_ROPE) return held_pays(epilogue, M, N, K) && held_takes(nullptr, K, nullptr, K, M, K) ? kHeld : kFew;
+  return route(epilogue, nullptr, K, nullptr, K, M, N, K, false, parts != 0, 0, workspace != 0).kernel;
+}
+
 extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void* c, int ldc, int c_dtype, int M, int N,
                             int K, int epilogue, const void* gamma, int gamma_dtype, float eps, const void* emit_gamma,
                             int emit_gamma_dtype, void* emit_h, int emit_ldh, float* emit_ss, const float* parts, int n_parts,
@@ -2292,92 +2341,57 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
   const NormExtras extra{emit_gamma, emit_gamma_dtype == kF32, (bf16*)emit_h, emit_ldh, emit_ss, parts, n_parts};
   if (M == 0) return 0;
   const bf16* W = (const bf16*)w;
-  const bool held = !gamma && !emit_h && epilogue != EPI_ACCUMULATE && held_pays(epilogue, M, N, K) && held_takes(a, lda, w, ldw, M, K);
-  const bool blocks = !held && !gamma && !parts && block_sizes(M, N, K, epilogue == EPI_SILU_MUL) && block_takes(a, lda, w, ldw, K);
-  const bool rings = ring_pays(epilogue, a, lda, w, ldw, M, N, K);
-  const BlockPlan undivided = blocks ? block_plan(M, N, K, epilogue == EPI_SILU_MUL, 1, 1) : BlockPlan{};
-  // a product that only stores needs no second pass: not divided where that takes less (QKV, 131 x 6,144 x 2,048: 16 us in slices, 13 whole)
-  auto whole = [&](const SplitPlan& plan) {
-    return blocks && epilogue != EPI_ACCUMULATE && plan.rm && undivided.us < block_plan(M, N, K, false, 2, 8).us;
-  };
-  if (split_ws != nullptr && M > 16 && !gamma && (!emit_h || emits == 2) && !parts) {  // more than the skinny kernels' best range
-    const SplitPlan plan = split_plan(M, N, K, epilogue == EPI_SILU_MUL);
-    if (plan.slices > 1 && (epilogue != EPI_SILU_MUL || N % 16 == 0) && (uintptr_t)split_ws % 16 == 0) {
-      GB_REQUIRE((long long)plan.floats <= split_ws_floats, "gemm_bf16: the split-k workspace holds %lld floats, %zu are needed",
-                 split_ws_floats, plan.floats);
-      const bf16* A = (const bf16*)a;
-#define GB_SP(EPI, CT) return launch_split<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, split_ws, plan, stream)
-      if (epilogue == EPI_ACCUMULATE)
-        return launch_split<EPI_ACCUMULATE, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, split_ws, plan, stream, &extra, eps);
-      if (!held && !whole(plan)) {
-        if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_SP(EPI_SILU_MUL, bf16);
-        if (epilogue == EPI_SILU_MUL) GB_SP(EPI_SILU_MUL, float);
-        if (c_dtype == kF32) GB_SP(EPI_STORE, float);
-        GB_SP(EPI_STORE, bf16);
-      }
-#undef GB_SP
-    }
-  }
-  if (held) {
-    const bf16* A = (const bf16*)a;
-#define GB_HD(EPI, CT) return launch_held<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream)
-    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_HD(EPI_SILU_MUL, bf16);
-    if (epilogue == EPI_SILU_MUL) GB_HD(EPI_SILU_MUL, float);
-    if (c_dtype == kF32) GB_HD(EPI_STORE, float);
-    GB_HD(EPI_STORE, bf16);
-#undef GB_HD
-  }
-  if (blocks && (M > 64 || epilogue != EPI_ACCUMULATE) && !emit_h && (!rings || undivided.us < ring_us(M, N, K, 1))) {
-    const bf16* A = (const bf16*)a;
-#define GB_BK(EPI, CT) return launch_block<EPI, CT>(undivided.rm, undivided.cn, A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
-    if (epilogue == EPI_ACCUMULATE) GB_BK(EPI_ACCUMULATE, float);
-    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_BK(EPI_SILU_MUL, bf16);
-    if (epilogue == EPI_SILU_MUL) GB_BK(EPI_SILU_MUL, float);
-    if (c_dtype == kF32) GB_BK(EPI_STORE, float);
-    GB_BK(EPI_STORE, bf16);
-#undef GB_BK
-  }
-  // 17 to 64 rows by very many rows of W that the held kernel does not take (a long k): measured twice as fast
-  // through the tiles below as through the skinny kernel with four column blocks (49,152 x 2,048: 102 -> about 50 us),
-  // and with two column blocks as fast or faster (49,152 x 960 at 17 to 32 rows: 30 -> 25 us)
-  const bool wide_head = M > 16 && N >= 32768 && !gamma && !parts;
-  if (M <= 64 && !wide_head) {
-    const int gf = gamma_dtype == kF32;
-    if (fold_pays(M, N) && epilogue != EPI_SILU_MUL && !parts) {
-      if (gamma) return launch_fold<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
-      if (epilogue == EPI_ACCUMULATE) return launch_fold<EPI_ACCUMULATE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
-      if (c_dtype == kF32) return launch_fold<EPI_STORE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
-      return launch_fold<EPI_STORE, false, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
-    }
-    if (gamma) {
-      if (epilogue == EPI_STORE) return launch_skinny<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
-      return launch_skinny<EPI_SILU_MUL, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
-    }
-#define GB_SK(EPI, CT) return launch_skinny<EPI, false, CT>(a, lda, W, ldw, (CT*)c, ldc, M, N, K, nullptr, 0, eps, extra, stream)
-    if (epilogue == EPI_STORE && c_dtype == kF32) GB_SK(EPI_STORE, float);
-    if (epilogue == EPI_STORE && c_dtype == kBF16) GB_SK(EPI_STORE, bf16);
-    if (epilogue == EPI_ACCUMULATE) GB_SK(EPI_ACCUMULATE, float);
-    if (epilogue == EPI_SILU_MUL && c_dtype == kF32) GB_SK(EPI_SILU_MUL, float);
-    GB_SK(EPI_SILU_MUL, bf16);
-#undef GB_SK
-  }
+  const Route r = route(epilogue, a, lda, w, ldw, M, N, K, gamma != nullptr, parts != nullptr, emits, split_ws != nullptr && (uintptr_t)split_ws % 16 == 0);
+  GB_REQUIRE((long long)r.split.floats <= split_ws_floats, "gemm_bf16: the split-k workspace holds %lld floats, %zu are needed",
+             split_ws_floats, r.split.floats);
   const bf16* A = (const bf16*)a;
-  if (ring_pays(epilogue, a, lda, w, ldw, M, N, K) && (epilogue != EPI_SILU_MUL || N % 2 == 0)) {
-#define GB_RG(EPI, CT) return launch_ring<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
-    if (epilogue == EPI_ACCUMULATE) GB_RG(EPI_ACCUMULATE, float);
-    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_RG(EPI_SILU_MUL, bf16);
-    if (epilogue == EPI_SILU_MUL) GB_RG(EPI_SILU_MUL, float);
-    if (c_dtype == kF32) GB_RG(EPI_STORE, float);
-    GB_RG(EPI_STORE, bf16);
-#undef GB_RG
+// (the launch, once for each epilogue and type of C that there is)
+#define GB_EACH(LAUNCH)                                                              \
+  if (epilogue == EPI_ACCUMULATE) return LAUNCH(EPI_ACCUMULATE, float);              \
+  if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) return LAUNCH(EPI_SILU_MUL, bf16); \
+  if (epilogue == EPI_SILU_MUL) return LAUNCH(EPI_SILU_MUL, float);                  \
+  if (c_dtype == kF32) return LAUNCH(EPI_STORE, float);                              \
+  return LAUNCH(EPI_STORE, bf16);
+#define GB_SP(EPI, CT) launch_split<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, split_ws, r.split, stream, &extra, eps)
+#define GB_HD(EPI, CT) launch_held<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream)
+#define GB_BK(EPI, CT) launch_block<EPI, CT>(r.block.rm, r.block.cn, A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
+#define GB_RG(EPI, CT) launch_ring<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
+#define GB_TL(EPI, CT) launch_tiled<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
+  switch (r.kernel) {
+    case kSlices: GB_EACH(GB_SP)
+    case kHeld:
+      if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) return GB_HD(EPI_SILU_MUL, bf16);
+      if (epilogue == EPI_SILU_MUL) return GB_HD(EPI_SILU_MUL, float);
+      if (c_dtype == kF32) return GB_HD(EPI_STORE, float);
+      return GB_HD(EPI_STORE, bf16);
+    case kBlock: GB_EACH(GB_BK)
+    case kRing: GB_EACH(GB_RG)
+    case kTiled: GB_EACH(GB_TL)
   }
-#define GB_TL(EPI, CT) return launch_tiled<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
-  if (epilogue == EPI_ACCUMULATE) GB_TL(EPI_ACCUMULATE, float);
-  if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) GB_TL(EPI_SILU_MUL, bf16);
-  if (epilogue == EPI_SILU_MUL) GB_TL(EPI_SILU_MUL, float);
-  if (c_dtype == kF32) GB_TL(EPI_STORE, float);
-  GB_TL(EPI_STORE, bf16);
 #undef GB_TL
+#undef GB_RG
+#undef GB_BK
+#undef GB_HD
+#undef GB_SP
+#undef GB_EACH
+  const int gf = gamma_dtype == kF32;
+  if (fold_pays(M, N) && epilogue != EPI_SILU_MUL && !parts) {
+    if (gamma) return launch_fold<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
+    if (epilogue == EPI_ACCUMULATE) return launch_fold<EPI_ACCUMULATE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
+    if (c_dtype == kF32) return launch_fold<EPI_STORE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
+    return launch_fold<EPI_STORE, false, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
+  }
+  if (gamma) {
+    if (epilogue == EPI_STORE) return launch_skinny<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
+    return launch_skinny<EPI_SILU_MUL, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
+  }
+#define GB_SK(EPI, CT) return launch_skinny<EPI, false, CT>(a, lda, W, ldw, (CT*)c, ldc, M, N, K, nullptr, 0, eps, extra, stream)
+  if (epilogue == EPI_STORE && c_dtype == kF32) GB_SK(EPI_STORE, float);
+  if (epilogue == EPI_STORE && c_dtype == kBF16) GB_SK(EPI_STORE, bf16);
+  if (epilogue == EPI_ACCUMULATE) GB_SK(EPI_ACCUMULATE, float);
+  if (epilogue == EPI_SILU_MUL && c_dtype == kF32) GB_SK(EPI_SILU_MUL, float);
+  GB_SK(EPI_SILU_MUL, bf16);
+#undef GB_SK
 }
 
 // A product whose epilogue is the clamped gated unit (see Glu): W stacks gate rows over up rows as for epilogue 2, C is

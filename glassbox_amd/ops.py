@@ -218,6 +218,7 @@ _SIGS = {
         "gb_gemm_bf16_glu": [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _f, _f, _f, _vp],
         "gb_gemm_bf16_split_floats": [_i, _i, _i],
         "gb_gemm_bf16_slices": [_i, _i, _i],
+        "gb_gemm_bf16_route": [_i, _i, _i, _i, _i, _i],
         # a, lda, w, ldw, workspace, its floats, M, N, K, stream
         "gb_gemm_bf16_partial": [_vp, _i, _vp, _i, _vp, C.c_longlong, _i, _i, _i, _vp],
         "gb_gemm_bf16_emit_parts": [_i, _i],
@@ -1498,6 +1499,15 @@ def gemm_split_floats(rows: int, n: int, k: int) -> int:
     f = _lib("gemm_bf16").gb_gemm_bf16_split_floats
     f.restype = C.c_longlong
     return int(f(int(rows), int(n), int(k)))
+
+
+def gemm_route(rows: int, n: int, k: int, silu_mul: bool = False, accumulate: bool = False, heads: bool = False, parts: bool = False,
+               workspace: bool = False) -> str:
+    """The kernel that ``gemm`` (``heads``: ``gemm_rope``) launches for a bfloat16 product of these sizes and options, without a norm to
+    do or to prepare: "tiled", "ring", "few" (the skinny or the folded kernel), "held", "block" or "slices" (of k)."""
+    epilogue = 3 if heads else 2 if silu_mul else 1 if accumulate else 0
+    return ("tiled", "ring", "few", "held", "block", "slices")[_lib("gemm_bf16").gb_gemm_bf16_route(
+        int(rows), int(n), int(k), epilogue, int(parts), int(workspace))]
 
 
 def gemm_slices(rows: int, n: int, k: int) -> int:
