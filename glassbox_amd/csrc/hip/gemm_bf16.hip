@@ -1291,24 +1291,47 @@ inline int held_groups(int tiles, int slices) {
   const int room = 256 / slices, each = (tiles + room - 1) / room;
   return (tiles + each - 1) / each;
 }
-// Where it pays (us, the skinny kernel, the wide tiles or narrow ones before / this one, each product alone):
+// Where it pays (us, the skinny kernel, the wide tiles or narrow ones before / this one, each product alone, weights cold):
 //   gate/up 28,672 x 4,096, 17 / 24 / 32 rows: 53 / 57 / 62 -> 42 / 45 / 45 (5.2 to 5.5 TB/s); vocabulary 128,256 x 4,096,
 //   24 rows: 242 -> 176 (6 TB/s); gate/up 16,384 x 2,048, 20 / 33 / 64 rows: 19 / 21.6 / 20.8 -> 15.7 / 17 / 18; gate/up 5,120 x 960
-//   behind partial sums of a norm, 20 / 53 rows: 8.6 / 12.5 -> 8.2 / 8.8; QKV 6,144 x 4,096, 24 rows 17.2 -> 15.3; 6,144 x 2,048,
-//   20 / 64 rows 11.2 / 16.7 -> 10.3 / 13.3.
-// Few tiles: a workgroup's rows of A are then more than its rows of W, and where a k of 960 is one block each for the sixteen waves of the
-// skinny kernel, those bring both as fast (QKV 1,600 x 960, 100 tiles, 53 rows: 6.6 -> 7.1; 3,072 x 960 with the unit, 192 tiles, 33 rows
-// 5.7 -> 5.9; 4,096 x 960 5.7 -> 5.7; a storing product of 160 tiles, which goes there in halves, 33 rows: 6.2 -> 5.5, of 128 tiles 4.6 ->
-// 5.4).  A longer k is several round trips there: from 2,048 on this one is ahead at 128 tiles (33 rows 8.7 -> 6.9, in slices of k before;
-// 17 rows 6.4 -> 5.8).  Of a k below 768 those are four waves, and this one's eight are ahead (960 x 576, 60 tiles, 53 rows: 7.1 -> 6.2).
+//   behind partial sums of a norm, 53 rows: 12.5 -> 8.8; QKV 6,144 x 4,096, 24 rows 17.2 -> 15.3; 6,144 x 2,048, 20 / 64 rows
+//   11.2 / 16.7 -> 10.3 / 13.3.
+// What it saves is A, read once a workgroup and not once a tile or two: as many bytes as k and rows are large.  What it costs is the
+// same for any k: the ring's start and, a tile, eight waves' sums that meet.  So it is ahead from a k on that is the smaller the
+// more rows there are, the more the other kernel spends on a row (a norm's scale, the rotation) and the more tiles a workgroup has; where
+// other kernels take the rows another way too (the block kernel a gated unit of 33 rows and more, the tiled one a vocabulary),
+// from a larger one.  held_from gives that k; it was read off times of both at 64 <= k <= 4,096, 17 to 64 rows and 60 to 2,048 tiles (of
+// 9,600 products it takes 1 % that are more than 4 % slower here, and leaves 7 % that would be more than 4 % faster).  us, the other
+// kernel / this one, at the sides of a line: 256 tiles of a storing product, 24 rows, k 1,280 / 1,536: 5.4 / 5.7, 6.6 / 6.1; 300 tiles of a
+// gated unit behind a norm, 24 rows, k 960 / 1,280: 7.5 / 7.9, 10.3 / 8.8; 64 rows, k 320 / 576: 8.3 / 8.2, 9.8 / 8.6.
+// A k of 128: 2.9 / 4.4 at 257 tiles.  Few tiles (up to 256, one a workgroup): a workgroup's rows of A are then more than its rows of
+// W, and the skinny kernel's sixteen waves (a k of 768 and more) bring both as fast until a k is several round trips there; its four (a
+// shorter k) are behind from 576 on (960 x 576, 53 rows: 7.1 -> 6.2), and so are its half tiles of storing products from 160 tiles on.
 inline int held_tiles(int epi, int N) { return epi == EPI_SILU_MUL ? (N / 2 + 7) / 8 : (N + 15) / 16; }
-inline bool held_pays(int epi, int M, int N, int K) {
+inline int held_from(int epi, int M, int tiles, int K, bool parts) {
+  const int mt = (M + 15) / 16;
+  const bool heads = epi == EPI_ROPE || (epi == EPI_STORE && parts);
+  if (tiles <= 256) {
+    if (K < 768) {
+      if (mt == 2 || !(parts || (epi == EPI_STORE && tiles >= 160 && tiles < 256))) return 576;
+      return mt == 4 && parts ? 64 : 320;
+    }
+    if (epi == EPI_STORE && !parts && tiles == 256) return mt == 2 ? 1536 : 1024;
+    return mt == 2 && tiles < 160 ? 3072 : 768;
+  }
+  if (mt == 2) return tiles <= 512 ? 1280 : tiles <= 1024 ? 768 : 576;
+  if (heads) return tiles >= 384 ? 256 : mt == 3 ? 1280 : 640;
+  if (parts) return mt == 3 ? 576 : 448;
+  if (epi == EPI_SILU_MUL) return tiles <= 512 ? 1280 : 2048;
+  return tiles >= 2048 ? 768 : mt == 4 ? 576 : tiles <= 512 ? 960 : 640;
+}
+inline bool held_pays(int epi, int M, int N, int K, bool parts) {
   const int tiles = held_tiles(epi, N);
   if (epi == EPI_ROPE) {   // a wave prepares one turn at finishing
     const int groups = held_groups(tiles, 1);
     if ((tiles + groups - 1) / groups > HWAVES / (M <= 32 ? 2 : 4)) return false;
   }
-  return tiles >= (K < 768 ? 60 : K >= 2048 ? 128 : epi == EPI_STORE ? 160 : 257);
+  return tiles >= (K < 768 ? 60 : K >= 2048 ? 128 : epi == EPI_STORE ? 160 : 257) && K >= held_from(epi, M, tiles, K, parts);
 }
 template <int EPI, typename CT>
 int launch_held(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice, int slices, float eps,
@@ -2238,7 +2261,7 @@ struct Route {
 inline Route route(int epi, const void* a, int lda, const void* w, int ldw, int M, int N, int K, bool gamma, bool parts, int emits, bool workspace) {
   Route r{kTiled, BlockPlan{}, SplitPlan{}};
   const bool silu = epi == EPI_SILU_MUL;
-  const bool held = !gamma && !emits && epi != EPI_ACCUMULATE && held_pays(epi, M, N, K) && held_takes(a, lda, w, ldw, M, K);
+  const bool held = !gamma && !emits && epi != EPI_ACCUMULATE && held_pays(epi, M, N, K, parts) && held_takes(a, lda, w, ldw, M, K);
   const bool blocks = !held && !gamma && !parts && block_sizes(M, N, K, silu) && block_takes(a, lda, w, ldw, K);
   const bool rings = ring_pays(epi, a, lda, w, ldw, M, N, K);
   if (blocks) r.block = block_plan(M, N, K, silu, 1, 1);
@@ -2310,7 +2333,7 @@ extern "C" int gb_gemm_bf16_partial(const void* a, int lda, const void* w, int l
 // The kernel that gb_gemm_bf16 (epilogues 0 to 2, no gamma, no norm to prepare; with a workspace or without) or gb_gemm_bf16_rope
 // (epilogue 3, no gamma) launches for these sizes: 0 tiled, 1 ring, 2 skinny or folded, 3 held, 4 block, 5 slices of k.
 extern "C" int gb_gemm_bf16_route(int M, int N, int K, int epilogue, int parts, int workspace) {
-  if (epilogue == EPI_ROPE) return held_pays(epilogue, M, N, K) && held_takes(nullptr, K, nullptr, K, M, K) ? kHeld : kFew;
+  if (epilogue == EPI_ROPE) return held_pays(epilogue, M, N, K, parts != 0) && held_takes(nullptr, K, nullptr, K, M, K) ? kHeld : kFew;
   return route(epilogue, nullptr, K, nullptr, K, M, N, K, false, parts != 0, 0, workspace != 0).kernel;
 }
 
@@ -2487,7 +2510,7 @@ extern "C" int gb_gemm_bf16_rope(const void* a, int lda, const void* w, int ldw,
   GB_REQUIRE(!parts || n_parts > 0, "gemm_bf16_rope: partial sums of a norm without a count");
   const NormExtras extra{nullptr, 0, nullptr, 0, nullptr, parts, n_parts};
   const RopeExtras rope{cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, 0};
-  if (!gamma && held_pays(EPI_ROPE, M, N, K) && held_takes(a, lda, w, ldw, M, K))
+  if (!gamma && held_pays(EPI_ROPE, M, N, K, parts != nullptr) && held_takes(a, lda, w, ldw, M, K))
     return launch_held<EPI_ROPE, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream, rope);
   if (gamma)
     return launch_skinny<EPI_ROPE, true, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, gamma, gamma_dtype == kF32,

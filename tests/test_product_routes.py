@@ -1,0 +1,39 @@
+"""Which kernel takes a bfloat16 product (``csrc/hip/gemm_bf16.hip``, ``route``): the built library's own answers on either side of the
+lines that were measured.  Only sizes go in, so no GPU is needed."""
+import ctypes
+import os
+
+import pytest
+
+from glassbox_amd import build
+
+KERNELS = ("tiled", "ring", "few", "held", "block", "slices")
+EPILOGUES = {"store": 0, "add": 1, "unit": 2, "heads": 3}
+
+
+@pytest.fixture(scope="module")
+def route():
+    build.ensure(["gemm_bf16"])
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(build.__file__), "_lib", "libgb_gemm_bf16.so"))
+
+    def ask(epilogue, M, N, K, parts=False, workspace=False):
+        return KERNELS[lib.gb_gemm_bf16_route(M, N, K, EPILOGUES[epilogue], int(parts), int(workspace))]
+    return ask
+
+
+@pytest.mark.parametrize("epilogue,M,N,K,parts,kernel", [
+    # what the held kernel is for: the products of some ten to sixty requests on the shapes of four models
+    ("unit", 53, 5120, 960, True, "held"), ("unit", 24, 28672, 4096, True, "held"), ("unit", 20, 16384, 2048, True, "held"),
+    ("heads", 24, 6144, 4096, True, "held"), ("heads", 64, 6144, 2048, True, "held"), ("heads", 53, 960, 576, True, "held"),
+    ("store", 24, 128256, 4096, False, "held"), ("store", 53, 49152, 960, False, "held"), ("store", 17, 49152, 2048, False, "held"),
+    # a short k, where a tile's fixed costs are more than reading the rows again (k of 128 by 4,112 rows of W, 17 rows: 4.4 us, 2.9)
+    ("store", 17, 4112, 128, False, "few"), ("store", 64, 2048, 256, False, "few"), ("store", 32, 8192, 320, False, "few"),
+    ("heads", 24, 6144, 256, False, "few"), ("unit", 17, 16384, 256, True, "few"),
+    # two tiles a workgroup and two column blocks of rows: from a k of 1,280 on
+    ("unit", 24, 5120, 960, True, "few"), ("unit", 24, 5120, 1280, True, "held"), ("heads", 17, 4608, 960, False, "few"),
+    ("heads", 32, 4608, 1280, False, "held"), ("store", 24, 4112, 1024, False, "few"), ("store", 24, 4112, 1280, False, "held"),
+    # 49 rows and more behind a norm: from a shorter one
+    ("unit", 64, 5120, 384, True, "few"), ("unit", 64, 5120, 448, True, "held"), ("heads", 49, 4608, 576, True, "few"),
+    ("heads", 49, 4608, 640, True, "held")])
+def test_products_of_17_to_64_rows_go_to_the_held_kernel_where_it_is_ahead(route, epilogue, M, N, K, parts, kernel):
+    assert route(epilogue, M, N, K, parts) == kernel
