@@ -994,13 +994,48 @@ inline BlockPlan block_plan(int M, int N, int K, bool silu, int least_slices, in
 inline bool block_takes(const void* a, int lda, const void* w, int ldw, int K) {
   return K % RBK == 0 && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
 }
-// Sizes that are the block kernel's, if the operands allow: short products whose k is not formed into a gated unit stay with the tiled
-// kernel, whose fewer k-steps ahead start sooner (1,600 x 960, 131 rows: 6.3 us, 7.0 here).  Up to 64 rows: what the held kernel cannot hold.
+// Sizes that the block kernel can take, if the operands allow; where it does, see block_pays.  Up to 64 rows: what the held kernel does not
+// take.  A product that is not formed into a gated unit stays with the tiled kernel, whose fewer k-steps ahead start sooner, below a k of
+// 1,024 (3,840 x 960, 65 to 128 rows: 6.3 to 6.6 us; 1,600 x 960, 131 rows 6.3, 7.0 here).
 inline bool block_sizes(int M, int N, int K, bool silu) { return M > 32 && K % RBK == 0 && N % 8 == 0 && (silu ? N % 16 == 0 : K >= 1024); }
 // What the ring kernel takes, alike: a k-step of its 256 x 256 tiles 1.75 us.
 inline float ring_us(int M, int N, int K, int slices) {
   const long long tiles = (long long)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN) * slices;
   return 3.5f + (float)((tiles + 255) / 256) * ((K / slices + RBK - 1) / RBK) * 1.75f + (slices > 1 ? 3.5f + slices * (float)M * N * 8.f / 4.5e6f : 0.f);
+}
+
+// Where the block kernel takes a product whole, with the tile of `p`; else the ring kernel where it can, the tiled one, or (up to 64 rows) the
+// skinny one.  block_plan's estimate says little about those, whose smaller workgroups share a compute unit, so the lines are measured
+// ones (9,000 products of 65 to 1,000 rows, 512 to 16,384 rows of W, k 256 to 8,192, of which 1 % are more than 4 % slower here than the
+// other kernel, 2 % the other way round; us, the other kernel / this one).
+//  * Beside the ring kernel: a storing product whose 256 x 256 tiles are one round stays there (300 x 32,768 x 4,096: 107 / 126), and
+//    so does one for which the plan is tiles of 256 rows (512 x 49,152 x 3,072: 112 / 134); a gated unit goes by the estimates.
+//  * Beside the tiled kernel it is ahead from where that has more than 256 workgroups (400 x 8,192 x 1,792: 24.4 / 20.8).  Below that a
+//    compute unit has one workgroup either way and the tiled one starts sooner: 64-row tiles 256 x 4,096 x 1,280 7.8 / 9.6, ahead
+//    here only with a long k and enough of them (256 x 3,072 x 8,192: 41.9 / 39.4); 128-row tiles 192 x 8,192 x 2,560 25.7 / 30.4, but
+//    not where the plan is narrow tiles and the rows are no whole 128s (added into C, 1,000 x 1,600 x 1,280 17.4 / 13.9, but 640 x 2,560 x
+//    1,280 10.3 / 11.9); up to 128 rows from 128 workgroups on (65 x 6,144 x 1,536 11.4 / 9.9).
+//    Large tiles that leave compute units without one: 512 x 12,288 x 1,280 25.8 / 29.2 (192 tiles of 256 x 128), 640 x 5,120 x 1,024
+//    15.4 / 21.7 (216 of 160 x 96); or that are a second round: 640 x 12,288 x 1,024 24.2 / 28.1.
+//  * A gated unit: ahead of the tiled kernel everywhere but with those, and with tiles as tall as the tiled kernel's and a short k
+//    (512 x 8,192 x 256: 6.9 / 7.5).  Beside the skinny kernel (up to 64 rows) with more than 2,048 gates, or a k of 1,024 and more, or
+//    a very short one (33 x 4,096 x 960: 5.6 / 6.9; 33 x 8,208 x 960: 9.2 / 8.6).
+//  * A vocabulary at up to 64 rows: from 65,536 rows of W on (48 x 49,152 x 4,096: 92 / 97, 128,256: 246 / 234).
+inline bool block_pays(int epi, int M, int N, int K, const BlockPlan& p, bool rings) {
+  const bool silu = epi == EPI_SILU_MUL;
+  const long long tiles = (long long)((M + 32 * p.rm - 1) / (32 * p.rm)) * ((N + 32 * p.cn - 1) / (32 * p.cn));
+  if (rings) {
+    const long long ring = (long long)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN);
+    return p.us < ring_us(M, N, K, 1) && (silu || (ring > 256 && p.rm < 8));
+  }
+  if (M <= 64) return silu ? N > 4096 || K >= 1024 || K < 192 : N < 32768 || N >= 65536;
+  if (tiles > 256 && tiles <= 512 && N < 32768) return false;
+  const TiledGrid g = tiled_grid(epi, M, N);
+  if (M <= 128 && !silu) return g.groups() >= 128;
+  if ((p.rm == 8 && tiles < 224) || (p.cn == 3 && tiles < 240)) return false;
+  if (silu) return !(p.cn == 4 && (p.rm == 4 || p.rm == 8) && K < 640);
+  if (g.bm == 64) return g.groups() > 256 || (g.groups() > 128 && K >= 2560 && N > 2048);
+  return g.groups() > 256 || (p.cn == 2 && M % 128 != 0);
 }
 
 // Slots of a tile: what fits LDS, once (one workgroup a compute unit) or, of the small tiles, twice.
@@ -1319,11 +1354,12 @@ inline int held_from(int epi, int M, int tiles, int K, bool parts) {
     if (epi == EPI_STORE && !parts && tiles == 256) return mt == 2 ? 1536 : 1024;
     return mt == 2 && tiles < 160 ? 3072 : 768;
   }
-  if (mt == 2) return tiles <= 512 ? 1280 : tiles <= 1024 ? 768 : 576;
+  if (mt == 2) return tiles <= 512 ? 1280 : tiles < 768 ? 768 : tiles <= 1024 || tiles > 2048 ? 576 : epi == EPI_SILU_MUL && !parts ? 448 : 640;
   if (heads) return tiles >= 384 ? 256 : mt == 3 ? 1280 : 640;
   if (parts) return mt == 3 ? 576 : 448;
   if (epi == EPI_SILU_MUL) return tiles <= 512 ? 1280 : 2048;
-  return tiles >= 2048 ? 768 : mt == 4 ? 576 : tiles <= 512 ? 960 : 640;
+  if (tiles >= 2048 && tiles < 4096) return 768;
+  return mt == 4 || tiles >= 768 ? 576 : tiles <= 512 ? 960 : 640;
 }
 inline bool held_pays(int epi, int M, int N, int K, bool parts) {
   const int tiles = held_tiles(epi, N);
@@ -1392,6 +1428,8 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
   // the block kernel's tiles, and as many slices as suit them, for a product that is divided; others keep what is in p
   auto in_blocks = [&](const SplitPlan& p) {
     if (!block_sizes(M, N, K, silu)) return p;
+    // (few columns, many rows and a long k: 64-row tiles that are one to a compute unit keep theirs; 512 x 960 x 4,096 15.4 us, 17.4 in blocks)
+    if (M > 64 && N <= 1024 && K >= 4096 && p.bm == 64 && !p.ring && (N + 127) / 128 * ((M + 63) / 64) * p.slices >= 224) return p;
     const BlockPlan b = block_plan(M, N, K, false, 2, 8);
     if (!b.rm || (p.ring && (M >= 1024 || ring_us(M, N, K, p.slices) <= b.us))) return p;
     return SplitPlan{p.bm, b.slices, b.k_slice, (size_t)b.slices * M * N, false, false, b.rm, b.cn, b.us};
@@ -2265,15 +2303,16 @@ inline Route route(int epi, const void* a, int lda, const void* w, int ldw, int 
   const bool blocks = !held && !gamma && !parts && block_sizes(M, N, K, silu) && block_takes(a, lda, w, ldw, K);
   const bool rings = ring_pays(epi, a, lda, w, ldw, M, N, K);
   if (blocks) r.block = block_plan(M, N, K, silu, 1, 1);
+  bool whole = false;
   if (workspace && M > 16 && !gamma && emits != 1 && !parts) {  // more than the skinny kernels' best range
     r.split = split_plan(M, N, K, silu);
     if (r.split.slices <= 1 || (silu && N % 16 != 0)) r.split = SplitPlan{};
     // a product that only stores needs no second pass: not divided where that takes less (QKV, 131 x 6,144 x 2,048: 16 us in slices, 13 whole)
-    const bool whole = blocks && epi != EPI_ACCUMULATE && r.split.rm && r.block.us < r.split.us;
+    whole = blocks && epi != EPI_ACCUMULATE && r.split.rm && r.block.us < r.split.us;
     if (r.split.slices > 1 && !held && !whole) return r.kernel = kSlices, r;
   }
   if (held) return r.kernel = kHeld, r;
-  if (blocks && (M > 64 || epi != EPI_ACCUMULATE) && !emits && (!rings || r.block.us < ring_us(M, N, K, 1))) return r.kernel = kBlock, r;
+  if (blocks && (M > 64 || epi != EPI_ACCUMULATE) && !emits && (whole || block_pays(epi, M, N, K, r.block, rings))) return r.kernel = kBlock, r;
   // 17 to 64 rows by very many rows of W that the held kernel does not take (a long k): measured twice as fast
   // through the tiles as through the skinny kernel with four column blocks (49,152 x 2,048: 102 -> about 50 us),
   // and with two column blocks as fast or faster (49,152 x 960 at 17 to 32 rows: 30 -> 25 us)

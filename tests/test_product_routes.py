@@ -37,3 +37,31 @@ def route():
     ("heads", 49, 4608, 640, True, "held")])
 def test_products_of_17_to_64_rows_go_to_the_held_kernel_where_it_is_ahead(route, epilogue, M, N, K, parts, kernel):
     assert route(epilogue, M, N, K, parts) == kernel
+
+
+@pytest.mark.parametrize("epilogue,M,N,K,kernel", [
+    # short prompts, turns and mixed steps on the shapes of four models
+    ("unit", 131, 16384, 2048, "block"), ("unit", 512, 16384, 2048, "block"), ("unit", 611, 5120, 960, "block"), ("unit", 131, 28672, 4096, "block"),
+    ("store", 131, 6144, 2048, "block"), ("store", 512, 6144, 2048, "block"),
+    # one workgroup a compute unit either way: the tiled kernel starts sooner (256 x 4,096 x 1,280: 7.8 us, 9.6 in blocks)
+    ("store", 256, 4096, 1280, "tiled"), ("add", 512, 512, 2048, "tiled"), ("store", 300, 512, 8192, "tiled"), ("add", 640, 2560, 1280, "tiled"),
+    ("add", 1000, 1600, 1280, "block"), ("store", 400, 8192, 1792, "block"), ("store", 256, 3072, 8192, "block"), ("store", 256, 2048, 8192, "tiled"),
+    ("store", 65, 6144, 1536, "block"), ("store", 65, 2048, 1536, "tiled"),
+    # large tiles that leave units idle or are a second round, or as tall as the tiled kernel's over a short k
+    ("unit", 512, 12288, 1280, "tiled"), ("unit", 640, 12288, 1024, "tiled"), ("add", 640, 5120, 1024, "tiled"), ("unit", 512, 8192, 256, "tiled"),
+    ("unit", 512, 8192, 1024, "block"),
+    # a gated unit of up to 64 rows: few gates and a k below 1,024 stay with the skinny kernel
+    ("unit", 33, 4096, 960, "few"), ("unit", 33, 4096, 1024, "block"), ("unit", 33, 8208, 960, "block"), ("unit", 48, 3072, 128, "block"),
+    # a vocabulary: 256 x 256 tiles in one round, and up to 64 rows the tiles
+    ("store", 300, 32768, 4096, "ring"), ("store", 512, 49152, 3072, "ring"), ("store", 48, 49152, 4096, "tiled"), ("store", 48, 128256, 4096, "block"),
+    # rows of W that 8 does not divide, and a k below 1,024
+    ("store", 128, 3840, 960, "tiled"), ("store", 128, 9001, 2048, "tiled")])
+def test_products_of_some_hundred_rows_go_to_the_block_kernel_where_it_is_ahead(route, epilogue, M, N, K, kernel):
+    assert route(epilogue, M, N, K) == kernel
+
+
+@pytest.mark.parametrize("epilogue,M,N,K,kernel", [
+    ("add", 24, 4096, 14336, "slices"), ("add", 131, 2048, 8192, "slices"), ("add", 611, 960, 2560, "slices"), ("add", 2048, 2048, 8192, "slices"),
+    ("add", 24, 576, 1536, "few"), ("store", 131, 6144, 2048, "block"), ("store", 24, 6144, 4096, "held")])
+def test_products_with_a_workspace_divide_k_where_that_is_ahead(route, epilogue, M, N, K, kernel):
+    assert route(epilogue, M, N, K, workspace=True) == kernel
