@@ -1451,7 +1451,10 @@ inline SplitPlan split_plan(int M, int N, int K, bool silu = false) {
       p.slices = 1, p.k_slice = 0;
     }
   }
-  if (M > 64 && M <= 128 && K % RBK == 0 && N % 8 == 0 && (N + 31) / 32 >= 192) return p;   // narrow tiles fill the chip
+  // 65 to 128 rows by many rows of W: the block kernel's tiles fill the chip by themselves, and what slices save is less than their second
+  // pass costs until k is long (the time whole over the time in slices, 65 to 128 rows by 6,144 to 16,384 added into C, median and ends: k 2,048
+  // 0.83, 0.64 to 1.01; 4,096 0.96, 0.77 to 1.20; 8,192 1.05, 0.87 to 1.40; 14,336 1.32, 1.15 to 1.65: 96 x 8,192 x 14,336 94 and 57 us)
+  if (M > 64 && M <= 128 && K <= 8192 && K % RBK == 0 && N % 8 == 0 && N > 6112) return p;
   const int tiles = ((N + 127) / 128) * ((M + p.bm - 1) / p.bm);
   if (tiles >= 192 || N % 8 != 0) return p;
   // measured on SmolLM2-1.7B shapes: a long k (the down projection) always gains; a short one where the skinny kernel is at its weakest (33

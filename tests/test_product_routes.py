@@ -62,6 +62,8 @@ def test_products_of_some_hundred_rows_go_to_the_block_kernel_where_it_is_ahead(
 
 @pytest.mark.parametrize("epilogue,M,N,K,kernel", [
     ("add", 24, 4096, 14336, "slices"), ("add", 131, 2048, 8192, "slices"), ("add", 611, 960, 2560, "slices"), ("add", 2048, 2048, 8192, "slices"),
+    # 65 to 128 rows by many rows of W: a long k only (96 x 8,192 x 14,336: 94 us whole, 57 in slices)
+    ("add", 96, 8192, 8192, "block"), ("add", 96, 8192, 14336, "slices"), ("store", 100, 6144, 16384, "slices"), ("add", 128, 16384, 28672, "slices"),
     ("add", 24, 576, 1536, "few"), ("store", 131, 6144, 2048, "block"), ("store", 24, 6144, 4096, "held")])
 def test_products_with_a_workspace_divide_k_where_that_is_ahead(route, epilogue, M, N, K, kernel):
     assert route(epilogue, M, N, K, workspace=True) == kernel
