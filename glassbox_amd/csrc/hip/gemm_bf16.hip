@@ -814,7 +814,7 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
 // slices) -> 13.2, 512 rows 23.9 -> 21.6; first passes in slices: 2,048 x 8,192, 131 rows 19.1 -> 13.9, 960 x 2,560, 611 rows 10.7 -> 9.9.
 template <int RM, int CN, int S, int EPI, typename CT>
 __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w, int ldw,
-                                                            CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice, Glu glu) {
+                                                            CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice) {
   constexpr int BM = 32 * RM, BN = 32 * CN, ROWS = BM + BN, L = ROWS / 32;   // L: loads of a wave that bring its share of a slot
   static_assert((S - 1) * L < 64, "a wave counts at most 63 loads on their way");
   if (k_slice > 0) {  // split k: workgroup z of a tile sums its own slice of k into its own copy of C
@@ -935,7 +935,7 @@ __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16* __restri
     for (int j = 0; j < OUT; ++j) {
       if constexpr (EPI == EPI_SILU_MUL) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[j][r] = gated_unit(acc[i][2 * j][r], acc[i][2 * j + 1][r], glu);
+        for (int r = 0; r < 4; ++r) v[j][r] = gated_unit(acc[i][2 * j][r], acc[i][2 * j + 1][r], Glu{});
       } else {
         v[j] = acc[i][j];
       }
@@ -1043,14 +1043,14 @@ constexpr int block_slots(int rm, int cn) { return rm + cn <= 5 ? 80 / (4 * (rm 
 
 template <int EPI, typename CT>
 int launch_block(int rm, int cn, const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice,
-                 int slices, hipStream_t stream, Glu glu = Glu{}) {
+                 int slices, hipStream_t stream) {
   const int cols = EPI == EPI_SILU_MUL ? N / 2 : N, bn = EPI == EPI_SILU_MUL ? 16 * cn : 32 * cn;
   const dim3 grid((cols + bn - 1) / bn, (M + 32 * rm - 1) / (32 * rm), slices), block(256);
   GB_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
 #define GB_B(RM, CN)                                                                                                              \
   if (rm == (RM) && cn == (CN)) {                                                                                                 \
     hipLaunchKernelGGL((gemm_block_kernel<(RM), (CN), block_slots((RM), (CN)), EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, \
-                       ldc, M, N, K, slices > 1 ? k_slice : 0, glu);                                                              \
+                       ldc, M, N, K, slices > 1 ? k_slice : 0);                                                                   \
     return launched("gemm_bf16 (block)");                                                                                         \
   }
   GB_B(2, 2) GB_B(3, 2) GB_B(4, 2) GB_B(5, 2) GB_B(6, 2) GB_B(2, 4) GB_B(3, 4) GB_B(4, 4) GB_B(5, 4) GB_B(6, 4) GB_B(8, 4)

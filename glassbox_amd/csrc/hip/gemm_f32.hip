@@ -667,10 +667,11 @@ extern "C" int gb_gemm_f32_step(const float* a, int lda, const float* w, int ldw
                                        (!slots || (nkv > 0 && k_pages && v_pages && page_size > 0))),
              "gemm_f32_step: N=%d is not (nh + 2 nkv) hd with nh=%d nkv=%d hd=%d, or pages or angles are missing", N, nh, nkv, hd);
   const StepExtras ex{gamma, eps, cosv, sinv, slots, (float*)k_pages, (float*)v_pages, nh, nkv, hd, page_size};
+  if (!gamma && epilogue == EPI_PLAIN) return gb_gemm_f32(a, lda, w, ldw, c, ldc, M, N, K, 0, stream);
 #define GB_STEP(MT, R, EPI)                                                                                                 \
   if (epilogue == EPI && (M <= 1) == (MT == 1) && R == (N > kNarrow ? 16 : N > 4 * kTwoAUnit ? 8 : 4)) {                      \
     if (gamma) launch_skinny<MT, R, EPI, true>(a, lda, w, ldw, c, ldc, M, N, K, 0, stream, ex);                             \
-    else launch_skinny<MT, R, EPI, false>(a, lda, w, ldw, c, ldc, M, N, K, 0, stream, ex);                                  \
+    else if constexpr (EPI != EPI_PLAIN) launch_skinny<MT, R, EPI, false>(a, lda, w, ldw, c, ldc, M, N, K, 0, stream, ex);  \
   }
 #define GB_STEPS(EPI) GB_STEP(1, 4, EPI) GB_STEP(1, 8, EPI) GB_STEP(1, 16, EPI) GB_STEP(2, 4, EPI) GB_STEP(2, 8, EPI) GB_STEP(2, 16, EPI)
   GB_STEPS(EPI_PLAIN) GB_STEPS(EPI_UNIT) GB_STEPS(EPI_HEADS)
