@@ -322,8 +322,8 @@ def test_gemm_bf16_gated_unit_at_the_ends_of_its_range(M):
 @pytest.mark.parametrize("clamped", [False, True])
 def test_gemm_bf16_gated_unit_of_large_gates(M, clamped):
     """Gates up to the largest a bfloat16 holds, beside an up of 0 among others: silu(gate) is the gate itself there, and
-    nothing on the way to it may leave the range (few rows, the stream kernel, tiles, the ring; the clamped unit with a
-    limit that no gate reaches)."""
+    nothing on the way to it may leave the range (few rows, blocks, tiles, the ring; the clamped unit with a limit that no
+    gate reaches)."""
     from glassbox_amd import ops
     I, K = 4096, 128
     gates = torch.tensor([2.0 ** 123, 2.0 ** 124, 2.2e37, 2.0 ** 127, 3e38, -3e38, 1e30]).bfloat16().float()
@@ -342,7 +342,7 @@ def test_gemm_bf16_gated_unit_of_large_gates(M, clamped):
 
 
 def test_gemm_bf16_gated_unit_rounds_alike_by_every_route():
-    """One row of float32 results with SiLU-multiply, alone and among so many rows that the stream kernel, the tiles, the
+    """One row of float32 results with SiLU-multiply, alone and among so many rows that the block kernel, the tiles, the
     ring or slices of k take the product: the sums are exact (one nonzero k), so what the unit makes of them is the same to
     the bit."""
     from glassbox_amd import ops
@@ -489,7 +489,7 @@ def test_gemm_bf16_of_few_rows_that_divides_k_does_the_next_norm(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 96, 4096), (33, 2048, 2048), (64, 2048, 8192), (100, 2048, 4160),
-                                   # 128 narrow tiles are not enough to go without slices (Llama-3-8B's O and down projections)
+                                   # few tiles of a long k (Llama-3-8B's O and down projections)
                                    (96, 4096, 8192), (128, 4096, 4096),
                                    # 65 to 128 rows by many rows of W: from a k above 8,192 on
                                    (96, 6160, 8256), (65, 8192, 9216),
@@ -537,19 +537,18 @@ def test_gemm_bf16_divides_k_over_workgroups(M, N, K, mode):
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 6144, 2048), (128, 16384, 2048), (96, 6144, 8192),
-                                   # one, two, three k-steps: fewer than either ring is deep; and more than both
+                                   # one, two, three k-steps, and seventeen
                                    (100, 4096, 64), (128, 4128, 128), (100, 5000, 192), (70, 6200, 1024), (128, 8200, 1088),
-                                   # so many narrow tiles that a workgroup takes 64 columns
+                                   # very many columns, a short k
                                    (128, 24600, 320), (96, 32760, 512),
-                                   # 17 to 64 rows by very many rows of W: the wide tiles, not the skinny kernel
+                                   # 17 to 64 rows by very many rows of W and a short k: the wide tiles, not the skinny kernel
                                    (64, 49152, 256), (40, 33000, 192), (20, 40000, 192),
-                                   # a narrow model's products: few narrow tiles and a k too short to divide; and up to
-                                   # 256 rows (two row tiles) where the wide tiles would be fewer still
+                                   # a narrow model's products: few tiles and a k too short to divide
                                    (96, 2560, 960), (200, 5120, 960), (256, 2500, 448), (129, 2100, 128)])
 @pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
 def test_gemm_bf16_streams_products_of_some_hundred_rows(M, N, K, mode):
-    """65 to 128 rows (to 256 in a narrow model), a k that is a multiple of 64: tiles of 128 rows by 32 or 64 columns, both operands through
-    rings in LDS, no slices of k where the narrow tiles alone fill the chip (with or without a workspace on offer).
+    """65 to 128 rows (to 256 in a narrow model), a k that is a multiple of 64, or a vocabulary at up to 64 rows: the block and the tiled
+    kernel and, for the last, the held one, without slices of k (with or without a workspace on offer).
     Against float64, the same bits on every run, rows and columns beyond the last tile's edge untouched."""
     from glassbox_amd import ops
     if mode == "silu" and N % 16:
@@ -611,37 +610,73 @@ def test_gemm_bf16_blocks_of_some_hundred_rows(M, N, K, mode):
     assert torch.equal(outs[0], outs[1])
 
 
+# sizes that the held kernel takes in every mode below (a storing product of 160 to 255 tiles of 16 rows of W, or a long k), at the edges of
+# its registers, rings and tiles: column blocks of rows, k-blocks a wave (none for some waves, the most), columns that no tile divides
+HELD = [(17, 2576, 576), (32, 2600, 960), (33, 2564, 320), (48, 4072, 448), (49, 2568, 1088), (64, 2561, 1984), (24, 8240, 4096), (33, 12290, 2048),
+        (17, 6152, 2112), (64, 5130, 1344), (31, 2050, 3136)]
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 2056, 64), (32, 2050, 576), (33, 2048, 960), (48, 8250, 1984), (49, 4112, 2048), (64, 5120, 960),
                                    # a wave's most blocks of k; tiles that do not divide among the workgroups; a short k and few tiles
-                                   (24, 8240, 4096), (31, 33000, 448), (20, 976, 128), (64, 960, 704), (17, 6152, 2112)])
-@pytest.mark.parametrize("mode", ["bf16", "f32", "silu", "parts", "padded"])
+                                   (31, 33000, 448), (20, 976, 128), (64, 960, 704)] + HELD)
+@pytest.mark.parametrize("mode", ["bf16", "f32", "silu", "silu_f32", "parts", "parts_f32", "padded"])
 def test_gemm_bf16_holds_the_rows_and_streams_w(M, N, K, mode):
-    """17 to 64 rows by many rows of W, held in the registers of a workgroup for every compute unit: against the product in
-    float64, alone, with the gated unit, behind the partial sums of a norm, and into rows that are no whole words."""
+    """17 to 64 rows by many rows of W, held in the registers of a workgroup for every compute unit (HELD; the others lie on either side
+    of where that pays): against the product in float64, alone, with the gated unit, behind the partial sums of a norm, and into
+    rows that are no whole words."""
+    from glassbox_amd import ops
+    held = (M, N, K) in HELD
+    if mode[:4] in ("silu", "part"):
+        N -= N % 16
+    parts = 75 if mode.startswith("parts") else 0
+    if held and mode in ("bf16", "f32", "padded"):
+        assert ops.gemm_route(M, N, K) == "held"
+    check_held(M, N, K, silu=mode.startswith("silu") or (parts > 0 and N % 32 == 0), n_parts=parts, f32=mode.endswith("f32") or mode == "padded",
+               padded=mode == "padded")
+
+
+@pytest.mark.parametrize("M,N,K,silu", [(17, 16384, 3072, True), (32, 6160, 3072, False), (64, 5120, 960, True), (49, 960, 64, True), (33, 5120, 576, True),
+                                        (53, 6144, 2048, False)])
+@pytest.mark.parametrize("n", [255, 256, 257, 384, 511])
+def test_gemm_bf16_held_rows_behind_many_partial_sums(M, N, K, silu, n):
+    """Partial sums of a norm up to and beyond the 256 that the held kernel asks for at once (a row of 3,072 leaves 384)."""
+    from glassbox_amd import ops
+    assert ops.gemm_route(M, N, K, silu_mul=silu, parts=True) == "held"
+    check_held(M, N, K, silu=silu, n_parts=n, f32=True, padded=False)
+
+
+def sum_bound(a, w):
+    """What a float32 sum of products of 16-bit numbers may be off by: sqrt(K) roundings' worth of 2^-24 of a partial sum, which is
+    about the product of the rows' lengths at most; eight times that."""
+    K = a.shape[1]
+    return 8 * 2 ** -24 * math.sqrt(K) * a.double().norm(dim=1).max().item() * w.double().norm(dim=1).max().item()
+
+
+def check_held(M, N, K, silu, n_parts, f32, padded):
     from glassbox_amd import ops
     a, w = rnd(M, K, seed=M).bfloat16(), (rnd(N, K, seed=N) / math.sqrt(K)).bfloat16()
-    prod = a.double() @ w.double().T
-    scale, parts = None, None
-    if mode == "parts":
-        n, eps = 75, 1e-5
-        parts = rnd(n, 64, seed=5).abs().float() + 0.1
-        prod = prod / torch.sqrt(parts[:, :M].double().sum(0) / K + eps).unsqueeze(1)
-        parts = (to_dev(parts), n, eps)
-    silu = mode in ("silu", "parts") and N % 16 == 0
-    want = prod if not silu else prod[:, :N // 2] / (1 + torch.exp(-prod[:, :N // 2])) * prod[:, N // 2:]
+    prod, tol, parts, scale = a.double() @ w.double().T, sum_bound(a, w), None, None
+    if n_parts:
+        eps = 1e-5
+        sums = rnd(n_parts, 64, seed=5).abs().float() * (75 / n_parts) + 0.1
+        scale = 1 / torch.sqrt(sums[:, :M].double().sum(0) / K + eps)
+        prod, tol = prod * scale.unsqueeze(1), tol * scale.max().item()
+        parts = (to_dev(sums), n_parts, eps)
+    want = prod
+    bound = torch.full_like(prod, tol) + 2 ** -21 * prod.abs()      # (the scale: a few roundings of 2^-24)
+    if silu:
+        g, u = prod[:, :N // 2], prod[:, N // 2:]
+        want = g / (1 + torch.exp(-g)) * u
+        # |d silu / dg| < 1.1, |silu(g)| <= |g|; the unit's own arithmetic a few roundings
+        bound = bound[:, :N // 2] * 1.1 * u.abs() + bound[:, N // 2:] * g.abs() + tol * tol * 1.1 + 2 ** -20 * want.abs()
     cols = want.shape[1]
-    room = torch.full((M, cols + 3), 7.0, device=DEV, dtype=torch.float32 if mode in ("f32", "padded") else torch.bfloat16)
-    out = room[:, 1:cols + 1] if mode == "padded" else room.view(-1)[:M * cols].view(M, cols)
+    room = torch.full((M, cols + 3), 7.0, device=DEV, dtype=torch.float32 if f32 else torch.bfloat16)
+    out = room[:, 1:cols + 1] if padded else room.view(-1)[:M * cols].view(M, cols)
     ops.gemm(to_dev(a), to_dev(w), out, silu_mul=silu, rms_parts=parts)
-    got = out.cpu().double()
-    # a float32 sum of K products of 16-bit numbers: at most K roundings of 2^-24 of the sum of their magnitudes
-    size = a.double().abs() @ w.double().abs().T
-    tol = 2 ** -24 * K * size.max().item() * 1.5
-    if mode not in ("f32", "padded"):
-        # and of the result to 16 bits (the scale, the unit and its exponential: a few units of 2^-22)
-        tol = 2 ** -8 * want.abs().max().item() + 4 * tol * max(1.0, prod.abs().max().item())
-    assert (got - want).abs().max().item() <= tol
-    if mode == "padded":
+    if not f32:
+        bound = bound * 1.01 + 2 ** -8 * want.abs()
+    assert ((out.cpu().double() - want).abs() <= bound).all()
+    if padded:
         assert (room[:, 0] == 7.0).all() and (room[:, cols + 1:] == 7.0).all()
     again = torch.empty_like(out)
     ops.gemm(to_dev(a), to_dev(w), again, silu_mul=silu, rms_parts=parts)
@@ -649,9 +684,10 @@ def test_gemm_bf16_holds_the_rows_and_streams_w(M, N, K, mode):
     # a row's bits do not depend on the rows beside it
     if M > 33:
         few = torch.empty(M - 1, cols, device=DEV, dtype=out.dtype)
-        ops.gemm(to_dev(a[1:]), to_dev(w), few, silu_mul=silu,
-                 rms_parts=None if parts is None else (to_dev(torch.cat([parts[0].cpu()[:, 1:], parts[0].cpu()[:, :1]], 1)), *parts[1:]))
-        assert torch.equal(few, out[1:])
+        if (M - 1 + 15) // 16 == (M + 15) // 16:   # (as many column blocks: the same kernel)
+            ops.gemm(to_dev(a[1:]), to_dev(w), few, silu_mul=silu,
+                     rms_parts=None if parts is None else (to_dev(torch.cat([parts[0].cpu()[:, 1:], parts[0].cpu()[:, :1]], 1)), *parts[1:]))
+            assert torch.equal(few, out[1:])
 
 
 def test_gemm_bf16_split_k_is_the_same_on_every_run():
@@ -861,10 +897,50 @@ def test_gemm_bf16_rotates_and_writes_the_cache(M, nh, nkv, hd, K, normed):
 
 
 @pytest.mark.parametrize("M,nh,nkv,hd,K", [(17, 32, 32, 64, 2048), (24, 32, 8, 128, 4096), (64, 32, 32, 64, 2048), (33, 9, 3, 64, 576),
-                                           (48, 31, 9, 48, 128), (32, 40, 0, 64, 1024), (19, 129, 1, 16, 64), (64, 60, 2, 64, 1984)])
+                                           (48, 31, 9, 48, 128), (32, 40, 0, 64, 1024), (19, 129, 1, 16, 64), (64, 60, 2, 64, 1984),
+                                           (48, 31, 9, 48, 2048), (32, 40, 0, 64, 2048), (19, 131, 1, 16, 4096), (64, 60, 3, 64, 1984)])
 def test_gemm_bf16_rotates_and_writes_the_cache_with_the_rows_held(M, nh, nkv, hd, K):
-    """The same where a workgroup holds the rows and walks over several tiles of W (a wave then prepares one of them)."""
+    """The same where a workgroup holds the rows and walks over several tiles of W (a wave then prepares one of them), and, of a short k,
+    beside where it does."""
+    from glassbox_amd import ops
+    assert ops.gemm_route(M, (nh + 2 * nkv) * hd, K, heads=True) == ("few" if K in (64, 128, 1024) or nkv == 2 else "held")
     test_gemm_bf16_rotates_and_writes_the_cache(M, nh, nkv, hd, K, False)
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K,n,kernel", [
+    (20, 9, 3, 64, 576, 72, "held"), (49, 9, 3, 64, 576, 72, "held"), (32, 32, 8, 96, 3072, 384, "held"), (24, 32, 8, 128, 4096, 256, "held"),
+    (64, 32, 32, 64, 2048, 257, "held"), (33, 32, 8, 48, 2048, 511, "held"), (17, 24, 8, 64, 512, 64, "few"), (8, 9, 3, 64, 576, 72, "few"),
+    (40, 15, 5, 64, 960, 120, "few")])
+def test_gemm_bf16_rotates_behind_the_partial_sums_of_a_norm(M, nh, nkv, hd, K, n, kernel):
+    """The stacked q/k/v product of rows whose norm comes as partial sums: the scale is in what is rotated, in the rows and in both
+    pages.  Against float64, element by element."""
+    from glassbox_amd import ops
+    N, page, eps = (nh + 2 * nkv) * hd, 16, 1e-5
+    assert ops.gemm_route(M, N, K, heads=True, parts=True) == kernel
+    g = torch.Generator().manual_seed(M + n)
+    a, w = (rnd(M, K, seed=1) * 0.5).bfloat16(), (rnd(N, K, seed=2) / math.sqrt(K)).bfloat16()
+    stride = ops.parts_stride(M)
+    sums = torch.rand(n, stride, generator=g) * 20 + 0.1
+    scale = 1 / torch.sqrt(sums[:, :M].double().sum(0) / K + eps)
+    angles = torch.rand(M, hd // 2, generator=g) * 6
+    cos, sin = angles.cos(), angles.sin()
+    slots = torch.randperm(5 * page, generator=g)[:M].to(torch.int32)
+    prod = ((a.double() @ w.double().T) * scale.unsqueeze(1)).view(M, nh + 2 * nkv, hd)
+    lo, hi = prod[..., :hd // 2], prod[..., hd // 2:]
+    c, s = cos.double().unsqueeze(1), sin.double().unsqueeze(1)
+    want = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    want[:, nh + nkv:] = prod[:, nh + nkv:]
+    size = torch.cat([lo.abs() + hi.abs()] * 2, -1)
+    bound = 2 * sum_bound(a, w) * scale.max().item() + 2 ** -21 * size + 2 ** -8 * want.abs()
+    k_pages = torch.zeros(ops.key_pages_shape(5, nkv, page, hd), device=DEV, dtype=torch.bfloat16)
+    v_pages = torch.zeros(5, nkv, hd, page, device=DEV, dtype=torch.bfloat16)
+    qkv = torch.full((M, N), 9.0, device=DEV, dtype=torch.bfloat16)
+    ops.gemm_rope(to_dev(a), to_dev(w), qkv, nh, nkv, hd, to_dev(cos), to_dev(sin), to_dev(slots), k_pages, v_pages, rms_parts=(to_dev(sums), n, eps))
+    rows = qkv.cpu().double().view(M, nh + 2 * nkv, hd)
+    assert ((rows - want).abs() <= bound).all()
+    keys, idx = ops.unpack_keys(k_pages).cpu().double(), slots.long()
+    assert torch.equal(keys[idx // page, :, idx % page, :], rows[:, nh:nh + nkv])
+    assert torch.equal(v_pages.cpu().double()[idx // page, :, :, idx % page], rows[:, nh + nkv:])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -1001,10 +1077,10 @@ def test_attention_plain_spread_over_workgroups_gives_the_bits_of_one_workgroup(
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nkv,hd", [(2, 64), (8, 32), (4, 16)])
-def test_attention_plain_asks_for_values_ahead_where_workgroups_are_few(dtype, nkv, hd):
-    """32-bit launches of up to 640 workgroups over contexts of 200 keys and more ask for a chunk's values before its scores: chunks
-    that end around a page and around 256 keys, as a launch of few rows, of the last and the first number of rows on either side
-    of the line, with the longest context on either side of where it counts, and spread over workgroups: the same bits, and those of the float64 formula."""
+def test_attention_plain_of_few_workgroups_and_of_more_gives_the_same_bits(dtype, nkv, hd):
+    """32-bit launches of up to 2,048 workgroups over contexts of 64 keys and more (32 up to 256 workgroups), in one chunk or spread over
+    workgroups, ask for a chunk's keys and values at once: chunks that end around a page and around 256 keys, on either side of each
+    of these lines: the same bits, and those of the float64 formula."""
     from glassbox_amd import ops
     nh = 8
     ctx_lens = [1, 17, 191, 192, 193, 239, 240, 241, 255, 256, 257, 447, 448, 700]
@@ -1013,8 +1089,8 @@ def test_attention_plain_asks_for_values_ahead_where_workgroups_are_few(dtype, n
     q, scale = rnd(n, nh * hd, seed=12).to(dtype), 1 / math.sqrt(hd)
     rest = (to_dev(tables), to_dev(ops.pack_keys(k_pages)), to_dev(v_pages), nh, scale, 0)
 
-    def rows(count, spread=False, longest=700):
-        seq = [i % n for i in range(count)]
+    def rows(count, spread=False, longest=700, among=n):
+        seq = [i % among for i in range(count)]
         pos = torch.tensor([ctx_lens[i] - 1 for i in seq], dtype=torch.int32, device=DEV)
         out = torch.full((count, nh * hd), 7.0, device=DEV, dtype=dtype)
         floats = ops.attention_plain_split_floats(count, nh, hd, 16, 700) if spread else 0
@@ -1025,9 +1101,13 @@ def test_attention_plain_asks_for_values_ahead_where_workgroups_are_few(dtype, n
     few = rows(n)
     for count, longest in ((10, 256), (10, 200), (10, 199), (n, 0)):    # (the first ten contexts are of up to 256 keys)
         assert torch.equal(rows(count, longest=longest), few[:count])
+    # 256 and 264 workgroups, 2,048 and 2,056; the longest context on either side of 32 and of 64 keys and of one chunk (one that is
+    # longer than it was said to be is walked all the same)
+    for count, longest in ((32, 31), (32, 32), (33, 32), (33, 63), (33, 64), (33, 257), (256, 63), (256, 64), (256, 256), (257, 256)):
+        assert torch.equal(rows(count, longest=longest, among=10), few[[i % 10 for i in range(count)]])
     want = plain_attention_rows(q, ks, vs, list(range(n)), [c - 1 for c in ctx_lens], nh, scale, 0)
     assert (few.double() - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2 ** -7)
-    for count in (n, 26, 27):               # three chunks each: 336, 624 and 648
+    for count in (n, 26, 27, 85, 86):       # three chunks each: 336, 624 and 648, 2,040 and 2,064
         assert torch.equal(rows(count, spread=True), few[[i % n for i in range(count)]])
 
 
