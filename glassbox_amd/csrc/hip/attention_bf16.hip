@@ -928,11 +928,17 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
   // without spilling: Llama-3-8B shapes at 32 and 64 requests, 1,500 to 4,096 keys, 15 to 25 % faster with four)
   // Eight waves for what is left to four of those, where no unit has a second workgroup whose loads could fill the gaps (us, four / eight
   // waves: 3 x 1 heads of 64, 300 keys 5.35 / 4.87, 8 x 32 of 512 9.8 / 8.7; heads of 128, 20 x 8 of 600 and 1,000 15.0 / 13.0 and 21.5 /
-  // 19.6, of a quarter to all of 1,000 20.2 / 18.2, 24 x 8 of 1,700 34.5 / 32.1, 32 x 8 of 4,000 88.1 / 86.6); up to 256 keys four
-  // waves have a tile each.
+  // 19.6, of a quarter to all of 1,000 20.2 / 18.2, 24 x 8 of 1,700 34.5 / 32.1, 32 x 8 of 4,000 88.1 / 86.6).  Up to 256 keys, in the
+  // context or in the window, four waves have a tile each, and larger workgroups only start later (85 x 3 heads of 64, 30 keys 5.0 / 5.8;
+  // 8 x 32 behind a window of 64 5.7 / 6.6).  A recorded step gives 512 for any contexts up to there (context_bucket): eight waves then
+  // only where the workgroups are so few that the short contexts lose nothing (1 x 3 heads of 64: 30, 250 and 500 keys 4.1 / 4.2, 4.3 /
+  // 4.3, 6.8 / 6.2; but 8 x 3 4.3 / 4.4, 5.3 / 5.9, 7.7 / 7.0; heads of 128, 8 x 8 5.4 / 5.6, 7.4 / 7.4, 10.9 / 9.8, 24 x 8 6.3 / 6.6, 9.1 /
+  // 9.0, 13.9 / 13.0).
   const bool plain = ex.softcap <= 0.f && ex.slopes == nullptr && ex.span == 0, alone = n_decode * nkv <= 256;
   int waves = (splits == 1 && max_context > 512 && hd <= 64 && 16 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) ? 16 : 4;
-  if (waves == 4 && plain && splits == 1 && alone && max_context > 256 && 8 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) waves = 8;
+  const int seen = window > 0 ? min(max_context, window + keep_first) : max_context;   // keys that a row reads at most
+  const bool known = max_context != 512 || n_decode * nkv <= (hd <= 64 ? 16 : 64);
+  if (waves == 4 && plain && splits == 1 && alone && known && seen > 256 && 8 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) waves = 8;
   const size_t lds = (size_t)waves * (32 + (size_t)hd * G) * sizeof(float);
   const dim3 grid(splits, nkv, n_decode), block(waves * 64);
   // capped and sloped scores are kernels of their own (bfloat16 results only), so that the others' score loops are what they were

@@ -1400,7 +1400,10 @@ def test_tuned_decode_gives_a_request_the_same_bits_in_every_row_and_head(nkv, G
 
 
 @pytest.mark.parametrize("nh,nkv,hd,lens,bucket,window", [
-    # eight waves: a tile each or none, more tiles than waves in runs and beyond; the most workgroups, and one more
+    # eight waves: a tile each or none, more tiles than waves in runs and beyond; the most workgroups, and one more; and where a bucket of
+    # 512 or a window of up to 256 keys leaves them to four (the last workgroups that eight take, and more)
+    (32, 32, 64, [500, 449, 64, 65, 510, 320, 17, 257], 510, 0), (15, 5, 16, [511], 511, 300), (15, 5, 16, [400, 511], 511, 256), (15, 5, 16, [400, 511], 511, 257),
+    (12, 4, 64, [512, 30, 250, 320], 512, 0), (12, 4, 64, [512, 30, 250, 320, 1], 512, 0), (8, 4, 128, [300, 512] * 8, 512, 0), (8, 4, 128, [300, 512] * 8 + [9], 512, 0),
     (9, 3, 64, [257, 1, 300], 300, 0), (32, 32, 64, [512, 449, 64, 65, 500, 320, 17, 511], 512, 0), (15, 5, 16, [511], 512, 100),
     (32, 8, 128, [700] * 19 + [1, 129], 768, 0), (16, 8, 96, [2048, 1999] * 12, 2048, 0), (8, 4, 128, [1900] * 64, 2048, 300),
     (8, 4, 128, [300] * 65, 512, 0)])
