@@ -591,15 +591,17 @@ inline int own_pairs(int hd, int page_size) {
   return 0;
 }
 
-// Where the early kernel pays: sixteen pages' words of values are loaded whatever a chunk holds, so where units have several
-// workgroups, contexts of 64 keys and more (us, chunk_alone / early: 15 workgroups of 20 keys 5.6 / 5.8, 240 of 20 and 33 keys
-// 6.3 / 6.1 and 7.3 / 6.3; 600 of 20, 48, 64 and 256 keys 7.6 / 8.6, 8.3 / 8.9, 9.2 / 9.2 and 19.3 / 15.9; 1,200 of 64 and 256
-// 14.8 / 13.8 and 38.5 / 26.3; 1,800, four chunks a request of 1,000 keys, 42.0 / 39.8).  Nor where a workgroup walks several
-// chunks, of which the last may be short.
-constexpr int kEarlyGroups = 2048, kEarlyAlone = 256, kEarlyKeys = 64, kEarlyAloneKeys = 32;
+// Where the early kernel pays: sixteen pages' words of values are loaded whatever a chunk holds, while chunk_alone takes four pages at
+// once.  So from contexts of three pages on where every unit has one workgroup (us, chunk_alone / early, heads of 64: 9 to 120
+// workgroups of 32 keys 5.4 / 5.6, 240 of 33 7.3 / 6.3), from four where it has up to two and a half (360 of 48 and 64 keys 7.6 / 7.6 and
+// 8.3 / 7.6, 600 of 64 and 100 9.0 / 9.1 and 11.5 / 10.5), from seven beyond (960 of 64, 100 and 200 keys 10.0 / 11.8, 13.2 / 13.9 and 20.6 /
+// 19.2; 2,048 19.2 / 21.0, 25.8 / 24.6 and 51.7 / 44.7; 1,800, four chunks a request of 1,000 keys, 42.0 / 39.8).  Nor where a
+// workgroup walks several chunks, of which the last may be short.
+constexpr int kEarlyGroups = 2048;
+inline int early_keys(long long workgroups) { return workgroups <= 256 ? 33 : workgroups <= 640 ? 64 : 112; }
 inline bool early_pays(const Shape& sh, bool spread, long long workgroups, int max_context) {
   return sh.page_size == kEarlyPage && sh.hd % 8 == 0 && sh.hd <= 64 && sh.window == 0 && sh.span == 0 && workgroups <= kEarlyGroups &&
-         max_context >= (workgroups <= kEarlyAlone ? kEarlyAloneKeys : kEarlyKeys) && (spread || max_context <= kChunk);
+         max_context >= early_keys(workgroups) && (spread || max_context <= kChunk);
 }
 
 // The early kernel, if it is for these sizes (false: it is not).

@@ -1078,8 +1078,8 @@ def test_attention_plain_spread_over_workgroups_gives_the_bits_of_one_workgroup(
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nkv,hd", [(2, 64), (8, 32), (4, 16)])
 def test_attention_plain_of_few_workgroups_and_of_more_gives_the_same_bits(dtype, nkv, hd):
-    """32-bit launches of up to 2,048 workgroups over contexts of 64 keys and more (32 up to 256 workgroups), in one chunk or spread over
-    workgroups, ask for a chunk's keys and values at once: chunks that end around a page and around 256 keys, on either side of each
+    """32-bit launches of up to 2,048 workgroups over contexts of 33, 64 or 112 keys and more (up to 256, up to 640 and more workgroups), in
+    one chunk or spread over workgroups, ask for a chunk's keys and values at once: chunks that end around a page and around 256 keys, on either side of each
     of these lines: the same bits, and those of the float64 formula."""
     from glassbox_amd import ops
     nh = 8
@@ -1101,9 +1101,9 @@ def test_attention_plain_of_few_workgroups_and_of_more_gives_the_same_bits(dtype
     few = rows(n)
     for count, longest in ((10, 256), (10, 200), (10, 199), (n, 0)):    # (the first ten contexts are of up to 256 keys)
         assert torch.equal(rows(count, longest=longest), few[:count])
-    # 256 and 264 workgroups, 2,048 and 2,056; the longest context on either side of 32 and of 64 keys and of one chunk (one that is
-    # longer than it was said to be is walked all the same)
-    for count, longest in ((32, 31), (32, 32), (33, 32), (33, 63), (33, 64), (33, 257), (256, 63), (256, 64), (256, 256), (257, 256)):
+    # 256 and 264 workgroups, 640 and 648, 2,048 and 2,056; the longest context on either side of 33, 64 and 112 keys and of one chunk (one
+    # that is longer than it was said to be is walked all the same)
+    for count, longest in ((32, 32), (32, 33), (33, 33), (33, 63), (33, 64), (33, 257), (80, 64), (81, 64), (81, 111), (81, 112), (256, 256), (257, 256)):
         assert torch.equal(rows(count, longest=longest, among=10), few[[i % 10 for i in range(count)]])
     want = plain_attention_rows(q, ks, vs, list(range(n)), [c - 1 for c in ctx_lens], nh, scale, 0)
     assert (few.double() - want).abs().max().item() < (2e-5 if dtype == torch.float32 else 2 ** -7)
