@@ -585,10 +585,12 @@ inline bool skinny_pays(int M, int N, int K) {
 }
 
 // A step's kernels in one: where the skinny kernel runs anyway, up to two rows; with the norm, as long as the rows that a
-// workgroup norms for itself leave LDS for two workgroups a unit (160 KB: 2 x (64 for W, 2 for the sums, 10)).
+// workgroup norms for itself leave LDS for two workgroups a unit (160 KB: 2 x (64 for W, 2 for the sums, 10)), and not before very many
+// rows of W of a short k, whose workgroups each wait for the norm and have little else to do (16,384 rows, us, apart / in one: k 256 with
+// the unit 12.4 / 13.9, k 576 17.2 / 17.4, k 1,024 22.3 / 21.6; 8,192 rows of 256 8.7 / 6.0).
 inline bool step_takes(int M, int N, int K, bool norm) {
   return M >= 1 && M <= kStepMaxRows && K % 4 == 0 && N % 2 == 0 && skinny_pays(M, N, K) &&
-         (!norm || M * ((K + kSlice - 1) / kSlice) * kSlice <= kNormedFloats);
+         (!norm || (M * ((K + kSlice - 1) / kSlice) * kSlice <= kNormedFloats && (K >= 512 || N <= 8192)));
 }
 
 inline bool words_of_16_bytes(const void* p, int ld) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && ld % 4 == 0; }

@@ -188,6 +188,9 @@ def test_gemm_step_f32_gives_the_bits_of_the_kernels_it_replaces(M, K, inter, nh
     assert ran
     # refused where it does not apply
     assert not ops.step_f32_takes(M, 2, 2564 if M == 1 else 1284, True) and not ops.step_f32_takes(3, 64, 64, False)
+    # nor, with the norm, before very many rows of W of a short k
+    assert not ops.step_f32_takes(M, 16384, 508, True) and ops.step_f32_takes(M, 16384, 512, True) and ops.step_f32_takes(M, 16384, 508, False)
+    assert ops.step_f32_takes(M, 8192, 64, True) and not ops.step_f32_takes(M, 8194, 64, True)
     with pytest.raises(ops.KernelError):
         ops.gemm_step_f32(to_dev(rnd(3, 64)), to_dev(rnd(8, 64)), f32(3, 8))
 
