@@ -18,8 +18,8 @@
 //
 // Decoding splits a request's context into chunks of a multiple of 256 keys, one workgroup per
 // (chunk, kv head, request), whose waves (sixteen where one workgroup takes a whole context of more
-// than 512 keys and the head size allows, eight of other whole contexts where workgroups are few, else four) take runs of up to five neighbouring tiles of 64
-// keys, or tiles in turn; partial results are merged in a fixed order (waves in LDS, chunks by a
+// than 512 keys and the head size allows, eight of other whole contexts where workgroups are few and the keys that a row sees known to
+// be more than 256, else four) take runs of up to five neighbouring tiles of 64 keys, or tiles in turn; partial results are merged in a fixed order (waves in LDS, chunks by a
 // second kernel), so the result is the same on every run and in every row of a step.
 // crates/glassbox-core/src/model.rs:285-312 is the formula.
 #include "attention_bf16.h"

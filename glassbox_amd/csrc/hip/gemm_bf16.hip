@@ -812,6 +812,8 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
 // 16,384 x 2,048, 70 / 131 / 300 / 512 rows 22.4 / 28.6 / 39.4 / 46.2 -> 18.2 / 21.8 / 29.4 / 39.4 (744 -> 872 TFLOP/s at the last); 5,120 x 960, 131 /
 // 420 / 1,000 rows 10.5 / 13.4 / 25.5 -> 7.3 / 10.9 / 16.3; 28,672 x 4,096, 131 rows 78 -> 55 (4.2 TB/s of W); QKV 6,144 x 2,048, 131 rows 19.5 (in
 // slices) -> 13.2, 512 rows 23.9 -> 21.6; first passes in slices: 2,048 x 8,192, 131 rows 19.1 -> 13.9, 960 x 2,560, 611 rows 10.7 -> 9.9.
+// In a step of short kernels, whose caches the kernels between have used, the shortest of these gain less or nothing: the 960 x 2,560
+// and 5,120 x 960 products of a prompt of 611 rows take 11.2 to 12.5 and 13.9 to 15.4 there.
 template <int RM, int CN, int S, int EPI, typename CT>
 __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w, int ldw,
                                                             CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice) {
