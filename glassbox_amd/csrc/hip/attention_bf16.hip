@@ -626,25 +626,43 @@ __device__ __forceinline__ void store_part(const f32x16 (&acc)[(HD + 31) / 32], 
   }
 }
 
-// Adds the parts in their order: one workgroup of HD threads per (row, head).
+// Adds the parts in their order, four dimensions a thread; all parts' cells are asked for at once.
+constexpr int kMaxParts = 8;
 template <typename OT>
-__global__ void prefill_parts_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml, OT* __restrict__ out,
-                                     int out_stride, int first_row, int n_rows, int nh, int hd, int parts, float c,
-                                     const float* __restrict__ sinks) {
-  const int row = blockIdx.x / nh, head = blockIdx.x % nh, d = threadIdx.x;
-  if (d >= hd) return;
-  const size_t cell = (size_t)row * nh + head, stride = (size_t)n_rows * nh;
+__global__ __launch_bounds__(256) void prefill_parts_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
+                                                            OT* __restrict__ out, int out_stride, int first_row, int n_rows, int nh,
+                                                            int hd, int parts, float c, const float* __restrict__ sinks) {
+  const int words = hd / 4;
+  const size_t cells = (size_t)n_rows * nh, i = (size_t)blockIdx.x * 256 + threadIdx.x, cell = i / words;
+  if (cell >= cells) return;
+  const int d = (int)(i - cell * words) * 4;
+  float2 ml[kMaxParts];
+  f32x4 acc[kMaxParts];
+#pragma unroll
+  for (int k = 0; k < kMaxParts; ++k)
+    if (k < parts) {
+      ml[k] = *reinterpret_cast<const float2*>(part_ml + (k * cells + cell) * 2);
+      acc[k] = *reinterpret_cast<const f32x4*>(part_acc + (k * cells + cell) * hd + d);
+    }
   float top = -INFINITY;
-  for (int k = 0; k < parts; ++k) top = fmaxf(top, part_ml[(k * stride + cell) * 2]);
-  float val = 0.f, l = 0.f;
-  for (int k = 0; k < parts; ++k) {
-    const float mk = part_ml[(k * stride + cell) * 2];
-    const float f = mk == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mk - top) * c);
-    val += part_acc[(k * stride + cell) * hd + d] * f;
-    l += part_ml[(k * stride + cell) * 2 + 1] * f;
-  }
+#pragma unroll
+  for (int k = 0; k < kMaxParts; ++k)
+    if (k < parts) top = fmaxf(top, ml[k].x);
+  f32x4 val = {0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+#pragma unroll
+  for (int k = 0; k < kMaxParts; ++k)
+    if (k < parts) {
+      const float f = ml[k].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((ml[k].x - top) * c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) val[r] += acc[k][r] * f;
+      l += ml[k].y * f;
+    }
+  const int row = (int)(cell / nh), head = (int)(cell - (size_t)row * nh);
   if (sinks) l += __builtin_amdgcn_exp2f(sinks[head] * 1.4426950408889634f - top * c);
-  store_out(out + (size_t)(first_row + row) * out_stride + (size_t)head * hd + d, val / l);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) val[r] /= l;
+  store_out4(out + (size_t)(first_row + row) * out_stride + (size_t)head * hd + d, val);
 }
 
 // The waves of a group that shared a block's keys add up their maxima, sums and accumulators into wave 0 through LDS,
@@ -893,6 +911,283 @@ __global__ __launch_bounds__(64 * PAIRS * SPLIT, 2) void prefill_kernel(const bf
   }
 }
 
+// ---------------------------------------------------------------------------- prefill, tiles of keys shared through LDS
+// Heads of 64 and 128, bfloat16 results, scores as they are (with windows, kept keys, runs and sinks).  prefill_kernel's
+// arithmetic, a block of 32 tokens of one query head a wave, but the key and value fragments of 64 keys lie in LDS, where
+// R waves of a workgroup read them: with fragments from the caches into each wave's registers, heads of 128 (32 tokens a
+// fragment) were bound by what the caches give, 17 TB/s, and heads of 64 had one wave a SIMD, whose exponentials and MFMAs
+// follow each other.  The blocks of a kv head's query heads are counted through, a token block's heads side by side, so that
+// a workgroup's waves share their keys for grouped heads as for neighbouring tokens.  What bounds it now: the vector
+// arithmetic of the softmax, some 1,100 cycles for 64 keys (half of them exponentials) beside 512 (heads of 64) or 1,024 (of
+// 128) of MFMAs, which other waves of the SIMD overlap.
+// A tile is copied by global_load_lds, a lane's 16 bytes each, from the page to where the fragments are read without bank
+// conflicts; of two places one is filled while the other is read, one barrier a tile.  More places, the values asked for
+// earlier and higher priorities around the MFMAs gave nothing.
+// S waves a block take its tiles in turn (and meet in hand_over) where the blocks alone leave SIMDs without a second wave,
+// and `parts` workgroups where even that leaves compute units idle: shared_plan.
+// Before and after, us: 6,151 tokens, 32 heads over 8 of 128: 512, 313 (990 TFLOP/s); 2,048 tokens, 32 heads of 64: 38.0, 32.0;
+// 8,192: 395, 306; 131 tokens behind 3,900: 35.7, 24.8; 482 behind 512: 19.1, 14.6; five prompts of 77 to 172, 15 heads over 5:
+// 11.4, 8.1; 60 tokens, 32 heads: 11.0, 4.7.
+typedef __attribute__((address_space(3))) void lds_void;
+
+// the larger of a lane's number and that of the lane 32 further on (or back)
+__device__ __forceinline__ float max_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Tile i of a workgroup: the tiles of 64 over the kept first keys, then those from `win0` on.
+struct TileKeys {
+  int kept, win0;
+  __device__ __forceinline__ int of(int i) const { return i < kept ? i * 64 : win0 + (i - kept) * 64; }
+};
+
+// COUNT KB into LDS: lane i's 16 bytes at base + off go to lds + 16 i, and so on every 1,024 bytes on both sides.  (Not the
+// builtin: the compiler would wait for every such copy before it reads any of LDS; who reads waits and meets at a barrier first.)
+template <int COUNT>
+__device__ __forceinline__ void copy_to_lds(uint32_t lds, const void* base, uint32_t off) {
+#define GB_COPY(AT) "\n\tglobal_load_lds_dwordx4 %1, %2 offset:" AT
+#define GB_COPIES(LIST) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" LIST ::"s"(lds), "v"(off), "s"(base) : "memory", "m0")
+  static_assert(COUNT >= 1 && COUNT <= 4, "offsets of 12 bits");
+  if constexpr (COUNT == 1) GB_COPIES(GB_COPY("0"));
+  if constexpr (COUNT == 2) GB_COPIES(GB_COPY("0") GB_COPY("1024"));
+  if constexpr (COUNT == 3) GB_COPIES(GB_COPY("0") GB_COPY("1024") GB_COPY("2048"));
+  if constexpr (COUNT == 4) GB_COPIES(GB_COPY("0") GB_COPY("1024") GB_COPY("2048") GB_COPY("3072"));
+#undef GB_COPIES
+#undef GB_COPY
+}
+
+template <int LEFT>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory");
+}
+
+// One wave's block of 32 tokens over the 64 keys of a tile in LDS.  above: some of its tokens do not see the last of these
+// keys; below: some do not see the first (window, run of positions).
+template <int HD>
+__device__ __forceinline__ void shared_attend(float& m, float& l, f32x16 (&acc)[HD / 32], const bf16x8 (&qf)[HD / 16],
+                                              const char* tile, int kb, int lo, int hi, int keep, bool above, bool below, float c, int lane) {
+  constexpr int KS = HD / 16, DB = HD / 32, kAhead = 2;
+  const int g = lane >> 5, col = lane & 31;
+  const char* k_at = tile + (col >> 4) * (HD * 32) + g * 256 + (col & 15) * 16;
+  const char* v_at = tile + HD * 128 + lane * 16;
+  f32x16 s[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(k_at + t * (HD * 64) + ks * 512), qf[ks], s[t], 0, 0, 0);
+  }
+  bf16x8 vf[kAhead][DB];   // the values of the first groups of keys are asked for before the softmax
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+    for (int b = 0; b < DB; ++b) vf[u][b] = *reinterpret_cast<const bf16x8*>(v_at + (u * DB + b) * 1024);
+  __builtin_amdgcn_sched_barrier(0);
+  if (above) {  // the same for the whole wave
+    const int room = hi - kb - 8 * g;   // the last key that counts, from this lane's first on
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * t + 16 * (r >> 3) + 4 * ((r >> 2) & 1) + (r & 3) > room) s[t][r] = -INFINITY;
+  }
+  if (below) {
+    const int from = lo - kb - 8 * g, kept = keep - kb - 8 * g;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = 32 * t + 16 * (r >> 3) + 4 * ((r >> 2) & 1) + (r & 3);
+        if (key < from && key >= kept) s[t][r] = -INFINITY;
+      }
+  }
+  float mx = s[0][0];
+#pragma unroll
+  for (int r = 1; r < 32; ++r) mx = fmaxf(mx, s[r >> 4][r & 15]);
+  mx = max_halves(mx);
+  if (__any(mx > m)) {
+    const float m_new = fmaxf(m, mx);
+    const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - m_new) * c);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] *= alpha;
+  }
+  const float mc = m == -INFINITY ? 0.f : m * c;  // (-inf: no key yet)
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[t][r] = __builtin_amdgcn_exp2f(fmaf(s[t][r], c, -mc));
+      sum += s[t][r];
+    }
+  l += sum;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    bf16x8 pf;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pf[e] = (bf16)s[u >> 1][8 * (u & 1) + e];
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+      acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u < kAhead ? vf[u < kAhead ? u : 0][b]
+                                                               : *reinterpret_cast<const bf16x8*>(v_at + (u * DB + b) * 1024),
+                                                   pf, acc[b], 0, 0, 0);
+  }
+}
+
+// floor(a / b), the same in all lanes; without the long division of integers below 2^21, where the product's error stays
+// below half of 1 / b
+__device__ __forceinline__ int small_quotient(int a, int b) {
+  if (b == 1) return a;
+  if (a >= 1 << 21) return a / b;
+  return __builtin_amdgcn_readfirstlane((int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b)));
+}
+
+// grid (kv heads, requests from seq_base on, tiles x parts from tiles_from - 1 down), R x S waves a workgroup: R blocks side by side, S waves a
+// block that take the tiles of keys in turn; JOBS = 8 / R, rounded up.
+template <int HD, int JOBS, int S>
+__global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
+    const bf16* __restrict__ q, int q_stride, bf16* __restrict__ out, int out_stride, const int32_t* __restrict__ q_start,
+    const int32_t* __restrict__ q_len, const int32_t* __restrict__ pos0, int seq_base, const int32_t* __restrict__ tables,
+    int table_stride, const bf16* __restrict__ kp, const bf16* __restrict__ vp, int nh, int nkv, int page_shift, float scale,
+    int window, int keep, float* __restrict__ part_acc, float* __restrict__ part_ml, int parts, int tiles_from,
+    int first_row, int n_rows, Extra ex) {
+  constexpr int KS = HD / 16, DB = HD / 32, STAGES = 2, TILE = 256 * HD;   // bytes of 64 keys and values
+  __shared__ __align__(16) char ring[STAGES * S * TILE];
+  const int tid = threadIdx.x, lane = tid & 63, R = blockDim.x / (64 * S);
+  const int wave_of_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = S == 1 ? 0 : small_quotient(wave_of_all, R), wave = wave_of_all - half * R;
+  const int kvh = blockIdx.x, seq = seq_base + blockIdx.y;
+  const int qlen = q_len[seq], p0 = pos0[seq], start = q_start[seq];
+  // everything that the first loads need is asked for at once
+  asm volatile("" ::"s"(qlen), "s"(p0), "s"(start), "s"(q_stride), "s"(table_stride), "s"(nkv), "s"(page_shift), "s"(nh), "s"(parts),
+               "s"(window), "s"(keep), "s"(ex.span), "s"(tiles_from), "s"((int)blockDim.x));
+  const size_t row0 = (size_t)start;
+  // the most work first: the last tokens of all heads, then those before them
+  const int back = tiles_from - 1 - (int)blockIdx.z, tile_no = small_quotient(back, parts), part = back - tile_no * parts;
+  const int G = small_quotient(nh, nkv), blocks = (qlen + 31) / 32, units = blocks * G, unit0 = tile_no * R;
+  if (unit0 >= units) return;  // the whole workgroup
+  const int unit = unit0 + wave;
+  const bool works = unit < units;
+  const int block = works ? small_quotient(unit, G) : 0, head = kvh * G + (works ? unit - block * G : 0);
+  const int col = lane & 31, g = lane >> 5;
+  PageSource src{kp, vp, tables + (size_t)seq * table_stride, nkv, kvh, page_shift, 0, 0, (keep + 15) & ~15};
+  const float c = scale * 1.4426950408889634f;
+  // the keys that any of the workgroup's tokens sees
+  const int b_first = small_quotient(unit0, G), b_last = small_quotient(min(unit0 + R, units) - 1, G);
+  const int first = first_key(p0 + 32 * b_first, window, ex.span), last = p0 + min(32 * b_last + 32, qlen) - 1;
+  src.tlo = first & ~15;
+  src.thi = last & ~15;
+  TileKeys keys;
+  keys.win0 = first & ~63;
+  keys.kept = min((keep + 63) >> 6, keys.win0 >> 6);
+  const int n_tiles = keys.kept + ((last - keys.win0) >> 6) + 1;
+  // this workgroup's tiles, this wave's the (S i + half)-th of them
+  const int i0 = small_quotient(n_tiles * part, parts), i1 = small_quotient(n_tiles * (part + 1), parts);
+
+  const int tok = 32 * block + col;
+  const bool valid = works && tok < qlen;
+  // A tile is eight copies of 16 keys' or values' worth, JOBS a wave (the last ones twice where the waves do not divide them).
+  // This lane's place in a page: of the keys piece lane / 16 (of four), slot by the order of a score tile's rows (load_keys);
+  // of the values dimension lane % 32, keys 8 (lane / 32) on.
+  const int r16 = lane & 15, key16 = ((r16 >> 2) & 1) * 8 + (r16 >> 3) * 4 + (r16 & 3);
+  const uint32_t k_off = (((uint32_t)(lane >> 4) << page_shift) + key16) * 16, v_off = ((uint32_t)col << page_shift) * 2 + 16 * g;
+  const uint32_t ring_at = (uint32_t)(uintptr_t)(lds_void*)ring + half * TILE;
+  auto group_of = [&](int j) {   // the job's group of 16 keys, + 4 for values
+    const int job = wave + j * R;
+    return job < 8 ? job : wave;
+  };
+  const int i_end = max(i0, i1 - 1);
+  // of tile i (the last one in place of those beyond it) and a job's group of 16 keys: the key that says which page it is
+  auto key_at = [&](int i, int j) {
+    const int k = keys.of(min(i, i_end)) + 16 * (group_of(j) & 3);
+    return min(k < src.keep16 ? k : max(k, src.tlo), src.thi);
+  };
+  const uint64_t page_bytes = (uint64_t)(nkv * HD * 2) << page_shift;
+  const char* k_base = (const char*)(kp + (((size_t)kvh * HD) << page_shift));
+  const char* v_base = (const char*)(vp + (((size_t)kvh * HD) << page_shift));
+  uint32_t page[JOBS];
+  auto look_up = [&](int i) {
+#pragma unroll
+    for (int j = 0; j < JOBS; ++j)
+      page[j] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(src.table) + (uint32_t)(key_at(i, j) >> page_shift << 2));
+  };
+  auto copy_tile = [&](int i, int slot) {
+#pragma unroll
+    for (int j = 0; j < JOBS; ++j) {
+      const int job = group_of(j);
+      const char* base = (job >= 4 ? v_base : k_base) + (uint64_t)page[j] * page_bytes;
+      const uint32_t off = job >= 4 ? v_off : k_off, to = ring_at + slot * (S * TILE) + job * (HD * 32);
+      if (page_shift == 4) {   // a page is a group of keys: what lies side by side in the page does in LDS
+        copy_to_lds<DB>(to, base, off);
+      } else {
+        const int in_page = key_at(i, j) & ((1 << page_shift) - 1);
+        base += job >= 4 ? in_page * 2 : in_page * 16;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) copy_to_lds<1>(to + b * 1024, base + ((size_t)(64 * b) << page_shift), off);
+      }
+    }
+  };
+  look_up(i0 + half);
+  bf16x8 qf[KS];
+  const bf16* q_row = q + (row0 + min(tok, qlen - 1)) * q_stride + (size_t)head * HD + 8 * g;   // (a column without a token: any)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = load8(q_row + 16 * ks);
+  copy_tile(i0 + half, 0);
+  look_up(i0 + half + S);
+
+  const int p = p0 + tok;
+  const int lo = valid ? first_key(p, window, ex.span) : 1, hi = valid ? p : 0;
+  const BlockRange range = block_range(32 * block, qlen, p0, window, ex.span);
+  float m = -INFINITY, l = 0.f;
+  f32x16 acc[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));   // waited for here, and not in every step
+  int slot = 0;
+  for (int i = i0; i < i1; i += S) {
+    wait_copies<0>();
+    __builtin_amdgcn_s_barrier();   // these tiles have arrived, and every wave has left the ones before
+    asm volatile("" ::: "memory");
+    if (i + S < i1) {
+      copy_tile(i + half + S, slot ^ 1);
+      look_up(i + half + 2 * S);
+    }
+    const int kb = keys.of(i + half);
+    // (a tile of kept first keys is seen by all; another one by the blocks whose range it meets)
+    if (works && (S == 1 || i + half < i1) && kb <= range.last && (kb + 63 >= range.first || kb < keep))
+      shared_attend<HD>(m, l, acc, qf, ring + (slot * S + half) * TILE, kb, lo, hi, keep, !range.whole || kb + 63 > range.free_hi,
+                        !range.whole || kb < range.free_lo, c, lane);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // what was read of this tile is in registers
+    slot ^= 1;
+  }
+  if constexpr (S > 1) {
+    __syncthreads();
+    float* handed = reinterpret_cast<float*>(ring) + wave * ((S / 2) * DB * 16 * 64);
+    float* handed_ml = reinterpret_cast<float*>(ring) + R * ((S / 2) * DB * 16 * 64) + wave * ((S / 2) * 128);
+    hand_over<DB, S>(m, l, acc, handed, handed_ml, half, lane, c, false);
+    if (half != 0) return;
+  }
+  const float total = l + __shfl_xor(l, 32, kWave);
+  if (!valid) return;
+  if (parts > 1) {
+    const size_t cell = ((size_t)part * n_rows + (row0 + tok - first_row)) * nh + head;
+    store_part<HD>(acc, m, total, part_acc + cell * HD, part_ml + cell * 2, g);
+  } else {
+    const float sink = ex.sinks ? __builtin_amdgcn_exp2f(ex.sinks[head] * 1.4426950408889634f - m * c) : 0.f;
+    store_block<HD, bf16>(acc, total + sink, out + (row0 + tok) * out_stride + (size_t)head * HD, g);
+  }
+}
+
 #define GB_FOR_HEAD_SIZES(X) X(16) X(32) X(48) X(64) X(80) X(96) X(112) X(128)
 
 }  // namespace
@@ -1108,10 +1403,76 @@ inline PrefillPlan prefill_plan(int max_q_len, int max_context, int nh, int n_se
   return p;
 }
 
+// How prefill_shared_kernel spreads a step's portions: R blocks x S waves a block a workgroup, `parts` workgroups a block's
+// keys.  From times of 130 steps (one to eight portions of 17 to 8,192 tokens, behind none to 8,000 keys; 9 to 32 heads) with
+// every shape: the lines below are within 1.03 of the best shape in the geometric mean.  N counts the blocks of all heads, T the
+// longest context's tiles of 64 keys.  us, at the lines' two sides (R x S):
+//   few tiles: a wave a block; more waves only wait for each other at the end (60 tokens of 32 heads: 2 x 1 4.7, 2 x 2 5.8)
+//   many blocks: four of them share what comes into LDS, and there are waves enough (eight prompts of 835 tokens, 32 heads: 4 x 1
+//   33.7, 4 x 2 39.8, 2 x 2 45.2; 7,091 tokens 236, 248, 302; but 5,693 178, 163, 196)
+//   fewer: two waves a block, then two blocks a workgroup (2,048 tokens of 32 heads: 4 x 2 31.9, 2 x 2 34.5; 1,028: 22.7, 20.3)
+//   a few hundred: four waves a block (721 tokens: 2 x 4 14.8, 2 x 2 15.2; 249 behind 1,200 twice: 19.9, 24.9; 3,803 tokens of 9
+//   heads: 43, 56)
+//   fewer still and many tiles: the keys of a block over several workgroups, as long as all are resident (140 tokens behind 4,935:
+//   2 x 2 in five parts 24.9, in six 29.6, 2 x 4 48; 700 tokens of 15 heads behind 3,000, N 330: 34.0 in four parts, 2 x 4 38.4, but 1,139 of 9 heads, N 324: 16.8, 16.2)
+struct SharedPlan {
+  int rows, split, parts;
+};
+inline SharedPlan shared_plan(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
+  const long long blocks = (max_q_len + 31) / 32, heads = (long long)nh * n_seqs, N = blocks * heads;
+  const long long T = (max(max_context, max_q_len) + 63) / 64, pairs = (blocks + 1) / 2 * heads;
+  if (hd <= 64) {
+    if (T == 1) return {2, 1, 1};
+    if (N >= 6500 || N >= 400 * T) return {4, 1, 1};
+    if (N >= 2500) return {4, 2, 1};
+    if (T <= 3 || N >= (T < 32 ? 1000 : 1200)) return {2, 2, 1};
+    if (N > 256 || T < 16) return {2, 4, 1};
+    return {2, 2, (int)max(1ll, min(min(8ll, 512 / pairs), T / 5))};
+  }
+  if (T <= 2) return {2, 1, 1};
+  if (N >= 2500 || N >= 210 * T) return {4, 1, 1};
+  if (N >= 900) return {4, 2, 1};
+  if (N > 256 || T < 16) return {2, 2, 1};
+  return {2, 2, (int)max(1ll, min(min(8ll, 256 / pairs), T / 8))};
+}
+inline bool shared_takes(int hd) { return hd == 64 || hd == 128; }
+
+// rows * 100 + split * 10 + parts of the plan above (0: head sizes it is not for)
+extern "C" int gb_attention_prefill_shape(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
+  if (!shared_takes(hd)) return 0;
+  const SharedPlan p = shared_plan(max_q_len, max_context, nh, n_seqs, hd);
+  return p.rows * 100 + p.split * 10 + p.parts;
+}
+
+template <int HD>
+static void prefill_shared_launch(const bf16* q, int q_stride, bf16* out, int out_stride, const int32_t* q_start, const int32_t* q_len,
+                                  const int32_t* pos0, int seq_base, int n_seqs, int max_q_len, const int32_t* tables,
+                                  int table_stride, const bf16* kp, const bf16* vp, int nh, int nkv, int page_shift, float scale,
+                                  int window, int keep, float* part_acc, float* part_ml, const SharedPlan& plan, int first_row,
+                                  int n_rows, const Extra& ex, hipStream_t stream) {
+  const int units = (max_q_len + 31) / 32 * (nh / nkv), tiles = (units + plan.rows - 1) / plan.rows;
+  // (a grid's third dimension ends at 65,535: longer ones in several launches, the most work first)
+  for (int from = tiles * plan.parts; from > 0; from -= 65535) {
+#define GB_LAUNCH(JOBS, S)                                                                                                      \
+  hipLaunchKernelGGL((prefill_shared_kernel<HD, JOBS, S>), dim3(nkv, n_seqs, min(from, 65535)), dim3(64 * plan.rows * S), 0,    \
+                     stream, q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, tables, table_stride, kp, vp, nh,    \
+                     nkv, page_shift, scale, window, keep, part_acc, part_ml, plan.parts, from, first_row, n_rows, ex)
+    if (plan.rows == 4 && plan.split == 1) GB_LAUNCH(2, 1);
+    if (plan.rows == 4 && plan.split == 2) GB_LAUNCH(2, 2);
+    if (plan.rows == 2 && plan.split == 1) GB_LAUNCH(4, 1);
+    if (plan.rows == 2 && plan.split == 2) GB_LAUNCH(4, 2);
+    if constexpr (HD <= 64) {
+      if (plan.rows == 2 && plan.split == 4) GB_LAUNCH(4, 4);
+    }
+#undef GB_LAUNCH
+  }
+}
+
 // Workgroups that would share a pair's keys with these sizes (1: none do); the caller then provides
 // parts * rows * nh * (hd + 2) floats for their sums, rows being all rows of the portions.
 extern "C" int gb_attention_prefill_parts(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
-  return prefill_plan(max_q_len, max_context, nh, n_seqs, hd).parts;
+  const int parts = prefill_plan(max_q_len, max_context, nh, n_seqs, hd).parts;
+  return shared_takes(hd) ? max(parts, shared_plan(max_q_len, max_context, nh, n_seqs, hd).parts) : parts;
 }
 
 // Requests seq_base .. seq_base+n_seqs-1 of the step (prompt portions); max_q_len is the longest portion and
@@ -1136,9 +1497,11 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
              "attention_prefill: q rows must be 16-byte aligned and out rows 8-byte aligned");
   GB_REQUIRE(n_seqs <= 65535 && nh <= 65535, "attention_prefill: too many requests or heads for one launch");
   if (n_seqs == 0 || max_q_len <= 0) return 0;
+  const bool shared = std::is_same<OT, bf16>::value && shared_takes(hd) && ex.softcap == 0.f && ex.slopes == nullptr;
+  const SharedPlan shared_by = shared_plan(max_q_len, max_context, nh, n_seqs, hd);
   const PrefillPlan plan = prefill_plan(max_q_len, max_context, nh, n_seqs, hd);
   int per_group = plan.per_group, split = plan.split;
-  const int parts = plan.parts;
+  const int parts = shared ? shared_by.parts : plan.parts;
   // over runs of positions the pairs are not equal work: one pair a workgroup and more waves a pair, as long as all are in
   // the chip at once (2,048 tokens, 16 heads, runs of 1,536: 27.6 -> 23.1 us; not for 32 heads, nor for short runs)
   const long long pairs = (long long)((max_q_len + 63) / 64) * nh * n_seqs;
@@ -1171,7 +1534,7 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
     } else if (sloped) {                                           \
       if constexpr (kCanCap) GB_LAUNCH_AS(HD, QB, PAIRS, SPLIT, kSloped); \
     } else {                                                       \
-      GB_LAUNCH_AS(HD, QB, PAIRS, SPLIT, kPlainScores);                  \
+      if constexpr (!(kCanCap && (HD == 64 || HD == 128))) GB_LAUNCH_AS(HD, QB, PAIRS, SPLIT, kPlainScores); \
     }                                                              \
   } while (0)
 #define GB_CASE(HD)                                        \
@@ -1187,13 +1550,22 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
       if (per_group == 1 && split == 8) GB_LAUNCH(HD, 1, 1, 8); \
     }                                                      \
   }
-  GB_FOR_HEAD_SIZES(GB_CASE)
+  if (shared) {
+    if constexpr (kCanCap) {
+      const auto run = hd == 64 ? prefill_shared_launch<64> : prefill_shared_launch<128>;
+      run((const bf16*)q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, n_seqs, max_q_len, tables, table_stride,
+          (const bf16*)k_pages, (const bf16*)v_pages, nh, nkv, page_shift, scale, window, keep_first, part_acc, part_ml, shared_by,
+          first_row, n_rows, ex, stream);
+    }
+  } else {
+    GB_FOR_HEAD_SIZES(GB_CASE)
+  }
 #undef GB_CASE
 #undef GB_LAUNCH
 #undef GB_LAUNCH_AS
   if (int rc = launched("attention_prefill")) return rc;
   if (parts > 1) {
-    hipLaunchKernelGGL(prefill_parts_kernel<OT>, dim3((unsigned)(n_rows * nh)), dim3((hd + 63) / 64 * 64), 0, stream, part_acc,
+    hipLaunchKernelGGL(prefill_parts_kernel<OT>, dim3((unsigned)(((long long)n_rows * nh * (hd / 4) + 255) / 256)), dim3(256), 0, stream, part_acc,
                        part_ml, out, out_stride, first_row, n_rows, nh, hd, parts, scale * 1.4426950408889634f, ex.sinks);
     return launched("attention_prefill (second pass)");
   }

@@ -1534,6 +1534,45 @@ def test_tuned_prefill_behind_histories_that_windows_and_runs_leave_out(nh, nkv,
     assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
 
 
+@pytest.mark.parametrize("shape,nh,nkv,hd,q_lens,history,window,keep,chunk", [
+    # one tile of keys; a request of one block beside one of two; a block whose last token is its first
+    (211, 6, 2, 64, [33, 2, 64], 0, 0, 0, 0), (211, 8, 8, 128, [64, 31], 0, 0, 0, 0),
+    # two waves a block: three tiles (the last one a wave's alone); a window that leaves out tiles of the later blocks, kept keys
+    (221, 15, 5, 64, [65, 190], 0, 0, 0, 0), (221, 32, 32, 64, [1025], 0, 300, 70, 0), (221, 8, 1, 128, [257], 40, 0, 0, 0),
+    # four waves a block: five tiles, and one tile for some tokens; runs of positions; a group of three heads over two blocks
+    (241, 9, 3, 64, [300, 17], 0, 0, 0, 0), (241, 8, 8, 64, [700], 33, 0, 0, 256), (241, 9, 3, 64, [129], 1300, 200, 20, 0),
+    # four blocks a workgroup, of one head and of several; a last workgroup of one block
+    (411, 32, 32, 64, [161] * 8, 0, 0, 0, 0), (411, 32, 4, 128, [300, 295, 225, 33], 0, 0, 0, 0), (411, 64, 16, 64, [545, 3290], 0, 0, 0, 0),
+    (421, 40, 8, 64, [2081], 0, 0, 0, 0), (421, 32, 32, 128, [1000], 0, 150, 64, 0),
+    # several workgroups a block's keys: parts of unequal tiles, all eight, and tokens that see none of a part's
+    (225, 32, 32, 64, [131], 1500, 0, 0, 0), (228, 4, 2, 64, [40, 3], 2700, 0, 0, 0), (224, 8, 2, 128, [100, 37], 2000, 0, 0, 0),
+    (223, 6, 2, 64, [90], 3000, 1000, 30, 0)])
+@pytest.mark.parametrize("page", [16, 32, 128])
+def test_tuned_prefill_of_every_shape(shape, nh, nkv, hd, q_lens, history, window, keep, chunk, page):
+    """The kernel whose waves share tiles of keys, in each of its workgroups' shapes (blocks a workgroup, waves a block,
+    workgroups a block's keys), against the plain kernel; result rows wider than the heads are left alone."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    seen = max(q_lens) + (min(history, window + keep) if window else history)
+    assert ops._lib("attention_bf16").gb_attention_prefill_shape(max(q_lens), seen, nh, len(q_lens), hd) == shape
+    ctx_lens = [history + n for n in q_lens]
+    k_pages, v_pages, tables, _, _ = paged_setup(ctx_lens, nkv, hd, page, seed=hd + nh, dtype=torch.bfloat16)
+    ctx = BareContext(q_lens, ctx_lens, tables)
+    q = to_dev((rnd(sum(q_lens), nh * hd, seed=14) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    wide = torch.full((sum(q_lens), nh * hd + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    sinks = to_dev(rnd(nh, seed=5).float()) if chunk or window else None
+    twin = torch.zeros_like(q)
+    ops.attention_prefill(q, wide[:, :nh * hd], ctx, cache, nh, 1 / math.sqrt(hd), window, keep, chunk, sinks=sinks)
+    ops.attention_plain(q, twin, ctx.positions, torch.tensor(ctx.tok_seq, dtype=torch.int32, device=DEV), ctx.tables[0],
+                        cache.k_pages, cache.v_pages, nh, 1 / math.sqrt(hd), window, keep_first=keep, chunk=chunk, sinks=sinks)
+    # softmax weights in bfloat16 (2^-9 of each value's share) and a bfloat16 result on either side
+    close = (wide[:, :nh * hd].float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())
+    bad = torch.nonzero(~close.all(dim=1)).flatten().tolist()
+    assert not bad, f"rows {bad[:8]} (request, position) {[(ctx.tok_seq[i], ctx.pos_list[i]) for i in bad[:8]]}"
+    assert bool((wide[:, nh * hd:] == 7.0).all())
+
+
 @pytest.mark.parametrize("nh,ctxlen,qlen", [(2, 200, 90), (64, 1200, 1090)])   # 32 and 64 tokens a wave
 def test_tuned_prefill_sees_exactly_the_causal_keys(nh, ctxlen, qlen):
     """A portion in the middle of a request (it starts at position 110): token t must find a marked
