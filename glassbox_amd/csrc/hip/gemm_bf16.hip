@@ -416,8 +416,9 @@ int launch_tiled(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 }
 
 // ------------------------------------------------------------------------- ring
-// Large products (many rows, many 256 x 256 tiles): a workgroup of 2 x 2 waves with a 256 x 256 tile, a wave 8 x 8 tiles of
-// 16 x 16, whose sums fill the accumulation registers (one wave a SIMD).  Operands go from memory straight into LDS
+// Large products (many rows, many tiles): a workgroup of 2 x 2 waves with a tile of 256 x 256, a wave 8 x 8 tiles of
+// 16 x 16, whose sums fill the accumulation registers (one wave a SIMD); or of 256 columns and fewer rows, 32 H, where tiles
+// of 256 would leave many compute units idle in a last round (ring_rows).  Operands go from memory straight into LDS
 // (global_load_lds, 16 bytes a lane: a wave's instruction fills 1 KB of LDS in lane order, so the lane decides which
 // piece of memory lands where), in k-steps of 64, so that an instruction brings eight whole lines of 128 bytes.  LDS, all
 // of it, is a ring of five slots of 256 rows by 64 of k: A and W of the k-step that is multiplied, A and W of the next
@@ -482,11 +483,274 @@ template <> __device__ __forceinline__ void store_c4<bf16>(bf16* c, const f32x4&
   *reinterpret_cast<bf16x4*>(c) = o;
 }
 
+// One tile of 32 H rows by 256 rows of W.  GROUPED: see the kernel.
+template <int EPI, typename CT, bool GROUPED, int H>
+__device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], const bf16* __restrict__ a, int lda, const bf16* __restrict__ w,
+                                          int ldw, CT* __restrict__ c, int ldc, int M, int N, int K, bool head, int bx, int m0,
+                                          int up_off, const Groups& grp, const Glu& glu) {
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / RGN, wn = wave % RGN;
+  const int half = N / 2;  // EPI_SILU_MUL: number of gate rows
+  // row of W behind row r of the workgroup's W tile (r = wn * 128 + j * 16 + column); with EPI_SILU_MUL a wave's
+  // even column tiles hold gate rows and the odd ones the up rows that belong to them
+  auto w_row = [&](int r) -> int {
+    if (EPI == EPI_SILU_MUL) {
+      const int j = r % (RT * 16) / 16;
+      const int n = bx * (RBN / 2) + r / (RT * 16) * (RT / 2 * 16) + j / 2 * 16 + r % 16;
+      return n < half ? (j % 2 ? up_off + n : n) : 0;
+    }
+    return min(bx * RBN + r, N - 1);
+  };
+  // a wave's load instruction moves 8 rows x 8 pieces; rows beyond M or N are read from a row that exists
+  const bf16* asrc[H];
+  const bf16* wsrc[RL];
+#pragma unroll
+  for (int t = 0; t < H; ++t) {
+    const int row = (wave * H + t) * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
+    int arow = min(m0 + row, M - 1);
+    if constexpr (GROUPED) {
+      if (grp.rows) arow = grp.rows[arow];
+    }
+    asrc[t] = a + (size_t)arow * lda + piece * 8;
+  }
+#pragma unroll
+  for (int t = 0; t < RL; ++t) {
+    const int row = (wave * RL + t) * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
+    wsrc[t] = w + (size_t)w_row(row) * ldw + piece * 8;
+  }
+  auto load_a = [&](int t, int slot, int k0) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(asrc[t] + k0), (lds_void*)&ring[slot][(wave * H + t) * 8 * RBK], 16, 0, 0);
+  };
+  auto load_w = [&](int t, int slot, int k0) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[t] + k0), (lds_void*)&ring[slot][(wave * RL + t) * 8 * RBK], 16, 0, 0);
+  };
+  f32x4 acc[H][RT];
+#pragma unroll
+  for (int i = 0; i < H; ++i)
+#pragma unroll
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+
+  // operand of block kh (0, 1): row lane % 16 of a 16-row tile, piece 4 kh + lane / 16
+  uint32_t off[2];
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh) off[kh] = 2 * ((lane % 16) * RBK + (((4 * kh + lane / 16) ^ ((lane >> 1) & 7)) * 8));
+  constexpr uint32_t SLOT = 2 * RBM * RBK, TILE = 2 * 16 * RBK;
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&ring[0][0];
+  const uint32_t abase = base + wm * H * TILE, wbase = base + wn * RT * TILE;
+
+  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end,
+  // in its second half, between whose MFMAs nothing else stands: a branch each eight of them, which their time hides.  (us of
+  // two experts of eight a token, 2,048 tokens, 4,096 units of 2,048, gate/up and down, traced: 159 and 113; a branch before
+  // every MFMA 226 and 152; the kernel with k-steps of 32 175 and 112.)
+  const int live = GROUPED ? __builtin_amdgcn_readfirstlane(min(max((M - m0 - wm * RT * 16 + 15) / 16, 0), RT)) : RT;
+
+  // k-steps; the last may hold a half that counts as zeros
+  const int steps = ring_steps(K), dead = ring_dead_half(K, head);
+  auto k_of = [&](int s) { return ring_step_at(s, K, head); };
+  bf16x8 fa[2][H], fw[2][RT];
+  auto read_a = [&](int set, int t, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
+  };
+  auto read_w = [&](int set, int t, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
+  };
+  constexpr int LIVE_FROM = RT / 2;
+  static_assert(RT == 8 && H >= 4 && H <= 8 && 2 * RT <= RT * LIVE_FROM / 2 && 4 * RL <= RT * LIVE_FROM,
+                "the reads and the loads stand among the first half's MFMAs");
+  // The 8 H MFMAs of operand set `set`; among them the reads of the other set from ra and rw, and (with `more`) a slot's
+  // loads from memory: of A among those of set 0, of W among those of set 1.
+  auto block = [&](auto which, uint32_t ra, uint32_t rw, bool more, int slot, int k0) {
+    constexpr int set = decltype(which)::value;
+#pragma unroll
+    for (int at = 0; at < H * RT; ++at) {
+      const int i = at / RT, j = (i & 1) ? RT - 1 - at % RT : at % RT;
+      if constexpr (GROUPED) {
+        if (i >= LIVE_FROM) {
+          if (at % RT == 0)
+            asm volatile(
+                "s_cmp_le_i32 %17, %18\n\ts_cbranch_scc1 .Lbeyond%=\n\t"
+                "v_mfma_f32_16x16x32_bf16 %0, %8, %16, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %9, %16, %1\n\t"
+                "v_mfma_f32_16x16x32_bf16 %2, %10, %16, %2\n\tv_mfma_f32_16x16x32_bf16 %3, %11, %16, %3\n\t"
+                "v_mfma_f32_16x16x32_bf16 %4, %12, %16, %4\n\tv_mfma_f32_16x16x32_bf16 %5, %13, %16, %5\n\t"
+                "v_mfma_f32_16x16x32_bf16 %6, %14, %16, %6\n\tv_mfma_f32_16x16x32_bf16 %7, %15, %16, %7\n.Lbeyond%=:"
+                : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]),
+                  "+a"(acc[i][6]), "+a"(acc[i][7])
+                : "v"(fw[set][0]), "v"(fw[set][1]), "v"(fw[set][2]), "v"(fw[set][3]), "v"(fw[set][4]), "v"(fw[set][5]),
+                  "v"(fw[set][6]), "v"(fw[set][7]), "v"(fa[set][i]), "s"(live), "n"(i) : "scc");
+          continue;
+        }
+      }
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
+      if (at % 2 == 0 && at / 2 < H) read_a(set ^ 1, at / 2, ra);
+      else if (at % 2 == 0 && at / 2 < H + RT) read_w(set ^ 1, at / 2 - H, rw);
+      else if (at % 4 == 1 && at / 4 < (set == 1 ? RL : H) && more) {
+        if constexpr (set == 1) load_w(at / 4, slot, k0);
+        else load_a(at / 4, slot, k0);
+      }
+    }
+  };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
+#pragma unroll
+  for (int t = 0; t < H; ++t) load_a(t, 0, k_of(0));
+#pragma unroll
+  for (int t = 0; t < RL; ++t) load_w(t, 1, k_of(0));
+  if (steps > 1) {
+#pragma unroll
+    for (int t = 0; t < H; ++t) load_a(t, 2, k_of(1));
+#pragma unroll
+    for (int t = 0; t < RL; ++t) load_w(t, 3, k_of(1));
+    vm_wait<H + RL>();
+  } else {
+    vm_wait<0>();
+  }
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    if (t < H) read_a(0, t, abase + off[0]);
+    read_w(0, t, wbase + SLOT + off[0]);
+  }
+  int sa = 0, sw = 1;   // this k-step's slots
+  auto behind = [](int slot, int by) { return slot + by >= RING_SLOTS ? slot + by - RING_SLOTS : slot + by; };
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    const bool more = s + 2 < steps;
+    const int na = behind(sa, 2), nw = behind(sw, 2), k2 = k_of(s + 2);
+    lds_wait<0>(fa[0], fw[0]);
+    if (dead == 0 && s + 1 == steps) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) fa[0][min(t, H - 1)] = fw[0][t] = zero8();
+    }
+    block(First{}, abase + sa * SLOT + off[1], wbase + sw * SLOT + off[1], more, behind(sa, 4), k2);
+    lds_wait<0>(fa[1], fw[1]);
+    if constexpr (GROUPED) {
+      if (dead == 1) {   // (the only k-step)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) fa[1][min(t, H - 1)] = fw[1][t] = zero8();
+      }
+    }
+    if (more) vm_wait<H>();   // (A of k-step s + 2 may still be on its way)
+    else vm_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    block(Second{}, abase + na * SLOT + off[0], wbase + nw * SLOT + off[0], more, sa, k2);   // (behind the last: read, not used)
+    sa = na, sw = nw;
+  }
+  lds_wait<0>(fa[0], fw[0]);
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results, which the compiler does not know to wait for
+#pragma unroll
+  for (int i = 0; i < H; ++i)
+#pragma unroll
+    for (int j = 0; j < RT; ++j) asm volatile("" : "+a"(acc[i][j]));
+
+  // A lane holds row lane % 16 of a tile and its columns 4 (lane / 16) .. + 3.
+  constexpr int OUT = EPI == EPI_SILU_MUL ? RT / 2 : RT;   // column tiles of the wave's results
+  const int cols = EPI == EPI_SILU_MUL ? half : N;
+  const int gm0 = m0 + wm * H * 16, gn0 = bx * (RGN * OUT * 16) + wn * (OUT * 16);
+  auto result = [&](int i, int j, float factor) -> f32x4 {   // of row tile i, column tile j of the results
+    if constexpr (EPI == EPI_SILU_MUL) {
+      f32x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = gated_unit(acc[i][2 * j][r] * factor, acc[i][2 * j + 1][r] * factor, glu);
+      return v;
+    } else {
+      return acc[i][j];
+    }
+  };
+  const bool scaled = GROUPED && EPI == EPI_SILU_MUL && grp.in_scale;
+  if (gn0 + OUT * 16 <= cols && (size_t)ldc * sizeof(CT) % 16 == 0 && (uintptr_t)c % 16 == 0) {   // the same for the whole wave
+    if constexpr (sizeof(CT) == 2) {
+      // As they lie, a store of the wave would write 32 bytes of 16 rows; so bfloat16 results go through LDS (32 KB of the
+      // wave's own: every wave has read its last operands) and out in runs of 128 or 256 bytes (8,192 x 16,384 x 128, a
+      // product that is mostly epilogue: 109 -> 83 us).
+      constexpr int ROW = OUT * 32, PIECES = ROW / 16;   // bytes and 16-byte pieces of a row
+      static_assert(RT * 16 * ROW * RGM * RGN <= (int)sizeof(ring), "the waves' rows fit the ring");
+      char* own = reinterpret_cast<char*>(&ring[0][0]) + wave * (RT * 16 * ROW);
+#pragma unroll
+      for (int i = 0; i < H; ++i) {
+        const int row = i * 16 + lane % 16;
+        const float factor = scaled ? grp.in_scale[min(gm0 + row, M - 1)] : 1.f;
+#pragma unroll
+        for (int j = 0; j < OUT; ++j)   // half a piece; piece p of a row lies at position p ^ (row % PIECES)
+          store_c4<CT>(reinterpret_cast<CT*>(own + row * ROW + ((2 * j + lane / 32) ^ (row % PIECES)) * 16 + lane / 16 % 2 * 8), result(i, j, factor));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      constexpr int RUN = 64 / PIECES, STORES = H * 16 / RUN;   // rows a store of the wave covers
+      constexpr int AT_ONCE = STORES % 8 == 0 ? 8 : STORES % 7 == 0 ? 7 : STORES % 6 == 0 ? 6 : STORES % 5 == 0 ? 5 : 4;
+      static_assert(STORES % AT_ONCE == 0, "whole turns");
+#pragma unroll
+      for (int it = 0; it < STORES; it += AT_ONCE) {
+        f32x4 v[AT_ONCE];
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+          const int row = (it + u) * RUN + lane / PIECES;
+          v[u] = *reinterpret_cast<const f32x4*>(own + row * ROW + ((lane % PIECES) ^ (row % PIECES)) * 16);
+        }
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+          const int row = (it + u) * RUN + lane / PIECES;
+          if (gm0 + row < M) *reinterpret_cast<f32x4*>(c + (size_t)(gm0 + row) * ldc + gn0 + lane % PIECES * 8) = v[u];
+        }
+      }
+    } else {
+      // 64 bytes of 16 rows a store: through LDS and out in runs of 256 they were no faster.  What is added to: the old values
+      // of two row tiles are on their way while a third's are added to (8,192 x 4,096 x 4,096: 233 -> 228 us).
+      constexpr int DEEP = EPI == EPI_ACCUMULATE ? 3 : 1;
+      f32x4 old[DEEP][OUT];
+      auto to_of = [&](int i) { return c + (size_t)min(gm0 + i * 16 + lane % 16, M - 1) * ldc + gn0 + 4 * (lane / 16); };
+      auto ask = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < OUT; ++j) old[i % DEEP][j] = *reinterpret_cast<const f32x4*>(to_of(i) + j * 16);
+      };
+      if constexpr (EPI == EPI_ACCUMULATE) {
+        ask(0);
+        ask(1);
+      }
+#pragma unroll
+      for (int i = 0; i < H; ++i) {
+        const int gm = gm0 + i * 16 + lane % 16;
+        if constexpr (EPI == EPI_ACCUMULATE) {
+          if (i + 2 < H) ask(i + 2);
+        }
+        if (gm < M) {
+          CT* to = to_of(i);
+          const float factor = scaled ? grp.in_scale[gm] : 1.f;
+#pragma unroll
+          for (int j = 0; j < OUT; ++j) {
+            f32x4 v = result(i, j, factor);
+            if constexpr (EPI == EPI_ACCUMULATE) v = old[i % DEEP][j] + v;
+            store_c4<CT>(to + j * 16, v);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    return;
+  }
+  // the last columns of C, or rows of C that are no 16-byte words
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    const int gm = gm0 + i * 16 + lane % 16;
+    if (gm >= M) continue;
+    const float factor = scaled ? grp.in_scale[gm] : 1.f;
+#pragma unroll
+    for (int j = 0; j < OUT; ++j) {
+      const f32x4 v = result(i, j, factor);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gn = gn0 + j * 16 + 4 * (lane / 16) + r;
+        if (gn < cols) store_c<CT>(c + (size_t)gm * ldc + gn, v[r], EPI == EPI_ACCUMULATE);
+      }
+    }
+  }
+}
+
 // GROUPED: as the tiled kernel's (row tiles of 256 rows); a product that divides k writes grp.slice_rows rows a slice.
-template <int EPI, typename CT, bool GROUPED = false>
+template <int EPI, typename CT, bool GROUPED = false, int H = RT, int SHORT = RT>
 __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w, int ldw,
-                                                           CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice, Groups grp,
-                                                           Glu glu) {
+                                                           CT* __restrict__ c, int ldc, int M, int N, int K, int k_slice, int tall,
+                                                           Groups grp, Glu glu) {
   int bx = blockIdx.x, by = blockIdx.y;
   bool head = false;   // GROUPED: the slice begins the row (other products' slices are of 64 and more: it is all one to them)
   if (k_slice > 0) {  // split k: workgroup z of a tile sums its own slice of k into its own copy of C
@@ -515,260 +779,18 @@ __global__ __launch_bounds__(RGM * RGN * 64, 1) void gemm_ring_kernel(const bf16
     K = min(k_slice, K - z * k_slice);
   }
   __shared__ __attribute__((aligned(16))) bf16 ring[RING_SLOTS][RBM * RBK];
-  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int wm = wave / RGN, wn = wave % RGN;
-  int m0 = by * RBM;
-  const int half = N / 2;  // EPI_SILU_MUL: number of gate rows
-  int up_off = half;       // and how far behind its gate row an up row lies
   if constexpr (GROUPED) {
     const int32_t* tile = grp.map + 3 * by;
     const int group = tile[0];
     if (group < 0) return;   // (the whole workgroup)
-    m0 = tile[1];
-    M = tile[2];
-    w += (size_t)group * grp.w_stride;
-    up_off = grp.up_off;
-  }
-  // row of W behind row r of the workgroup's W tile (r = wn * 128 + j * 16 + column); with EPI_SILU_MUL a wave's
-  // even column tiles hold gate rows and the odd ones the up rows that belong to them
-  auto w_row = [&](int r) -> int {
-    if (EPI == EPI_SILU_MUL) {
-      const int j = r % (RT * 16) / 16;
-      const int n = bx * (RBN / 2) + r / (RT * 16) * (RT / 2 * 16) + j / 2 * 16 + r % 16;
-      return n < half ? (j % 2 ? up_off + n : n) : 0;
-    }
-    return min(bx * RBN + r, N - 1);
-  };
-  // a wave's load instruction moves 8 rows x 8 pieces; rows beyond M or N are read from a row that exists
-  const bf16* asrc[RL];
-  const bf16* wsrc[RL];
-#pragma unroll
-  for (int t = 0; t < RL; ++t) {
-    const int row = (wave * RL + t) * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
-    int arow = min(m0 + row, M - 1);
-    if constexpr (GROUPED) {
-      if (grp.rows) arow = grp.rows[arow];
-    }
-    asrc[t] = a + (size_t)arow * lda + piece * 8;
-    wsrc[t] = w + (size_t)w_row(row) * ldw + piece * 8;
-  }
-  auto load_a = [&](int t, int slot, int k0) {
-    __builtin_amdgcn_global_load_lds((glb_void*)(asrc[t] + k0), (lds_void*)&ring[slot][(wave * RL + t) * 8 * RBK], 16, 0, 0);
-  };
-  auto load_w = [&](int t, int slot, int k0) {
-    __builtin_amdgcn_global_load_lds((glb_void*)(wsrc[t] + k0), (lds_void*)&ring[slot][(wave * RL + t) * 8 * RBK], 16, 0, 0);
-  };
-  f32x4 acc[RT][RT];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < RT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
-
-  // operand of block kh (0, 1): row lane % 16 of a 16-row tile, piece 4 kh + lane / 16
-  uint32_t off[2];
-#pragma unroll
-  for (int kh = 0; kh < 2; ++kh) off[kh] = 2 * ((lane % 16) * RBK + (((4 * kh + lane / 16) ^ ((lane >> 1) & 7)) * 8));
-  constexpr uint32_t SLOT = 2 * RBM * RBK, TILE = 2 * 16 * RBK;
-  const uint32_t base = (uint32_t)(uintptr_t)(lds_void*)&ring[0][0];
-  const uint32_t abase = base + wm * RT * TILE, wbase = base + wn * RT * TILE;
-
-  // GROUPED: a group's last tile may hold few rows: a wave leaves out the MFMAs of rows of 16 that lie beyond the group's end,
-  // in its second half, between whose MFMAs nothing else stands: a branch each eight of them, which their time hides.  (us of
-  // two experts of eight a token, 2,048 tokens, 4,096 units of 2,048, gate/up and down, traced: 159 and 113; a branch before
-  // every MFMA 226 and 152; the kernel with k-steps of 32 175 and 112.)
-  const int live = GROUPED ? __builtin_amdgcn_readfirstlane(min(max((M - m0 - wm * RT * 16 + 15) / 16, 0), RT)) : RT;
-
-  // k-steps; the last may hold a half that counts as zeros
-  const int steps = ring_steps(K), dead = ring_dead_half(K, head);
-  auto k_of = [&](int s) { return ring_step_at(s, K, head); };
-  bf16x8 fa[2][RT], fw[2][RT];
-  auto read_a = [&](int set, int t, uint32_t addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
-  };
-  auto read_w = [&](int set, int t, uint32_t addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][t]) : "v"(addr), "n"(t * TILE) : "memory");
-  };
-  constexpr int LIVE_FROM = RT / 2;
-  static_assert(RT == 8 && 2 * RT <= RT * LIVE_FROM / 2 && 4 * RL <= RT * LIVE_FROM, "the reads and the loads stand among the first half's MFMAs");
-  // The 64 MFMAs of operand set `set`; among them the reads of the other set from ra and rw, and (with `more`) a slot's
-  // loads from memory: of A among those of set 0, of W among those of set 1.
-  auto block = [&](auto which, uint32_t ra, uint32_t rw, bool more, int slot, int k0) {
-    constexpr int set = decltype(which)::value;
-#pragma unroll
-    for (int at = 0; at < RT * RT; ++at) {
-      const int i = at / RT, j = (i & 1) ? RT - 1 - at % RT : at % RT;
-      if constexpr (GROUPED) {
-        if (i >= LIVE_FROM) {
-          if (at % RT == 0)
-            asm volatile(
-                "s_cmp_le_i32 %17, %18\n\ts_cbranch_scc1 .Lbeyond%=\n\t"
-                "v_mfma_f32_16x16x32_bf16 %0, %8, %16, %0\n\tv_mfma_f32_16x16x32_bf16 %1, %9, %16, %1\n\t"
-                "v_mfma_f32_16x16x32_bf16 %2, %10, %16, %2\n\tv_mfma_f32_16x16x32_bf16 %3, %11, %16, %3\n\t"
-                "v_mfma_f32_16x16x32_bf16 %4, %12, %16, %4\n\tv_mfma_f32_16x16x32_bf16 %5, %13, %16, %5\n\t"
-                "v_mfma_f32_16x16x32_bf16 %6, %14, %16, %6\n\tv_mfma_f32_16x16x32_bf16 %7, %15, %16, %7\n.Lbeyond%=:"
-                : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]),
-                  "+a"(acc[i][6]), "+a"(acc[i][7])
-                : "v"(fw[set][0]), "v"(fw[set][1]), "v"(fw[set][2]), "v"(fw[set][3]), "v"(fw[set][4]), "v"(fw[set][5]),
-                  "v"(fw[set][6]), "v"(fw[set][7]), "v"(fa[set][i]), "s"(live), "n"(i) : "scc");
-          continue;
-        }
-      }
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fw[set][j]), "v"(fa[set][i]));
-      if (at % 2 == 0 && at / 2 < RT) read_a(set ^ 1, at / 2, ra);
-      else if (at % 2 == 0 && at / 2 < 2 * RT) read_w(set ^ 1, at / 2 - RT, rw);
-      else if (at % 4 == 1 && at / 4 < RL && more) {
-        if constexpr (set == 1) load_w(at / 4, slot, k0);
-        else load_a(at / 4, slot, k0);
-      }
-    }
-  };
-  using First = std::integral_constant<int, 0>;
-  using Second = std::integral_constant<int, 1>;
-#pragma unroll
-  for (int t = 0; t < RL; ++t) load_a(t, 0, k_of(0));
-#pragma unroll
-  for (int t = 0; t < RL; ++t) load_w(t, 1, k_of(0));
-  if (steps > 1) {
-#pragma unroll
-    for (int t = 0; t < RL; ++t) load_a(t, 2, k_of(1));
-#pragma unroll
-    for (int t = 0; t < RL; ++t) load_w(t, 3, k_of(1));
-    vm_wait<2 * RL>();
+    ring_tile<EPI, CT, true, H>(ring, a, lda, w + (size_t)group * grp.w_stride, ldw, c, ldc, tile[2], N, K, head, bx, tile[1], grp.up_off, grp, glu);
+  } else if (SHORT == H || by < tall) {
+    ring_tile<EPI, CT, false, H>(ring, a, lda, w, ldw, c, ldc, M, N, K, head, bx, by * (32 * H), N / 2, grp, glu);
   } else {
-    vm_wait<0>();
-  }
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    read_a(0, t, abase + off[0]);
-    read_w(0, t, wbase + SLOT + off[0]);
-  }
-  int sa = 0, sw = 1;   // this k-step's slots
-  auto behind = [](int slot, int by) { return slot + by >= RING_SLOTS ? slot + by - RING_SLOTS : slot + by; };
-#pragma unroll 1
-  for (int s = 0; s < steps; ++s) {
-    const bool more = s + 2 < steps;
-    const int na = behind(sa, 2), nw = behind(sw, 2), k2 = k_of(s + 2);
-    lds_wait<0>(fa[0], fw[0]);
-    if (dead == 0 && s + 1 == steps) {
-#pragma unroll
-      for (int t = 0; t < RT; ++t) fa[0][t] = fw[0][t] = zero8();
-    }
-    block(First{}, abase + sa * SLOT + off[1], wbase + sw * SLOT + off[1], more, behind(sa, 4), k2);
-    lds_wait<0>(fa[1], fw[1]);
-    if constexpr (GROUPED) {
-      if (dead == 1) {   // (the only k-step)
-#pragma unroll
-        for (int t = 0; t < RT; ++t) fa[1][t] = fw[1][t] = zero8();
-      }
-    }
-    if (more) vm_wait<RL>();   // (A of k-step s + 2 may still be on its way)
-    else vm_wait<0>();
-    __builtin_amdgcn_s_barrier();
-    block(Second{}, abase + na * SLOT + off[0], wbase + nw * SLOT + off[0], more, sa, k2);   // (behind the last: read, not used)
-    sa = na, sw = nw;
-  }
-  lds_wait<0>(fa[0], fw[0]);
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results, which the compiler does not know to wait for
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < RT; ++j) asm volatile("" : "+a"(acc[i][j]));
-
-  // A lane holds row lane % 16 of a tile and its columns 4 (lane / 16) .. + 3.
-  constexpr int OUT = EPI == EPI_SILU_MUL ? RT / 2 : RT;   // column tiles of the wave's results
-  const int cols = EPI == EPI_SILU_MUL ? half : N;
-  const int gm0 = m0 + wm * RT * 16, gn0 = bx * (RGN * OUT * 16) + wn * (OUT * 16);
-  auto result = [&](int i, int j, float factor) -> f32x4 {   // of row tile i, column tile j of the results
-    if constexpr (EPI == EPI_SILU_MUL) {
-      f32x4 v;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = gated_unit(acc[i][2 * j][r] * factor, acc[i][2 * j + 1][r] * factor, glu);
-      return v;
-    } else {
-      return acc[i][j];
-    }
-  };
-  const bool scaled = GROUPED && EPI == EPI_SILU_MUL && grp.in_scale;
-  if (gn0 + OUT * 16 <= cols && (size_t)ldc * sizeof(CT) % 16 == 0 && (uintptr_t)c % 16 == 0) {   // the same for the whole wave
-    if constexpr (sizeof(CT) == 2) {
-      // As they lie, a store of the wave would write 32 bytes of 16 rows; so bfloat16 results go through LDS (32 KB of the
-      // wave's own: every wave has read its last operands) and out in runs of 128 or 256 bytes (8,192 x 16,384 x 128, a
-      // product that is mostly epilogue: 109 -> 83 us).
-      constexpr int ROW = OUT * 32, PIECES = ROW / 16;   // bytes and 16-byte pieces of a row
-      static_assert(RT * 16 * ROW * RGM * RGN <= (int)sizeof(ring), "the waves' rows fit the ring");
-      char* own = reinterpret_cast<char*>(&ring[0][0]) + wave * (RT * 16 * ROW);
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        const int row = i * 16 + lane % 16;
-        const float factor = scaled ? grp.in_scale[min(gm0 + row, M - 1)] : 1.f;
-#pragma unroll
-        for (int j = 0; j < OUT; ++j)   // half a piece; piece p of a row lies at position p ^ (row % PIECES)
-          store_c4<CT>(reinterpret_cast<CT*>(own + row * ROW + ((2 * j + lane / 32) ^ (row % PIECES)) * 16 + lane / 16 % 2 * 8), result(i, j, factor));
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      constexpr int AT_ONCE = 8, RUN = 64 / PIECES;   // rows a store of the wave covers
-#pragma unroll
-      for (int it = 0; it < RT * 16 / RUN; it += AT_ONCE) {
-        f32x4 v[AT_ONCE];
-#pragma unroll
-        for (int u = 0; u < AT_ONCE; ++u) {
-          const int row = (it + u) * RUN + lane / PIECES;
-          v[u] = *reinterpret_cast<const f32x4*>(own + row * ROW + ((lane % PIECES) ^ (row % PIECES)) * 16);
-        }
-#pragma unroll
-        for (int u = 0; u < AT_ONCE; ++u) {
-          const int row = (it + u) * RUN + lane / PIECES;
-          if (gm0 + row < M) *reinterpret_cast<f32x4*>(c + (size_t)(gm0 + row) * ldc + gn0 + lane % PIECES * 8) = v[u];
-        }
-      }
-    } else {
-      // 64 bytes of 16 rows a store: through LDS and out in runs of 256 they were no faster
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        const int gm = gm0 + i * 16 + lane % 16;
-        if (gm < M) {
-          CT* to = c + (size_t)gm * ldc + gn0 + 4 * (lane / 16);
-          const float factor = scaled ? grp.in_scale[gm] : 1.f;
-          f32x4 old[OUT];   // a row's old values are all asked for before any is added to
-          if constexpr (EPI == EPI_ACCUMULATE)
-#pragma unroll
-            for (int j = 0; j < OUT; ++j) old[j] = *reinterpret_cast<const f32x4*>(to + j * 16);
-#pragma unroll
-          for (int j = 0; j < OUT; ++j) {
-            f32x4 v = result(i, j, factor);
-            if constexpr (EPI == EPI_ACCUMULATE) v = old[j] + v;
-            store_c4<CT>(to + j * 16, v);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    return;
-  }
-  // the last columns of C, or rows of C that are no 16-byte words
-#pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int gm = gm0 + i * 16 + lane % 16;
-    if (gm >= M) continue;
-    const float factor = scaled ? grp.in_scale[gm] : 1.f;
-#pragma unroll
-    for (int j = 0; j < OUT; ++j) {
-      const f32x4 v = result(i, j, factor);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gn = gn0 + j * 16 + 4 * (lane / 16) + r;
-        if (gn < cols) store_c<CT>(c + (size_t)gm * ldc + gn, v[r], EPI == EPI_ACCUMULATE);
-      }
-    }
+    ring_tile<EPI, CT, false, SHORT>(ring, a, lda, w, ldw, c, ldc, M, N, K, head, bx, tall * (32 * (H - SHORT)) + by * (32 * SHORT), N / 2, grp, glu);
   }
 }
 
-// The ring kernel pays where its tiles occupy at least three quarters of the compute units, from two row tiles on, and the
-// loads are whole 16-byte pieces.  (us, gate/up with SiLU-multiply, before / with it: 320 x 28,672 x 4,096 139 / 104,
-// 512 rows 156 / 106, 1,000 rows 283 / 203; 611 x 16,384 x 2,048 58 / 53, 1,000 rows 79 / 57.)
 constexpr int RING_MIN_ROWS = 257;
 // With slices of k: a thousand rows, or enough rows times k that a slice's sums, which go through memory, are the smaller
 // part (611 x 2,048 x 8,192 47.5 / 44.9, but 512 rows 34.8 / 43.2; 320 x 4,096 x 14,336 78 / 69, 1,000 rows 177 / 118; 611 x
@@ -778,20 +800,21 @@ inline bool ring_takes(const void* a, int lda, const void* w, int ldw, int K) {
   return K % RING_K == 0 && K >= RING_MIN_K && lda % 8 == 0 && ldw % 8 == 0 && (uintptr_t)a % 16 == 0 &&
          (uintptr_t)w % 16 == 0;
 }
-inline bool ring_pays(int epi, const void* a, int lda, const void* w, int ldw, int M, int N, int K) {
-  if (!ring_takes(a, lda, w, ldw, K)) return false;
-  const int cols = epi == EPI_SILU_MUL ? N / 2 : N, bn = epi == EPI_SILU_MUL ? RBN / 2 : RBN;
-  const long long tiles = (long long)((M + RBM - 1) / RBM) * ((cols + bn - 1) / bn);
-  return M >= RING_MIN_ROWS && tiles >= 192;
-}
+inline int ring_columns(int epi, int N) { return epi == EPI_SILU_MUL ? (N / 2 + RBN / 2 - 1) / (RBN / 2) : (N + RBN - 1) / RBN; }
 
 template <int EPI, typename CT>
-int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, hipStream_t stream,
-                Glu glu = Glu{}) {
-  const int cols = EPI == EPI_SILU_MUL ? N / 2 : N, bn = EPI == EPI_SILU_MUL ? RBN / 2 : RBN;
-  const dim3 grid((cols + bn - 1) / bn, (M + RBM - 1) / RBM), block(RGM * RGN * 64);
+int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, int k_slice, int slices,
+                hipStream_t stream, Glu glu = Glu{}) {
+  const int columns = ring_columns(EPI, N);
+  const RingRows rows = ring_rows(M, columns * slices, k_slice ? k_slice : K);
+  const dim3 grid(columns, rows.tiles, slices), block(RGM * RGN * 64);
   GB_REQUIRE(grid.y <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
-  hipLaunchKernelGGL((gemm_ring_kernel<EPI, CT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, N, K, 0, Groups{}, glu);
+#define GB_H(H, SHORT)                                                                                                 \
+  if (rows.height == H && (SHORT == H) == (H == 8 && rows.tall == rows.tiles))                                         \
+    hipLaunchKernelGGL((gemm_ring_kernel<EPI, CT, false, H, SHORT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, \
+                       N, K, k_slice, rows.tall, Groups{}, glu);
+  GB_H(8, 8) GB_H(8, 7) GB_H(7, 6) GB_H(6, 5) GB_H(5, 4)
+#undef GB_H
   return launched("gemm_bf16 (ring)");
 }
 
@@ -1023,8 +1046,31 @@ inline float ring_us(int M, int N, int K, int slices) {
 //    (512 x 8,192 x 256: 6.9 / 7.5).  Beside the skinny kernel (up to 64 rows) with more than 2,048 gates, or a k of 1,024 and more, or
 //    a very short one (33 x 4,096 x 960: 5.6 / 6.9; 33 x 8,208 x 960: 9.2 / 8.6).
 //  * A vocabulary at up to 64 rows: from 65,536 rows of W on (48 x 49,152 x 4,096: 92 / 97, 128,256: 246 / 234).
+// The ring kernel pays where its tiles of 256 occupy at least three quarters of the compute units, from two row tiles on, and the
+// loads are whole 16-byte pieces; and wherever its estimate with the heights of ring_rows is below the block kernel's, which is
+// also a bound below the tiled kernel's time.  (That estimate is some 10 % low for several rounds of tiles, and this one by what a
+// tile's old values take.)  Not for one round of them where the tiled kernel's workgroups are resident at once (640 x 12,288 x 1,024
+// 23.0 / 22.4; 930 x 8,192 x 3,072 53 / 58; 420 x 12,288 x 1,280 25.5 / 28.7).  Of 260 products of 200 to 8,192 rows, random sizes among them, one is more than 3 % slower than with
+// the first line alone (3,931 x 14,672 x 576: 146 / 156); us, the block or tiled kernel / this one: 1,350 x 6,144 x 4,096 104 / 69,
+// 2,200 x 4,096 x 14,336 372 / 237, 4,500 x 2,048 x 8,192 207 / 146, 700 x 16,384 x 2,048 with SiLU-multiply 60 / 48, 350 x 28,672 x
+// 4,096 115 / 87, 4,096 x 5,120 x 960 58 / 47, 2,900 x 3,072 x 576 23.0 / 18.3.
+inline bool ring_fills(int epi, int M, int N) { return M >= RING_MIN_ROWS && (long long)((M + RBM - 1) / RBM) * ring_columns(epi, N) >= 192; }
+inline bool ring_ahead(int epi, int M, int N, int K) {
+  const bool silu = epi == EPI_SILU_MUL;
+  if (M < RING_MIN_ROWS || K % RBK != 0 || N % (silu ? 16 : 8) != 0) return false;
+  const int columns = ring_columns(epi, N);
+  const RingRows r = ring_rows(M, columns, K);
+  const bool one_round = (long long)r.tiles * columns <= 256;
+  if (one_round && tiled_grid(epi, M, N).groups() <= 512) return false;
+  const float added = epi == EPI_ACCUMULATE ? 1.25f * (float)r.height : 0.f;
+  return r.us + added <= (one_round ? 1.f : 1.1f) * block_plan(M, N, K, silu, 1, 1).us;
+}
+inline bool ring_pays(int epi, const void* a, int lda, const void* w, int ldw, int M, int N, int K) {
+  return ring_takes(a, lda, w, ldw, K) && (ring_fills(epi, M, N) || ring_ahead(epi, M, N, K));
+}
 inline bool block_pays(int epi, int M, int N, int K, const BlockPlan& p, bool rings) {
   const bool silu = epi == EPI_SILU_MUL;
+  if (rings && ring_ahead(epi, M, N, K)) return false;
   const long long tiles = (long long)((M + 32 * p.rm - 1) / (32 * p.rm)) * ((N + 32 * p.cn - 1) / (32 * p.cn));
   if (rings) {
     const long long ring = (long long)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN);
@@ -1660,9 +1706,9 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
   if (held) {
     if (int rc = launch_held<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, 0.f, nullptr, 0, stream)) return rc;
   }
-  if (ring)
-    hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, float>), dim3((N + RBN - 1) / RBN, (M + RBM - 1) / RBM, plan.slices), dim3(RGM * RGN * 64),
-                       0, stream, a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, Groups{}, Glu{});
+  if (ring) {
+    if (int rc = launch_ring<EPI_STORE, float>(a, lda, w, ldw, ws, N, M, N, K, plan.k_slice, plan.slices, stream)) return rc;
+  }
 #define GB_S(WM, FULL)                                                                                                   \
   if (!ring && !blocks && !held && (plan.bm == 64 * WM) && kfull == FULL)                                                                   \
     hipLaunchKernelGGL((gemm_tiled_kernel<WM, 2, 1, EPI_STORE, FULL, float>), grid, block, 0, stream, a, lda, w, ldw, ws, \
@@ -2422,7 +2468,7 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
 #define GB_SP(EPI, CT) launch_split<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, split_ws, r.split, stream, &extra, eps)
 #define GB_HD(EPI, CT) launch_held<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream)
 #define GB_BK(EPI, CT) launch_block<EPI, CT>(r.block.rm, r.block.cn, A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
-#define GB_RG(EPI, CT) launch_ring<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
+#define GB_RG(EPI, CT) launch_ring<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, 0, 1, stream)
 #define GB_TL(EPI, CT) launch_tiled<EPI, CT>(A, lda, W, ldw, (CT*)c, ldc, M, N, K, stream)
   switch (r.kernel) {
     case kSlices: GB_EACH(GB_SP)
@@ -2475,7 +2521,7 @@ extern "C" int gb_gemm_bf16_glu(const void* a, int lda, const void* w, int ldw, 
     return launch_skinny<EPI_SILU_MUL, false, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
   }
   if (ring_pays(EPI_SILU_MUL, a, lda, w, ldw, M, N, K))
-    return launch_ring<EPI_SILU_MUL, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, stream, glu);
+    return launch_ring<EPI_SILU_MUL, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, 0, 1, stream, glu);
   return launch_tiled<EPI_SILU_MUL, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, stream, glu);
 }
 
@@ -2515,11 +2561,11 @@ extern "C" int gb_gemm_bf16_grouped(const void* a, int lda, const int32_t* rows,
     const int rbn = epilogue == EPI_SILU_MUL ? RBN / 2 : RBN;
     const dim3 rgrid((cols + rbn - 1) / rbn, tiles, slices), rblock(RGM * RGN * 64);
     if (epilogue == EPI_SILU_MUL)
-      hipLaunchKernelGGL((gemm_ring_kernel<EPI_SILU_MUL, bf16, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (bf16*)c, ldc, 0, N, K, 0, grp, Glu{limit, alpha, plus});
+      hipLaunchKernelGGL((gemm_ring_kernel<EPI_SILU_MUL, bf16, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (bf16*)c, ldc, 0, N, K, 0, 0, grp, Glu{limit, alpha, plus});
     else if (c_dtype == kF32)
-      hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, float, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (float*)c, ldc, 0, N, K, k_slice, grp, Glu{});
+      hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, float, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (float*)c, ldc, 0, N, K, k_slice, 0, grp, Glu{});
     else
-      hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, bf16, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (bf16*)c, ldc, 0, N, K, 0, grp, Glu{});
+      hipLaunchKernelGGL((gemm_ring_kernel<EPI_STORE, bf16, true>), rgrid, rblock, 0, stream, A, lda, W, ldw, (bf16*)c, ldc, 0, N, K, 0, 0, grp, Glu{});
     return launched("gemm_bf16 (grouped ring)");
   }
   const dim3 grid((cols + bn - 1) / bn, tiles), block(256);

@@ -280,6 +280,35 @@ def test_gemm_bf16_large_products_through_the_lds_ring(M, N, K, mode):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("M,N,K", [
+    # tiles of 256 and 224 rows, 224 and 192, 192 and 160, 160 and 128; one row in the last 32; a last column tile partly outside
+    (1185, 11200, 640), (1601, 8112, 160), (641, 28672, 160), (705, 16320, 640), (1185, 16320, 160), (1313, 11200, 640)])
+@pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
+def test_gemm_bf16_ring_with_tiles_of_two_heights(M, N, K, mode):
+    """Rows dealt to tiles of fewer than 256 rows, every epilogue: the last row of each tile and the first of the next among
+    those compared, and rows of C beyond the product left alone."""
+    from glassbox_amd import ops
+    lib = ops._lib("gemm_bf16")
+    epi = {"bf16": 0, "f32": 0, "f32+": 1, "silu": 2}[mode]
+    assert lib.gb_gemm_bf16_route(M, N, K, epi, 0, 0) == 1
+    a, w = rnd(M, K, seed=11).bfloat16() * 0.25, rnd(N, K, seed=12).bfloat16() * 0.25
+    full = a.float() @ w.float().T
+    c0 = rnd(M, N, seed=13)
+    cols = N // 2 if mode == "silu" else N
+    want = full + c0 if mode == "f32+" else full
+    if mode == "silu":
+        g, u = full[:, :cols], full[:, cols:]
+        want = g / (1 + torch.exp(-g)) * u
+    room = torch.full((M + 40, cols), 7.0, device=DEV, dtype=torch.bfloat16 if mode in ("bf16", "silu") else torch.float32)
+    if mode == "f32+":
+        room[:M] = to_dev(c0)
+    ops.gemm(to_dev(a), to_dev(w), room[:M], accumulate=(mode == "f32+"), silu_mul=(mode == "silu"))
+    # sums of K products in 32-bit on either side, and the result's rounding
+    tol = 1e-5 * math.sqrt(K) + (2 ** -8) * want.abs().max().item() * (mode in ("bf16", "silu"))
+    assert (room[:M].cpu().float() - want).abs().max().item() <= tol
+    assert bool((room[M:] == 7.0).all())
+
+
 @pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
 @pytest.mark.parametrize("pad,shift", [(8, 0), (2, 0), (6, 2), (0, 4)])
 def test_gemm_bf16_ring_writes_rows_that_are_no_whole_words(mode, pad, shift):

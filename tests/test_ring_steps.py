@@ -15,6 +15,10 @@ extern "C" int numbers(int i) { return i == 0 ? gb::RBK : i == 1 ? gb::RING_K : 
 extern "C" int steps(int K) { return gb::ring_steps(K); }
 extern "C" int step_at(int s, int K, int head) { return gb::ring_step_at(s, K, head != 0); }
 extern "C" int dead_half(int K, int head) { return gb::ring_dead_half(K, head != 0); }
+extern "C" int rows(int M, int columns, int K, int i) {
+  const gb::RingRows r = gb::ring_rows(M, columns, K);
+  return i == 0 ? r.height : i == 1 ? r.tall : r.tiles;
+}
 """
 
 
@@ -49,3 +53,24 @@ def test_every_slice_reads_inside_its_row_and_counts_each_k_once(ring):
                     dead = ring.dead_half(size, int(z == 0)) if s + 1 == ring.steps(size) else -1
                     seen += [begin + i for i in range(step) if i // unit != dead]
                 assert seen == list(range(at, at + size)), (K, slices, z)
+
+
+@pytest.mark.parametrize("columns", [1, 7, 16, 24, 64, 112, 255, 256, 1000])
+def test_tiles_hold_every_row_once(ring, columns):
+    """The dealing of rows to tiles of two heights: as many rows of 32 as there are, none of them in two tiles, heights that the
+    kernel is built for, and 256 wherever the compute units are filled by that."""
+    for M in list(range(257, 2100)) + list(range(2100, 9000, 37)) + [30000, 65536, 131072 + 5, 1 << 20]:
+        for K in (128, 2048, 14336):
+            height, tall, tiles = (ring.rows(M, columns, K, i) for i in range(3))
+            assert 5 <= height <= 8 and 1 <= tall <= tiles, (M, K)
+            assert tall * height + (tiles - tall) * (height - 1) == -(-M // 32), (M, K)
+    for M in (512, 2048, 8192):
+        if M // 256 * columns % 256 == 0:
+            assert ring.rows(M, columns, 4096, 0) == 8 and ring.rows(M, columns, 4096, 2) == M // 256
+
+
+@pytest.mark.parametrize("M,columns,K,heights", [
+    (6151, 16, 14336, (7, 13, 30)), (6151, 24, 4096, (7, 7, 31)), (2048, 24, 2048, (7, 4, 10)), (5487, 16, 4096, (6, 12, 32)), (2048, 64, 2048, (8, 8, 8))])
+def test_tiles_where_256_rows_leave_units_idle(ring, M, columns, K, heights):
+    """The numbers of tiles that were the fastest of those measured."""
+    assert tuple(ring.rows(M, columns, K, i) for i in range(3)) == heights
