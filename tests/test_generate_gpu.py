@@ -162,6 +162,30 @@ def test_sampling_kernel_on_rows_of_ties_and_edge_settings():
     assert checked == 192
 
 
+@pytest.mark.parametrize("vocab", [1023, 1024, 1027, 4099, 49152])
+@pytest.mark.parametrize("ties", [False, True])
+def test_sampling_kernel_where_few_candidates_are_sorted(vocab, ties):
+    """Top-k on either side of where the candidates are found first and sorted (512), with more of one value than the kernel
+    sorts (1,024), and of rows with few more tokens than it has threads; the other filters behind it."""
+    from glassbox_amd.sampling import SamplerConfig, sample_rows
+    rng = random.Random(vocab)
+    g = torch.Generator().manual_seed(vocab)
+    ks = [1, 2, 50, 63, 64, 500, 511, 512, 513, 1000, 1022]
+    logits = torch.randn(len(ks) + 3, vocab, generator=g)
+    if ties:
+        logits = (logits * 8).round() / 8
+    logits[-1, 1000:] -= 20.0                                  # a thousand before all others
+    logits[-2, :] = 1.0                                        # all equal: more of one value than are sorted, or just as many
+    logits[-3] = logits[-3] * 6
+    cfgs = [SamplerConfig(temperature=0.9, top_k=k, top_p=rng.choice([1.0, 0.97, 0.5]), min_p=rng.choice([0.0, 0.0, 0.05])) for k in ks]
+    cfgs += [SamplerConfig(temperature=1.0, top_k=20, top_p=0.9, min_p=0.2), SamplerConfig(temperature=1.0, top_k=9, top_p=0.5),
+             SamplerConfig(temperature=1.0, top_k=40, top_p=0.7)]
+    us = [rng.random() for _ in cfgs]
+    toks, cands = sample_rows(logits.clone().to(DEV), cfgs, us, [[]] * len(cfgs))
+    for r, c in enumerate(cfgs):
+        check_sampled(logits[r].tolist(), [], c, us[r], toks[r], cands[r])
+
+
 def test_temperature_draws_follow_the_softmax():
     from glassbox_amd.sampling import Rng, SamplerConfig, sample_rows
     logits = torch.tensor([[0.0, math.log(2.0), math.log(5.0), -30.0]], device=DEV).repeat(64, 1)
