@@ -187,6 +187,34 @@ def test_streams_kernels():
         assert (h2.cpu().to(F64) - ps.rms(u2, 1e-5, f(gamma))).abs().max() < 2e-5
 
 
+@pytest.mark.parametrize("S", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n, d", [(2, 2048), (3, 4), (1, 4096), (5, 252), (2, 4100)])
+@pytest.mark.parametrize("gamma_dtype, out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32),
+                                                   (torch.bfloat16, torch.float32)])
+def test_streams_norm_with_a_word_a_thread(S, n, d, gamma_dtype, out_dtype):
+    """Rows of up to 4,096 columns and up to four streams take the kernel that holds a row in registers, others the general one:
+    the update, the weighted sum and the norm against 64 bits, with rows picked and with the sums asked for."""
+    from glassbox_amd import ops
+    torch.manual_seed(S * d)
+    f = lambda t: t.float().to(F64)
+    X, y = torch.randn(S, n, d), torch.randn(n, d)
+    w_in, w_out, mix = torch.randn(S), torch.randn(S), torch.randn(S, S)
+    gamma = (torch.rand(d) + 0.5).to(gamma_dtype)
+    new = torch.stack([sum(f(mix)[s, t] * f(X)[s] for s in range(S)) + f(w_out)[t] * f(y) for t in range(S)])
+    tol = (2 ** -8 if out_dtype == torch.bfloat16 else 2e-5)
+    Xd, h, total = _dev(X), torch.empty(n, d, device=DEV, dtype=out_dtype), torch.empty(n, d, device=DEV)
+    ops.streams_norm(Xd, _dev(w_in), gamma.to(DEV), 1e-5, h, total=total, update=(_dev(mix), _dev(w_out), _dev(y)))
+    u = sum(f(w_in)[s] * new[s] for s in range(S))
+    want = ps.rms(u, 1e-5, f(gamma))
+    assert (Xd.cpu().to(F64) - new).abs().max() < 2e-5 and (total.cpu().to(F64) - u).abs().max() < 1e-4
+    assert ((h.cpu().to(F64) - want).abs() <= tol * (1 + want.abs())).all()
+    rows = _i32([n - 1, 0])
+    picked = torch.empty(2, d, device=DEV, dtype=out_dtype)
+    ops.streams_norm(Xd, None, gamma.to(DEV), 1e-5, picked, rows=rows)
+    want = ps.rms(new.sum(0)[[n - 1, 0]], 1e-5, f(gamma))
+    assert ((picked.cpu().to(F64) - want).abs() <= tol * (1 + want.abs())).all()
+
+
 # ------------------------------------------------------------------------------------------ attention
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("window, keep", [(24, 5), (16, 16), (300, 2), (7, 40), (33, 0)])
