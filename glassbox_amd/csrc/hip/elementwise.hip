@@ -317,10 +317,10 @@ __device__ __forceinline__ void rope_store_pieces(int t, int idx, bf16* __restri
                                                   const float* __restrict__ cosv, const float* __restrict__ sinv,
                                                   const int32_t* __restrict__ slots, bf16* __restrict__ k_pages,
                                                   bf16* __restrict__ v_pages, int nh, int nkv, int hd, int page_size,
-                                                  int rotate, int v_rows) {
+                                                  int rotate) {
   const int half = hd / 2, lanes = half / 8;  // lanes a head
   const int unit = idx / lanes, j = (idx % lanes) * 8;
-  const int units = nh + nkv + ((slots && t < v_rows) ? nkv : 0);  // rows from v_rows on: values are stored by tiles
+  const int units = nh + nkv + (slots ? nkv : 0);
   if (unit >= units) return;
   bf16* head = qkv + (size_t)t * row_stride + (size_t)unit * hd;
   const bool is_v = unit >= nh + nkv, is_k = unit >= nh && !is_v;
@@ -361,14 +361,14 @@ __device__ __forceinline__ void rope_store_pieces(int t, int idx, bf16* __restri
 __global__ void rope_store_pieces_kernel(bf16* __restrict__ qkv, int row_stride, const float* __restrict__ cosv,
                                          const float* __restrict__ sinv, const int32_t* __restrict__ slots,
                                          bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int nh, int nkv, int hd,
-                                         int page_size, int rotate, int v_rows) {
+                                         int page_size, int rotate) {
   // The chip deals workgroups round its 8 dies by their number, and each die has a second-level cache of its own: a
   // die takes a run of neighbouring tokens, whose 16-byte pieces lie side by side in a key page, so that the cache
   // writes back whole lines
   int t = blockIdx.x;
   if (gridDim.x % 8 == 0) t = (t % 8) * (gridDim.x / 8) + t / 8;
   rope_store_pieces(t, blockIdx.y * blockDim.x + threadIdx.x, qkv, row_stride, cosv, sinv, slots, k_pages, v_pages, nh,
-                    nkv, hd, page_size, rotate, v_rows);
+                    nkv, hd, page_size, rotate);
 }
 
 // Values of prompt portions, sixteen positions at a time: the transposed page holds the sixteen slots
@@ -376,10 +376,11 @@ __global__ void rope_store_pieces_kernel(bf16* __restrict__ qkv, int row_stride,
 // 16-byte words instead of two bytes at a time.  grid (groups of 16 positions, kv heads, requests
 // from seq_base on); request s has q_len[s] rows from row q_start[s] on, the first at position pos0[s].
 template <typename T>
-__device__ __forceinline__ void store_values_tile(int group, int kvh, int seq, T* tile, const T* __restrict__ qkv,
-                                                  int row_stride, const int32_t* __restrict__ slots, T* __restrict__ v_pages,
-                                                  const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
-                                                  const int32_t* __restrict__ pos0, int nh, int nkv, int hd, int page_size) {
+__device__ __forceinline__ void store_values_tile(int tid, int threads, int group, int kvh, int seq, T* tile,
+                                                  const T* __restrict__ qkv, int row_stride, const int32_t* __restrict__ slots,
+                                                  T* __restrict__ v_pages, const int32_t* __restrict__ q_start,
+                                                  const int32_t* __restrict__ q_len, const int32_t* __restrict__ pos0, int nh,
+                                                  int nkv, int hd, int page_size) {
   const int ld = hd + 2;  // tile: [16][hd + 2]
   const int first = pos0[seq], n = q_len[seq];
   const int p_lo = (first / 16 + group) * 16;  // the group's first position
@@ -387,7 +388,8 @@ __device__ __forceinline__ void store_values_tile(int group, int kvh, int seq, T
   if (j_lo >= n) return;
   const int row0 = q_start[seq];
   const int chunks = hd / 8;
-  for (int idx = threadIdx.x; idx < 16 * chunks; idx += blockDim.x) {
+  // (a part of the workgroup without a head only goes to the barrier)
+  for (int idx = kvh < nkv ? tid : 16 * chunks; idx < 16 * chunks; idx += threads) {
     const int i = idx / chunks, ch = idx % chunks, j = j_lo + i;
     if (j < 0 || j >= n) continue;
     const T* src = qkv + (size_t)(row0 + j) * row_stride + (size_t)(nh + nkv + kvh) * hd + ch * 8;
@@ -398,12 +400,13 @@ __device__ __forceinline__ void store_values_tile(int group, int kvh, int seq, T
     for (int e = 0; e < 8; ++e) tile[i * ld + ch * 8 + e] = got[e];
   }
   __syncthreads();
+  if (kvh >= nkv) return;
   // the page and the first slot of the group, from any token of it that exists
   const int j_any = max(j_lo, 0);
   const int slot_any = slots[row0 + j_any];
   const int page = slot_any / page_size, off0 = slot_any % page_size - (j_any - j_lo);
   T* dst_page = v_pages + ((size_t)page * nkv + kvh) * hd * page_size + off0;
-  for (int idx = threadIdx.x; idx < 2 * hd; idx += blockDim.x) {
+  for (int idx = tid; idx < 2 * hd; idx += threads) {
     const int d = idx / 2, h8 = idx % 2;
     T* dst = dst_page + (size_t)d * page_size + 8 * h8;
     const int i0 = 8 * h8;
@@ -433,31 +436,96 @@ __global__ void store_values_kernel(const T* __restrict__ qkv, int row_stride, c
                                     const int32_t* __restrict__ q_len, const int32_t* __restrict__ pos0, int seq_base,
                                     int nh, int nkv, int hd, int page_size) {
   extern __shared__ unsigned char tile_bytes[];
-  store_values_tile<T>(blockIdx.x, blockIdx.y, seq_base + blockIdx.z, reinterpret_cast<T*>(tile_bytes), qkv, row_stride, slots,
-                       v_pages, q_start, q_len, pos0, nh, nkv, hd, page_size);
+  store_values_tile<T>(threadIdx.x, blockDim.x, blockIdx.x, blockIdx.y, seq_base + blockIdx.z, reinterpret_cast<T*>(tile_bytes), qkv,
+                       row_stride, slots, v_pages, q_start, q_len, pos0, nh, nkv, hd, page_size);
 }
 
-// Both at once for bfloat16 steps with prompt portions: the first `rope_blocks` workgroups rotate and write keys
-// (and the values of single-token rows), the rest turn the portions' values tile by tile.  The two have nothing to
-// wait for in each other, and one launch costs a step of some hundred rows less than two.
-__global__ void rope_and_values_kernel(bf16* __restrict__ qkv, int row_stride, const float* __restrict__ cosv,
+// The queries and keys of one token in rope_store_pieces' way, the same piece of U heads `step` apart: what turns them is read once.
+template <int U>
+__device__ __forceinline__ void rope_heads(int t, int unit, int step, int j, bf16* __restrict__ qkv, int row_stride,
+                                           const float* __restrict__ cosv, const float* __restrict__ sinv,
+                                           const int32_t* __restrict__ slots, bf16* __restrict__ k_pages, int nh, int nkv, int hd,
+                                           int page_size, int rotate) {
+  const int half = hd / 2, units = nh + nkv;
+  bf16* row = qkv + (size_t)t * row_stride + j;
+  bf16x8 x0[U], x1[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const bf16* head = row + (size_t)min(unit + u * step, units - 1) * hd;
+    x0[u] = *reinterpret_cast<const bf16x8*>(head);
+    x1[u] = *reinterpret_cast<const bf16x8*>(head + half);
+  }
+  const int slot = slots && unit + (U - 1) * step >= nh ? slots[t] : -1;
+  const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
+  if (rotate) {
+    const float* cr = cosv + (size_t)t * half + j;
+    const float* sr = sinv + (size_t)t * half + j;
+    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cr), c1 = *reinterpret_cast<const f32x4*>(cr + 4);
+    const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr), s1 = *reinterpret_cast<const f32x4*>(sr + 4);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float c = e < 4 ? c0[e] : c1[e - 4], sn = e < 4 ? s0[e] : s1[e - 4];
+        const float a = (float)x0[u][e], b = (float)x1[u][e];
+        x0[u][e] = (bf16)(a * c - b * sn);
+        x1[u][e] = (bf16)(b * c + a * sn);
+      }
+      if (unit + u * step < units) {   // rotated keys stay in the row too: parts may read them back
+        bf16* head = row + (size_t)(unit + u * step) * hd;
+        *reinterpret_cast<bf16x8*>(head) = x0[u];
+        *reinterpret_cast<bf16x8*>(head + half) = x1[u];
+      }
+    }
+  }
+  if (slot < 0) return;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int at = unit + u * step;
+    if (at < nh || at >= units) continue;
+    bf16* dst = k_pages + ((size_t)page * nkv + (at - nh)) * page_size * hd;
+    *reinterpret_cast<bf16x8*>(dst + key_offset(off, j, page_size, 8)) = x0[u];
+    *reinterpret_cast<bf16x8*>(dst + key_offset(off, half + j, page_size, 8)) = x1[u];
+  }
+}
+
+// All of a bfloat16 step with prompt portions in one launch: the first `rope_blocks` workgroups rotate and write keys, the next
+// `row_blocks` write the values of the single-token rows, a dimension a lane, and the rest turn the portions' values tile by tile,
+// `heads` (a power of two) of a tile a workgroup.
+// What bounds a rotation is the lines that its lanes write: a lane's 16 bytes of a key page lie 256 from its neighbour's where the
+// lanes of a wave take the pieces of one token.  So they take a piece of sixteen tokens, whose places in the page are
+// neighbours, and of U heads where there are tokens enough.  A value row's lanes write two bytes every 32, whatever the split; a
+// lane with 16 of them, one after the other, took twice as long as all else in a step of 30 rows and a portion.
+// us, a token a workgroup (and the values apart from 1,025 rows on) / so, 32 heads of 64: 2,048 tokens 16.8 / 14.4; 482 and 30
+// rows 9.6 / 7.0; 131 5.0 / 4.8; 1,555 of two prompts 16.6 / 12.1; 6,151 tokens, 32 heads over 8 of 128, 48.0 / 41.3.
+template <int U>
+__global__ __launch_bounds__(256) void rope_and_values_kernel(bf16* __restrict__ qkv, int row_stride, const float* __restrict__ cosv,
                                        const float* __restrict__ sinv, const int32_t* __restrict__ slots,
-                                       bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int nh, int nkv, int hd,
-                                       int page_size, int rotate, int v_rows, int rope_blocks, int rope_y,
+                                       bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int rows, int nh, int nkv, int hd,
+                                       int page_size, int rotate, int rope_blocks, int rope_y, int row_blocks, int row_y,
                                        const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
-                                       const int32_t* __restrict__ pos0, int seq_base, int groups) {
+                                       const int32_t* __restrict__ pos0, int seq_base, int groups, int heads) {
   extern __shared__ unsigned char tile_bytes[];
-  const int b = blockIdx.x;
+  const int tid = threadIdx.x;
+  int b = blockIdx.x;
   if (b < rope_blocks) {
-    // a die (workgroups b, b + 8, ...) takes a run of neighbouring tokens, as in the kernel above
-    const int r = rope_blocks % 8 == 0 ? (b % 8) * (rope_blocks / 8) + b / 8 : b;
-    rope_store_pieces(r / rope_y, (r % rope_y) * blockDim.x + threadIdx.x, qkv, row_stride, cosv, sinv, slots, k_pages, v_pages,
-                      nh, nkv, hd, page_size, rotate, v_rows);
+    const int t = b / rope_y * 16 + tid % 16, idx = b % rope_y * (16 * U) + tid / 16, lanes = hd / 16;
+    if (t < rows && idx / lanes < nh + nkv)
+      rope_heads<U>(t, idx / lanes, 16 / lanes, idx % lanes * 8, qkv, row_stride, cosv, sinv, slots, k_pages, nh, nkv, hd, page_size, rotate);
     return;
   }
-  const int v = b - rope_blocks;
-  store_values_tile<bf16>(v % groups, v / groups % nkv, seq_base + v / (groups * nkv), reinterpret_cast<bf16*>(tile_bytes), qkv,
-                          row_stride, slots, v_pages, q_start, q_len, pos0, nh, nkv, hd, page_size);
+  b -= rope_blocks;
+  if (b < row_blocks) {
+    const int t = b / row_y, i = b % row_y * 256 + tid, slot = slots[t];
+    if (i < nkv * hd && slot >= 0)
+      v_pages[((size_t)(slot / page_size) * nkv * hd + i) * page_size + slot % page_size] = qkv[(size_t)t * row_stride + (size_t)(nh + nkv) * hd + i];
+    return;
+  }
+  b -= row_blocks;
+  const int blocks = (nkv + heads - 1) / heads, threads = 256 / heads, part = tid / threads;
+  store_values_tile<bf16>(tid % threads, threads, b % groups, b / groups % blocks * heads + part, seq_base + b / (groups * blocks),
+                          reinterpret_cast<bf16*>(tile_bytes) + part * (16 * (hd + 2)), qkv, row_stride, slots, v_pages, q_start, q_len,
+                          pos0, nh, nkv, hd, page_size);
 }
 
 // Rows v_rows .. n-1 are prompt portions described by q_start, q_len and pos0 of requests seq_base ..
@@ -481,17 +549,22 @@ extern "C" int gb_rope_store(void* qkv, int dtype, int row_stride, const float* 
                             (!rotate || ((uintptr_t)cosv % 8 == 0 && (uintptr_t)sinv % 8 == 0));
   const bool pieces = dtype == kBF16 && hd % 16 == 0 && row_stride % 8 == 0 && (uintptr_t)qkv % 16 == 0 &&
                       (uintptr_t)k_pages % 16 == 0 && (!rotate || ((uintptr_t)cosv % 16 == 0 && (uintptr_t)sinv % 16 == 0));
-  // one launch for both while the launch it saves weighs more than the value tiles' larger workgroups in it cost
-  // (2,048 tokens: 22.6 us in one launch, 13.9 + 6.9 in two; 128 tokens: 4.7 against 3.6 + 3.7)
-  if (tiles && pieces && n <= 1024) {
-    const int units = nh + 2 * nkv, lanes = units * (hd / 16);
-    const int threads = lanes >= 256 ? 256 : 64;
-    const int rope_y = (lanes + threads - 1) / threads, groups = (max_q_len + 15) / 16 + 1;
-    const long long blocks = (long long)n * rope_y + (long long)groups * nkv * n_seqs;
+  if (tiles && pieces) {
+    // Four heads a lane where a lane's piece is the same of all and 256 workgroups are left; two of some thousands of tokens, whose
+    // heads lie too far apart to be written back together (32 heads of 64, one / two / four: 1,024 tokens 10.4 / 9.5 / 8.9, 2,048
+    // 15.7 / 14.8 / 14.4, 4,096 32.9 / 32.4 / 32.6, 8,192 62.8 / 62.5 / 70.0).
+    const bool several = 16 % (hd / 16) == 0 && (long long)n * (nh + nkv) * hd >= 16 * 256 * 256 * 4LL;
+    const int each = !several ? 16 : n < 4096 ? 64 : 32, rope_y = ((nh + nkv) * (hd / 16) + each - 1) / each;
+    const int groups = (max_q_len + 15) / 16 + 1;
+    const int heads = hd <= 32 ? 4 : hd <= 64 ? 2 : 1;   // 2 hd threads finish a tile's words
+    const int row_y = (nkv * hd + 255) / 256;
+    const long long rope_blocks = (n + 15LL) / 16 * rope_y, row_blocks = (long long)v_rows * row_y;
+    const long long blocks = rope_blocks + row_blocks + (long long)groups * ((nkv + heads - 1) / heads) * n_seqs;
     GB_REQUIRE(blocks < (1ll << 31), "rope_store: %lld workgroups are too many for one launch", blocks);
-    hipLaunchKernelGGL(rope_and_values_kernel, dim3((unsigned)blocks), dim3(threads), 16 * (hd + 2) * sizeof(bf16), stream,
-                       (bf16*)qkv, row_stride, cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, rotate,
-                       v_rows, n * rope_y, rope_y, q_start, q_len, pos0, seq_base, groups);
+    const auto kernel = each == 64 ? rope_and_values_kernel<4> : each == 32 ? rope_and_values_kernel<2> : rope_and_values_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), heads * 16 * (hd + 2) * sizeof(bf16), stream,
+                       (bf16*)qkv, row_stride, cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, n, nh, nkv, hd, page_size, rotate,
+                       (int)rope_blocks, rope_y, (int)row_blocks, row_y, q_start, q_len, pos0, seq_base, groups, heads);
     return launched("rope_store (with the portions' values)");
   }
   if (tiles) {
@@ -516,7 +589,7 @@ extern "C" int gb_rope_store(void* qkv, int dtype, int row_stride, const float* 
     const dim3 grid(n, (lanes + threads - 1) / threads);
     GB_REQUIRE(grid.y <= 65535, "rope_store: %d heads are too many for one launch", units);
     hipLaunchKernelGGL(rope_store_pieces_kernel, grid, dim3(threads), 0, stream, (bf16*)qkv, row_stride, cosv, sinv, slots,
-                       (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, rotate, v_rows);
+                       (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, rotate);
     return launched("rope_store");
   }
   if (pairs_of_two) {

@@ -1008,6 +1008,38 @@ def test_rope_store_writes_values_of_portions_in_tiles(dtype, hd, page):
     assert results[0][2].abs().sum() > 0
 
 
+@pytest.mark.parametrize("nh,nkv,hd,page,q_lens,n_dec", [
+    # one, four and two heads a lane; heads that a workgroup's lanes do not divide, and more lanes than heads are left
+    (32, 32, 64, 16, [1] * 30 + [482], 30), (9, 3, 64, 16, [1, 1, 17, 40], 2), (5, 2, 48, 32, [33, 15], 0), (6, 3, 96, 16, [1, 700], 1),
+    (32, 32, 64, 16, [1, 1023], 1), (34, 9, 64, 64, [777, 778], 0), (30, 5, 128, 16, [1100], 0), (40, 24, 16, 16, [1, 4200], 1),
+    (30, 3, 32, 16, [4099], 0), (15, 5, 64, 16, [4097], 0)])
+def test_rope_store_of_steps_with_portions_in_one_launch(nh, nkv, hd, page, q_lens, n_dec):
+    """Rotation, key writes, values of single rows and of portions in one launch, against every row written by itself."""
+    from glassbox_amd import ops
+    pos0 = [(5 * i) % 23 + (9 if i < n_dec else 0) for i in range(len(q_lens))]
+    n, slots, next_page = sum(q_lens), [], 0
+    for length, first in zip(q_lens, pos0):
+        count = -(-(first + length) // page)
+        mine = [next_page + (7 * i) % count for i in range(count)] if count % 7 else list(range(next_page, next_page + count))
+        next_page += count
+        slots += [mine[p // page] * page + p % page for p in range(first, first + length)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    q_start = np.concatenate([[0], np.cumsum(q_lens)[:-1]]).tolist()
+    qkv = rnd(n, (nh + 2 * nkv) * hd, seed=5).bfloat16()
+    cos, sin = torch.rand(n, hd // 2, device=DEV), torch.rand(n, hd // 2, device=DEV)
+    for rotate in (True, False):
+        results = []
+        for portions in (None, (n_dec, i32(q_start), i32(q_lens), i32(pos0), n_dec, len(q_lens) - n_dec, max(q_lens))):
+            k_pages = torch.zeros(ops.key_pages_shape(next_page, nkv, page, hd), device=DEV, dtype=torch.bfloat16)
+            v_pages = torch.zeros(next_page, nkv, hd, page, device=DEV, dtype=torch.bfloat16)
+            buf = to_dev(qkv.clone())
+            ops.rope_store(buf, cos, sin, i32(slots), k_pages, v_pages, nh, nkv, hd, rotate=rotate, portions=portions)
+            results.append((buf, k_pages, v_pages))
+        for a, b in zip(*results):
+            assert torch.equal(a, b)
+        assert results[0][2].abs().sum() > 0
+
+
 # ---------------------------------------------------------------------- attention
 def paged_setup(ctx_lens, nkv, hd, page, seed, dtype, scatter=True):
     """Keys and values of several requests scattered over pages in a shuffled order."""
