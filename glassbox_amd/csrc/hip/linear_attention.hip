@@ -23,7 +23,8 @@
 // Around it: `retention_prep` (rotation of the first `rot` dimensions of the q and k heads in rotate-half pairs,
 // k scaled), `gla_prep` (q scaled, decays sigmoid(z)^(1/tau) from the low-rank projection z = A2 t + b), and
 // `head_norm_gate` (each head's output divided by its root mean square, an optional weight over dv, times
-// silu(gate), written in the activations' type for the output projection).
+// silu(gate), written in the activations' type for the output projection).  Steps of few tokens a request do all of it in
+// one launch (`gb_linear_heads`).
 #include "common.h"
 
 using namespace gb;
@@ -62,60 +63,154 @@ struct Segment {
   }
 };
 
-template <typename T, int R, bool GATED>
+// R rows of a column of the state from and to memory, by words of four where a key's channels are whole words of them.
+template <int R>
+__device__ __forceinline__ void load_rows(float (&x)[R], const float* __restrict__ src, bool live, int rows, int words) {
+  if (R % 4 == 0 && words) {
+#pragma unroll
+    for (int m = 0; m + 3 < R; m += 4) {
+      const f32x4 w = live && m < rows ? *reinterpret_cast<const f32x4*>(src + m) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[m + e] = w[e];
+    }
+    return;
+  }
+#pragma unroll
+  for (int m = 0; m < R; ++m) x[m] = live && m < rows ? src[m] : 0.f;
+}
+
+template <int R>
+__device__ __forceinline__ void store_rows(float* __restrict__ dst, const float (&x)[R], int rows, int words) {
+  if (R % 4 == 0 && words) {
+#pragma unroll
+    for (int m = 0; m + 3 < R; m += 4)
+      if (m < rows) *reinterpret_cast<f32x4*>(dst + m) = f32x4{x[m], x[m + 1], x[m + 2], x[m + 3]};
+    return;
+  }
+#pragma unroll
+  for (int m = 0; m < R; ++m)
+    if (m < rows) dst[m] = x[m];
+}
+
+// The sums of U tokens by C columns, which all eight lanes of a column hold, side by side to memory: a lane writes one of them.
+template <int U, int C>
+__device__ __forceinline__ float mine_of(const float (&part)[U][C], int rg) {
+  float x = part[0][0];
+#pragma unroll
+  for (int i = 1; i < U * C; ++i) {
+    const float other = part[i / C][i % C];   // (a value, not a place to choose: the sums stay in registers)
+    x = rg == i ? +other : +x;
+  }
+  return x;
+}
+
+// What the heads' kernel makes of the projection's rows by itself.
+template <typename T>
+struct Heads {
+  const T* proj;
+  int stride, q_off, k_off, g_off, rot;
+  const float *cosv, *sinv;
+  float q_scale, k_scale;
+  const float *z, *z_bias;
+  float inv_tau;
+  const float* norm;
+  float eps;
+  T* gated;
+};
+
+__device__ __forceinline__ float log_sigmoid(float z) {
+  // log(1 / (1 + exp(-z))) without overflow on either side
+  return z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
+}
+
+// C columns a lane, 32 C a workgroup.  A token costs a lane 3 R C multiply-adds and the reads of its R rows of q, k and the decay
+// from LDS; both pipes are near full.  Everything else stays off them: the lanes of a column share the writes of its sums, one wave a
+// head keeps the product of the decays, and the state comes by words.  us, before / so: 2 single tokens, 32 heads of 64 by 64
+// 5.1 / 3.7, 64 of them 39.6 / 17.3; with the second kernel 1,555 rows of two requests 93.8 / 67.1, 6,000 of one 602 / 249 (most of
+// it the end states of segments, by words); 2,048 rows, 32 heads of 64 by 65 186 / 115, 16 of 128 by 128 273 / 142.  The bits are the same.
+// FUSED: the projection's rows in, the normed and gated rows out (a workgroup then has all of its head's columns, 64 at most): what
+// the preparing kernels and head_norm_gate do, by the same arithmetic, with no rows between them through memory.  A step of two
+// tokens, 32 heads of 64: 16.1 us in three launches, 6.5 in this one.
+template <typename T, int R, bool GATED, int C, bool FUSED>
 __global__ __launch_bounds__(kThreads) void scan_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ a, const float* __restrict__ head_decay,
     const T* __restrict__ v, int v_stride, float* __restrict__ out, float* __restrict__ state,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ state_slots, int nh, int dk, int dv, int sc, int a_head, int segs, int seg_len, float* __restrict__ seg_state,
-    float* __restrict__ seg_decay) {
+    float* __restrict__ seg_decay, int words, Heads<T> hd) {
   constexpr int DKP = R * kLanesCol;                       // rows, padded
   constexpr int PER = (kTokens * DKP) / kThreads;          // staged elements a thread and array (R >= 2)
-  __shared__ float qs[kTokens][DKP], ks[kTokens][DKP], ds[GATED ? kTokens : 1][GATED ? DKP : 1];
-  __shared__ float vs[kTokens][kColsBlock];
+  constexpr int COLS = kColsBlock * C;
+  __shared__ __attribute__((aligned(16))) float qs[kTokens][DKP], ks[kTokens][DKP], ds[GATED ? kTokens : 1][GATED ? DKP : 4];
+  __shared__ __attribute__((aligned(16))) float vs[kTokens][COLS], os[FUSED ? kTokens : 1][FUSED ? COLS : 4];
   const Segment sg(q_start, q_len, blockIdx.z, segs, seg_len);
   if (sg.seg >= sg.n_segs) return;
-  const int seq = sg.seq, h = blockIdx.y, col0 = blockIdx.x * kColsBlock;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int rg = lane % kLanesCol;                          // which R rows of the column
-  const int cb = wave * kColsWave + lane / kLanesCol;       // column within the block
+  const int seq = sg.seq, h = blockIdx.y, col0 = blockIdx.x * COLS;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int rg = lane % kLanesCol;                                // which R rows of the columns
+  const int cb = (wave * kColsWave + lane / kLanesCol) * C;       // first column within the block
   const int col = col0 + cb;
   const int first = sg.first, count = sg.count;
   const int width = nh * dk;
-  const bool live = col < dv;
+  const bool idle = col0 + wave * kColsWave * C >= dv;      // a wave without columns only stages
   const bool cut = sg.n_segs > 1;                           // the request's portion runs as several segments
+  const bool track = GATED && cut && blockIdx.x == 0 && wave == 0;   // the wave that keeps the segment's decays
 
-  float S[R], P[GATED ? R : 1];
-  float* slot_row = state + (((size_t)state_slots[seq] * nh + h) * sc + (live ? col : 0)) * dk + rg * R;
+  float S[C][R], P[GATED ? R : 1];
   // where the end state goes: the request's slot, or, of a segment, the workspace
-  float* srow = cut ? seg_state + (((size_t)blockIdx.z * nh + h) * dv + (live ? col : 0)) * dk + rg * R : slot_row;
+  float* slot_row = state + (((size_t)state_slots[seq] * nh + h) * sc + col) * dk + rg * R;
+  float* srow = cut ? seg_state + (((size_t)blockIdx.z * nh + h) * dv + col) * dk + rg * R : slot_row;
   // a request's first tokens start from an empty state, whatever the slot held; so does every segment but the first
   const bool fresh = pos0[seq] == 0 || sg.seg > 0;
 #pragma unroll
-  for (int m = 0; m < R; ++m) S[m] = (!fresh && live && rg * R + m < dk) ? slot_row[m] : 0.f;
+  for (int c = 0; c < C; ++c) load_rows<R>(S[c], slot_row + (size_t)c * dk, !fresh && col + c < dv, dk - rg * R, words);
 #pragma unroll
   for (int m = 0; m < (GATED ? R : 1); ++m) P[m] = 1.f;
   const float decay = GATED ? 1.f : head_decay[h];
 
-  float nq[PER], nk[PER], na[GATED ? PER : 1], nv[2];
+  float nq[PER], nk[PER], na[GATED ? PER : 1], nv[2 * C];
   auto fetch = [&](int t0) {   // tokens t0 .. t0 + kTokens - 1 of this request's rows into registers
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const int idx = tid + e * kThreads, tok = idx / DKP, ch = idx % DKP;
       const bool ok = t0 + tok < count && ch < dk;
-      const size_t at = (size_t)(first + t0 + tok) * width + (size_t)h * dk + ch;
-      nq[e] = ok ? q[at] : 0.f;
-      nk[e] = ok ? k[at] : 0.f;
-      if (GATED) na[e] = ok ? a[a_head ? (size_t)(first + t0 + tok) * nh + h : at] : 0.f;
+      if constexpr (FUSED) {
+        nq[e] = nk[e] = 0.f;
+        if (GATED) na[e] = 0.f;
+        if (!ok) continue;
+        const size_t t = (size_t)(first + t0 + tok);
+        const T* qr = hd.proj + t * hd.stride + hd.q_off + h * dk;
+        const T* kr = hd.proj + t * hd.stride + hd.k_off + h * dk;
+        float xq = to_f(qr[ch]), xk = to_f(kr[ch]);
+        if (GATED) {
+          float z = hd.z[t * width + h * dk + ch];
+          z += hd.z_bias ? hd.z_bias[h * dk + ch] : 0.f;
+          na[e] = expf(log_sigmoid(z) * hd.inv_tau);
+        } else if (ch < hd.rot) {
+          const int half = hd.rot / 2;
+          const bool lower = ch < half;
+          const int i = lower ? ch : ch - half, o = lower ? ch + half : ch - half;
+          const float cs = hd.cosv[t * half + i], sn = hd.sinv[t * half + i], oq = to_f(qr[o]), ok2 = to_f(kr[o]);
+          xq = lower ? xq * cs - oq * sn : xq * cs + oq * sn;
+          xk = lower ? xk * cs - ok2 * sn : xk * cs + ok2 * sn;
+        }
+        nq[e] = GATED ? xq * hd.q_scale : xq;
+        nk[e] = GATED ? xk : xk * hd.k_scale;
+      } else {
+        const size_t at = (size_t)(first + t0 + tok) * width + (size_t)h * dk + ch;
+        nq[e] = ok ? q[at] : 0.f;
+        nk[e] = ok ? k[at] : 0.f;
+        if (GATED) na[e] = ok ? a[a_head ? (size_t)(first + t0 + tok) * nh + h : at] : 0.f;
+      }
     }
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int idx = tid + e * kThreads, tok = idx / kColsBlock, c = idx % kColsBlock;
+    for (int e = 0; e < 2 * C; ++e) {
+      const int idx = tid + e * kThreads, tok = idx / COLS, c = idx % COLS;
       const bool ok = t0 + tok < count && col0 + c < dv;
       nv[e] = ok ? to_f(v[(size_t)(first + t0 + tok) * v_stride + (size_t)h * dv + col0 + c]) : 0.f;
     }
   };
-  static_assert(kTokens * kColsBlock == 2 * kThreads, "two staged values of v a thread");
+  static_assert(kTokens * kColsBlock == 2 * kThreads, "two staged values of v a thread and column of its lane");
 
   fetch(0);
   for (int t0 = 0; t0 < count; t0 += kTokens) {
@@ -128,21 +223,25 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
       if (GATED) (&ds[0][0])[idx] = na[e];
     }
 #pragma unroll
-    for (int e = 0; e < 2; ++e) (&vs[0][0])[tid + e * kThreads] = nv[e];
+    for (int e = 0; e < 2 * C; ++e) (&vs[0][0])[tid + e * kThreads] = nv[e];
     __syncthreads();
     if (t0 + kTokens < count) fetch(t0 + kTokens);
     const int here = min(kTokens, count - t0);
     // U tokens at a time: their operands are read from LDS together, the state goes through them in order (one
     // multiply-add a token and row is all that waits for the token before), and their outputs' sums over the rows and
-    // over the eight lanes of a column run side by side
-    constexpr int U = R <= 8 ? 4 : R == 16 ? 2 : 1;
+    // over the eight lanes of a column run side by side.  (Few tokens, FUSED: one at a time, in less code.)
+    constexpr int U = FUSED ? 1 : R <= 8 ? 4 : R == 16 ? 2 : 1;
+    static_assert(U * C <= kLanesCol, "a lane a sum");
     float* orow = out + (size_t)(first + t0) * ((size_t)nh * dv) + (size_t)h * dv + col;
-    int j = 0;
+    const int my_t = rg / C, my_c = rg % C;   // the sum that this lane writes
+    const bool writes = rg < U * C && col + my_c < dv;
+    int j = idle ? here : 0;
     for (; j + U <= here; j += U) {
-      float kk[U][R], qq[U][R], aa[GATED ? U : 1][GATED ? R : 1], vv[U], part[U];
+      float kk[U][R], qq[U][R], aa[GATED ? U : 1][GATED ? R : 1], vv[U][C], part[U][C];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        vv[u] = vs[j + u][cb];
+#pragma unroll
+        for (int c = 0; c < C; ++c) vv[u][c] = vs[j + u][cb + c];
 #pragma unroll
         for (int m = 0; m < R; ++m) {
           kk[u][m] = ks[j + u][rg * R + m];
@@ -152,43 +251,87 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        part[u] = 0.f;
 #pragma unroll
-        for (int m = 0; m < R; ++m) {
-          S[m] = fmaf(GATED ? aa[u][m] : decay, S[m], kk[u][m] * vv[u]);
-          part[u] = fmaf(S[m], qq[u][m], part[u]);
+        for (int c = 0; c < C; ++c) {
+          part[u][c] = 0.f;
+#pragma unroll
+          for (int m = 0; m < R; ++m) {
+            S[c][m] = fmaf(GATED ? aa[u][m] : decay, S[c][m], kk[u][m] * vv[u][c]);
+            part[u][c] = fmaf(S[c][m], qq[u][m], part[u][c]);
+          }
         }
-        if (GATED && cut) {
+      }
+      if (GATED && track) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
 #pragma unroll
           for (int m = 0; m < R; ++m) P[m] *= aa[u][m];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < C; ++c) part[u][c] = sum8(part[u][c]);
+      const float x = mine_of<U, C>(part, rg);
+      if (FUSED) {
+        if (writes) os[j][cb + my_c] = x;
+      } else if (writes) {
+        orow[(size_t)(j + my_t) * ((size_t)nh * dv) + my_c] = x;
+      }
+    }
+    if constexpr (U > 1) {
+      for (; j < here; ++j) {   // the same sums, token by token
+        float part[1][C];
+  #pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const float vv = vs[j][cb + c];
+          part[0][c] = 0.f;
+  #pragma unroll
+          for (int m = 0; m < R; ++m) {
+            S[c][m] = fmaf(GATED ? ds[j][rg * R + m] : decay, S[c][m], ks[j][rg * R + m] * vv);
+            part[0][c] = fmaf(S[c][m], qs[j][rg * R + m], part[0][c]);
+          }
         }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) part[u] = sum8(part[u]);
-      if (rg == 0 && live) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) orow[(size_t)(j + u) * ((size_t)nh * dv)] = part[u];
+        if (GATED && track) {
+  #pragma unroll
+          for (int m = 0; m < R; ++m) P[m] *= ds[j][rg * R + m];
+        }
+  #pragma unroll
+        for (int c = 0; c < C; ++c) part[0][c] = sum8(part[0][c]);
+        const float x = mine_of<1, C>(part, rg);
+        if (rg < C && col + rg < dv) orow[(size_t)j * ((size_t)nh * dv) + rg] = x;
       }
     }
-    for (; j < here; ++j) {   // the same sums, token by token
-      const float vv = vs[j][cb];
-      float part = 0.f;
+    if constexpr (FUSED) {   // head_norm_gate_words_kernel's sums: sixteen lanes a token, four values a lane
+      static_assert(kThreads == 16 * kTokens, "sixteen lanes a token");
+      typedef T quad __attribute__((ext_vector_type(4)));
+      __syncthreads();
+      const int tok = tid / 16, d0 = tid % 16 * 4;
+      const bool mine = tok < here && d0 < dv;
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+      if (mine) x = *reinterpret_cast<const f32x4*>(&os[tok][d0]);
+      float ss = 0.f;
 #pragma unroll
-      for (int m = 0; m < R; ++m) {
-        S[m] = fmaf(GATED ? ds[j][rg * R + m] : decay, S[m], ks[j][rg * R + m] * vv);
-        part = fmaf(S[m], qs[j][rg * R + m], part);
-        if (GATED && cut) P[m] *= ds[j][rg * R + m];
+      for (int e = 0; e < 4; ++e) ss = fmaf(x[e], x[e], ss);
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) ss += __shfl_xor(ss, off, kWave);
+      const float s = 1.0f / sqrtf(ss / (float)dv + hd.eps);
+      if (mine) {
+        const size_t t = (size_t)(first + t0 + tok);
+        const quad g4 = *reinterpret_cast<const quad*>(hd.proj + t * hd.stride + hd.g_off + h * dv + d0);
+        quad y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = to_f(g4[e]);
+          y[e] = from_f<T>(((hd.norm ? hd.norm[d0 + e] : 1.0f) * (x[e] * s)) * (g / (1.0f + expf(-g))));
+        }
+        *reinterpret_cast<quad*>(hd.gated + (t * nh + h) * dv + d0) = y;
       }
-      part = sum8(part);
-      if (rg == 0 && live) orow[(size_t)j * ((size_t)nh * dv)] = part;
     }
   }
-  if (live) {
 #pragma unroll
-    for (int m = 0; m < R; ++m)
-      if (rg * R + m < dk) srow[m] = S[m];
-  }
-  if (GATED && cut && blockIdx.x == 0 && cb == 0) {   // the segment's decays, once a head
+  for (int c = 0; c < C; ++c)
+    if (col + c < dv) store_rows<R>(srow + (size_t)c * dk, S[c], dk - rg * R, words);
+  if (GATED && track && cb == 0) {   // the segment's decays, once a head
     float* drow = seg_decay + ((size_t)blockIdx.z * nh + h) * dk + rg * R;
 #pragma unroll
     for (int m = 0; m < R; ++m)
@@ -197,22 +340,22 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
 }
 
 // The second kernel of a portion that ran as segments (see the top of the file): same grid, same lanes.
-template <int R, bool GATED>
+template <int R, bool GATED, int C>
 __global__ __launch_bounds__(kThreads) void scan_join_kernel(
     const float* __restrict__ q, const float* __restrict__ a, const float* __restrict__ head_decay, float* __restrict__ out,
     float* __restrict__ state, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
     const int32_t* __restrict__ state_slots, int nh, int dk, int dv, int sc, int a_head, int segs, int seg_len, const float* __restrict__ seg_state,
-    const float* __restrict__ seg_decay) {
+    const float* __restrict__ seg_decay, int words) {
   constexpr int DKP = R * kLanesCol;
   constexpr int PER = (kTokens * DKP) / kThreads;
-  __shared__ float qs[kTokens][DKP], ds[GATED ? kTokens : 1][GATED ? DKP : 1];
+  __shared__ __attribute__((aligned(16))) float qs[kTokens][DKP], ds[GATED ? kTokens : 1][GATED ? DKP : 4];
   const Segment sg(q_start, q_len, blockIdx.z, segs, seg_len);
   if (sg.n_segs <= 1 || sg.seg == 0 || sg.seg >= sg.n_segs) return;   // nothing was cut, or the segment started from the state
-  const int h = blockIdx.y, col0 = blockIdx.x * kColsBlock;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int rg = lane % kLanesCol, cb = wave * kColsWave + lane / kLanesCol, col = col0 + cb;
+  const int h = blockIdx.y, col0 = blockIdx.x * kColsBlock * C;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int rg = lane % kLanesCol, cb = (wave * kColsWave + lane / kLanesCol) * C, col = col0 + cb;
   const int first = sg.first, count = sg.count, width = nh * dk;
-  const bool live = col < dv;
+  const bool idle = col0 + wave * kColsWave * C >= dv;
   const float decay = GATED ? 1.f : head_decay[h];
   float whole = 1.f;   // a full segment's decay, for a decay a head: the same products in the same order as token by token
   if (!GATED)
@@ -220,30 +363,27 @@ __global__ __launch_bounds__(kThreads) void scan_join_kernel(
 
   // the state this segment should have started from: the end states of the segments before it, folded in order
   const size_t cell0 = (size_t)sg.seq * segs;
-  auto e_row = [&](int sgm) { return seg_state + ((((cell0 + sgm) * nh + h) * dv + (live ? col : 0)) * dk) + rg * R; };
-  float S0[R];
+  auto e_row = [&](int sgm, int c) { return seg_state + ((((cell0 + sgm) * nh + h) * dv + col + c) * dk) + rg * R; };
+  float S0[C][R];
 #pragma unroll
-  for (int m = 0; m < R; ++m) S0[m] = (live && rg * R + m < dk) ? e_row(0)[m] : 0.f;
-  constexpr int F = R <= 8 ? 4 : 1;   // segments whose end states are asked for together
+  for (int c = 0; c < C; ++c) load_rows<R>(S0[c], e_row(0, c), col + c < dv, dk - rg * R, words);
+  constexpr int F = R <= 8 ? 4 / C : 1;   // segments whose end states are asked for together
   for (int s0 = 1; s0 < sg.seg; s0 += F) {
-    float e[F][R], d[F][GATED ? R : 1];
+    float e[F][C][R], d[F][GATED ? R : 1];
 #pragma unroll
     for (int f = 0; f < F; ++f) {
       const int sgm = min(s0 + f, sg.seg - 1);
-      const float* ep = e_row(sgm);
-      const float* dp = seg_decay + ((cell0 + sgm) * nh + h) * dk + rg * R;
 #pragma unroll
-      for (int m = 0; m < R; ++m) {
-        const bool ok = live && rg * R + m < dk;
-        e[f][m] = ok ? ep[m] : 0.f;
-        if (GATED) d[f][m] = ok ? dp[m] : 0.f;
-      }
+      for (int c = 0; c < C; ++c) load_rows<R>(e[f][c], e_row(sgm, c), col + c < dv, dk - rg * R, words);
+      if constexpr (GATED) load_rows<R>(d[f], seg_decay + ((cell0 + sgm) * nh + h) * dk + rg * R, true, dk - rg * R, words);
     }
 #pragma unroll
     for (int f = 0; f < F; ++f) {
       if (s0 + f >= sg.seg) break;
 #pragma unroll
-      for (int m = 0; m < R; ++m) S0[m] = fmaf(GATED ? d[f][m] : whole, S0[m], e[f][m]);
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int m = 0; m < R; ++m) S0[c][m] = fmaf(GATED ? d[f][m] : whole, S0[c][m], e[f][c][m]);
     }
   }
 
@@ -274,16 +414,20 @@ __global__ __launch_bounds__(kThreads) void scan_join_kernel(
     const int here = min(kTokens, count - t0);
     float* orow = out + (size_t)(first + t0) * ((size_t)nh * dv) + (size_t)h * dv + col;
     constexpr int U = R <= 8 ? 4 : R == 16 ? 2 : 1;   // tokens at a time, as in the first kernel
+    static_assert(U * C <= kLanesCol, "a lane a sum");
+    const int my_t = rg / C, my_c = rg % C;
+    const bool writes = rg < U * C && col + my_c < dv;
     // what the first kernel left of these tokens' outputs, asked for before the arithmetic that is added to it
-    float was[kTokens];
+    float was[kTokens / U];
 #pragma unroll
-    for (int u = 0; u < kTokens; ++u) was[u] = (rg == 0 && live && u < here) ? orow[(size_t)u * ((size_t)nh * dv)] : 0.f;
-    int j = 0;
+    for (int i = 0; i < kTokens / U; ++i)
+      was[i] = writes && i * U + my_t < here ? orow[(size_t)(i * U + my_t) * ((size_t)nh * dv) + my_c] : 0.f;
+    int j = idle ? here : 0;
 #pragma unroll
     for (int jj = 0; jj < kTokens; jj += U) {
-      if (jj + U > here) break;
+      if (idle || jj + U > here) break;
       j = jj + U;
-      float qq[U][R], aa[GATED ? U : 1][GATED ? R : 1], part[U];
+      float qq[U][R], aa[GATED ? U : 1][GATED ? R : 1], part[U][C];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -294,37 +438,50 @@ __global__ __launch_bounds__(kThreads) void scan_join_kernel(
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        part[u] = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; ++c) part[u][c] = 0.f;
 #pragma unroll
         for (int m = 0; m < R; ++m) {
           P[m] *= GATED ? aa[u][m] : decay;
-          part[u] = fmaf(qq[u][m] * P[m], S0[m], part[u]);
+          const float qp = qq[u][m] * P[m];
+#pragma unroll
+          for (int c = 0; c < C; ++c) part[u][c] = fmaf(qp, S0[c][m], part[u][c]);
         }
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) part[u] = sum8(part[u]);
-      if (rg == 0 && live) {
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int u = 0; u < U; ++u) orow[(size_t)(jj + u) * ((size_t)nh * dv)] = was[jj + u] + part[u];
-      }
+        for (int c = 0; c < C; ++c) part[u][c] = sum8(part[u][c]);
+      const float x = mine_of<U, C>(part, rg);
+      if (writes) orow[(size_t)(jj + my_t) * ((size_t)nh * dv) + my_c] = was[jj / U] + x;
     }
     for (; j < here; ++j) {
-      float part = 0.f;
+      float part[1][C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) part[0][c] = 0.f;
 #pragma unroll
       for (int m = 0; m < R; ++m) {
         P[m] *= GATED ? ds[j][rg * R + m] : decay;
-        part = fmaf(qs[j][rg * R + m] * P[m], S0[m], part);
+        const float qp = qs[j][rg * R + m] * P[m];
+#pragma unroll
+        for (int c = 0; c < C; ++c) part[0][c] = fmaf(qp, S0[c][m], part[0][c]);
       }
-      part = sum8(part);
-      if (rg == 0 && live) orow[(size_t)j * ((size_t)nh * dv)] += part;
+#pragma unroll
+      for (int c = 0; c < C; ++c) part[0][c] = sum8(part[0][c]);
+      const float x = mine_of<1, C>(part, rg);
+      if (rg < C && col + rg < dv) orow[(size_t)j * ((size_t)nh * dv) + rg] += x;
     }
   }
-  if (sg.seg == sg.n_segs - 1 && live) {   // the request's state after the portion
-    const float* e = e_row(sg.seg);
-    float* srow = state + (((size_t)state_slots[sg.seq] * nh + h) * sc + col) * dk + rg * R;
+  if (sg.seg == sg.n_segs - 1) {   // the request's state after the portion
 #pragma unroll
-    for (int m = 0; m < R; ++m)
-      if (rg * R + m < dk) srow[m] = fmaf(P[m], S0[m], e[m]);
+    for (int c = 0; c < C; ++c) {
+      if (col + c >= dv) continue;
+      float e[R];
+      load_rows<R>(e, e_row(sg.seg, c), true, dk - rg * R, words);
+#pragma unroll
+      for (int m = 0; m < R; ++m) e[m] = fmaf(P[m], S0[c][m], e[m]);
+      store_rows<R>(state + (((size_t)state_slots[sg.seq] * nh + h) * sc + col + c) * dk + rg * R, e, dk - rg * R, words);
+    }
   }
 }
 
@@ -353,11 +510,6 @@ __global__ void retention_prep_kernel(const T* __restrict__ proj, int stride, in
     if (is_k) k32[(size_t)t * width + c] = x * k_scale;
     else q32[(size_t)t * width + c] = x;
   }
-}
-
-__device__ __forceinline__ float log_sigmoid(float z) {
-  // log(1 / (1 + exp(-z))) without overflow on either side
-  return z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
 }
 
 // q32 = q * q_scale, k32 = k, decay[t, c] = sigmoid(z)^(1/tau) with z = sum_r A2[c, r] low[t, r] + b[c]; with `zin`
@@ -606,24 +758,50 @@ __global__ __launch_bounds__(4 * kWave) void mlstm_out_kernel(const float* __res
 }
 
 template <typename T, bool GATED>
-int launch_scan(int R, dim3 grid, hipStream_t stream, const float* q, const float* k, const float* a, const float* head_decay,
+int launch_scan(int R, hipStream_t stream, const float* q, const float* k, const float* a, const float* head_decay,
                 const void* v, int v_stride, float* out, float* state, const int32_t* q_start, const int32_t* q_len,
-                const int32_t* pos0, const int32_t* slots, int nh, int dk, int dv, int sc, int a_head, int segs, int seg_len, float* seg_state,
-                float* seg_decay) {
-#define GB_SCAN(RR)                                                                                                          \
-  case RR:                                                                                                                   \
-    hipLaunchKernelGGL((scan_kernel<T, RR, GATED>), grid, dim3(kThreads), 0, stream, q, k, a, head_decay, (const T*)v, v_stride, \
-                       out, state, q_start, q_len, pos0, slots, nh, dk, dv, sc, a_head, segs, seg_len, seg_state, seg_decay); \
+                const int32_t* pos0, const int32_t* slots, int n_seqs, int nh, int dk, int dv, int sc, int a_head, int segs, int seg_len,
+                float* seg_state, float* seg_decay) {
+  const int words = dk % 4 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)seg_state % 16 == 0;
+  // Sixteen rows a lane: two columns a lane where that still leaves a workgroup for every compute unit.  A column of fewer rows
+  // keeps its lanes as busy with its own sums as LDS with its reads (us, one / two columns: 2,048 rows, 16 heads of 128 by 128 180.7 /
+  // 142.1; 32 of 64 by 65 115 / 136; 1,555 rows of two requests, 32 of 64 by 64 67.1 / 72.9); more have no registers for two.
+  const long long wide = (dv + 2 * kColsBlock - 1) / (2 * kColsBlock) * (long long)nh * n_seqs * segs;
+  const int C = R == 16 && dv > kColsBlock && wide >= 256 ? 2 : 1;
+  const dim3 grid((unsigned)((dv + kColsBlock * C - 1) / (kColsBlock * C)), (unsigned)nh, (unsigned)(n_seqs * segs));
+#define GB_SCAN(RR, CC)                                                                                                      \
+  if (R == RR && C == CC) {                                                                                                  \
+    hipLaunchKernelGGL((scan_kernel<T, RR, GATED, CC, false>), grid, dim3(kThreads), 0, stream, q, k, a, head_decay, (const T*)v, \
+                       v_stride, out, state, q_start, q_len, pos0, slots, nh, dk, dv, sc, a_head, segs, seg_len, seg_state,   \
+                       seg_decay, words, Heads<T>());                                                                        \
     if (segs > 1)                                                                                                            \
-      hipLaunchKernelGGL((scan_join_kernel<RR, GATED>), grid, dim3(kThreads), 0, stream, q, a, head_decay, out, state, q_start, \
-                         q_len, slots, nh, dk, dv, sc, a_head, segs, seg_len, (const float*)seg_state, (const float*)seg_decay); \
+      hipLaunchKernelGGL((scan_join_kernel<RR, GATED, CC>), grid, dim3(kThreads), 0, stream, q, a, head_decay, out, state, q_start, \
+                         q_len, slots, nh, dk, dv, sc, a_head, segs, seg_len, (const float*)seg_state, (const float*)seg_decay, \
+                         words);                                                                                             \
+    return launched("linear_scan");                                                                                          \
+  }
+  GB_SCAN(2, 1) GB_SCAN(4, 1) GB_SCAN(8, 1) GB_SCAN(16, 1) GB_SCAN(32, 1) GB_SCAN(16, 2)
+#undef GB_SCAN
+  return fail("linear_scan: no kernel for %d rows a lane", R);
+}
+
+template <typename T, bool GATED>
+int launch_heads(int R, hipStream_t stream, const Heads<T>& heads, int v_off, const float* head_decay, float* state,
+                 const int32_t* q_start, const int32_t* q_len, const int32_t* pos0, const int32_t* slots, int n_seqs, int nh, int dk,
+                 int dv, int sc) {
+  const int words = dk % 4 == 0 && (uintptr_t)state % 16 == 0;
+#define GB_HEADS(RR)                                                                                                         \
+  case RR:                                                                                                                   \
+    hipLaunchKernelGGL((scan_kernel<T, RR, GATED, 2, true>), dim3(1, (unsigned)nh, (unsigned)n_seqs), dim3(kThreads), 0, stream, \
+                       nullptr, nullptr, nullptr, head_decay, heads.proj + v_off, heads.stride, nullptr, state, q_start, q_len,  \
+                       pos0, slots, nh, dk, dv, sc, 0, 1, 0, nullptr, nullptr, words, heads);                                \
     break;
   switch (R) {
-    GB_SCAN(2) GB_SCAN(4) GB_SCAN(8) GB_SCAN(16) GB_SCAN(32)
-    default: return fail("linear_scan: no kernel for %d rows a lane", R);
+    GB_HEADS(2) GB_HEADS(4) GB_HEADS(8)
+    default: return fail("linear_heads: no kernel for %d rows a lane", R);
   }
-#undef GB_SCAN
-  return launched("linear_scan");
+#undef GB_HEADS
+  return launched("linear_heads");
 }
 
 }  // namespace
@@ -659,15 +837,47 @@ extern "C" int gb_linear_scan(const float* q, const float* k, const float* a, co
   float* seg_decay = segs > 1 ? seg_ws + (size_t)n_seqs * segs * nh * dv * dk : nullptr;
   int R = 2;
   while (R * kLanesCol < dk) R *= 2;
-  const dim3 grid((unsigned)((dv + kColsBlock - 1) / kColsBlock), (unsigned)nh, (unsigned)(n_seqs * segs));
   const bool gated = a != nullptr;
   if (v_dtype == kF32)
-    return gated ? launch_scan<float, true>(R, grid, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay)
-                 : launch_scan<float, false>(R, grid, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay);
+    return gated ? launch_scan<float, true>(R, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay)
+                 : launch_scan<float, false>(R, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay);
   if (v_dtype == kBF16)
-    return gated ? launch_scan<bf16, true>(R, grid, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay)
-                 : launch_scan<bf16, false>(R, grid, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay);
+    return gated ? launch_scan<bf16, true>(R, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay)
+                 : launch_scan<bf16, false>(R, stream, q, k, a, head_decay, v, v_stride, out, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols, a_head, segs, seg_len, seg_state, seg_decay);
   return fail("linear_scan: unknown dtype %d", v_dtype);
+}
+
+// gb_retention_prep (no z) or gb_gla_prep (with z, the decays' products [n, nh * dk] float32), gb_linear_scan and
+// gb_head_norm_gate in one launch, for heads of up to 64 key and value channels: proj [n, stride] holds q, k, v and the gate at
+// the given columns, out [n, nh * dv] is in its type.  For steps of few tokens a request: every token's q, k and decay are
+// prepared by the one workgroup that walks the head's whole state.
+extern "C" int gb_linear_heads(const void* proj, int dtype, int stride, int q_off, int k_off, int v_off, int g_off, const float* cosv,
+                               const float* sinv, int rot, float q_scale, float k_scale, const float* z, const float* z_bias,
+                               float inv_tau, const float* head_decay, const float* norm, float eps, void* out, float* state,
+                               const int32_t* q_start, const int32_t* q_len, const int32_t* pos0, const int32_t* state_slots,
+                               int n_seqs, int nh, int dk, int dv, int state_cols, hipStream_t stream) {
+  GB_REQUIRE(n_seqs >= 0 && nh > 0 && dk > 0 && dv > 0 && dk <= 64 && dv <= 64 && dv % 4 == 0 && state_cols >= dv,
+             "linear_heads: bad sizes requests=%d heads=%d dk=%d dv=%d state columns=%d", n_seqs, nh, dk, dv, state_cols);
+  GB_REQUIRE((z != nullptr) != (head_decay != nullptr), "linear_heads: a decay a head or a decay a key channel, one of the two");
+  GB_REQUIRE(rot >= 0 && rot <= dk && rot % 2 == 0 && (rot == 0 || (!z && cosv && sinv)), "linear_heads: %d rotated dimensions", rot);
+  GB_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && g_off >= 0 && q_off + nh * dk <= stride && k_off + nh * dk <= stride &&
+                 v_off + nh * dv <= stride && g_off + nh * dv <= stride, "linear_heads: heads beyond the row");
+  const int gw = dtype == kF32 ? 16 : 8;   // a word of four values
+  GB_REQUIRE(dtype == kF32 || dtype == kBF16, "linear_heads: unknown dtype %d", dtype);
+  GB_REQUIRE(stride % 4 == 0 && g_off % 4 == 0 && (uintptr_t)proj % gw == 0 && (uintptr_t)out % gw == 0,
+             "linear_heads: the gate or the result does not lie at words");
+  GB_REQUIRE(n_seqs <= 65535 && nh <= 65535, "linear_heads: too many requests or heads for one launch");
+  if (n_seqs == 0) return 0;
+  int R = 2;
+  while (R * kLanesCol < dk) R *= 2;
+  if (dtype == kF32) {
+    const Heads<float> heads{(const float*)proj, stride, q_off, k_off, g_off, rot, cosv, sinv, q_scale, k_scale, z, z_bias, inv_tau, norm, eps, (float*)out};
+    return z ? launch_heads<float, true>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols)
+             : launch_heads<float, false>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols);
+  }
+  const Heads<bf16> heads{(const bf16*)proj, stride, q_off, k_off, g_off, rot, cosv, sinv, q_scale, k_scale, z, z_bias, inv_tau, norm, eps, (bf16*)out};
+  return z ? launch_heads<bf16, true>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols)
+           : launch_heads<bf16, false>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols);
 }
 
 extern "C" int gb_retention_prep(const void* proj, int dtype, int stride, int q_off, int k_off, const float* cosv,
@@ -805,6 +1015,7 @@ extern "C" int gb_mlstm_out(const float* o, const float* coef, const void* gate,
 }
 
 GB_TAPED(gb_linear_scan)
+GB_TAPED(gb_linear_heads)
 GB_TAPED(gb_retention_prep)
 GB_TAPED(gb_gla_prep)
 GB_TAPED(gb_head_norm_gate)

@@ -185,6 +185,10 @@ _SIGS = {
         # dk, dv, state columns a head, decay a head (0/1), segments, rows a segment, workspace, its floats, stream
         "gb_linear_scan": [_vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp,
                            C.c_longlong, _vp],
+        # proj, dtype, stride, q_off, k_off, v_off, g_off, cos, sin, rot, q_scale, k_scale, z, z_bias, 1 / tau, head_decay,
+        # norm weight, eps, out, state, q_start, q_len, pos0, state slots, requests, heads, dk, dv, state columns, stream
+        "gb_linear_heads": [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _f, _f, _vp, _vp, _f, _vp, _vp, _f, _vp, _vp, _vp, _vp, _vp,
+                            _vp, _i, _i, _i, _i, _i, _vp],
         # z, ldz, bias_i, bias_f, cap, coef, state, floats a head, where m lies, q_start, q_len, pos0, state slots,
         # requests, heads, rows, every request one row (0/1), stream
         "gb_mlstm_gates": [_vp, _i, _vp, _vp, _f, _vp, _vp, C.c_longlong, C.c_longlong, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -862,6 +866,52 @@ def linear_scan(q32: torch.Tensor, k32: torch.Tensor, v: torch.Tensor, out: torc
             _p(state), _p(ctx.q_start), _p(ctx.q_len), _p(ctx.pos0), _p(ctx.state_slots), ctx.num_seqs, n_heads, key_dim,
             value_dim, int(state.shape[2]), 1 if a_head else 0, int(segments), LINEAR_SEGMENT, _p(workspace) if segments > 1 else None,
             workspace.numel() if segments > 1 else 0, _stream())
+
+
+LINEAR_HEADS_TOKENS = 16   # linear_attention.hip: tokens of a request that a workgroup stages at a time
+
+
+def linear_heads_takes(proj: torch.Tensor, max_q_len: int, key_dim: int, value_dim: int, g_off: int) -> bool:
+    """Whether ``linear_heads`` does a step whose longest portion has ``max_q_len`` rows: of few tokens a request, and of heads
+    that one workgroup holds."""
+    return (max_q_len <= LINEAR_HEADS_TOKENS and key_dim <= 64 and value_dim <= 64 and value_dim % 4 == 0 and g_off % 4 == 0
+            and proj.stride(0) % 4 == 0 and proj.data_ptr() % (16 if proj.dtype == torch.float32 else 8) == 0)
+
+
+def linear_heads(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, out: torch.Tensor, state: torch.Tensor, ctx,
+                 n_heads: int, key_dim: int, value_dim: int, eps: float, norm_weight: Optional[torch.Tensor] = None,
+                 cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None, rot: int = 0, q_scale: float = 1.0,
+                 k_scale: float = 1.0, z: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None, tau: float = 1.0,
+                 head_decay: Optional[torch.Tensor] = None) -> None:
+    """``retention_prep`` (with ``head_decay``) or ``gla_prep`` (with ``z``), ``linear_scan`` and ``head_norm_gate`` in one launch,
+    by the same arithmetic, where ``linear_heads_takes`` says so: queries, keys, values and the gate at columns of the
+    projection's rows, ``out`` [n, heads * value_dim] contiguous in its type."""
+    _dev(proj, out, state, norm_weight, cos, sin, z, z_bias, head_decay)
+    n = proj.shape[0]
+    if rot:
+        for t in (cos, sin):
+            if t is None or t.dtype != torch.float32 or not t.is_contiguous() or t.shape[1] != rot // 2 or t.shape[0] < n:
+                raise KernelError("linear_heads: cos/sin must be contiguous float32 [n, rot / 2]")
+    if z is not None:
+        _f32_rows(z, (n, n_heads * key_dim), "z")
+        if z_bias is not None:
+            _f32_rows(z_bias, (n_heads * key_dim,), "z_bias")
+    if head_decay is not None:
+        _f32_rows(head_decay, (n_heads,), "head_decay")
+    if norm_weight is not None:
+        _f32_rows(norm_weight, (value_dim,), "norm weight")
+    if out.dtype != proj.dtype or tuple(out.shape) != (n, n_heads * value_dim) or not out.is_contiguous():
+        raise KernelError("linear_heads: out must be contiguous [n, heads * value_dim] of the projection's type")
+    if max(q_off, k_off) + n_heads * key_dim > proj.shape[1] or max(v_off, g_off) + n_heads * value_dim > proj.shape[1]:
+        raise KernelError("linear_heads: the heads lie beyond the projection's rows")
+    if (state.dtype != torch.float32 or not state.is_contiguous() or state.dim() != 4 or state.shape[1] != n_heads
+            or state.shape[2] < value_dim or state.shape[3] != key_dim):
+        raise KernelError("linear_heads: state must be contiguous float32 [slots, heads, value_dim or more, key_dim]")
+    lib = _lib("linear_attention")
+    _launch(lib, lib.gb_linear_heads, _p(proj), dtype_code(proj), _rows(proj, "proj"), int(q_off), int(k_off), int(v_off),
+            int(g_off), _p(cos) if rot else None, _p(sin) if rot else None, int(rot), float(q_scale), float(k_scale), _p(z),
+            _p(z_bias), 1.0 / float(tau), _p(head_decay), _p(norm_weight), float(eps), _p(out), _p(state), _p(ctx.q_start),
+            _p(ctx.q_len), _p(ctx.pos0), _p(ctx.state_slots), ctx.num_seqs, n_heads, key_dim, value_dim, int(state.shape[2]), _stream())
 
 
 def head_norm_gate(o: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.Tensor], out: torch.Tensor, n_heads: int,

@@ -78,6 +78,18 @@ class _LinearMixer(Mixer):
             product(ctx, h, self.w_in, proj)
         return proj
 
+    def _at_once(self, ctx, proj, residual, cache, store, norm_weight, **kind) -> bool:
+        """All of a step of few tokens a request in one launch, where there is one for it, and the output projection."""
+        g_off = 2 * self.qk_dim + self.v_dim
+        if (cache is None or cache.state is None
+                or not ops.linear_heads_takes(proj, int(ctx.host["max_q_len"]), self.key_dim, self.value_dim, g_off)):
+            return False
+        gated = ctx.buffer("lin_gated", (proj.shape[0], self.v_dim), ctx.dtype)
+        ops.linear_heads(proj, 0, self.qk_dim, 2 * self.qk_dim, g_off, gated, cache.state, ctx, self.n_heads, self.key_dim,
+                         self.value_dim, self.eps, norm_weight=norm_weight, **kind)
+        product(ctx, gated, self.wo, residual, accumulate=not store)
+        return True
+
     def _finish(self, ctx, proj, q32, k32, residual, cache, store, norm_weight, decay=None, head_decay=None):
         n = proj.shape[0]
         if cache is None or cache.state is None:
@@ -124,9 +136,12 @@ class Retention(_LinearMixer):
         """Adds the mixed rows into ``residual``, or with ``store`` writes them there (float32 either way)."""
         n = h.shape[0]
         proj = self._project(ctx, h)
+        cos, sin = self.position.table(ctx) if self.position is not None else (None, None)
+        if self._at_once(ctx, proj, residual, cache, store, None, cos=cos, sin=sin, rot=self.rot_dims,
+                         k_scale=1.0 / math.sqrt(self.key_dim), head_decay=self.head_decay):
+            return
         q32 = ctx.buffer("lin_q", (n, self.qk_dim), torch.float32)
         k32 = ctx.buffer("lin_k", (n, self.qk_dim), torch.float32)
-        cos, sin = self.position.table(ctx) if self.position is not None else (None, None)
         ops.retention_prep(proj, 0, self.qk_dim, cos, sin, q32, k32, self.n_heads, self.key_dim, self.rot_dims,
                            1.0 / math.sqrt(self.key_dim))
         self._finish(ctx, proj, q32, k32, residual, cache, store, None, head_decay=self.head_decay)
@@ -173,9 +188,6 @@ class GatedLinearAttention(_LinearMixer):
         main = 2 * self.qk_dim + 2 * self.v_dim
         # (the narrow rows of the decay and the filling rows behind them, where the rest is whole words)
         proj = self._project(ctx, h, tail=self.w_in.shape[0] - main if main % 8 == 0 else 0)
-        q32 = ctx.buffer("lin_q", (n, self.qk_dim), torch.float32)
-        k32 = ctx.buffer("lin_k", (n, self.qk_dim), torch.float32)
-        decay = ctx.buffer("lin_decay", (n, self.qk_dim), torch.float32)
         low_off, rank = 2 * self.qk_dim + 2 * self.v_dim, self.w_a2.shape[1]
         z = None
         if ctx.dtype == torch.float32 or (rank % 8 == 0 and low_off % 8 == 0):
@@ -183,6 +195,12 @@ class GatedLinearAttention(_LinearMixer):
             # take: inside the kernel)
             z = ctx.buffer("lin_z", (n, self.qk_dim), torch.float32)
             product(ctx, proj[:, low_off:low_off + rank], self.w_a2, z)
+            if self._at_once(ctx, proj, residual, cache, store, self.norm_weight, q_scale=1.0 / math.sqrt(self.key_dim), z=z,
+                             z_bias=self.a2_bias, tau=self.tau):
+                return
+        q32 = ctx.buffer("lin_q", (n, self.qk_dim), torch.float32)
+        k32 = ctx.buffer("lin_k", (n, self.qk_dim), torch.float32)
+        decay = ctx.buffer("lin_decay", (n, self.qk_dim), torch.float32)
         ops.gla_prep(proj, 0, self.qk_dim, low_off, self.w_a2, self.a2_bias, q32, k32, decay,
                      1.0 / math.sqrt(self.key_dim), self.tau, z=z)
         self._finish(ctx, proj, q32, k32, residual, cache, store, self.norm_weight, decay=decay)

@@ -157,6 +157,78 @@ def test_decays_of_key_channels_and_the_gated_head_norm():
             assert (out.cpu().to(F64) - want).abs().max() < 1e-5, (T, H, dv)
 
 
+def _step(lens, pos0):
+    starts = np.cumsum([0] + list(lens))[:-1]
+    return SimpleNamespace(q_start=_i32(starts), q_len=_i32(lens), pos0=_i32(pos0), state_slots=_i32(range(len(lens))), num_seqs=len(lens))
+
+
+@pytest.mark.parametrize("dk, dv, kind", [(128, 128, "channel"), (128, 65, "token"), (100, 33, "head"), (66, 100, "channel"),
+                                          (70, 64, "head")])
+def test_heads_with_two_columns_a_lane(dk, dv, kind):
+    """Steps that fill the chip give a lane two columns of the state (of 65 to 128 rows); the same rows a head at a time give it
+    one.  Column by column the sums are the same: outputs and states bit for bit, cut into segments and not."""
+    from glassbox_amd import ops
+    torch.manual_seed(dk * dv)
+    H, lens, pos0 = 64, [5, 200, 1, 19], [7, 0, 3, 0]
+    for lens in (lens, [300, 2, 517, 129]):
+        n, ctx = sum(lens), _step(lens, pos0)
+        q, k = torch.randn(n, H, dk, device=DEV), torch.randn(n, H, dk, device=DEV)
+        v = torch.randn(n, H, dv, device=DEV).bfloat16()
+        a = {"channel": torch.rand(n, H, dk, device=DEV) * 0.2 + 0.8, "token": torch.rand(n, H, device=DEV) * 0.2 + 0.8,
+             "head": torch.linspace(0.9, 0.999, H, device=DEV)}[kind]
+        state = torch.randn(len(lens), H, dv, dk, device=DEV)
+        segments = ops.linear_scan_segments(max(lens))
+
+        def scan(heads, st):
+            mine = lambda t: t[:, heads].contiguous().reshape(n, -1)
+            out = torch.full((n, st.shape[1] * dv), float("nan"), device=DEV)
+            ws = torch.full((len(lens) * segments * st.shape[1] * (dv + 1) * dk,), float("nan"), device=DEV) if segments > 1 else None
+            decay = {"channel": {"decay": mine(a)} if kind == "channel" else {}, "token": {"token_decay": mine(a)} if kind == "token" else {},
+                     "head": {"head_decay": a[heads].contiguous()} if kind == "head" else {}}[kind]
+            ops.linear_scan(mine(q), mine(k), mine(v), out, st, ctx, st.shape[1], dk, dv, segments=segments, workspace=ws, **decay)
+            return out.view(n, -1, dv)
+        all_state = state.clone()
+        together = scan(slice(0, H), all_state)
+        for h in (0, H - 1):
+            one = state[:, h:h + 1].contiguous()
+            assert torch.equal(scan(slice(h, h + 1), one), together[:, h:h + 1]) and torch.equal(one, all_state[:, h:h + 1])
+        assert torch.isfinite(together).all()
+
+
+@pytest.mark.parametrize("H, dk, dv, rot, dtype", [(32, 64, 64, 64, torch.bfloat16), (3, 24, 40, 8, torch.float32),
+                                                  (5, 10, 4, 0, torch.bfloat16), (2, 64, 12, 2, torch.float32), (1, 6, 64, 6, torch.bfloat16)])
+def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, dtype):
+    """What prepares q, k and the decays, the recurrence and the gated norm at once, against the three by themselves: the same
+    arithmetic, whatever the tokens a request brings (and more than the sixteen that are staged at a time)."""
+    from glassbox_amd import ops
+    torch.manual_seed(H + dk + dv)
+    QK, V, eps = H * dk, H * dv, 1e-5
+    off = [0, QK, 2 * QK, 2 * QK + V]
+    off[3] += -off[3] % 4
+    for lens, pos0 in (([1, 1], [5, 0]), ([1, 16, 3, 2], [9, 0, 4, 0]), ([17, 40], [0, 2])):
+        n, ctx = sum(lens), _step(lens, pos0)
+        proj = torch.randn(n, off[3] + V + -(off[3] + V) % 4, device=DEV).to(dtype)
+        assert ops.linear_heads_takes(proj, 16, dk, dv, off[3])
+        cos, sin = torch.rand(n, max(rot // 2, 1), device=DEV), torch.rand(n, max(rot // 2, 1), device=DEV)
+        z, bias, w = torch.randn(n, QK, device=DEV) * 4, torch.randn(QK, device=DEV), torch.rand(dv, device=DEV) + 0.5
+        before = torch.randn(len(lens), H, dv + 2, dk, device=DEV)
+        for kind in ("head", "channel"):
+            q32, k32, decay = (torch.empty(n, QK, device=DEV) for _ in range(3))
+            if kind == "head":
+                ops.retention_prep(proj, off[0], off[1], cos, sin, q32, k32, H, dk, rot, 0.125)
+                how = {"cos": cos, "sin": sin, "rot": rot, "k_scale": 0.125, "head_decay": torch.linspace(0.9, 0.999, H, device=DEV)}
+                a = {"head_decay": how["head_decay"]}
+            else:
+                ops.gla_prep(proj, off[0], off[1], 0, torch.zeros(QK, 1, device=DEV, dtype=dtype), bias, q32, k32, decay, 0.25, 16.0, z=z)
+                how, a = {"q_scale": 0.25, "z": z, "z_bias": bias, "tau": 16.0, "norm_weight": w}, {"decay": decay}
+            states, o = [before.clone(), before.clone()], torch.empty(n, V, device=DEV)
+            outs = [torch.full((n, V), float("nan"), device=DEV, dtype=dtype) for _ in range(2)]
+            ops.linear_scan(q32, k32, proj[:, off[2]:off[2] + V], o, states[0], ctx, H, dk, dv, **a)
+            ops.head_norm_gate(o, proj[:, off[3]:off[3] + V], how.get("norm_weight"), outs[0], H, dv, eps)
+            ops.linear_heads(proj, *off, outs[1], states[1], ctx, H, dk, dv, eps, **how)
+            assert torch.equal(states[0], states[1]) and torch.equal(outs[0], outs[1]), (kind, lens)
+
+
 # ------------------------------------------------------------------------------------------ streams
 def test_streams_kernels():
     from glassbox_amd import ops
