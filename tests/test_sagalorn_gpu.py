@@ -195,6 +195,28 @@ def test_heads_with_two_columns_a_lane(dk, dv, kind):
         assert torch.isfinite(together).all()
 
 
+@pytest.mark.parametrize("H, dk, rot, dtype", [(32, 64, 64, torch.bfloat16), (5, 12, 8, torch.float32), (3, 24, 8, torch.bfloat16),
+                                               (1, 4, 0, torch.float32), (33, 64, 16, torch.bfloat16)])
+def test_rows_prepared_by_words(H, dk, rot, dtype):
+    """Four values a lane, against the same rows one column further on (which do not lie at words): the same bits."""
+    from glassbox_amd import ops
+    torch.manual_seed(H * dk + rot)
+    n, W = 37, H * dk
+    wide = torch.randn(n, 2 * W + 8, device=DEV).to(dtype)
+    shifted = torch.zeros_like(wide)
+    shifted[:, 1:] = wide[:, :-1]
+    cos, sin = torch.rand(n, max(rot // 2, 1), device=DEV), torch.rand(n, max(rot // 2, 1), device=DEV)
+    z, bias, a2 = torch.randn(n, W, device=DEV) * 4, torch.randn(W, device=DEV), torch.zeros(W, 1, device=DEV, dtype=dtype)
+    got = []
+    for proj, at in ((wide, 0), (shifted, 1)):
+        q32, k32, q, k, decay = (torch.full((n, W), float("nan"), device=DEV) for _ in range(5))
+        ops.retention_prep(proj, at + 4, at + 4 + W, cos, sin, q32, k32, H, dk, rot, 0.125)
+        ops.gla_prep(proj, at + 4, at + 4 + W, 0, a2, bias, q, k, decay, 0.25, 16.0, z=z)
+        got.append((q32, k32, q, k, decay))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("H, dk, dv, rot, dtype", [(32, 64, 64, 64, torch.bfloat16), (3, 24, 40, 8, torch.float32),
                                                   (5, 10, 4, 0, torch.bfloat16), (2, 64, 12, 2, torch.float32), (1, 6, 64, 6, torch.bfloat16)])
 def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, dtype):
