@@ -14,7 +14,8 @@
 // so neither scores nor probabilities pass through LDS, and keys and values go from memory into
 // MFMA operands directly.  Pages: keys [page][kv head][hd / 8][slot][8], values [page][kv head][hd][slot].
 // A prompt portion's columns are 32 or 64 consecutive tokens of one query head, with the same
-// scheme on the 32x32x16 instruction (described at its kernel).
+// scheme on the 32x32x16 instruction (described at its kernels; for heads of 64 and 128 the tiles
+// of keys and values come through LDS, which the waves of a workgroup share).
 //
 // Decoding splits a request's context into chunks of a multiple of 256 keys, one workgroup per
 // (chunk, kv head, request), whose waves (sixteen where one workgroup takes a whole context of more

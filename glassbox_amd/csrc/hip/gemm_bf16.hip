@@ -10,8 +10,8 @@
 //    can be its epilogue.  Its workgroups can also divide k (split k: a second pass adds their sums in order).
 //  * block  (some hundred rows): tiles of 64 to 256 rows by 64 to 128 columns, whichever move the fewest bytes, both operands
 //    straight into LDS several k-steps ahead.
-//  * ring   (some hundred rows and more, enough 256x256 tiles to fill the chip): 2x2 waves, a wave 8x8 tiles of
-//    v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
+//  * ring   (257 rows and more, where its tiles of 256 columns by 128 to 256 rows are ahead): 2x2 waves, a wave up to 8x8
+//    tiles of v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
 //  * skinny (M <= 64, decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
 //    rows of W are few); its
 //    waves take interleaved 64-wide k blocks, stream W straight from memory into MFMA operands

@@ -4,12 +4,12 @@
 // The reference sorts the candidates by descending logit and then works on prefixes of that
 // order: top-k keeps the first k, min-p the ones at least p_max*min_p, top-p the shortest prefix
 // whose probability reaches top_p, and the draw walks the same order until the running
-// probability passes a uniform number.  Nothing here sorts.  The order is a 52-bit key per
-// token (the logit's bits made monotone, then the token id, so equal logits go by id), and
-// "the first element where the running weight crosses a target" is found by a search over
-// bins of values and then of keys (see the sampler below), with weights that are whole numbers,
-// so that the result does not depend on timing.  The uniform number comes from the host, which
-// owns each request's generator.
+// probability passes a uniform number.  Only the few candidates of a row with a top-k are
+// sorted here (sample_few).  The order is a 52-bit key per token (the logit's bits made monotone,
+// then the token id, so equal logits go by id), and "the first element where the running weight
+// crosses a target" is found by a search over bins of values and then of keys (see the sampler
+// below), with weights that are whole numbers, so that the result does not depend on timing.  The
+// uniform number comes from the host, which owns each request's generator.
 #include "common.h"
 
 using namespace gb;
