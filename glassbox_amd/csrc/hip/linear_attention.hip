@@ -111,7 +111,9 @@ struct Heads {
   int stride, q_off, k_off, g_off, rot;
   const float *cosv, *sinv;
   float q_scale, k_scale;
-  const float *z, *z_bias;
+  const T* a2;   // the decays' second matrix [nh * dk, rank], or nullptr (a decay a head)
+  int low_off, rank;
+  const float* z_bias;
   float inv_tau;
   const float* norm;
   float eps;
@@ -130,7 +132,7 @@ __device__ __forceinline__ float log_sigmoid(float z) {
 // it the end states of segments, by words); 2,048 rows, 32 heads of 64 by 65 186 / 115, 16 of 128 by 128 273 / 142.  The bits are the same.
 // FUSED: the projection's rows in, the normed and gated rows out (a workgroup then has all of its head's columns, 64 at most): what
 // the preparing kernels and head_norm_gate do, by the same arithmetic, with no rows between them through memory.  A step of two
-// tokens, 32 heads of 64: 16.1 us in three launches, 6.5 in this one.
+// tokens, 32 heads of 64: a decay a head 14.2 us in three launches, 6.1 in this one; a decay a key channel 20.7 in four, 7.4.
 template <typename T, int R, bool GATED, int C, bool FUSED>
 __global__ __launch_bounds__(kThreads) void scan_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ a, const float* __restrict__ head_decay,
@@ -168,6 +170,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
   for (int m = 0; m < (GATED ? R : 1); ++m) P[m] = 1.f;
   const float decay = GATED ? 1.f : head_decay[h];
 
+  typedef T quad __attribute__((ext_vector_type(4)));
   float nq[PER], nk[PER], na[GATED ? PER : 1], nv[2 * C];
   auto fetch = [&](int t0) {   // tokens t0 .. t0 + kTokens - 1 of this request's rows into registers
 #pragma unroll
@@ -183,7 +186,15 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
         const T* kr = hd.proj + t * hd.stride + hd.k_off + h * dk;
         float xq = to_f(qr[ch]), xk = to_f(kr[ch]);
         if (GATED) {
-          float z = hd.z[t * width + h * dk + ch];
+          const T* w = hd.a2 + (size_t)(h * dk + ch) * hd.rank;
+          const T* low = hd.proj + t * hd.stride + hd.low_off;
+          float z = 0.f;
+#pragma unroll 4
+          for (int r = 0; r < hd.rank; r += 4) {
+            const quad w4 = *reinterpret_cast<const quad*>(w + r), l4 = *reinterpret_cast<const quad*>(low + r);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) z = fmaf(to_f(w4[m]), to_f(l4[m]), z);
+          }
           z += hd.z_bias ? hd.z_bias[h * dk + ch] : 0.f;
           na[e] = expf(log_sigmoid(z) * hd.inv_tau);
         } else if (ch < hd.rot) {
@@ -303,7 +314,6 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
     }
     if constexpr (FUSED) {   // head_norm_gate_words_kernel's sums: sixteen lanes a token, four values a lane
       static_assert(kThreads == 16 * kTokens, "sixteen lanes a token");
-      typedef T quad __attribute__((ext_vector_type(4)));
       __syncthreads();
       const int tok = tid / 16, d0 = tid % 16 * 4;
       const bool mine = tok < here && d0 < dv;
@@ -908,37 +918,43 @@ extern "C" int gb_linear_scan(const float* q, const float* k, const float* a, co
   return fail("linear_scan: unknown dtype %d", v_dtype);
 }
 
-// gb_retention_prep (no z) or gb_gla_prep (with z, the decays' products [n, nh * dk] float32), gb_linear_scan and
-// gb_head_norm_gate in one launch, for heads of up to 64 key and value channels: proj [n, stride] holds q, k, v and the gate at
-// the given columns, out [n, nh * dv] is in its type.  For steps of few tokens a request: every token's q, k and decay are
-// prepared by the one workgroup that walks the head's whole state.
+// gb_retention_prep (no a2) or gb_gla_prep (with a2 [nh * dk, rank], whose products with the rows' narrow columns are summed here as
+// there), gb_linear_scan and gb_head_norm_gate in one launch, for heads of up to 64 key and value channels: proj [n, stride] holds q,
+// k, v, the gate and the narrow columns at the given places, out [n, nh * dv] is in its type.  For steps of few tokens a request: every
+// token's q, k and decay are prepared by the one workgroup that walks the head's whole state.
 extern "C" int gb_linear_heads(const void* proj, int dtype, int stride, int q_off, int k_off, int v_off, int g_off, const float* cosv,
-                               const float* sinv, int rot, float q_scale, float k_scale, const float* z, const float* z_bias,
-                               float inv_tau, const float* head_decay, const float* norm, float eps, void* out, float* state,
-                               const int32_t* q_start, const int32_t* q_len, const int32_t* pos0, const int32_t* state_slots,
-                               int n_seqs, int nh, int dk, int dv, int state_cols, hipStream_t stream) {
+                               const float* sinv, int rot, float q_scale, float k_scale, const void* a2, int low_off, int rank,
+                               const float* z_bias, float inv_tau, const float* head_decay, const float* norm, float eps, void* out,
+                               float* state, const int32_t* q_start, const int32_t* q_len, const int32_t* pos0,
+                               const int32_t* state_slots, int n_seqs, int nh, int dk, int dv, int state_cols, hipStream_t stream) {
   GB_REQUIRE(n_seqs >= 0 && nh > 0 && dk > 0 && dv > 0 && dk <= 64 && dv <= 64 && dv % 4 == 0 && state_cols >= dv,
              "linear_heads: bad sizes requests=%d heads=%d dk=%d dv=%d state columns=%d", n_seqs, nh, dk, dv, state_cols);
-  GB_REQUIRE((z != nullptr) != (head_decay != nullptr), "linear_heads: a decay a head or a decay a key channel, one of the two");
-  GB_REQUIRE(rot >= 0 && rot <= dk && rot % 2 == 0 && (rot == 0 || (!z && cosv && sinv)), "linear_heads: %d rotated dimensions", rot);
+  GB_REQUIRE((a2 != nullptr) != (head_decay != nullptr), "linear_heads: a decay a head or a decay a key channel, one of the two");
+  GB_REQUIRE(rot >= 0 && rot <= dk && rot % 2 == 0 && (rot == 0 || (!a2 && cosv && sinv)), "linear_heads: %d rotated dimensions", rot);
   GB_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && g_off >= 0 && q_off + nh * dk <= stride && k_off + nh * dk <= stride &&
                  v_off + nh * dv <= stride && g_off + nh * dv <= stride, "linear_heads: heads beyond the row");
   const int gw = dtype == kF32 ? 16 : 8;   // a word of four values
   GB_REQUIRE(dtype == kF32 || dtype == kBF16, "linear_heads: unknown dtype %d", dtype);
   GB_REQUIRE(stride % 4 == 0 && g_off % 4 == 0 && (uintptr_t)proj % gw == 0 && (uintptr_t)out % gw == 0,
              "linear_heads: the gate or the result does not lie at words");
+  GB_REQUIRE(!a2 || (rank > 0 && rank % 4 == 0 && low_off >= 0 && low_off % 4 == 0 && low_off + rank <= stride && (uintptr_t)a2 % gw == 0),
+             "linear_heads: %d narrow columns at %d are no whole words of the row", rank, low_off);
   GB_REQUIRE(n_seqs <= 65535 && nh <= 65535, "linear_heads: too many requests or heads for one launch");
   if (n_seqs == 0) return 0;
   int R = 2;
   while (R * kLanesCol < dk) R *= 2;
+#define GB_HEADS_OF(T)                                                                                                          \
+  const Heads<T> heads{(const T*)proj, stride, q_off, k_off, g_off, rot, cosv, sinv, q_scale, k_scale, (const T*)a2, low_off, rank, \
+                       z_bias, inv_tau, norm, eps, (T*)out};                                                                   \
+  return a2 ? launch_heads<T, true>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, \
+                                    dv, state_cols)                                                                            \
+            : launch_heads<T, false>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, \
+                                     dk, dv, state_cols)
   if (dtype == kF32) {
-    const Heads<float> heads{(const float*)proj, stride, q_off, k_off, g_off, rot, cosv, sinv, q_scale, k_scale, z, z_bias, inv_tau, norm, eps, (float*)out};
-    return z ? launch_heads<float, true>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols)
-             : launch_heads<float, false>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols);
+    GB_HEADS_OF(float);
   }
-  const Heads<bf16> heads{(const bf16*)proj, stride, q_off, k_off, g_off, rot, cosv, sinv, q_scale, k_scale, z, z_bias, inv_tau, norm, eps, (bf16*)out};
-  return z ? launch_heads<bf16, true>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols)
-           : launch_heads<bf16, false>(R, stream, heads, v_off, head_decay, state, q_start, q_len, pos0, state_slots, n_seqs, nh, dk, dv, state_cols);
+  GB_HEADS_OF(bf16);
+#undef GB_HEADS_OF
 }
 
 extern "C" int gb_retention_prep(const void* proj, int dtype, int stride, int q_off, int k_off, const float* cosv,

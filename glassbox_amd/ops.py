@@ -185,10 +185,10 @@ _SIGS = {
         # dk, dv, state columns a head, decay a head (0/1), segments, rows a segment, workspace, its floats, stream
         "gb_linear_scan": [_vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp,
                            C.c_longlong, _vp],
-        # proj, dtype, stride, q_off, k_off, v_off, g_off, cos, sin, rot, q_scale, k_scale, z, z_bias, 1 / tau, head_decay,
-        # norm weight, eps, out, state, q_start, q_len, pos0, state slots, requests, heads, dk, dv, state columns, stream
-        "gb_linear_heads": [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _f, _f, _vp, _vp, _f, _vp, _vp, _f, _vp, _vp, _vp, _vp, _vp,
-                            _vp, _i, _i, _i, _i, _i, _vp],
+        # proj, dtype, stride, q_off, k_off, v_off, g_off, cos, sin, rot, q_scale, k_scale, a2, low_off, rank, z_bias, 1 / tau,
+        # head_decay, norm weight, eps, out, state, q_start, q_len, pos0, state slots, requests, heads, dk, dv, state columns, stream
+        "gb_linear_heads": [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _f, _f, _vp, _i, _i, _vp, _f, _vp, _vp, _f, _vp, _vp, _vp, _vp,
+                            _vp, _vp, _i, _i, _i, _i, _i, _vp],
         # z, ldz, bias_i, bias_f, cap, coef, state, floats a head, where m lies, q_start, q_len, pos0, state slots,
         # requests, heads, rows, every request one row (0/1), stream
         "gb_mlstm_gates": [_vp, _i, _vp, _vp, _f, _vp, _vp, C.c_longlong, C.c_longlong, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -868,32 +868,45 @@ def linear_scan(q32: torch.Tensor, k32: torch.Tensor, v: torch.Tensor, out: torc
             workspace.numel() if segments > 1 else 0, _stream())
 
 
-LINEAR_HEADS_TOKENS = 16   # linear_attention.hip: tokens of a request that a workgroup stages at a time
+# linear_attention.hip: tokens of a request that a workgroup stages at a time, and up to how many of them the sums over a decay's
+# middle (of so many columns at most) are made beside a head's recurrence.  us, at once / apart, 32 heads of 64, a middle of 64: one
+# token of 2 and 64 requests 5.9 / 11.2 and 18.8 / 28.8, 8 tokens of 1 and 64 9.4 / 12.1 and 38.2 / 39.9, 12 of 64 50.2 / 47.4, 16 of
+# one 14.3 / 13.3; a decay a head, 16 tokens of 1 and 64 9.0 / 9.6 and 31.5 / 38.0.
+LINEAR_HEADS_TOKENS = 16
+LINEAR_HEADS_SUMS = 8
+LINEAR_HEADS_RANK = 128
 
 
-def linear_heads_takes(proj: torch.Tensor, max_q_len: int, key_dim: int, value_dim: int, g_off: int) -> bool:
+def linear_heads_takes(proj: torch.Tensor, max_q_len: int, key_dim: int, value_dim: int, g_off: int,
+                       a2: Optional[torch.Tensor] = None, low_off: int = 0) -> bool:
     """Whether ``linear_heads`` does a step whose longest portion has ``max_q_len`` rows: of few tokens a request, and of heads
-    that one workgroup holds."""
+    that one workgroup holds (a decay's middle of up to ``LINEAR_HEADS_RANK``: every head reads it for each of its channels)."""
+    word = 16 if proj.dtype == torch.float32 else 8
+    if a2 is not None and (max_q_len > LINEAR_HEADS_SUMS or a2.shape[1] > LINEAR_HEADS_RANK or a2.shape[1] % 4 or low_off % 4 or a2.data_ptr() % word):
+        return False
     return (max_q_len <= LINEAR_HEADS_TOKENS and key_dim <= 64 and value_dim <= 64 and value_dim % 4 == 0 and g_off % 4 == 0
-            and proj.stride(0) % 4 == 0 and proj.data_ptr() % (16 if proj.dtype == torch.float32 else 8) == 0)
+            and proj.stride(0) % 4 == 0 and proj.data_ptr() % word == 0)
 
 
 def linear_heads(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, out: torch.Tensor, state: torch.Tensor, ctx,
                  n_heads: int, key_dim: int, value_dim: int, eps: float, norm_weight: Optional[torch.Tensor] = None,
                  cos: Optional[torch.Tensor] = None, sin: Optional[torch.Tensor] = None, rot: int = 0, q_scale: float = 1.0,
-                 k_scale: float = 1.0, z: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None, tau: float = 1.0,
-                 head_decay: Optional[torch.Tensor] = None) -> None:
-    """``retention_prep`` (with ``head_decay``) or ``gla_prep`` (with ``z``), ``linear_scan`` and ``head_norm_gate`` in one launch,
+                 k_scale: float = 1.0, a2: Optional[torch.Tensor] = None, low_off: int = 0, z_bias: Optional[torch.Tensor] = None,
+                 tau: float = 1.0, head_decay: Optional[torch.Tensor] = None) -> None:
+    """``retention_prep`` (with ``head_decay``) or ``gla_prep`` (with ``a2``, summed there), ``linear_scan`` and ``head_norm_gate`` in one launch,
     by the same arithmetic, where ``linear_heads_takes`` says so: queries, keys, values and the gate at columns of the
     projection's rows, ``out`` [n, heads * value_dim] contiguous in its type."""
-    _dev(proj, out, state, norm_weight, cos, sin, z, z_bias, head_decay)
+    _dev(proj, out, state, norm_weight, cos, sin, a2, z_bias, head_decay)
     n = proj.shape[0]
     if rot:
         for t in (cos, sin):
             if t is None or t.dtype != torch.float32 or not t.is_contiguous() or t.shape[1] != rot // 2 or t.shape[0] < n:
                 raise KernelError("linear_heads: cos/sin must be contiguous float32 [n, rot / 2]")
-    if z is not None:
-        _f32_rows(z, (n, n_heads * key_dim), "z")
+    if a2 is not None:
+        if a2.dtype != proj.dtype or not a2.is_contiguous() or a2.shape[0] != n_heads * key_dim:
+            raise KernelError("linear_heads: a2 must be contiguous [heads * key_dim, rank] of the projection's type")
+        if low_off + a2.shape[1] > proj.shape[1]:
+            raise KernelError("linear_heads: the decay's middle lies beyond the projection's rows")
         if z_bias is not None:
             _f32_rows(z_bias, (n_heads * key_dim,), "z_bias")
     if head_decay is not None:
@@ -909,8 +922,8 @@ def linear_heads(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: 
         raise KernelError("linear_heads: state must be contiguous float32 [slots, heads, value_dim or more, key_dim]")
     lib = _lib("linear_attention")
     _launch(lib, lib.gb_linear_heads, _p(proj), dtype_code(proj), _rows(proj, "proj"), int(q_off), int(k_off), int(v_off),
-            int(g_off), _p(cos) if rot else None, _p(sin) if rot else None, int(rot), float(q_scale), float(k_scale), _p(z),
-            _p(z_bias), 1.0 / float(tau), _p(head_decay), _p(norm_weight), float(eps), _p(out), _p(state), _p(ctx.q_start),
+            int(g_off), _p(cos) if rot else None, _p(sin) if rot else None, int(rot), float(q_scale), float(k_scale), _p(a2),
+            int(low_off), int(a2.shape[1]) if a2 is not None else 0, _p(z_bias), 1.0 / float(tau), _p(head_decay), _p(norm_weight), float(eps), _p(out), _p(state), _p(ctx.q_start),
             _p(ctx.q_len), _p(ctx.pos0), _p(ctx.state_slots), ctx.num_seqs, n_heads, key_dim, value_dim, int(state.shape[2]), _stream())
 
 

@@ -82,7 +82,8 @@ class _LinearMixer(Mixer):
         """All of a step of few tokens a request in one launch, where there is one for it, and the output projection."""
         g_off = 2 * self.qk_dim + self.v_dim
         if (cache is None or cache.state is None
-                or not ops.linear_heads_takes(proj, int(ctx.host["max_q_len"]), self.key_dim, self.value_dim, g_off)):
+                or not ops.linear_heads_takes(proj, int(ctx.host["max_q_len"]), self.key_dim, self.value_dim, g_off, kind.get("a2"),
+                                              kind.get("low_off", 0))):
             return False
         gated = ctx.buffer("lin_gated", (proj.shape[0], self.v_dim), ctx.dtype)
         ops.linear_heads(proj, 0, self.qk_dim, 2 * self.qk_dim, g_off, gated, cache.state, ctx, self.n_heads, self.key_dim,
@@ -189,15 +190,15 @@ class GatedLinearAttention(_LinearMixer):
         # (the narrow rows of the decay and the filling rows behind them, where the rest is whole words)
         proj = self._project(ctx, h, tail=self.w_in.shape[0] - main if main % 8 == 0 else 0)
         low_off, rank = 2 * self.qk_dim + 2 * self.v_dim, self.w_a2.shape[1]
+        if self._at_once(ctx, proj, residual, cache, store, self.norm_weight, q_scale=1.0 / math.sqrt(self.key_dim), a2=self.w_a2,
+                         low_off=low_off, z_bias=self.a2_bias, tau=self.tau):
+            return
         z = None
         if ctx.dtype == torch.float32 or (rank % 8 == 0 and low_off % 8 == 0):
             # the second matrix of the decay's projection as a product of its own (sizes that a bfloat16 product does not
             # take: inside the kernel)
             z = ctx.buffer("lin_z", (n, self.qk_dim), torch.float32)
             product(ctx, proj[:, low_off:low_off + rank], self.w_a2, z)
-            if self._at_once(ctx, proj, residual, cache, store, self.norm_weight, q_scale=1.0 / math.sqrt(self.key_dim), z=z,
-                             z_bias=self.a2_bias, tau=self.tau):
-                return
         q32 = ctx.buffer("lin_q", (n, self.qk_dim), torch.float32)
         k32 = ctx.buffer("lin_k", (n, self.qk_dim), torch.float32)
         decay = ctx.buffer("lin_decay", (n, self.qk_dim), torch.float32)

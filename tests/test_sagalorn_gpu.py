@@ -217,9 +217,10 @@ def test_rows_prepared_by_words(H, dk, rot, dtype):
         assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("H, dk, dv, rot, dtype", [(32, 64, 64, 64, torch.bfloat16), (3, 24, 40, 8, torch.float32),
-                                                  (5, 10, 4, 0, torch.bfloat16), (2, 64, 12, 2, torch.float32), (1, 6, 64, 6, torch.bfloat16)])
-def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, dtype):
+@pytest.mark.parametrize("H, dk, dv, rot, rank, dtype", [
+    (32, 64, 64, 64, 64, torch.bfloat16), (3, 24, 40, 8, 4, torch.float32), (5, 10, 4, 0, 20, torch.bfloat16),
+    (2, 64, 12, 2, 128, torch.float32), (1, 6, 64, 6, 8, torch.bfloat16)])
+def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, rank, dtype):
     """What prepares q, k and the decays, the recurrence and the gated norm at once, against the three by themselves: the same
     arithmetic, whatever the tokens a request brings (and more than the sixteen that are staged at a time)."""
     from glassbox_amd import ops
@@ -229,10 +230,12 @@ def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, dtype):
     off[3] += -off[3] % 4
     for lens, pos0 in (([1, 1], [5, 0]), ([1, 16, 3, 2], [9, 0, 4, 0]), ([17, 40], [0, 2])):
         n, ctx = sum(lens), _step(lens, pos0)
-        proj = torch.randn(n, off[3] + V + -(off[3] + V) % 4, device=DEV).to(dtype)
-        assert ops.linear_heads_takes(proj, 16, dk, dv, off[3])
+        low = off[3] + V
+        proj = torch.randn(n, low + rank, device=DEV).to(dtype)
+        a2 = torch.randn(QK, rank, device=DEV).to(dtype)
+        assert ops.linear_heads_takes(proj, 16, dk, dv, off[3]) and ops.linear_heads_takes(proj, 8, dk, dv, off[3], a2, low)
         cos, sin = torch.rand(n, max(rot // 2, 1), device=DEV), torch.rand(n, max(rot // 2, 1), device=DEV)
-        z, bias, w = torch.randn(n, QK, device=DEV) * 4, torch.randn(QK, device=DEV), torch.rand(dv, device=DEV) + 0.5
+        bias, w = torch.randn(QK, device=DEV), torch.rand(dv, device=DEV) + 0.5
         before = torch.randn(len(lens), H, dv + 2, dk, device=DEV)
         for kind in ("head", "channel"):
             q32, k32, decay = (torch.empty(n, QK, device=DEV) for _ in range(3))
@@ -241,8 +244,8 @@ def test_heads_of_short_steps_in_one_launch(H, dk, dv, rot, dtype):
                 how = {"cos": cos, "sin": sin, "rot": rot, "k_scale": 0.125, "head_decay": torch.linspace(0.9, 0.999, H, device=DEV)}
                 a = {"head_decay": how["head_decay"]}
             else:
-                ops.gla_prep(proj, off[0], off[1], 0, torch.zeros(QK, 1, device=DEV, dtype=dtype), bias, q32, k32, decay, 0.25, 16.0, z=z)
-                how, a = {"q_scale": 0.25, "z": z, "z_bias": bias, "tau": 16.0, "norm_weight": w}, {"decay": decay}
+                ops.gla_prep(proj, off[0], off[1], low, a2, bias, q32, k32, decay, 0.25, 16.0)
+                how, a = {"q_scale": 0.25, "a2": a2, "low_off": low, "z_bias": bias, "tau": 16.0, "norm_weight": w}, {"decay": decay}
             states, o = [before.clone(), before.clone()], torch.empty(n, V, device=DEV)
             outs = [torch.full((n, V), float("nan"), device=DEV, dtype=dtype) for _ in range(2)]
             ops.linear_scan(q32, k32, proj[:, off[2]:off[2] + V], o, states[0], ctx, H, dk, dv, **a)
