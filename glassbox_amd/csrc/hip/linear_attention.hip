@@ -125,6 +125,68 @@ __device__ __forceinline__ float log_sigmoid(float z) {
   return (z >= 0.f ? 0.f : z) - log1pf(expf(-fabsf(z)));
 }
 
+// Four values from p on; WORDS: they lie at a word of four.
+template <bool WORDS, typename T>
+__device__ __forceinline__ f32x4 four_of(const T* p) {
+  typedef T quad __attribute__((ext_vector_type(4)));
+  if constexpr (WORDS) {
+    const quad q = *reinterpret_cast<const quad*>(p);
+    return f32x4{to_f(q[0]), to_f(q[1]), to_f(q[2]), to_f(q[3])};
+  } else {
+    return f32x4{to_f(p[0]), to_f(p[1]), to_f(p[2]), to_f(p[3])};
+  }
+}
+
+// A decay's sum over its middle.  32-bit: as every 32-bit product sums a cell, slices of 64 one after the other, a chain of fused
+// multiply-adds each, so that a token's decay has the same bits from here and from a product.  bfloat16: eight chains, whose
+// error against 64 bits is that of the matrix cores' sums or below (a middle of 64: 4.0e-8 of the result, the product 4.2e-8, one
+// chain 5.1e-8; of 128 4.8e-8, 5.0e-8 and 7.3e-8).
+template <bool WORDS, typename T, typename L>
+__device__ __forceinline__ float middle_sum(const T* __restrict__ w, const L* __restrict__ low, int rank) {
+  if constexpr (std::is_same<T, float>::value) {
+    float z = 0.f, s = 0.f;
+    int r = 0;
+#pragma unroll 4
+    for (; r + 4 <= rank; r += 4) {
+      if (r % 64 == 0) {
+        z += s;
+        s = 0.f;
+      }
+      const f32x4 a = four_of<WORDS>(w + r), b = four_of<WORDS>(low + r);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) s = fmaf(a[m], b[m], s);
+    }
+    if constexpr (!WORDS) {
+      if (r % 64 == 0) {
+        z += s;
+        s = 0.f;
+      }
+      for (; r < rank; ++r) s = fmaf(w[r], low[r], s);
+    }
+    z += s;
+    return z;
+  } else {
+    float c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    int r = 0;
+#pragma unroll 2
+    for (; r + 8 <= rank; r += 8) {
+      const f32x4 a0 = four_of<WORDS>(w + r), b0 = four_of<WORDS>(low + r);
+      const f32x4 a1 = four_of<WORDS>(w + r + 4), b1 = four_of<WORDS>(low + r + 4);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        c[m] = fmaf(a0[m], b0[m], c[m]);
+        c[4 + m] = fmaf(a1[m], b1[m], c[4 + m]);
+      }
+    }
+    if (r < rank) {
+#pragma unroll
+      for (int m = 0; m < 7; ++m)
+        if (r + m < rank) c[m] = fmaf(to_f(w[r + m]), to_f(low[r + m]), c[m]);
+    }
+    return ((c[0] + c[4]) + (c[2] + c[6])) + ((c[1] + c[5]) + (c[3] + c[7]));
+  }
+}
+
 // C columns a lane, 32 C a workgroup.  A token costs a lane 3 R C multiply-adds and the reads of its R rows of q, k and the decay
 // from LDS; both pipes are near full.  Everything else stays off them: the lanes of a column share the writes of its sums, one wave a
 // head keeps the product of the decays, and the state comes by words.  us, before / so: 2 single tokens, 32 heads of 64 by 64
@@ -132,9 +194,11 @@ __device__ __forceinline__ float log_sigmoid(float z) {
 // it the end states of segments, by words); 2,048 rows, 32 heads of 64 by 65 186 / 115, 16 of 128 by 128 273 / 142.  The bits are the same.
 // FUSED: the projection's rows in, the normed and gated rows out (a workgroup then has all of its head's columns, 64 at most): what
 // the preparing kernels and head_norm_gate do, by the same arithmetic, with no rows between them through memory.  A step of two
-// tokens, 32 heads of 64: a decay a head 14.2 us in three launches, 6.1 in this one; a decay a key channel 20.7 in four, 7.4.
+// tokens, 32 heads of 64: a decay a head 14.2 us in three launches, 6.1 in this one; a decay a key channel 20.7 in four, 7.4 with
+// the sums over its middle still a product of their own and 5.8 without.  (FUSED in 32-bit takes 129 registers where it may: a
+// wave a SIMD fewer.)
 template <typename T, int R, bool GATED, int C, bool FUSED>
-__global__ __launch_bounds__(kThreads) void scan_kernel(
+__global__ __launch_bounds__(kThreads, FUSED ? 4 : 1) void scan_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ a, const float* __restrict__ head_decay,
     const T* __restrict__ v, int v_stride, float* __restrict__ out, float* __restrict__ state,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ pos0,
@@ -186,15 +250,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(
         const T* kr = hd.proj + t * hd.stride + hd.k_off + h * dk;
         float xq = to_f(qr[ch]), xk = to_f(kr[ch]);
         if (GATED) {
-          const T* w = hd.a2 + (size_t)(h * dk + ch) * hd.rank;
-          const T* low = hd.proj + t * hd.stride + hd.low_off;
-          float z = 0.f;
-#pragma unroll 4
-          for (int r = 0; r < hd.rank; r += 4) {
-            const quad w4 = *reinterpret_cast<const quad*>(w + r), l4 = *reinterpret_cast<const quad*>(low + r);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) z = fmaf(to_f(w4[m]), to_f(l4[m]), z);
-          }
+          float z = middle_sum<true>(hd.a2 + (size_t)(h * dk + ch) * hd.rank, hd.proj + t * hd.stride + hd.low_off, hd.rank);
           z += hd.z_bias ? hd.z_bias[h * dk + ch] : 0.f;
           na[e] = expf(log_sigmoid(z) * hd.inv_tau);
         } else if (ch < hd.rot) {
@@ -577,8 +633,7 @@ __global__ void gla_prep_kernel(const T* __restrict__ proj, int stride, int q_of
     if (zin) {
       z = zin[(size_t)t * width + c];
     } else {
-      const T* w = a2 + (size_t)c * rank;
-      for (int r = 0; r < rank; ++r) z = fmaf(to_f(w[r]), low[r], z);
+      z = middle_sum<false>(a2 + (size_t)c * rank, low, rank);
     }
     z += a2_bias ? a2_bias[c] : 0.f;
     decay[(size_t)t * width + c] = expf(log_sigmoid(z) * inv_tau);

@@ -157,6 +157,30 @@ def test_decays_of_key_channels_and_the_gated_head_norm():
             assert (out.cpu().to(F64) - want).abs().max() < 1e-5, (T, H, dv)
 
 
+@pytest.mark.parametrize("rank", [96, 127, 128])
+def test_a_decays_sum_in_bfloat16_is_no_one_long_chain(rank):
+    """The sum over a decay's middle inside the kernels: eight chains, whose error against 64 bits is two thirds of one chain's for
+    these sizes (4.8e-8 of the result and 7.1e-8 at 128), as a product's is."""
+    from glassbox_amd import ops
+    torch.manual_seed(rank)
+    n, W = 16, 1024
+    low, a2 = (torch.randn(n, rank) * 4).bfloat16(), torch.randn(W, rank).bfloat16()
+    terms = low.to(F64)[:, None] * a2.to(F64)[None]
+    want = terms.sum(-1)
+    chain = torch.zeros(n, W)
+    for r in range(rank):
+        chain = (chain.to(F64) + terms[..., r]).float()
+    proj = torch.zeros(n, 2 * W + rank, dtype=torch.bfloat16)
+    proj[:, 2 * W:] = low
+    q, k, decay = (torch.empty(n, W, device=DEV) for _ in range(3))
+    ops.gla_prep(proj.to(DEV), 0, W, 2 * W, a2.to(DEV), None, q, k, decay, 1.0, 1.0)
+    far = (want < -20) & (want > -80)                          # there the decay is exp(z), its relative error that of z itself
+    assert far.sum() > 2000
+    rms = lambda e: e[far].pow(2).mean().sqrt().item()
+    got, one = rms(decay.cpu().to(F64) / want.exp() - 1), rms(chain.to(F64) - want)
+    assert got < 0.85 * one, (got, one)
+
+
 def _step(lens, pos0):
     starts = np.cumsum([0] + list(lens))[:-1]
     return SimpleNamespace(q_start=_i32(starts), q_len=_i32(lens), pos0=_i32(pos0), state_slots=_i32(range(len(lens))), num_seqs=len(lens))
@@ -510,6 +534,25 @@ def test_in_32_bit_the_cutting_changes_no_bit_of_the_recurrent_layers(model_dirs
     whole = helpers.replay(eng, helpers.schedule_whole(requests))
     for steps in (helpers.schedule_chunks(requests), helpers.schedule_tail(requests, 40),
                   helpers.schedule_mixed(requests, seed=1, live=2, tail=10)[0]):
+        got = helpers.replay(eng, steps)
+        assert all(np.array_equal(got[r], whole[r]) for r in requests)
+
+
+@pytest.mark.parametrize("rank", [64, 68, 96, 128])
+def test_in_32_bit_the_cutting_changes_no_bit_of_the_gated_layers(model_dirs, rank):
+    """Decays with a middle of one and of two slices of 64: a token's decay has the same bits whether it comes in a long portion
+    (a product of its own) or in a short one (summed beside the recurrence)."""
+    from glassbox_amd.config import config_from_dict
+    from glassbox_amd.engine import Engine
+    from glassbox_amd.weights import write_random_model
+    gla = dict(CASES["Q"]["layers"][0])
+    gla["mixer"] = dict(gla["mixer"], rank=rank)
+    folder = write_random_model(config_from_dict(dict(CASES["Q"], layers=[gla])), os.path.join(model_dirs.base, f"sagalorn_gated_{rank}"), 4,
+                                std=0.1, norm_init="uniform")
+    requests = {"a": helpers.random_tokens(130, 90, seed=1), "b": helpers.random_tokens(130, 33, seed=2)}
+    eng = Engine(folder, dtype="float32", max_tokens=256, max_seqs=2)
+    whole = helpers.replay(eng, helpers.schedule_whole(requests))
+    for steps in (helpers.schedule_chunks(requests), helpers.schedule_chunks(requests, (8, 1, 30)), helpers.schedule_tail(requests, 40)):
         got = helpers.replay(eng, steps)
         assert all(np.array_equal(got[r], whole[r]) for r in requests)
 
