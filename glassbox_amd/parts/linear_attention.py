@@ -81,7 +81,7 @@ class _LinearMixer(Mixer):
     def _at_once(self, ctx, proj, residual, cache, store, norm_weight, **kind) -> bool:
         """All of a step of few tokens a request in one launch, where there is one for it, and the output projection."""
         g_off = 2 * self.qk_dim + self.v_dim
-        if (cache is None or cache.state is None
+        if (not ctx.tuned or cache is None or cache.state is None
                 or not ops.linear_heads_takes(proj, int(ctx.host["max_q_len"]), self.key_dim, self.value_dim, g_off, kind.get("a2"),
                                               kind.get("low_off", 0))):
             return False

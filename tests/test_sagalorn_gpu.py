@@ -557,6 +557,30 @@ def test_in_32_bit_the_cutting_changes_no_bit_of_the_gated_layers(model_dirs, ra
         assert all(np.array_equal(got[r], whole[r]) for r in requests)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_the_engine_of_plain_kernels_fuses_nothing_of_the_recurrent_layers(model_dirs, dtype, monkeypatch):
+    """What the tuned kernels are compared with: one kernel an operation, in steps of every length."""
+    from glassbox_amd import ops
+    from glassbox_amd.engine import Engine
+    folder = folder_of(model_dirs.base, "Q")
+    calls = []
+    for name in ("linear_heads", "linear_scan", "retention_prep", "gla_prep", "head_norm_gate"):
+        def counted(*args, _name=name, _call=getattr(ops, name), **kwargs):
+            calls.append(_name)
+            return _call(*args, **kwargs)
+        monkeypatch.setattr(ops, name, counted)
+    requests = {"a": helpers.random_tokens(130, 30, seed=1)}
+    got = {}
+    for kernels in ("plain", "auto"):
+        calls.clear()
+        eng = Engine(folder, dtype=dtype, max_tokens=64, max_seqs=1, graph_decode=False, layer_tapes=False, kernels=kernels)
+        got[kernels] = helpers.replay(eng, helpers.schedule_chunks(requests, (20, 1, 5, 4)))["a"]
+        assert calls.count("linear_heads") == (0 if kernels == "plain" else 2 * 3)        # two layers; the steps of 1, 5 and 4 rows
+        assert all(calls.count(n) == m * (4 if kernels == "plain" else 1) for n, m in (("linear_scan", 2), ("head_norm_gate", 2),
+                                                                                       ("retention_prep", 1), ("gla_prep", 1)))
+    _check({"a": got["plain"]}, folder, requests, dtype, "plain kernels")
+
+
 # ------------------------------------------------------------------------------------------ generation
 @pytest.mark.parametrize("name", ["P", "Q"])
 def test_greedy_generation_through_the_entry_points(model_dirs, name):
