@@ -422,7 +422,10 @@ __device__ __forceinline__ bool sample_few(Row& r, u64 best_key, int k, float mp
   });
   __syncthreads();
   const int n = (int)min(found[16], (unsigned int)(TPB + 1));
-  if (n > TPB) return false;
+  if (n > TPB) {
+    __syncthreads();   // select() clears the counts, which all threads have to have read
+    return false;
+  }
   if (tid < n) {
     const u64 key = keys[tid];
     int rank = 0;

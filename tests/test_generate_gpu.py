@@ -186,6 +186,26 @@ def test_sampling_kernel_where_few_candidates_are_sorted(vocab, ties):
         check_sampled(logits[r].tolist(), [], c, us[r], toks[r], cands[r])
 
 
+@pytest.mark.parametrize("vocab", [1025, 2048, 5000])
+def test_sampling_kernel_on_many_rows_with_more_ties_than_are_sorted(vocab):
+    """Rows of few values, more than 1,024 tokens of them at or above the k-th: no thread may go on to the searches before all
+    have seen how many there are.  Every row against the reference, and a second time."""
+    from glassbox_amd.sampling import SamplerConfig, sample_rows
+    rng = random.Random(vocab)
+    g = torch.Generator().manual_seed(vocab)
+    n = 96
+    logits = torch.zeros(n, vocab)
+    logits[1::3] = torch.randint(0, 2, (n // 3, vocab), generator=g) * 0.001      # apart below the bound's 16 bits
+    logits[2::3, :12] += torch.randn(n // 3, 12, generator=g).abs()
+    cfgs = [SamplerConfig(temperature=1.0, top_k=rng.choice([13, 40, 300, 512]), top_p=rng.choice([1.0, 0.9]), min_p=rng.choice([0.0, 0.05]))
+            for _ in range(n)]
+    us = [rng.random() for _ in cfgs]
+    first = sample_rows(logits.clone().to(DEV), cfgs, us, [[]] * n)
+    assert list(map(list, first)) == list(map(list, sample_rows(logits.clone().to(DEV), cfgs, us, [[]] * n)))
+    for r, c in enumerate(cfgs):
+        check_sampled(logits[r].tolist(), [], c, us[r], first[0][r], first[1][r])
+
+
 def test_temperature_draws_follow_the_softmax():
     from glassbox_amd.sampling import Rng, SamplerConfig, sample_rows
     logits = torch.tensor([[0.0, math.log(2.0), math.log(5.0), -30.0]], device=DEV).repeat(64, 1)
