@@ -206,6 +206,28 @@ def test_sampling_kernel_on_many_rows_with_more_ties_than_are_sorted(vocab):
         check_sampled(logits[r].tolist(), [], c, us[r], first[0][r], first[1][r])
 
 
+@pytest.mark.parametrize("vocab", [1024, 1025, 4099, 16384])
+@pytest.mark.parametrize("mask", [-math.inf, -3.3e38, -1e4])
+def test_sampling_kernel_behind_masks_that_leave_few_tokens(vocab, mask):
+    """One token fewer than top-k left, as many, one more, a thousand: which way a row takes depends on that."""
+    from glassbox_amd.sampling import SamplerConfig, sample_rows
+    rng = random.Random(vocab)
+    g = torch.Generator().manual_seed(vocab)
+    cfgs, rows = [], []
+    for k in (1, 2, 40, 256, 257, 511):
+        for left in (k - 1, k, k + 1, 1000):
+            row = torch.full((vocab,), mask)
+            keep = torch.randperm(vocab, generator=g)[:left]
+            row[keep] = torch.randn(left, generator=g) * 2
+            rows.append(row)
+            cfgs.append(SamplerConfig(temperature=1.0, top_k=k, top_p=rng.choice([1.0, 0.9]), min_p=rng.choice([0.0, 0.02])))
+    us = [rng.random() for _ in cfgs]
+    toks, cands = sample_rows(torch.stack(rows).to(DEV), cfgs, us, [[]] * len(cfgs))
+    for r, c in enumerate(cfgs):
+        if bool((rows[r] > mask).any()) or mask > -math.inf:      # (a row without any token left has no answer)
+            check_sampled(rows[r].tolist(), [], c, us[r], toks[r], cands[r])
+
+
 def test_temperature_draws_follow_the_softmax():
     from glassbox_amd.sampling import Rng, SamplerConfig, sample_rows
     logits = torch.tensor([[0.0, math.log(2.0), math.log(5.0), -30.0]], device=DEV).repeat(64, 1)
