@@ -32,38 +32,45 @@ __device__ __forceinline__ uint64_t composite(float v, int idx) {
 // ---------------------------------------------------------------------------- argmax
 // first maximum wins (sampler.rs:49-57) = the largest composite key
 constexpr int ARGMAX_TPB = 1024;
+template <bool WORDS>
 __global__ __launch_bounds__(ARGMAX_TPB) void argmax_kernel(const float* __restrict__ logits, int32_t* __restrict__ out, int V) {
   __shared__ uint64_t best[ARGMAX_TPB / kWave];
   const float* row = logits + (size_t)blockIdx.x * V;
   uint64_t b = 0;
-  // What bounds it is round trips to memory (a workgroup is alone with its row): four loads of four tokens on their way a thread
-  // where rows begin at 16 bytes (128,256 tokens: 18.7 us with four loads of one, 14.9 now; 49,152: 9.7, 8.6), else of one token.
+  // What bounds it is round trips to memory while a workgroup has its compute unit for itself: four loads of four tokens on their way
+  // a thread, from the row's first word of 16 bytes on (us, four loads of one token / so: 128,256 tokens 16.8 / 13.1, 128 rows of them
+  // 21.9 / 15.5; 50,257, an odd number, 8.3 / 7.0).  Beyond a row a unit (WORDS false) a unit's two rows fill what it can have on its
+  // way, and one token a load it stays (300 rows of 49,152: 13.8 / 14.8; 512: 17.6 / 17.4).
   auto take = [&](float v, int i) {
     const uint64_t c = composite(v, i);
     b = c > b ? c : b;
   };
-  const int words = ((uintptr_t)row & 15) == 0 ? V / 4 : 0;
+  const int lead = WORDS ? min((int)(-((uintptr_t)row / 4) & 3), V) : 0, words = WORDS ? (V - lead) / 4 : 0;
+  const float* at = row + lead;
+  if (WORDS && (int)threadIdx.x < lead) take(row[threadIdx.x], threadIdx.x);
 #pragma unroll 1
   for (int w0 = threadIdx.x; w0 < words; w0 += 4 * ARGMAX_TPB) {
     f32x4 v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (w0 + j * ARGMAX_TPB < words) v[j] = *reinterpret_cast<const f32x4*>(row + 4 * (size_t)(w0 + j * ARGMAX_TPB));
+      if (w0 + j * ARGMAX_TPB < words) v[j] = *reinterpret_cast<const f32x4*>(at + 4 * (size_t)(w0 + j * ARGMAX_TPB));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (w0 + j * ARGMAX_TPB < words) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) take(v[j][e], 4 * (w0 + j * ARGMAX_TPB) + e);
+        for (int e = 0; e < 4; ++e) take(v[j][e], lead + 4 * (w0 + j * ARGMAX_TPB) + e);
       }
   }
-#pragma unroll 1
-  for (int i0 = 4 * words + threadIdx.x; i0 < V; i0 += 4 * ARGMAX_TPB) {
+  for (int i0 = lead + 4 * words + threadIdx.x; i0 < V; i0 += 4 * ARGMAX_TPB) {
     float v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = i0 + j * ARGMAX_TPB < V ? row[i0 + j * ARGMAX_TPB] : 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (i0 + j * ARGMAX_TPB < V) take(v[j], i0 + j * ARGMAX_TPB);
+    for (int j = 0; j < 4; ++j) {
+      const int i = i0 + j * ARGMAX_TPB;
+      const uint64_t c = i < V ? composite(v[j], i) : 0;
+      b = c > b ? c : b;
+    }
   }
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) {
@@ -591,7 +598,7 @@ __global__ __launch_bounds__(TPB) void sample_kernel(float* __restrict__ logits,
 extern "C" int gb_argmax(const float* logits, int32_t* out, int rows, int V, hipStream_t stream) {
   GB_REQUIRE(rows >= 0 && V > 0 && V <= (1 << IDX_BITS), "argmax: vocabulary %d is outside 1..%d", V, 1 << IDX_BITS);
   if (rows == 0) return 0;
-  hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(ARGMAX_TPB), 0, stream, logits, out, V);
+  hipLaunchKernelGGL(rows <= 256 ? argmax_kernel<true> : argmax_kernel<false>, dim3(rows), dim3(ARGMAX_TPB), 0, stream, logits, out, V);
   return launched("argmax");
 }
 

@@ -162,6 +162,25 @@ def test_sampling_kernel_on_rows_of_ties_and_edge_settings():
     assert checked == 192
 
 
+@pytest.mark.parametrize("rows", [7, 256, 257])
+@pytest.mark.parametrize("vocab", [1, 2, 3, 6, 4097, 16387, 20006])
+def test_argmax_of_rows_that_begin_anywhere(rows, vocab):
+    """Rows that begin at every place in a word of 16 bytes, from one token on; the maximum at either end and in the words between,
+    the first of two."""
+    from glassbox_amd import ops
+    g = torch.Generator().manual_seed(vocab)
+    for shift in range(4):
+        flat = torch.randn(rows * vocab + 4, generator=g)
+        logits = flat[shift:shift + rows * vocab].view(rows, vocab)
+        for r, at in enumerate((0, vocab - 1, vocab // 2, max(0, vocab - 2), min(1, vocab - 1), min(3, vocab - 1), max(0, vocab - 4))):
+            logits[r, at] = 9.0
+            logits[r, vocab - 1] = 9.0
+        out = torch.empty(rows, dtype=torch.int32, device=DEV)
+        ops.argmax(flat.to(DEV)[shift:shift + rows * vocab].view(rows, vocab), out)
+        first = (logits == logits.max(dim=1, keepdim=True).values).int().argmax(dim=1)
+        assert out.tolist() == first.tolist()
+
+
 @pytest.mark.parametrize("vocab", [1023, 1024, 1027, 4099, 49152])
 @pytest.mark.parametrize("ties", [False, True])
 def test_sampling_kernel_where_few_candidates_are_sorted(vocab, ties):
