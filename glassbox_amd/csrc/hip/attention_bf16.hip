@@ -1172,6 +1172,7 @@ __global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
     slot ^= 1;
   }
   if constexpr (S > 1) {
+    wait_copies<0>();   // (a part without a tile has copied one all the same, to where sums are handed over)
     __syncthreads();
     float* handed = reinterpret_cast<float*>(ring) + wave * ((S / 2) * DB * 16 * 64);
     float* handed_ml = reinterpret_cast<float*>(ring) + R * ((S / 2) * DB * 16 * 64) + wave * ((S / 2) * 128);

@@ -1634,6 +1634,29 @@ def test_tuned_prefill_of_every_shape(shape, nh, nkv, hd, q_lens, history, windo
     assert bool((wide[:, nh * hd:] == 7.0).all())
 
 
+@pytest.mark.parametrize("shape,nh,nkv,hd,q_lens,history", [
+    (228, 4, 2, 64, [3, 40], [0, 2700]), (227, 4, 2, 64, [40, 2, 33], [2300, 0, 70]), (226, 6, 3, 64, [17, 64], [1, 2100]),
+    (228, 4, 1, 128, [3, 40], [0, 4200]), (225, 4, 4, 128, [60, 2], [2700, 130])])
+@pytest.mark.parametrize("page", [16, 64])
+def test_tuned_prefill_of_short_requests_beside_long_ones(shape, nh, nkv, hd, q_lens, history, page):
+    """Requests with fewer tiles of keys than the workgroups that the longest one's are spread over: some of theirs have no tile,
+    and hand over nothing."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    ctx_lens = [h + n for h, n in zip(history, q_lens)]
+    assert ops._lib("attention_bf16").gb_attention_prefill_shape(max(q_lens), max(ctx_lens), nh, len(q_lens), hd) == shape
+    k_pages, v_pages, tables, _, _ = paged_setup(ctx_lens, nkv, hd, page, seed=hd + nh, dtype=torch.bfloat16)
+    ctx = BareContext(q_lens, ctx_lens, tables)
+    q = to_dev((rnd(sum(q_lens), nh * hd, seed=14) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out, twin = torch.zeros_like(q), torch.zeros_like(q)
+    ops.attention_prefill(q, out, ctx, cache, nh, 1 / math.sqrt(hd), 0)
+    ops.attention_plain(q, twin, ctx.positions, torch.tensor(ctx.tok_seq, dtype=torch.int32, device=DEV), ctx.tables[0],
+                        cache.k_pages, cache.v_pages, nh, 1 / math.sqrt(hd), 0)
+    # softmax weights in bfloat16 (2^-9 of each value's share) and a bfloat16 result on either side
+    assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
+
+
 @pytest.mark.parametrize("nh,ctxlen,qlen", [(2, 200, 90), (64, 1200, 1090)])   # 32 and 64 tokens a wave
 def test_tuned_prefill_sees_exactly_the_causal_keys(nh, ctxlen, qlen):
     """A portion in the middle of a request (it starts at position 110): token t must find a marked
