@@ -800,11 +800,12 @@ __global__ __launch_bounds__(64 * PAIRS * SPLIT, 2) void prefill_kernel(const bf
     // the tiles of 64 keys in order: both blocks as far as the earlier one's keys reach (with a window the later
     // one may see none of them yet: they are masked), then, with a window after a gap, the later block alone
     // with kept first keys: their tiles of 64 first (as far as they lie before the window's first tile), both blocks live
-    const int win0 = range[0].first & ~63, kept_end = min((keep + 63) & ~63, win0);
+    // (the later block sees all of them, also those behind the earlier block's last token)
+    const int win0 = range[0].first & ~63, kept_tiles = (keep + 63) & ~63, kept_end = min(kept_tiles, win0);
     auto after = [&](int kb) {
       int next = kb + 64;
       if (kb < kept_end && next >= kept_end) next = win0;
-      if (has_second && kb <= range[0].last && next > range[0].last && next + 63 < range[1].first) next = range[1].first & ~63;
+      if (has_second && next >= kept_tiles && next > range[0].last && next + 63 < range[1].first) next = range[1].first & ~63;
       return next;
     };
     auto my_next = [&](int kb) {  // the waves of a pair (in all the workgroups that share it) take the tiles in turn
@@ -820,7 +821,6 @@ __global__ __launch_bounds__(64 * PAIRS * SPLIT, 2) void prefill_kernel(const bf
       // the tiles in order: the kept first keys (both blocks); the earlier block's tiles that lie before everything
       // the later block sees (its window, or its run of positions, begins behind them: the earlier block alone); the
       // tiles both see; then the later block alone
-      const int kept_tiles = (keep + 63) & ~63;
       while (kb <= range[0].last && kb < kept_tiles) {
         const int next = my_next(kb);
         attend64_q32<HD, 2, 3, 2, WIDE, MODE>(m, l, acc, q_lds, q_at, kf, vf, src, kb, next, lo, hi, true, c, lane, keep, cap_in, cap_out, at);

@@ -1634,6 +1634,31 @@ def test_tuned_prefill_of_every_shape(shape, nh, nkv, hd, q_lens, history, windo
     assert bool((wide[:, nh * hd:] == 7.0).all())
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 2, 16), (6, 2, 32), (2, 1, 48), (6, 3, 64), (4, 4, 80), (3, 1, 96), (2, 2, 112), (4, 2, 128)])
+@pytest.mark.parametrize("window,keep,q_lens,history", [(44, 200, [572, 14], 0), (44, 200, [85, 300], 53), (20, 97, [400], 0), (100, 65, [33, 700], 0),
+                                                        (16, 130, [333], 7), (300, 500, [900], 0), (44, 200, [300], 1605)])
+@pytest.mark.parametrize("softcap,wide", [(0.0, False), (20.0, False), (0.0, True)])
+def test_tuned_prefill_with_more_kept_first_keys_than_a_tile_holds(nh, nkv, hd, window, keep, q_lens, history, softcap, wide):
+    """A prompt's first tokens see few of the kept keys, its last ones all of them, beside a window that begins far behind: every
+    kernel and way of sharing the keys, against the plain kernel."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    ctx_lens = [history + n for n in q_lens]
+    k_pages, v_pages, tables, _, _ = paged_setup(ctx_lens, nkv, hd, 16, seed=hd + nh, dtype=torch.bfloat16)
+    ctx = BareContext(q_lens, ctx_lens, tables)
+    q = to_dev((rnd(sum(q_lens), nh * hd, seed=14) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    out, twin = (torch.zeros(q.shape, device=DEV, dtype=torch.float32 if wide else torch.bfloat16) for _ in range(2))
+    twin = torch.zeros_like(q)
+    ops.attention_prefill(q, out, ctx, cache, nh, 1 / math.sqrt(hd), window, keep, softcap=softcap)
+    ops.attention_plain(q, twin, ctx.positions, torch.tensor(ctx.tok_seq, dtype=torch.int32, device=DEV), ctx.tables[0],
+                        cache.k_pages, cache.v_pages, nh, 1 / math.sqrt(hd), window, keep_first=keep, softcap=softcap)
+    # softmax weights in bfloat16 (2^-9 of each value's share) and a bfloat16 result on either side
+    close = (out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())
+    bad = torch.nonzero(~close.all(dim=1)).flatten().tolist()
+    assert not bad, f"{len(bad)} rows, {bad[:8]} (request, position) {[(ctx.tok_seq[i], ctx.pos_list[i]) for i in bad[:8]]}"
+
+
 @pytest.mark.parametrize("shape,nh,nkv,hd,q_lens,history", [
     (228, 4, 2, 64, [3, 40], [0, 2700]), (227, 4, 2, 64, [40, 2, 33], [2300, 0, 70]), (226, 6, 3, 64, [17, 64], [1, 2100]),
     (228, 4, 1, 128, [3, 40], [0, 4200]), (225, 4, 4, 128, [60, 2], [2700, 130])])
