@@ -38,7 +38,8 @@ inline RingRows ring_rows(int M, int columns, int K) {
     return (float)((K + RBK - 1) / RBK) * 0.0806f * ((float)h + 1.5f) * (1.f + 1.09f * (float)n / 256.f) + 6.f;
   };
   RingRows best{};
-  for (int tiles = (rows + 7) / 8, last = tiles + 24; tiles <= last; ++tiles) {
+  const int least = (rows + 7) / 8;   // (that many in any case; more only while they fit a grid's second dimension)
+  for (int tiles = least; tiles <= least + 24 && (tiles == least || tiles <= 65535); ++tiles) {
     const int height = (rows + tiles - 1) / tiles, tall = rows - tiles * (height - 1);
     if (height < 5 && best.tiles) break;
     const long long all = (long long)tiles * columns, whole = all / 256, high = ((long long)tall * columns + 255) / 256;

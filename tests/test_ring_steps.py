@@ -69,6 +69,17 @@ def test_tiles_hold_every_row_once(ring, columns):
             assert ring.rows(M, columns, 4096, 0) == 8 and ring.rows(M, columns, 4096, 2) == M // 256
 
 
+@pytest.mark.parametrize("columns", [1, 3, 7, 24, 112])
+def test_the_most_rows_that_a_grid_holds_stay_within_it(ring, columns):
+    """A grid's second dimension ends at 65,535: as many tiles of 256 rows are taken, and tiles of fewer rows only as long as they fit."""
+    for tiles in list(range(65500, 65536)):
+        for M in (256 * tiles, 256 * tiles - 95):
+            for K in (128, 2048):
+                height, tall, dealt = (ring.rows(M, columns, K, i) for i in range(3))
+                assert dealt <= 65535, (M, K)
+                assert tall * height + (dealt - tall) * (height - 1) == -(-M // 32), (M, K)
+
+
 @pytest.mark.parametrize("M,columns,K,heights", [
     (6151, 16, 14336, (7, 13, 30)), (6151, 24, 4096, (7, 7, 31)), (2048, 24, 2048, (7, 4, 10)), (5487, 16, 4096, (6, 12, 32)), (2048, 64, 2048, (8, 8, 8))])
 def test_tiles_where_256_rows_leave_units_idle(ring, M, columns, K, heights):
