@@ -1051,7 +1051,7 @@ __device__ __forceinline__ int small_quotient(int a, int b) {
 }
 
 // grid (kv heads, requests from seq_base on, tiles x parts from tiles_from - 1 down), R x S waves a workgroup: R blocks side by side, S waves a
-// block that take the tiles of keys in turn; JOBS = 8 / R, rounded up.
+// block that take the tiles of keys in turn; R x JOBS = 8.
 template <int HD, int JOBS, int S>
 __global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
     const bf16* __restrict__ q, int q_stride, bf16* __restrict__ out, int out_stride, const int32_t* __restrict__ q_start,
@@ -1094,16 +1094,13 @@ __global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
 
   const int tok = 32 * block + col;
   const bool valid = works && tok < qlen;
-  // A tile is eight copies of 16 keys' or values' worth, JOBS a wave (the last ones twice where the waves do not divide them).
+  // A tile is eight copies of 16 keys' or values' worth, JOBS a wave.
   // This lane's place in a page: of the keys piece lane / 16 (of four), slot by the order of a score tile's rows (load_keys);
   // of the values dimension lane % 32, keys 8 (lane / 32) on.
   const int r16 = lane & 15, key16 = ((r16 >> 2) & 1) * 8 + (r16 >> 3) * 4 + (r16 & 3);
   const uint32_t k_off = (((uint32_t)(lane >> 4) << page_shift) + key16) * 16, v_off = ((uint32_t)col << page_shift) * 2 + 16 * g;
   const uint32_t ring_at = (uint32_t)(uintptr_t)(lds_void*)ring + half * TILE;
-  auto group_of = [&](int j) {   // the job's group of 16 keys, + 4 for values
-    const int job = wave + j * R;
-    return job < 8 ? job : wave;
-  };
+  auto group_of = [&](int j) { return wave + j * R; };   // the job's group of 16 keys, + 4 for values
   const int i_end = max(i0, i1 - 1);
   // of tile i (the last one in place of those beyond it) and a job's group of 16 keys: the key that says which page it is
   auto key_at = [&](int i, int j) {
@@ -1447,27 +1444,29 @@ extern "C" int gb_attention_prefill_shape(int max_q_len, int max_context, int nh
 }
 
 template <int HD>
-static void prefill_shared_launch(const bf16* q, int q_stride, bf16* out, int out_stride, const int32_t* q_start, const int32_t* q_len,
-                                  const int32_t* pos0, int seq_base, int n_seqs, int max_q_len, const int32_t* tables,
-                                  int table_stride, const bf16* kp, const bf16* vp, int nh, int nkv, int page_shift, float scale,
-                                  int window, int keep, float* part_acc, float* part_ml, const SharedPlan& plan, int first_row,
-                                  int n_rows, const Extra& ex, hipStream_t stream) {
+static int prefill_shared_launch(const bf16* q, int q_stride, bf16* out, int out_stride, const int32_t* q_start, const int32_t* q_len,
+                                 const int32_t* pos0, int seq_base, int n_seqs, int max_q_len, const int32_t* tables,
+                                 int table_stride, const bf16* kp, const bf16* vp, int nh, int nkv, int page_shift, float scale,
+                                 int window, int keep, float* part_acc, float* part_ml, const SharedPlan& plan, int first_row,
+                                 int n_rows, const Extra& ex, hipStream_t stream) {
   const int units = (max_q_len + 31) / 32 * (nh / nkv), tiles = (units + plan.rows - 1) / plan.rows;
   // (a grid's third dimension ends at 65,535: longer ones in several launches, the most work first)
   for (int from = tiles * plan.parts; from > 0; from -= 65535) {
 #define GB_LAUNCH(JOBS, S)                                                                                                      \
-  hipLaunchKernelGGL((prefill_shared_kernel<HD, JOBS, S>), dim3(nkv, n_seqs, min(from, 65535)), dim3(64 * plan.rows * S), 0,    \
-                     stream, q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, tables, table_stride, kp, vp, nh,    \
-                     nkv, page_shift, scale, window, keep, part_acc, part_ml, plan.parts, from, first_row, n_rows, ex)
-    if (plan.rows == 4 && plan.split == 1) GB_LAUNCH(2, 1);
-    if (plan.rows == 4 && plan.split == 2) GB_LAUNCH(2, 2);
-    if (plan.rows == 2 && plan.split == 1) GB_LAUNCH(4, 1);
-    if (plan.rows == 2 && plan.split == 2) GB_LAUNCH(4, 2);
+  if (plan.rows * (JOBS) == 8 && plan.split == (S)) {                                                                           \
+    hipLaunchKernelGGL((prefill_shared_kernel<HD, JOBS, S>), dim3(nkv, n_seqs, min(from, 65535)), dim3(64 * plan.rows * (S)),   \
+                       0, stream, q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, tables, table_stride, kp, vp,   \
+                       nh, nkv, page_shift, scale, window, keep, part_acc, part_ml, plan.parts, from, first_row, n_rows, ex);   \
+    continue;                                                                                                                   \
+  }
+    GB_LAUNCH(2, 1) GB_LAUNCH(2, 2) GB_LAUNCH(4, 1) GB_LAUNCH(4, 2)
     if constexpr (HD <= 64) {
-      if (plan.rows == 2 && plan.split == 4) GB_LAUNCH(4, 4);
+      GB_LAUNCH(4, 4)
     }
 #undef GB_LAUNCH
+    return fail("attention_prefill: no kernel for %d blocks of %d waves a workgroup", plan.rows, plan.split);
   }
+  return launched("attention_prefill");
 }
 
 // Workgroups that would share a pair's keys with these sizes (1: none do); the caller then provides
@@ -1555,9 +1554,10 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
   if (shared) {
     if constexpr (kCanCap) {
       const auto run = hd == 64 ? prefill_shared_launch<64> : prefill_shared_launch<128>;
-      run((const bf16*)q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, n_seqs, max_q_len, tables, table_stride,
-          (const bf16*)k_pages, (const bf16*)v_pages, nh, nkv, page_shift, scale, window, keep_first, part_acc, part_ml, shared_by,
-          first_row, n_rows, ex, stream);
+      const int rc = run((const bf16*)q, q_stride, out, out_stride, q_start, q_len, pos0, seq_base, n_seqs, max_q_len, tables,
+                         table_stride, (const bf16*)k_pages, (const bf16*)v_pages, nh, nkv, page_shift, scale, window, keep_first,
+                         part_acc, part_ml, shared_by, first_row, n_rows, ex, stream);
+      if (rc) return rc;
     }
   } else {
     GB_FOR_HEAD_SIZES(GB_CASE)

@@ -809,6 +809,7 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
   const RingRows rows = ring_rows(M, columns * slices, k_slice ? k_slice : K);
   const dim3 grid(columns, rows.tiles, slices), block(RGM * RGN * 64);
   GB_REQUIRE(grid.y <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
+  GB_REQUIRE(ring_has(rows.height), "gemm_bf16: no ring kernel for tiles of %d rows (M=%d)", 32 * rows.height, M);
 #define GB_H(H, SHORT)                                                                                                 \
   if (rows.height == H && (SHORT == H) == (H == 8 && rows.tall == rows.tiles))                                         \
     hipLaunchKernelGGL((gemm_ring_kernel<EPI, CT, false, H, SHORT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, \

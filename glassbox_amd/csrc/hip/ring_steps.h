@@ -32,6 +32,7 @@ struct RingRows {
   int height, tall, tiles;   // of 32 rows: the tall tiles; how many of them, the others being one less; all tiles
   float us;                  // the estimate
 };
+constexpr bool ring_has(int height) { return height >= 5 && height <= 8; }   // what the kernel is built for: 129 rows and more are dealt so
 inline RingRows ring_rows(int M, int columns, int K) {
   const int rows = (M + 31) / 32;
   auto round_us = [&](int h, long long n) {

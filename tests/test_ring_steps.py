@@ -15,6 +15,7 @@ extern "C" int numbers(int i) { return i == 0 ? gb::RBK : i == 1 ? gb::RING_K : 
 extern "C" int steps(int K) { return gb::ring_steps(K); }
 extern "C" int step_at(int s, int K, int head) { return gb::ring_step_at(s, K, head != 0); }
 extern "C" int dead_half(int K, int head) { return gb::ring_dead_half(K, head != 0); }
+extern "C" int has(int height) { return gb::ring_has(height); }
 extern "C" int rows(int M, int columns, int K, int i) {
   const gb::RingRows r = gb::ring_rows(M, columns, K);
   return i == 0 ? r.height : i == 1 ? r.tall : r.tiles;
@@ -67,6 +68,13 @@ def test_tiles_hold_every_row_once(ring, columns):
     for M in (512, 2048, 8192):
         if M // 256 * columns % 256 == 0:
             assert ring.rows(M, columns, 4096, 0) == 8 and ring.rows(M, columns, 4096, 2) == M // 256
+
+
+def test_rows_too_few_for_any_tile_are_told_from_the_others(ring):
+    """A launch refuses a height that no kernel has, in place of launching nothing: up to 128 rows, and none of more."""
+    for columns in (1, 16, 300):
+        for M in range(1, 1500):
+            assert bool(ring.has(ring.rows(M, columns, 2048, 0))) == (M > 128), M
 
 
 @pytest.mark.parametrize("columns", [1, 3, 7, 24, 112])
