@@ -336,6 +336,30 @@ def test_streams_norm_with_a_word_a_thread(S, n, d, gamma_dtype, out_dtype):
     assert ((picked.cpu().to(F64) - want).abs() <= tol * (1 + want.abs())).all()
 
 
+@pytest.mark.parametrize("S", [1, 2, 3, 4])
+@pytest.mark.parametrize("n, d", [(2, 2048), (3, 4), (1, 4096), (5, 252), (7, 1028)])
+@pytest.mark.parametrize("gamma_dtype, out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("weights", [False, True])
+def test_streams_norm_with_a_word_a_thread_gives_the_bits_of_the_general_kernel(S, n, d, gamma_dtype, out_dtype, weights):
+    """The same expressions in the same order: a gamma that begins 8 bytes behind a word of 16 is the general kernel's."""
+    from glassbox_amd import ops
+    torch.manual_seed(S * d + n)
+    X, y = torch.randn(S, n, d), torch.randn(n, d)
+    w_in, w_out, mix = torch.randn(S), torch.randn(S), torch.randn(S, S)
+    gamma = (torch.rand(d) + 0.5).to(gamma_dtype)
+    got = []
+    for shift in (0, 8 // gamma.element_size()):
+        g = torch.zeros(d + 16, device=DEV, dtype=gamma_dtype)[shift:shift + d]
+        g.copy_(gamma)
+        assert (g.data_ptr() % 16 == 0) == (shift == 0)
+        Xd, h, total = _dev(X), torch.empty(n, d, device=DEV, dtype=out_dtype), torch.empty(n, d, device=DEV)
+        first = torch.empty_like(h)
+        ops.streams_norm(Xd, _dev(w_in) if weights else None, g, 1e-5, first)
+        ops.streams_norm(Xd, _dev(w_in) if weights else None, g, 1e-5, h, total=total, update=(_dev(mix), _dev(w_out), _dev(y)))
+        got.append((first, Xd, total, h))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 # ------------------------------------------------------------------------------------------ attention
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("window, keep", [(24, 5), (16, 16), (300, 2), (7, 40), (33, 0)])
