@@ -1365,6 +1365,8 @@ extern "C" int gb_attention_decode_bf16_static(const void* q, int q_stride, void
 // workgroups first (four a workgroup only if that still gives every compute unit one), then a pair's keys over
 // waves (four a workgroup; eight where even single pairs leave compute units idle), and where the pairs are at most
 // half the compute units and the contexts long, over `parts` workgroups whose sums a second pass adds.
+// For head sizes other than 64 and 128, and for those with capped or sloped scores or 32-bit results (else: shared_plan).  The figures
+// below are of plain scores and bfloat16 results, measured while heads of 64 and 128 came here with those too.
 struct PrefillPlan {
   int per_group, split, parts;
 };
@@ -1503,8 +1505,9 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
   const PrefillPlan plan = prefill_plan(max_q_len, max_context, nh, n_seqs, hd);
   int per_group = plan.per_group, split = plan.split;
   const int parts = shared ? shared_by.parts : plan.parts;
-  // over runs of positions the pairs are not equal work: one pair a workgroup and more waves a pair, as long as all are in
-  // the chip at once (2,048 tokens, 16 heads, runs of 1,536: 27.6 -> 23.1 us; not for 32 heads, nor for short runs)
+  // prefill_kernel: over runs of positions the pairs are not equal work: one pair a workgroup and more waves a pair, as long as all
+  // are in the chip at once (2,048 tokens, 16 heads of 64, runs of 1,536, when they came here: 27.6 -> 23.1 us; not for 32 heads, nor
+  // for short runs)
   const long long pairs = (long long)((max_q_len + 63) / 64) * nh * n_seqs;
   if (ex.span >= 1024 && hd <= 64 && per_group == 2 && pairs < 768) per_group = 1, split = 4;
   float *part_acc = nullptr, *part_ml = nullptr;

@@ -1024,7 +1024,9 @@ inline bool block_takes(const void* a, int lda, const void* w, int ldw, int K) {
 // take.  A product that is not formed into a gated unit stays with the tiled kernel, whose fewer k-steps ahead start sooner, below a k of
 // 1,024 (3,840 x 960, 65 to 128 rows: 6.3 to 6.6 us; 1,600 x 960, 131 rows 6.3, 7.0 here).
 inline bool block_sizes(int M, int N, int K, bool silu) { return M > 32 && K % RBK == 0 && N % 8 == 0 && (silu ? N % 16 == 0 : K >= 1024); }
-// What the ring kernel takes, alike: a k-step of its 256 x 256 tiles 1.75 us.
+// What the ring kernel takes beside that, for the lines below and the slices of k, which were measured with tiles of 256 x 256 alone:
+// a k-step of a round of them 1.75 us.  (The launch deals rows by ring_rows, whose estimate of a full round is 1.60; where the two
+// kernels are compared by time, that one decides: ring_ahead.)
 inline float ring_us(int M, int N, int K, int slices) {
   const long long tiles = (long long)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN) * slices;
   return 3.5f + (float)((tiles + 255) / 256) * ((K / slices + RBK - 1) / RBK) * 1.75f + (slices > 1 ? 3.5f + slices * (float)M * N * 8.f / 4.5e6f : 0.f);

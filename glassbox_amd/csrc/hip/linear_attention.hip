@@ -6,9 +6,9 @@
 //
 // The state is 32-bit and lives in a slot per live request, [heads, dv, dk]: a column of S (one value channel)
 // lies in a row of memory.  Columns never meet: column j of S_t depends on column j of S_(t-1), k_t and v_t[j]
-// alone.  So a wave owns eight columns, eight lanes a column, a lane R = ceil(dk / 8) of its rows in registers, and
-// walks its request's tokens of the step in order: the same additions in the same order whether a prompt comes
-// whole, in portions or token by token.  A workgroup (four waves, 32 columns of one head) stages the tokens'
+// alone.  So a wave owns eight columns, or sixteen (C of them a lane), eight lanes a column, a lane R = ceil(dk / 8) of its
+// rows in registers, and walks its request's tokens of the step in order: the same additions in the same order whether a
+// prompt comes whole, in portions or token by token.  A workgroup (four waves, 32 C columns of one head) stages the tokens'
 // q, k and decays through LDS sixteen tokens at a time, the next sixteen on their way from memory meanwhile.
 // q, k and the decays come in 32-bit (what the kernels below prepare), v in the activations' type.
 //
