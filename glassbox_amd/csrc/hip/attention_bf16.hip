@@ -926,6 +926,8 @@ __global__ __launch_bounds__(64 * PAIRS * SPLIT, 2) void prefill_kernel(const bf
 // earlier and higher priorities around the MFMAs gave nothing.
 // S waves a block take its tiles in turn (and meet in hand_over) where the blocks alone leave SIMDs without a second wave,
 // and `parts` workgroups where even that leaves compute units idle: shared_plan.
+// A block with columns that have no token masks the tiles that its last token needs masked, and no others: masked in every one, it
+// was what the launch waited for (31 tokens behind 2,017, 32 heads over 8 of 128: 18.2 us, 15.5 so; 500 behind 7,500: 140, 102).
 // Before and after, us: 6,151 tokens, 32 heads over 8 of 128: 512, 313 (990 TFLOP/s); 2,048 tokens, 32 heads of 64: 38.0, 32.0;
 // 8,192: 395, 306; 131 tokens behind 3,900: 35.7, 24.8; 482 behind 512: 19.1, 14.6; five prompts of 77 to 172, 15 heads over 5:
 // 11.4, 8.1; 60 tokens, 32 heads: 11.0, 4.7.
@@ -1140,8 +1142,8 @@ __global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
   copy_tile(i0 + half, 0);
   look_up(i0 + half + S);
 
-  const int p = p0 + tok;
-  const int lo = valid ? first_key(p, window, ex.span) : 1, hi = valid ? p : 0;
+  // (a column without a token goes with the last one: as one that sees nothing it would have every tile of its block masked)
+  const int hi = p0 + min(tok, qlen - 1), lo = first_key(hi, window, ex.span);
   const BlockRange range = block_range(32 * block, qlen, p0, window, ex.span);
   float m = -INFINITY, l = 0.f;
   f32x16 acc[DB];
@@ -1163,8 +1165,8 @@ __global__ __launch_bounds__(512, 2) void prefill_shared_kernel(
     const int kb = keys.of(i + half);
     // (a tile of kept first keys is seen by all; another one by the blocks whose range it meets)
     if (works && (S == 1 || i + half < i1) && kb <= range.last && (kb + 63 >= range.first || kb < keep))
-      shared_attend<HD>(m, l, acc, qf, ring + (slot * S + half) * TILE, kb, lo, hi, keep, !range.whole || kb + 63 > range.free_hi,
-                        !range.whole || kb < range.free_lo, c, lane);
+      shared_attend<HD>(m, l, acc, qf, ring + (slot * S + half) * TILE, kb, lo, hi, keep, kb + 63 > range.free_hi, kb < range.free_lo, c,
+                        lane);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // what was read of this tile is in registers
     slot ^= 1;
   }
