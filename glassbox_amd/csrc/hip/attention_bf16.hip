@@ -1418,21 +1418,36 @@ inline PrefillPlan prefill_plan(int max_q_len, int max_context, int nh, int n_se
 //   heads: 43, 56)
 //   fewer still and many tiles: the keys of a block over several workgroups, as long as all are resident (140 tokens behind 4,935:
 //   2 x 2 in five parts 24.9, in six 29.6, 2 x 4 48; 700 tokens of 15 heads behind 3,000, N 330: 34.0 in four parts, 2 x 4 38.4, but 1,139 of 9 heads, N 324: 16.8, 16.2)
+//   portions of one block (up to 32 tokens): the blocks side by side are a kv head's query heads alone, so that the workgroups are
+//   counted with the kv heads, and each has its unit's LDS almost for itself.  Heads of 128: from nine or eleven tiles on a block's
+//   keys go to several workgroups (20 tokens, 32 heads over 8, behind 540: 13.1 in one, 11.4 in three; behind 780: 16.2, 11.6 in four;
+//   three portions of 31 behind 550: 13.6, 14.4; with a second pass of many rows, eight portions behind 870, 16.9 in one, 18.8 in
+//   two), and beyond a workgroup a unit one wave a block, two
+//   workgroups a unit (16 portions of 32 heads behind 400: 2 x 1 22.5, 2 x 2 27.5).  Heads of 64 there: 2 x 2, not 2 x 4 (32
+//   portions, 15 heads over 5, behind 550: 2 x 4 19.2, 2 x 2 16.4)
 struct SharedPlan {
   int rows, split, parts;
 };
-inline SharedPlan shared_plan(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
+inline SharedPlan shared_plan(int max_q_len, int max_context, int nh, int nkv, int n_seqs, int hd) {
   const long long blocks = (max_q_len + 31) / 32, heads = (long long)nh * n_seqs, N = blocks * heads;
   const long long T = (max(max_context, max_q_len) + 63) / 64, pairs = (blocks + 1) / 2 * heads;
+  const long long groups = (nh / nkv + 1) / 2 * (long long)nkv * n_seqs;   // workgroups of two blocks, of portions of one block
   if (hd <= 64) {
     if (T == 1) return {2, 1, 1};
     if (N >= 6500 || N >= 400 * T) return {4, 1, 1};
     if (N >= 2500) return {4, 2, 1};
+    if (blocks == 1 && groups > 256) return {2, 2, 1};
     if (T <= 3 || N >= (T < 32 ? 1000 : 1200)) return {2, 2, 1};
     if (N > 256 || T < 16) return {2, 4, 1};
     return {2, 2, (int)max(1ll, min(min(8ll, 512 / pairs), T / 5))};
   }
   if (T <= 2) return {2, 1, 1};
+  if (blocks == 1 && nh == nkv && N > 256) return {2, 1, 1};
+  if (blocks == 1 && groups <= 256) {
+    if (T < (groups <= 32 ? 9 : 11) || (T < 16 && groups > 64)) return {2, 2, 1};
+    if (groups > 128 && groups * 3 <= 512 && T >= 48) return {2, 2, 3};
+    return {2, 2, (int)max(1ll, min(min(8ll, 256 / groups), T < 16 ? (T + 3) / 4 : T / 8))};
+  }
   if (N >= 2500 || N >= 210 * T) return {4, 1, 1};
   if (N >= 900) return {4, 2, 1};
   if (N > 256 || T < 16) return {2, 2, 1};
@@ -1441,10 +1456,14 @@ inline SharedPlan shared_plan(int max_q_len, int max_context, int nh, int n_seqs
 inline bool shared_takes(int hd) { return hd == 64 || hd == 128; }
 
 // rows * 100 + split * 10 + parts of the plan above (0: head sizes it is not for)
-extern "C" int gb_attention_prefill_shape(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
-  if (!shared_takes(hd)) return 0;
-  const SharedPlan p = shared_plan(max_q_len, max_context, nh, n_seqs, hd);
+extern "C" int gb_attention_prefill_shape_of(int max_q_len, int max_context, int nh, int nkv, int n_seqs, int hd) {
+  if (!shared_takes(hd) || nkv <= 0 || nh % nkv) return 0;
+  const SharedPlan p = shared_plan(max_q_len, max_context, nh, nkv, n_seqs, hd);
   return p.rows * 100 + p.split * 10 + p.parts;
+}
+// The same with a kv head a query head: what portions of more than one block get in any case.
+extern "C" int gb_attention_prefill_shape(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
+  return gb_attention_prefill_shape_of(max_q_len, max_context, nh, nh, n_seqs, hd);
 }
 
 template <int HD>
@@ -1476,8 +1495,12 @@ static int prefill_shared_launch(const bf16* q, int q_stride, bf16* out, int out
 // Workgroups that would share a pair's keys with these sizes (1: none do); the caller then provides
 // parts * rows * nh * (hd + 2) floats for their sums, rows being all rows of the portions.
 extern "C" int gb_attention_prefill_parts(int max_q_len, int max_context, int nh, int n_seqs, int hd) {
-  const int parts = prefill_plan(max_q_len, max_context, nh, n_seqs, hd).parts;
-  return shared_takes(hd) ? max(parts, shared_plan(max_q_len, max_context, nh, n_seqs, hd).parts) : parts;
+  int parts = prefill_plan(max_q_len, max_context, nh, n_seqs, hd).parts;
+  if (shared_takes(hd)) {   // (whatever the number of kv heads)
+    for (int nkv = 1; nkv <= nh; ++nkv)
+      if (nh % nkv == 0) parts = max(parts, shared_plan(max_q_len, max_context, nh, nkv, n_seqs, hd).parts);
+  }
+  return parts;
 }
 
 // Requests seq_base .. seq_base+n_seqs-1 of the step (prompt portions); max_q_len is the longest portion and
@@ -1503,7 +1526,7 @@ static int prefill_launch(const void* q, int q_stride, OT* out, int out_stride, 
   GB_REQUIRE(n_seqs <= 65535 && nh <= 65535, "attention_prefill: too many requests or heads for one launch");
   if (n_seqs == 0 || max_q_len <= 0) return 0;
   const bool shared = std::is_same<OT, bf16>::value && shared_takes(hd) && ex.softcap == 0.f && ex.slopes == nullptr;
-  const SharedPlan shared_by = shared_plan(max_q_len, max_context, nh, n_seqs, hd);
+  const SharedPlan shared_by = shared_plan(max_q_len, max_context, nh, nkv, n_seqs, hd);
   const PrefillPlan plan = prefill_plan(max_q_len, max_context, nh, n_seqs, hd);
   int per_group = plan.per_group, split = plan.split;
   const int parts = shared ? shared_by.parts : plan.parts;

@@ -1682,6 +1682,46 @@ def test_tuned_prefill_of_short_requests_beside_long_ones(shape, nh, nkv, hd, q_
     assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
 
 
+@pytest.mark.parametrize("shape,nh,nkv,hd,q_lens,history", [
+    # few tiles; from nine or eleven on several workgroups a block; many requests; beyond a workgroup a unit; three parts of long ones
+    (221, 8, 2, 128, [31, 2], 480), (223, 8, 2, 128, [31, 2], 500), (221, 33, 33, 128, [31, 2], 600), (223, 8, 2, 128, [31, 2], 640), (224, 9, 3, 128, [17], 860), (221, 32, 8, 128, [5] * 17, 700),
+    (211, 32, 32, 128, [3, 32, 17] * 3, 150), (223, 43, 43, 128, [20, 9, 31], 3050), (222, 40, 8, 128, [32, 3] * 2, 1100),
+    (221, 32, 32, 64, [3, 32, 17] * 3, 300), (221, 15, 5, 64, [31, 2] * 13, 250), (241, 15, 5, 64, [31, 2] * 12, 250)])
+def test_tuned_prefill_of_portions_of_one_block(shape, nh, nkv, hd, q_lens, history):
+    """Portions of up to 32 tokens, whose workgroups hold query heads of a kv head side by side: every way of spreading them, and
+    blocks with columns without a token."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    ctx_lens = [history + n for n in q_lens]
+    lib = ops._lib("attention_bf16")
+    assert lib.gb_attention_prefill_shape_of(max(q_lens), max(ctx_lens), nh, nkv, len(q_lens), hd) == shape
+    assert ops._prefill_parts(max(q_lens), max(ctx_lens), nh, len(q_lens), hd) >= shape % 10
+    k_pages, v_pages, tables, _, _ = paged_setup(ctx_lens, nkv, hd, 16, seed=hd + nh, dtype=torch.bfloat16)
+    ctx = BareContext(q_lens, ctx_lens, tables)
+    q = to_dev((rnd(sum(q_lens), nh * hd, seed=14) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    for window, keep, chunk in ((0, 0, 0), (history - 60, 20, 0), (0, 0, history - 33)):
+        out, twin = torch.zeros_like(q), torch.zeros_like(q)
+        ops.attention_prefill(q, out, ctx, cache, nh, 1 / math.sqrt(hd), window, keep, chunk)
+        ops.attention_plain(q, twin, ctx.positions, torch.tensor(ctx.tok_seq, dtype=torch.int32, device=DEV), ctx.tables[0],
+                            cache.k_pages, cache.v_pages, nh, 1 / math.sqrt(hd), window, keep_first=keep, chunk=chunk)
+        # softmax weights in bfloat16 (2^-9 of each value's share) and a bfloat16 result on either side
+        assert ((out.float() - twin.float()).abs() <= 2 ** -7 * (1 + twin.float().abs())).all()
+
+
+@pytest.mark.parametrize("group", [1, 2, 3, 4, 6, 12])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_the_workspace_of_a_portion_suffices_for_any_number_of_kv_heads(group, hd):
+    from glassbox_amd import ops
+    lib = ops._lib("attention_bf16")
+    for nkv in (1, 2, 5, 8, 11, 32):
+        for n in (1, 2, 3, 5, 8, 17, 40):
+            for q_len in (3, 32, 33, 200):
+                for context in (q_len, 600, 710, 1100, 3100, 8000):
+                    shape = lib.gb_attention_prefill_shape_of(q_len, context, nkv * group, nkv, n, hd)
+                    assert 1 <= shape % 10 <= ops._prefill_parts(q_len, context, nkv * group, n, hd)
+
+
 @pytest.mark.parametrize("nh,ctxlen,qlen", [(2, 200, 90), (64, 1200, 1090)])   # 32 and 64 tokens a wave
 def test_tuned_prefill_sees_exactly_the_causal_keys(nh, ctxlen, qlen):
     """A portion in the middle of a request (it starts at position 110): token t must find a marked
