@@ -891,9 +891,13 @@ int launch_scan(int R, hipStream_t stream, const float* q, const float* k, const
   const int words = dk % 4 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)seg_state % 16 == 0;
   // Sixteen rows a lane: two columns a lane where that still leaves a workgroup for every compute unit.  A column of fewer rows
   // keeps its lanes as busy with its own sums as LDS with its reads (us, one / two columns: 2,048 rows, 16 heads of 128 by 128 180.7 /
-  // 142.1; 32 of 64 by 65 115 / 136; 1,555 rows of two requests, 32 of 64 by 64 67.1 / 72.9); more have no registers for two.
+  // 142.1; 32 of 64 by 65 115 / 136; 1,555 rows of two requests, 32 of 64 by 64 67.1 / 72.9); more have no registers for two.  Portions
+  // that are not cut: two workgroups a unit, since few of a step's requests may bring its rows (222 rows beside three single tokens, 32
+  // heads of 128 by 128 89 / 116, one column a lane before this choice 99; eight of 200 rows, 16 heads, 88 / 97; 16 of 120 rows, 16
+  // heads of 96 by 128, 140 / 104).  Not where a key's channels are no whole words, whose loads take as long as the sums (101 rows, 32
+  // heads of 65 by 256, 40.7 / 49.9).
   const long long wide = (dv + 2 * kColsBlock - 1) / (2 * kColsBlock) * (long long)nh * n_seqs * segs;
-  const int C = R == 16 && dv > kColsBlock && wide >= 256 ? 2 : 1;
+  const int C = R == 16 && words && dv > kColsBlock && wide >= (segs > 1 ? 256 : 512) ? 2 : 1;
   const dim3 grid((unsigned)((dv + kColsBlock * C - 1) / (kColsBlock * C)), (unsigned)nh, (unsigned)(n_seqs * segs));
 #define GB_SCAN(RR, CC)                                                                                                      \
   if (R == RR && C == CC) {                                                                                                  \
