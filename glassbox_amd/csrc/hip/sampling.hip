@@ -545,8 +545,9 @@ __global__ __launch_bounds__(TPB) void sample_kernel(float* __restrict__ logits,
   // then all tokens lie above the bound, and the pass that finds candidates would be for nothing (4,099 tokens, five of them left, k
   // 50: 67 us by the searches, 72.6 with it).  Nor for very many candidates of a small vocabulary, whose sort costs what the searches
   // do (4,099 tokens, no other filter, the searches / so: k 256 30.1 / 21.6, 512 26.8 / 29.6; 32,000 tokens, k 512 65 / 40).
+  // (1,024 tokens, a mask that leaves fewer than k: 39 / 46.)
   const int most = V < 16384 ? MOST_OF_BESTS / 2 : MOST_OF_BESTS;
-  if (k > 0 && k < V && k <= most && V >= TPB && (V == TPB || __syncthreads_count(best > least) >= k)) {
+  if (k > 0 && k < V && k <= most && V >= TPB && __syncthreads_count(best > least) >= k) {
     u64 chosen = 0;
     if (sample_few(r, composite(best, best_at), k, min_p[rix], top_p[rix], uniform[rix], sh, &chosen, &count)) {
       if (count <= 1) chosen = b;
@@ -598,7 +599,8 @@ __global__ __launch_bounds__(TPB) void sample_kernel(float* __restrict__ logits,
 extern "C" int gb_argmax(const float* logits, int32_t* out, int rows, int V, hipStream_t stream) {
   GB_REQUIRE(rows >= 0 && V > 0 && V <= (1 << IDX_BITS), "argmax: vocabulary %d is outside 1..%d", V, 1 << IDX_BITS);
   if (rows == 0) return 0;
-  hipLaunchKernelGGL(rows <= 256 ? argmax_kernel<true> : argmax_kernel<false>, dim3(rows), dim3(ARGMAX_TPB), 0, stream, logits, out, V);
+  // (rows of less than a token a thread: 151 tokens 3.2 us, by words 3.6)
+  hipLaunchKernelGGL(rows <= 256 && V >= 1024 ? argmax_kernel<true> : argmax_kernel<false>, dim3(rows), dim3(ARGMAX_TPB), 0, stream, logits, out, V);
   return launched("argmax");
 }
 

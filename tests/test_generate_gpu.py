@@ -163,7 +163,7 @@ def test_sampling_kernel_on_rows_of_ties_and_edge_settings():
 
 
 @pytest.mark.parametrize("rows", [7, 256, 257])
-@pytest.mark.parametrize("vocab", [1, 2, 3, 6, 4097, 16387, 20006])
+@pytest.mark.parametrize("vocab", [1, 2, 3, 6, 1023, 1026, 4097, 16387, 20006])
 def test_argmax_of_rows_that_begin_anywhere(rows, vocab):
     """Rows that begin at every place in a word of 16 bytes, from one token on; the maximum at either end and in the words between,
     the first of two."""
