@@ -440,65 +440,17 @@ __global__ void store_values_kernel(const T* __restrict__ qkv, int row_stride, c
                        row_stride, slots, v_pages, q_start, q_len, pos0, nh, nkv, hd, page_size);
 }
 
-// The queries and keys of one token in rope_store_pieces' way, the same piece of U heads `step` apart: what turns them is read once.
-template <int U>
-__device__ __forceinline__ void rope_heads(int t, int unit, int step, int j, bf16* __restrict__ qkv, int row_stride,
-                                           const float* __restrict__ cosv, const float* __restrict__ sinv,
-                                           const int32_t* __restrict__ slots, bf16* __restrict__ k_pages, int nh, int nkv, int hd,
-                                           int page_size, int rotate) {
-  const int half = hd / 2, units = nh + nkv;
-  bf16* row = qkv + (size_t)t * row_stride + j;
-  bf16x8 x0[U], x1[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const bf16* head = row + (size_t)min(unit + u * step, units - 1) * hd;
-    x0[u] = *reinterpret_cast<const bf16x8*>(head);
-    x1[u] = *reinterpret_cast<const bf16x8*>(head + half);
-  }
-  const int slot = slots && unit + (U - 1) * step >= nh ? slots[t] : -1;
-  const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
-  if (rotate) {
-    const float* cr = cosv + (size_t)t * half + j;
-    const float* sr = sinv + (size_t)t * half + j;
-    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cr), c1 = *reinterpret_cast<const f32x4*>(cr + 4);
-    const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr), s1 = *reinterpret_cast<const f32x4*>(sr + 4);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float c = e < 4 ? c0[e] : c1[e - 4], sn = e < 4 ? s0[e] : s1[e - 4];
-        const float a = (float)x0[u][e], b = (float)x1[u][e];
-        x0[u][e] = (bf16)(a * c - b * sn);
-        x1[u][e] = (bf16)(b * c + a * sn);
-      }
-      if (unit + u * step < units) {   // rotated keys stay in the row too: parts may read them back
-        bf16* head = row + (size_t)(unit + u * step) * hd;
-        *reinterpret_cast<bf16x8*>(head) = x0[u];
-        *reinterpret_cast<bf16x8*>(head + half) = x1[u];
-      }
-    }
-  }
-  if (slot < 0) return;
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int at = unit + u * step;
-    if (at < nh || at >= units) continue;
-    bf16* dst = k_pages + ((size_t)page * nkv + (at - nh)) * page_size * hd;
-    *reinterpret_cast<bf16x8*>(dst + key_offset(off, j, page_size, 8)) = x0[u];
-    *reinterpret_cast<bf16x8*>(dst + key_offset(off, half + j, page_size, 8)) = x1[u];
-  }
-}
-
 // All of a bfloat16 step with prompt portions in one launch: the first `rope_blocks` workgroups rotate and write keys, the next
 // `row_blocks` write the values of the single-token rows, a dimension a lane, and the rest turn the portions' values tile by tile,
 // `heads` (a power of two) of a tile a workgroup.
 // What bounds a rotation is the lines that its lanes write: a lane's 16 bytes of a key page lie 256 from its neighbour's where the
-// lanes of a wave take the pieces of one token.  So they take a piece of sixteen tokens, whose places in the page are
-// neighbours, and of U heads where there are tokens enough.  A value row's lanes write two bytes every 32, whatever the split; a
-// lane with 16 of them, one after the other, took twice as long as all else in a step of 30 rows and a portion.
-// us, a token a workgroup (and the values apart from 1,025 rows on) / so, 32 heads of 64: 2,048 tokens 16.8 / 14.4; 482 and 30
-// rows 9.6 / 7.0; 131 5.0 / 4.8; 1,555 of two prompts 16.6 / 12.1; 6,151 tokens, 32 heads over 8 of 128, 48.0 / 41.3.
-template <int U>
+// lanes of a wave take the pieces of one token, and the places beside them are other tokens'.  So lanes side by side take a piece of
+// two tokens, and a die (workgroups b, b + 8, ...) a run of neighbouring tokens, whose pieces its second-level cache brings together
+// before it writes them back.  (One token a workgroup in such runs, two apart, sixteen lanes a piece and up to four heads a lane; two in
+// runs, us: 32 heads of 64, 2,048 tokens 11.8, 13.0, 12.7, 12.2; 32 over 8 of 128, 482 4.7, 4.7, 5.5, 4.6, 1,024 6.7, 6.6, 8.7, 6.6,
+// 6,151 26.3, 30.1, 31.5, 27.3; 15 over 5 of 64, 2,048 5.5, 5.0, 5.6, 5.0.)
+// A value row's lanes write two bytes every 32, whatever the split; a lane with 16 of them, one after the other, took twice as long as
+// all else in a step of 30 rows and a portion (482 and 30 rows 9.6, 7.0 with a dimension a lane).
 __global__ __launch_bounds__(256) void rope_and_values_kernel(bf16* __restrict__ qkv, int row_stride, const float* __restrict__ cosv,
                                        const float* __restrict__ sinv, const int32_t* __restrict__ slots,
                                        bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int rows, int nh, int nkv, int hd,
@@ -509,9 +461,10 @@ __global__ __launch_bounds__(256) void rope_and_values_kernel(bf16* __restrict__
   const int tid = threadIdx.x;
   int b = blockIdx.x;
   if (b < rope_blocks) {
-    const int t = b / rope_y * 16 + tid % 16, idx = b % rope_y * (16 * U) + tid / 16, lanes = hd / 16;
-    if (t < rows && idx / lanes < nh + nkv)
-      rope_heads<U>(t, idx / lanes, 16 / lanes, idx % lanes * 8, qkv, row_stride, cosv, sinv, slots, k_pages, nh, nkv, hd, page_size, rotate);
+    const int r = b % 8 * (rope_blocks / 8) + min(b % 8, rope_blocks % 8) + b / 8;
+    const int t = r / rope_y * 2 + tid % 2, idx = r % rope_y * 128 + tid / 2;
+    if (t < rows && idx < (nh + nkv) * (hd / 16))
+      rope_store_pieces(t, idx, qkv, row_stride, cosv, sinv, slots, k_pages, v_pages, nh, nkv, hd, page_size, rotate);
     return;
   }
   b -= rope_blocks;
@@ -550,19 +503,14 @@ extern "C" int gb_rope_store(void* qkv, int dtype, int row_stride, const float* 
   const bool pieces = dtype == kBF16 && hd % 16 == 0 && row_stride % 8 == 0 && (uintptr_t)qkv % 16 == 0 &&
                       (uintptr_t)k_pages % 16 == 0 && (!rotate || ((uintptr_t)cosv % 16 == 0 && (uintptr_t)sinv % 16 == 0));
   if (tiles && pieces) {
-    // Four heads a lane where a lane's piece is the same of all and 256 workgroups are left; two of some thousands of tokens, whose
-    // heads lie too far apart to be written back together (32 heads of 64, one / two / four: 1,024 tokens 10.4 / 9.5 / 8.9, 2,048
-    // 15.7 / 14.8 / 14.4, 4,096 32.9 / 32.4 / 32.6, 8,192 62.8 / 62.5 / 70.0).
-    const bool several = 16 % (hd / 16) == 0 && (long long)n * (nh + nkv) * hd >= 16 * 256 * 256 * 4LL;
-    const int each = !several ? 16 : n < 4096 ? 64 : 32, rope_y = ((nh + nkv) * (hd / 16) + each - 1) / each;
+    const int rope_y = ((nh + nkv) * (hd / 16) + 127) / 128;
     const int groups = (max_q_len + 15) / 16 + 1;
     const int heads = hd <= 32 ? 4 : hd <= 64 ? 2 : 1;   // 2 hd threads finish a tile's words
     const int row_y = (nkv * hd + 255) / 256;
-    const long long rope_blocks = (n + 15LL) / 16 * rope_y, row_blocks = (long long)v_rows * row_y;
+    const long long rope_blocks = (n + 1LL) / 2 * rope_y, row_blocks = (long long)v_rows * row_y;
     const long long blocks = rope_blocks + row_blocks + (long long)groups * ((nkv + heads - 1) / heads) * n_seqs;
     GB_REQUIRE(blocks < (1ll << 31), "rope_store: %lld workgroups are too many for one launch", blocks);
-    const auto kernel = each == 64 ? rope_and_values_kernel<4> : each == 32 ? rope_and_values_kernel<2> : rope_and_values_kernel<1>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), heads * 16 * (hd + 2) * sizeof(bf16), stream,
+    hipLaunchKernelGGL(rope_and_values_kernel, dim3((unsigned)blocks), dim3(256), heads * 16 * (hd + 2) * sizeof(bf16), stream,
                        (bf16*)qkv, row_stride, cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, n, nh, nkv, hd, page_size, rotate,
                        (int)rope_blocks, rope_y, (int)row_blocks, row_y, q_start, q_len, pos0, seq_base, groups, heads);
     return launched("rope_store (with the portions' values)");
