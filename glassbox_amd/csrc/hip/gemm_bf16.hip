@@ -707,14 +707,19 @@ __device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], c
         ask(0);
         ask(1);
       }
+      // (what is stored goes by one place that moves on: eight of them at once were more than the registers hold, and 52 bytes a lane
+      // of scratch: 1,157 x 11,280 x 128 18.7 us)
+      CT* at = c + (size_t)(gm0 + lane % 16) * ldc + gn0 + 4 * (lane / 16);
 #pragma unroll
       for (int i = 0; i < H; ++i) {
         const int gm = gm0 + i * 16 + lane % 16;
         if constexpr (EPI == EPI_ACCUMULATE) {
           if (i + 2 < H) ask(i + 2);
+        } else {
+          asm volatile("" : "+v"(at));
         }
         if (gm < M) {
-          CT* to = to_of(i);
+          CT* to = EPI == EPI_ACCUMULATE ? to_of(i) : at;
           const float factor = scaled ? grp.in_scale[gm] : 1.f;
 #pragma unroll
           for (int j = 0; j < OUT; ++j) {
@@ -723,6 +728,7 @@ __device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], c
             store_c4<CT>(to + j * 16, v);
           }
         }
+        at += (size_t)16 * ldc;
         __builtin_amdgcn_sched_barrier(0);
       }
     }
