@@ -659,7 +659,8 @@ __device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], c
     }
   };
   const bool scaled = GROUPED && EPI == EPI_SILU_MUL && grp.in_scale;
-  if (gn0 + OUT * 16 <= cols && (size_t)ldc * sizeof(CT) % 16 == 0 && (uintptr_t)c % 16 == 0) {   // the same for the whole wave
+  const bool words = (size_t)ldc * sizeof(CT) % 16 == 0 && (uintptr_t)c % 16 == 0;   // rows of C are whole words
+  if (gn0 + OUT * 16 <= cols && words) {   // the same for the whole wave
     if constexpr (sizeof(CT) == 2) {
       // As they lie, a store of the wave would write 32 bytes of 16 rows; so bfloat16 results go through LDS (32 KB of the
       // wave's own: every wave has read its last operands) and out in runs of 128 or 256 bytes (8,192 x 16,384 x 128, a
@@ -734,7 +735,33 @@ __device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], c
     }
     return;
   }
-  // the last columns of C, or rows of C that are no 16-byte words
+  // The last columns of C: four of them a lane, where none of a lane's lies beyond.  (One after the other, a column's old value was
+  // waited for before the next one's was asked for, 256 of them, and the launch waited for those tiles.  us, so / now: added to, 8,192 x
+  // 5,344 x 512 139 / 96, 7,161 x 3,552 x 960 113 / 71; stored in 32-bit 83 / 73, 65 / 60.)
+  if (words && cols % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const int gm = gm0 + i * 16 + lane % 16, gn = gn0 + 4 * (lane / 16);
+      if (gm >= M) continue;
+      CT* to = c + (size_t)gm * ldc + gn;
+      const float factor = scaled ? grp.in_scale[gm] : 1.f;
+      f32x4 old[OUT];
+      if constexpr (EPI == EPI_ACCUMULATE)
+#pragma unroll
+        for (int j = 0; j < OUT; ++j)
+          if (gn + j * 16 < cols) old[j] = *reinterpret_cast<const f32x4*>(to + j * 16);
+#pragma unroll
+      for (int j = 0; j < OUT; ++j) {
+        f32x4 v = result(i, j, factor);
+        if (gn + j * 16 >= cols) continue;
+        if constexpr (EPI == EPI_ACCUMULATE) v = old[j] + v;
+        store_c4<CT>(to + j * 16, v);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return;
+  }
+  // rows of C that are no 16-byte words
 #pragma unroll
   for (int i = 0; i < H; ++i) {
     const int gm = gm0 + i * 16 + lane % 16;
@@ -1062,8 +1089,10 @@ inline float ring_us(int M, int N, int K, int slices) {
 // loads are whole 16-byte pieces; and wherever its estimate with the heights of ring_rows is below the block kernel's, which is
 // also a bound below the tiled kernel's time.  (That estimate is some 10 % low for several rounds of tiles, and this one by what a
 // tile's old values take.)  Not for one round of them where the tiled kernel's workgroups are resident at once (640 x 12,288 x 1,024
-// 23.0 / 22.4; 930 x 8,192 x 3,072 53 / 58; 420 x 12,288 x 1,280 25.5 / 28.7).  Of 260 products of 200 to 8,192 rows, random sizes among them, one is more than 3 % slower than with
-// the first line alone (3,931 x 14,672 x 576: 146 / 156); us, the block or tiled kernel / this one: 1,350 x 6,144 x 4,096 104 / 69,
+// 23.0 / 22.4; 930 x 8,192 x 3,072 53 / 58; 420 x 12,288 x 1,280 25.5 / 28.7).  Of 1,800 random
+// products of 260 to 8,192 rows and a k of 128 to 2,048 six are more than 4 % slower than with the first line and tiles of 256 alone
+// (456 x 23,440 x 320 with SiLU-multiply 18.0 / 21.0, 789 x 16,928 x 192 20.9 / 24.3, 1,439 x 10,880 x 2,048 with SiLU-multiply 72 / 79);
+// their geometric mean is 0.93.  us, the block or tiled kernel / this one: 1,350 x 6,144 x 4,096 104 / 69,
 // 2,200 x 4,096 x 14,336 372 / 237, 4,500 x 2,048 x 8,192 207 / 146, 700 x 16,384 x 2,048 with SiLU-multiply 60 / 48, 350 x 28,672 x
 // 4,096 115 / 87, 4,096 x 5,120 x 960 58 / 47, 2,900 x 3,072 x 576 23.0 / 18.3.
 inline bool ring_fills(int epi, int M, int N) { return M >= RING_MIN_ROWS && (long long)((M + RBM - 1) / RBM) * ring_columns(epi, N) >= 192; }

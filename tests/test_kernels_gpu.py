@@ -328,6 +328,33 @@ def test_gemm_bf16_ring_writes_rows_that_are_no_whole_words(mode, pad, shift):
     assert bool((c[:, cols:] == 0.5).all()) and bool((room[:shift] == 0.5).all())
 
 
+@pytest.mark.parametrize("mode", ["bf16", "f32", "f32+", "silu"])
+@pytest.mark.parametrize("over", [8, 16, 72, 120, 128, 136, 200, 248, 6, 130])
+def test_gemm_bf16_ring_writes_the_last_columns_alike_by_words_and_one_by_one(mode, over):
+    """Column tiles that C ends in: written four columns a lane, and, where rows of C are no words, one at a time."""
+    from glassbox_amd import ops
+    M, cols, K = (2050, 6912 + (over + 7) // 8 * 8, 128) if mode == "silu" else (1030, 13824 + over, 128)
+    N = 2 * cols if mode == "silu" else cols
+    assert ops.gemm_route(M, N, K, silu_mul=mode == "silu", accumulate=mode == "f32+") == "ring"
+    a, w = to_dev(rnd(M, K, seed=11).bfloat16() * 0.25), to_dev(rnd(N, K, seed=12).bfloat16() * 0.25)
+    dtype = torch.bfloat16 if mode in ("bf16", "silu") else torch.float32
+    got = []
+    for pad in ((-cols) % 8, (-cols) % 8 + 1):
+        c = torch.full((M + 1, cols + pad), 0.5, device=DEV, dtype=dtype)
+        ops.gemm(a, w, c[:M, :cols], accumulate=(mode == "f32+"), silu_mul=(mode == "silu"))
+        assert bool((c[:, cols:] == 0.5).all()) and bool((c[M:] == 0.5).all())
+        got.append(c[:M, :cols].clone())
+    assert torch.equal(*got)
+    rows = [0, 255, 256, M - 1]
+    want = a[rows].double() @ w.double().T
+    if mode == "silu":
+        want = torch.nn.functional.silu(want[:, :cols]) * want[:, cols:]
+    want = want + (0.5 if mode == "f32+" else 0)
+    # sums of K products in 32-bit, and the result's rounding
+    tol = 1e-5 * math.sqrt(K) + (2 ** -8) * want.abs().max().item() * (mode in ("bf16", "silu"))
+    assert (got[0][rows].double() - want).abs().max().item() <= tol
+
+
 @pytest.mark.parametrize("M", [5, 300, 1600])
 def test_gemm_bf16_gated_unit_at_the_ends_of_its_range(M):
     """silu(gate) * up where the exponential or its reciprocal leaves the range, in the kernels that form it in their
