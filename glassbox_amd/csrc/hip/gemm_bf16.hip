@@ -708,8 +708,8 @@ __device__ __forceinline__ void ring_tile(bf16 (&ring)[RING_SLOTS][RBM * RBK], c
         ask(0);
         ask(1);
       }
-      // (what is stored goes by one place that moves on: eight of them at once were more than the registers hold, and 52 bytes a lane
-      // of scratch: 1,157 x 11,280 x 128 18.7 us)
+      // (what is stored goes by one place that moves on: eight of them at once were more than the registers hold: 1,157 x 11,280 x 128
+      // in 32-bit 18.9 / 17.1 us)
       CT* at = c + (size_t)(gm0 + lane % 16) * ldc + gn0 + 4 * (lane / 16);
 #pragma unroll
       for (int i = 0; i < H; ++i) {
@@ -844,7 +844,7 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
   GB_REQUIRE(grid.y <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
   GB_REQUIRE(ring_has(rows.height), "gemm_bf16: no ring kernel for tiles of %d rows (M=%d)", 32 * rows.height, M);
   // as few tiles as there can be: all of 256 rows, the last one as it comes (some of 224 among them end no sooner, and two heights are
-  // two loops to fetch: 1,157 x 11,280 x 128 16.8 / 18.7 us, 2,473 x 2,576 x 13,312 in two slices 190 / 200)
+  // two loops to fetch: 2,473 x 2,576 x 13,312 in two slices 188 / 198 us)
   const int tall = rows.height == 8 && rows.tiles == (M + RBM - 1) / RBM ? rows.tiles : rows.tall;
 #define GB_H(H, SHORT)                                                                                                 \
   if (rows.height == H && (SHORT == H) == (H == 8 && tall == rows.tiles))                                              \
