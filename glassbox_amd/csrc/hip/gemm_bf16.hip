@@ -843,9 +843,11 @@ int launch_ring(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, 
   const dim3 grid(columns, rows.tiles, slices), block(RGM * RGN * 64);
   GB_REQUIRE(grid.y <= 65535, "gemm_bf16: M=%d needs more than 65535 row tiles", M);
   GB_REQUIRE(ring_has(rows.height), "gemm_bf16: no ring kernel for tiles of %d rows (M=%d)", 32 * rows.height, M);
-  // as few tiles as there can be: all of 256 rows, the last one as it comes (some of 224 among them end no sooner, and two heights are
-  // two loops to fetch: 2,473 x 2,576 x 13,312 in two slices 188 / 198 us)
-  const int tall = rows.height == 8 && rows.tiles == (M + RBM - 1) / RBM ? rows.tiles : rows.tall;
+  // as few tiles as there can be, and one round of them: all of 256 rows, the last one as it comes (some of 224 among them end no
+  // sooner, and two heights are two loops to fetch: 2,473 x 2,576 x 13,312 in two slices 188 / 198 us; but eleven rounds, 6,151 x 28,672 x
+  // 4,096 with SiLU-multiply, 1,157 / 1,122)
+  const bool least = rows.height == 8 && rows.tiles == (M + RBM - 1) / RBM && (long long)rows.tiles * columns * slices <= 256;
+  const int tall = least ? rows.tiles : rows.tall;
 #define GB_H(H, SHORT)                                                                                                 \
   if (rows.height == H && (SHORT == H) == (H == 8 && tall == rows.tiles))                                              \
     hipLaunchKernelGGL((gemm_ring_kernel<EPI, CT, false, H, SHORT>), grid, block, 0, stream, a, lda, w, ldw, c, ldc, M, \
