@@ -3,7 +3,7 @@
 // (crates/glassbox-core/src/kernels.rs:381,586).  Both operands are contiguous along k, which
 // is the layout MFMA operands want: every lane loads 8 consecutive k as one 16-byte word.
 //
-// Six kernels:
+// Seven kernels:
 //  * tiled  (M > 64, prompt portions): a workgroup of 2x2 waves, each wave a block of 2x2 or 2x1
 //    v_mfma_f32_32x32x16_bf16 tiles (workgroup tile 128x128 or 128x64; 64 rows high where the taller tiles would be
 //    few), operands staged through LDS in k-steps of 64 with two buffers; the SiLU-multiply of stacked gate/up rows
@@ -12,7 +12,7 @@
 //    straight into LDS several k-steps ahead.
 //  * ring   (257 rows and more, where its tiles of 256 columns by 128 to 256 rows are ahead): 2x2 waves, a wave up to 8x8
 //    tiles of v_mfma_f32_16x16x32_bf16; operands go from memory straight into a ring of LDS buffers in k-steps of 64.
-//  * skinny (M <= 64, decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
+//  * skinny (17 to 64 rows, or up to 64 with the norm on the way; decoding): bound by reading W once.  A workgroup owns 16 or 32 rows of W (8 where the
 //    rows of W are few); its
 //    waves take interleaved 64-wide k blocks, stream W straight from memory into MFMA operands
 //    (v_mfma_f32_16x16x32_bf16, W as the A operand so that the 16 rows fill the tile) and combine
@@ -21,8 +21,8 @@
 //    into the residual.
 //  * held   (17 to 64 rows by many rows of W, decode steps of a busy server): a workgroup a compute unit holds the rows of
 //    A in registers and streams tiles of W through LDS.
-//  * folded (M <= 8 and few rows of W): the skinny kernel with two k ranges side by side in a tile,
-//    so that a workgroup owns 8 rows of W and there are twice as many workgroups.
+//  * few    (M <= 16, decode steps): 8 rows of W over two k ranges side by side in a tile, so that loads bring whole lines, all of
+//    them asked for at once.  (folded: the same tiles with the norm on the way, up to 8 rows by few rows of W.)
 // In all, every output cell is summed in an order fixed by (K, kernel) alone, not by M or by
 // the cell's neighbours.  C is bfloat16 or float32; accumulation (+=) is into float32.
 #include <type_traits>
@@ -60,13 +60,22 @@ __device__ __forceinline__ float gated_unit(float g, float u, const Glu& p) {
   return g / (1.0f + __expf(-(p.alpha * g))) * (u + p.plus);
 }
 
+// A lane's 16 bytes, or zeros where it has nothing to read: then the address is one of zeros, so that a run of loads stays one
+// stretch of code, which a branch round each of them would cut up.  (Named as global memory: of an address that is one of two the
+// compiler cannot tell, and would wait for all loads where it needs the first.)
+__device__ const bf16x8 kZeros = {};
+__device__ __forceinline__ const bf16x8 __attribute__((address_space(1))) * or_zeros(bool ok, const bf16* p) {
+  typedef const bf16x8 __attribute__((address_space(1))) * global_words;
+  return ok ? (global_words)(uintptr_t)p : (global_words)(uintptr_t)&kZeros;
+}
+
 // What a product of at most 64 rows may do for the RMS norm that follows it or precedes it.
-//  * emit (the folded kernel for up to 8 rows, the skinny kernel beyond; accumulating into the float32 residual):
+//  * emit (gemm_few_kernel for up to 16 rows, the skinny kernel beyond; accumulating into the float32 residual):
 //    besides the new residual r it writes h[m, n] = bf16(gamma[n] * r[m, n]), the operand of the next product, and
 //    for every tile of columns (8 or 16: gb_gemm_bf16_emit_parts says how many tiles) the sums over them of
 //    r[m, n]^2 to ss[tile * stride + m]: the next norm's pass over the residual is done where the residual is made.
 //    stride = parts_stride(M): 8 for up to 8 rows, 64 beyond.
-//  * parts (the skinny kernel): the rows of A are such an h; the product is scaled by
+//  * parts (the same two, and the held kernel): the rows of A are such an h; the product is scaled by
 //    1 / sqrt(sum of the n_parts partial sums of row m / K + eps), added up in the order of the tiles.
 __host__ __device__ __forceinline__ int parts_stride(int M) { return M <= 8 ? 8 : 64; }
 struct NormExtras {
@@ -80,7 +89,7 @@ struct NormExtras {
   Glu glu;   // the gated unit of an EPI_SILU_MUL product
 };
 
-// EPI_ROPE (the skinny kernel; the QKV product of a decode step): W stacks nh query heads, nkv key heads
+// EPI_ROPE (gemm_few_kernel, the skinny and the held kernel; the QKV product of a decode step): W stacks nh query heads, nkv key heads
 // and nkv value heads of hd rows each.  The product rotates query and key heads by the angles of each
 // row's position (pairs (i, i + hd/2), crates/glassbox-core/src/model.rs:102-115) while the sums are
 // still 32-bit, writes the stacked rows to C as usual, and the key and value heads straight into the
@@ -94,6 +103,8 @@ struct RopeExtras {
   bf16* v_pages;
   int nh, nkv, hd, page_size;
   int three_halves;  // the launch gives a workgroup a tile and a half (see three_halves_tile), not two tiles
+  float per_tile;    // 8 / hd: heads a tile of 8 rows (the kernel for up to 8 rows of A), and the page size as a shift
+  int page_shift;    // (-1: no power of two)
 };
 
 // Tiles of the skinny kernel's rotating product, 8 pairs each, dealt a tile and a half to a workgroup: workgroup g
@@ -1718,20 +1729,18 @@ __global__ __launch_bounds__(1024) void splitk_reduce_norm_few_kernel(const floa
 inline bool fold_pays(int M, int N) { return M <= 8 && (N + 15) / 16 < 256; }
 
 // What an accumulating product of these sizes can do for the RMS norm that reads the residual after it:
-// 0 nothing; 1 (the folded kernel for at most 8 rows, the skinny kernel up to 64) the operand bf16(gamma * r) and
+// 0 nothing; 1 (gemm_few_kernel for at most 16 rows, the skinny kernel up to 64) the operand bf16(gamma * r) and
 // partial sums, see NormExtras;
 // 2 (a product that divides k, given its workspace) the whole norm, in the pass that adds the slices.
 inline int emit_mode(int M, int N, int K) {
-  if (fold_pays(M, N)) return 1;
   if (M > 16 && N % 4 == 0 && N <= SPLIT_NORM_MAX && split_plan(M, N, K).slices > 1) return 2;
   if (M <= 64 && !(M > 16 && N >= 32768)) return 1;  // the skinny kernel
   return 0;
 }
 // Tiles of columns for which an emitting product of these sizes writes partial sums.
 inline int emit_parts(int M, int N) {
-  if (fold_pays(M, N)) return (N + 7) / 8;
   if (M > 64) return 0;
-  return (N + 15) / 16 < 256 ? (N + 7) / 8 : (N + 15) / 16;  // the skinny kernel: half tiles while the tiles are few
+  return (N + 15) / 16 < 256 ? (N + 7) / 8 : (N + 15) / 16;  // half tiles while the tiles are few
 }
 
 template <int EPI, typename CT>
@@ -1813,8 +1822,8 @@ __device__ __forceinline__ bf16x8 from_lane(bf16x8 v, int lane) {
 template <bool RMS>
 __device__ __forceinline__ bf16x8 load_a(const void* a, int lda, int m, int k, bool ok, const void* gamma, int gamma_f32,
                                          float& ss) {
+  if (!RMS) return *or_zeros(ok, (const bf16*)a + (size_t)m * lda + k);
   if (!ok) return zero8();
-  if (!RMS) return load8((const bf16*)a + (size_t)m * lda + k);
   const float* x = (const float*)a + (size_t)m * lda + k;
   const f32x4 x0 = *reinterpret_cast<const f32x4*>(x), x1 = *reinterpret_cast<const f32x4*>(x + 4);
   float g[8];
@@ -1841,53 +1850,20 @@ __device__ __forceinline__ bf16x8 load_a(const void* a, int lda, int m, int k, b
   return out;
 }
 
-// (Up to 16 rows, sixteen waves, two row tiles and two loads in flight: the kernel needs exactly 64 registers a lane,
-// with which two workgroups share a compute unit, one's loads on their way while the other adds up and stores.  One
-// register more and only one fits: decode steps of one to eight requests were 4 % slower.)
 template <int MT, int WAVES, int ITERS, int RT, int EPI, bool RMS, typename CT, bool HALF = false>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __restrict__ a, int lda,
+__global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_kernel(const void* __restrict__ a, int lda,
                                                                  const bf16* __restrict__ w, int ldw, CT* __restrict__ c,
                                                                  int ldc, int M, int N, int K, const void* __restrict__ gamma,
                                                                  int gamma_f32, float eps, NormExtras extra, RopeExtras rope) {
   __shared__ float part[WAVES][RT][MT][64][4];
   __shared__ float sspart[RMS ? WAVES : 1][MT][64];
-  constexpr int PJ = WAVES * 64 / (MT * 16) < 64 ? WAVES * 64 / (MT * 16) : 64;  // threads that share a row's partial sums
-  __shared__ float red[RMS ? 1 : PJ][MT * 16];  // (with RMS the rows bring no partial sums)
+  constexpr int LR = MT == 1 ? 16 : MT == 2 ? 32 : 64;  // lanes of a wave that stand for different rows in the sums below
+  __shared__ float red[RMS ? 1 : WAVES][MT * 16];       // (with RMS the rows bring no partial sums)
   __shared__ float emit_sq[4][RT][MT][16];
   const float* __restrict__ parts = extra.parts;
   const int n_parts = extra.n_parts;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int r = lane % 16, q = lane / 16;
-  // Partial sums of squares of the rows, one per tile of the product that made them: some threads a row add up
-  // every so-manieth, the epilogue adds up theirs, both in a fixed order.  Up to 8 rows (8 floats a tile): J8 threads a
-  // row, few terms each.  Beyond (64 floats a tile): PJ threads a row, and where a thread has many terms, four loads
-  // at a time are asked for before any is added (one after the other they would each wait).  The first form is kept
-  // as it is on purpose: with it the sixteen-wave kernel needs 64 registers and fits twice on a compute unit, with
-  // the general form alone the compiler keeps one or two more through the main loop.
-  constexpr int J8 = WAVES * 8 < 64 ? WAVES * 8 : 64;
-  float* red8 = &red[0][0];  // [J8][8]
-  if (!RMS && parts != nullptr) {
-    if (M <= 8) {
-      for (int t = tid; t < 8 * J8; t += WAVES * 64) {
-        const int m = t & 7, j = t >> 3;
-        float sum = 0.f;
-        for (int p = j; p < n_parts; p += J8) sum += parts[p * 8 + m];
-        red8[j * 8 + m] = sum;
-      }
-    } else {
-      const int m = tid % (MT * 16), j = tid / (MT * 16);
-      float sum = 0.f;
-      if (m < M && j < PJ)
-        for (int p = j; p < n_parts; p += 4 * PJ) {
-          float got[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) got[u] = p + u * PJ < n_parts ? parts[(p + u * PJ) * 64 + m] : 0.f;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) sum += got[u];
-        }
-      if (j < PJ) red[j][m] = sum;
-    }
-  }
   const bf16* wrow[RT];
   bool row_ok[RT];
 #pragma unroll
@@ -1922,17 +1898,39 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
       for (int e = 0; e < 4; ++e) acc[rt][t][e] = 0.f;
   }
 
+  // Partial sums of squares of the rows, one per tile of the product that made them (64 floats a tile): a lane a row, four loads
+  // asked for at once, before W, and added up behind the requests for W, which so do not wait for them.
+  float got[4] = {0.f, 0.f, 0.f, 0.f};
+  if (!RMS && parts != nullptr && lane % LR < M) {
+    const float* mine = parts + lane % LR;
+    constexpr int STEP = WAVES * 64 / LR;
+    const int p0 = wave * (64 / LR) + lane / LR;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (p0 + u * STEP < n_parts) got[u] = mine[(p0 + u * STEP) * 64];
+    for (int p = p0 + 4 * STEP; p < n_parts; p += STEP) got[0] += mine[p * 64];
+  }
   // a 64-wide k block is two MFMA steps of 32: lane group q holds k = 8q..8q+7 of each
-  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
-    bf16x8 wf[RT][ITERS][2];
+  bf16x8 wf[RT][ITERS][2];
+  auto ask = [&](int kbeg) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
         const int k = kbeg + (wave + WAVES * it) * 64 + q * 8;
-        wf[rt][it][0] = (row_ok[rt] && k < K) ? load8(wrow[rt] + k) : zero8();
-        wf[rt][it][1] = (row_ok[rt] && k + 32 < K) ? load8(wrow[rt] + k + 32) : zero8();
+        wf[rt][it][0] = *or_zeros(row_ok[rt] && k < K, wrow[rt] + k);
+        wf[rt][it][1] = *or_zeros(row_ok[rt] && k + 32 < K, wrow[rt] + k + 32);
       }
+  };
+  ask(0);
+  if (!RMS && parts != nullptr) {
+    float sum = ((got[0] + got[1]) + got[2]) + got[3];
+#pragma unroll
+    for (int o = LR; o < 64; o <<= 1) sum += __shfl_xor(sum, o, kWave);
+    if (lane < LR && lane < MT * 16) red[wave][lane] = sum;
+  }
+  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
+    if (kbeg > 0) ask(kbeg);
     if (MT == 1) {
       bf16x8 xf[ITERS][2];
 #pragma unroll
@@ -1941,6 +1939,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
         xf[it][0] = load_a<RMS>(a, lda, r, k, r < M && k < K, gamma, gamma_f32, ss[0]);
         xf[it][1] = load_a<RMS>(a, lda, r, k + 32, r < M && k + 32 < K, gamma, gamma_f32, ss[0]);
       }
+      if (!RMS) __builtin_amdgcn_sched_barrier(0);   // all loads of a slice are asked for before the first is waited for
 #pragma unroll
       for (int it = 0; it < ITERS; ++it)
 #pragma unroll
@@ -2048,15 +2047,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
       scale = 1.0f / sqrtf(tot / (float)K + eps);
     } else if (parts != nullptr) {
       float tot = 0.f;
-      if (M <= 8) {
-        if (l % 16 < 8) {
-#pragma unroll 8
-          for (int j = 0; j < J8; ++j) tot += red8[j * 8 + l % 16];
-        }
-      } else {
-#pragma unroll 8
-        for (int j = 0; j < PJ; ++j) tot += red[j][t * 16 + l % 16];
-      }
+#pragma unroll
+      for (int wv = 0; wv < WAVES; ++wv) tot += red[wv][t * 16 + l % 16];
       scale = 1.0f / sqrtf(tot / (float)K + eps);
     }
 #pragma unroll
@@ -2176,27 +2168,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
   }
 }
 
-// ------------------------------------------------------------------------ folded (M <= 8)
-// With at most 8 rows of A, a 16 x 16 tile has room for two k ranges side by side.  Rows 0..7 of the
-// tile are 8 rows of W over one part of a 128-wide k block (k 0..31 and 64..95 of it) and rows 8..15 the same
-// 8 rows of W over the other (k 32..63 and 96..127); columns 0..7 are the rows of A over the first part,
-// columns 8..15 over the second.  Cells (n, m) and (n + 8, m + 8) then hold the two halves of one sum; the other two
-// quarters of the tile pair the wrong halves and are dropped.  A workgroup so owns 8 rows of W, not
-// 16, and a product with few rows of W (decoding: the O and down projections) has a workgroup for
-// every compute unit: one compute unit draws only a fraction of the memory bandwidth.  The halves of a lane's two
-// loads are chosen so that one load instruction of the wave reads whole 128-byte lines of its 8 rows (k 0..63 of
-// the block, then 64..127), and the loads are nontemporal: W is read once (the down projection of the
-// SmolLM2-1.7B shapes at 8 rows 11.0 -> 10.3 us, the O projection 5.1 -> 4.7; with half lines an instruction,
-// nontemporal loads were slower than plain ones).
-template <int WAVES, int ITERS, int RT, int EPI, bool RMS, typename CT>
-__global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __restrict__ a, int lda,
-                                                               const bf16* __restrict__ w, int ldw, CT* __restrict__ c,
-                                                               int ldc, int M, int N, int K, const void* __restrict__ gamma,
-                                                               int gamma_f32, float eps, NormExtras extra) {
-  static_assert(EPI != EPI_SILU_MUL && WAVES >= 4, "folded tiles store or accumulate; the first four waves finish");
+// ------------------------------------------------------------------------ folded (M <= 8, with the norm)
+// At most 8 rows of A that are still to be normed by few rows of W (a first layer's product): the tiles of gemm_few_kernel below,
+// 8 rows of W over two k ranges (k 0..31 and 64..95 of a 128-wide block, and 32..63 and 96..127), in waves that gather the sum of
+// squares on the way (load_a).  The loads are nontemporal: W is read once.
+template <int WAVES, int ITERS, int RT>
+__global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __restrict__ a, int lda, const bf16* __restrict__ w, int ldw,
+                                                               bf16* __restrict__ c, int ldc, int M, int N, int K,
+                                                               const void* __restrict__ gamma, int gamma_f32, float eps) {
+  static_assert(WAVES >= 4, "the first four waves finish");
   __shared__ float part[WAVES][RT][64][4];
-  __shared__ float sspart[RMS ? WAVES : 1][64];
-  __shared__ float squares[RT][8][8];
+  __shared__ float sspart[WAVES][64];
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int r = lane % 16, q = lane / 16;
   const int r8 = r & 7, khalf = (r >> 3) * 32;  // row of W and of A; which quarter of a k block: a load of the wave reads whole 128-byte lines
@@ -2214,25 +2196,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __res
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[rt][e] = 0.f;
-
-  // D[n, m]: lane l holds column m = l%16 and rows n = 4*(l/16) + e; thread tid of the first four waves owns cell
-  // (l = tid/4, e = tid%4) at the end.  What it will need from memory then (the cell's old value, the gamma of a norm
-  // to prepare) is asked for now, so that it arrives under the stream of W and not after it.
-  const int l = (tid % 256) / 4, e = tid % 4;
-  const int nrow = 4 * (l / 16) + e, m = l % 16;
-  const bool emits = EPI == EPI_ACCUMULATE && extra.emit_h != nullptr;
-  const bool mine = tid < 256 && nrow < 8 && m < 8;
-  float old[RT], emit_g[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int n = (blockIdx.x * RT + rt) * 8 + nrow;
-    old[rt] = emit_g[rt] = 0.f;
-    if (mine && m < M && n < N) {
-      if (EPI == EPI_ACCUMULATE) old[rt] = (float)c[(size_t)m * ldc + n];
-      if (emits) emit_g[rt] = extra.emit_gamma_f32 ? ((const float*)extra.emit_gamma)[n] : (float)((const bf16*)extra.emit_gamma)[n];
-    }
-  }
-
   for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 128) {
     bf16x8 wf[RT][ITERS][2], xf[ITERS][2];
 #pragma unroll
@@ -2240,14 +2203,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __res
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
         const int k = kbeg + (wave + WAVES * it) * 128 + khalf + q * 8;
-        wf[rt][it][0] = (row_ok[rt] && k < K) ? load8_once(wrow[rt] + k) : zero8();
-        wf[rt][it][1] = (row_ok[rt] && k + 64 < K) ? load8_once(wrow[rt] + k + 64) : zero8();
+        wf[rt][it][0] = __builtin_nontemporal_load(or_zeros(row_ok[rt] && k < K, wrow[rt] + k));
+        wf[rt][it][1] = __builtin_nontemporal_load(or_zeros(row_ok[rt] && k + 64 < K, wrow[rt] + k + 64));
       }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const int k = kbeg + (wave + WAVES * it) * 128 + khalf + q * 8;
-      xf[it][0] = load_a<RMS>(a, lda, r8, k, r8 < M && k < K, gamma, gamma_f32, ss);
-      xf[it][1] = load_a<RMS>(a, lda, r8, k + 64, r8 < M && k + 64 < K, gamma, gamma_f32, ss);
+      xf[it][0] = load_a<true>(a, lda, r8, k, r8 < M && k < K, gamma, gamma_f32, ss);
+      xf[it][1] = load_a<true>(a, lda, r8, k + 64, r8 < M && k + 64 < K, gamma, gamma_f32, ss);
     }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it)
@@ -2261,74 +2224,332 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __res
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) part[wave][rt][lane][e] = acc[rt][e];
-  if (RMS) sspart[wave][lane] = ss;
+  sspart[wave][lane] = ss;
   __syncthreads();
-  if (tid >= 256) return;
-  if (!mine && !emits) return;
-  float scale = 1.f;
-  if (RMS && mine) {
-    // sum(x^2) of row m: its k were spread over the waves, the four lane groups and the two halves
-    float tot = 0.f;
+  // D[n, m]: lane l holds column m = l%16 and rows n = 4*(l/16) + e; thread tid of the first four waves owns cell
+  // (l = tid/4, e = tid%4)
+  const int l = (tid % 256) / 4, e = tid % 4;
+  const int nrow = 4 * (l / 16) + e, m = l % 16;
+  if (tid >= 256 || nrow >= 8 || m >= M) return;
+  // sum(x^2) of row m: its k were spread over the waves, the four lane groups and the two halves
+  float tot = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv)
+  for (int wv = 0; wv < WAVES; ++wv)
 #pragma unroll
-      for (int qq = 0; qq < 4; ++qq) tot += sspart[wv][m + 16 * qq] + sspart[wv][m + 8 + 16 * qq];
-    scale = 1.0f / sqrtf(tot / (float)K + eps);
-  }
+    for (int qq = 0; qq < 4; ++qq) tot += sspart[wv][m + 16 * qq] + sspart[wv][m + 8 + 16 * qq];
+  const float scale = 1.0f / sqrtf(tot / (float)K + eps);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int n = (blockIdx.x * RT + rt) * 8 + nrow;
-    float now = 0.f;  // the cell's new value
-    if (mine && m < M && n < N) {
-      float sum = 0.f;
+    if (n >= N) continue;
+    float sum = 0.f;
 #pragma unroll
-      for (int wv = 0; wv < WAVES; ++wv) sum += part[wv][rt][l][e] + part[wv][rt][l + 40][e];  // cell (n + 8, m + 8)
-      now = EPI == EPI_ACCUMULATE ? old[rt] + sum * scale : sum * scale;
-      c[(size_t)m * ldc + n] = (CT)now;
-      if (emits) extra.emit_h[(size_t)m * extra.emit_ldh + n] = (bf16)(emit_g[rt] * now);
-    }
-    if (emits && mine) squares[rt][m][nrow] = now * now;
-  }
-  if (!emits) return;
-  __syncthreads();  // the waves that are still here
-  if (mine && nrow == 0) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      float tot = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) tot += squares[rt][m][j];
-      extra.emit_ss[(size_t)(blockIdx.x * RT + rt) * 8 + m] = tot;
-    }
+    for (int wv = 0; wv < WAVES; ++wv) sum += part[wv][rt][l][e] + part[wv][rt][l + 40][e];  // cell (n + 8, m + 8)
+    c[(size_t)m * ldc + n] = (bf16)(sum * scale);
   }
 }
 
-template <int EPI, bool RMS, typename CT>
-int launch_fold(const void* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, const void* gamma,
-                int gamma_f32, float eps, const NormExtras& extra, hipStream_t stream) {
+inline int launch_fold(const void* a, int lda, const bf16* w, int ldw, bf16* c, int ldc, int M, int N, int K, const void* gamma,
+                       int gamma_f32, float eps, hipStream_t stream) {
   const int tiles = (N + 7) / 8, blocks = (K + 127) / 128;  // 128-wide k blocks
   const int waves = blocks >= 16 ? 16 : 4;  // (eight blocks on sixteen waves were measured no faster than on four)
   const int rt = tiles >= 512 ? 2 : 1;
   const int iters = (blocks + waves - 1) / waves >= 2 ? 2 : 1;  // four loads in flight a wave were measured no faster
 #define GB_CFG(WV, IT, RT)                                                                                                \
   if (waves == WV && iters == IT && rt == RT)                                                                             \
-    hipLaunchKernelGGL((gemm_fold_kernel<WV, IT, RT, EPI, RMS, CT>), dim3((tiles + RT - 1) / RT), dim3(WV * 64), 0, stream, \
-                       a, lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra);
+    hipLaunchKernelGGL((gemm_fold_kernel<WV, IT, RT>), dim3((tiles + RT - 1) / RT), dim3(WV * 64), 0, stream, a, lda, w, ldw, c, \
+                       ldc, M, N, K, gamma, gamma_f32, eps);
   GB_CFG(4, 1, 1) GB_CFG(4, 1, 2) GB_CFG(4, 2, 1) GB_CFG(4, 2, 2)
   GB_CFG(16, 1, 1) GB_CFG(16, 1, 2) GB_CFG(16, 2, 1) GB_CFG(16, 2, 2)
 #undef GB_CFG
   return launched("gemm_bf16 (folded)");
 }
 
-// Waves per workgroup, loads in flight per wave and row tiles per workgroup.
+// -------------------------------------------------------------------------- few (M <= 16)
+// Decode steps of up to sixteen requests.  A tile is 8 rows of W whose two ranges of 32 of a 64-wide k block stand side by side
+// in a 16 x 16 MFMA tile (rows n and n + 8 the same row of W, columns m and m + 8 the same row of A, each over its own range; the
+// cells (n, m) and (n + 8, m + 8) are the halves of a sum, the other two quarters are dropped), so that a load instruction of a
+// wave reads whole 128-byte lines of 8 rows (bare reads of 16,384 x 2,048 in half lines of 16 rows 13.0 us, in whole lines,
+// nontemporal, 11.4).  MB blocks of 8 rows of A share W's words.
+// Such a kernel lasts a few microseconds and is made of trips to memory one behind the other, so everything that it reads is asked
+// for before the first of it is waited for: the partial sums of the norm before it (a word of four rows a thread), what the
+// epilogue needs, W and the rows of A, up to a k of 2,048 at once (longer ones in turns).  Rows of W that the rotation or the
+// gated unit pairs lie in one tile, four pairs, the partners mirrored (row n and 7 - n), and a cell's partner and a row's squares
+// come by lane moves: one barrier in all.   parts / emit / rotation: as NormExtras and RopeExtras say.
+// In steps of one row (of eight), the kernels before (16 rows of W a tile in half lines, partial sums one behind the other before
+// W; 8 rows for the products by few rows of W) and now: SmolLM2-1.7B gate/up 13.9 -> 12.5 us (15.6 -> 13.8), QKV 9.5 -> 7.1
+// (10.1 -> 8.1), down 9.2 -> 8.0 (11.0 -> 10.5), vocabulary 35.7 -> 31.3 (40.4 -> 34.4); SmolLM2-135M a layer 17.3 -> 14.5.
+__device__ __forceinline__ float lane_mirror8(float v) {   // the value of lane 7 - n of the eight neighbouring lanes
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ float lane_quad(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// lanes (g, i) with g < 2 and i < 8 of a 16 x 16 result: v + the cell eight rows and eight columns further on
+__device__ __forceinline__ float plus_folded(float v) {
+  const unsigned t = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true);   // lane i + 8 of the row of 16
+  const auto halves = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+  const unsigned upper = halves[1];                                                                      // of the upper half of the wave
+  return v + __builtin_bit_cast(float, upper);
+}
+
+template <int MB, int WAVES, int ITERS, int RT, int EPI, typename CT>
+__global__ __launch_bounds__(WAVES * 64, WAVES >= 8 ? 4 : 1) void gemm_few_kernel(
+    const bf16* __restrict__ a, const bf16* __restrict__ w, const float* __restrict__ parts, int lda, int ldw, int M, int N, int K, int n_parts,
+    CT* __restrict__ c, int ldc, float eps, NormExtras extra, RopeExtras rope) {
+  static_assert(EPI != EPI_ACCUMULATE || RT != 3, "partial sums of two tiles meet");
+  constexpr int CELLS = RT * MB, OWN = (CELLS + WAVES - 1) / WAVES;   // blocks of 8 x 8 cells; those that a wave finishes
+  constexpr bool PAIRS = EPI == EPI_ACCUMULATE && RT > 1;             // partial sums of 16 columns
+  __shared__ __attribute__((aligned(16))) float part[WAVES][CELLS][64];   // [row of A][row of the tile]
+  __shared__ __attribute__((aligned(16))) float red[WAVES][8 * MB];
+  __shared__ float squares[PAIRS ? CELLS : 1][8];
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int r8 = lane & 7, kpos = ((lane >> 3) & 1) * 32 + (lane >> 4) * 8;
+  // words of four rows' partial sums: of up to 8 rows 8 floats a tile, beyond 64 of which 16 are wanted
+  f32x4 got = {0.f, 0.f, 0.f, 0.f};
+  if (parts != nullptr) {
+    auto word = [&](int i) { return *reinterpret_cast<const f32x4*>(parts + (MB == 1 ? 4 * i : 64 * (i >> 2) + 4 * (i & 3))); };
+    if (tid < 2 * MB * n_parts) got = word(tid);
+    for (int i = tid + WAVES * 64; i < 2 * MB * n_parts; i += WAVES * 64) got += word(i);
+  }
+  // the pair of row n of a tile whose rows are four pairs
+  auto pair_of = [](int n) { return n < 4 ? n : 7 - n; };
+  auto head_of = [&](int tile) { return (int)(((float)tile + 0.5f) * rope.per_tile); };   // tile / (hd / 8), exact below 2^21 tiles
+  // the cells of this lane in the epilogue: row n of tile cell / MB, row m of A in block cell % MB
+  const int n = lane & 7;
+  float old[OWN], gamma[OWN], cs[OWN], sn[OWN];
+  int slot[OWN], head[OWN], pair[OWN];
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int cell = wave + WAVES * i, own = blockIdx.x * RT + cell / MB, m = cell % MB * 8 + (lane >> 3);
+    old[i] = gamma[i] = sn[i] = 0.f;
+    cs[i] = 1.f;
+    slot[i] = head[i] = pair[i] = 0;
+    if (cell >= CELLS) continue;
+    if (EPI == EPI_ACCUMULATE && m < M && own * 8 + n < N) {
+      old[i] = (float)c[(size_t)m * ldc + own * 8 + n];
+      if (extra.emit_h != nullptr)
+        gamma[i] = extra.emit_gamma_f32 ? ((const float*)extra.emit_gamma)[own * 8 + n] : (float)((const bf16*)extra.emit_gamma)[own * 8 + n];
+    }
+    if (EPI == EPI_ROPE) {
+      head[i] = head_of(own);
+      pair[i] = (own - head[i] * (rope.hd / 8)) * 4 + pair_of(n);
+      if (m < M && own * 8 < N) {
+        if (rope.slots != nullptr) slot[i] = rope.slots[m];
+        if (rope.cosv != nullptr && head[i] < rope.nh + rope.nkv) {
+          cs[i] = rope.cosv[(size_t)m * (rope.hd / 2) + pair[i]];
+          sn[i] = rope.sinv[(size_t)m * (rope.hd / 2) + pair[i]];
+        }
+      }
+    }
+  }
+  // (rows beyond N or M are read from one that exists: what comes of them is not stored)
+  const bf16* wrow[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int tile = blockIdx.x * RT + rt;
+    int row;
+    if (EPI == EPI_SILU_MUL) {
+      const int j = min(tile * 4 + pair_of(r8), N / 2 - 1);
+      row = r8 < 4 ? j : N / 2 + j;
+    } else if (EPI == EPI_ROPE) {
+      const int h = head_of(tile);
+      row = min(h * rope.hd + (tile - h * (rope.hd / 8)) * 4 + pair_of(r8) + (r8 < 4 ? 0 : rope.hd / 2), N - 1);
+    } else {
+      row = min(tile * 8 + r8, N - 1);
+    }
+    wrow[rt] = w + (size_t)row * ldw + kpos;
+  }
+  const bf16* xrow[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) xrow[mb] = a + (size_t)min(mb * 8 + r8, M - 1) * lda + kpos;
+  f32x4 acc[RT][MB];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[rt][mb][e] = 0.f;
+
+  // A wave's 64-wide blocks of a turn: every WAVES-th, so that the waves read side by side (one row by 16,384 x 2,048 12.3 us, in runs
+  // 13.3); of a short k, where that makes no difference, a run of neighbouring ones
+  auto block_of = [&](int it) { return WAVES == 4 ? wave * ITERS + it : wave + WAVES * it; };
+  constexpr int TURN = ITERS * WAVES * 64;
+  for (int kbeg = 0; kbeg < K; kbeg += TURN) {
+    bf16x8 wf[RT][ITERS], xf[MB][ITERS];
+    if (kbeg + TURN <= K) {
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const int k = kbeg + block_of(it) * 64;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) wf[rt][it] = load8_once(wrow[rt] + k);
+      }
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) xf[mb][it] = load8(xrow[mb] + kbeg + block_of(it) * 64);
+    } else {  // the last turn of a k that is not of whole turns: zeros beyond it
+#pragma unroll
+      for (int it = 0; it < ITERS; ++it) {
+        const int k = kbeg + block_of(it) * 64;
+        const bool ok = k + kpos < K;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) wf[rt][it] = __builtin_nontemporal_load(or_zeros(ok, wrow[rt] + k));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) xf[mb][it] = *or_zeros(ok, xrow[mb] + k);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);   // all loads of a turn are asked for before the first is waited for
+    if (kbeg == 0 && parts != nullptr) {
+#pragma unroll
+      for (int o = 2 * MB; o < 64; o <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) got[e] += __shfl_xor(got[e], o, kWave);
+      if (lane < 2 * MB) *reinterpret_cast<f32x4*>(&red[wave][4 * lane]) = got;
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[rt][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[rt][it], xf[mb][it], acc[rt][mb], 0, 0, 0);
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = plus_folded(acc[rt][mb][e]);
+      if (lane < 32 && (lane & 15) < 8) *reinterpret_cast<f32x4*>(&part[wave][rt * MB + mb][(lane & 7) * 8 + 4 * (lane >> 4)]) = v;
+    }
+  __syncthreads();
+  if (wave >= CELLS) return;
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int cell = wave + WAVES * i, own = blockIdx.x * RT + cell / MB, m = cell % MB * 8 + (lane >> 3);
+    if (cell >= CELLS) continue;
+    float v = part[0][cell][lane];
+#pragma unroll
+    for (int wv = 1; wv < WAVES; ++wv) v += part[wv][cell][lane];
+    if (parts != nullptr) {
+      float tot = red[0][m];
+#pragma unroll
+      for (int wv = 1; wv < WAVES; ++wv) tot += red[wv][m];
+      v *= 1.0f / sqrtf(tot / (float)K + eps);
+    }
+    if (EPI == EPI_SILU_MUL) {
+      const float u = lane_mirror8(v);
+      if (m < M && n < 4 && own * 4 + n < N / 2) c[(size_t)m * ldc + own * 4 + n] = (CT)gated_unit(v, u, extra.glu);
+    } else if (EPI == EPI_ROPE) {
+      const float p = lane_mirror8(v);
+      if (m >= M || own * 8 >= N) continue;
+      const int half = rope.hd / 2, dim = n < 4 ? pair[i] : half + pair[i];
+      const bf16 yb = (bf16)(n < 4 ? v * cs[i] - p * sn[i] : v * cs[i] + p * sn[i]);
+      c[(size_t)m * ldc + head[i] * rope.hd + dim] = (CT)yb;
+      if (rope.slots != nullptr && head[i] >= rope.nh) {
+        const int page = rope.page_shift >= 0 ? slot[i] >> rope.page_shift : slot[i] / rope.page_size, off = slot[i] - page * rope.page_size;
+        if (head[i] < rope.nh + rope.nkv)
+          rope.k_pages[((size_t)page * rope.nkv + (head[i] - rope.nh)) * rope.page_size * rope.hd + key_offset(off, dim, rope.page_size, 8)] = yb;
+        else
+          rope.v_pages[(((size_t)page * rope.nkv + (head[i] - rope.nh - rope.nkv)) * rope.hd + dim) * rope.page_size + off] = yb;
+      }
+    } else {
+      const int col = own * 8 + n;
+      const bool mine = m < M && col < N;
+      const float now = EPI == EPI_ACCUMULATE ? old[i] + v : v;
+      if (mine) c[(size_t)m * ldc + col] = (CT)now;
+      if (EPI == EPI_ACCUMULATE && extra.emit_h != nullptr) {
+        if (mine) extra.emit_h[(size_t)m * extra.emit_ldh + col] = (bf16)(gamma[i] * now);
+        float sq = mine ? now * now : 0.f;   // the squares of a row over the tile's columns, in a fixed order
+        sq += lane_mirror8(sq);
+        sq += lane_quad<0xB1>(sq);
+        sq += lane_quad<0x4E>(sq);
+        if (PAIRS) {
+          if (n == 0) squares[cell][lane >> 3] = sq;
+        } else if (n == 0 && m < M && own * 8 < N) {
+          extra.emit_ss[(size_t)own * (MB == 1 ? 8 : 64) + m] = sq;
+        }
+      }
+    }
+  }
+  if (PAIRS && extra.emit_h != nullptr) {
+    __syncthreads();  // the waves that are still here
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int cell = wave + WAVES * i, own = blockIdx.x * RT + cell / MB, m = cell % MB * 8 + (lane >> 3);
+      if (cell < CELLS && cell / MB % 2 == 0 && n == 0 && m < M && own * 8 < N)
+        extra.emit_ss[(size_t)(own / 2) * (MB == 1 ? 8 : 64) + m] = squares[cell][lane >> 3] + squares[cell + MB][lane >> 3];
+    }
+  }
+}
+
+// How a product of up to 16 rows is cut: tiles a workgroup, its waves, and the 64-wide k blocks a wave asks for at once.
+struct FewPlan {
+  int rt, waves, iters;
+};
+inline FewPlan few_plan(int epi, int M, int N, int K) {
+  const int tiles = epi == EPI_SILU_MUL ? (N / 2 + 3) / 4 : (N + 7) / 8, blocks = (K + 63) / 64;
+  FewPlan p;
+  // A workgroup for every compute unit, and no more than four tiles each (accumulating: two tiles where emit_parts() has sums of 16
+  // columns).  Beyond 8 rows the rows of A are as much traffic as W: as many tiles a workgroup as its registers hold (12 rows by
+  // 16,384 x 2,048 with two tiles 16.2 us, four 15.3; by 6,144 x 4,096 two 16.2, three 12.6).
+  if (epi == EPI_ACCUMULATE) p.rt = (N + 15) / 16 < 256 ? 1 : tiles < 1024 ? 2 : 4;
+  else p.rt = tiles < (M > 8 ? 256 : 512) ? 1 : tiles < 768 ? 2 : tiles < 1024 ? 3 : 4;
+  // All of k at once where the registers hold it: a second turn of the loop begins behind the first one's last bytes (one row by
+  // 960 x 2,560: 40 blocks in one turn of eight waves 3.77 us, in one of sixteen with a third of them empty 4.26).
+  if (blocks <= 8) p.waves = 4, p.iters = 2;
+  else if (blocks <= 12 && (M <= 8 || p.rt == 1)) p.waves = 4, p.iters = 3;
+  else if (blocks <= 16 || (M > 8 && p.rt > 3)) p.waves = 8, p.iters = 2;
+  else if (blocks <= 32 || p.rt > 2) p.waves = 8, p.iters = 4;
+  else if (blocks <= 40 && M <= 8 && p.rt == 1) p.waves = 8, p.iters = 5;
+  else p.waves = 16, p.iters = blocks <= 64 || p.rt == 2 || M > 8 ? 4 : 8;
+  return p;
+}
+
+template <int MB, int EPI, typename CT>
+int launch_few_mb(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, float eps, const NormExtras& extra,
+                  hipStream_t stream, const RopeExtras& rope) {
+  const int tiles = EPI == EPI_SILU_MUL ? (N / 2 + 3) / 4 : (N + 7) / 8;
+  const FewPlan p = few_plan(EPI, M, N, K);
+  bool found = false;
+#define GB_FEW(WV, IT, R)                                                                                                     \
+  if constexpr (!(EPI == EPI_ACCUMULATE && R == 3))                                                                           \
+    if (p.waves == WV && p.iters == IT && p.rt == R) {                                                                        \
+      found = true;                                                                                                           \
+      hipLaunchKernelGGL((gemm_few_kernel<MB, WV, IT, R, EPI, CT>), dim3((tiles + R - 1) / R), dim3(WV * 64), 0, stream, a, w, \
+                         extra.parts, lda, ldw, M, N, K, extra.n_parts, c, ldc, eps, extra, rope);                            \
+    }
+#define GB_FEWS(WV, IT) GB_FEW(WV, IT, 1) GB_FEW(WV, IT, 2) GB_FEW(WV, IT, 3) GB_FEW(WV, IT, 4)
+  GB_FEWS(4, 2) GB_FEWS(4, 3) GB_FEWS(8, 2) GB_FEW(8, 4, 1) GB_FEW(8, 4, 2) GB_FEW(8, 4, 3) GB_FEW(16, 4, 1) GB_FEW(16, 4, 2)
+  if constexpr (MB == 1) { GB_FEW(8, 4, 4) GB_FEW(8, 5, 1) GB_FEW(16, 8, 1) }
+#undef GB_FEWS
+#undef GB_FEW
+  GB_REQUIRE(found, "gemm_bf16: no kernel of %d tiles, %d waves and %d blocks for up to 16 rows", p.rt, p.waves, p.iters);
+  return launched("gemm_bf16 (few rows)");
+}
+
+template <int EPI, typename CT>
+int launch_few(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K, float eps, const NormExtras& extra,
+               hipStream_t stream, const RopeExtras& rope = RopeExtras{}) {
+  RopeExtras rp = rope;
+  if (EPI == EPI_ROPE) {
+    rp.per_tile = 8.0f / (float)rope.hd;
+    rp.page_shift = rope.page_size > 0 && (rope.page_size & (rope.page_size - 1)) == 0 ? __builtin_ctz(rope.page_size) : -1;
+  }
+  if (M <= 8) return launch_few_mb<1, EPI, CT>(a, lda, w, ldw, c, ldc, M, N, K, eps, extra, stream, rp);
+  return launch_few_mb<2, EPI, CT>(a, lda, w, ldw, c, ldc, M, N, K, eps, extra, stream, rp);
+}
+
+// Waves per workgroup, k blocks in flight per wave and row tiles per workgroup.
 inline void skinny_plan(int tiles, int K, int mt, int* waves, int* iters, int* rt) {
-  // measured on SmolLM2-1.7B and Llama-3-8B shapes: sixteen waves a workgroup keep the most loads in
-  // flight; two row tiles a workgroup halve the re-reading of A once that still leaves workgroups for
+  // two row tiles a workgroup halve the re-reading of A once that still leaves workgroups for
   // three quarters of the compute units (384 tiles: better with two; 256 tiles: better with one)
   const int blocks = (K + 63) / 64;               // 64-wide k blocks
+  *rt = tiles >= 384 ? 2 : 1;
   // A wave's k blocks come one after the other, each a round trip to memory: from twelve blocks on sixteen waves take
   // one or two each (a k of 960, fifteen blocks: a decode step of SmolLM2-360M 4 to 8 % faster than with four waves)
   *waves = blocks >= 12 ? 16 : 4;
-  *rt = tiles >= 384 ? 2 : 1;
   const int per_wave = (blocks + *waves - 1) / *waves;
   *iters = (mt == 1 && per_wave >= 2) ? 2 : 1;
 }
@@ -2349,7 +2570,7 @@ int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, 
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, (IT), 1, EPI, RMS, CT, true>), dim3(halves), dim3(WV * 64), 0, stream, a, \
                        lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rope);
       GB_HALF(4, 1) GB_HALF(16, 1)
-      if (MT == 1) { GB_HALF(4, MT == 1 ? 2 : 1) GB_HALF(16, MT == 1 ? 2 : 1) }
+      if constexpr (MT == 1) { GB_HALF(4, 2) GB_HALF(16, 2) }
 #undef GB_HALF
       return launched("gemm_bf16 (skinny, half tiles)");
     }
@@ -2362,11 +2583,9 @@ int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, 
   if (waves == WV && iters == (IT) && rt == RT)                                                                            \
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, (IT), RT, EPI, RMS, CT>), dim3(groups), dim3(WV * 64), 0, stream, a, lda, \
                        w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rp);
-  // the configurations skinny_plan can ask for: two loads in flight only with one column block
+  // the configurations skinny_plan can ask for
   GB_CFG(4, 1, 1) GB_CFG(4, 1, 2) GB_CFG(16, 1, 1) GB_CFG(16, 1, 2)
-  if (MT == 1) {
-    GB_CFG(4, MT == 1 ? 2 : 1, 1) GB_CFG(4, MT == 1 ? 2 : 1, 2) GB_CFG(16, MT == 1 ? 2 : 1, 1) GB_CFG(16, MT == 1 ? 2 : 1, 2)
-  }
+  if constexpr (MT == 1) { GB_CFG(4, 2, 1) GB_CFG(4, 2, 2) GB_CFG(16, 2, 1) GB_CFG(16, 2, 2) }
 #undef GB_CFG
   return launched("gemm_bf16 (skinny)");
 }
@@ -2378,13 +2597,15 @@ int launch_skinny(const void* a, int lda, const bf16* w, int ldw, CT* c, int ldc
   const int mt = (M + 15) / 16;
 #define GB_MT(T) \
   if (mt == T) return launch_skinny_mt<T, EPI, RMS, CT>(tiles, a, lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rope, stream);
-  GB_MT(1) GB_MT(2) GB_MT(3)
+  if constexpr (RMS) { GB_MT(1) }   // (up to 16 rows that are normed already: gemm_few_kernel)
+  GB_REQUIRE(mt > 1, "gemm_bf16: the skinny kernel takes up to 16 rows with the norm alone");
+  GB_MT(2) GB_MT(3)
 #undef GB_MT
   return launch_skinny_mt<4, EPI, RMS, CT>(tiles, a, lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rope, stream);
 }
 
 // Which kernel takes a product, and how.  `emits`: emit_mode if the next norm is to be prepared, else 0; `workspace`: one is there.
-enum : int { kTiled = 0, kRing = 1, kFew = 2 /* skinny or folded */, kHeld = 3, kBlock = 4, kSlices = 5 };
+enum : int { kTiled = 0, kRing = 1, kFew = 2 /* few, skinny or folded */, kHeld = 3, kBlock = 4, kSlices = 5 };
 struct Route {
   int kernel;
   BlockPlan block;   // the block kernel's tile for the whole product, where it may take it
@@ -2531,11 +2752,14 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
 #undef GB_SP
 #undef GB_EACH
   const int gf = gamma_dtype == kF32;
-  if (fold_pays(M, N) && epilogue != EPI_SILU_MUL && !parts) {
-    if (gamma) return launch_fold<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
-    if (epilogue == EPI_ACCUMULATE) return launch_fold<EPI_ACCUMULATE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
-    if (c_dtype == kF32) return launch_fold<EPI_STORE, false, float>(a, lda, W, ldw, (float*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
-    return launch_fold<EPI_STORE, false, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
+  if (gamma && fold_pays(M, N) && epilogue != EPI_SILU_MUL)
+    return launch_fold(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, stream);
+  if (!gamma && M <= 16) {
+    if (epilogue == EPI_ACCUMULATE) return launch_few<EPI_ACCUMULATE, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, eps, extra, stream);
+    if (epilogue == EPI_SILU_MUL && c_dtype == kBF16) return launch_few<EPI_SILU_MUL, bf16>(A, lda, W, ldw, (bf16*)c, ldc, M, N, K, eps, extra, stream);
+    if (epilogue == EPI_SILU_MUL) return launch_few<EPI_SILU_MUL, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, eps, extra, stream);
+    if (c_dtype == kF32) return launch_few<EPI_STORE, float>(A, lda, W, ldw, (float*)c, ldc, M, N, K, eps, extra, stream);
+    return launch_few<EPI_STORE, bf16>(A, lda, W, ldw, (bf16*)c, ldc, M, N, K, eps, extra, stream);
   }
   if (gamma) {
     if (epilogue == EPI_STORE) return launch_skinny<EPI_STORE, true, bf16>(a, lda, W, ldw, (bf16*)c, ldc, M, N, K, gamma, gf, eps, extra, stream);
@@ -2561,6 +2785,7 @@ extern "C" int gb_gemm_bf16_glu(const void* a, int lda, const void* w, int ldw, 
   const Glu glu{limit, alpha, plus};
   if (M <= 64) {
     const NormExtras extra{nullptr, 0, nullptr, 0, nullptr, nullptr, 0, glu};
+    if (M <= 16) return launch_few<EPI_SILU_MUL, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, 0.f, extra, stream);
     return launch_skinny<EPI_SILU_MUL, false, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, 0.f, extra, stream);
   }
   if (ring_pays(EPI_SILU_MUL, a, lda, w, ldw, M, N, K))
@@ -2642,12 +2867,13 @@ extern "C" int gb_gemm_bf16_rope(const void* a, int lda, const void* w, int ldw,
              "gemm_bf16_rope: gamma must be aligned float32 or bfloat16, and not given together with parts");
   GB_REQUIRE(!parts || n_parts > 0, "gemm_bf16_rope: partial sums of a norm without a count");
   const NormExtras extra{nullptr, 0, nullptr, 0, nullptr, parts, n_parts};
-  const RopeExtras rope{cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, 0};
+  const RopeExtras rope{cosv, sinv, slots, (bf16*)k_pages, (bf16*)v_pages, nh, nkv, hd, page_size, 0, 0.f, -1};
   if (!gamma && held_pays(EPI_ROPE, M, N, K, parts != nullptr) && held_takes(a, lda, w, ldw, M, K))
     return launch_held<EPI_ROPE, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, 0, 1, eps, parts, n_parts, stream, rope);
   if (gamma)
     return launch_skinny<EPI_ROPE, true, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, gamma, gamma_dtype == kF32,
                                                eps, extra, stream, rope);
+  if (M <= 16) return launch_few<EPI_ROPE, bf16>((const bf16*)a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, eps, extra, stream, rope);
   return launch_skinny<EPI_ROPE, false, bf16>(a, lda, (const bf16*)w, ldw, (bf16*)c, ldc, M, N, K, nullptr, 0, eps, extra,
                                               stream, rope);
 }

@@ -510,6 +510,38 @@ def test_gemm_bf16_prepares_the_next_norm(M, N, K, N2, silu, gamma_dtype):
     assert ((out.float() - again.float()).abs() <= 2 ** -6 * (1 + again.float().abs())).all()
 
 
+@pytest.mark.parametrize("N,K", [
+    # one tile, part of one, and the last workgroup's tiles beyond the rows of W; k of a part of a block, of whole blocks, of a part
+    # of a turn: four waves of two and three blocks, eight of two, four and five, sixteen of four and eight, and more turns than one
+    (8, 8), (4, 64), (20, 520), (9, 776), (264, 1000), (2056, 1032), (40, 2048), (72, 2104), (136, 2568), (88, 4096), (48, 8200),
+    # two, three and four tiles a workgroup, the last one's beyond the rows of W
+    (4100, 584), (4104, 2632), (6148, 264), (6152, 2056), (8204, 968), (8216, 2112)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+def test_gemm_bf16_of_up_to_16_rows(M, N, K):
+    """The products of a decode step against float64, and what one row holds stays its own: a row of A and a row of W
+    that are not finite touch their row and their column of the result alone (the two k ranges of a tile stand side by side)."""
+    from glassbox_amd import ops
+    a, w = rnd(M, K, seed=1).bfloat16(), (rnd(N, K, seed=2) / math.sqrt(K)).bfloat16()
+    da, dw = to_dev(a), to_dev(w)
+    want = a.double() @ w.double().T
+    c = torch.full((M, N), 9.0, device=DEV)
+    ops.gemm(da, dw, c)
+    tol = 1e-4    # 32-bit sums of products of numbers of variance 1 / K: 2^-24 sqrt(K) terms at most, K <= 8,200
+    assert (c.cpu().double() - want).abs().max().item() <= tol
+    if N >= 16:
+        half = N // 16 * 8
+        act = torch.full((M, half), 9.0, device=DEV, dtype=torch.bfloat16)
+        ops.gemm(da, dw[:2 * half], act, silu_mul=True)
+        g, u = want[:, :half], want[:, half:2 * half]
+        unit = g / (1 + torch.exp(-g)) * u
+        assert (act.cpu().double() - unit).abs().max().item() <= 2 ** -8 * unit.abs().max().item() + 10 * tol
+    wild_a, wild_w = a.clone(), w.clone()
+    wild_a[M - 1, K - 1], wild_w[N - 1, 0] = float("nan"), float("inf")
+    ops.gemm(to_dev(wild_a), to_dev(wild_w), c)
+    finite = torch.isfinite(c.cpu())
+    assert finite[:M - 1, :N - 1].all() and not finite[M - 1].any() and not finite[:, N - 1].any()
+
+
 @pytest.mark.parametrize("M,N,K", [(2048, 2048, 8192), (128, 2048, 2048), (40, 1008, 4104), (300, 960, 2560), (64, 2048, 8192)])
 @pytest.mark.parametrize("gamma_dtype", [torch.float32, torch.bfloat16])
 def test_gemm_bf16_that_divides_k_does_the_next_norm(M, N, K, gamma_dtype):
