@@ -351,6 +351,8 @@ struct StepExtras {
   float* k_pages;
   float* v_pages;
   int nh, nkv, hd, page_size;
+  float per_half;   // 2 / hd, and page_size as a shift (-1: no power of two): the kernel has no time for divisions
+  int page_shift;
 };
 
 constexpr int kNormedFloats = 2560;   // of the rows that a workgroup norms (step_takes)
@@ -418,14 +420,15 @@ void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
   const int cr = tid % R, cm = tid / R;
   // the row of W behind row t of the workgroup's (beyond the last: that one again)
   const int half = EPI == EPI_HEADS ? ex.hd / 2 : N / 2;
+  auto head_of = [&](int p) { return (int)(((float)p + 0.5f) * ex.per_half); };   // p / half, exact below 2^21 pairs
   auto w_row = [&](int t) -> int {
     if constexpr (EPI == EPI_PLAIN) return min(n0 + t, N - 1);
     const int pair = min(n0 / 2 + t % (R / 2), N / 2 - 1);
-    return (EPI == EPI_HEADS ? pair / half * ex.hd + pair % half : pair) + (t >= R / 2 ? half : 0);
+    return (EPI == EPI_HEADS ? pair + head_of(pair) * half : pair) + (t >= R / 2 ? half : 0);   // (a head's rows are twice its pairs)
   };
   // with EPI_HEADS the pair that a thread finishes
   const int pair = n0 / 2 + cr;
-  const int head = EPI == EPI_HEADS ? pair / half : 0, at = EPI == EPI_HEADS ? pair % half : 0;
+  const int head = EPI == EPI_HEADS ? head_of(pair) : 0, at = EPI == EPI_HEADS ? pair - head * half : 0;
   const bool finishes = EPI != EPI_PLAIN && cm < MT && cm < M && cr < R / 2 && pair < N / 2;
   const bool is_value = EPI == EPI_HEADS && head >= ex.nh + ex.nkv;
   float cs = 1.f, sn = 0.f;
@@ -454,7 +457,7 @@ void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
         const int k = (s0 + mine) * kSlice + 4 * word;
         const float* from = w + (size_t)w_row(row) * ldw + (k < K ? k : 0);
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)(uintptr_t)from,
-                                         (__attribute__((address_space(3))) uint32_t*)(uint32_t)(uintptr_t)(wl + unit * 256), 16, 0, 0);
+                                         (__attribute__((address_space(3))) uint32_t*)(uint32_t)(uintptr_t)(wl + unit * 256), 16, 0, 2);   // (nontemporal: read once)
       }
       // What the end will want from memory is asked for under W: a cell's old value; a pair's angle and its row's place in the pages.
       // (Not before W: the compiler would wait for it there.)
@@ -542,7 +545,7 @@ void gemm_f32_skinny_kernel(const float* __restrict__ a, int lda,
           row[at] = y0;
           row[half + at] = y1;
           if (slot >= 0) {
-            const int page = slot / ex.page_size, off = slot % ex.page_size, piece = key_piece(ex.hd);
+            const int page = ex.page_shift >= 0 ? slot >> ex.page_shift : slot / ex.page_size, off = slot - page * ex.page_size, piece = key_piece(ex.hd);
             if (is_value) {
               float* to = ex.v_pages + ((size_t)page * ex.nkv + (head - ex.nh - ex.nkv)) * ex.hd * ex.page_size + off;
               to[(size_t)at * ex.page_size] = y0;
@@ -668,7 +671,8 @@ extern "C" int gb_gemm_f32_step(const float* a, int lda, const float* w, int ldw
   GB_REQUIRE(epilogue != EPI_HEADS || (hd >= 2 && hd % 2 == 0 && nh > 0 && nkv >= 0 && N == (nh + 2 * nkv) * hd && (cosv == nullptr) == (sinv == nullptr) &&
                                        (!slots || (nkv > 0 && k_pages && v_pages && page_size > 0))),
              "gemm_f32_step: N=%d is not (nh + 2 nkv) hd with nh=%d nkv=%d hd=%d, or pages or angles are missing", N, nh, nkv, hd);
-  const StepExtras ex{gamma, eps, cosv, sinv, slots, (float*)k_pages, (float*)v_pages, nh, nkv, hd, page_size};
+  const StepExtras ex{gamma, eps, cosv, sinv, slots, (float*)k_pages, (float*)v_pages, nh, nkv, hd, page_size, hd > 0 ? 2.0f / (float)hd : 0.f,
+                      page_size > 0 && (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1};
   if (!gamma && epilogue == EPI_PLAIN) return gb_gemm_f32(a, lda, w, ldw, c, ldc, M, N, K, 0, stream);
 #define GB_STEP(MT, R, EPI)                                                                                                 \
   if (epilogue == EPI && (M <= 1) == (MT == 1) && R == (N > kNarrow ? 16 : N > 4 * kTwoAUnit ? 8 : 4)) {                      \
