@@ -1567,7 +1567,7 @@ def gemm_split_floats(rows: int, n: int, k: int) -> int:
 def gemm_route(rows: int, n: int, k: int, silu_mul: bool = False, accumulate: bool = False, heads: bool = False, parts: bool = False,
                workspace: bool = False) -> str:
     """The kernel that ``gemm`` (``heads``: ``gemm_rope``) launches for a bfloat16 product of these sizes and options, without a norm to
-    do or to prepare: "tiled", "ring", "few" (the skinny or the folded kernel), "held", "block" or "slices" (of k)."""
+    do or to prepare: "tiled", "ring", "few" (the kernels of up to 64 rows), "held", "block" or "slices" (of k)."""
     epilogue = 3 if heads else 2 if silu_mul else 1 if accumulate else 0
     return ("tiled", "ring", "few", "held", "block", "slices")[_lib("gemm_bf16").gb_gemm_bf16_route(
         int(rows), int(n), int(k), epilogue, int(parts), int(workspace))]

@@ -218,7 +218,7 @@ def emit_target(ctx, n: int, width: int, in_features: int, emit, tag: str):
     """Buffers for a product of n rows, ``width`` columns and ``in_features`` of k that is asked
     (``emit=(gamma, eps)``) to prepare the next norm: ``(gemm emit argument, PreNormed or Normed to hand on)``, or
     ``(None, None)`` when nothing is asked or this step's product cannot do it (a 32-bit step, sizes that neither
-    the folded kernel nor a product that divides k takes)."""
+    the kernels of few rows nor a product that divides k takes)."""
     from .. import ops
     if emit is None or ctx.dtype != torch.bfloat16 or not ctx.fuse_norms:
         return None, None
