@@ -62,7 +62,8 @@ __device__ __forceinline__ float gated_unit(float g, float u, const Glu& p) {
 
 // A lane's 16 bytes, or zeros where it has nothing to read: then the address is one of zeros, so that a run of loads stays one
 // stretch of code, which a branch round each of them would cut up.  (Named as global memory: of an address that is one of two the
-// compiler cannot tell, and would wait for all loads where it needs the first.)
+// compiler cannot tell, and would wait for all loads where it needs the first.)  For kernels that ask for all they read at once;
+// a long loop is faster with the branches (see gemm_skinny_kernel).
 __device__ const bf16x8 kZeros = {};
 __device__ __forceinline__ const bf16x8 __attribute__((address_space(1))) * or_zeros(bool ok, const bf16* p) {
   typedef const bf16x8 __attribute__((address_space(1))) * global_words;
@@ -1806,6 +1807,14 @@ int launch_split(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc,
 // and writes act[m, j] = gate / (1 + exp(-gate)) * up (crates/glassbox-core/src/model.rs:336-340)
 // to C[M, N/2].
 
+// 16 bytes of a lane that has something to read, else zeros: without a branch (SHORT) or with one, and the address behind it (before
+// it, it costs the kernels that norm their rows the registers with which two workgroups fit on a unit).
+template <bool SHORT>
+__device__ __forceinline__ bf16x8 load_word(bool ok, const bf16* row, int k) {
+  if constexpr (SHORT) return *or_zeros(ok, row + k);
+  else return ok ? load8(row + k) : zero8();
+}
+
 // The A operand of one lane: 8 consecutive k of row m.  Plain: bfloat16 rows as they are.  RMS: the
 // rows are the float32 residual; the operand is bf16(gamma[k] * x[k]) and sum(x^2) is gathered on
 // the way, so that the caller can scale the finished product by 1/sqrt(mean(x^2) + eps): the RMS
@@ -1819,10 +1828,10 @@ __device__ __forceinline__ bf16x8 from_lane(bf16x8 v, int lane) {
   return __builtin_bit_cast(bf16x8, w);
 }
 
-template <bool RMS>
+template <bool RMS, bool SHORT = false>
 __device__ __forceinline__ bf16x8 load_a(const void* a, int lda, int m, int k, bool ok, const void* gamma, int gamma_f32,
                                          float& ss) {
-  if (!RMS) return *or_zeros(ok, (const bf16*)a + (size_t)m * lda + k);
+  if (!RMS) return load_word<SHORT>(ok, (const bf16*)a + (size_t)m * lda, k);
   if (!ok) return zero8();
   const float* x = (const float*)a + (size_t)m * lda + k;
   const f32x4 x0 = *reinterpret_cast<const f32x4*>(x), x1 = *reinterpret_cast<const f32x4*>(x + 4);
@@ -1850,7 +1859,10 @@ __device__ __forceinline__ bf16x8 load_a(const void* a, int lda, int m, int k, b
   return out;
 }
 
-template <int MT, int WAVES, int ITERS, int RT, int EPI, bool RMS, typename CT, bool HALF = false>
+// SHORT (rows that are normed already, where skinny_short() says so): the partial sums of the norm are asked for before W and added up
+// behind its requests, and loads are without branches, so that all of a turn are asked for at once.  Otherwise the sums come first and
+// loads are masked: many turns, and the traffic of many rows, are slower with an address chosen for every load and zeros fetched.
+template <int MT, int WAVES, int ITERS, int RT, int EPI, bool RMS, bool SHORT, typename CT, bool HALF = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_kernel(const void* __restrict__ a, int lda,
                                                                  const bf16* __restrict__ w, int ldw, CT* __restrict__ c,
                                                                  int ldc, int M, int N, int K, const void* __restrict__ gamma,
@@ -1899,7 +1911,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_ke
   }
 
   // Partial sums of squares of the rows, one per tile of the product that made them (64 floats a tile): a lane a row, four loads
-  // asked for at once, before W, and added up behind the requests for W, which so do not wait for them.
+  // at once and then eight (one behind the other the rest of 384 tiles' sums cost 48 rows by 16,384 x 3,072 7 of 45 us).
   float got[4] = {0.f, 0.f, 0.f, 0.f};
   if (!RMS && parts != nullptr && lane % LR < M) {
     const float* mine = parts + lane % LR;
@@ -1908,29 +1920,34 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_ke
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (p0 + u * STEP < n_parts) got[u] = mine[(p0 + u * STEP) * 64];
-    for (int p = p0 + 4 * STEP; p < n_parts; p += STEP) got[0] += mine[p * 64];
+    for (int p = p0 + 4 * STEP; p < n_parts; p += 8 * STEP) {
+      float more[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) more[u] = p + u * STEP < n_parts ? mine[(p + u * STEP) * 64] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) got[u % 4] += more[u];
+    }
   }
+  auto add_up = [&] {
+    if (RMS || parts == nullptr) return;
+    float sum = ((got[0] + got[1]) + got[2]) + got[3];
+#pragma unroll
+    for (int o = LR; o < 64; o <<= 1) sum += __shfl_xor(sum, o, kWave);
+    if (lane < LR && lane < MT * 16) red[wave][lane] = sum;
+  };
+  if (!SHORT) add_up();
   // a 64-wide k block is two MFMA steps of 32: lane group q holds k = 8q..8q+7 of each
-  bf16x8 wf[RT][ITERS][2];
-  auto ask = [&](int kbeg) {
+  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
+    bf16x8 wf[RT][ITERS][2];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
         const int k = kbeg + (wave + WAVES * it) * 64 + q * 8;
-        wf[rt][it][0] = *or_zeros(row_ok[rt] && k < K, wrow[rt] + k);
-        wf[rt][it][1] = *or_zeros(row_ok[rt] && k + 32 < K, wrow[rt] + k + 32);
+        wf[rt][it][0] = load_word<SHORT>(row_ok[rt] && k < K, wrow[rt], k);
+        wf[rt][it][1] = load_word<SHORT>(row_ok[rt] && k + 32 < K, wrow[rt], k + 32);
       }
-  };
-  ask(0);
-  if (!RMS && parts != nullptr) {
-    float sum = ((got[0] + got[1]) + got[2]) + got[3];
-#pragma unroll
-    for (int o = LR; o < 64; o <<= 1) sum += __shfl_xor(sum, o, kWave);
-    if (lane < LR && lane < MT * 16) red[wave][lane] = sum;
-  }
-  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
-    if (kbeg > 0) ask(kbeg);
+    if (SHORT && kbeg == 0) add_up();
     if (MT == 1) {
       bf16x8 xf[ITERS][2];
 #pragma unroll
@@ -1964,8 +1981,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_ke
             // for 16 bytes of another row: lane 4R + Q loads piece Q of row R, and the operand's lane (row lane%16,
             // piece lane/16) takes it from there through the LDS crossbar.
             const int m = t * 16 + (lane >> 2), ka = k - q * 8 + (lane & 3) * 8;
-            const bf16x8 y0 = load_a<false>(a, lda, m, ka, m < M && ka < K, gamma, gamma_f32, ss[t]);
-            const bf16x8 y1 = load_a<false>(a, lda, m, ka + 32, m < M && ka + 32 < K, gamma, gamma_f32, ss[t]);
+            const bf16x8 y0 = load_a<false, SHORT>(a, lda, m, ka, m < M && ka < K, gamma, gamma_f32, ss[t]);
+            const bf16x8 y1 = load_a<false, SHORT>(a, lda, m, ka + 32, m < M && ka + 32 < K, gamma, gamma_f32, ss[t]);
             x0 = from_lane(y0, 4 * r + q);
             x1 = from_lane(y1, 4 * r + q);
           }
@@ -2554,6 +2571,13 @@ inline void skinny_plan(int tiles, int K, int mt, int* waves, int* iters, int* r
   *iters = (mt == 1 && per_wave >= 2) ? 2 : 1;
 }
 
+// Whether rows that are normed already take the form for a short k (SHORT): up to 2,048, two turns of sixteen waves (us, without /
+// with: 17 rows by 1,600 x 960 5.6 / 5.2, by 2,048 x 2,048 7.2 / 5.9, 40 rows by 1,600 x 960 6.9 / 6.7; 64 rows by 49,152 x 2,048 43.6 /
+// 43.5; beyond, 40 rows by 16,384 x 3,072 36.4 / 38.9, 32 by 28,672 x 8,192 120 / 140), and up to 32 rows with one tile a workgroup of any
+// k (17 rows by 4,096 x 5,120 17.4 / 15.0, 32 rows 17.5 / 16.1), but of half a tile only up to 24 (by 960 x 2,560 17 rows 7.6 / 6.8, 24
+// rows 7.7 / 7.6, 32 rows 7.7 / 8.1).
+inline bool skinny_short(int M, int K, int rt, bool half) { return K <= 2048 || (M <= 32 && rt == 1 && (!half || M <= 24)); }
+
 template <int MT, int EPI, bool RMS, typename CT>
 int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, CT* c, int ldc, int M, int N, int K,
                      const void* gamma, int gamma_f32, float eps, const NormExtras& extra, const RopeExtras& rope,
@@ -2565,12 +2589,12 @@ int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, 
     // workgroups of 8 rows of W, half of each tile left empty, so that twice as many compute units draw on memory.
     if (tiles < 256 && extra.parts == nullptr) {
       const int halves = (N + 7) / 8;
-#define GB_HALF(WV, IT)                                                                                                    \
-  if (waves == WV && iters == (IT))                                                                                        \
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, (IT), 1, EPI, RMS, CT, true>), dim3(halves), dim3(WV * 64), 0, stream, a, \
+      const bool brief = skinny_short(M, K, 1, true);
+#define GB_HALF(WV, SHORT)                                                                                                 \
+  if (waves == WV && brief == SHORT)                                                                                       \
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, 1, 1, EPI, RMS, SHORT, CT, true>), dim3(halves), dim3(WV * 64), 0, stream, a, \
                        lda, w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rope);
-      GB_HALF(4, 1) GB_HALF(16, 1)
-      if constexpr (MT == 1) { GB_HALF(4, 2) GB_HALF(16, 2) }
+      GB_HALF(4, true) GB_HALF(16, true) GB_HALF(16, false)
 #undef GB_HALF
       return launched("gemm_bf16 (skinny, half tiles)");
     }
@@ -2579,13 +2603,16 @@ int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, 
   RopeExtras rp = rope;
   rp.three_halves = (EPI == EPI_ROPE && rt == 2 && tiles % 3 == 0) ? 1 : 0;
   const int groups = rp.three_halves ? 2 * tiles / 3 : (tiles + rt - 1) / rt;
-#define GB_CFG(WV, IT, RT)                                                                                                 \
-  if (waves == WV && iters == (IT) && rt == RT)                                                                            \
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, (IT), RT, EPI, RMS, CT>), dim3(groups), dim3(WV * 64), 0, stream, a, lda, \
+  const bool brief = !RMS && skinny_short(M, K, rt, false);
+#define GB_CFG(WV, IT, RT, SHORT)                                                                                          \
+  if (waves == WV && iters == IT && rt == RT && brief == SHORT)                                                            \
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, WV, IT, RT, EPI, RMS, SHORT, CT>), dim3(groups), dim3(WV * 64), 0, stream, a, lda, \
                        w, ldw, c, ldc, M, N, K, gamma, gamma_f32, eps, extra, rp);
-  // the configurations skinny_plan can ask for
-  GB_CFG(4, 1, 1) GB_CFG(4, 1, 2) GB_CFG(16, 1, 1) GB_CFG(16, 1, 2)
-  if constexpr (MT == 1) { GB_CFG(4, 2, 1) GB_CFG(4, 2, 2) GB_CFG(16, 2, 1) GB_CFG(16, 2, 2) }
+  // the configurations skinny_plan and skinny_short can ask for
+  GB_CFG(4, 1, 1, !RMS) GB_CFG(4, 1, 2, !RMS) GB_CFG(16, 1, 1, !RMS) GB_CFG(16, 1, 2, !RMS)
+  if constexpr (!RMS) { GB_CFG(16, 1, 2, false) }
+  if constexpr (!RMS && MT > 2) { GB_CFG(16, 1, 1, false) }
+  if constexpr (RMS && MT == 1) { GB_CFG(4, 2, 1, false) GB_CFG(4, 2, 2, false) GB_CFG(16, 2, 1, false) GB_CFG(16, 2, 2, false) }
 #undef GB_CFG
   return launched("gemm_bf16 (skinny)");
 }

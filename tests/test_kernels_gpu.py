@@ -469,6 +469,9 @@ def test_gemm_bf16_fused_rms_norm(N, K, M, silu, gamma_dtype):
                                            (12, 960, 2560, 2880, False), (40, 24704, 128, 512, False), (64, 352, 64, 176, True),
                                            (20, 4096, 1024, 1024, True), (9, 72, 264, 48, False), (17, 2048, 1024, 16384, True),
                                            (20, 960, 960, 5120, True), (33, 960, 776, 1600, False),
+                                           # a k beyond 2,048: half tiles of up to 24 rows and of more, one tile, two
+                                           (20, 968, 2056, 256, False), (32, 968, 2056, 256, False), (32, 5128, 2304, 256, False),
+                                           (24, 6160, 2568, 256, False), (33, 24704, 2056, 256, False),
                                            # at most 8 rows by so many rows of W that the folded kernel does not pay
                                            (5, 4096, 512, 256, False)])
 @pytest.mark.parametrize("gamma_dtype", [torch.float32, torch.bfloat16])
@@ -733,6 +736,22 @@ def test_gemm_bf16_held_rows_behind_many_partial_sums(M, N, K, silu, n):
     """Partial sums of a norm up to and beyond the 256 that the held kernel asks for at once (a row of 3,072 leaves 384)."""
     from glassbox_amd import ops
     assert ops.gemm_route(M, N, K, silu_mul=silu, parts=True) == "held"
+    check_held(M, N, K, silu=silu, n_parts=n, f32=True, padded=False)
+
+
+@pytest.mark.parametrize("M,N,K,n", [
+    # a k of up to 2,048, beyond with one tile a workgroup and up to 32 rows, and beyond; as many partial sums as are asked for at once,
+    # up to eight more a lane, and several rounds of eight; k of whole turns and of part of one
+    (33, 1600, 2040, 255), (40, 1600, 2056, 256), (17, 4096, 5120, 320), (24, 1280, 8192, 640), (32, 6160, 5120, 511), (33, 6160, 2056, 129),
+    (48, 2576, 3072, 384), (64, 6160, 3080, 1025), (17, 6160, 4104, 130),
+    # half a tile a workgroup: up to 24 rows, and up to 32 of a short k and of a longer one
+    (24, 968, 2560, 0), (25, 968, 2560, 0), (32, 1000, 2048, 0)])
+@pytest.mark.parametrize("silu", [False, True])
+def test_gemm_bf16_of_17_to_64_rows_of_a_short_and_of_a_long_k(M, N, K, n, silu):
+    """The kernel that streams W through all of a workgroup's waves in both of its forms, against float64."""
+    from glassbox_amd import ops
+    N -= N % 16 if silu else 0
+    assert ops.gemm_route(M, N, K, silu_mul=silu, parts=n > 0) == "few"
     check_held(M, N, K, silu=silu, n_parts=n, f32=True, padded=False)
 
 
@@ -1001,7 +1020,10 @@ def test_gemm_bf16_rotates_and_writes_the_cache_with_the_rows_held(M, nh, nkv, h
 @pytest.mark.parametrize("M,nh,nkv,hd,K,n,kernel", [
     (20, 9, 3, 64, 576, 72, "held"), (49, 9, 3, 64, 576, 72, "held"), (32, 32, 8, 96, 3072, 384, "held"), (24, 32, 8, 128, 4096, 256, "held"),
     (64, 32, 32, 64, 2048, 257, "held"), (33, 32, 8, 48, 2048, 511, "held"), (17, 24, 8, 64, 512, 64, "few"), (8, 9, 3, 64, 576, 72, "few"),
-    (40, 15, 5, 64, 960, 120, "few")])
+    (40, 15, 5, 64, 960, 120, "few"),
+    # a longer k than 2,048: a tile and a half, one tile and two tiles a workgroup
+    (20, 72, 12, 64, 5120, 320, "few"), (24, 8, 4, 64, 2304, 300, "few"), (40, 15, 5, 64, 2560, 160, "few"), (64, 32, 8, 128, 4096, 256, "few"),
+    (24, 50, 2, 128, 5120, 320, "few")])
 def test_gemm_bf16_rotates_behind_the_partial_sums_of_a_norm(M, nh, nkv, hd, K, n, kernel):
     """The stacked q/k/v product of rows whose norm comes as partial sums: the scale is in what is rotated, in the rows and in both
     pages.  Against float64, element by element."""
