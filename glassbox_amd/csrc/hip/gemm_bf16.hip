@@ -2220,8 +2220,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_fold_kernel(const void* __res
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
         const int k = kbeg + (wave + WAVES * it) * 128 + khalf + q * 8;
-        wf[rt][it][0] = __builtin_nontemporal_load(or_zeros(row_ok[rt] && k < K, wrow[rt] + k));
-        wf[rt][it][1] = __builtin_nontemporal_load(or_zeros(row_ok[rt] && k + 64 < K, wrow[rt] + k + 64));
+        wf[rt][it][0] = (row_ok[rt] && k < K) ? load8_once(wrow[rt] + k) : zero8();
+        wf[rt][it][1] = (row_ok[rt] && k + 64 < K) ? load8_once(wrow[rt] + k + 64) : zero8();
       }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
