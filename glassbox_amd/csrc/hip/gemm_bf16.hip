@@ -2462,7 +2462,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES >= 8 ? 4 : 1) void gemm_few_kerne
       const float p = lane_mirror8(v);
       if (m >= M || own * 8 >= N) continue;
       const int half = rope.hd / 2, dim = n < 4 ? pair[i] : half + pair[i];
-      const bf16 yb = (bf16)(n < 4 ? v * cs[i] - p * sn[i] : v * cs[i] + p * sn[i]);
+      // (a value, and any head without angles, is no sum with its partner: of a partner that is not finite 0 would make a NaN)
+      const bool turns = rope.cosv != nullptr && head[i] < rope.nh + rope.nkv;
+      const bf16 yb = (bf16)(!turns ? v : n < 4 ? v * cs[i] - p * sn[i] : v * cs[i] + p * sn[i]);
       c[(size_t)m * ldc + head[i] * rope.hd + dim] = (CT)yb;
       if (rope.slots != nullptr && head[i] >= rope.nh) {
         const int page = rope.page_shift >= 0 ? slot[i] >> rope.page_shift : slot[i] / rope.page_size, off = slot[i] - page * rope.page_size;

@@ -1056,6 +1056,35 @@ def test_gemm_bf16_rotates_behind_the_partial_sums_of_a_norm(M, nh, nkv, hd, K, 
     assert torch.equal(v_pages.cpu().double()[idx // page, :, :, idx % page], rows[:, nh + nkv:])
 
 
+@pytest.mark.parametrize("M,K", [(1, 64), (8, 2048), (9, 72), (16, 1032), (20, 64), (48, 2048)])
+@pytest.mark.parametrize("angles", [True, False])
+def test_gemm_bf16_rotation_leaves_values_alone(M, K, angles):
+    """A dimension of a value that is not finite stays that dimension's, in the row and in the page; and so does one of a query or a
+    key where the call has no angles, while with angles it reaches the one that it is paired with and no other."""
+    from glassbox_amd import ops
+    nh, nkv, hd, page = 4, 2, 32, 16
+    heads = nh + 2 * nkv
+    a, w = rnd(M, K, seed=1).bfloat16(), (rnd(heads * hd, K, seed=2) / math.sqrt(K)).bfloat16()
+    wild = [(1, 5), (nh + 1, hd // 2 + 3), (nh + nkv, 2), (nh + 2 * nkv - 1, hd - 1)]      # (head, dimension): query, key, two values
+    want = torch.zeros(M, heads, hd, dtype=torch.bool)
+    for (head, d), value in zip(wild, [float("inf"), float("nan"), float("inf"), float("nan")]):
+        w[head * hd + d] = value
+        want[:, head, d] = True
+        if angles and head < nh + nkv:
+            want[:, head, (d + hd // 2) % hd] = True
+    turn = torch.rand(M, hd // 2, generator=torch.Generator().manual_seed(3)) * 6
+    slots = torch.randperm(4 * page, generator=torch.Generator().manual_seed(4))[:M].to(torch.int32)
+    k_pages = torch.zeros(ops.key_pages_shape(4, nkv, page, hd), device=DEV, dtype=torch.bfloat16)
+    v_pages = torch.zeros(4, nkv, hd, page, device=DEV, dtype=torch.bfloat16)
+    qkv = torch.full((M, heads * hd), 9.0, device=DEV, dtype=torch.bfloat16)
+    ops.gemm_rope(to_dev(a), to_dev(w), qkv, nh, nkv, hd, to_dev(turn.cos()) if angles else None, to_dev(turn.sin()) if angles else None,
+                  to_dev(slots), k_pages, v_pages)
+    assert torch.equal(~torch.isfinite(qkv.cpu()).view(M, heads, hd), want)
+    idx = slots.long()
+    assert torch.equal(~torch.isfinite(ops.unpack_keys(k_pages).cpu())[idx // page, :, idx % page, :], want[:, nh:nh + nkv])
+    assert torch.equal(~torch.isfinite(v_pages.cpu())[idx // page, :, :, idx % page], want[:, nh + nkv:])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("hd,page", [(16, 16), (64, 16), (128, 32), (40, 16)])
 def test_rope_store_writes_values_of_portions_in_tiles(dtype, hd, page):
