@@ -2323,9 +2323,11 @@ __global__ __launch_bounds__(WAVES * 64, WAVES >= 8 ? 4 : 1) void gemm_few_kerne
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r8 = lane & 7, kpos = ((lane >> 3) & 1) * 32 + (lane >> 4) * 8;
   // words of four rows' partial sums: of up to 8 rows 8 floats a tile, beyond 64 of which 16 are wanted
+  // (the sums are floats of a caller's: words of them need not begin at 16 bytes)
+  typedef float floats4 __attribute__((ext_vector_type(4), aligned(4)));
   f32x4 got = {0.f, 0.f, 0.f, 0.f};
   if (parts != nullptr) {
-    auto word = [&](int i) { return *reinterpret_cast<const f32x4*>(parts + (MB == 1 ? 4 * i : 64 * (i >> 2) + 4 * (i & 3))); };
+    auto word = [&](int i) -> f32x4 { return *reinterpret_cast<const floats4*>(parts + (MB == 1 ? 4 * i : 64 * (i >> 2) + 4 * (i & 3))); };
     if (tid < 2 * MB * n_parts) got = word(tid);
     for (int i = tid + WAVES * 64; i < 2 * MB * n_parts; i += WAVES * 64) got += word(i);
   }

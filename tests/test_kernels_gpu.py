@@ -755,6 +755,28 @@ def test_gemm_bf16_of_17_to_64_rows_of_a_short_and_of_a_long_k(M, N, K, n, silu)
     check_held(M, N, K, silu=silu, n_parts=n, f32=True, padded=False)
 
 
+@pytest.mark.parametrize("M,K", [(1, 64), (8, 2048), (9, 776), (16, 2048), (20, 960), (48, 2048)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_gemm_bf16_takes_partial_sums_anywhere(M, K, off):
+    """Partial sums are floats of the caller's, also where they are no 16-byte words: a view that begins some floats on gives the bits of
+    a tensor of its own, in a product and in the rotating one."""
+    from glassbox_amd import ops
+    nh, nkv, hd, n, eps, stride = 4, 2, 32, 75, 1e-5, ops.parts_stride(M)
+    a, w = to_dev(rnd(M, K, seed=1).bfloat16()), to_dev((rnd((nh + 2 * nkv) * hd, K, seed=2) / math.sqrt(K)).bfloat16())
+    room = to_dev(torch.rand(n * stride + off, generator=torch.Generator().manual_seed(off)) * 20 + 0.1)
+    outs = [[], []]
+    for out, parts in zip(outs, (room[off:], room[off:].clone())):
+        c = torch.empty(M, w.shape[0], device=DEV)
+        ops.gemm(a, w, c, rms_parts=(parts, n, eps))
+        qkv = torch.empty(M, w.shape[0], device=DEV, dtype=torch.bfloat16)
+        ops.gemm_rope(a, w, qkv, nh, nkv, hd, None, None, None, None, None, rms_parts=(parts, n, eps))
+        out += [c.cpu(), qkv.cpu()]
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    scale = 1 / torch.sqrt(room[off:].cpu().double().view(n, stride)[:, :M].sum(0) / K + eps)
+    want = a.cpu().double() @ w.cpu().double().T * scale.unsqueeze(1)
+    assert ((outs[0][0].double() - want).abs() <= sum_bound(a.cpu(), w.cpu()) * scale.max().item() + 2 ** -21 * want.abs()).all()
+
+
 def sum_bound(a, w):
     """What a float32 sum of products of 16-bit numbers may be off by: sqrt(K) roundings' worth of 2^-24 of a partial sum, which is
     about the product of the rows' lengths at most; eight times that."""
