@@ -2511,20 +2511,43 @@ struct FewPlan {
 };
 inline FewPlan few_plan(int epi, int M, int N, int K) {
   const int tiles = epi == EPI_SILU_MUL ? (N / 2 + 3) / 4 : (N + 7) / 8, blocks = (K + 63) / 64;
-  FewPlan p;
-  // A workgroup for every compute unit, and no more than four tiles each (accumulating: two tiles where emit_parts() has sums of 16
-  // columns).  Beyond 8 rows the rows of A are as much traffic as W: as many tiles a workgroup as its registers hold (12 rows by
-  // 16,384 x 2,048 with two tiles 16.2 us, four 15.3; by 6,144 x 4,096 two 16.2, three 12.6).
-  if (epi == EPI_ACCUMULATE) p.rt = (N + 15) / 16 < 256 ? 1 : tiles < 1024 ? 2 : 4;
-  else p.rt = tiles < (M > 8 ? 256 : 512) ? 1 : tiles < 768 ? 2 : tiles < 1024 ? 3 : 4;
-  // All of k at once where the registers hold it: a second turn of the loop begins behind the first one's last bytes (one row by
-  // 960 x 2,560: 40 blocks in one turn of eight waves 3.77 us, in one of sixteen with a third of them empty 4.26).
-  if (blocks <= 8) p.waves = 4, p.iters = 2;
-  else if (blocks <= 12 && (M <= 8 || p.rt == 1)) p.waves = 4, p.iters = 3;
-  else if (blocks <= 16 || (M > 8 && p.rt > 3)) p.waves = 8, p.iters = 2;
-  else if (blocks <= 32 || p.rt > 2) p.waves = 8, p.iters = 4;
-  else if (blocks <= 40 && M <= 8 && p.rt == 1) p.waves = 8, p.iters = 5;
-  else p.waves = 16, p.iters = blocks <= 64 || p.rt == 2 || M > 8 ? 4 : 8;
+  const bool many = M > 8;
+  FewPlan p{1, 4, 2};
+  // The compute unit with the most tiles ends last, so as many tiles a workgroup as leave it the fewest (8 rows by 5,120 x 960, 640 tiles,
+  // in threes 4.56 us, in twos, 320 workgroups, 5.18; 9 rows by 8,000 x 1,040, 1,000 tiles, in fours 6.0, in threes, 334 workgroups,
+  // 8.5).  Beyond that more tiles share the rows of A, which beyond 8 rows are as much traffic as W and weigh more; of a k of up to 512 more
+  // than two only leave fewer waves (9 rows by 8,064 x 384 in fours 4.25, in twos 3.96).  Accumulating: two or four where emit_parts()
+  // has sums of 16 columns, else one.
+  if (epi != EPI_ACCUMULATE || (N + 15) / 16 >= 256) {
+    const int step = epi == EPI_ACCUMULATE ? 2 : 1;
+    int least = 0;
+    for (int rt = step; rt <= (blocks <= 8 ? 2 : 4); rt += step) {
+      const int cost = ((tiles + rt - 1) / rt + 255) / 256 * (many ? 5 * rt + 6 : 10 * rt + 3);
+      if (rt == step || cost < least) least = cost, p.rt = rt;
+    }
+  }
+  // All of k at once where it is short; of a longer one turns of eight waves, whose two, three or four blocks a wave leave the least of the
+  // last turn empty, the most that do (one row by 4,096 x 14,336 in turns of 32 blocks 19.7 us, of 64 21.0; 9 rows by 960 x 2,560 in turns of
+  // 24 5.4, of 64 5.7).  Beyond 8 rows four only of up to two tiles a workgroup and a k of up to 4,096 (9 rows by 2,048 x 8,192 with two 11.1,
+  // with four 11.7), and of four tiles not three: the registers of two such workgroups a unit end there.
+  if (blocks <= 8) return p;
+  if (blocks <= 12) {
+    p.iters = 3;
+    return p;
+  }
+  p.waves = 8;
+  if (!many && p.rt == 1 && blocks > 32 && blocks <= 40) {
+    p.iters = 5;   // (one row by 960 x 2,560 in one turn 3.8 us, in two of 24 blocks 4.1)
+    return p;
+  }
+  if (!many && p.rt == 1 && blocks > 120 && blocks <= 128) {
+    p.waves = 16, p.iters = 8;   // (eight rows by 2,048 x 8,192 in one turn 9.7 us, in four 10.0; one row 8.0 and 7.8)
+    return p;
+  }
+  auto asked = [&](int it) { return (blocks + 8 * it - 1) / (8 * it) * (10 * it + 1); };
+  const int most = !many || (p.rt <= 2 && blocks <= 64) ? 4 : p.rt == 4 ? 2 : 3;
+  for (int it = 3; it <= most; ++it)
+    if (asked(it) < asked(p.iters)) p.iters = it;
   return p;
 }
 
@@ -2542,8 +2565,10 @@ int launch_few_mb(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc
                          extra.parts, lda, ldw, M, N, K, extra.n_parts, c, ldc, eps, extra, rope);                            \
     }
 #define GB_FEWS(WV, IT) GB_FEW(WV, IT, 1) GB_FEW(WV, IT, 2) GB_FEW(WV, IT, 3) GB_FEW(WV, IT, 4)
-  GB_FEWS(4, 2) GB_FEWS(4, 3) GB_FEWS(8, 2) GB_FEW(8, 4, 1) GB_FEW(8, 4, 2) GB_FEW(8, 4, 3) GB_FEW(16, 4, 1) GB_FEW(16, 4, 2)
-  if constexpr (MB == 1) { GB_FEW(8, 4, 4) GB_FEW(8, 5, 1) GB_FEW(16, 8, 1) }
+  // (what few_plan can ask for)
+  GB_FEW(4, 2, 1) GB_FEW(4, 2, 2) GB_FEWS(4, 3) GB_FEWS(8, 2) GB_FEW(8, 3, 1) GB_FEW(8, 3, 2) GB_FEW(8, 3, 3)
+  GB_FEW(8, 4, 1) GB_FEW(8, 4, 2)
+  if constexpr (MB == 1) { GB_FEW(8, 3, 4) GB_FEW(8, 4, 3) GB_FEW(8, 4, 4) GB_FEW(8, 5, 1) GB_FEW(16, 8, 1) }
 #undef GB_FEWS
 #undef GB_FEW
   GB_REQUIRE(found, "gemm_bf16: no kernel of %d tiles, %d waves and %d blocks for up to 16 rows", p.rt, p.waves, p.iters);

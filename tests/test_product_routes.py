@@ -2,6 +2,7 @@
 lines that were measured.  Only sizes go in, so no GPU is needed."""
 import ctypes
 import os
+import re
 
 import pytest
 
@@ -67,3 +68,13 @@ def test_products_of_some_hundred_rows_go_to_the_block_kernel_where_it_is_ahead(
     ("add", 24, 576, 1536, "few"), ("store", 131, 6144, 2048, "block"), ("store", 24, 6144, 4096, "held")])
 def test_products_with_a_workspace_divide_k_where_that_is_ahead(route, epilogue, M, N, K, kernel):
     assert route(epilogue, M, N, K, workspace=True) == kernel
+
+
+def test_kernels_of_up_to_16_rows_keep_everything_in_registers():
+    """Such a kernel lasts a few microseconds: scratch would be traffic of every lane beside the one pass over W.  Read from what the
+    compiler notes beside each kernel of the built library."""
+    build.ensure(["gemm_bf16"])
+    with open(build.find_current("gemm_bf16"), "rb") as fh:
+        notes = re.findall(rb"\.name(?:\xd9.|\xda..)(\w*gemm_few_kernel\w*)\xbb\.private_segment_fixed_size(.)", fh.read(), re.DOTALL)
+    assert len(notes) > 100
+    assert [name.decode() for name, scratch in notes if scratch != b"\0"] == []
