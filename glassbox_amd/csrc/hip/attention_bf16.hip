@@ -104,30 +104,36 @@ struct Pages {
 };
 // the key whose page stands for the tile of 16 from kt: itself, or one inside the keys known to have pages
 __device__ __forceinline__ int tile_key(int kt, int clamp_lo, int clamp_hi) { return min(max(kt, clamp_lo & ~15), clamp_hi & ~15); }
-// key / P by a multiplication: P is 16 times some number d, and magic = ceil(2^32 / d) (0: d is 1).  Exact for powers of two, and while
-// (key / 16) d < 2^32 for others.  (A division of numbers that a kernel is given costs some forty instructions one behind the
-// other, and eight of them stood before a wave's first request for keys: with these, and the first entries of the page table asked for
-// beside the position, one request of 300 keys, 9 heads on 3, 6.2 -> 5.8 us; of 3,800, 32 heads in 16 chunks, 8.9 -> 8.5.)
+// key / P by a multiplication: with 2^shift < P <= 2^(shift + 1) and magic = ceil(2^(32 + shift) / P), of 32 bits, exact for every key
+// below 2^31 (magic P is less than P, at most 2^(shift + 1), over 2^(32 + shift)).  (A division of numbers that a kernel is given costs some
+// forty instructions one behind the other, and eight of them stood before a wave's first request for keys: with these, and the first entries
+// of the page table asked for beside the position, one request of 300 keys, 9 heads on 3, 6.2 -> 5.8 us; of 3,800, 32 heads in 16 chunks,
+// 8.9 -> 8.5.)
 // (DIV: by the division all the same: sixteen waves have many tiles each and not a first one that counts, 53 requests of up to 2,300 keys
 // a step 1,834 us, by the multiplication 1,844.)
-template <bool DIV>
-__device__ __forceinline__ int page_index(int key, unsigned magic, int P) {
-  if (DIV) return key / P;
-  const unsigned t = (unsigned)key >> 4;
-  return (int)(magic ? __umulhi(t, magic) : t);
+struct PageQuotient {
+  unsigned magic, shift;
+};
+inline PageQuotient page_quotient(int P) {
+  const unsigned shift = 31 - __builtin_clz((unsigned)P - 1);
+  return {(unsigned)(((1ull << (32 + shift)) + P - 1) / P), shift};
 }
 template <bool DIV>
-__device__ __forceinline__ Pages pages_of(const int32_t* __restrict__ table, unsigned magic, int P, int kbase, int clamp_lo, int clamp_hi) {
+__device__ __forceinline__ int page_index(int key, const PageQuotient& of, int P) {
+  return DIV ? key / P : (int)(__umulhi((unsigned)key, of.magic) >> of.shift);
+}
+template <bool DIV>
+__device__ __forceinline__ Pages pages_of(const int32_t* __restrict__ table, const PageQuotient& quotient, int P, int kbase, int clamp_lo, int clamp_hi) {
   Pages p;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) p.of[t] = table[page_index<DIV>(tile_key(kbase + 16 * t, clamp_lo, clamp_hi), magic, P)];
+  for (int t = 0; t < 4; ++t) p.of[t] = table[page_index<DIV>(tile_key(kbase + 16 * t, clamp_lo, clamp_hi), quotient, P)];
   return p;
 }
 
 template <int HD, bool WIDE = false, int MODE = kPlainScores, bool DIV = false>
 __device__ __forceinline__ void attend64(Running<HD>& st, const bf16x8* qf, const bf16* __restrict__ kp,
                                          const bf16* __restrict__ vp, const Pages& pages, int nkv, int kvh,
-                                         int P, unsigned magic, int kbase, int lo, int hi, int clamp_lo, int clamp_hi, float scale,
+                                         int P, const PageQuotient& quotient, int kbase, int lo, int hi, int clamp_lo, int clamp_hi, float scale,
                                          int lane, float softcap = 0.f, float slope = 0.f, int pos = 0) {
   constexpr int KS = (HD + 31) / 32, DB = HD / 16;
   const int j = lane & 15, c = lane >> 4;
@@ -136,7 +142,7 @@ __device__ __forceinline__ void attend64(Running<HD>& st, const bf16x8* qf, cons
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int page = pages.of[t];
-    const int key0 = tile_key(kbase + 16 * t, clamp_lo, clamp_hi), slot0 = key0 - page_index<DIV>(key0, magic, P) * P;
+    const int key0 = tile_key(kbase + 16 * t, clamp_lo, clamp_hi), slot0 = key0 - page_index<DIV>(key0, quotient, P) * P;
     // pieces of 8 dimensions, of each the page's slots side by side (key_piece()): the 16 lanes of a group read 256 bytes
     const bf16* kb = kp + ((size_t)page * nkv + kvh) * P * HD + (slot0 + j) * 8;
 #pragma unroll
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
                                                             const int32_t* __restrict__ tables, int table_stride,
                                                             const bf16* __restrict__ kp, const bf16* __restrict__ vp, int nh,
                                                             int nkv, int P, float scale, int window, int keep, int chunk,
-                                                            int splits, int G, unsigned page_magic, unsigned group_magic, Extra ex) {
+                                                            int splits, int G, PageQuotient quotient, unsigned group_magic, Extra ex) {
   constexpr int KS = (HD + 31) / 32, DB = HD / 16;
   constexpr bool WIDE = std::is_same<OT, float>::value;
   extern __shared__ float decode_lds[];
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   if (AHEAD) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kb = split * chunk + (w + kvh + 5 * s) % WAVES * 64;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) ahead.of[t] = tables[(size_t)s * table_stride + min(page_index<DIV>(kb + 16 * t, page_magic, P), table_stride - 1)];
+    for (int t = 0; t < 4; ++t) ahead.of[t] = tables[(size_t)s * table_stride + min(page_index<DIV>(kb + 16 * t, quotient, P), table_stride - 1)];
   }
   const int lo = first_key(pos, window, MODE == kPlainScores ? 0 : ex.span);
   const int c0 = (MODE == kPlainScores ? 0 : chunks_from(lo, ex.span)) + split * chunk;
@@ -298,15 +304,15 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
 #pragma unroll
     for (int t = 0; t < 4; ++t) next.of[t] = t <= last ? ahead.of[t] : last >= 2 ? ahead.of[2] : last == 1 ? ahead.of[1] : ahead.of[0];
   } else {
-    next = pages_of<DIV>(table, page_magic, P, c0 + first * 64, lo, pos);
+    next = pages_of<DIV>(table, quotient, P, c0 + first * 64, lo, pos);
   }
   for (int kb = c0 + first * 64; kb < stop; kb += step) {
     // the kept first keys of these 64, then those inside the window (a tile can hold both kinds)
-    if (kb < kept) attend64<HD, WIDE, MODE, DIV>(st, qf, kp, vp, pages_of<DIV>(table, page_magic, P, kb, 0, kept - 1), nkv, kvh, P, page_magic, kb, col < G ? 0 : 1, col < G ? kept - 1 : 0, 0, kept - 1, scale, lane, ex.softcap, slope, pos);
+    if (kb < kept) attend64<HD, WIDE, MODE, DIV>(st, qf, kp, vp, pages_of<DIV>(table, quotient, P, kb, 0, kept - 1), nkv, kvh, P, quotient, kb, col < G ? 0 : 1, col < G ? kept - 1 : 0, 0, kept - 1, scale, lane, ex.softcap, slope, pos);
     const Pages now = next;
-    next = pages_of<DIV>(table, page_magic, P, kb + step, lo, pos);   // (beyond the last tile: its last page, not used)
+    next = pages_of<DIV>(table, quotient, P, kb + step, lo, pos);   // (beyond the last tile: its last page, not used)
     if (kb + 64 <= lo) continue;
-    attend64<HD, WIDE, MODE, DIV>(st, qf, kp, vp, now, nkv, kvh, P, page_magic, kb, col_lo, col_hi, lo, pos, scale, lane, ex.softcap, slope, pos);
+    attend64<HD, WIDE, MODE, DIV>(st, qf, kp, vp, now, nkv, kvh, P, quotient, kb, col_lo, col_hi, lo, pos, scale, lane, ex.softcap, slope, pos);
   }
   st.l += __shfl_xor(st.l, 16, kWave);
   st.l += __shfl_xor(st.l, 32, kWave);
@@ -1266,10 +1272,8 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
   if (waves == 4 && plain && splits == 1 && alone && known && seen > 256 && 8 * (32 + (size_t)hd * G) * sizeof(float) <= 65536) waves = 8;
   const size_t lds = (size_t)waves * (32 + (size_t)hd * G) * sizeof(float);
   const dim3 grid(splits, nkv, n_decode), block(waves * 64);
-  const unsigned sixteens = page_size / 16, page_magic = sixteens == 1 ? 0 : (unsigned)(((1ull << 32) + sixteens - 1) / sixteens);
+  const PageQuotient quotient = page_quotient(page_size);
   const unsigned group_magic = (65536 + G - 1) / G;
-  GB_REQUIRE((sixteens & (sixteens - 1)) == 0 || ((long long)max_context + 64) / 16 * sixteens < (1ll << 32),
-             "attention_decode: a context of %d keys in pages of %d", max_context, page_size);
   // capped and sloped scores are kernels of their own (bfloat16 results only), so that the others' score loops are what they were
   constexpr bool kCanCap = std::is_same<OT, bf16>::value;
   const bool cap = ex.softcap > 0.f, sloped = ex.slopes != nullptr;
@@ -1278,7 +1282,7 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
 #define GB_DECODE(HD, WAVES, MODE)                                                                                         \
   hipLaunchKernelGGL((decode_kernel<HD, WAVES, OT, MODE>), grid, block, lds, stream, (const bf16*)q, q_stride, out, out_stride, \
                      (float*)ws_acc, (float*)ws_ml, positions, tables, table_stride, (const bf16*)k_pages,                  \
-                     (const bf16*)v_pages, nh, nkv, page_size, scale, window, keep_first, chunk, splits, G, page_magic, group_magic, ex)
+                     (const bf16*)v_pages, nh, nkv, page_size, scale, window, keep_first, chunk, splits, G, quotient, group_magic, ex)
 #define GB_CASE(HD)                                                 \
   if (hd == HD) {                                                   \
     if (cap) {                                                      \

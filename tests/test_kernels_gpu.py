@@ -1642,6 +1642,32 @@ def test_tuned_decode_finds_one_far_key_in_every_chunk_position():
             assert (out.cpu().float()[0] - want).abs().max().item() < 2e-2, f"key at {target} was not found"
 
 
+@pytest.mark.parametrize("page,ctxlen", [(1200016, 1200216), (48, 70000), (65552, 131204)])
+def test_tuned_decode_finds_a_key_in_pages_of_any_size(page, ctxlen):
+    """Page numbers come by a multiplication: pages that are no power of two, up to ones of more than a million keys.  All keys are zeros but
+    one: at the ends of pages, of the context, and of a chunk."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    nh, nkv, hd = 2, 1, 16
+    n_pages = -(-ctxlen // page)
+    chunk = ops.decode_chunk(1, nkv, ctxlen, hd)
+    values = rnd(ctxlen, hd, seed=3).bfloat16()
+    v_pages = torch.zeros(n_pages, page, hd, dtype=torch.bfloat16)
+    v_pages.view(-1, hd)[:ctxlen] = values
+    tables = torch.arange(n_pages, dtype=torch.int32).flip(0)[None]          # the last page first
+    v_pages = to_dev(v_pages[tables[0].long()].transpose(1, 2)[:, None].contiguous())
+    q = rnd(1, nh * hd, seed=2).bfloat16()
+    q[0, hd:] = q[0, :hd]
+    for target in (0, page - 1, page, ctxlen - 1, chunk - 1, chunk):
+        k_pages = torch.zeros(n_pages, nkv, page, hd, dtype=torch.bfloat16)
+        k_pages[tables[0, target // page], 0, target % page] = q[0, :hd] * 40
+        cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=v_pages, group=0)
+        out = torch.zeros(1, nh * hd, device=DEV, dtype=torch.bfloat16)
+        ops.attention_decode(to_dev(q), out, BareContext([1], [ctxlen], tables, max_context=ctxlen), cache, nh, 1 / math.sqrt(hd), 0)
+        # (its weight is e^(10 |q|^2), of the others together ctxlen)
+        assert (out.cpu().float().view(nh, hd) - values[target].float()).abs().max().item() < 2e-2, f"key at {target} was not found"
+
+
 def test_tuned_decode_over_tens_of_thousands_of_keys():
     """Contexts of 40,000 and 33,333 keys beside one of 5: some hundred and sixty chunks a request for the second
     pass to merge, block tables of 2,500 pages.  Against the plain kernel on random keys, and with one key made to
