@@ -23,8 +23,8 @@
 //    A in registers and streams tiles of W through LDS.
 //  * few    (M <= 16, decode steps): 8 rows of W over two k ranges side by side in a tile, so that loads bring whole lines, all of
 //    them asked for at once.  (folded: the same tiles with the norm on the way, up to 8 rows by few rows of W.)
-// In all, every output cell is summed in an order fixed by (K, kernel) alone, not by M or by
-// the cell's neighbours.  C is bfloat16 or float32; accumulation (+=) is into float32.
+// In all, every output cell is summed in an order fixed by the product's sizes (they choose the kernel and how it divides k), not by
+// what its neighbours hold.  C is bfloat16 or float32; accumulation (+=) is into float32.
 #include <type_traits>
 
 #include "common.h"
@@ -1725,8 +1725,8 @@ __global__ __launch_bounds__(1024) void splitk_reduce_norm_few_kernel(const floa
   }
 }
 
-// Folded tiles pay when the product has at most 8 rows and whole tiles of 16 rows of W would leave
-// compute units without a workgroup (measured: with 384 such tiles they no longer do).
+// Rows that are normed on the way: the folded kernel pays when there are at most 8 of them and whole tiles of 16 rows of W
+// would leave compute units without a workgroup (measured: with 384 such tiles it no longer does).
 inline bool fold_pays(int M, int N) { return M <= 8 && (N + 15) / 16 < 256; }
 
 // What an accumulating product of these sizes can do for the RMS norm that reads the residual after it:
@@ -1735,7 +1735,7 @@ inline bool fold_pays(int M, int N) { return M <= 8 && (N + 15) / 16 < 256; }
 // 2 (a product that divides k, given its workspace) the whole norm, in the pass that adds the slices.
 inline int emit_mode(int M, int N, int K) {
   if (M > 16 && N % 4 == 0 && N <= SPLIT_NORM_MAX && split_plan(M, N, K).slices > 1) return 2;
-  if (M <= 64 && !(M > 16 && N >= 32768)) return 1;  // the skinny kernel
+  if (M <= 64 && !(M > 16 && N >= 32768)) return 1;
   return 0;
 }
 // Tiles of columns for which an emitting product of these sizes writes partial sums.
@@ -1862,14 +1862,15 @@ __device__ __forceinline__ bf16x8 load_a(const void* a, int lda, int m, int k, b
 // SHORT (rows that are normed already, where skinny_short() says so): the partial sums of the norm are asked for before W and added up
 // behind its requests, and loads are without branches, so that all of a turn are asked for at once.  Otherwise the sums come first and
 // loads are masked: many turns, and the traffic of many rows, are slower with an address chosen for every load and zeros fetched.
+// (MT = 1, up to 16 rows: only with RMS.  Rows of so few that are normed already are gemm_few_kernel's.)
 template <int MT, int WAVES, int ITERS, int RT, int EPI, bool RMS, bool SHORT, typename CT, bool HALF = false>
-__global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_kernel(const void* __restrict__ a, int lda,
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __restrict__ a, int lda,
                                                                  const bf16* __restrict__ w, int ldw, CT* __restrict__ c,
                                                                  int ldc, int M, int N, int K, const void* __restrict__ gamma,
                                                                  int gamma_f32, float eps, NormExtras extra, RopeExtras rope) {
   __shared__ float part[WAVES][RT][MT][64][4];
   __shared__ float sspart[RMS ? WAVES : 1][MT][64];
-  constexpr int LR = MT == 1 ? 16 : MT == 2 ? 32 : 64;  // lanes of a wave that stand for different rows in the sums below
+  constexpr int LR = MT == 2 ? 32 : 64;                 // lanes of a wave that stand for different rows in the sums below
   __shared__ float red[RMS ? 1 : WAVES][MT * 16];       // (with RMS the rows bring no partial sums)
   __shared__ float emit_sq[4][RT][MT][16];
   const float* __restrict__ parts = extra.parts;
@@ -1956,7 +1957,6 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : 1) void gemm_skinny_ke
         xf[it][0] = load_a<RMS>(a, lda, r, k, r < M && k < K, gamma, gamma_f32, ss[0]);
         xf[it][1] = load_a<RMS>(a, lda, r, k + 32, r < M && k + 32 < K, gamma, gamma_f32, ss[0]);
       }
-      if (!RMS) __builtin_amdgcn_sched_barrier(0);   // all loads of a slice are asked for before the first is waited for
 #pragma unroll
       for (int it = 0; it < ITERS; ++it)
 #pragma unroll
@@ -2290,7 +2290,7 @@ inline int launch_fold(const void* a, int lda, const bf16* w, int ldw, bf16* c, 
 // nontemporal, 11.4).  MB blocks of 8 rows of A share W's words.
 // Such a kernel lasts a few microseconds and is made of trips to memory one behind the other, so everything that it reads is asked
 // for before the first of it is waited for: the partial sums of the norm before it (a word of four rows a thread), what the
-// epilogue needs, W and the rows of A, up to a k of 2,048 at once (longer ones in turns).  Rows of W that the rotation or the
+// epilogue needs, W and the rows of A, as much of k at once as the registers hold (few_plan).  Rows of W that the rotation or the
 // gated unit pairs lie in one tile, four pairs, the partners mirrored (row n and 7 - n), and a cell's partner and a row's squares
 // come by lane moves: one barrier in all.   parts / emit / rotation: as NormExtras and RopeExtras say.
 // In steps of one row (of eight), the kernels before (16 rows of W a tile in half lines, partial sums one behind the other before
@@ -2614,7 +2614,7 @@ int launch_skinny_mt(int tiles, const void* a, int lda, const bf16* w, int ldw, 
   int waves, iters, rt;
   skinny_plan(tiles, K, MT, &waves, &iters, &rt);
   if constexpr ((EPI == EPI_STORE || EPI == EPI_ACCUMULATE) && !RMS) {
-    // Few rows of W (a narrow model's O and down projections, beyond the 8 rows of A that the folded kernel takes):
+    // Few rows of W (a narrow model's O and down projections of more than 16 rows):
     // workgroups of 8 rows of W, half of each tile left empty, so that twice as many compute units draw on memory.
     if (tiles < 256 && extra.parts == nullptr) {
       const int halves = (N + 7) / 8;
@@ -2675,7 +2675,7 @@ inline Route route(int epi, const void* a, int lda, const void* w, int ldw, int 
   const bool rings = ring_pays(epi, a, lda, w, ldw, M, N, K);
   if (blocks) r.block = block_plan(M, N, K, silu, 1, 1);
   bool whole = false;
-  if (workspace && M > 16 && !gamma && emits != 1 && !parts) {  // more than the skinny kernels' best range
+  if (workspace && M > 16 && !gamma && emits != 1 && !parts) {  // (gemm_few_kernel's rows are never divided)
     r.split = split_plan(M, N, K, silu);
     if (r.split.slices <= 1 || (silu && N % 16 != 0)) r.split = SplitPlan{};
     // a product that only stores needs no second pass: not divided where that takes less (QKV, 131 x 6,144 x 2,048: 16 us in slices, 13 whole)
@@ -2741,7 +2741,7 @@ extern "C" int gb_gemm_bf16_partial(const void* a, int lda, const void* w, int l
 }
 
 // The kernel that gb_gemm_bf16 (epilogues 0 to 2, no gamma, no norm to prepare; with a workspace or without) or gb_gemm_bf16_rope
-// (epilogue 3, no gamma) launches for these sizes: 0 tiled, 1 ring, 2 skinny or folded, 3 held, 4 block, 5 slices of k.
+// (epilogue 3, no gamma) launches for these sizes: 0 tiled, 1 ring, 2 few or skinny, 3 held, 4 block, 5 slices of k.
 extern "C" int gb_gemm_bf16_route(int M, int N, int K, int epilogue, int parts, int workspace) {
   if (epilogue == EPI_ROPE) return held_pays(epilogue, M, N, K, parts != 0) && held_takes(nullptr, K, nullptr, K, M, K) ? kHeld : kFew;
   return route(epilogue, nullptr, K, nullptr, K, M, N, K, false, parts != 0, 0, workspace != 0).kernel;
@@ -2831,7 +2831,7 @@ extern "C" int gb_gemm_bf16(const void* a, int lda, const void* w, int ldw, void
 }
 
 // A product whose epilogue is the clamped gated unit (see Glu): W stacks gate rows over up rows as for epilogue 2, C is
-// bfloat16 [M, N / 2].  Up to 64 rows the skinny kernel, beyond them the ring or the tiled kernel.
+// bfloat16 [M, N / 2].  Up to 16 rows gemm_few_kernel, up to 64 the skinny kernel, beyond them the ring or the tiled kernel.
 extern "C" int gb_gemm_bf16_glu(const void* a, int lda, const void* w, int ldw, void* c, int ldc, int M, int N, int K,
                                 float limit, float alpha, float plus, hipStream_t stream) {
   GB_REQUIRE(M > 0 && N > 0 && N % 2 == 0 && K > 0 && K % 8 == 0, "gemm_bf16_glu: bad sizes M=%d N=%d K=%d", M, N, K);
