@@ -464,16 +464,19 @@ def test_gemm_bf16_fused_rms_norm(N, K, M, silu, gamma_dtype):
 
 @pytest.mark.parametrize("M,N,K,N2,silu", [(1, 64, 176, 96, False), (5, 352, 64, 176, True), (8, 2048, 2048, 6144, False),
                                            (8, 2048, 8192, 16384, True), (3, 960, 2560, 2880, False),
-                                           # more than 8 rows: the skinny kernel emits (tiles of 8 columns while they are
-                                           # few, of 16 beyond), and takes the partial sums of up to 64 rows
+                                           # more than 8 rows (tiles of 8 columns while they are few, of 16 beyond), and more than 16: the
+                                           # skinny kernel emits and takes the partial sums of up to 64
                                            (12, 960, 2560, 2880, False), (40, 24704, 128, 512, False), (64, 352, 64, 176, True),
                                            (20, 4096, 1024, 1024, True), (9, 72, 264, 48, False), (17, 2048, 1024, 16384, True),
                                            (20, 960, 960, 5120, True), (33, 960, 776, 1600, False),
                                            # a k beyond 2,048: half tiles of up to 24 rows and of more, one tile, two
                                            (20, 968, 2056, 256, False), (32, 968, 2056, 256, False), (32, 5128, 2304, 256, False),
                                            (24, 6160, 2568, 256, False), (33, 24704, 2056, 256, False),
-                                           # at most 8 rows by so many rows of W that the folded kernel does not pay
-                                           (5, 4096, 512, 256, False)])
+                                           # up to 16 rows, sums of 16 columns: two tiles a workgroup, of a number that two does not divide, and
+                                           # four; four waves of two blocks and of three, eight of two, three and four
+                                           (5, 4096, 512, 256, False), (12, 4096, 512, 256, False), (16, 8200, 264, 256, False), (5, 8216, 520, 256, False),
+                                           (5, 8192, 520, 256, False), (9, 4104, 2632, 256, False), (9, 4104, 776, 256, True), (16, 8200, 1032, 256, False),
+                                           (16, 4096, 2048, 256, False)])
 @pytest.mark.parametrize("gamma_dtype", [torch.float32, torch.bfloat16])
 def test_gemm_bf16_prepares_the_next_norm(M, N, K, N2, silu, gamma_dtype):
     """The product that adds into the residual and, on its way out, writes what the RMS norm that reads
@@ -845,7 +848,7 @@ def test_gemm_bf16_one_hot_rows_and_columns():
     ops.gemm(to_dev(a), to_dev(w.bfloat16()), c)
     want = a.float()[:, [(7 * n + 3) % K for n in range(N)]]
     assert torch.equal(c.cpu(), want)
-    for rows in (9, 8, 5, 1):   # the skinny kernel, and the one that folds two k ranges into a tile
+    for rows in (17, 9, 8, 5, 1):   # the skinny kernel, and the one that folds two k ranges into a tile
         c2 = torch.zeros(rows, N, device=DEV)
         ops.gemm(to_dev(a[:rows]), to_dev(w.bfloat16()), c2)
         assert torch.equal(c2.cpu(), want[:rows]), rows
@@ -1050,13 +1053,34 @@ def test_gemm_bf16_rotates_behind_the_partial_sums_of_a_norm(M, nh, nkv, hd, K, 
     """The stacked q/k/v product of rows whose norm comes as partial sums: the scale is in what is rotated, in the rows and in both
     pages.  Against float64, element by element."""
     from glassbox_amd import ops
-    N, page, eps = (nh + 2 * nkv) * hd, 16, 1e-5
-    assert ops.gemm_route(M, N, K, heads=True, parts=True) == kernel
+    assert ops.gemm_route(M, (nh + 2 * nkv) * hd, K, heads=True, parts=True) == kernel
+    check_rotation(M, nh, nkv, hd, K, n, 16)
+
+
+# one tile a workgroup, two, three and four, with each number of waves and blocks that few_plan (csrc/hip/gemm_bf16.hip) gives them; the
+# last workgroup's tiles beyond the rows of W, k of whole turns and of part of one; pages that are a power of two and pages that are not
+@pytest.mark.parametrize("M,nh,nkv,hd,K,n,page", [
+    (9, 4, 2, 16, 72, 0, 48), (16, 32, 16, 64, 520, 64, 16), (12, 15, 5, 64, 776, 97, 48), (16, 64, 16, 64, 704, 0, 64), (9, 96, 16, 64, 640, 80, 48),
+    (16, 8, 4, 48, 1032, 0, 80), (9, 48, 8, 64, 1000, 125, 16), (12, 32, 32, 64, 1032, 129, 48), (16, 96, 16, 64, 1000, 0, 16),
+    (9, 8, 2, 128, 2568, 321, 48), (16, 48, 8, 64, 2600, 0, 32), (12, 32, 8, 128, 4096, 256, 16), (9, 8, 4, 64, 2048, 256, 48),
+    (16, 40, 12, 64, 2048, 0, 16), (12, 32, 32, 64, 2048, 256, 48), (12, 32, 32, 64, 2048, 0, 16), (16, 50, 1, 80, 448, 56, 48),
+    (8, 96, 16, 64, 1536, 192, 48), (5, 32, 32, 64, 2048, 256, 80), (8, 97, 16, 64, 2048, 0, 16), (1, 8, 2, 128, 2560, 320, 48),
+    (8, 8, 4, 16, 8192, 0, 48)])
+def test_gemm_bf16_of_up_to_16_rows_rotates_and_writes_pages_of_any_size(M, nh, nkv, hd, K, n, page):
+    check_rotation(M, nh, nkv, hd, K, n, page)
+
+
+def check_rotation(M, nh, nkv, hd, K, n, page):
+    """A rotating product, behind n partial sums of a norm or (n = 0) of rows as they are, against float64 element by element."""
+    from glassbox_amd import ops
+    N, eps = (nh + 2 * nkv) * hd, 1e-5
     g = torch.Generator().manual_seed(M + n)
     a, w = (rnd(M, K, seed=1) * 0.5).bfloat16(), (rnd(N, K, seed=2) / math.sqrt(K)).bfloat16()
     stride = ops.parts_stride(M)
-    sums = torch.rand(n, stride, generator=g) * 20 + 0.1
-    scale = 1 / torch.sqrt(sums[:, :M].double().sum(0) / K + eps)
+    scale = torch.ones(M, dtype=torch.float64)
+    if n:
+        sums = torch.rand(n, stride, generator=g) * 20 + 0.1
+        scale = 1 / torch.sqrt(sums[:, :M].double().sum(0) / K + eps)
     angles = torch.rand(M, hd // 2, generator=g) * 6
     cos, sin = angles.cos(), angles.sin()
     slots = torch.randperm(5 * page, generator=g)[:M].to(torch.int32)
@@ -1070,12 +1094,33 @@ def test_gemm_bf16_rotates_behind_the_partial_sums_of_a_norm(M, nh, nkv, hd, K, 
     k_pages = torch.zeros(ops.key_pages_shape(5, nkv, page, hd), device=DEV, dtype=torch.bfloat16)
     v_pages = torch.zeros(5, nkv, hd, page, device=DEV, dtype=torch.bfloat16)
     qkv = torch.full((M, N), 9.0, device=DEV, dtype=torch.bfloat16)
-    ops.gemm_rope(to_dev(a), to_dev(w), qkv, nh, nkv, hd, to_dev(cos), to_dev(sin), to_dev(slots), k_pages, v_pages, rms_parts=(to_dev(sums), n, eps))
+    ops.gemm_rope(to_dev(a), to_dev(w), qkv, nh, nkv, hd, to_dev(cos), to_dev(sin), to_dev(slots), k_pages, v_pages, rms_parts=(to_dev(sums), n, eps) if n else None)
     rows = qkv.cpu().double().view(M, nh + 2 * nkv, hd)
     assert ((rows - want).abs() <= bound).all()
     keys, idx = ops.unpack_keys(k_pages).cpu().double(), slots.long()
     assert torch.equal(keys[idx // page, :, idx % page, :], rows[:, nh:nh + nkv])
     assert torch.equal(v_pages.cpu().double()[idx // page, :, :, idx % page], rows[:, nh + nkv:])
+    free = torch.ones(5 * page, dtype=torch.bool)
+    free[idx] = False
+    idx = torch.nonzero(free).flatten()
+    assert (keys[idx // page, :, idx % page, :] == 0).all() and (v_pages.cpu()[idx // page, :, :, idx % page] == 0).all()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 12, 16, 17])
+@pytest.mark.parametrize("N,K", [(16, 8), (264, 520), (5120, 960), (8208, 2048), (16384, 1032)])
+def test_gemm_bf16_clamped_unit_of_few_rows(M, N, K):
+    """min(g, limit) sigmoid(alpha g) (clamp(u) + plus) at the limits' edges and inside them, against float64 element by element."""
+    from glassbox_amd import ops
+    a, w = (rnd(M, K, seed=1) * 3).bfloat16(), (rnd(N, K, seed=2) / math.sqrt(K)).bfloat16()
+    limit, alpha, plus = 4.0, 1.702, 1.0
+    prod, tol = a.double() @ w.double().T, sum_bound(a, w)
+    g, u = prod[:, :N // 2].clamp(max=limit), prod[:, N // 2:].clamp(-limit, limit)
+    want = g / (1 + torch.exp(-alpha * g)) * (u + plus)
+    # |d (g sigmoid(alpha g)) / dg| < 1.1 and its size at most |g|; the unit's own arithmetic a few roundings; one to 16 bits
+    bound = tol * (1.1 * (u + plus).abs() + g.abs()) + 1.1 * tol * tol + 2 ** -20 * (1 + want.abs()) + 2 ** -8 * want.abs()
+    out = torch.full((M, N // 2), 9.0, device=DEV, dtype=torch.bfloat16)
+    ops.gemm_glu(to_dev(a), to_dev(w), out, limit, alpha, plus)
+    assert ((out.cpu().double() - want).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("M,K", [(1, 64), (8, 2048), (9, 72), (16, 1032), (20, 64), (48, 2048)])
