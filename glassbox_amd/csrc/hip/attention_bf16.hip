@@ -24,6 +24,8 @@
 // second kernel), so the result is the same on every run and in every row of a step.
 // crates/glassbox-core/src/model.rs:285-312 is the formula.
 #include "attention_bf16.h"
+#include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "common.h"
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
                                                             const int32_t* __restrict__ tables, int table_stride,
                                                             const bf16* __restrict__ kp, const bf16* __restrict__ vp, int nh,
                                                             int nkv, int P, float scale, int window, int keep, int chunk,
-                                                            int splits, int G, PageQuotient quotient, unsigned group_magic, Extra ex) {
+                                                            int splits, int G, PageQuotient quotient, unsigned group_magic, int row_keys, Extra ex) {
   constexpr int KS = (HD + 31) / 32, DB = HD / 16;
   constexpr bool WIDE = std::is_same<OT, float>::value;
   extern __shared__ float decode_lds[];
@@ -248,13 +250,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   float* sm_acc = sm_l + WAVES * 16;      // [WAVES][HD][G]
   const int pos = positions[s];
   // A wave that takes its tiles in turn knows its first one before it knows how long the context is: the tile's entries of the page
-  // table (inside the row, wherever they lie) are asked for beside the position and not behind it.
+  // table (inside the row, wherever they lie) are asked for beside the position and not behind it.  They are the ones wanted where a row
+  // holds the position's page (row_keys: the keys that table_stride entries stand for), which rows that lie over each other need not.
   constexpr bool AHEAD = MODE == kPlainScores && WAVES <= 8 && HD <= 64, DIV = WAVES == 16;
   Pages ahead;
   if (AHEAD) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kb = split * chunk + (w + kvh + 5 * s) % WAVES * 64;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) ahead.of[t] = tables[(size_t)s * table_stride + min(page_index<DIV>(kb + 16 * t, quotient, P), table_stride - 1)];
+    for (int t = 0; t < 4; ++t) ahead.of[t] = tables[(size_t)s * table_stride + min(page_index<DIV>(kb + 16 * t, quotient, P), max(table_stride, 1) - 1)];
   }
   const int lo = first_key(pos, window, MODE == kPlainScores ? 0 : ex.span);
   const int c0 = (MODE == kPlainScores ? 0 : chunks_from(lo, ex.span)) + split * chunk;
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_kernel(const bf16* __restri
   const int first = run ? wave * each : place, step = run ? 64 : 64 * WAVES;
   const int stop = run ? min(c0 + (first + each) * 64, end) : end;
   Pages next;
-  if (AHEAD && c0 + first * 64 >= (lo & ~15)) {
+  if (AHEAD && pos < row_keys && c0 + first * 64 >= (lo & ~15)) {
     // (tiles of 16 beyond the last key stand for the one that holds it, as in tile_key)
     const int last = (pos - (c0 + first * 64)) >> 4;
 #pragma unroll
@@ -1233,6 +1236,7 @@ extern "C" int gb_attention_supported_head_size(int hd) { return hd >= 16 && hd 
 // q, out: rows 0 .. n_decode-1 are the decoding requests (one row each).  ws_acc must hold
 // n_decode*nh*splits*hd floats and ws_ml n_decode*nh*splits*2, with splits = ceil(max_context / chunk).
 // keep_first > 0 (with a window): keys 0 .. keep_first-1 are read wherever the window has moved past them.
+// Each row of the tables is table_stride entries that exist: entries behind those that a context needs may be read, and are not used.
 template <typename OT>
 static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, void* ws_acc, void* ws_ml,
                          const int32_t* positions, const int32_t* tables, int table_stride, const void* k_pages,
@@ -1273,6 +1277,7 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
   const size_t lds = (size_t)waves * (32 + (size_t)hd * G) * sizeof(float);
   const dim3 grid(splits, nkv, n_decode), block(waves * 64);
   const PageQuotient quotient = page_quotient(page_size);
+  const int row_keys = (int)std::min<long long>(std::max(table_stride, 0) * (long long)page_size, INT_MAX);
   const unsigned group_magic = (65536 + G - 1) / G;
   // capped and sloped scores are kernels of their own (bfloat16 results only), so that the others' score loops are what they were
   constexpr bool kCanCap = std::is_same<OT, bf16>::value;
@@ -1282,7 +1287,7 @@ static int decode_launch(const void* q, int q_stride, OT* out, int out_stride, v
 #define GB_DECODE(HD, WAVES, MODE)                                                                                         \
   hipLaunchKernelGGL((decode_kernel<HD, WAVES, OT, MODE>), grid, block, lds, stream, (const bf16*)q, q_stride, out, out_stride, \
                      (float*)ws_acc, (float*)ws_ml, positions, tables, table_stride, (const bf16*)k_pages,                  \
-                     (const bf16*)v_pages, nh, nkv, page_size, scale, window, keep_first, chunk, splits, G, quotient, group_magic, ex)
+                     (const bf16*)v_pages, nh, nkv, page_size, scale, window, keep_first, chunk, splits, G, quotient, group_magic, row_keys, ex)
 #define GB_CASE(HD)                                                 \
   if (hd == HD) {                                                   \
     if (cap) {                                                      \

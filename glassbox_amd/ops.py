@@ -1924,6 +1924,18 @@ def decode_chunk(n_decode: int, n_kv_heads: int, max_context: int, head_dim: int
     return max(256, -(-chunk // 256) * 256)
 
 
+def _whole_rows(tables: torch.Tensor):
+    """Block tables and the entries from row to row, all of which the decode kernel may read: tables cut from wider ones whose last
+    row would reach beyond their memory are copied."""
+    rows, width = tables.shape
+    row = tables.stride(0)
+    if row == width or rows == 1:
+        return tables, width
+    if row > width and tables.storage_offset() + rows * row > tables.untyped_storage().nbytes() // tables.element_size():
+        return tables.contiguous(), width
+    return tables, row
+
+
 def attention_decode(q: torch.Tensor, out: torch.Tensor, ctx, cache, n_heads: int, scale: float, window: int,
                      keep_first: int = 0, chunk: int = 0, softcap: float = 0.0, sinks: Optional[torch.Tensor] = None,
                      slopes: Optional[torch.Tensor] = None) -> None:
@@ -1934,7 +1946,7 @@ def attention_decode(q: torch.Tensor, out: torch.Tensor, ctx, cache, n_heads: in
     _, nkv, page, hd = _check_pages(k_pages, v_pages, torch.bfloat16, "attention_decode")
     if q.dtype != torch.bfloat16 or out.dtype not in (torch.bfloat16, torch.float32) or q.shape[1] != n_heads * hd:
         raise KernelError("attention_decode: q must be bfloat16 [n, heads * head size], out bfloat16 or float32")
-    tables = ctx.tables[cache.group]
+    tables, row = _whole_rows(ctx.tables[cache.group])
     max_context = int(ctx.host["max_context"])
     mask_chunk = int(chunk)   # the runs of positions a token sees; ``chunk`` below is the keys a workgroup takes
     if mask_chunk:            # what is divided over workgroups is a run, from the tile of 64 keys that it begins in
@@ -1946,17 +1958,17 @@ def attention_decode(q: torch.Tensor, out: torch.Tensor, ctx, cache, n_heads: in
     lib = _lib("attention_bf16")
     if mask_chunk or softcap or sinks is not None or slopes is not None:
         _launch(lib, lib.gb_attention_decode_bf16_by, _p(q), _rows(q, "q"), _p(out), _rows(out, "out"),
-                1 if out.dtype == torch.float32 else 0, _p(ws_acc), _p(ws_ml), _p(ctx.positions), _p(tables), tables.stride(0),
+                1 if out.dtype == torch.float32 else 0, _p(ws_acc), _p(ws_ml), _p(ctx.positions), _p(tables), row,
                 _p(k_pages), _p(v_pages), n_dec, n_heads, nkv, hd, page, float(scale), int(window), int(keep_first), mask_chunk,
                 float(softcap), _p(_sinks(sinks, n_heads)), _p(_sinks(slopes, n_heads)), chunk, max_context, _stream())
         return
     if keep_first or out.dtype == torch.float32:
         _launch(lib, lib.gb_attention_decode_bf16_out32 if out.dtype == torch.float32 else lib.gb_attention_decode_bf16_keep, _p(q), _rows(q, "q"), _p(out), _rows(out, "out"), _p(ws_acc), _p(ws_ml),
-                _p(ctx.positions), _p(tables), tables.stride(0), _p(k_pages), _p(v_pages), n_dec, n_heads, nkv, hd, page,
+                _p(ctx.positions), _p(tables), row, _p(k_pages), _p(v_pages), n_dec, n_heads, nkv, hd, page,
                 float(scale), int(window), int(keep_first), chunk, max_context, _stream())
         return
     _launch(lib, lib.gb_attention_decode_bf16, _p(q), _rows(q, "q"), _p(out), _rows(out, "out"), _p(ws_acc), _p(ws_ml),
-                                             _p(ctx.positions), _p(tables), tables.stride(0), _p(k_pages), _p(v_pages),
+                                             _p(ctx.positions), _p(tables), row, _p(k_pages), _p(v_pages),
                                              n_dec, n_heads, nkv, hd, page, float(scale), int(window), chunk,
                                              max_context, _stream())
 

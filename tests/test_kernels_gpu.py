@@ -1713,6 +1713,40 @@ def test_tuned_decode_finds_a_key_in_pages_of_any_size(page, ctxlen):
         assert (out.cpu().float().view(nh, hd) - values[target].float()).abs().max().item() < 2e-2, f"key at {target} was not found"
 
 
+@pytest.mark.parametrize("layout", ["a column turned", "one row for all", "rows over each other", "the end of a wider table", "the middle of one"])
+def test_tuned_decode_takes_block_tables_of_any_row_stride(layout):
+    """A row's first entries are asked for before the position is known, wherever the rows lie: the bits of tables of their own."""
+    from types import SimpleNamespace
+    from glassbox_amd import ops
+    nh, nkv, hd, n = 6, 2, 64, 1 if layout == "a column turned" else 3
+    k_pages, v_pages, tables, _, _ = paged_setup([300], nkv, hd, 16, seed=8, dtype=torch.bfloat16)
+    width = tables.shape[1]
+    rows = tables.expand(n, -1).contiguous()
+    if layout == "a column turned":
+        view = to_dev(tables[0][:, None].contiguous()).t()
+    elif layout == "one row for all":
+        view = to_dev(tables).expand(n, -1)
+    elif layout == "rows over each other":
+        view = torch.as_strided(to_dev(torch.cat([tables[0], tables[0][:4]])), (n, width), (2, 1))
+        rows = view.cpu().contiguous()
+    else:
+        below, at = (0, 9) if layout == "the end of a wider table" else (1, 4)
+        wide = torch.full((n + below, width + 9), -1, dtype=torch.int32)
+        wide[:n, at:at + width] = rows
+        view = to_dev(wide)[:n, at:at + width]
+    lens = [300, 17, 290][:n]
+    q = to_dev((rnd(n, nh * hd, seed=6) * 0.7).bfloat16())
+    cache = SimpleNamespace(k_pages=to_dev(ops.pack_keys(k_pages)), v_pages=to_dev(v_pages), group=0)
+    outs = []
+    for t in (to_dev(rows), view):
+        ctx = BareContext([1] * n, lens, rows, max_context=300)
+        ctx.tables = [t]
+        out = torch.zeros(n, nh * hd, device=DEV, dtype=torch.bfloat16)
+        ops.attention_decode(q, out, ctx, cache, nh, 1 / math.sqrt(hd), 0)
+        outs.append(out.cpu())
+    assert view.stride() != to_dev(rows).stride() and torch.equal(*outs)
+
+
 def test_tuned_decode_over_tens_of_thousands_of_keys():
     """Contexts of 40,000 and 33,333 keys beside one of 5: some hundred and sixty chunks a request for the second
     pass to merge, block tables of 2,500 pages.  Against the plain kernel on random keys, and with one key made to
