@@ -2294,8 +2294,9 @@ inline int launch_fold(const void* a, int lda, const bf16* w, int ldw, bf16* c, 
 // gated unit pairs lie in one tile, four pairs, the partners mirrored (row n and 7 - n), and a cell's partner and a row's squares
 // come by lane moves: one barrier in all.   parts / emit / rotation: as NormExtras and RopeExtras say.
 // In steps of one row (of eight), the kernels before (16 rows of W a tile in half lines, partial sums one behind the other before
-// W; 8 rows for the products by few rows of W) and now: SmolLM2-1.7B gate/up 13.9 -> 12.5 us (15.6 -> 13.8), QKV 9.5 -> 7.1
-// (10.1 -> 8.1), down 9.2 -> 8.0 (11.0 -> 10.5), vocabulary 35.7 -> 31.3 (40.4 -> 34.4); SmolLM2-135M a layer 17.3 -> 14.5.
+// W; 8 rows for the products by few rows of W) and now: SmolLM2-1.7B gate/up 13.9 -> 12.6 us (15.6 -> 13.3), QKV 9.5 -> 7.1
+// (10.1 -> 7.7), down 9.2 -> 8.0 (11.0 -> 9.8), vocabulary 35.7 -> 31.0 (40.4 -> 33.8); SmolLM2-135M a layer 17.3 -> 13.6.  (Slower is a
+// gate/up of 9 rows and more, a k of up to 400 and very many rows of W: 9 rows by 98,304 x 264 13.8 -> 15.6, in no number of tiles less.)
 __device__ __forceinline__ float lane_mirror8(float v) {   // the value of lane 7 - n of the eight neighbouring lanes
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));
 }
