@@ -1921,12 +1921,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (p0 + u * STEP < n_parts) got[u] = mine[(p0 + u * STEP) * 64];
-    for (int p = p0 + 4 * STEP; p < n_parts; p += 8 * STEP) {
-      float more[8];
+    constexpr int AT_ONCE = SHORT ? 4 : 8;
+    for (int p = p0 + 4 * STEP; p < n_parts; p += AT_ONCE * STEP) {
+      float more[AT_ONCE];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) more[u] = p + u * STEP < n_parts ? mine[(p + u * STEP) * 64] : 0.f;
+      for (int u = 0; u < AT_ONCE; ++u) more[u] = p + u * STEP < n_parts ? mine[(p + u * STEP) * 64] : 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) got[u % 4] += more[u];
+      for (int u = 0; u < AT_ONCE; ++u) got[u % 4] += more[u];
     }
   }
   auto add_up = [&] {
@@ -1936,10 +1937,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
     for (int o = LR; o < 64; o <<= 1) sum += __shfl_xor(sum, o, kWave);
     if (lane < LR && lane < MT * 16) red[wave][lane] = sum;
   };
-  if (!SHORT) add_up();
   // a 64-wide k block is two MFMA steps of 32: lane group q holds k = 8q..8q+7 of each
-  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
-    bf16x8 wf[RT][ITERS][2];
+  bf16x8 wf[RT][ITERS][2];
+  auto ask = [&](int kbeg) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -1948,7 +1948,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const void* __r
         wf[rt][it][0] = load_word<SHORT>(row_ok[rt] && k < K, wrow[rt], k);
         wf[rt][it][1] = load_word<SHORT>(row_ok[rt] && k + 32 < K, wrow[rt], k + 32);
       }
-    if (SHORT && kbeg == 0) add_up();
+  };
+  if (SHORT) ask(0);
+  add_up();
+  for (int kbeg = 0; kbeg < K; kbeg += ITERS * WAVES * 64) {
+    if (!SHORT || kbeg > 0) ask(kbeg);
     if (MT == 1) {
       bf16x8 xf[ITERS][2];
 #pragma unroll
