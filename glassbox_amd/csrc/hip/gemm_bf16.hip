@@ -2532,9 +2532,11 @@ inline FewPlan few_plan(int epi, int M, int N, int K) {
     }
   }
   // All of k at once where it is short; of a longer one turns of eight waves, whose two, three or four blocks a wave leave the least of the
-  // last turn empty, the most that do (one row by 4,096 x 14,336 in turns of 32 blocks 19.7 us, of 64 21.0; 9 rows by 960 x 2,560 in turns of
-  // 24 5.4, of 64 5.7).  Beyond 8 rows four only of up to two tiles a workgroup and a k of up to 4,096 (9 rows by 2,048 x 8,192 with two 11.1,
-  // with four 11.7), and of four tiles not three: the registers of two such workgroups a unit end there.
+  // last turn empty, the most that do (one row by 28,672 x 4,096 38.3 us in turns of 32 blocks of four tiles, of two tiles 35.7).  Beyond 8 rows
+  // four only of up to two tiles a workgroup and a k of up to 4,096, and of four tiles not three: the registers of two such workgroups a unit
+  // end there.  In which order a cell is summed depends on the waves, not on the turns.  Few tiles by a k beyond 2,048 (O and down projections)
+  // have sixteen waves: eight would be 2 to 6 % faster (one row by 4,096 x 14,336 19.7 us, 21.0), but sum in another order, and a model of 32 such
+  // layers in 16 bits ends further from the results it had (0.011 of the logits' norm) than those may move.
   if (blocks <= 8) return p;
   if (blocks <= 12) {
     p.iters = 3;
@@ -2545,8 +2547,8 @@ inline FewPlan few_plan(int epi, int M, int N, int K) {
     p.iters = 5;   // (one row by 960 x 2,560 in one turn 3.8 us, in two of 24 blocks 4.1)
     return p;
   }
-  if (!many && p.rt == 1 && blocks > 120 && blocks <= 128) {
-    p.waves = 16, p.iters = 8;   // (eight rows by 2,048 x 8,192 in one turn 9.7 us, in four 10.0; one row 8.0 and 7.8)
+  if (blocks > 32 && p.rt <= 2 && tiles < 768) {
+    p.waves = 16, p.iters = blocks <= 64 || p.rt == 2 || many ? 4 : 8;
     return p;
   }
   auto asked = [&](int it) { return (blocks + 8 * it - 1) / (8 * it) * (10 * it + 1); };
@@ -2572,7 +2574,7 @@ int launch_few_mb(const bf16* a, int lda, const bf16* w, int ldw, CT* c, int ldc
 #define GB_FEWS(WV, IT) GB_FEW(WV, IT, 1) GB_FEW(WV, IT, 2) GB_FEW(WV, IT, 3) GB_FEW(WV, IT, 4)
   // (what few_plan can ask for)
   GB_FEW(4, 2, 1) GB_FEW(4, 2, 2) GB_FEWS(4, 3) GB_FEWS(8, 2) GB_FEW(8, 3, 1) GB_FEW(8, 3, 2) GB_FEW(8, 3, 3)
-  GB_FEW(8, 4, 1) GB_FEW(8, 4, 2)
+  GB_FEW(8, 4, 1) GB_FEW(8, 4, 2) GB_FEW(16, 4, 1) GB_FEW(16, 4, 2)
   if constexpr (MB == 1) { GB_FEW(8, 3, 4) GB_FEW(8, 4, 3) GB_FEW(8, 4, 4) GB_FEW(8, 5, 1) GB_FEW(16, 8, 1) }
 #undef GB_FEWS
 #undef GB_FEW
